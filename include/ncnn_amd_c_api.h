@@ -288,6 +288,13 @@ typedef struct __ncnn_hipmat_t* ncnn_hipmat_t;
 int ncnnhip_net_upload(ncnn_net_t net, const ncnn_mat_t mat, ncnn_hipmat_t* out);
 void ncnnhip_hipmat_destroy(ncnn_hipmat_t m);
 int ncnnhip_hipmat_download(const ncnn_hipmat_t m, ncnn_mat_t* out);
+/* A view of dense caller-owned memory, [n][c][h][w] without padding between planes or samples (a numpy array, say), and the
+ * form of ncnn_extractor_input for memory the caller takes back on return: the upload starts in the call.  Returns 1 (nothing
+ * fed) when the blob is not consumed on the device: feed it with ncnn_extractor_input then.  index -1: by name. */
+ncnn_mat_t ncnnhip_mat_create_external_dense(int w, int h, int c, int n, void* data, size_t elemsize);
+int ncnnhip_extractor_input_copied(ncnn_extractor_t ex, int index, const char* name, const ncnn_mat_t mat);
+/* dims, w, h, d, c, n, elemsize, cstep, nstep of a Mat, in one call */
+void ncnnhip_mat_get_layout(const ncnn_mat_t mat, size_t layout[9]);
 int ncnnhip_extractor_input_hipmat(ncnn_extractor_t ex, const char* name, const ncnn_hipmat_t m);
 int ncnnhip_extractor_extract_hipmat(ncnn_extractor_t ex, const char* name, ncnn_hipmat_t* out);
 int ncnnhip_extractor_synchronize(ncnn_extractor_t ex);

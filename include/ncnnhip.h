@@ -69,6 +69,13 @@ int ncnnhip_memcpy_d2d(void* dst_dev, const void* src_dev, size_t bytes, void* s
 int ncnnhip_memset(void* dev, int byte, size_t bytes, void* stream);
 /* rows x row_bytes between two pitched device buffers (appending to a key/value cache whose rows grow) */
 int ncnnhip_copy2d(void* dst_dev, size_t dst_pitch, const void* src_dev, size_t src_pitch, size_t row_bytes, size_t rows, void* stream);
+/* Page-locked host memory, which kernels and copies reach over PCIe without a bounce buffer: what uploads and downloads are
+ * staged through (the reference's VkAllocator hands out host-visible staging buffers, src/allocator.h:267-300).
+ * ncnnhip_copy moves `bytes` with a kernel; either side may be device memory or such host memory.  For small transfers that
+ * is one launch instead of a copy command with a set-up of its own. */
+int ncnnhip_host_malloc(void** host, size_t bytes);
+int ncnnhip_host_free(void* host);
+int ncnnhip_copy(void* dst, const void* src, size_t bytes, void* stream);
 int ncnnhip_event_create(void** event);
 int ncnnhip_event_destroy(void* event);
 int ncnnhip_event_record(void* event, void* stream);

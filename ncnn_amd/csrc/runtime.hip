@@ -27,6 +27,18 @@ int map_hip_error(hipError_t e, const char* what)
     return e == hipErrorOutOfMemory ? NCNNHIP_OOM : NCNNHIP_ERROR;
 }
 
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+// 16 bytes per thread where both sides are aligned, the rest byte by byte.  Bound by PCIe or by the launch: it moves the
+// small blobs at the ends of a pass (scores, vectors), where a copy command costs more than the transfer.
+__global__ __launch_bounds__(256) void copy_kernel(unsigned char* __restrict__ dst, const unsigned char* __restrict__ src, size_t vectors, size_t bytes)
+{
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < vectors) reinterpret_cast<v4i*>(dst)[i] = reinterpret_cast<const v4i*>(src)[i];
+    const size_t j = vectors * 16 + i;
+    if (j < bytes) dst[j] = src[j];
+}
+
 } // namespace ncnnhip
 
 using namespace ncnnhip;
@@ -247,6 +259,34 @@ int ncnnhip_memset(void* dev, int byte, size_t bytes, void* stream)
     if (bytes == 0) return NCNNHIP_OK;
     NCNNHIP_CHECK(hipMemsetAsync(dev, byte, bytes, as_stream(stream)));
     return NCNNHIP_OK;
+}
+
+int ncnnhip_host_malloc(void** host, size_t bytes)
+{
+    NCNNHIP_REQUIRE(host, "null out pointer");
+    *host = 0;
+    NCNNHIP_CHECK(hipHostMalloc(host, bytes ? bytes : 4, hipHostMallocDefault));
+    return NCNNHIP_OK;
+}
+
+int ncnnhip_host_free(void* host)
+{
+    NCNNHIP_REQUIRE(host, "ncnnhip_host_free: null pointer");
+    NCNNHIP_CHECK(hipHostFree(host));
+    return NCNNHIP_OK;
+}
+
+int ncnnhip_copy(void* dst, const void* src, size_t bytes, void* stream)
+{
+    NCNNHIP_REQUIRE(dst && src, "ncnnhip_copy: null pointer");
+    if (bytes == 0) return NCNNHIP_OK;
+    // the tail (or everything, when a side is not aligned) goes one byte per thread, from the same thread index on
+    const size_t vectors = ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15) == 0 ? bytes / 16 : 0;
+    const size_t threads = vectors > bytes - vectors * 16 ? vectors : bytes - vectors * 16;
+    NCNNHIP_REQUIRE(threads <= (size_t)0x7fffffff * 256, "ncnnhip_copy: %zu bytes", bytes);
+    hipLaunchKernelGGL(copy_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, as_stream(stream), (unsigned char*)dst, (const unsigned char*)src, vectors,
+                       bytes);
+    return launch_status("copy_kernel");
 }
 
 int ncnnhip_event_create(void** event)

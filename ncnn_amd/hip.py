@@ -72,6 +72,9 @@ _SIGNATURES = {
     "ncnnhip_memcpy_d2h": [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p],
     "ncnnhip_memcpy_d2d": [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p],
     "ncnnhip_memset": [C.c_void_p, C.c_int, C.c_size_t, C.c_void_p],
+    "ncnnhip_host_malloc": [c_void_pp, C.c_size_t],
+    "ncnnhip_host_free": [C.c_void_p],
+    "ncnnhip_copy": [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p],
     "ncnnhip_event_create": [c_void_pp],
     "ncnnhip_event_destroy": [C.c_void_p],
     "ncnnhip_event_record": [C.c_void_p, C.c_void_p],

@@ -114,6 +114,8 @@ def lib():
             "ncnn_extractor_input": (ci, [vp, C.c_char_p, vp]), "ncnn_extractor_extract": (ci, [vp, C.c_char_p, C.POINTER(vp)]),
             "ncnnhip_register_int8_layers": (ci, [vp]), "ncnnhip_register_attention_layer": (ci, [vp]), "ncnnhip_extractor_attach_stream": (vp, [vp]), "ncnnhip_extractor_detach_stream": (None, [vp]),
             "ncnnhip_net_upload": (ci, [vp, vp, C.POINTER(vp)]), "ncnnhip_hipmat_destroy": (None, [vp]), "ncnnhip_hipmat_download": (ci, [vp, C.POINTER(vp)]),
+            "ncnnhip_mat_create_external_dense": (vp, [ci, ci, ci, ci, vp, cs]), "ncnnhip_extractor_input_copied": (ci, [vp, ci, C.c_char_p, vp]),
+            "ncnnhip_mat_get_layout": (None, [vp, C.POINTER(cs * 9)]),
             "ncnnhip_extractor_input_hipmat": (ci, [vp, C.c_char_p, vp]), "ncnnhip_extractor_extract_hipmat": (ci, [vp, C.c_char_p, C.POINTER(vp)]),
             "ncnnhip_extractor_synchronize": (ci, [vp]),
             "ncnnhip_extractor_set_layer_timing": (None, [vp, ci]), "ncnnhip_extractor_layer_timing": (ci, [vp, C.c_char_p, cs, C.POINTER(cs)]),
@@ -244,23 +246,26 @@ class Mat:
             buf[:, : h * w] = a[b].reshape(c, h * w)
         return m
 
+    @classmethod
+    def view(cls, a):
+        """A view of a [c][h][w] or [n][c][h][w] array for a call that has read it when it returns; other shapes as from_numpy."""
+        a = np.ascontiguousarray(a)
+        if a.ndim not in (3, 4) or a.dtype not in (np.float32, np.int8) or 0 in a.shape:
+            return cls.from_numpy(a)
+        n, c, h, w = a.shape if a.ndim == 4 else (1,) + a.shape
+        return cls(lib().ncnnhip_mat_create_external_dense(w, h, c, n, a.ctypes.data, a.dtype.itemsize), keep=a)
+
     def to_numpy(self):
         """1-D -> [w], 2-D -> [h][w], 3-D -> [c][h][w]; a batch adds a leading [n]."""
-        es = self.elemsize
-        dt = np.int8 if es == 1 else np.float32
-        d, w, h, c, n = self.dims, self.w, self.h, self.c, self.n
-        samples = []
-        for b in range(n):
-            base = lib().ncnn_mat_get_batch_data(self.h_, b)
-            if d == 1:
-                a = np.ctypeslib.as_array(C.cast(base, C.POINTER(C.c_uint8)), shape=(w * es,)).view(dt).copy()
-            elif d == 2:
-                a = np.ctypeslib.as_array(C.cast(base, C.POINTER(C.c_uint8)), shape=(w * h * es,)).view(dt).reshape(h, w).copy()
-            else:
-                buf = np.ctypeslib.as_array(C.cast(base, C.POINTER(C.c_uint8)), shape=(self.cstep * c * es,)).view(dt).reshape(c, self.cstep)
-                a = buf[:, : h * w].reshape(c, h, w).copy()
-            samples.append(a)
-        return np.stack(samples) if n > 1 else samples[0]
+        layout = (C.c_size_t * 9)()
+        lib().ncnnhip_mat_get_layout(self.h_, C.byref(layout))
+        dims, w, h, _, c, n, es, cstep, nstep = layout
+        shape, step = {1: ((w,), (es,)), 2: ((h, w), (w * es, es))}.get(dims, ((c, h, w), (cstep * es, w * es, es)))
+        if n > 1:
+            shape, step = (n,) + shape, (nstep * es,) + step
+        last = sum((s - 1) * t for s, t in zip(shape, step)) + es if 0 not in shape else 0
+        buf = (C.c_uint8 * max(last, es)).from_address(lib().ncnn_mat_get_data(self.h_)) if last else bytearray(es)
+        return np.ndarray(shape, np.int8 if es == 1 else np.float32, buf, 0, step).copy()
 
 
 # ---- Net / Extractor -------------------------------------------------------------------------------
@@ -326,7 +331,7 @@ class HipGraph:
             pass
 
     def update_input(self, array):
-        m = array if isinstance(array, Mat) else Mat.from_numpy(array)
+        m = array if isinstance(array, Mat) else Mat.view(array)
         ret = lib().ncnnhip_graph_update_input(self.h_, m.h_)
         if ret != 0:
             raise RuntimeError("update_input returned %d" % ret)
@@ -360,7 +365,7 @@ class Net:
 
     def upload(self, array):
         """numpy [c][h][w] / [n][c][h][w] -> device-resident blob usable as input of any extractor of this net."""
-        m = array if isinstance(array, Mat) else Mat.from_numpy(array)
+        m = array if isinstance(array, Mat) else Mat.view(array)
         out = C.c_void_p()
         ret = lib().ncnnhip_net_upload(self.h_, m.h_, C.byref(out))
         if ret != 0:
@@ -468,6 +473,12 @@ class Extractor:
         lib().ncnn_option_destroy(opt)
 
     def input(self, name, array):
+        if not isinstance(array, Mat):
+            # one copy, straight into the upload, when the blob goes to the device; else the Mat holds a copy of the values
+            index, text = (name, None) if isinstance(name, int) else (-1, name.encode())
+            view = Mat.view(array) if np.ndim(array) in (3, 4) else None
+            if view is not None and lib().ncnnhip_extractor_input_copied(self.h_, index, text, view.h_) == 0:
+                return 0
         m = array if isinstance(array, Mat) else Mat.from_numpy(array)
         self._inputs.append(m)
         if isinstance(name, int):  # a blob by number, the only way into a net loaded from the binary .param form in ncnn

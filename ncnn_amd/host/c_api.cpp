@@ -534,6 +534,24 @@ int ncnnhip_hipmat_download(const ncnn_hipmat_t m, ncnn_mat_t* out)
     *out = (ncnn_mat_t) new Mat(host);
     return ret;
 }
+ncnn_mat_t ncnnhip_mat_create_external_dense(int w, int h, int c, int n, void* data, size_t elemsize)
+{
+    Mat* m = new Mat(w, h, c, data, elemsize);
+    m->cstep = (size_t)w * h;
+    m->nstep = m->cstep * c;
+    m->n = n < 1 ? 1 : n;
+    return (ncnn_mat_t)m;
+}
+int ncnnhip_extractor_input_copied(ncnn_extractor_t ex, int index, const char* name, const ncnn_mat_t mat)
+{
+    return index < 0 ? E(ex)->input_copied(name, *M(mat)) : E(ex)->input_copied(index, *M(mat));
+}
+void ncnnhip_mat_get_layout(const ncnn_mat_t mat, size_t layout[9])
+{
+    const Mat& m = *M(mat);
+    const size_t v[9] = {(size_t)m.dims, (size_t)m.w, (size_t)m.h, (size_t)m.d, (size_t)m.c, (size_t)m.n, m.elemsize, m.cstep, m.nstep};
+    memcpy(layout, v, sizeof(v));
+}
 int ncnnhip_extractor_input_hipmat(ncnn_extractor_t ex, const char* name, const ncnn_hipmat_t m)
 {
     return E(ex)->input(name, *(const HipMat*)m);

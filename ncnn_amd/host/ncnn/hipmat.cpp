@@ -1,5 +1,10 @@
 #include "hipmat.h"
 
+#include <string.h>
+
+#include <algorithm>
+
+#include "hostcopy.h"
 #include "ncnnhip.h"
 
 namespace ncnn {
@@ -225,14 +230,61 @@ size_t HipPool::pooled_bytes() const
     return s;
 }
 
-HipCommand::HipCommand(bool blobs_cross_streams) : stream(0), ready(false), pool(new HipPool(blobs_cross_streams)), zero_ws(0), zero_ws_bytes(0) {}
+HipCommand::HipCommand(bool blobs_cross_streams)
+    : stream(0), ready(false), cross_streams(blobs_cross_streams), next_stage(0), pool(new HipPool(blobs_cross_streams)), zero_ws(0), zero_ws_bytes(0)
+{
+    for (int i = 0; i < STAGES; i++)
+    {
+        stages[i].data = 0;
+        stages[i].event = 0;
+        stages[i].pending = false;
+    }
+}
 
 HipCommand::~HipCommand()
 {
     // whatever was enqueued on this stream has finished before the stream goes; the buffers go with the pool's last owner
     if (ready) ncnnhip_stream_synchronize(stream);
     if (zero_ws) ncnnhip_free(zero_ws);
+    for (int i = 0; i < STAGES; i++)
+    {
+        if (stages[i].event) ncnnhip_event_destroy(stages[i].event);
+        if (stages[i].data) ncnnhip_host_free(stages[i].data);
+    }
     if (stream) ncnnhip_stream_destroy(stream);
+}
+
+// Chunks of an upload: 2 MB, so that the copy of one chunk into page-locked memory, the transfer of the one before and the
+// set-up of both overlap and little is exposed at either end.
+static const size_t STAGE_BYTES = (size_t)2 << 20;
+
+// the next staging buffer, free to be written by the host; 0 when there is none to be had (the caller then copies from
+// pageable memory)
+HipCommand::Stage* HipCommand::take_stage()
+{
+    Stage* s = &stages[next_stage];
+    if (!s->data)
+    {
+        void* p = 0;
+        if (!s->event && ncnnhip_event_create(&s->event) != 0)
+        {
+            s->event = 0;
+            return 0;
+        }
+        if (ncnnhip_host_malloc(&p, STAGE_BYTES) != 0 || !p) return 0;
+        s->data = (unsigned char*)p;
+        s->pending = false;
+    }
+    if (s->pending && ncnnhip_event_synchronize(s->event) != 0) return 0;
+    s->pending = false;
+    next_stage = (next_stage + 1) % STAGES;
+    return s;
+}
+
+int HipCommand::mark_stage(Stage* s)
+{
+    s->pending = true;
+    return ncnnhip_event_record(s->event, stream);
 }
 
 void* HipCommand::zeroed_workspace(size_t bytes)
@@ -333,27 +385,117 @@ int HipCommand::upload_into(const Mat& src, HipMat& dst)
         NCNN_LOGE("HipCommand::upload_into: the host blob does not have the device blob's shape and type");
         return -1;
     }
-    if (src.dims == 3)
+    const int rc = src.dims == 3 ? upload_planes(src, dst) : upload_samples(src, dst);
+    return hip_status(rc, "upload");
+}
+
+// Planar image(s) to channels-last: pieces of a few whole samples, or of a pixel range of one sample, are copied into a
+// staging buffer, and a layout kernel reads them there over PCIe and writes the device blob: one pass, no copy in device
+// memory, and the host prepares piece i + 1 while piece i is on its way.
+int HipCommand::upload_planes(const Mat& src, HipMat& dst)
+{
+    const int es = (int)src.elemsize;
+    const size_t hw = (size_t)src.w * src.h;
+    const size_t align = 16 / es;                                      // staged planes start on 16 bytes
+    const size_t sample_bytes = (hw + align - 1) / align * align * src.c * es;
+    const int per_piece = (int)std::min<size_t>((size_t)src.n, STAGE_BYTES / sample_bytes); // 0: a sample needs several pieces
+    const size_t most = per_piece ? hw : STAGE_BYTES / es / src.c / align * align;       // pixels of a piece
+    int rc = 0;
+    bool staged = most > 0;
+    for (int b = 0; staged && b < src.n && rc == 0; b += std::max(per_piece, 1))
     {
-        // planar bytes as they lie on the host, then one layout kernel
+        const int samples = std::min(std::max(per_piece, 1), src.n - b);
+        for (size_t p0 = 0; staged && p0 < hw && rc == 0; p0 += most)
+        {
+            const size_t len = std::min(most, hw - p0);
+            size_t cstep = (len + align - 1) / align * align, nstep = cstep * src.c;
+            Stage* s = take_stage();
+            if (!s)
+            {
+                staged = false;
+                break;
+            }
+            if (len == hw && src.nstep * samples * es <= STAGE_BYTES)
+            {
+                // whole samples: one run of memory, strides as they are
+                cstep = src.cstep;
+                nstep = src.n > 1 ? src.nstep : src.cstep * src.c;
+                const size_t run = (nstep * (samples - 1) + cstep * (src.c - 1) + hw) * es;
+                parallel_copy(s->data, (const unsigned char*)src.data + (size_t)b * nstep * es, run);
+            }
+            else
+            {
+                for (int i = 0; i < samples; i++)
+                    for (int q = 0; q < src.c; q++)
+                        memcpy(s->data + (i * nstep + q * cstep) * es, (const unsigned char*)src.data + ((size_t)(b + i) * src.nstep + q * src.cstep + p0) * es, len * es);
+            }
+            unsigned char* to = (unsigned char*)dst.data + ((size_t)b * hw + p0) * dst.cp * es;
+            if (dst.narrow())
+                rc = ncnnhip_chw_to_nhwc4_f32((const float*)s->data, src.c, (int)len, samples, cstep, nstep, (float*)to, stream);
+            else
+                rc = ncnnhip_chw_to_nhwc(s->data, es, src.c, (int)len, samples, cstep, nstep, to, stream);
+            const int mark = mark_stage(s);
+            if (rc == 0) rc = mark;
+        }
+    }
+    if (!staged && rc == 0)
+    {
+        // no page-locked memory: planar bytes as they lie on the host, then one layout kernel
         ScopedScratch scratch(this);
         void* staging = scratch.get(host_bytes(src));
-        if (!staging) return -100;
-        int rc = ncnnhip_memcpy_h2d(staging, src.data, host_bytes(src), stream);
+        if (!staging) return NCNNHIP_OOM;
+        rc = ncnnhip_memcpy_h2d(staging, src.data, host_bytes(src), stream);
         if (rc == 0 && dst.narrow())
             rc = ncnnhip_chw_to_nhwc4_f32((const float*)staging, src.c, src.w * src.h, src.n, src.cstep, src.nstep, (float*)dst.data, stream);
         else if (rc == 0)
-            rc = ncnnhip_chw_to_nhwc(staging, (int)src.elemsize, src.c, src.w * src.h, src.n, src.cstep, src.nstep, dst.data, stream);
+            rc = ncnnhip_chw_to_nhwc(staging, es, src.c, src.w * src.h, src.n, src.cstep, src.nstep, dst.data, stream);
         // the copy out of pageable host memory must have left the caller's buffer before we return
         if (rc == 0) rc = ncnnhip_stream_synchronize(stream);
-        return hip_status(rc, "upload");
+        return rc;
     }
+    // whoever reads the blob on another stream has nothing to wait on
+    if (rc == 0 && cross_streams) rc = ncnnhip_stream_synchronize(stream);
+    return rc;
+}
+
+// vectors and matrices: dense samples, nstep apart on the host
+int HipCommand::upload_samples(const Mat& src, HipMat& dst)
+{
     const size_t sample = (size_t)src.w * src.h * src.elemsize;
+    const size_t pitch = src.nstep * src.elemsize;
     int rc = 0;
-    for (int b = 0; b < src.n && rc == 0; b++)
-        rc = ncnnhip_memcpy_h2d((unsigned char*)dst.data + sample * b, (const unsigned char*)src.data + src.nstep * b * src.elemsize, sample, stream);
-    if (rc == 0) rc = ncnnhip_stream_synchronize(stream);
-    return hip_status(rc, "upload");
+    bool staged = true;
+    const size_t total = sample * src.n;
+    // one run of `total` bytes on the device, cut into staging buffers wherever they end
+    for (size_t at = 0; staged && at < total && rc == 0; at += STAGE_BYTES)
+    {
+        const size_t len = std::min(STAGE_BYTES, total - at);
+        Stage* s = take_stage();
+        if (!s)
+        {
+            staged = false;
+            break;
+        }
+        for (size_t done = 0; done < len;)
+        {
+            const size_t b = (at + done) / sample, o = (at + done) % sample;
+            const size_t run = std::min(sample - o, len - done);
+            parallel_copy(s->data + done, (const unsigned char*)src.data + b * pitch + o, run);
+            done += run;
+        }
+        rc = ncnnhip_copy((unsigned char*)dst.data + at, s->data, len, stream);
+        const int mark = mark_stage(s);
+        if (rc == 0) rc = mark;
+    }
+    if (!staged && rc == 0)
+    {
+        for (int b = 0; b < src.n && rc == 0; b++)
+            rc = ncnnhip_memcpy_h2d((unsigned char*)dst.data + sample * b, (const unsigned char*)src.data + pitch * b, sample, stream);
+        if (rc == 0) rc = ncnnhip_stream_synchronize(stream);
+        return rc;
+    }
+    if (rc == 0 && cross_streams) rc = ncnnhip_stream_synchronize(stream);
+    return rc;
 }
 
 int HipCommand::widen(const HipMat& src, HipMat& dst)
@@ -380,27 +522,47 @@ int HipCommand::download(const HipMat& blob, Mat& dst, Allocator* allocator)
         if (ret != 0) return ret;
     }
     if (src.dims == 3)
-    {
         dst.create(src.w, src.h, src.c, src.elemsize, 1, src.n, allocator);
-        if (dst.empty()) return -100;
-        ScopedScratch scratch(this);
-        void* staging = scratch.get(host_bytes(dst));
-        if (!staging) return -100;
-        int rc = ncnnhip_nhwc_to_chw(src.data, (int)src.elemsize, src.c, src.w * src.h, src.n, staging, dst.cstep, dst.nstep, stream);
-        if (rc == 0) rc = ncnnhip_memcpy_d2h(dst.data, staging, host_bytes(dst), stream);
-        if (rc == 0) rc = ncnnhip_stream_synchronize(stream);
-        return hip_status(rc, "download");
-    }
-    if (src.dims == 1)
+    else if (src.dims == 1)
         dst.create(src.w, src.elemsize, 1, src.n, allocator);
     else
         dst.create(src.w, src.h, src.elemsize, 1, src.n, allocator);
     if (dst.empty()) return -100;
     const size_t sample = (size_t)src.w * src.h * src.elemsize;
+    const size_t total = src.dims == 3 ? host_bytes(dst) : sample * src.n;
+    // What fits a staging buffer (the scores of a batch, a small feature map) leaves in one launch that writes page-locked
+    // memory over PCIe: a copy command out of the device costs about 20 us of set-up for each sample.
+    Stage* s = total <= STAGE_BYTES ? take_stage() : 0;
     int rc = 0;
-    for (int b = 0; b < src.n && rc == 0; b++)
-        rc = ncnnhip_memcpy_d2h((unsigned char*)dst.data + dst.nstep * b * dst.elemsize, (const unsigned char*)src.data + sample * b, sample, stream);
+    if (src.dims == 3)
+    {
+        ScopedScratch scratch(this);
+        void* staging = s ? s->data : scratch.get(total);
+        if (!staging) return -100;
+        rc = ncnnhip_nhwc_to_chw(src.data, (int)src.elemsize, src.c, src.w * src.h, src.n, staging, dst.cstep, dst.nstep, stream);
+        if (rc == 0 && !s) rc = ncnnhip_memcpy_d2h(dst.data, staging, total, stream);
+        if (rc == 0) rc = ncnnhip_stream_synchronize(stream);
+        if (rc == 0 && s)
+        {
+            // plane by plane: the padding between planes was not written
+            const size_t plane = sample;
+            for (int b = 0; b < src.n; b++)
+                for (int q = 0; q < src.c; q++)
+                {
+                    const size_t at = (b * dst.nstep + q * dst.cstep) * dst.elemsize;
+                    memcpy((unsigned char*)dst.data + at, s->data + at, plane);
+                }
+        }
+        return hip_status(rc, "download");
+    }
+    const size_t pitch = dst.nstep * dst.elemsize;
+    if (s)
+        rc = ncnnhip_copy(s->data, src.data, total, stream);
+    else
+        for (int b = 0; b < src.n && rc == 0; b++) rc = ncnnhip_memcpy_d2h((unsigned char*)dst.data + pitch * b, (const unsigned char*)src.data + sample * b, sample, stream);
     if (rc == 0) rc = ncnnhip_stream_synchronize(stream);
+    if (rc == 0 && s)
+        for (int b = 0; b < src.n; b++) memcpy((unsigned char*)dst.data + pitch * b, s->data + sample * b, sample);
     return hip_status(rc, "download");
 }
 

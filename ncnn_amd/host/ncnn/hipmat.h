@@ -131,7 +131,9 @@ public:
     // (the arrival counters of the K-split convolution); used by one kernel at a time, like everything on this stream
     void* zeroed_workspace(size_t bytes);
 
-    // host Mat (planar, any batch) -> device blob and back; download synchronises the stream
+    // Host Mat (planar, any batch) -> device blob and back.  An upload has left src's memory when it returns (it goes through
+    // page-locked staging buffers of this command); the device blob is ready in stream order, and for a command whose blobs
+    // cross streams when the call returns.  download synchronises the stream.
     int upload(const Mat& src, HipMat& dst);
     int upload_into(const Mat& src, HipMat& dst); // dst exists and has src's shape: new values for the same buffer
     int widen(const HipMat& src, HipMat& dst);    // narrow blob -> ordinary 16-channel-padded blob (enqueued, not waited for)
@@ -145,6 +147,25 @@ private:
     HipCommand& operator=(const HipCommand&);
     friend class HipMat;
     bool ready;
+    bool cross_streams; // blobs of this command are read on other streams
+    // Page-locked staging buffers, STAGE_BYTES each, made when first used and given back with the command.  A transfer takes
+    // them in turn; before one is filled again the event recorded behind its last use is waited for.
+    enum
+    {
+        STAGES = 3
+    };
+    struct Stage
+    {
+        unsigned char* data;
+        void* event;
+        bool pending; // work that reads or writes it may still be running
+    };
+    Stage stages[STAGES];
+    int next_stage;
+    Stage* take_stage();
+    int mark_stage(Stage* s);
+    int upload_planes(const Mat& src, HipMat& dst);
+    int upload_samples(const Mat& src, HipMat& dst);
     std::shared_ptr<HipPool> pool;
     void* zero_ws;
     size_t zero_ws_bytes;

@@ -1,0 +1,129 @@
+#include "hostcopy.h"
+
+#include <string.h>
+#include <unistd.h>
+
+#include <atomic>
+#include <condition_variable>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+namespace ncnn {
+
+namespace {
+
+// one core copies at about 24 GB/s, PCIe takes 56: four keep ahead of it with room for slow cores
+const int HELPERS = 3;
+const size_t PIECE = 256 * 1024;
+// a helper that has finished looks for the next chunk of the same upload for this many turns (about 100 us) before it sleeps
+const int SPINS = 2000;
+
+class CopyPool
+{
+public:
+    CopyPool() : owner(getpid()), generation(0), stop(false), open(false), next(0), active(0), dst(0), src(0), bytes(0)
+    {
+        const unsigned cores = std::thread::hardware_concurrency();
+        const int count = cores > (unsigned)HELPERS ? HELPERS : 0;
+        for (int i = 0; i < count; i++) threads.push_back(std::thread(&CopyPool::help, this));
+    }
+    ~CopyPool()
+    {
+        if (getpid() != owner) // a forked child has none of the threads
+        {
+            for (size_t i = 0; i < threads.size(); i++) threads[i].detach();
+            return;
+        }
+        {
+            std::lock_guard<std::mutex> g(lock);
+            stop = true;
+            generation.fetch_add(1);
+        }
+        wake.notify_all();
+        for (size_t i = 0; i < threads.size(); i++) threads[i].join();
+    }
+
+    bool copy(void* _dst, const void* _src, size_t _bytes)
+    {
+        if (threads.empty() || getpid() != owner || !user.try_lock()) return false;
+        {
+            std::lock_guard<std::mutex> g(lock);
+            dst = (unsigned char*)_dst;
+            src = (const unsigned char*)_src;
+            bytes = _bytes;
+            next.store(0);
+            open = true;
+            generation.fetch_add(1);
+        }
+        wake.notify_all();
+        work();
+        {
+            std::lock_guard<std::mutex> g(lock);
+            open = false; // a helper that wakes up only now has nothing to do here
+        }
+        while (active.load(std::memory_order_acquire) != 0) __builtin_ia32_pause();
+        user.unlock();
+        return true;
+    }
+
+private:
+    void work()
+    {
+        for (;;)
+        {
+            const size_t at = next.fetch_add(PIECE);
+            if (at >= bytes) return;
+            memcpy(dst + at, src + at, bytes - at < PIECE ? bytes - at : PIECE);
+        }
+    }
+    void help()
+    {
+        unsigned long long seen = 0;
+        for (;;)
+        {
+            for (int i = 0; i < SPINS && generation.load(std::memory_order_acquire) == seen; i++) __builtin_ia32_pause();
+            bool join;
+            {
+                std::unique_lock<std::mutex> g(lock);
+                while (generation.load() == seen) wake.wait(g);
+                seen = generation.load();
+                if (stop) return;
+                join = open;
+                if (join) active.fetch_add(1);
+            }
+            if (!join) continue;
+            work();
+            active.fetch_sub(1, std::memory_order_release);
+        }
+    }
+
+    std::vector<std::thread> threads;
+    const pid_t owner;
+    std::mutex user; // one copy at a time
+    std::mutex lock;
+    std::condition_variable wake;
+    std::atomic<unsigned long long> generation;
+    bool stop;
+    bool open; // the current job still takes helpers
+    std::atomic<size_t> next;
+    std::atomic<int> active; // helpers inside the current job
+    unsigned char* dst;
+    const unsigned char* src;
+    size_t bytes;
+};
+
+} // namespace
+
+void parallel_copy(void* dst, const void* src, size_t bytes)
+{
+    // below 1 MB (40 us) one thread is done before the others are awake
+    if (bytes >= 4 * PIECE)
+    {
+        static CopyPool pool;
+        if (pool.copy(dst, src, bytes)) return;
+    }
+    memcpy(dst, src, bytes);
+}
+
+} // namespace ncnn

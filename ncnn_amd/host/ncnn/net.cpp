@@ -1441,6 +1441,28 @@ int Extractor::input(int blob_index, const Mat& in)
     return 0;
 }
 
+int Extractor::input_copied(const char* blob_name, const Mat& in)
+{
+    const int bi = d->net->find_blob_index_by_name(blob_name);
+    if (bi < 0) return -1;
+    return input_copied(bi, in);
+}
+
+int Extractor::input_copied(int blob_index, const Mat& in)
+{
+    if (blob_index < 0 || blob_index >= (int)d->st.host.size()) return -1;
+    const int ci = d->net->d->blobs[(size_t)blob_index].consumer;
+    if (!d->opt.use_hip_compute || ci < 0) return 1;
+    const Layer* consumer = d->net->d->layers[(size_t)ci];
+    if (!consumer->support_hip || (consumer->featmask & (1 << 4))) return 1;
+    if (!d->st.cmd) d->st.cmd = d->net->d->acquire_command();
+    HipMat dev;
+    if (d->st.cmd->upload(in, dev) != 0) return 1;
+    d->st.dev[(size_t)blob_index] = dev;
+    d->st.host[(size_t)blob_index].release();
+    return 0;
+}
+
 int Extractor::input(const char* blob_name, const HipMat& in)
 {
     const int bi = d->net->find_blob_index_by_name(blob_name);
@@ -1671,7 +1693,8 @@ int HipGraph::record(const Net& net, const char* input_name, const HipMat& input
 int HipGraph::update_input(const Mat& src)
 {
     if (!d->exec) return -1;
-    return d->cmd->upload_into(src, d->input);
+    const int ret = d->cmd->upload_into(src, d->input);
+    return ret != 0 ? ret : d->cmd->synchronize(); // the blob may be read on other streams too
 }
 
 int HipGraph::launch()

@@ -91,6 +91,11 @@ public:
 
     int input(const char* blob_name, const Mat& in);
     int input(int blob_index, const Mat& in);
+    // Feeds a host blob whose memory the caller takes back on return: the upload to the device is started here (and overlaps
+    // whatever the host does until extract) instead of when the first layer runs.  1 when the blob's consumer does not run
+    // on the device or there was no memory for it: nothing was fed, use input().
+    int input_copied(const char* blob_name, const Mat& in);
+    int input_copied(int blob_index, const Mat& in);
     // type 0: int8 results are expanded to fp32; type 1: returned as stored
     int extract(const char* blob_name, Mat& feat, int type = 0);
     int extract(int blob_index, Mat& feat, int type = 0);
