@@ -32,19 +32,6 @@ struct ConvFusion
     float q8_scale;
 };
 
-// The same kernel as a plain Gemm (a 1x1 convolution whose "pixels" are the rows of A): Gemm's dequantising epilogue
-//   out = alpha * ((float)acc * (1/(sA_i*sB)) + beta*C)     or, one B scale per column,  ((float)acc * (1/sA_i)) * (1/sB_j)
-// (Gemm::forward_int8, src/layer/gemm.cpp:509-555) replaces the convolution's.
-struct GemmTail
-{
-    const float* a_scales; // [M]
-    const float* b_scales; // [1] or [N]
-    int per_col;
-    const float* c;
-    int bt; // -1 none, 0 scalar, 1/2 per row, 4 per column
-    float alpha, beta;
-};
-
 // Workspace contract of the channels-last convolutions: the first SPLIT_COUNTER_BYTES hold one arrival counter per
 // output tile of a K-split launch.  They must be zero when a call starts (the caller clears the workspace once, after
 // allocating it) and are zero again when it has finished; the rest is scratch without a contract.
@@ -81,11 +68,6 @@ bool conv_pointwise_stem_fits(const NhwcGeom& g, const ConvEpilogue& epi, const 
 bool conv_resident_fits(const NhwcGeom& g, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp);
 int launch_conv_resident(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream);
 int launch_conv_pointwise(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, int out_cp, hipStream_t stream);
-
-// D[M][N] = A[M][K] * B[N][K]^T through the pipelined kernel; handled = false when the shape does not fit it
-// (K % 64, N % 4, strides, alignment) and the caller should take another kernel.
-int launch_gemm_via_conv_pipelined(const int8_t* aq, size_t aq_stride, const int8_t* bq, size_t bq_stride, int M, int N, int K, const GemmTail& tail,
-                                   float* out, size_t out_stride, hipStream_t stream, bool* handled);
 
 // InnerProduct as a 1x1 convolution over the activation rows (rows = pixels, K = channels): same epilogue as the
 // convolution (scale_in, bias, activation), dense fp32 output with row stride out_stride.  handled = false when the

@@ -86,13 +86,12 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
         partial = (int32_t*)((char*)workspace + SPLIT_COUNTER_BYTES);
     }
     dim3 grid((unsigned)blocks), block(256);
-    const GemmTail no_gemm = {0, 0, 0, 0, -1, 1.f, 1.f};
     // addressing mode (the kernel's MODE); the K-split kernels exist for modes 0, 1 and 3 only (a narrow-input layer has
     // too few K steps to be split)
     const int mode = dense ? 1 : ((g.tapK == 16 || g.tapK == 32) && p.splits == 1) ? 2 : (g.tapK % 64 == 0 && g.tapK == g.Cp) ? 3 : 0;
     if (p.splits > 1) return launch_pipe_split(p, mode, wpk, x, g, epi, fusion, out_cp, out_cp, partial, counters, stream);
 #define LAUNCH_PIPE_MODE(BM_, BN_, MODE_)                                                                                                                \
-    hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<BM_, BN_, PIPE_RING, false, false, MODE_>), grid, block, 0, stream, wpk, x, g, epi, fusion, no_gemm, out_cp, \
+    hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<BM_, BN_, PIPE_RING, false, MODE_>), grid, block, 0, stream, wpk, x, g, epi, fusion, out_cp, \
                        out_cp, p.tiles_m, p.tiles_n, p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, (const float*)0, 0)
 #define LAUNCH_PIPE(BM_, BN_)                  \
     do                                         \
@@ -149,7 +148,6 @@ int launch_fc_via_conv_pipelined(const int8_t* x, size_t x_stride, int rows, int
     g.cout = num_output;
     g.pad_word = 0;
     const ConvFusion no_fusion = {0, 0, 0, 0.f};
-    const GemmTail no_gemm = {0, 0, 0, 0, -1, 1.f, 1.f};
     const PipePlan p = plan_pipelined(num_output, rows, K / 64);
     int32_t* partial = 0;
     unsigned* counters = 0;
@@ -168,7 +166,7 @@ int launch_fc_via_conv_pipelined(const int8_t* x, size_t x_stride, int rows, int
     }
     if (p.splits > 1) return launch_pipe_split(p, 1, weight, x, g, epi, no_fusion, (int)out_stride, num_output, partial, counters, stream);
 #define LAUNCH_FC(BN_)                                                                                                                                \
-    hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<64, BN_, PIPE_RING, false, false, 1>), grid, block, 0, stream, weight, x, g, epi, no_fusion, no_gemm, \
+    hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<64, BN_, PIPE_RING, false, 1>), grid, block, 0, stream, weight, x, g, epi, no_fusion, \
                        (int)out_stride, num_output, p.tiles_m, p.tiles_n, p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, (const float*)0, 0)
     if (p.bn == 256)
         LAUNCH_FC(256);

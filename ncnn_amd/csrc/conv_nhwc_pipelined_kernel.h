@@ -1,6 +1,6 @@
 // The pipelined channels-last convolution kernel and its launch plan, shared by the translation units that instantiate it
-// (conv_nhwc_pipelined.hip: one workgroup per tile; conv_nhwc_pipelined_split.hip: K split over workgroups, and the Gemm
-// form; conv_nhwc_pipelined_staged.hip: the quantising loader).  Splitting the instantiations over three files is for
+// (conv_nhwc_pipelined.hip: one workgroup per tile; conv_nhwc_pipelined_split.hip: K split over workgroups;
+// conv_nhwc_pipelined_staged.hip: the quantising loader).  Splitting the instantiations over three files is for
 // build time only.
 //
 // int8 Convolution (group 1, zero border) on channels-last blobs, pipelined for the gfx950 matrix cores.
@@ -59,7 +59,7 @@ __device__ __forceinline__ uint32_t pack4(const v4f& v)
 }
 
 // MODE: how a lane finds its source bytes.  0: any geometry; 1: dense (1x1, stride 1, unpadded: one row of npix pixels,
-// also Gemm and InnerProduct); 2: taps of 16 or 32 bytes (the narrow-input image), a whole number of taps per K step.
+// also InnerProduct); 2: taps of 16 or 32 bytes (the narrow-input image), a whole number of taps per K step.
 // 3: any geometry whose taps are whole 64-byte steps (tapK % 64 == 0): a K step then lies inside ONE tap, the same for every
 // lane, so the walk over taps is wavefront-uniform scalar arithmetic, and a lane's bounds test and address are computed
 // once per tap instead of once per step (a tap of 256 channels is four steps: the other three are a load and an add).
@@ -73,14 +73,14 @@ __device__ __forceinline__ uint32_t pack4(const v4f& v)
 // stage would have.  The weights of the tile (BN * K bytes) are requested in full before that and land in a region of
 // their own while the loader works, so the K loop touches LDS only: no waits on memory, no barriers.  x points at the
 // fp32 / fp16 blob, same channels-last geometry counted in values.
-template<int BM, int BN, int STAGES, bool SPLITK, bool GEMM, int MODE, int AIN = 1>
+template<int BM, int BN, int STAGES, bool SPLITK, int MODE, int AIN = 1>
 __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* __restrict__ wpk, const int8_t* __restrict__ x, NhwcGeom g, ConvEpilogue epi,
-                                                                   ConvFusion fusion, GemmTail gemm, int out_cp, int col_limit, int tiles_m, int tiles_n, int splits, int steps_per_split, unsigned magic_n, int32_t* __restrict__ partial, unsigned* __restrict__ counters,
+                                                                   ConvFusion fusion, int out_cp, int col_limit, int tiles_m, int tiles_n, int splits, int steps_per_split, unsigned magic_n, int32_t* __restrict__ partial, unsigned* __restrict__ counters,
                                                                    const float* __restrict__ a_scale, int a_cache_bytes)
 {
     constexpr bool dense = MODE == 1;
     constexpr bool STAGED = AIN != 1;
-    static_assert(!STAGED || (!GEMM && MODE != 2 && MODE != 3), "the quantising loader exists for convolutions on ordinary blobs");
+    static_assert(!STAGED || (MODE != 2 && MODE != 3), "the quantising loader exists for convolutions on ordinary blobs");
     constexpr int TM = BM / 64, TN = BN / 64; // 32x32 blocks per wavefront along pixels / channels
     constexpr int LAR = BM / 64;              // 64-row groups of the activation tile
     constexpr int LA = STAGED ? 0 : LAR, LB = BN / 64; // direct-to-LDS loads per wavefront per stage
@@ -335,7 +335,6 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
     // sum of its latencies).  Only the raw loads happen here, from clamped indices and always-valid pointers: a select
     // or a branch on the values would make the wavefront wait for them on the spot.
     float raw_s_in[BN / 64], raw_bias[BN / 64], raw_s_out[BN / 64];
-    if (!GEMM)
     {
         const float* bias_src = epi.bias ? epi.bias : epi.scale_in;
         const float* s_out_src = epi.scale_out ? epi.scale_out : epi.scale_in;
@@ -769,68 +768,11 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
     {
         const int ch = col0 + wn * CW + c * 32 + l32;
         real[c] = ch < g.cout; // channels from cout up to out_cp are the blob's zero padding
-        if (GEMM)
-        {
-            // s_in: 1/sB_j (one scale per column) ; bias: beta*C_j (C broadcast per column)
-            s_in[c] = (real[c] && gemm.per_col) ? div_rn(1.f, gemm.b_scales[ch]) : 0.f;
-            bias[c] = (real[c] && gemm.bt == 4) ? mul_rn(gemm.c[ch], gemm.beta) : 0.f;
-            s_out[c] = 0.f;
-        }
-        else
-        {
-            s_in[c] = real[c] ? raw_s_in[c] : 0.f;
-            // no bias: -0, the one value whose addition changes nothing (x + -0 = x for every x, -0 included)
-            bias[c] = (real[c] && epi.bias) ? raw_bias[c] : -0.f;
-            s_out[c] = (real[c] && to_int8) ? raw_s_out[c] : 0.f;
-        }
+        s_in[c] = real[c] ? raw_s_in[c] : 0.f;
+        // no bias: -0, the one value whose addition changes nothing (x + -0 = x for every x, -0 included)
+        bias[c] = (real[c] && epi.bias) ? raw_bias[c] : -0.f;
+        s_out[c] = (real[c] && to_int8) ? raw_s_out[c] : 0.f;
     }
-    if (GEMM)
-    {
-        const float sb0 = gemm.b_scales[0];
-        const float c0 = gemm.bt == 0 ? mul_rn(gemm.c[0], gemm.beta) : 0.f;
-#pragma unroll
-        for (int a = 0; a < TM; a++)
-        {
-#pragma unroll
-            for (int r = 0; r < 16; r++)
-            {
-                const int pl = 8 * (r >> 2) + 4 * lhi + (r & 3);
-                int row = row0 + wm * (BM / 2) + a * 32 + pl;
-                if (row >= g.npix) row = g.npix - 1; // rows beyond M are staged but never stored
-                const float sa = gemm.a_scales[row];
-                const float rowscale = gemm.per_col ? div_rn(1.f, sa) : div_rn(1.f, mul_rn(sa, sb0));
-                const float crow = (gemm.bt == 1 || gemm.bt == 2) ? mul_rn(gemm.c[row], gemm.beta) : 0.f;
-#pragma unroll
-                for (int c = 0; c < TN; c++)
-                {
-                    float f = mul_rn((float)acc[a][c][r], rowscale);
-                    if (gemm.per_col) f = mul_rn(f, s_in[c]);
-                    if (gemm.bt == 4)
-                        f = add_rn(f, bias[c]);
-                    else if (gemm.bt == 0)
-                        f = add_rn(f, c0);
-                    else if (gemm.bt >= 0)
-                        f = add_rn(f, crow);
-                    f = mul_rn(f, gemm.alpha);
-                    tile[pl * LD + c * 32 + l32] = f;
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int it = 0; it < G / 2; it++)
-            {
-                const int idx = it * 64 + lane;
-                const int p = idx / G, j = idx - p * G;
-                const v4f v = *reinterpret_cast<const v4f*>(tile + p * LD + 4 * j);
-                const int pix = row0 + wm * (BM / 2) + a * 32 + p;
-                const int ch4 = col0 + wn * CW + 4 * j;
-                if (pix < g.npix && ch4 < col_limit) *reinterpret_cast<v4f*>(static_cast<float*>(epi.out) + (size_t)pix * out_cp + ch4) = v;
-            }
-            if (a + 1 < TM) __syncthreads();
-        }
-        return;
-    }
-
     // the activation type is uniform: branch on it once, outside the unrolled loops
     auto finish = [&](auto act_tag) {
         constexpr int ACT = decltype(act_tag)::value;

@@ -80,17 +80,16 @@ int launch_conv_nhwc_staged(const NhwcGeom& g_in, const int8_t* wpk, const void*
         cache_bytes = (size_t)std::min<long long>(pixels * g.Cp, (long long)room) & ~(size_t)15;
     }
     dim3 grid((unsigned)(p.tiles_m * p.tiles_n * p.splits)), block(256);
-    const GemmTail no_gemm = {0, 0, 0, 0, -1, 1.f, 1.f};
     const int8_t* xb = static_cast<const int8_t*>(x);
 #define LAUNCH_STAGED(BN_, SPLIT_, MODE_, AIN_)                                                                                                              \
     do                                                                                                                                                       \
     {                                                                                                                                                        \
-        auto kernel = conv_nhwc_pipelined_kernel<64, BN_, PIPE_RING, SPLIT_, false, MODE_, AIN_>;                                                                    \
+        auto kernel = conv_nhwc_pipelined_kernel<64, BN_, PIPE_RING, SPLIT_, MODE_, AIN_>;                                                                    \
         static std::once_flag once;                                                                                                                          \
         static hipError_t attr = hipSuccess;                                                                                                                 \
         std::call_once(once, [&]() { attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)STAGED_LDS_LIMIT); });  \
         NCNNHIP_CHECK(attr);                                                                                                                                 \
-        hipLaunchKernelGGL(kernel, grid, block, tile_bytes + cache_bytes, stream, wpk, xb, g, epi, fusion, no_gemm, out_cp, out_cp, p.tiles_m, p.tiles_n, \
+        hipLaunchKernelGGL(kernel, grid, block, tile_bytes + cache_bytes, stream, wpk, xb, g, epi, fusion, out_cp, out_cp, p.tiles_m, p.tiles_n, \
                            p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, x_scale, (int)cache_bytes);                               \
     } while (0)
 #define LAUNCH_STAGED_IN(BN_, MODE_)                 \

@@ -1,21 +1,15 @@
-// int8 Gemm and InnerProduct launchers on top of the MFMA tile contraction.
+// int8 Gemm and InnerProduct: the few-row kernels, and which kernel a shape gets.
 #include "conv_nhwc.h"
 #include "epilogues.h"
+#include "gemm_int8_general.h"
 #include "mfma_tile.h"
 
 namespace ncnnhip {
 
-template<int BM, int BN, typename Epilogue>
-__global__ __launch_bounds__(256) void gemm_tile_kernel(DenseOperand a, DenseOperand b, Epilogue epi, int M, int N, int K)
-{
-    mfma_tile_body<BM, BN, DenseOperand, Epilogue>(a, b, epi, M, N, K, blockIdx.y * BM, blockIdx.x * BN);
-}
-
 // skinny case (up to a few dozen activation rows): one wavefront per output channel streams the weight row with
 // 16-byte loads, multiplies it against up to 8 activation rows at a time held in registers (v_dot4_i32_i8) and
 // reduces with cross-lane adds; no matrix cores involved.  The layer is bound by reading the weights once.
-// ROW_FIRST: the epilogue takes (activation row, output column, acc), as Gemm's does; else (output channel, row, acc)
-template<typename Epilogue, bool ROW_FIRST>
+template<typename Epilogue>
 __global__ __launch_bounds__(256) void fc_gemv_kernel(const int8_t* __restrict__ x, size_t xs, int rows, int K,
                                                        const int8_t* __restrict__ wgt, size_t ws, int num_output, Epilogue epi, int vec)
 {
@@ -61,13 +55,7 @@ __global__ __launch_bounds__(256) void fc_gemv_kernel(const int8_t* __restrict__
             int v = acc[r];
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-            if (lane == 0 && r < nr)
-            {
-                if (ROW_FIRST)
-                    epi(r0 + r, p, v);
-                else
-                    epi(p, r0 + r, v);
-            }
+            if (lane == 0 && r < nr) epi(p, r0 + r, v);
         }
     }
 }
@@ -76,8 +64,11 @@ __global__ __launch_bounds__(256) void fc_gemv_kernel(const int8_t* __restrict__
 // (v_mfma_i32_16x16x64_i8: the rows of B as one operand, the rows of A as the other, so a lane ends up with four consecutive
 // columns of one output row); eight steps of B and A are requested before the first product; the four partial tiles are
 // added through LDS.  B is read once; A (at most 16 x K bytes) comes from the cache.
+// ANY: rows that begin at any byte and K that is no multiple of 64: 16-byte loads at any address, and the wavefront whose turn
+// it would be multiplies what is left of K (K >= 16).
+// ROW_FIRST: the epilogue takes (activation row, output column, acc), as Gemm's does; else (output channel, row, acc)
 typedef int v4i_sk __attribute__((ext_vector_type(4)));
-template<typename Epilogue, bool ROW_FIRST>
+template<typename Epilogue, bool ROW_FIRST, bool ANY>
 __global__ __launch_bounds__(256) void gemm_skinny_int8_kernel(const int8_t* __restrict__ a, size_t as, int M_total, const int8_t* __restrict__ b, size_t bs, int N, int K,
                                                                 Epilogue epi)
 {
@@ -93,6 +84,16 @@ __global__ __launch_bounds__(256) void gemm_skinny_int8_kernel(const int8_t* __r
     const int8_t* ap = a + (size_t)arow * as + q * 16;
     const int ksteps = K >> 6;
     v4i_sk acc = {0, 0, 0, 0};
+    // what is left of K: a chunk that K ends in is cut out of the row's last 16 bytes
+    const bool tail = ANY && (K & 63) != 0 && (ksteps & 3) == wave;
+    const int tail_drop = ksteps * 64 + q * 16 + 16 - K;
+    v4i_sk tw = {0, 0, 0, 0}, tx = {0, 0, 0, 0};
+    if (tail)
+    {
+        const int k = tail_drop > 0 ? K - 16 - q * 16 : ksteps * 64;
+        tw = load16(bp + k);
+        tx = load16(ap + k);
+    }
     for (int k0 = wave; k0 < ksteps; k0 += 32) // this wavefront's steps k0, k0 + 4, ..., eight at a time
     {
         v4i_sk wv[8], xv[8];
@@ -101,12 +102,17 @@ __global__ __launch_bounds__(256) void gemm_skinny_int8_kernel(const int8_t* __r
         {
             const int ks = k0 + 4 * u;
             const int kk = ks < ksteps ? ks : k0; // past the end: a step that is there, its product dropped below
-            wv[u] = *reinterpret_cast<const v4i_sk*>(bp + (size_t)kk * 64);
-            xv[u] = *reinterpret_cast<const v4i_sk*>(ap + (size_t)kk * 64);
+            wv[u] = ANY ? load16(bp + (size_t)kk * 64) : *reinterpret_cast<const v4i_sk*>(bp + (size_t)kk * 64);
+            xv[u] = ANY ? load16(ap + (size_t)kk * 64) : *reinterpret_cast<const v4i_sk*>(ap + (size_t)kk * 64);
         }
 #pragma unroll
         for (int u = 0; u < 8; u++)
             if (k0 + 4 * u < ksteps) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wv[u], xv[u], acc, 0, 0, 0);
+    }
+    if (tail)
+    {
+        const int drop = tail_drop < 0 ? 0 : tail_drop > 16 ? 16 : tail_drop;
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(drop_bytes(tw, drop), drop_bytes(tx, drop), acc, 0, 0, 0);
     }
 #pragma unroll
     for (int r = 0; r < 4; r++) red[wave][lane][r] = acc[r];
@@ -132,29 +138,10 @@ __global__ __launch_bounds__(256) void gemm_skinny_int8_kernel(const int8_t* __r
 static bool launch_fc_skinny(const int8_t* x_dev, size_t x_stride, int rows, int num_input, int num_output, const int8_t* weight_dev, const FcEpilogue& epi,
                              hipStream_t stream);
 
-#ifndef GEMM_GEMV_MAX_ROWS
-#define GEMM_GEMV_MAX_ROWS 4
-#endif
-#ifndef GEMM_SKINNY_MIN_ROWS
-#define GEMM_SKINNY_MIN_ROWS 0
-#endif
-#ifndef GEMM_SKINNY_MAX_ROWS
-#define GEMM_SKINNY_MAX_ROWS 48
-#endif
+constexpr int GEMM_SKINNY_MAX_ROWS = 48;
 static inline bool aligned16(const void* p)
 {
     return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
-}
-
-static DenseOperand make_dense(const int8_t* base, size_t stride, int rows, int K)
-{
-    DenseOperand d;
-    d.base = base;
-    d.stride = stride;
-    d.rows = rows;
-    d.K = K;
-    d.vec = aligned16(base) && stride % 16 == 0;
-    return d;
 }
 
 int launch_gemm_int8_pipelined(const int8_t* aq, size_t aq_stride, const int8_t* bq, size_t bq_stride, int M, int N, int K,
@@ -179,7 +166,7 @@ static bool launch_fc_skinny(const int8_t* x_dev, size_t x_stride, int rows, int
     if (!fc_skinny_takes(rows, num_input, num_output)) return false;
     if (!aligned16(x_dev) || !aligned16(weight_dev) || x_stride % 16 != 0) return false;
     const int groups16 = (rows + 15) / 16;
-    hipLaunchKernelGGL((gemm_skinny_int8_kernel<FcEpilogue, false>), dim3(ceil_div(num_output, 16), groups16), dim3(256), 0, stream, x_dev, x_stride, rows, weight_dev,
+    hipLaunchKernelGGL((gemm_skinny_int8_kernel<FcEpilogue, false, false>), dim3(ceil_div(num_output, 16), groups16), dim3(256), 0, stream, x_dev, x_stride, rows, weight_dev,
                        (size_t)num_input, num_output, num_input, epi);
     return true;
 }
@@ -217,28 +204,19 @@ int ncnnhip_gemm_int8(const int8_t* aq_dev, size_t aq_stride, const int8_t* bq_d
     epi.N = N;
     epi.acc_out = acc_out_dev;
 
-    // up to four rows of A whose shape the matrix-core form above does not take (K % 64, unaligned rows): one wavefront per row
-    // of B with v_dot4.  Quantise + Gemm, one / four rows: 4096 x 4096 19.6 / 20.3 -> 9.2 / 12.3 us, 11008 x 4096
-    // 21.9 / 22.0 -> 16.9 / 23.3, 1024 x 1024 9.5 / 9.5 -> 7.0 / 8.1.  (Eight pieces of the weight row requested at once per
-    // lane instead of one were measured: no better at 4096 x 4096, worse on the other two.)
     // up to 16 rows of A, or up to 48 while reading B once per 16 rows (about 3 us + groups x bytes of B at 4 TB/s, from the cache
-    // after the first) stays below what the tiled kernels take for so few rows (about 4 us + K / 300): quantise + Gemm for
-    // 16 / 32 / 48 rows 4096 x 4096 20.6 / 21.2 / 21.4 -> 10.1 / 13.6 / 17.3 us, 11008 x 4096 22.1 -> 17.6 at 16 rows (beyond:
-    // tiled), 1024 x 1024 9.9 / 10.2 / 10.3 -> 7.2 / 7.5 / 7.3; one row 19.6 -> 8.7 / 21.9 -> 13.7 / 9.5 -> 7.5
+    // after the first) stays below what the general kernel takes for so few rows (about 4 us + K / 450): quantise + Gemm for
+    // 16 / 32 rows 4096 x 4096 10.1 / 13.6 us, 1024 x 1024 7.2 / 7.5; one row 8.7 / 7.5
     const int groups16 = (M + 15) / 16;
-    const bool skinny_pays = M <= 16 || 3.0 + groups16 * ((double)N * (double)K / 4.0e6) <= 4.0 + K / 300.0;
-    if (skinny_pays && M > GEMM_SKINNY_MIN_ROWS && M <= GEMM_SKINNY_MAX_ROWS && N >= 64 && K % 64 == 0 && aligned16(aq_dev) && aligned16(bq_dev) && aq_stride % 16 == 0 && bq_stride % 16 == 0)
+    const bool skinny_pays = M <= 16 || 3.0 + groups16 * ((double)N * (double)K / 4.0e6) <= 4.0 + K / 450.0;
+    if (skinny_pays && M <= GEMM_SKINNY_MAX_ROWS && N >= 64 && K >= 16)
     {
-        hipLaunchKernelGGL((gemm_skinny_int8_kernel<GemmEpilogue, true>), dim3(ceil_div(N, 16), ceil_div(M, 16)), dim3(256), 0, as_stream(stream), aq_dev, aq_stride, M, bq_dev, bq_stride, N, K,
-                           epi);
+        const dim3 grid(ceil_div(N, 16), ceil_div(M, 16));
+        if (K % 64 == 0 && aligned16(aq_dev) && aligned16(bq_dev) && aq_stride % 16 == 0 && bq_stride % 16 == 0)
+            hipLaunchKernelGGL((gemm_skinny_int8_kernel<GemmEpilogue, true, false>), grid, dim3(256), 0, as_stream(stream), aq_dev, aq_stride, M, bq_dev, bq_stride, N, K, epi);
+        else
+            hipLaunchKernelGGL((gemm_skinny_int8_kernel<GemmEpilogue, true, true>), grid, dim3(256), 0, as_stream(stream), aq_dev, aq_stride, M, bq_dev, bq_stride, N, K, epi);
         return launch_status("gemm_skinny_int8_kernel");
-    }
-    if (M <= GEMM_GEMV_MAX_ROWS && N >= 64)
-    {
-        const int vec = (aligned16(aq_dev) && aligned16(bq_dev) && aq_stride % 16 == 0 && bq_stride % 16 == 0) ? 1 : 0;
-        hipLaunchKernelGGL((fc_gemv_kernel<GemmEpilogue, true>), dim3(ceil_div(N, 4)), dim3(256), 0, as_stream(stream), aq_dev, aq_stride, M, K, bq_dev, bq_stride, N, epi,
-                           vec);
-        return launch_status("fc_gemv_kernel");
     }
     // big aligned problems: the 256x256 kernel (it needs a few hundred tiles to fill the chip)
     bool handled = false;
@@ -248,34 +226,14 @@ int ncnnhip_gemm_int8(const int8_t* aq_dev, size_t aq_stride, const int8_t* bq_d
         ret = launch_gemm_int8_pipelined(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, epi, as_stream(stream), &handled);
         if (handled) return ret;
     }
-    // too few 256x256 tiles for that: the same ring on 128x128 tiles, from 48 of them up (below, the 64-row tiles of the convolution
-    // kernel spread the work over more CUs)
+    // too few 256x256 tiles for that: the same ring on 128x128 tiles, from 48 of them up (below, the general kernel's 64-row tiles
+    // spread the work over more CUs)
     if ((long long)(M / 128) * (N / 128) >= 48)
     {
         ret = launch_gemm_int8_ring128(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, epi, as_stream(stream), &handled);
         if (handled) return ret;
     }
-    // anything else with K % 64 == 0: the convolution's pipelined kernel run as a 1x1 convolution over the rows of A
-    if (!output_transpose && !acc_out_dev)
-    {
-        GemmTail tail;
-        tail.a_scales = a_scales_dev;
-        tail.b_scales = b_scales_dev;
-        tail.per_col = epi.per_col;
-        tail.c = c_dev;
-        tail.bt = epi.bt;
-        tail.alpha = alpha;
-        tail.beta = beta;
-        ret = launch_gemm_via_conv_pipelined(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, tail, out_dev, out_stride, as_stream(stream), &handled);
-        if (handled) return ret;
-    }
-
-    DenseOperand a = make_dense(aq_dev, aq_stride, M, K);
-    DenseOperand b = make_dense(bq_dev, bq_stride, N, K);
-    dim3 grid(ceil_div(N, 128), ceil_div(M, 128));
-    NCNNHIP_REQUIRE(grid.y <= 65535, "ncnnhip_gemm_int8: M too large");
-    hipLaunchKernelGGL((gemm_tile_kernel<128, 128, GemmEpilogue>), grid, dim3(256), 0, as_stream(stream), a, b, epi, M, N, K);
-    return launch_status("gemm_tile_kernel");
+    return launch_gemm_int8_general(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, epi, as_stream(stream));
 }
 
 int ncnnhip_innerproduct_int8(const int8_t* x_dev, size_t x_stride, int rows, int num_input, int num_output,
@@ -299,17 +257,12 @@ int ncnnhip_innerproduct_int8(const int8_t* x_dev, size_t x_stride, int rows, in
     if (rows <= 64)
     {
         const int vec = aligned16(x_dev) && aligned16(weight_dev) && x_stride % 16 == 0 && num_input % 16 == 0;
-        hipLaunchKernelGGL((fc_gemv_kernel<FcEpilogue, false>), dim3(ceil_div(num_output, 4)), dim3(256), 0, as_stream(stream), x_dev, x_stride, rows,
+        hipLaunchKernelGGL((fc_gemv_kernel<FcEpilogue>), dim3(ceil_div(num_output, 4)), dim3(256), 0, as_stream(stream), x_dev, x_stride, rows,
                            num_input, weight_dev, (size_t)num_input, num_output, epi, vec);
         return launch_status("fc_gemv_kernel");
     }
 
-    DenseOperand a = make_dense(weight_dev, (size_t)num_input, num_output, num_input);
-    DenseOperand b = make_dense(x_dev, x_stride, rows, num_input);
-    dim3 grid(ceil_div(rows, 64), ceil_div(num_output, 128));
-    NCNNHIP_REQUIRE(grid.y <= 65535, "ncnnhip_innerproduct_int8: num_output too large");
-    hipLaunchKernelGGL((gemm_tile_kernel<128, 64, FcEpilogue>), grid, dim3(256), 0, as_stream(stream), a, b, epi, num_output, rows, num_input);
-    return launch_status("gemm_tile_kernel<fc>");
+    return launch_fc_int8_general(x_dev, x_stride, weight_dev, (size_t)num_input, rows, num_output, num_input, epi, as_stream(stream));
 }
 
 int ncnnhip_innerproduct_workspace_bytes(int rows, int num_input, int num_output, size_t* workspace_bytes)

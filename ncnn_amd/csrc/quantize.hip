@@ -92,12 +92,14 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(const float*
     }
 }
 
-// Rows of up to 8192 aligned floats: the row is read ONCE into registers (NV float4 per thread), reduced, and quantised
+// Rows of up to 8192 floats: the row is read ONCE into registers (NV float4 per thread), reduced, and quantised
 // from the registers -- 5 bytes of traffic per element instead of 9.
 // NT: the fp32 source is larger than the chip's last-level cache can hold on to, so it is read with non-temporal loads and
 // leaves the cache to the int8 rows the Gemm is about to read (8192 x 8192: 88 -> 57 us; smaller sources are re-read from
 // the cache by the next pass over the same buffer and lose 1 us this way).
-template<int NV, bool NT>
+// ANY: rows that begin on any float and end anywhere: the same loads and stores at the address there is, the last 1 to 3 values one
+// by one (4000 x 4033: 27 us with the two-sweep kernel).
+template<int NV, bool NT, bool ANY>
 __global__ __launch_bounds__(256) void quantize_rows_dynamic_reg_kernel(const float* __restrict__ a, size_t as, int cols,
                                                                          int8_t* __restrict__ aq, size_t aqs, float* __restrict__ scales, int tiled)
 {
@@ -107,7 +109,9 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_reg_kernel(const fl
     // tiled: the 256x256 Gemm kernel's operand layout, [r / 256][k / 64][r % 256][k % 64]; word i of the row (bytes 4i .. 4i+3)
     // is word i % 16 of K step i / 16
     uint32_t* qr = tiled ? reinterpret_cast<uint32_t*>(aq + ((size_t)(r >> 8) * (cols >> 6) * 256 + (r & 255)) * 64) : reinterpret_cast<uint32_t*>(aq + (size_t)r * aqs);
-    const int n4 = cols >> 2; // cols % 4 == 0 here
+    const int n4 = cols >> 2, rest = ANY ? cols & 3 : 0;
+    typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+    typedef uint32_t u32_any __attribute__((aligned(1)));
     float4 v[NV];
     float m = 0.f;
 #pragma unroll
@@ -120,6 +124,22 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_reg_kernel(const fl
             const v4f_nt t = i < n4 ? __builtin_nontemporal_load(reinterpret_cast<const v4f_nt*>(ar) + i) : v4f_nt{0.f, 0.f, 0.f, 0.f};
             v[j] = float4{t[0], t[1], t[2], t[3]};
         }
+        else if (ANY)
+        {
+            v[j] = float4{0.f, 0.f, 0.f, 0.f};
+            const float* row = reinterpret_cast<const float*>(ar);
+            if (i < n4)
+            {
+                const v4f_any t = *reinterpret_cast<const v4f_any*>(row + (size_t)i * 4);
+                v[j] = float4{t[0], t[1], t[2], t[3]};
+            }
+            else if (i == n4)
+            {
+                if (rest > 0) v[j].x = row[(size_t)i * 4];
+                if (rest > 1) v[j].y = row[(size_t)i * 4 + 1];
+                if (rest > 2) v[j].z = row[(size_t)i * 4 + 2];
+            }
+        }
         else
             v[j] = i < n4 ? ar[i] : float4{0.f, 0.f, 0.f, 0.f};
         m = fmaxf(m, fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
@@ -131,10 +151,19 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_reg_kernel(const fl
     for (int j = 0; j < NV; j++)
     {
         const int i = threadIdx.x + j * 256;
-        if (i < n4)
+        if (i < n4 || (ANY && i == n4 && rest))
         {
             const uint32_t q4 = pack4((int)float2int8_as_float(mul_rn(v[j].x, s)), (int)float2int8_as_float(mul_rn(v[j].y, s)),
                                       (int)float2int8_as_float(mul_rn(v[j].z, s)), (int)float2int8_as_float(mul_rn(v[j].w, s)));
+            if (ANY)
+            {
+                int8_t* to = aq + (size_t)r * aqs + (size_t)i * 4;
+                if (i < n4)
+                    *reinterpret_cast<u32_any*>(to) = q4;
+                else
+                    for (int e = 0; e < rest; e++) to[e] = (int8_t)(q4 >> (8 * e));
+                continue;
+            }
             uint32_t* dst = qr + (tiled ? (size_t)(i >> 4) * 4096 + (i & 15) : (size_t)i);
             *dst = q4;
         }
@@ -241,19 +270,23 @@ static int quantize_rows_impl(const float* a_dev, size_t a_stride, int rows, int
 {
     const bool vec = aligned(a_dev, 16) && aligned(aq_dev, 4) && a_stride % 4 == 0 && aq_stride % 4 == 0;
     NCNNHIP_REQUIRE(!tiled || (vec && cols <= 8192), "ncnnhip_gemm_quantize_rows_tiled: needs 16-byte aligned rows of at most 8192 values");
-    if (vec && cols % 4 == 0 && cols <= 8192)
+    if (cols <= 8192)
     {
         const int nv = ceil_div(cols, 1024);
-        const bool nt = (size_t)rows * cols * sizeof(float) > ((size_t)128 << 20);
-#define LAUNCH_REG(NV_)                                                                                                                          \
-    do                                                                                                                                           \
-    {                                                                                                                                            \
-        if (nt)                                                                                                                                  \
-            hipLaunchKernelGGL((quantize_rows_dynamic_reg_kernel<NV_, true>), dim3(rows), dim3(256), 0, as_stream(stream), a_dev, a_stride, cols, \
-                               aq_dev, aq_stride, scales_dev, tiled);                                                                            \
-        else                                                                                                                                     \
-            hipLaunchKernelGGL((quantize_rows_dynamic_reg_kernel<NV_, false>), dim3(rows), dim3(256), 0, as_stream(stream), a_dev, a_stride,     \
-                               cols, aq_dev, aq_stride, scales_dev, tiled);                                                                      \
+        const bool any = !vec || cols % 4 != 0;
+        const bool nt = !any && (size_t)rows * cols * sizeof(float) > ((size_t)128 << 20);
+#define LAUNCH_REG_AS(NV_, NT_, ANY_)                                                                                                            \
+    hipLaunchKernelGGL((quantize_rows_dynamic_reg_kernel<NV_, NT_, ANY_>), dim3(rows), dim3(256), 0, as_stream(stream), a_dev, a_stride, cols,    \
+                       aq_dev, aq_stride, scales_dev, tiled)
+#define LAUNCH_REG(NV_)                         \
+    do                                          \
+    {                                           \
+        if (any)                                \
+            LAUNCH_REG_AS(NV_, false, true);    \
+        else if (nt)                            \
+            LAUNCH_REG_AS(NV_, true, false);    \
+        else                                    \
+            LAUNCH_REG_AS(NV_, false, false);   \
     } while (0)
         if (nv <= 1)
             LAUNCH_REG(1);
@@ -264,6 +297,7 @@ static int quantize_rows_impl(const float* a_dev, size_t a_stride, int rows, int
         else
             LAUNCH_REG(8);
 #undef LAUNCH_REG
+#undef LAUNCH_REG_AS
     }
     else if (vec)
         hipLaunchKernelGGL(quantize_rows_dynamic_kernel<true>, dim3(rows), dim3(256), 0, as_stream(stream), a_dev, a_stride, cols, aq_dev, aq_stride, scales_dev);

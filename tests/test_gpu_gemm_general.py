@@ -1,0 +1,41 @@
+"""The int8 Gemm on rows that begin and end at any byte, at the edges of its tiles, K steps and dispatch: against the oracle, bit for
+bit (src/layer/gemm.cpp:745-966)."""
+import numpy as np
+import pytest
+
+from oracle import oracle
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def rt():
+    import ncnn_amd
+    return ncnn_amd.Runtime(0)
+
+
+SHAPES = [
+    # K: below a vector, one vector, around the few-row kernel's 64 and the tiles' 128 bytes, several steps with every kind of rest
+    (65, 63, 15), (17, 64, 16), (63, 65, 17), (64, 129, 63), (129, 64, 65), (127, 128, 127), (128, 127, 128), (66, 70, 129), (130, 66, 143), (70, 70, 271), (64, 64, 400),
+    # few rows (one workgroup per 16 rows of B), with K of 0 and more whole 64-byte steps
+    (1, 64, 16), (3, 65, 63), (16, 79, 65), (17, 100, 321), (2, 63, 77), (1, 130, 2047),
+    # two groups of wavefronts per tile from K = 3072, one K step more or less than the other's
+    (70, 65, 3072), (130, 65, 3073), (65, 66, 3200), (64, 64, 3327),
+    # 128 x 128 tiles from 1536 tiles of 64 x 64
+    (2497, 2497, 33), (1, 5000, 50), (3000, 2176, 130),
+]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_gemm_int8_any_shape_equals_the_oracle(rt, m, n, k):
+    print("[case]", m, n, k, flush=True)
+    a, bq, sb, bias = cases.gemm_case(m + n + k, m, n, k, per_col=k % 2 == 0)
+    aq, sa = rt.gemm_quantize_rows(a)
+    want_q, want_s = oracle.gemm_quantize_rows(a)
+    assert np.array_equal(aq, want_q) and np.array_equal(sa, want_s)
+    want, wacc = oracle.gemm_int8(aq, bq, sa, sb, bias, 4, 0.5, 1.5, False, want_acc=True)
+    assert np.array_equal(rt.gemm_int8(aq, bq, sa, sb, bias, 4, 0.5, 1.5), want)
+    # the general form of the epilogue: accumulators too, the output transposed
+    got, acc = rt.gemm_int8(aq, bq, sa, sb, bias, 4, 0.5, 1.5, output_transpose=True, want_acc=True)
+    assert np.array_equal(acc, wacc) and np.array_equal(got.T, want)
