@@ -1,0 +1,47 @@
+"""Block-quantised Gemm on more than 16 fp16 activation rows: groups of 16 rows, tiles of 16 weight rows and the K steps of 64 at
+their edges, every packed layout, alone and with several matrices in one call: against the oracle and a float64 value."""
+import numpy as np
+import pytest
+
+from ncnn_amd import synth
+from oracle import oracle
+from tests import npref
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+
+@pytest.fixture(scope="module")
+def rt():
+    import ncnn_amd
+    return ncnn_amd.Runtime(0)
+
+
+def _check(got, a, packed, scales, bits, block, c=None, bt=-1, alpha=1.0, beta=1.0):
+    # every product q * a is exact; what differs from the references is the order of the fp32 additions (see the random walk)
+    val, floor = npref.blockquant_gemm_f64(a, packed, scales, bits, block, None, c, bt, alpha, beta)
+    ref = oracle.gemm_blockquant(a, packed, scales, bits, block, None, c, bt, alpha, beta)
+    tol = 1e-5 * floor + 1e-30
+    assert np.all(np.abs(got - ref) <= tol) and np.all(np.abs(got - val) <= tol)
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 15, 16), (32, 16, 64), (33, 17, 80), (48, 200, 512), (49, 65, 576), (64, 130, 1040), (65, 33, 192), (130, 96, 128), (18, 4200, 256)])
+@pytest.mark.parametrize("bits,block", [(8, 64), (8, 32), (6, 128), (6, 32), (4, 64), (4, 32)])
+def test_many_fp16_rows(rt, m, n, k, bits, block):
+    print("[case]", m, n, k, bits, block, flush=True)
+    a, packed, scales = synth.blockquant_operands(m + n + k, m, n, k, bits, block)
+    c = np.random.default_rng(n).normal(size=(1, n)).astype(F)
+    pw, pd = rt.blockquant_pack(packed, scales, block, bits=bits, k=k)
+    got = rt.gemm_blockquant_packed(a.astype(np.float16), pw, pd, n, c, 4, 0.75, 1.5, bits=bits, block=block)
+    _check(got, a, packed, scales, bits, block, c, 4, 0.75, 1.5)
+
+
+@pytest.mark.parametrize("m", [17, 40, 100])
+def test_several_matrices_in_one_call(rt, m):
+    k, ns = 192, (50, 16, 700)
+    ops = [synth.blockquant_operands(10 + i, m, n, k, 4, 64) for i, n in enumerate(ns)]
+    a = ops[0][0]
+    mats = [rt.blockquant_pack(p, s, 64, bits=4, k=k) + (n, None, -1, 1.0, 1.0) for (_, p, s), n in zip(ops, ns)]
+    outs = rt.gemm_blockquant_packed_multi(a.astype(np.float16), mats, bits=4, block=64)
+    for (_, p, s), got in zip(ops, outs):
+        _check(got, a, p, s, 4, 64)
