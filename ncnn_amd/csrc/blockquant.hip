@@ -2016,6 +2016,24 @@ int ncnnhip_blockquant_pack(const uint8_t* b_host, const float* scales_host, int
     return NCNNHIP_OK;
 }
 
+// fp16 rows: which of the two forms takes M rows of N x K weights (N: of all matrices of the launch).  The one-pass kernel holds a
+// workgroup's whole share of K in registers: the shortest start, nothing shared between tiles.  The many-row kernel reads the
+// activations once for up to six tiles.  Measured over N 2048 to 27648, K 1024 to 13824, 5 to 16 rows, us one-pass / many-row:
+// unpacked fields (4 and 6 bits) cross at 20 M weights -- 4352 x 4096 8.3 / 8.7, 5120 x 5120 10.8 / 10.2, 22016 x 4096 23.6 /
+// 17.7 --, 8 bits where the activations weigh too: in blocks of 32 11008 x 4096 5 rows 11.4 / 12.7, 16 rows 14.5 / 13.5, 22016 x
+// 4096 5 rows 24.2 / 20.9; in longer ones 12288 x 4096 12 rows 13.1 / 13.3, 16 rows 14.3 / 13.5.  Beyond K = 8192 the one-pass
+// kernel has no room for more than 4 rows (5120 x 13824 4 bits 16 rows 71.5 / 18.5); 8 bits in longer blocks then run
+// blockquant8_mfma_kernel, better for small weights (4096 x 11008 8 rows 12.3 / 14.8, 5120 x 13824 24.0 / 19.9).
+static bool many_rows_f16(int M, long long N, int K, int bits, int block)
+{
+    if (M <= 4) return false;
+    if (M > 16) return true;
+    const long long weights = N * K;
+    if (bits != 8) return K > 8192 || weights > 20000000;
+    if (halves_layout(bits, block)) return K > 8192 || weights * M > 450000000;
+    return weights * M > 750000000 || (K > 8192 && weights > 64000000);
+}
+
 // shared body of the two packed entry points; ain = 2 (fp16 activations) or 4 (fp32)
 static int gemm_blockquant_packed(const char* who, const void* a_dev, int ain, size_t a_stride, int M, int N, int K, const uint8_t* packed_w_dev,
                                   const float* packed_descale_dev, int bits, int block, const float* in_scales_dev, const float* c_dev, int broadcast_type_c,
@@ -2037,7 +2055,7 @@ static int gemm_blockquant_packed(const char* who, const void* a_dev, int ain, s
     const float4* dpk = reinterpret_cast<const float4*>(packed_descale_dev);
     const int split = block == 32 ? 1 : 0;
     hipStream_t st = as_stream(stream);
-    if (ain == 2 && M > 16)
+    if (ain == 2 && many_rows_f16(M, N, K, bits, block))
     {
         BqMulti one;
         memset(&one, 0, sizeof(one));
@@ -2297,8 +2315,7 @@ int ncnnhip_gemm_blockquant_packed_multi(const void* a_dev, int a_elemsize, size
                                       broadcast_type_c ? broadcast_type_c[i] : -1, alpha ? alpha[i] : 1.f, beta ? beta[i] : 1.f, out_dev[i], out_stride[i], stream);
     };
     const bool halves = halves_layout(bits, block);
-    const bool many_rows = a_elemsize == 2 && M > 16; // fp16 rows beyond the one-pass kernel's: the many-row kernel takes all matrices at once too
-    bool one_pass = count > 1 && M >= 1 && K >= 1 && K % 16 == 0 && K <= 16384 && (many_rows || M <= (a_elemsize == 2 ? 16 : 4)) && (bits == 4 || bits == 6 || bits == 8) &&
+    bool one_pass = count > 1 && M >= 1 && K >= 1 && K % 16 == 0 && K <= 16384 && (a_elemsize == 2 || M <= 4) && (bits == 4 || bits == 6 || bits == 8) &&
                     (block == 32 || block == 64 || block == 128) && a_stride >= (size_t)K && a_stride % (16 / a_elemsize) == 0 && al16(a_dev) &&
                     (!in_scales_dev || al16(in_scales_dev));
     BqMulti mm;
@@ -2326,7 +2343,7 @@ int ncnnhip_gemm_blockquant_packed_multi(const void* a_dev, int a_elemsize, size
         mm.tile_end[i] = (int)tiles, mm.N[i] = 0, mm.bt[i] = -1, mm.alpha[i] = mm.beta[i] = 1.f;
         mm.wpk[i] = 0, mm.dpk[i] = 0, mm.c[i] = 0, mm.out[i] = 0, mm.out_stride[i] = 0;
     }
-    if (one_pass && many_rows) return launch_blockquant_rows_f16(static_cast<const uint16_t*>(a_dev), a_stride, M, K, bits, block, mm, as_stream(stream));
+    if (one_pass && a_elemsize == 2 && many_rows_f16(M, tiles * 16, K, bits, block)) return launch_blockquant_rows_f16(static_cast<const uint16_t*>(a_dev), a_stride, M, K, bits, block, mm, as_stream(stream));
     if (one_pass)
     {
         const int split = block == 32 ? 1 : 0;

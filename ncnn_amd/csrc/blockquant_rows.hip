@@ -1,4 +1,4 @@
-// Block-quantised Gemm on 17 fp16 activation rows and more: every weight is read once for up to 64 rows.
+// Block-quantised Gemm on many fp16 activation rows (from 5, by weights: many_rows_f16): every weight is read once for up to 64 rows.
 //
 // The few-row kernels (blockquant.hip) multiply 16 rows per pass over the weights; 48 rows were three passes of a launch each.
 // Here a workgroup owns RT tiles of 16 weight rows and MG groups of 16 activation rows and deals the K steps of 64 out to its

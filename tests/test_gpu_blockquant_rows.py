@@ -1,4 +1,4 @@
-"""Block-quantised Gemm on more than 16 fp16 activation rows: groups of 16 rows, tiles of 16 weight rows and the K steps of 64 at
+"""Block-quantised Gemm on many fp16 activation rows: groups of 16 rows, tiles of 16 weight rows and the K steps of 64 at
 their edges, every packed layout, alone and with several matrices in one call: against the oracle and a float64 value."""
 import numpy as np
 import pytest
@@ -34,6 +34,11 @@ def test_many_fp16_rows(rt, m, n, k, bits, block):
     pw, pd = rt.blockquant_pack(packed, scales, block, bits=bits, k=k)
     got = rt.gemm_blockquant_packed(a.astype(np.float16), pw, pd, n, c, 4, 0.75, 1.5, bits=bits, block=block)
     _check(got, a, packed, scales, bits, block, c, 4, 0.75, 1.5)
+
+
+@pytest.mark.parametrize("m,n,k,bits,block", [(5, 40, 8208, 4, 64), (13, 33, 9216, 6, 32), (16, 20, 8704, 8, 32), (5, 19600, 1024, 4, 128), (7, 7000, 9200, 8, 64)])
+def test_few_fp16_rows_of_large_weights(rt, m, n, k, bits, block):
+    test_many_fp16_rows(rt, m, n, k, bits, block)
 
 
 @pytest.mark.parametrize("m", [17, 40, 100])
