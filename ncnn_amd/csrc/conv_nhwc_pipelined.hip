@@ -10,6 +10,7 @@ constexpr int SPLIT_MIN_STEPS = 12;
 PipePlan plan_pipelined(int cout, long long npix, int steps)
 {
     PipePlan p;
+    p.groups = 1;
     // channel tile: the width that pads the channel count least (padded channels cost matrix-core time and unbalance the
     // wavefronts' epilogues: 144 channels in one 256-wide tile ran 34 us, in three 64-wide tiles 21), the wider on a tie
     p.bn = 64;
@@ -45,6 +46,30 @@ PipePlan plan_pipelined(int cout, long long npix, int steps)
     return p;
 }
 
+PipePlan plan_pipelined_groups(int cout, long long npix, int steps)
+{
+    PipePlan p = plan_pipelined(cout, npix, steps);
+    const long long t = (long long)p.tiles_m * p.tiles_n;
+    // With no more tiles than compute units a 64 x 64 tile has a unit to itself, and four wavefronts there wait for each K
+    // step's loads in turn; sixteen have four steps under way.  us, four wavefronts -> sixteen, one layer alone:
+    //   1x1 1024 -> 256 on 14x14: batch 1 6.3 -> 5.6, batch 16 6.5 -> 5.9    1x1 2048 -> 512 on 7x7: 8.2 -> 7.2, batch 16 9.3 -> 7.4
+    //   1x1 960 -> 160 on 7x7 6.0 -> 5.2    3x3 256 -> 256 on 14x14, batch 16 11.4 -> 8.7    3x3 512 -> 512 on 7x7, batch 16 12.7 -> 11.5
+    // Eight wavefronts gain about half of that.  392 tiles (3x3 128 -> 128 on 28x28, batch 16) share units already: the pass was
+    // 2 % slower with sixteen.  Below 8 steps there is too little to share.
+    if (p.bm != 64 || p.bn != 64 || steps < 8 || t > 256) return p;
+    // A few tiles of a long K want other compute units more than wavefronts of their own: 3x3 256 -> 256 on 14x14, batch 1
+    // (16 tiles) 8.1 in three splits and 8.5 in one with sixteen wavefronts, 512 -> 512 on 7x7 (8 tiles) 9.4 and 9.6.
+    if (p.splits >= 3 && t < 24) return p;
+    p.groups = 4;
+    // K is split over workgroups as well while they fit the chip, at least 24 steps each: 512 -> 512 on 7x7, batch 4 (32 tiles)
+    // 11.0 in six splits of four wavefronts, 10.1 in three of sixteen, 10.8 in four
+    const int room = (int)(256 / t), longest = steps / 24;
+    p.splits = std::max(1, std::min(p.splits, std::min(room, longest)));
+    p.steps_per_split = ceil_div(steps, p.splits);
+    p.splits = ceil_div(steps, p.steps_per_split);
+    return p;
+}
+
 size_t conv_nhwc_pipelined_workspace_words(int cout, long long npix, int steps)
 {
     const PipePlan p = plan_pipelined(cout, npix, steps);
@@ -66,7 +91,7 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
         g.H = g.outh = 1;
         g.W = g.outw = g.npix;
     }
-    PipePlan p = plan_pipelined(g.cout, g.npix, g.K / 64);
+    PipePlan p = plan_pipelined_groups(g.cout, g.npix, g.K / 64);
     // the narrow-input first layer has four K steps at most: from a million output pixels up, 128-pixel tiles halve the number of
     // workgroup prologues (ResNet-50's 7 x 7 first layer at batch 128: the pass 2.22 -> 2.20 ms; at batch 16, 0.2 M pixels, no gain)
     if ((g.tapK == 16 || g.tapK == 32) && p.splits == 1 && p.bm == 64 && g.npix >= (1 << 20))
@@ -85,27 +110,33 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
         counters = (unsigned*)workspace; // zero on entry (the caller cleared the workspace once), zero again on exit
         partial = (int32_t*)((char*)workspace + SPLIT_COUNTER_BYTES);
     }
-    dim3 grid((unsigned)blocks), block(256);
+    dim3 grid((unsigned)blocks), block((unsigned)(256 * p.groups));
     // addressing mode (the kernel's MODE); the K-split kernels exist for modes 0, 1 and 3 only (a narrow-input layer has
     // too few K steps to be split)
-    const int mode = dense ? 1 : ((g.tapK == 16 || g.tapK == 32) && p.splits == 1) ? 2 : (g.tapK % 64 == 0 && g.tapK == g.Cp) ? 3 : 0;
+    const int mode = dense ? 1 : (p.groups == 1 && (g.tapK == 16 || g.tapK == 32) && p.splits == 1) ? 2 : (g.tapK % 64 == 0 && g.tapK == g.Cp) ? 3 : 0;
     if (p.splits > 1) return launch_pipe_split(p, mode, wpk, x, g, epi, fusion, out_cp, out_cp, partial, counters, stream);
-#define LAUNCH_PIPE_MODE(BM_, BN_, MODE_)                                                                                                                \
-    hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<BM_, BN_, PIPE_RING, false, MODE_>), grid, block, 0, stream, wpk, x, g, epi, fusion, out_cp, \
+#define LAUNCH_PIPE_MODE(BM_, BN_, MODE_, GROUPS_)                                                                                                                 \
+    hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<BM_, BN_, PIPE_RING, false, MODE_, 1, GROUPS_>), grid, block, 0, stream, wpk, x, g, epi, fusion, out_cp, \
                        out_cp, p.tiles_m, p.tiles_n, p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, (const float*)0, 0)
 #define LAUNCH_PIPE(BM_, BN_)                  \
     do                                         \
     {                                          \
         if (mode == 1)                         \
-            LAUNCH_PIPE_MODE(BM_, BN_, 1);     \
+            LAUNCH_PIPE_MODE(BM_, BN_, 1, 1);  \
         else if (mode == 2)                    \
-            LAUNCH_PIPE_MODE(BM_, BN_, 2);     \
+            LAUNCH_PIPE_MODE(BM_, BN_, 2, 1);  \
         else if (mode == 3)                    \
-            LAUNCH_PIPE_MODE(BM_, BN_, 3);     \
+            LAUNCH_PIPE_MODE(BM_, BN_, 3, 1);  \
         else                                   \
-            LAUNCH_PIPE_MODE(BM_, BN_, 0);     \
+            LAUNCH_PIPE_MODE(BM_, BN_, 0, 1);  \
     } while (0)
-    if (p.bm == 128 && p.bn == 256)
+    if (p.groups == 4 && mode == 1)
+        LAUNCH_PIPE_MODE(64, 64, 1, 4);
+    else if (p.groups == 4 && mode == 3)
+        LAUNCH_PIPE_MODE(64, 64, 3, 4);
+    else if (p.groups == 4)
+        LAUNCH_PIPE_MODE(64, 64, 0, 4);
+    else if (p.bm == 128 && p.bn == 256)
         LAUNCH_PIPE(128, 256);
     else if (p.bm == 128 && p.bn == 128)
         LAUNCH_PIPE(128, 128);
@@ -148,7 +179,7 @@ int launch_fc_via_conv_pipelined(const int8_t* x, size_t x_stride, int rows, int
     g.cout = num_output;
     g.pad_word = 0;
     const ConvFusion no_fusion = {0, 0, 0, 0.f};
-    const PipePlan p = plan_pipelined(num_output, rows, K / 64);
+    const PipePlan p = plan_pipelined_groups(num_output, rows, K / 64);
     int32_t* partial = 0;
     unsigned* counters = 0;
     if (p.splits > 1)
@@ -157,7 +188,7 @@ int launch_fc_via_conv_pipelined(const int8_t* x, size_t x_stride, int rows, int
         partial = (int32_t*)((char*)workspace + SPLIT_COUNTER_BYTES);
     }
     NCNNHIP_REQUIRE((long long)p.tiles_m * p.tiles_n * p.splits * p.tiles_n < (1ll << 32), "innerproduct: too many tiles");
-    dim3 grid((unsigned)((long long)p.tiles_m * p.tiles_n * p.splits)), block(256);
+    dim3 grid((unsigned)((long long)p.tiles_m * p.tiles_n * p.splits)), block((unsigned)(256 * p.groups));
     // rows are few: only the 64-pixel tiles occur
     if (p.bm != 64)
     {
@@ -165,15 +196,17 @@ int launch_fc_via_conv_pipelined(const int8_t* x, size_t x_stride, int rows, int
         return NCNNHIP_OK;
     }
     if (p.splits > 1) return launch_pipe_split(p, 1, weight, x, g, epi, no_fusion, (int)out_stride, num_output, partial, counters, stream);
-#define LAUNCH_FC(BN_)                                                                                                                                \
-    hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<64, BN_, PIPE_RING, false, 1>), grid, block, 0, stream, weight, x, g, epi, no_fusion, \
+#define LAUNCH_FC(BN_, GROUPS_)                                                                                                                                \
+    hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<64, BN_, PIPE_RING, false, 1, 1, GROUPS_>), grid, block, 0, stream, weight, x, g, epi, no_fusion, \
                        (int)out_stride, num_output, p.tiles_m, p.tiles_n, p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, (const float*)0, 0)
     if (p.bn == 256)
-        LAUNCH_FC(256);
+        LAUNCH_FC(256, 1);
     else if (p.bn == 128)
-        LAUNCH_FC(128);
+        LAUNCH_FC(128, 1);
+    else if (p.groups == 4)
+        LAUNCH_FC(64, 4);
     else
-        LAUNCH_FC(64);
+        LAUNCH_FC(64, 1);
 #undef LAUNCH_FC
     return launch_status("conv_nhwc_pipelined_kernel<fc>");
 }

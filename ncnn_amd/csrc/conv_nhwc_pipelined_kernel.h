@@ -73,13 +73,19 @@ __device__ __forceinline__ uint32_t pack4(const v4f& v)
 // stage would have.  The weights of the tile (BN * K bytes) are requested in full before that and land in a region of
 // their own while the loader works, so the K loop touches LDS only: no waits on memory, no barriers.  x points at the
 // fp32 / fp16 blob, same channels-last geometry counted in values.
-template<int BM, int BN, int STAGES, bool SPLITK, int MODE, int AIN = 1>
-__global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* __restrict__ wpk, const int8_t* __restrict__ x, NhwcGeom g, ConvEpilogue epi,
+//
+// GROUPS: how many times four wavefronts a workgroup has: 1, or 4 on 64 x 64 tiles (plan_pipelined_groups).  Each four walk their own share of the
+// workgroup's K steps through a ring of their own; then the accumulators meet in LDS, [register / 4][thread] in 16-byte
+// words, and every four take 1/GROUPS of each block's pixels: they add up those registers of all groups (integer
+// addition: exact in any order) and run the epilogue for them.
+template<int BM, int BN, int STAGES, bool SPLITK, int MODE, int AIN = 1, int GROUPS = 1>
+__global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const int8_t* __restrict__ wpk, const int8_t* __restrict__ x, NhwcGeom g, ConvEpilogue epi,
                                                                    ConvFusion fusion, int out_cp, int col_limit, int tiles_m, int tiles_n, int splits, int steps_per_split, unsigned magic_n, int32_t* __restrict__ partial, unsigned* __restrict__ counters,
                                                                    const float* __restrict__ a_scale, int a_cache_bytes)
 {
     constexpr bool dense = MODE == 1;
     constexpr bool STAGED = AIN != 1;
+    static_assert(GROUPS == 1 || (!STAGED && BM == 64 && BN == 64 && GROUPS == 4), "several groups of wavefronts: 64 x 64 tiles of an int8 blob");
     static_assert(!STAGED || (MODE != 2 && MODE != 3), "the quantising loader exists for convolutions on ordinary blobs");
     constexpr int TM = BM / 64, TN = BN / 64; // 32x32 blocks per wavefront along pixels / channels
     constexpr int LAR = BM / 64;              // 64-row groups of the activation tile
@@ -87,11 +93,15 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
     static_assert(STAGES >= 2 && STAGES <= 7 && (STAGES - 2) * (LA + LB) < 64, "the vmcnt field counts to 63");
     constexpr int STAGE_BYTES = (BM + BN) * 64;
     constexpr int EPILOGUE_BYTES = 4 * 32 * (BN / 2 + 4) * 4; // per wavefront 32 pixels x (BN/2 + 4) floats
-    constexpr int SMEM_BYTES = (!STAGED && STAGES * STAGE_BYTES > EPILOGUE_BYTES) ? STAGES * STAGE_BYTES : EPILOGUE_BYTES;
+    constexpr int RING_BYTES = STAGES * STAGE_BYTES;
+    constexpr int SMEM_BYTES = (!STAGED && GROUPS * RING_BYTES > EPILOGUE_BYTES) ? GROUPS * RING_BYTES : EPILOGUE_BYTES;
+    constexpr int NR = 16 / GROUPS; // accumulators of a 32x32 block that a lane finishes ...
+    constexpr int PG = 32 / GROUPS; // ... and the pixels they belong to
     __shared__ __attribute__((aligned(1024))) int8_t smem[SMEM_BYTES];
 
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+    const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     const int wm = wave >> 1, wn = wave & 1;
     const int l32 = lane & 31, lhi = lane >> 5;
 
@@ -110,12 +120,21 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
     const int row0 = tm * BM, col0 = tn * BN;
 
     const int total_steps = g.K / 64;
-    const int step_begin = SPLITK ? split * steps_per_split : 0;
+    int step_begin = SPLITK ? split * steps_per_split : 0;
     int step_end = SPLITK ? step_begin + steps_per_split : total_steps;
     if (step_end > total_steps) step_end = total_steps;
+    int iterations = step_end - step_begin; // every wavefront of the workgroup meets this many barriers
+    if (GROUPS > 1)
+    {
+        // this group's share of the steps; the last groups may have fewer than the others, or none
+        iterations = (iterations + GROUPS - 1) / GROUPS;
+        const int begin = step_begin + group * iterations;
+        step_begin = begin < step_end ? begin : step_end;
+        step_end = step_begin + iterations < step_end ? step_begin + iterations : step_end;
+    }
     const int nk = step_end - step_begin;
     const int tile_steps = SPLITK ? steps_per_split : total_steps; // K steps the quantising loader's LDS regions are sized for
-    if (!SPLITK && nk <= 0) return; // (a split workgroup always has steps, and must reach the tile counter in any case)
+    if (!SPLITK && iterations <= 0) return; // (a split workgroup always has steps, and must reach the tile counter in any case)
 
     // ---- sources of this lane's loads.  Load i of a wavefront fills LDS rows i*64 + wave*16 .. +16 of the operand;
     // the lane's row is +lane/4 and it fetches source chunk (lane&3) ^ ((lane>>4)&3) into position lane&3.
@@ -221,7 +240,7 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
     auto issue = [&](int s) {
         // quantising loader: every step has its own place (written once); the address below is that place minus the
         // activation part a ring stage would start with
-        int8_t* stage = STAGED ? a_tile + tile_steps * (BM * 64) + s * (BN * 64) - BM * 64 + wave * 1024 : smem + (s % STAGES) * STAGE_BYTES + wave * 1024;
+        int8_t* stage = STAGED ? a_tile + tile_steps * (BM * 64) + s * (BN * 64) - BM * 64 + wave * 1024 : smem + group * RING_BYTES + (s % STAGES) * STAGE_BYTES + wave * 1024;
         if (dense)
         {
             // one tap, no border: the row's pixel exists or it does not (a_iy0 is 0 or hugely negative)
@@ -325,7 +344,7 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
 
     // fragment read offsets inside a stage: row l32 of each 32-row block, K chunk ks*2 + lhi, swizzled
     const int sw = (l32 >> 2) & 3;
-    const unsigned lds_base = (unsigned)(uintptr_t)(AS3 int8_t*)smem;
+    const unsigned lds_base = (unsigned)(uintptr_t)(AS3 int8_t*)smem + (unsigned)(group * RING_BYTES);
     const unsigned rd_a = (unsigned)((wm * (BM / 2) + l32) * 64);
     const unsigned rd_b = (unsigned)(BM * 64 + (wn * (BN / 2) + l32) * 64);
     const unsigned ch0 = (unsigned)(((0 + lhi) ^ sw) * 16), ch1 = (unsigned)(((2 + lhi) ^ sw) * 16);
@@ -659,8 +678,13 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
         __builtin_amdgcn_s_barrier();
     }
 
-    for (int t = 0; t < nk; t++)
+    for (int t = 0; t < iterations; t++)
     {
+        if (GROUPS > 1 && t >= nk) // a group with fewer steps than the others: the barrier only (uniform)
+        {
+            __builtin_amdgcn_s_barrier();
+            continue;
+        }
         if constexpr (!STAGED)
         {
             // this wavefront's loads of step t have landed (later stages may stay in flight) ...
@@ -712,24 +736,54 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
                 for (int c = 0; c < TN; c++) acc[a][c] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[ks][a], fb[ks][c], acc[a][c], 0, 0, 0);
     }
 
+    // what this lane finishes: its accumulators, or with several groups of wavefronts its share of their sum
+    typedef int accv __attribute__((ext_vector_type(NR)));
+    accv sum[TM][TN];
+    if constexpr (GROUPS == 1)
+    {
+#pragma unroll
+        for (int a = 0; a < TM; a++)
+#pragma unroll
+            for (int c = 0; c < TN; c++) sum[a][c] = acc[a][c];
+    }
+    else
+    {
+        v4i* meet = reinterpret_cast<v4i*>(smem); // [group][register / 4][thread of the group]: 16 KB a group, less than its ring
+        const int tid = threadIdx.x & 255;
+        __syncthreads(); // nobody reads the operand stages any more
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++)
+            meet[(group * 4 + r4) * 256 + tid] = v4i{acc[0][0][4 * r4], acc[0][0][4 * r4 + 1], acc[0][0][4 * r4 + 2], acc[0][0][4 * r4 + 3]};
+        __syncthreads();
+#pragma unroll
+        for (int i4 = 0; i4 < NR / 4; i4++)
+        {
+            v4i s = v4i{0, 0, 0, 0};
+#pragma unroll
+            for (int from = 0; from < GROUPS; from++) s += meet[(from * 4 + group * (NR / 4) + i4) * 256 + tid];
+#pragma unroll
+            for (int e = 0; e < 4; e++) sum[0][0][4 * i4 + e] = s[e];
+        }
+    }
+
     // ---- epilogue: lane = one output channel per 32-column block, registers = pixels
     if (SPLITK)
     {
         // Slice of this workgroup: [register][thread] int32.  The dump and its read-back are agent-scope atomic
         // stores / loads: they go to the coherence point of the whole device (the XCDs' L2s are not coherent with each
         // other inside a kernel) without the full L2 write-back and invalidate a fence would cost every workgroup.
-        constexpr int NREG = TM * TN * 16;
+        constexpr int NREG = TM * TN * NR, THREADS = 256 * GROUPS;
         const int tile_id = tm * tiles_n + tn;
         __shared__ unsigned arrived;
-        int* mine = partial + ((size_t)split * tiles_m * tiles_n + tile_id) * (size_t)(NREG * 256);
+        int* mine = partial + ((size_t)split * tiles_m * tiles_n + tile_id) * (size_t)(NREG * THREADS);
         // optimistic dump: the last workgroup would not need it, but it does not know yet that it is the last
 #pragma unroll
         for (int a = 0; a < TM; a++)
 #pragma unroll
             for (int c = 0; c < TN; c++)
 #pragma unroll
-                for (int r = 0; r < 16; r++)
-                    __hip_atomic_store(mine + ((a * TN + c) * 16 + r) * 256 + threadIdx.x, acc[a][c][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (int r = 0; r < NR; r++)
+                    __hip_atomic_store(mine + ((a * TN + c) * NR + r) * THREADS + threadIdx.x, sum[a][c][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         WAIT_VMCNT(0); // this wavefront's stores have reached the coherence point ...
         asm volatile("" ::: "memory");
         __syncthreads(); // ... and everybody else's in the workgroup, before the counter moves
@@ -739,18 +793,18 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
         for (int s2 = 0; s2 < splits; s2++)
         {
             if (s2 == split) continue;
-            const int* theirs = partial + ((size_t)s2 * tiles_m * tiles_n + tile_id) * (size_t)(NREG * 256);
+            const int* theirs = partial + ((size_t)s2 * tiles_m * tiles_n + tile_id) * (size_t)(NREG * THREADS);
 #pragma unroll
             for (int a = 0; a < TM; a++)
 #pragma unroll
                 for (int c = 0; c < TN; c++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++)
-                        acc[a][c][r] += __hip_atomic_load(theirs + ((a * TN + c) * 16 + r) * 256 + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    for (int r = 0; r < NR; r++)
+                        sum[a][c][r] += __hip_atomic_load(theirs + ((a * TN + c) * NR + r) * THREADS + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (threadIdx.x == 0) counters[tile_id] = 0u; // ready for the next launch
     }
-    // Through LDS, so that global memory sees whole runs of channels: each wavefront stages 32 pixels x CW channels of
+    // Through LDS, so that global memory sees whole runs of channels: each wavefront stages PG pixels x CW channels of
     // results as [pixel][channel] floats (the pipeline stages are free by now), then every lane takes 4 consecutive
     // channels of one pixel: a 16-byte residual load, a 16-byte fp32 store and a 4-byte int8 store, the wavefront
     // covering 64/(CW/4) pixel rows of CW contiguous channels per instruction.
@@ -758,7 +812,7 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
     constexpr int LD = CW + 4;      // row pitch in floats
     constexpr int G = CW / 4;       // 4-channel groups per row
     __syncthreads();                // nobody reads the operand stages any more
-    float* tile = reinterpret_cast<float*>(smem) + wave * (32 * LD);
+    float* tile = reinterpret_cast<float*>(smem) + (group * 4 + wave) * (PG * LD);
     const bool to_int8 = epi.scale_out != 0;
 
     float s_in[TN], bias[TN], s_out[TN];
@@ -788,16 +842,16 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
         {
             // The residual this lane will add in the read-out below is requested now, so that it arrives while the
             // accumulators are being converted (clamped addresses, nothing selected: see the tables above).
-            v4f resv[G / 2];
+            v4f resv[G / 2 / GROUPS];
             const bool with_residual = !to_int8 && fusion.residual != 0;
             if (with_residual)
             {
 #pragma unroll
-                for (int it = 0; it < G / 2; it++)
+                for (int it = 0; it < G / 2 / GROUPS; it++)
                 {
                     const int idx = it * 64 + lane;
                     const int p = idx / G, j = idx - p * G;
-                    int pix = row0 + wm * (BM / 2) + a * 32 + p;
+                    int pix = row0 + wm * (BM / 2) + a * 32 + group * PG + p;
                     int ch4 = col0 + wn * CW + 4 * j;
                     if (pix >= g.npix) pix = g.npix - 1;
                     if (ch4 >= col_limit) ch4 = col_limit - 4;
@@ -808,11 +862,11 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
             for (int c = 0; c < TN; c++)
             {
                 if (col0 + wn * CW + c * 32 >= col_limit) continue; // a whole 32-channel block of tile padding (uniform per wavefront)
-                float fr[16];
+                float fr[NR];
 #pragma unroll
-                for (int r = 0; r < 16; r++)
+                for (int r = 0; r < NR; r++)
                 {
-                    float f = add_rn(mul_rn((float)acc[a][c][r], s_in[c]), bias[c]);
+                    float f = add_rn(mul_rn((float)sum[a][c][r], s_in[c]), bias[c]);
                     if (ACT == 1)
                         f = fmaxf(f, 0.f);
                     else if (ACT == 3)
@@ -831,7 +885,7 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
                 if (to_int8)
                 {
 #pragma unroll
-                    for (int r = 0; r < 16; r += 4)
+                    for (int r = 0; r < NR; r += 4)
                     {
                         if (ACT == 103)
                             float2int8_as_float_bounded_x4(fr[r], fr[r + 1], fr[r + 2], fr[r + 3], q_lo[c], q_hi[c]);
@@ -843,7 +897,7 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
                 // behind the bounded clip a pad's (finite) value times its zero output scale rounds to zero too.
                 const bool clear_pads = ACT != 0 && ACT != 1 && !(ACT == 103 && to_int8);
 #pragma unroll
-                for (int r = 0; r < 16; r++)
+                for (int r = 0; r < NR; r++)
                 {
                     if (clear_pads && !real[c]) fr[r] = 0.f;
                     tile[(8 * (r >> 2) + 4 * lhi + (r & 3)) * LD + c * 32 + l32] = fr[r];
@@ -860,9 +914,9 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
                 {
                     const int idx = it * 64 + lane;
                     const int p = idx / G16, j = idx - p * G16;
-                    const int pix = row0 + wm * (BM / 2) + a * 32 + p;
+                    const int pix = row0 + wm * (BM / 2) + a * 32 + group * PG + p;
                     const int ch16 = col0 + wn * CW + 16 * j;
-                    if (p < 32 && pix < g.npix && ch16 < col_limit)
+                    if (p < PG && pix < g.npix && ch16 < col_limit)
                     {
                         float q[16];
 #pragma unroll
@@ -881,12 +935,12 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
             else
             {
 #pragma unroll
-            for (int it = 0; it < G / 2; it++)
+            for (int it = 0; it < G / 2 / GROUPS; it++)
             {
                 const int idx = it * 64 + lane;
                 const int p = idx / G, j = idx - p * G;
                 v4f v = *reinterpret_cast<const v4f*>(tile + p * LD + 4 * j);
-                const int pix = row0 + wm * (BM / 2) + a * 32 + p;
+                const int pix = row0 + wm * (BM / 2) + a * 32 + group * PG + p;
                 const int ch4 = col0 + wn * CW + 4 * j;
                 if (pix < g.npix && ch4 < col_limit)
                 {
@@ -946,10 +1000,15 @@ __global__ __launch_bounds__(256) void conv_nhwc_pipelined_kernel(const int8_t* 
 struct PipePlan
 {
     int bm, bn, tiles_m, tiles_n, splits, steps_per_split;
+    int groups; // groups of four wavefronts a workgroup has
 };
 
 // tile shape and K split for a problem of cout channels, npix pixels and `steps` 64-byte K steps
 PipePlan plan_pipelined(int cout, long long npix, int steps);
+
+// the same plan for an int8 blob, with K split over groups of wavefronts inside the workgroup where that is better; never
+// takes more scratch than plan_pipelined's
+PipePlan plan_pipelined_groups(int cout, long long npix, int steps);
 
 // multiplier that turns b / tiles_n into a high multiply, exact for b * tiles_n < 2^32 (tiles_n == 1 is special-cased)
 static inline unsigned tile_magic(int tiles_n)
