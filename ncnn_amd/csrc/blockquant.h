@@ -106,7 +106,7 @@ __device__ __forceinline__ void split_bf16x3(float v, unsigned& hi, unsigned& mi
 
 __device__ __forceinline__ unsigned bf16_pair(float even, float odd) // both exactly representable: truncation loses nothing
 {
-    return (__float_as_uint(even) >> 16) | (__float_as_uint(odd) & 0xFFFF0000u);
+    return __builtin_amdgcn_perm(__float_as_uint(odd), __float_as_uint(even), 0x07060302u);
 }
 
 // the 8 fields that bytes_to_halves / nibbles_to_halves / sixbit_to_halves turn into halves, as bf16

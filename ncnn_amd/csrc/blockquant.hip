@@ -1528,6 +1528,290 @@ __global__ __launch_bounds__(256) void blockquant_rows_bf16x3_kernel(const unsig
     }
 }
 
+// The same product where tiles are few: two groups of four wavefronts share a workgroup's tile of 64 activation rows x 32 * RW weight
+// rows, split K between them, each with a ring of two stages of its own, and add their sums through LDS.  A wavefront multiplies
+// half the activation rows with half the weight tiles, which halves the LDS reads a matrix-core instruction needs.  The groups run
+// half a step apart: while one reads and converts its operands, the other, on the same SIMDs, multiplies.  A stage is refilled as
+// soon as its operands are in registers, one and a half steps before they are due.
+// Bound by the issue slots of the conversions and the clock (1.6 to 2.1 GHz under this load); us with the split pass, 8 bits,
+// kernel above -> this one: 256 x 4096 x 4096 64 -> 50, 100 x 4096 x 11008 135 -> 93, 512 x 1024 x 1024 22.7 -> 19.3 (RW = 2);
+// 512 x 4096 x 4096 90 -> 78, 512 x 4096 x 11008 209 -> 178, 300 x 5120 x 5120 100 -> 86 (RW = 4).  Without the half step's
+// distance 512 x 4096 x 4096 took 85 us.  Error against 64 bits at that size: 1.79e-7 above, 1.44e-7 here.
+template<int BITS, bool HALVES, int RW>
+__global__ __launch_bounds__(512) void blockquant_rows_ksplit_bf16x3_kernel(const unsigned short* __restrict__ planes, int Mp, int Kp, int M, int N, int kblocks,
+                                                                      int ntiles, const unsigned char* __restrict__ wpk, const float4* __restrict__ dpk, int split,
+                                                                      const float* __restrict__ c, int bt, float alpha, float beta, float* __restrict__ out,
+                                                                      size_t out_stride)
+{
+    static_assert(HALVES || BITS == 8, "4- and 6-bit fields come in the halves layout");
+    static_assert(RW == 2 || RW == 4, "a tile of 16 weight rows is fetched by one of the two wavefronts that multiply it");
+    constexpr int STAGES = 2;
+    constexpr int RWL = RW / 2;        // weight tiles a wavefront fetches
+    constexpr int LOADS = 6 + 2 * RWL; // per wavefront and stage
+    constexpr int CW = 2;              // groups of 16 activation rows a wavefront multiplies
+    constexpr int PLANE = 64 * 128;
+    constexpr int ACT_BYTES = 3 * PLANE;
+    constexpr int W_OFF = ACT_BYTES, D_OFF = ACT_BYTES + 4 * RWL * 1024;
+    constexpr int STAGE_BYTES = D_OFF + 4 * RWL * 128;
+    constexpr int STEP_BYTES = 128 * BITS;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds_rows[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+    const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int wa = wave & 1, ww = wave >> 1; // the wavefront's half of the activation rows and of the weight tiles
+    const int m = lane & 15, kg = lane >> 4;
+    const int row0 = blockIdx.y * 64;
+    const int dper = HALVES ? 4 << split : 4;
+
+    // the RWL tiles the wavefront fetches (a tile beyond the last reads the last one again and stores nothing)
+    const unsigned char* wsrc[RWL];
+    const float4* dsrc[RWL];
+#pragma unroll
+    for (int rw = 0; rw < RWL; rw++)
+    {
+        const int t = ((int)blockIdx.x * 4 + wave) * RWL + rw;
+        const int tl = t < ntiles ? t : ntiles - 1;
+        wsrc[rw] = wpk + (size_t)tl * kblocks * STEP_BYTES + lane * 16;
+        dsrc[rw] = dpk + (size_t)tl * kblocks * dper + lane;
+    }
+    // activation loads: load i of wavefront w fills rows (i % 2) * 32 + w * 8 .. +8 of plane i / 2; lane l brings row + l / 8,
+    // the chunk that belongs at position l % 8
+    const unsigned short* asrc[6];
+#pragma unroll
+    for (int i = 0; i < 6; i++)
+    {
+        const int r = (i & 1) * 32 + wave * 8 + (lane >> 3);
+        const int ch = (lane & 7) ^ ((r >> 1) & 7);
+        asrc[i] = planes + ((size_t)(i >> 1) * Mp + row0 + r) * Kp + ch * 8;
+    }
+    auto issue = [&](int step, int slot) {
+        unsigned char* st = lds_rows + (group * STAGES + slot) * STAGE_BYTES;
+#pragma unroll
+        for (int i = 0; i < 6; i++)
+            __builtin_amdgcn_global_load_lds((const BQ_AS1 void*)(asrc[i] + (size_t)step * 64),
+                                             (BQ_AS3 void*)(st + (i >> 1) * PLANE + ((i & 1) * 32 + wave * 8) * 128), 16, 0, 0);
+#pragma unroll
+        for (int rw = 0; rw < RWL; rw++)
+        {
+            if (lane < STEP_BYTES / 16)
+                __builtin_amdgcn_global_load_lds((const BQ_AS1 void*)(wsrc[rw] + (size_t)step * STEP_BYTES), (BQ_AS3 void*)(st + W_OFF + (wave * RWL + rw) * 1024), 16, 0,
+                                                 0);
+        }
+#pragma unroll
+        for (int rw = 0; rw < RWL; rw++)
+        {
+            if (lane < dper)
+                __builtin_amdgcn_global_load_lds((const BQ_AS1 void*)(dsrc[rw] + (size_t)step * dper), (BQ_AS3 void*)(st + D_OFF + (wave * RWL + rw) * 128), 16, 0, 0);
+        }
+    };
+
+    v4f acc[RW][CW];
+#pragma unroll
+    for (int rw = 0; rw < RW; rw++)
+#pragma unroll
+        for (int cw = 0; cw < CW; cw++) acc[rw][cw] = v4f{0.f, 0.f, 0.f, 0.f};
+
+    // operand reads: row (wa * CW + cw) * 16 + m, chunk positions of the lane's two K groups (the swizzle does not depend on cw)
+    const int sw = (m >> 1) & 7;
+    const int rd_a = (wa * CW * 16 + m) * 128 + (((HALVES ? kg : 2 * kg) ^ sw) << 4);
+    const int rd_b = (wa * CW * 16 + m) * 128 + (((HALVES ? 4 + kg : 2 * kg + 1) ^ sw) << 4);
+    // K steps of this group of wavefronts; every wavefront of the workgroup goes through the same number of iterations
+    const int iterations = (kblocks + 1) / 2;
+    const int first = group * iterations;
+    const int end = first + iterations < kblocks ? first + iterations : kblocks;
+    const int last = kblocks - 1;
+    const unsigned lds_base = (unsigned)(uintptr_t)(BQ_AS3 unsigned char*)lds_rows + (unsigned)(group * STAGES * STAGE_BYTES);
+
+    issue(first < last ? first : last, 0);
+    issue(first + 1 < last ? first + 1 : last, 1);
+    int slot = 0; // the stage of this step
+    if (group == 1) __builtin_amdgcn_s_barrier(); // half a step behind the first group
+    for (int step = first; step < first + iterations; step++)
+    {
+        BQ_WAIT_VMCNT(LOADS);         // this wavefront's loads of the step have landed, the next step's may still be on their way
+        __builtin_amdgcn_s_barrier(); // and everybody else's
+        asm volatile("" ::: "memory");
+        // LDS is read with hand-written instructions and waits: the compiler treats a direct-to-LDS load as a store to all of LDS
+        // and would drain every load in flight (vmcnt(0)) in front of each read it emits itself.  A wait names the registers it
+        // covers as in/out operands, so nothing can use them ahead of it.
+        const unsigned st = lds_base + (unsigned)(slot * STAGE_BYTES);
+        if (step >= end) // (uniform: the last iteration of the second group, which has a step less)
+        {
+            __builtin_amdgcn_s_barrier();
+            break;
+        }
+        v4i_bq wq[RW], dq0[RW], dq1[RW];
+        v2i_bq wlo[RW]; // 4- and 6-bit: the lane's first 8 bytes
+        int whi[RW];    // 6-bit: its third dword
+        {
+            const unsigned wl = st + W_OFF + (unsigned)(ww * RW * 1024) + (unsigned)(lane * (BITS == 8 ? 16 : 8));
+            const unsigned wl3 = st + W_OFF + (unsigned)(ww * RW * 1024) + 512u + (unsigned)(lane * 4);
+            const unsigned dl = st + D_OFF + (unsigned)(ww * RW * 128) + (unsigned)(kg * 16);
+            const unsigned dl2 = dl + (unsigned)(split << 6);
+#pragma unroll
+            for (int rw = 0; rw < RW; rw++)
+            {
+                // every result register is written by its read and first touched after the wait below
+                if (BITS == 8)
+                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(wq[rw]) : "v"(wl), "n"(rw * 1024));
+                else
+                    asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(wlo[rw]) : "v"(wl), "n"(rw * 1024));
+                if (BITS == 6) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(whi[rw]) : "v"(wl3), "n"(rw * 1024));
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dq0[rw]) : "v"(dl), "n"(rw * 128));
+                if (HALVES) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dq1[rw]) : "v"(dl2), "n"(rw * 128));
+            }
+        }
+        // the six operand fragments of a 16-row group (3 planes x 2 halves of the step)
+        union Act
+        {
+            v4i_bq i4;
+            v8bf h;
+        };
+        Act ya[CW][3], yb[CW][3];
+        const unsigned ra = st + (unsigned)rd_a, rb = st + (unsigned)rd_b;
+        auto read_group = [&](int cw) {
+            const unsigned pa = ra + (unsigned)(cw * 2048), pb = rb + (unsigned)(cw * 2048);
+            asm volatile("ds_read_b128 %0, %1" : "=v"(ya[cw][0].i4) : "v"(pa));
+            asm volatile("ds_read_b128 %0, %1" : "=v"(yb[cw][0].i4) : "v"(pb));
+            asm volatile("ds_read_b128 %0, %1 offset:8192" : "=v"(ya[cw][1].i4) : "v"(pa));
+            asm volatile("ds_read_b128 %0, %1 offset:8192" : "=v"(yb[cw][1].i4) : "v"(pb));
+            asm volatile("ds_read_b128 %0, %1 offset:16384" : "=v"(ya[cw][2].i4) : "v"(pa));
+            asm volatile("ds_read_b128 %0, %1 offset:16384" : "=v"(yb[cw][2].i4) : "v"(pb));
+        };
+#pragma unroll
+        for (int cw = 0; cw < CW; cw++) read_group(cw);
+#pragma unroll
+        for (int rw = 0; rw < RW; rw++) // the weights are here, the activations' twelve reads may still be on their way (the later waits only tie their registers to the first)
+        {
+            if constexpr (BITS == 8)
+                asm volatile("s_waitcnt lgkmcnt(12)" : "+v"(wq[rw]));
+            else
+                asm volatile("s_waitcnt lgkmcnt(12)" : "+v"(wlo[rw]));
+            if constexpr (BITS == 6) asm volatile("" : "+v"(whi[rw]));
+        }
+        // 8-bit weights: the second half of the step is converted between the matrix-core instructions of the first
+        v8bf fa[RW], fb[RW];
+#pragma unroll
+        for (int rw = 0; rw < RW; rw++)
+        {
+            if constexpr (BITS == 8)
+                fa[rw] = bytes_to_bf16((unsigned)wq[rw][0], (unsigned)wq[rw][1]);
+            else if constexpr (BITS == 4)
+            {
+                fa[rw] = nibbles_to_bf16((unsigned)wlo[rw][0]);
+                fb[rw] = nibbles_to_bf16((unsigned)wlo[rw][1]);
+            }
+            else
+                sixbit_to_bf16((unsigned)wlo[rw][0], (unsigned)wlo[rw][1], (unsigned)whi[rw], fa[rw], fb[rw]);
+        }
+#pragma unroll
+        for (int cw = 0; cw < CW; cw++)
+            asm volatile("s_waitcnt lgkmcnt(0)"
+                         : "+v"(ya[cw][0].i4), "+v"(yb[cw][0].i4), "+v"(ya[cw][1].i4), "+v"(yb[cw][1].i4), "+v"(ya[cw][2].i4), "+v"(yb[cw][2].i4));
+#pragma unroll
+        for (int rw = 0; rw < RW; rw++)
+        {
+            asm volatile("" : "+v"(fa[rw]), "+v"(dq0[rw])); // converted on this side of the barrier
+            if constexpr (HALVES) asm volatile("" : "+v"(dq1[rw]));
+            if constexpr (BITS != 8) asm volatile("" : "+v"(fb[rw]));
+        }
+        __builtin_amdgcn_s_barrier(); // everybody of this group has read the stage; the other group reads and converts now
+        asm volatile("" ::: "memory");
+        issue(step + 2 < last ? step + 2 : last, slot);
+        slot ^= 1;
+#pragma unroll
+        for (int rw = 0; rw < RW; rw++) // multiplied on that side
+        {
+            asm volatile("" : "+v"(fa[rw]));
+            if constexpr (BITS == 8)
+            {
+                asm volatile("" : "+v"(wq[rw]));
+                fb[rw] = bytes_to_bf16((unsigned)wq[rw][2], (unsigned)wq[rw][3]);
+            }
+        }
+#pragma unroll
+        for (int cw = 0; cw < CW; cw++)
+        {
+            // the tiles' chains alternate, so that no instruction waits for the one right before it
+            v4f t0[RW], t1[RW];
+#pragma unroll
+            for (int rw = 0; rw < RW; rw++) t0[rw] = t1[rw] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int pn = 0; pn < 3; pn++)
+#pragma unroll
+                for (int rw = 0; rw < RW; rw++) t0[rw] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[rw], ya[cw][pn].h, t0[rw], 0, 0, 0);
+#pragma unroll
+            for (int pn = 0; pn < 3; pn++)
+#pragma unroll
+                for (int rw = 0; rw < RW; rw++)
+                {
+                    if (HALVES)
+                        t1[rw] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[rw], yb[cw][pn].h, t1[rw], 0, 0, 0);
+                    else
+                        t0[rw] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[rw], yb[cw][pn].h, t0[rw], 0, 0, 0);
+                }
+#pragma unroll
+            for (int rw = 0; rw < RW; rw++)
+            {
+                const float da[4] = {__int_as_float(dq0[rw][0]), __int_as_float(dq0[rw][1]), __int_as_float(dq0[rw][2]), __int_as_float(dq0[rw][3])};
+                const float db[4] = {__int_as_float(dq1[rw][0]), __int_as_float(dq1[rw][1]), __int_as_float(dq1[rw][2]), __int_as_float(dq1[rw][3])};
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                {
+                    if (HALVES)
+                        acc[rw][cw][r] = fmaf(t1[rw][r], db[r], fmaf(t0[rw][r], da[r], acc[rw][cw][r]));
+                    else
+                        acc[rw][cw][r] = fmaf(t0[rw][r], da[r], acc[rw][cw][r]);
+                }
+            }
+        }
+    }
+    if (group == 0) __builtin_amdgcn_s_barrier(); // the second group's last half step
+    BQ_WAIT_VMCNT(0); // the surplus loads of the last steps must not outlive the workgroup's LDS
+
+    // the second group hands its sums over through LDS, [tile, row group][thread] in 16-byte words, once nobody reads the stages
+    v4f* meet = reinterpret_cast<v4f*>(lds_rows);
+    const int tid = threadIdx.x & 255;
+    __syncthreads();
+    if (group == 1)
+    {
+#pragma unroll
+        for (int rw = 0; rw < RW; rw++)
+#pragma unroll
+            for (int cw = 0; cw < CW; cw++) meet[(rw * CW + cw) * 256 + tid] = acc[rw][cw];
+    }
+    __syncthreads();
+    if (group == 1) return;
+#pragma unroll
+    for (int rw = 0; rw < RW; rw++)
+#pragma unroll
+        for (int cw = 0; cw < CW; cw++) acc[rw][cw] += meet[(rw * CW + cw) * 256 + tid];
+
+    // accumulator r of lane l: weight row (l/16)*4 + r of the tile, activation row l%16 of the 16-row group
+#pragma unroll
+    for (int rw = 0; rw < RW; rw++)
+    {
+        const int t = ((int)blockIdx.x * 2 + ww) * RW + rw;
+#pragma unroll
+        for (int cw = 0; cw < CW; cw++)
+        {
+            const int i = row0 + (wa * CW + cw) * 16 + m;
+            if (i >= M) continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+            {
+                const int j = t * 16 + kg * 4 + r;
+                if (j < N)
+                {
+                    float v = acc[rw][cw][r];
+                    if (bt >= 0) v = add_rn(mul_rn(load_c(c, bt, i, j, N), beta), v);
+                    out[(size_t)i * out_stride + j] = mul_rn(v, alpha);
+                }
+            }
+        }
+    }
+}
+
 // ---- 5 to 16 activation rows in fp32, K up to 4096: weight-streaming shape, exact split made by a pass of its own ----
 // Between the four rows per pass of the few-row kernel (LDS cannot hold more rows' planes) and the tiled kernel (too few
 // workgroups to stream the weights at this row count): the few-row kernel's shape -- one workgroup per tile of 16 weight
@@ -2210,7 +2494,8 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
     hipLaunchKernelGGL(blockquant_split_activations_kernel, dim3((unsigned)((vectors + 256 * SPLIT_VECS - 1) / (256 * SPLIT_VECS))), dim3(256), 0, st, a_dev, a_stride, M, K, in_scales_dev, planes, Mp,
                        Kp);
     // Two tiles per wavefront and two stages: 66 KB of LDS, so two workgroups share a compute unit and one's loads, waits and
-    // vector work overlap the other's matrix-core instructions.  Measured at 1024 x 4096 x 4096 / 2048 x 11008 x 4096: 135 / 616 us;
+    // vector work overlap the other's matrix-core instructions.  Measured at 1024 x 4096 x 4096 / 2048 x 11008 x 4096: 135 / 616 us
+    // (138 / 568 -> 128 to 133 / 553 to 574 since the converted pairs are packed by one byte permute; the figures below are from before);
     // four tiles per wavefront with three stages (one workgroup per unit, half the LDS reads per instruction) 145 / 714 us; two
     // tiles with four stages (one workgroup per unit) 172 / 795 us.  While that leaves fewer workgroups than the chip has compute
     // units, one tile per wavefront (64 weight rows per workgroup) doubles them: 128 x 4096 x 4096 77 -> 58 us, 256 rows 82 -> 63,
@@ -2244,13 +2529,24 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
             }
         }
     }
+    // Up to one 64 x 64 tile per compute unit, the kernel that splits K inside the workgroup, one tile each; between that and one
+    // 64 x 128 tile per unit, the same with the larger tile, for 8-bit weights in the plain layout and K from 1536: 700 x 1536 x
+    // 1536 37.2 -> 35.3 us, 1000 x 2048 x 2048 52 -> 48, but an attention layer's 1500 x 1024 x 1024 was 1.5 us slower.  With the halves layout (two
+    // scales a step, and 4- or 6-bit fields) the larger tile measured no better than this file's other kernel: 4 bits, 512 x 4096 x
+    // 4096 83.0 against 83.4 us, 700 x 1536 x 1536 36 against 35; the smaller tile is better there too (256 x 4096 x 4096 59 -> 53).
+    // Beyond a round of the chip the two workgroups a unit holds of the other kernel win: 1024 x 4096 x 4096 128 against 140 us.
+    int ks_tiles = 0;
+    if ((long long)((ntiles + 3) / 4) * (Mp / 64) <= 256)
+        ks_tiles = 2;
+    else if (!halves && kblocks >= 24 && (long long)((ntiles + 7) / 8) * (Mp / 64) <= 256)
+        ks_tiles = 4;
     // (a ring of four stages where a workgroup has its compute unit to itself measured the same as two: 57.6 against 57.8 us at 128 x 4096 x 4096)
-    const dim3 grid((ntiles + 4 * rw_tiles - 1) / (4 * rw_tiles), Mp / 64);
-#define ROWS_RW(BITS_, HALVES_, RW_, STAGES_)                                                                                                                      \
+    const int wg_tiles = ks_tiles ? 2 * ks_tiles : 4 * rw_tiles;
+    const dim3 grid((ntiles + wg_tiles - 1) / wg_tiles, Mp / 64);
+#define ROWS_LAUNCH(KERNEL_, THREADS_, LDS_)                                                                                                                        \
     do                                                                                                                                                             \
     {                                                                                                                                                              \
-        auto kernel = blockquant_rows_bf16x3_kernel<BITS_, HALVES_, STAGES_, RW_>;                                                                                 \
-        const size_t lds = (size_t)(STAGES_) * (3 * 64 * 128 + 4 * (RW_) * 1024 + 4 * (RW_) * 128);                                                                  \
+        auto kernel = KERNEL_;                                                                                                                                     \
         static std::atomic<unsigned char> raised[64];                                                                                                              \
         int device = 0;                                                                                                                                            \
         NCNNHIP_CHECK(hipGetDevice(&device));                                                                                                                      \
@@ -2259,19 +2555,27 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
             NCNNHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));                     \
             if (device >= 0 && device < 64) raised[device].store(1, std::memory_order_release);                                                                    \
         }                                                                                                                                                          \
-        hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, planes, Mp, Kp, M, N, kblocks, ntiles, packed_w_dev, dpk, split, c_dev, bt, alpha, beta, out_dev, out_stride); \
+        hipLaunchKernelGGL(kernel, grid, dim3(THREADS_), LDS_, st, planes, Mp, Kp, M, N, kblocks, ntiles, packed_w_dev, dpk, split, c_dev, bt, alpha, beta, out_dev, out_stride); \
     } while (0)
-#define ROWS(BITS_, HALVES_)            \
-    do                                  \
-    {                                   \
-        if (rw_tiles == 1)                 \
-            ROWS_RW(BITS_, HALVES_, 1, 2); \
-        else if (rw_tiles == 3)            \
-            ROWS_RW(BITS_, HALVES_, 3, 2); \
-        else                               \
-            ROWS_RW(BITS_, HALVES_, 2, 2); \
+#define ROWS_RW(BITS_, HALVES_, RW_) \
+    ROWS_LAUNCH((blockquant_rows_bf16x3_kernel<BITS_, HALVES_, 2, RW_>), 256, (size_t)2 * (3 * 64 * 128 + 4 * (RW_) * 1024 + 4 * (RW_) * 128))
+#define ROWS_KS(BITS_, HALVES_, RW_) \
+    ROWS_LAUNCH((blockquant_rows_ksplit_bf16x3_kernel<BITS_, HALVES_, RW_>), 512, (size_t)4 * (3 * 64 * 128 + 2 * (RW_) * 1024 + 2 * (RW_) * 128))
+#define ROWS(BITS_, HALVES_)             \
+    do                                   \
+    {                                    \
+        if (ks_tiles == 2)               \
+            ROWS_KS(BITS_, HALVES_, 2);  \
+        else if (rw_tiles == 1)          \
+            ROWS_RW(BITS_, HALVES_, 1);  \
+        else if (rw_tiles == 3)          \
+            ROWS_RW(BITS_, HALVES_, 3);  \
+        else                             \
+            ROWS_RW(BITS_, HALVES_, 2);  \
     } while (0)
-    if (!halves)
+    if (ks_tiles == 4)
+        ROWS_KS(8, false, 4);
+    else if (!halves)
         ROWS(8, false);
     else if (bits == 8)
         ROWS(8, true);
@@ -2280,7 +2584,9 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
     else
         ROWS(4, true);
 #undef ROWS
+#undef ROWS_KS
 #undef ROWS_RW
+#undef ROWS_LAUNCH
     return launch_status("blockquant_rows_bf16x3_kernel");
 }
 

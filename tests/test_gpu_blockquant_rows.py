@@ -1,4 +1,4 @@
-"""Block-quantised Gemm on many fp16 activation rows: groups of 16 rows, tiles of 16 weight rows and the K steps of 64 at
+"""Block-quantised Gemm on many activation rows: groups of 16 rows, tiles of 16 weight rows and the K steps of 64 at
 their edges, every packed layout, alone and with several matrices in one call: against the oracle and a float64 value."""
 import numpy as np
 import pytest
@@ -50,3 +50,16 @@ def test_several_matrices_in_one_call(rt, m):
     outs = rt.gemm_blockquant_packed_multi(a.astype(np.float16), mats, bits=4, block=64)
     for (_, p, s), got in zip(ops, outs):
         _check(got, a, p, s, 4, 64)
+
+
+@pytest.mark.parametrize("m,n,k", [(129, 16, 16), (130, 72, 144), (191, 33, 64), (200, 1000, 1040), (1025, 1000, 320), (1025, 1000, 1552), (1024, 2048, 96), (1030, 2050, 128)])
+@pytest.mark.parametrize("bits,block", [(8, 64), (8, 32), (6, 128), (6, 32), (4, 64), (4, 32)])
+def test_many_fp32_rows(rt, m, n, k, bits, block):
+    """Both tile widths of the kernel that splits K inside a workgroup and the kernel beyond it: one K step (the second
+    half has none), odd and even numbers of steps, tiles beyond the last row and weight row."""
+    print("[case]", m, n, k, bits, block, flush=True)
+    a, packed, scales = synth.blockquant_operands(m + n + k, m, n, k, bits, block)
+    c = np.random.default_rng(n).normal(size=(m, n)).astype(F)
+    pw, pd = rt.blockquant_pack(packed, scales, block, bits=bits, k=k)
+    got = rt.gemm_blockquant_packed(a, pw, pd, n, c, 3, 0.75, 1.5, bits=bits, block=block, rows_kernel=True)
+    _check(got, a, packed, scales, bits, block, c, 3, 0.75, 1.5)
