@@ -7,7 +7,6 @@
 #include <condition_variable>
 #include <mutex>
 #include <thread>
-#include <vector>
 
 namespace ncnn {
 
@@ -19,34 +18,37 @@ const size_t PIECE = 256 * 1024;
 // a helper that has finished looks for the next chunk of the same upload for this many turns (about 100 us) before it sleeps
 const int SPINS = 2000;
 
+// Never destroyed: a child of fork() has the object but none of its threads, and there the destructor of the condition
+// variable would wait for sleepers that do not exist; and another thread may still be copying when the process exits.
 class CopyPool
 {
 public:
-    CopyPool() : owner(getpid()), generation(0), stop(false), open(false), next(0), active(0), dst(0), src(0), bytes(0)
+    CopyPool() : count(0), owner(getpid()), generation(0), stop(false), open(false), next(0), active(0), dst(0), src(0), bytes(0)
     {
-        const unsigned cores = std::thread::hardware_concurrency();
-        const int count = cores > (unsigned)HELPERS ? HELPERS : 0;
-        for (int i = 0; i < count; i++) threads.push_back(std::thread(&CopyPool::help, this));
-    }
-    ~CopyPool()
-    {
-        if (getpid() != owner) // a forked child has none of the threads
+        if (std::thread::hardware_concurrency() <= (unsigned)HELPERS) return;
+        while (count < HELPERS)
         {
-            for (size_t i = 0; i < threads.size(); i++) threads[i].detach();
-            return;
+            threads[count] = std::thread(&CopyPool::help, this);
+            count++;
         }
+    }
+    // The end of the process, or of the library in it: ends the helpers.  Whoever copies afterwards copies alone (user stays
+    // locked), and so does whoever copies just now: the helpers then sleep on until the process is gone.
+    void retire()
+    {
+        if (getpid() != owner || !user.try_lock()) return;
         {
             std::lock_guard<std::mutex> g(lock);
             stop = true;
             generation.fetch_add(1);
         }
         wake.notify_all();
-        for (size_t i = 0; i < threads.size(); i++) threads[i].join();
+        for (int i = 0; i < count; i++) threads[i].join();
     }
 
     bool copy(void* _dst, const void* _src, size_t _bytes)
     {
-        if (threads.empty() || getpid() != owner || !user.try_lock()) return false;
+        if (!count || getpid() != owner || !user.try_lock()) return false;
         {
             std::lock_guard<std::mutex> g(lock);
             dst = (unsigned char*)_dst;
@@ -98,7 +100,8 @@ private:
         }
     }
 
-    std::vector<std::thread> threads;
+    std::thread threads[HELPERS];
+    int count;
     const pid_t owner;
     std::mutex user; // one copy at a time
     std::mutex lock;
@@ -120,8 +123,13 @@ void parallel_copy(void* dst, const void* src, size_t bytes)
     // below 1 MB (40 us) one thread is done before the others are awake
     if (bytes >= 4 * PIECE)
     {
-        static CopyPool pool;
-        if (pool.copy(dst, src, bytes)) return;
+        static CopyPool* const pool = new CopyPool;
+        static const struct AtExit
+        {
+            ~AtExit() { pool->retire(); }
+        } at_exit;
+        (void)at_exit;
+        if (pool->copy(dst, src, bytes)) return;
     }
     memcpy(dst, src, bytes);
 }
