@@ -6,6 +6,8 @@
 #include <atomic>
 #include <condition_variable>
 #include <mutex>
+#include <new>
+#include <system_error>
 #include <thread>
 
 namespace ncnn {
@@ -26,10 +28,16 @@ public:
     CopyPool() : count(0), owner(getpid()), generation(0), stop(false), open(false), next(0), active(0), dst(0), src(0), bytes(0)
     {
         if (std::thread::hardware_concurrency() <= (unsigned)HELPERS) return;
-        while (count < HELPERS)
+        try
         {
-            threads[count] = std::thread(&CopyPool::help, this);
-            count++;
+            while (count < HELPERS)
+            {
+                threads[count] = std::thread(&CopyPool::help, this);
+                count++;
+            }
+        }
+        catch (const std::system_error&) // the process may have no more threads: with those there are, or with none
+        {
         }
     }
     // The end of the process, or of the library in it: ends the helpers.  Whoever copies afterwards copies alone (user stays
@@ -123,13 +131,16 @@ void parallel_copy(void* dst, const void* src, size_t bytes)
     // below 1 MB (40 us) one thread is done before the others are awake
     if (bytes >= 4 * PIECE)
     {
-        static CopyPool* const pool = new CopyPool;
+        static CopyPool* const pool = new (std::nothrow) CopyPool;
         static const struct AtExit
         {
-            ~AtExit() { pool->retire(); }
+            ~AtExit()
+            {
+                if (pool) pool->retire();
+            }
         } at_exit;
         (void)at_exit;
-        if (pool->copy(dst, src, bytes)) return;
+        if (pool && pool->copy(dst, src, bytes)) return;
     }
     memcpy(dst, src, bytes);
 }

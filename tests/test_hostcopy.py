@@ -11,12 +11,15 @@ HOST = os.path.join(ROOT, "ncnn_amd", "host", "ncnn")
 DRIVER = r'''
 #include "hostcopy.h"
 #include <atomic>
+#include <cerrno>
 #include <csignal>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <thread>
 #include <vector>
+#include <dlfcn.h>
+#include <pthread.h>
 #include <sys/wait.h>
 #include <unistd.h>
 
@@ -28,9 +31,19 @@ static bool copies(size_t bytes)
     return memcmp(a.data(), b.data(), bytes) == 0 && b[bytes] == 0;
 }
 
+// a process at its limit of threads: every creation from the allowed number on fails
+static std::atomic<int> threads_left(1 << 30);
+extern "C" int pthread_create(pthread_t* t, const pthread_attr_t* attr, void* (*start)(void*), void* arg)
+{
+    typedef int (*create)(pthread_t*, const pthread_attr_t*, void* (*)(void*), void*);
+    static const create real = (create)dlsym(RTLD_NEXT, "pthread_create");
+    return threads_left.fetch_sub(1) > 0 ? real(t, attr, start, arg) : EAGAIN;
+}
+
 int main(int argc, char** argv)
 {
     const char* what = argv[1];
+    if (!strncmp(what, "limit", 5)) threads_left = atoi(what + 5);
     for (size_t bytes : {(size_t)1, (size_t)1 << 20, (size_t)(3 << 20) + 5, (size_t)8 << 20})
         if (!copies(bytes)) return 2;
     if (!strcmp(what, "fork")) // the child copies and leaves through exit()
@@ -76,3 +89,9 @@ def driver(tmp_path_factory):
 def test_the_process_leaves(driver, what):
     """A forked child that leaves through exit() has the pool's object and none of its threads."""
     assert subprocess.run([driver, what], timeout=60).returncode == 0
+
+
+@pytest.mark.parametrize("threads", [0, 1, 2])
+def test_a_process_at_its_limit_of_threads_copies_with_those_it_gets(driver, threads):
+    p = subprocess.run([driver, "limit%d" % threads], timeout=60, capture_output=True, text=True)
+    assert p.returncode == 0, (p.returncode, p.stderr)
