@@ -46,6 +46,7 @@ int ncnnhip_device_synchronize(void);
  * instead of run; nothing may allocate, copy from pageable memory or synchronise on the capturing thread.  The
  * executable graph replays the same kernels on the same buffers. */
 int ncnnhip_stream_begin_capture(void* stream);
+int ncnnhip_stream_is_capturing(void* stream, int* capturing); /* *capturing: 1 between begin and end, else 0 */
 int ncnnhip_stream_end_capture(void* stream, void** graph_exec);
 int ncnnhip_graph_launch(void* graph_exec, void* stream);
 int ncnnhip_graph_destroy(void* graph_exec);

@@ -123,6 +123,15 @@ int ncnnhip_stream_begin_capture(void* stream)
     return NCNNHIP_OK;
 }
 
+int ncnnhip_stream_is_capturing(void* stream, int* capturing)
+{
+    NCNNHIP_REQUIRE(stream && capturing, "ncnnhip_stream_is_capturing: null pointer");
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    NCNNHIP_CHECK(hipStreamIsCapturing(as_stream(stream), &status));
+    *capturing = status != hipStreamCaptureStatusNone;
+    return NCNNHIP_OK;
+}
+
 int ncnnhip_stream_end_capture(void* stream, void** graph_exec)
 {
     NCNNHIP_REQUIRE(stream && graph_exec, "ncnnhip_stream_end_capture: null pointer");

@@ -60,6 +60,7 @@ _SIGNATURES = {
     "ncnnhip_attention_f32_append": [C.c_void_p, C.c_size_t, C.c_float, C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p,
                                      C.c_void_p, C.c_size_t, C.c_void_p],
     "ncnnhip_stream_begin_capture": [C.c_void_p],
+    "ncnnhip_stream_is_capturing": [C.c_void_p, C.POINTER(C.c_int)],
     "ncnnhip_stream_end_capture": [C.c_void_p, C.POINTER(C.c_void_p)],
     "ncnnhip_graph_launch": [C.c_void_p, C.c_void_p],
     "ncnnhip_graph_destroy": [C.c_void_p],

@@ -354,9 +354,25 @@ static size_t host_bytes(const Mat& m)
     return (m.n > 1 ? m.nstep * m.n : m.total()) * m.elemsize;
 }
 
-int HipCommand::upload(const Mat& src, HipMat& dst)
+// A transfer goes through a staging buffer that the host fills now and reuses later: recorded into a graph, a replay would
+// move whatever the buffer holds by then.
+int HipCommand::ready_for_transfer()
 {
     int ret = ensure_ready();
+    if (ret != 0) return ret;
+    int capturing = 0;
+    ret = hip_status(ncnnhip_stream_is_capturing(stream, &capturing), "ncnnhip_stream_is_capturing");
+    if (ret == 0 && capturing)
+    {
+        NCNN_LOGE("HipCommand: a blob cannot move between host and device while its stream is being captured");
+        ret = -1;
+    }
+    return ret;
+}
+
+int HipCommand::upload(const Mat& src, HipMat& dst)
+{
+    int ret = ready_for_transfer();
     if (ret != 0) return ret;
     if (src.empty() || src.elempack != 1 || (src.elemsize != 4u && src.elemsize != 1u) || src.dims < 1 || src.dims > 3)
     {
@@ -377,7 +393,7 @@ int HipCommand::upload(const Mat& src, HipMat& dst)
 
 int HipCommand::upload_into(const Mat& src, HipMat& dst)
 {
-    int ret = ensure_ready();
+    int ret = ready_for_transfer();
     if (ret != 0) return ret;
     if (src.empty() || dst.empty() || src.elempack != 1 || src.dims != dst.dims || src.elemsize != dst.elemsize || src.w != dst.w || src.n != dst.n
         || (src.dims >= 2 && src.h != dst.h) || (src.dims == 3 && src.c != dst.c) || src.dims < 1 || src.dims > 3)
@@ -513,7 +529,7 @@ int HipCommand::widen(const HipMat& src, HipMat& dst)
 int HipCommand::download(const HipMat& blob, Mat& dst, Allocator* allocator)
 {
     if (blob.empty()) return -1;
-    int ready_ret = ensure_ready();
+    int ready_ret = ready_for_transfer();
     if (ready_ret != 0) return ready_ret;
     HipMat src = blob;
     if (src.narrow())

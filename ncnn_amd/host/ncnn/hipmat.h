@@ -133,7 +133,7 @@ public:
 
     // Host Mat (planar, any batch) -> device blob and back.  An upload has left src's memory when it returns (it goes through
     // page-locked staging buffers of this command); the device blob is ready in stream order, and for a command whose blobs
-    // cross streams when the call returns.  download synchronises the stream.
+    // cross streams when the call returns.  download synchronises the stream.  While the stream is being captured both fail.
     int upload(const Mat& src, HipMat& dst);
     int upload_into(const Mat& src, HipMat& dst); // dst exists and has src's shape: new values for the same buffer
     int widen(const HipMat& src, HipMat& dst);    // narrow blob -> ordinary 16-channel-padded blob (enqueued, not waited for)
@@ -164,6 +164,7 @@ private:
     int next_stage;
     Stage* take_stage();
     int mark_stage(Stage* s);
+    int ready_for_transfer(); // ensure_ready, and an error while the stream is being captured
     int upload_planes(const Mat& src, HipMat& dst);
     int upload_samples(const Mat& src, HipMat& dst);
     std::shared_ptr<HipPool> pool;

@@ -44,3 +44,39 @@ def test_a_host_array_may_be_reused_once_it_was_fed():
     second.input("data", x)
     x[:] = 0
     assert np.array_equal(first.extract("fc"), want_a) and np.array_equal(second.extract("fc"), want_b)
+
+
+def test_a_pass_with_a_host_source_layer_cannot_be_recorded():
+    """A blob made on the host has to be uploaded in the middle of the pass: run eagerly, refused by a recording, and the
+    net works on afterwards (what a replay would do to it: tests/test_device_queue.py)."""
+    from ncnn_amd import host, modelwriter as mw
+    L = host.lib()
+    source = np.arange(-4, 8, dtype=np.float32).reshape(3, 4)
+    keep = []
+
+    def creator():
+        layer = L.ncnn_layer_create()
+        L.ncnn_layer_set_one_blob_only(layer, 0)
+
+        def forward_n(self, bottoms, n, tops, n2, opt):
+            m = host.Mat.from_numpy(source)
+            tops[0] = m.h_
+            m.h_ = None
+            return 0
+        keep.append(host.LayerTable._fields_[6][1](forward_n))
+        layer.contents.forward_n = keep[-1]
+        return layer
+    net = host.Net()
+    net.set_use_hip_compute(True)
+    net.register_custom_layer("Source", creator, lambda layer: L.ncnn_layer_destroy(layer))
+    lines = ["Input in0 0 1 data", "Source s 0 1 src", "ReLU r 1 1 src out"]
+    assert net.load_param_mem(mw.assemble_param(lines)) == 0 and net.load_model_mem(b"") == 0
+    x = np.ones((3, 4), np.float32)
+    blob = net.upload(x)
+    for _ in range(4):
+        assert np.array_equal(net.create_extractor().extract("out"), np.maximum(source, 0))
+    for output in ("out", "src"):
+        with pytest.raises(RuntimeError):
+            net.record("data", blob, output)
+    assert np.array_equal(net.create_extractor().extract("out"), np.maximum(source, 0))
+    assert np.array_equal(blob.to_numpy(), x)
