@@ -18,9 +18,9 @@ static int hip_status(int rc, const char* where)
 
 // ---- HipMat -----------------------------------------------------------------------------------
 
-HipMat::HipMat() : data(0), refcount(0), dims(0), w(0), h(0), c(0), n(0), cp(0), elemsize(0), q8_scale(0.f) {}
+HipMat::HipMat() : data(0), refcount(0), dims(0), w(0), h(0), c(0), n(0), cp(0), elemsize(0), q8_scale(0.f), uploaded(false) {}
 
-HipMat::HipMat(const HipMat& m) : data(m.data), refcount(m.refcount), pool(m.pool), dims(m.dims), w(m.w), h(m.h), c(m.c), n(m.n), cp(m.cp), elemsize(m.elemsize), q8(m.q8), q8_scale(m.q8_scale)
+HipMat::HipMat(const HipMat& m) : data(m.data), refcount(m.refcount), pool(m.pool), dims(m.dims), w(m.w), h(m.h), c(m.c), n(m.n), cp(m.cp), elemsize(m.elemsize), q8(m.q8), q8_scale(m.q8_scale), uploaded(m.uploaded)
 {
     if (refcount) __sync_fetch_and_add(refcount, 1);
 }
@@ -47,6 +47,7 @@ HipMat& HipMat::operator=(const HipMat& m)
     elemsize = m.elemsize;
     q8 = m.q8;
     q8_scale = m.q8_scale;
+    uploaded = m.uploaded;
     return *this;
 }
 
@@ -64,6 +65,7 @@ void HipMat::release()
     elemsize = 0;
     q8.reset();
     q8_scale = 0.f;
+    uploaded = false;
 }
 
 void HipMat::allocate(HipCommand* command)
@@ -388,7 +390,21 @@ int HipCommand::upload(const Mat& src, HipMat& dst)
     else
         dst.create(src.w, src.h, src.elemsize, src.n, this);
     if (dst.empty()) return -100;
-    return upload_into(src, dst);
+    ret = upload_into(src, dst);
+    dst.uploaded = ret == 0 && !cross_streams;
+    return ret;
+}
+
+int HipCommand::wait_for_uploads()
+{
+    for (int i = 0; i < STAGES; i++)
+    {
+        if (!stages[i].pending) continue;
+        const int rc = ncnnhip_event_synchronize(stages[i].event);
+        if (rc != 0) return hip_status(rc, "ncnnhip_event_synchronize");
+        stages[i].pending = false;
+    }
+    return 0;
 }
 
 int HipCommand::upload_into(const Mat& src, HipMat& dst)

@@ -107,6 +107,8 @@ public:
     // had its producer emit float2int8(value * q8_scale) directly because every consumer would quantise it so.
     std::shared_ptr<HipMat> q8;
     float q8_scale;
+    // an upload wrote the buffer and may still be on its way (HipCommand::wait_for_uploads); handles to it inherit this
+    bool uploaded;
 
 private:
     void allocate(HipCommand* cmd);
@@ -137,6 +139,7 @@ public:
     int upload(const Mat& src, HipMat& dst);
     int upload_into(const Mat& src, HipMat& dst); // dst exists and has src's shape: new values for the same buffer
     int widen(const HipMat& src, HipMat& dst);    // narrow blob -> ordinary 16-channel-padded blob (enqueued, not waited for)
+    int wait_for_uploads(); // until every upload of this command has arrived, not for the work behind them
     int download(const HipMat& src, Mat& dst, Allocator* allocator);
     int synchronize();
 

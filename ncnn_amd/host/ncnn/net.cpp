@@ -647,7 +647,7 @@ int NetPrivate::forward_layer(int layer_index, ExecState& st, const Option& opt)
 }
 
 // A layer with forward_hip: inputs are made device-resident (uploaded once if they only exist on the host), the
-// outputs stay in HBM.  Nothing here waits for the GPU; only an upload out of pageable memory does.
+// outputs stay in HBM.  Nothing here waits for the GPU; an upload waits only for the staging buffer it is about to fill.
 int NetPrivate::run_layer_hip(const Layer* layer, ExecState& st, const Option& opt) const
 {
     if (!st.cmd) st.cmd = acquire_command();
@@ -1510,6 +1510,8 @@ int Extractor::extract(int blob_index, HipMat& feat)
         if (!d->st.cmd) d->st.cmd = d->net->d->acquire_command();
         ret = d->st.cmd->upload(d->st.host[bi], d->st.dev[bi]);
     }
+    // what was not computed here but brought from the host is ready on any stream when it is handed out
+    if (ret == 0 && d->st.dev[bi].uploaded && d->st.cmd) ret = d->st.cmd->wait_for_uploads();
     feat = d->st.dev[bi];
     return ret;
 }

@@ -101,7 +101,8 @@ public:
     int extract(int blob_index, Mat& feat, int type = 0);
 
     // device-resident ends of the pipeline (the VkMat overloads of src/net.h:226-239): a blob that is already in
-    // HBM goes in without a copy; extract enqueues the work and hands back the blob where it lies, without waiting.
+    // HBM goes in without a copy; extract enqueues the work and hands back the blob where it lies, without waiting for the
+    // device (a blob that no device layer computed, only brought over from the host, has arrived on return).
     // synchronize() waits for everything this Extractor has enqueued.
     int input(const char* blob_name, const HipMat& in);
     int input(int blob_index, const HipMat& in);

@@ -151,7 +151,13 @@ int ncnnhip_event_synchronize(void* e)
 {
     Event* event = (Event*)e;
     if (event->captured) return -1;
-    return !event->passed || *event->passed ? 0 : run(event->stream);
+    while (event->passed && !*event->passed) // up to the event, not what lies behind it
+    {
+        Op op = event->stream->ops.front();
+        event->stream->ops.pop_front();
+        op();
+    }
+    return 0;
 }
 int ncnnhip_copy(void* dst, const void* src, size_t bytes, void* s)
 {
@@ -164,6 +170,17 @@ int ncnnhip_memcpy_h2d(void* dst, const void* src, size_t bytes, void* s)
     // pageable memory has been read when the call returns
     std::vector<unsigned char> held((const unsigned char*)src, (const unsigned char*)src + bytes);
     return enqueue(s, [=] { memcpy(dst, held.data(), bytes); });
+}
+int ncnnhip_chw_to_nhwc(const void* src, int elemsize, int c, int hw, int batch, size_t cstep, size_t nstep, void* dst, void* s)
+{
+    const int cp = (c + 15) / 16 * 16;
+    return enqueue(s, [=] {
+        memset(dst, 0, (size_t)batch * hw * cp * elemsize);
+        for (int b = 0; b < batch; b++)
+            for (int i = 0; i < hw; i++)
+                for (int q = 0; q < c; q++)
+                    memcpy((char*)dst + (((size_t)b * hw + i) * cp + q) * elemsize, (const char*)src + (nstep * b + cstep * q + i) * elemsize, elemsize);
+    });
 }
 int ncnnhip_relu(const void* src, void* dst, int elemsize, size_t count, float, void* s)
 {

@@ -87,3 +87,20 @@ assert np.array_equal(net.upload(x).to_numpy(), x)  # and the net still works
 ex = net.create_extractor()
 assert np.array_equal(ex.extract("out"), np.maximum(source, 0))
 ''' % {"output": output})
+
+
+def test_a_resident_blob_that_came_from_the_host_is_ready_on_return(child):
+    """Another Extractor may read it at once, on its own stream: a host layer's blob, and an input handed back.  A device
+    layer's result is handed back without waiting, as ever."""
+    child(r'''
+net = net_with(["Input in0 0 1 data", "ReLU r0 1 1 data out0", "Source s 0 1 src", "Split sp 1 2 src a b", "ReLU r1 1 1 a out1"])
+for name in ("src", "data", "b"):
+    ex = net.create_extractor()
+    ex.input("data", np.ones((8, 6, 6), F))
+    blob = ex.extract_resident(name)
+    assert fake.fake_pending() == 0, name
+ex = net.create_extractor()
+ex.input("data", np.ones((8, 6, 6), F))
+out = ex.extract_resident("out0")
+assert fake.fake_pending() > 0
+''')
