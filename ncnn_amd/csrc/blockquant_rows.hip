@@ -85,7 +85,7 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void blockquant_rows_f16_kerne
     auto issue = [&](int s, int slot) {
         unsigned char* st = ring + slot * STAGE;
         const int k0 = (step0 + s) * 64 + chunk0 * 8, k1 = (step0 + s) * 64 + (chunk0 ^ 4) * 8;
-        const int c0 = k0 < K ? k0 : 0, c1 = k1 < K ? k1 : 0; // K % 16 == 0; beyond it the weights are zero
+        const int c0 = k0 < K ? k0 : 0, c1 = k1 < K ? k1 : 0; // K % 16 == 0: a chunk is all in or all out; one beyond K is dropped after it was read
 #pragma unroll
         for (int i = 0; i < MG * 2; i++)
             __builtin_amdgcn_global_load_lds((const AS1 void*)(arow[i] + (i & 1 ? c1 : c0)), (AS3 void*)(st + i * 1024), 16, 0, 0);
@@ -159,6 +159,17 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void blockquant_rows_f16_kerne
         }
 #pragma unroll
         for (int g = 0; g < MG; g++) asm volatile("" : "+v"(xa[g].i4), "+v"(xb[g].i4));
+        if ((step0 + s) * 64 + 64 > K)
+        {
+            // the step K ends in: zeros for the chunks beyond it (their weights are zero, but zero times an infinity is not)
+            const int ka = (step0 + s) * 64 + kg * (HALVES ? 8 : 16), kb = ka + (HALVES ? 32 : 8);
+#pragma unroll
+            for (int g = 0; g < MG; g++)
+            {
+                if (ka >= K) xa[g].i4 = v4i_bq{0, 0, 0, 0};
+                if (kb >= K) xb[g].i4 = v4i_bq{0, 0, 0, 0};
+            }
+        }
 #pragma unroll
         for (int rt = 0; rt < RT; rt++)
         {

@@ -41,6 +41,25 @@ def test_few_fp16_rows_of_large_weights(rt, m, n, k, bits, block):
     test_many_fp16_rows(rt, m, n, k, bits, block)
 
 
+@pytest.mark.parametrize("m,n,k", [(20, 33, 80), (40, 16, 528), (66, 200, 1072), (17, 20, 48), (9, 20, 9168), (16, 4100, 9200)])
+@pytest.mark.parametrize("bits,block", [(8, 64), (8, 32), (6, 64), (4, 32), (4, 128)])
+def test_an_infinity_stays_an_infinity(rt, m, n, k, bits, block):
+    """K ends inside a step of 64: what is read in place of the values beyond K is the start of the row, and must not count.
+    With no other special value and no zero weight in its column, an infinite activation gives infinities and no NaN."""
+    print("[case]", m, n, k, bits, block, flush=True)
+    a, packed, scales = synth.blockquant_operands(m + n + k, m, n, k, bits, block)
+    a = a.astype(np.float16)
+    a[0, 0], a[1, 7], a[2, k - 1] = np.inf, -np.inf, np.inf
+    with np.errstate(invalid="ignore"):
+        want = oracle.gemm_blockquant(a.astype(F), packed, scales, bits, block)
+    pw, pd = rt.blockquant_pack(packed, scales, block, bits=bits, k=k)
+    got = rt.gemm_blockquant_packed(a, pw, pd, n, bits=bits, block=block)
+    assert np.array_equal(np.isnan(got[:3]), np.isnan(want[:3])) and np.isinf(want[:3]).any()
+    inf = np.isinf(want[:3])
+    assert np.array_equal(got[:3][inf], want[:3][inf])
+    _check(got[3:], a[3:].astype(F), packed, scales, bits, block)
+
+
 @pytest.mark.parametrize("m", [17, 40, 100])
 def test_several_matrices_in_one_call(rt, m):
     k, ns = 192, (50, 16, 700)
