@@ -60,6 +60,7 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void blockquant_rows_f16_kerne
 
     // this wavefront's K steps
     const int step0 = (int)((long long)kblocks * wave / nwaves), steps = (int)((long long)kblocks * (wave + 1) / nwaves) - step0;
+    const int ragged = (K & 63) ? kblocks - 1 - step0 : -1; // the step K ends in (the last wavefront's; beyond the others' steps)
 
     // sources.  Activations: load i brings rows i * 8 .. + 8 of the pass, lane l row l / 8 and the chunk that belongs at position l % 8
     const __half* arow[MG * 2];
@@ -85,7 +86,7 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void blockquant_rows_f16_kerne
     auto issue = [&](int s, int slot) {
         unsigned char* st = ring + slot * STAGE;
         const int k0 = (step0 + s) * 64 + chunk0 * 8, k1 = (step0 + s) * 64 + (chunk0 ^ 4) * 8;
-        const int c0 = k0 < K ? k0 : 0, c1 = k1 < K ? k1 : 0; // K % 16 == 0: a chunk is all in or all out; one beyond K is dropped after it was read
+        const int c0 = k0 < K ? k0 : 0, c1 = k1 < K ? k1 : 0; // K % 16 == 0: a chunk is all in or all out
 #pragma unroll
         for (int i = 0; i < MG * 2; i++)
             __builtin_amdgcn_global_load_lds((const AS1 void*)(arow[i] + (i & 1 ? c1 : c0)), (AS3 void*)(st + i * 1024), 16, 0, 0);
@@ -117,6 +118,15 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void blockquant_rows_f16_kerne
         issue(s + 1 < steps ? s + 1 : s, (s + 1) & 1);
         WAIT_VMCNT(LOADS);
         asm volatile("" ::: "memory");
+        if (s == ragged)
+        {
+            // zeros in place of the chunks beyond K: their weights are zero, but zero times an infinity is not
+            const v4i_bq zeros = {0, 0, 0, 0};
+            const int k0 = (step0 + s) * 64 + chunk0 * 8, k1 = (step0 + s) * 64 + (chunk0 ^ 4) * 8;
+#pragma unroll
+            for (int i = 0; i < MG * 2; i++)
+                if ((i & 1 ? k1 : k0) >= K) asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(base + at + lane * 16), "v"(zeros), "n"(i * 1024) : "memory");
+        }
         // LDS is read with hand-written instructions and waits: the compiler takes a direct-to-LDS load for a store to all of LDS
         // and would wait for everything in flight in front of each read it emits itself.
         v4i_bq wq[RT], dq0[RT], dq1[RT];
@@ -159,17 +169,6 @@ __global__ __launch_bounds__(ROWS_MAX_WAVES * 64) void blockquant_rows_f16_kerne
         }
 #pragma unroll
         for (int g = 0; g < MG; g++) asm volatile("" : "+v"(xa[g].i4), "+v"(xb[g].i4));
-        if ((step0 + s) * 64 + 64 > K)
-        {
-            // the step K ends in: zeros for the chunks beyond it (their weights are zero, but zero times an infinity is not)
-            const int ka = (step0 + s) * 64 + kg * (HALVES ? 8 : 16), kb = ka + (HALVES ? 32 : 8);
-#pragma unroll
-            for (int g = 0; g < MG; g++)
-            {
-                if (ka >= K) xa[g].i4 = v4i_bq{0, 0, 0, 0};
-                if (kb >= K) xb[g].i4 = v4i_bq{0, 0, 0, 0};
-            }
-        }
 #pragma unroll
         for (int rt = 0; rt < RT; rt++)
         {
