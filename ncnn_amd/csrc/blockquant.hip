@@ -542,8 +542,8 @@ __global__ __launch_bounds__(256) void blockquant8_mfma_kernel(const __half* __r
     const int Kp = kblocks * 64;
     const __half* lds_act = reinterpret_cast<const __half*>(lds_d + (size_t)kblocks * 4) + (size_t)(m < M ? m : 0) * Kp + kg * 16;
     // Every load is unconditional (a guarded load becomes a branch, and after a branch the compiler waits for ALL loads in
-    // flight, which empties the ring every step): a batch beyond the range re-reads the wave's first block and is cancelled
-    // by a zero descale; a lane whose 16-half chunk lies beyond K (only when K % 64 != 0) reads chunk 0 and selects zeros;
+    // flight, which empties the ring every step): a batch beyond the range re-reads the wave's first block and its sums
+    // are not taken over; a lane whose 16-half chunk lies beyond K (only when K % 64 != 0) reads chunk 0 and selects zeros;
     // lanes of activation rows >= M read row 0 and their results are never stored.
     auto load_batch = [&](int kb0, Batch& bt_) {
 #pragma unroll
@@ -601,8 +601,9 @@ __global__ __launch_bounds__(256) void blockquant8_mfma_kernel(const __half* __r
             v4f t = {0.f, 0.f, 0.f, 0.f};
             t = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa, xa.h, t, 0, 0, 0);
             t = __builtin_amdgcn_mfma_f32_16x16x32_f16(wb, xb.h, t, 0, 0, 0);
-            float4 d = lds_d[kb * 4 + kg];
-            if (!live) d = make_float4(0.f, 0.f, 0.f, 0.f); // a select, not a branch
+            const float4 d = lds_d[kb * 4 + kg];
+#pragma unroll
+            for (int r = 0; r < 4; r++) t[r] = live ? t[r] : 0.f; // a select, not a branch (and not a zero descale: t may be infinite)
             acc[0] = fmaf(t[0], d.x, acc[0]);
             acc[1] = fmaf(t[1], d.y, acc[1]);
             acc[2] = fmaf(t[2], d.z, acc[2]);
@@ -665,6 +666,18 @@ __global__ __launch_bounds__(256) void blockquant8_mfma_kernel(const __half* __r
     }
 }
 
+// What was read in place of activations that do not exist must not count: it meets weights or a descale of zero, but zero times an
+// infinity is not zero.
+__device__ __forceinline__ void drop_beyond(v4i_bq& a, v4i_bq& b, bool there)
+{
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+    {
+        a[e] = there ? a[e] : 0;
+        b[e] = there ? b[e] : 0;
+    }
+}
+
 // ---- the same contraction with every weight byte of a wavefront requested before the first one is used ----
 // A bandwidth kernel on this chip is paced by the bytes it has in flight: 8 TB/s times a microsecond of memory latency is
 // 8 MB, 32 KB per compute unit, and a matrix of 4096 rows is only 64 KB per compute unit in all.  So a workgroup still owns
@@ -682,6 +695,8 @@ __global__ __launch_bounds__(256) void blockquant8_mfma_kernel(const __half* __r
 //   operand mapping a 16-lane group touches 16 rows, 16 cache lines for 256 bytes, and the loads took four times the
 //   weight stream's share of the L1 pipe), and are turned into the operand mapping through 2.25 KB of LDS per wavefront
 //   when the block is multiplied.
+//   WHOLE: every wavefront has NB blocks and K ends with the last; else what does not exist is dropped (drop_beyond), which costs 4 %
+//   where it is not needed (8 x 4096 x 4096 6.1 -> 6.4 us, 8 x 12288 x 4096 11.9 -> 12.4).
 // BITS / HALVES: the packed layouts of ncnnhip_blockquant_pack.  HALVES = false is the 8-bit layout for quantisation
 // blocks of 64 or 128 (a lane's 16 weights are 16 consecutive K, one descale per 64).  HALVES = true serves 4- and 6-bit
 // fields and blocks of 32: the first matrix-core instruction of a 64-wide step covers K 0..31 and the second K 32..63
@@ -694,7 +709,7 @@ __global__ __launch_bounds__(256) void blockquant8_mfma_kernel(const __half* __r
 // bf16 (integers up to 128 are exact there).  Every
 // product is then the exact q * a of the reference and only the order of the fp32 additions differs, as with fp16
 // activations.  (A remainder below 2^-126 is a denormal and may be dropped by the matrix core: |a| < 2^-110 or so.)
-template<int BITS, bool HALVES, int NB, int MAXW, int MT, bool ACT_LDS, int AIN = 2, bool INSC = false>
+template<int BITS, bool HALVES, int NB, int MAXW, int MT, bool ACT_LDS, int AIN = 2, bool INSC = false, bool WHOLE = true>
 __global__ __launch_bounds__(MAXW * 64) void blockquant8_upfront_kernel(const void* __restrict__ a_, size_t a_stride, int M, int N_, int K, int kblocks,
                                                                         const unsigned char* __restrict__ wpk_, const float4* __restrict__ dpk_, int split,
                                                                         const float* __restrict__ in_scales, const float* __restrict__ c_, int bt_, float alpha_,
@@ -791,8 +806,8 @@ __global__ __launch_bounds__(MAXW * 64) void blockquant8_upfront_kernel(const vo
     if (HALVES) dreg2 = dt[lane + 64 < nkb * dper ? lane + 64 : 0];
     __builtin_amdgcn_sched_barrier(0);
     // (3) the weights, all of them; !ACT_LDS: each block's activations right behind its weights.  Lane l fetches 16 bytes of
-    // rows l/8 and l/8 + 8, piece l%8 of the block's 128 bytes per row; a chunk beyond K is read from the start of the row
-    // (it meets packed weights that are zero there), rows from M up repeat row 0 (their results are never stored).
+    // rows l/8 and l/8 + 8, piece l%8 of the block's 128 bytes per row; a chunk beyond K is read from the start of the
+    // row and zeroed when the block is multiplied, rows from M up repeat row 0 (their results are never stored).
     const unsigned char* wt = wpk + ((size_t)tile * kblocks + kb_base) * STEP_BYTES;
     v4i_bq w[BITS == 8 ? NB : 1]; // 8-bit: 16 bytes per lane and step
     v2i_bq w2[BITS != 8 ? NB : 1]; // 4-bit: all 8 bytes; 6-bit: the first two of three dwords
@@ -958,6 +973,7 @@ __global__ __launch_bounds__(MAXW * 64) void blockquant8_upfront_kernel(const vo
         {
             // the block's 16 rows x 128 bytes from the fetch mapping into the operand mapping (the wavefront's LDS operations
             // execute in order, so the next block's stores cannot overtake these reads)
+            if (!WHOLE) drop_beyond(a0[ACT_LDS ? 0 : i], a1[ACT_LDS ? 0 : i], i < nkb && (kb_base + i) * 64 + tr_piece * 8 < K);
             *reinterpret_cast<v4i_bq*>(tr_wr) = a0[ACT_LDS ? 0 : i];
             *reinterpret_cast<v4i_bq*>(tr_wr + 8 * TR_PITCH) = a1[ACT_LDS ? 0 : i];
             xa.i4 = *reinterpret_cast<const v4i_bq*>(act_rd);
@@ -1045,7 +1061,7 @@ __global__ __launch_bounds__(MAXW * 64) void blockquant8_upfront_kernel(const vo
 // The 5-to-16-row form for many weight rows: one workgroup takes TWO neighbouring tiles of 16 weight rows and multiplies both
 // with the same activation registers.  A tile's 64 KB of weights at K = 4096 come with 128 KB of activations through the same
 // L1; sharing them between two tiles takes that from 192 to 128 KB per tile (fp16 activations, K up to 4096).
-template<int BITS, bool HALVES, int NB, int MAXW>
+template<int BITS, bool HALVES, int NB, int MAXW, bool WHOLE>
 __global__ __launch_bounds__(MAXW * 64) void blockquant8_rows16_pair_kernel(const __half* __restrict__ a, size_t a_stride, int M, int N, int K, int kblocks,
                                                                             int ntiles, const unsigned char* __restrict__ wpk, const float4* __restrict__ dpk,
                                                                             int split, const float* __restrict__ c, int bt, float alpha, float beta,
@@ -1137,6 +1153,7 @@ __global__ __launch_bounds__(MAXW * 64) void blockquant8_rows16_pair_kernel(cons
             v4i_bq i4;
             v8h h;
         } xa, xb;
+        if (!WHOLE) drop_beyond(a0[i], a1[i], i < nkb && (kb_base + i) * 64 + tr_piece * 8 < K);
         *reinterpret_cast<v4i_bq*>(tr_wr) = a0[i];
         *reinterpret_cast<v4i_bq*>(tr_wr + 8 * TR_PITCH) = a1[i];
         xa.i4 = *reinterpret_cast<const v4i_bq*>(act_rd);
@@ -1914,7 +1931,7 @@ __global__ __launch_bounds__(512) void blockquant_rows16_bf16x3_kernel(const uin
         _Pragma("unroll") for (int q = 0; q < 6; q++) fr[slot_][q] = f_[q * 64];           \
     } while (0)
     // requests in the order their data is needed: the first steps' weights and operands interleaved, then the rest of the weights,
-    // then the descales (a step beyond the wavefront's range reads step 0 again and meets a zero descale)
+    // then the descales (a step beyond the wavefront's range reads step 0 again and is not added)
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < WIN; i++)
@@ -1933,14 +1950,8 @@ __global__ __launch_bounds__(512) void blockquant_rows16_bf16x3_kernel(const uin
 #pragma unroll
     for (int i = 0; i < NB; i++)
     {
-        const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-        const float4 a0 = dt[(size_t)(i < nkb ? i : 0) * dper + kg];
-        d0[i] = i < nkb ? a0 : z;
-        if (HALVES)
-        {
-            const float4 a1 = dt[(size_t)(i < nkb ? i : 0) * dper + (split << 2) + kg];
-            d1[HALVES ? i : 0] = i < nkb ? a1 : z;
-        }
+        d0[i] = dt[(size_t)(i < nkb ? i : 0) * dper + kg];
+        if (HALVES) d1[HALVES ? i : 0] = dt[(size_t)(i < nkb ? i : 0) * dper + (split << 2) + kg];
     }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -1982,6 +1993,12 @@ __global__ __launch_bounds__(512) void blockquant_rows16_bf16x3_kernel(const uin
         {
             R16_LOAD_FRAGS(slot, i + WIN);
             __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) // (not a zero descale: the products of step 0 may be infinite)
+        {
+            t0[r] = i < nkb ? t0[r] : 0.f;
+            if (HALVES) t1[r] = i < nkb ? t1[r] : 0.f;
         }
         const float4 da = d0[i];
         if (HALVES)
@@ -2048,6 +2065,7 @@ static int launch_upfront_one(const void* a, size_t a_stride, int M, int N, int 
         return NCNNHIP_OK;
     }
     auto kernel = blockquant8_upfront_kernel<BITS, HALVES, NB, MAXW, MT, ACT_LDS, AIN, INSC>;
+    auto kernel_any = blockquant8_upfront_kernel<BITS, HALVES, NB, MAXW, MT, ACT_LDS, AIN, INSC, ACT_LDS>; // (staged in LDS: dropped there)
     if (lds > 65536)
     {
         // more than the 64 KB a kernel gets by default: raise this kernel's limit once per device (the chip has 160 KB per compute
@@ -2058,14 +2076,15 @@ static int launch_upfront_one(const void* a, size_t a_stride, int M, int N, int 
         if (device < 0 || device >= 64 || !raised[device].load(std::memory_order_acquire))
         {
             NCNNHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            NCNNHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel_any), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
             if (device >= 0 && device < 64) raised[device].store(1, std::memory_order_release);
         }
     }
     BqMulti one;
     one.count = 0;
     const int grid = multi ? multi->tile_end[multi->count - 1] : (N + 15) / 16;
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(nwaves * 64), lds, stream, a, a_stride, M, N, K, kblocks, wpk, dpk, split, in_scales, c, bt, alpha, beta,
-                       out, out_stride, multi ? *multi : one);
+    hipLaunchKernelGGL((K % (64 * NB) == 0 ? kernel : kernel_any), dim3(grid), dim3(nwaves * 64), lds, stream, a, a_stride, M, N, K, kblocks, wpk, dpk, split, in_scales, c,
+                       bt, alpha, beta, out, out_stride, multi ? *multi : one);
     return launch_status("blockquant8_upfront_kernel");
 }
 
@@ -2134,8 +2153,9 @@ static int launch_blockquant8_upfront(const void* a, size_t a_stride, int M, int
             // many weight rows: two tiles per workgroup share the activation registers
             const int nwaves = (kblocks + 7) / 8;
             const size_t lds = (size_t)nwaves * (2 * (HALVES ? 1024 << split : 1024) + 16 * 144);
-            hipLaunchKernelGGL((blockquant8_rows16_pair_kernel<BITS, HALVES, 8, 8>), dim3((ntiles + 1) / 2), dim3(nwaves * 64), lds, stream,
-                               static_cast<const __half*>(a), a_stride, M, N, K, kblocks, ntiles, wpk, dpk, split, c, bt, alpha, beta, out, out_stride);
+            auto kernel = K % 512 == 0 ? blockquant8_rows16_pair_kernel<BITS, HALVES, 8, 8, true> : blockquant8_rows16_pair_kernel<BITS, HALVES, 8, 8, false>;
+            hipLaunchKernelGGL(kernel, dim3((ntiles + 1) / 2), dim3(nwaves * 64), lds, stream, static_cast<const __half*>(a), a_stride, M, N, K, kblocks, ntiles, wpk, dpk,
+                               split, c, bt, alpha, beta, out, out_stride);
             return launch_status("blockquant8_rows16_pair_kernel");
         }
         if (kblocks <= 64) UPFRONT(8, 8, 1, false);

@@ -41,10 +41,12 @@ def test_few_fp16_rows_of_large_weights(rt, m, n, k, bits, block):
     test_many_fp16_rows(rt, m, n, k, bits, block)
 
 
-@pytest.mark.parametrize("m,n,k", [(20, 33, 80), (40, 16, 528), (66, 200, 1072), (17, 20, 48), (9, 20, 9168), (16, 4100, 9200)])
+@pytest.mark.parametrize("m,n,k", [(20, 33, 80), (40, 16, 528), (66, 200, 1072), (17, 20, 48), (9, 20, 9168), (16, 4100, 9200),
+                                   (3, 20, 80), (5, 16, 192), (9, 40, 1072), (9, 4100, 1072), (16, 20, 4112), (5, 20, 8208), (9, 8200, 8208), (3, 8200, 9200)])
 @pytest.mark.parametrize("bits,block", [(8, 64), (8, 32), (6, 64), (4, 32), (4, 128)])
 def test_an_infinity_stays_an_infinity(rt, m, n, k, bits, block):
-    """K ends inside a step of 64: what is read in place of the values beyond K is the start of the row, and must not count.
+    """K ends inside a step of 64, or a wavefront has fewer steps than its neighbours: what is read in place of the values beyond
+    its share is the start of the row or of the share, and must not count.
     With no other special value and no zero weight in its column, an infinite activation gives infinities and no NaN."""
     print("[case]", m, n, k, bits, block, flush=True)
     a, packed, scales = synth.blockquant_operands(m + n + k, m, n, k, bits, block)
@@ -82,3 +84,20 @@ def test_many_fp32_rows(rt, m, n, k, bits, block):
     pw, pd = rt.blockquant_pack(packed, scales, block, bits=bits, k=k)
     got = rt.gemm_blockquant_packed(a, pw, pd, n, c, 3, 0.75, 1.5, bits=bits, block=block, rows_kernel=True)
     _check(got, a, packed, scales, bits, block, c, 3, 0.75, 1.5)
+
+
+@pytest.mark.parametrize("m,n,k,rows", [(1, 33, 80, False), (4, 20, 528, False), (9, 16, 1072, False), (5, 20, 80, True), (20, 33, 1072, True), (40, 16, 8208, True),
+                                        (70, 200, 528, True), (200, 1000, 1040, True)])
+@pytest.mark.parametrize("bits,block", [(8, 64), (8, 32), (6, 64), (4, 32)])
+def test_an_infinity_stays_an_infinity_fp32(rt, m, n, k, rows, bits, block):
+    """The same for fp32 rows: the one-pass form, the 16-row passes and the tiles of 64 rows."""
+    print("[case]", m, n, k, rows, bits, block, flush=True)
+    a, packed, scales = synth.blockquant_operands(m + n + k, m, n, k, bits, block, half_exact=False)
+    a[0, 0], a[m // 2, k - 1] = np.inf, -np.inf
+    with np.errstate(invalid="ignore"):
+        want = oracle.gemm_blockquant(a, packed, scales, bits, block)
+    pw, pd = rt.blockquant_pack(packed, scales, block, bits=bits, k=k)
+    got = rt.gemm_blockquant_packed(a, pw, pd, n, bits=bits, block=block, **({"rows_kernel": True} if rows else {}))
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isinf(want).any()
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf])
