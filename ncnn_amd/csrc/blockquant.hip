@@ -2395,7 +2395,22 @@ static int gemm_blockquant_packed(const char* who, const void* a_dev, int ain, s
 #undef UP_BITS
 #undef UP
     };
-    const int pass = ain == 4 ? 4 : 16; // rows per pass at most
+    if (ain == 2 && !halves)
+    {
+        bool handled = false; // (16 rows at most: many_rows_f16 has taken the others)
+        const int ret = upfront(0, M, &handled);
+        if (ret != NCNNHIP_OK || handled) return ret;
+        const __half* ah = static_cast<const __half*>(a_dev);
+        const size_t act_bytes = (size_t)M * kblocks * 64 * sizeof(__half);
+        if (act_bytes <= 32768 && tiles >= 512) // measured: pays from about 8192 weight rows (up to four rows of 4096), not for long rows (K = 11008) or few tiles
+            hipLaunchKernelGGL((blockquant8_mfma_kernel<BQ_MFMA_NS_LDS, 1, true>), dim3(tiles), dim3(256), (size_t)kblocks * 64 + act_bytes, st, ah, a_stride, M, N, K,
+                               kblocks, reinterpret_cast<const v4i_bq*>(packed_w_dev), dpk, c_dev, bt, alpha, beta, out_dev, out_stride);
+        else
+            hipLaunchKernelGGL((blockquant8_mfma_kernel<BQ_MFMA_NS, BQ_MFMA_U, false>), dim3(tiles), dim3(256), (size_t)kblocks * 64, st, ah, a_stride, M, N, K, kblocks,
+                               reinterpret_cast<const v4i_bq*>(packed_w_dev), dpk, c_dev, bt, alpha, beta, out_dev, out_stride);
+        return launch_status("blockquant8_mfma_kernel");
+    }
+    const int pass = ain == 4 ? 4 : M;
     for (int m0 = 0; m0 < M; m0 += pass)
     {
         const int mc = M - m0 < pass ? M - m0 : pass;
@@ -2403,39 +2418,22 @@ static int gemm_blockquant_packed(const char* who, const void* a_dev, int ain, s
         int ret = upfront(m0, mc, &handled);
         if (ret != NCNNHIP_OK) return ret;
         if (handled) continue;
-        if (halves || ain == 4)
+        // rows that do not fit in LDS together (long K; fp32: three planes per row): four, two, one at a time
+        for (int m1 = m0; m1 < m0 + mc;)
         {
-            // rows that do not fit in LDS together (long K; fp32: three planes per row): four, two, one at a time
-            for (int m1 = m0; m1 < m0 + mc;)
+            int rows = m0 + mc - m1 < 4 ? m0 + mc - m1 : 4;
+            for (;;)
             {
-                int rows = m0 + mc - m1 < 4 ? m0 + mc - m1 : 4;
-                for (;;)
-                {
-                    ret = upfront(m1, rows, &handled);
-                    if (ret != NCNNHIP_OK) return ret;
-                    if (handled || rows == 1) break;
-                    rows = rows > 2 ? 2 : 1;
-                }
-                NCNNHIP_REQUIRE(handled, "%s: no kernel for M %d K %d", who, M, K);
-                m1 += rows;
+                ret = upfront(m1, rows, &handled);
+                if (ret != NCNNHIP_OK) return ret;
+                if (handled || rows == 1) break;
+                rows = rows > 2 ? 2 : 1;
             }
-            continue;
+            NCNNHIP_REQUIRE(handled, "%s: no kernel for M %d K %d", who, M, K);
+            m1 += rows;
         }
-        const __half* ah = static_cast<const __half*>(a_dev);
-        const float* cc = c_dev;
-        if (cc && (bt == 1 || bt == 2)) cc += m0;
-        if (cc && bt == 3) cc += (size_t)m0 * N;
-        const size_t act_bytes = (size_t)mc * kblocks * 64 * sizeof(__half);
-        if (act_bytes <= 32768 && tiles >= 512) // measured: pays from about 8192 weight rows (up to four rows of 4096), not for long rows (K = 11008) or few tiles
-            hipLaunchKernelGGL((blockquant8_mfma_kernel<BQ_MFMA_NS_LDS, 1, true>), dim3(tiles), dim3(256), (size_t)kblocks * 64 + act_bytes, st,
-                               ah + (size_t)m0 * a_stride, a_stride, mc, N, K, kblocks, reinterpret_cast<const v4i_bq*>(packed_w_dev), dpk, cc, bt, alpha, beta,
-                               out_dev + (size_t)m0 * out_stride, out_stride);
-        else
-            hipLaunchKernelGGL((blockquant8_mfma_kernel<BQ_MFMA_NS, BQ_MFMA_U, false>), dim3(tiles), dim3(256), (size_t)kblocks * 64, st,
-                               ah + (size_t)m0 * a_stride, a_stride, mc, N, K, kblocks, reinterpret_cast<const v4i_bq*>(packed_w_dev), dpk, cc, bt, alpha, beta,
-                               out_dev + (size_t)m0 * out_stride, out_stride);
     }
-    return launch_status("blockquant8_mfma_kernel");
+    return NCNNHIP_OK;
 }
 
 int ncnnhip_gemm_blockquant_packed_f16a(const uint16_t* a_dev, size_t a_stride, int M, int N, int K, const uint8_t* packed_w_dev,

@@ -133,8 +133,9 @@ __global__ __launch_bounds__(256) void gemm_skinny_int8_kernel(const int8_t* __r
     }
 }
 
-// InnerProduct on 2 to 48 rows (a batch through the classifier of a net): the same kernel with InnerProduct's epilogue, under the
-// same estimate as Gemm's.  false: the shape is not one it takes.
+// InnerProduct on 2 to 48 rows (a batch through the classifier of a net): the same kernel with InnerProduct's epilogue, above 16 rows
+// under an estimate like Gemm's, against about 4 us + K / 300 for the convolution's kernel (ncnnhip_innerproduct_int8_ws).  false: the
+// shape is not one it takes.
 static bool launch_fc_skinny(const int8_t* x_dev, size_t x_stride, int rows, int num_input, int num_output, const int8_t* weight_dev, const FcEpilogue& epi,
                              hipStream_t stream);
 
