@@ -54,16 +54,24 @@ PipePlan plan_pipelined_groups(int cout, long long npix, int steps)
     // step's loads in turn; sixteen have four steps under way.  us, four wavefronts -> sixteen, one layer alone:
     //   1x1 1024 -> 256 on 14x14: batch 1 6.3 -> 5.6, batch 16 6.5 -> 5.9    1x1 2048 -> 512 on 7x7: 8.2 -> 7.2, batch 16 9.3 -> 7.4
     //   1x1 960 -> 160 on 7x7 6.0 -> 5.2    3x3 256 -> 256 on 14x14, batch 16 11.4 -> 8.7    3x3 512 -> 512 on 7x7, batch 16 12.7 -> 11.5
-    // Eight wavefronts gain about half of that.  392 tiles (3x3 128 -> 128 on 28x28, batch 16) share units already: the pass was
-    // 2 % slower with sixteen.  Below 8 steps there is too little to share.
+    // Eight wavefronts gain about half of that.  The lines, from 1x1 and 3x3 layers of 8 to 100 steps on 2 to 441 tiles:
+    //   beyond 256 tiles two of them share a unit and sixteen lose: 24 steps, 196 tiles 10.1 -> 7.2, 320 tiles 9.1 -> 12.2; 72 steps
+    //   196 tiles 16.2 -> 13.5, 320 tiles 20.9 -> 24.6;
+    //   with 8 and 9 steps they are up to 3 % slower alone (75 tiles 4.76 -> 4.84 and 4.94 -> 5.05), from 11 on faster (5.55 -> 5.42 at
+    //   12); the nets' passes, which have those layers too, were no slower with them.
     if (p.bm != 64 || p.bn != 64 || steps < 8 || t > 256) return p;
-    // A few tiles of a long K want other compute units more than wavefronts of their own: 3x3 256 -> 256 on 14x14, batch 1
-    // (16 tiles) 8.1 in three splits and 8.5 in one with sixteen wavefronts, 512 -> 512 on 7x7 (8 tiles) 9.4 and 9.6.
+    // A few tiles of a long K want other compute units more than wavefronts of their own.  Four wavefronts in splits / sixteen in one:
+    // 3x3 of 36 steps 16 tiles 8.2 / 8.5, 52 tiles 8.9 / 8.7; 45 steps 20 tiles 8.8 / 9.6.  (From 72 steps on three splits of sixteen
+    // would be better still: 20 tiles 10.4 -> 10.1, 1x1 of 100 steps 12.0 -> 10.4.)
     if (p.splits >= 3 && t < 24) return p;
     p.groups = 4;
     // K is split over workgroups as well while they fit the chip, at least 24 steps each: 512 -> 512 on 7x7, batch 4 (32 tiles)
-    // 11.0 in six splits of four wavefronts, 10.1 in three of sixteen, 10.8 in four
-    const int room = (int)(256 / t), longest = steps / 24;
+    // 11.0 in six splits of four wavefronts, 10.1 in three of sixteen, 10.8 in four; 1x1 of 100 steps, 52 tiles 14.9 / 12.0 / 11.1 / 11.7
+    // in one to four.  Up to 40 tiles two halves pay from 40 steps on: 3x3 of 41 steps, 28 tiles 9.7 in one, 8.8 in two (9.0 in three
+    // splits of four wavefronts), 1x1 of 46 steps 8.9 and 8.7; with 64 tiles 9.8 and 9.4, 9.2 and 9.3.
+    const int room = (int)(256 / t);
+    int longest = steps / 24;
+    if (longest < 2 && steps >= 40 && t <= 40) longest = 2;
     p.splits = std::max(1, std::min(p.splits, std::min(room, longest)));
     p.steps_per_split = ceil_div(steps, p.splits);
     p.splits = ceil_div(steps, p.steps_per_split);

@@ -22,8 +22,10 @@ SHAPES = [
     ("5x3 of 48 channels (a step meets several taps, K rounded up to 12 steps)", 1, 48, 10, 12, 72, (5, 3), (1, 1), (1, 1), (2, 2, 1, 1)),
     ("3x3 dilated, 18 steps", 1, 128, 12, 10, 128, (3, 3), (2, 2), (1, 1), (2, 2, 2, 2)),
     ("3x3, 36 steps, 52 tiles: one split", 4, 256, 14, 14, 256, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
-    ("3x3, 72 steps, 32 tiles: three splits of uneven groups", 4, 512, 7, 7, 512, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
-    ("1x1, 50 steps, 25 tiles: two splits", 1, 3200, 40, 40, 64, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0)),
+    ("3x3, 72 steps, 32 tiles: three splits", 4, 512, 7, 7, 512, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
+    ("1x1, 50 steps, 25 tiles: two splits of uneven groups", 1, 3200, 40, 40, 64, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0)),
+    ("3x3 of 288 channels, 41 steps, 28 tiles: two splits, 21 steps and 20", 1, 288, 14, 14, 448, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
+    ("1x1, 40 steps, 39 tiles: two splits", 1, 2560, 24, 34, 192, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0)),
 ]
 
 
