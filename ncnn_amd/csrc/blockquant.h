@@ -196,7 +196,8 @@ static inline bool halves_layout(int bits, int block)
     return bits != 8 || block == 32;
 }
 
-// From 17 rows of fp16 activations up (blockquant_rows.hip): every matrix of mm on the same rows, one launch.
+// Many rows of fp16 activations (blockquant_rows.hip; many_rows_f16 in blockquant.hip says from how many: 17 always, 5 on large
+// weights): every matrix of mm on the same rows, one launch.
 int launch_blockquant_rows_f16(const uint16_t* a, size_t a_stride, int M, int K, int bits, int block, const BqMulti& mm, hipStream_t stream);
 
 } // namespace ncnnhip

@@ -9,8 +9,9 @@
 //
 // What bounds it is not the weights but the activations: every workgroup reads all M x K of them (393 KB for 48 rows of 4096)
 // through its unit's L1, so MG and RT balance re-reading them against idle units (launch_blockquant_rows_f16).
-// us per launch against 16 rows per pass, weights from HBM, 4 bits: 4096 x 4096 48 rows 17.9 -> 11.2, 128 rows 48.8 -> 14.4;
-// 11008 x 4096 48 rows 35.4 -> 15.5; 4096 x 11008 48 rows 104 -> 19.4; 8 bits 11008 x 4096 48 rows 40.2 -> 17.6.
+// us per launch, 16 rows per pass -> here, weights from HBM, 4 bits in blocks of 64: 4096 x 4096 24 rows 11.9 -> 8.9, 48 rows 18.4 -> 10.8,
+// 128 rows 45.9 -> 14.6; 11008 x 4096 48 rows 37.3 -> 16.8; 4096 x 11008 48 rows 102 -> 21.5; 8 bits 48 rows 4096 x 4096 20.0 -> 11.3,
+// 11008 x 4096 42.6 -> 19.1, 4096 x 11008 48.0 -> 23.4.
 // A lane must fetch along a row (eight lanes = one 128-byte line) and read in operand order (lane = row), so the chunks of a row
 // are swizzled on the source side: chunk c of row r lands at position c ^ ((r / 2) % 8), conflict-free both ways.
 #include <atomic>
@@ -279,10 +280,12 @@ static int launch_one(const __half* a, size_t a_stride, int M, int K, int passes
 int launch_blockquant_rows_f16(const uint16_t* a_, size_t a_stride, int M, int K, int bits, int block, const BqMulti& mm, hipStream_t stream)
 {
     const __half* a = reinterpret_cast<const __half*>(a_);
-    // Groups of activation rows and tiles per workgroup.  A launch took about 3.7 us + rounds x K / 4096 x (1.8 MG + 1.6 RT) us over
-    // every pair measured (MG and RT 1 to 4, N and K 1024 to 11008, 17 to 128 rows, 4 and 8 bits; one workgroup per unit, 256
-    // units), so the cheapest pair is taken: 48 rows of 4096 x 11008 get 2 x 2 (19.4 us; 3 x 1 23.4),
-    // 11008 x 4096 3 x 3 (15.5 us, 230 workgroups; 3 x 2 are 344, a second round for 88 of them, 22.9).
+    // Groups of activation rows and tiles per workgroup: the cheapest pair under 3.7 us + rounds x K / 4096 x (1.8 MG + 1.6 RT) us (one
+    // workgroup per unit, 256 units).  As a forecast that is rough -- off by 13 % in the median and up to half over every pair of MG 1
+    // to 4 and RT 1, 2, 3, 4, 6 at N and K 1024 to 27648, 24 to 128 rows, 4 and 8 bits, weights from HBM -- but it ranks well: what it
+    // picks took 1 % more than the best pair in the median of those 120 launches, 10 % at most (24 rows of 5120 x 13824 at 4 bits 24.7
+    // us with 2 x 2, 1 x 3 22.4; 100 rows of 1024 x 8192 12.1, 2 x 1 11.2).  48 rows of 11008 x 4096 get 3 x 3: 230 workgroups;
+    // 3 x 2 are 344, a second round for 88 of them.
     const int rows16 = (M + 15) / 16;
     long long tiles = 0;
     for (int i = 0; i < mm.count; i++) tiles += (mm.N[i] + 15) / 16;

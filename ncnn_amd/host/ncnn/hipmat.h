@@ -151,8 +151,10 @@ private:
     friend class HipMat;
     bool ready;
     bool cross_streams; // blobs of this command are read on other streams
-    // Page-locked staging buffers, STAGE_BYTES each, made when first used and given back with the command.  A transfer takes
-    // them in turn; before one is filled again the event recorded behind its last use is waited for.
+    // Page-locked staging buffers, STAGE_BYTES (2 MB) each, made when a transfer first comes round to them and given back with
+    // the command: up to 6 MB for each command, so for each Extractor that was ever alive at the same time as the others, for
+    // the net's uploads, and for each thread that downloads resident blobs, until the net or the thread goes.  A transfer
+    // takes them in turn; before one is filled again the event recorded behind its last use is waited for.
     enum
     {
         STAGES = 3

@@ -6,8 +6,8 @@
 
 namespace ncnn {
 
-// Copies like memcpy.  From a few hundred KB up the bytes are shared out between the calling thread and a few helper threads
-// of the process; a second caller that finds them busy copies alone.
+// Copies like memcpy.  From 1 MB up the bytes are shared out between the calling thread and a few helper threads of the
+// process; a second caller that finds them busy copies alone, and so does a forked child.
 void parallel_copy(void* dst, const void* src, size_t bytes);
 
 } // namespace ncnn
