@@ -260,12 +260,18 @@ class Mat:
         layout = (C.c_size_t * 9)()
         lib().ncnnhip_mat_get_layout(self.h_, C.byref(layout))
         dims, w, h, _, c, n, es, cstep, nstep = layout
+        base = lib().ncnn_mat_get_data(self.h_)
+        if not base or not dims:
+            raise ValueError("an empty Mat has no values")
+        if es not in (1, 4):
+            if dims != 1 or w * es % 4:
+                raise ValueError("a Mat of %d dimensions with elements of %d bytes has no array form" % (dims, es))
+            w, es, nstep = w * es // 4, 4, nstep * es // 4  # a vector of packed or of 2-byte elements: its bytes as fp32
         shape, step = {1: ((w,), (es,)), 2: ((h, w), (w * es, es))}.get(dims, ((c, h, w), (cstep * es, w * es, es)))
         if n > 1:
             shape, step = (n,) + shape, (nstep * es,) + step
-        last = sum((s - 1) * t for s, t in zip(shape, step)) + es if 0 not in shape else 0
-        buf = (C.c_uint8 * max(last, es)).from_address(lib().ncnn_mat_get_data(self.h_)) if last else bytearray(es)
-        return np.ndarray(shape, np.int8 if es == 1 else np.float32, buf, 0, step).copy()
+        last = sum((s - 1) * t for s, t in zip(shape, step)) + es
+        return np.ndarray(shape, np.int8 if es == 1 else np.float32, (C.c_uint8 * last).from_address(base), 0, step).copy()
 
 
 # ---- Net / Extractor -------------------------------------------------------------------------------

@@ -564,3 +564,19 @@ def test_datareader_tables_feed_the_loaders():
     dr = L.ncnn_datareader_create()
     assert L.ncnn_net_load_param_datareader(host.Net().h_, dr) == -1 and L.ncnn_net_load_param_bin_datareader(host.Net().h_, dr) == -1
     L.ncnn_datareader_destroy(dr)
+
+
+def test_to_numpy_of_mats_that_are_not_plain_values():
+    """An empty Mat and matrices of packed or 2-byte elements have no array form; a vector of them is its bytes as fp32."""
+    L = host.lib()
+    buf = np.arange(64, dtype=np.float32)
+    vector = host.Mat(L.ncnn_mat_create_external_1d_elem(3, buf.ctypes.data, 16, 4, None), keep=buf)
+    assert np.array_equal(vector.to_numpy(), buf[:12])
+    assert np.array_equal(host.Mat(L.ncnn_mat_create_external_1d_elem(4, buf.ctypes.data, 2, 1, None), keep=buf).to_numpy(), buf[:2])
+    L.ncnn_mat_create.restype = C.c_void_p
+    for mat in (host.Mat(L.ncnn_mat_create_external_1d_elem(3, buf.ctypes.data, 2, 1, None), keep=buf),
+                host.Mat(L.ncnn_mat_create_external_2d_elem(3, 2, buf.ctypes.data, 16, 4, None), keep=buf),
+                host.Mat(L.ncnn_mat_create_external_2d_elem(4, 2, buf.ctypes.data, 2, 1, None), keep=buf),
+                host.Mat(L.ncnn_mat_create_3d_elem(1, 1, 1, 16, 4, None)), host.Mat(L.ncnn_mat_create())):
+        with pytest.raises(ValueError):
+            mat.to_numpy()
