@@ -408,10 +408,11 @@ int ncnnhip_gemm_blockquant_packed_f16a(const uint16_t* a_dev, size_t a_stride, 
                                         size_t out_stride, void* stream);
 
 /* The layer's own contract on the packed weights: fp32 activations a [M][K] (16-byte aligned rows, K % 16 == 0,
- * K <= 16384: ncnnhip_gemm_blockquant_packed_supported says whether a K qualifies), optional in_scales [K], any M (rows
- * go four at a time, fewer where K is long).  Each activation (times its input scale) is split exactly into three bf16
- * numbers, so every product is the reference's q * a and the result differs from ncnnhip_gemm_blockquant's only by the
- * order of the fp32 additions.  From 32 rows up ncnnhip_gemm_blockquant (fp32 matrix cores, one pass) is the faster call. */
+ * K <= 16384: ncnnhip_gemm_blockquant_packed_supported says whether a K qualifies), optional in_scales [K], any M
+ * (up to 4 rows, fewer where K is long, on the kernel of decoding; more in passes of up to 32).  Each activation (times its
+ * input scale) is split exactly into three bf16 numbers, so every product is the reference's q * a and the result differs
+ * from ncnnhip_gemm_blockquant's only by the order of the fp32 additions.  From about 128 rows up
+ * ncnnhip_gemm_blockquant_packed_rows is the faster call. */
 int ncnnhip_gemm_blockquant_packed_supported(int K);
 int ncnnhip_gemm_blockquant_packed(const float* a_dev, size_t a_stride, int M, int N, int K, const uint8_t* packed_w_dev,
                                    const float* packed_descale_dev, int bits, int block, const float* in_scales_dev,
@@ -421,7 +422,7 @@ int ncnnhip_gemm_blockquant_packed(const float* a_dev, size_t a_stride, int M, i
 /* Several packed weight matrices on the SAME activation rows in one launch: the gate and up projections of a decoder layer, the
  * q / k / v projections of an attention layer -- in the reference one Gemm / MultiHeadAttention projection after the other
  * (src/layer/gemm.cpp:425-483 per matrix); the results are those of `count` calls of ncnnhip_gemm_blockquant_packed(_f16a), bit
- * for bit.  a_elemsize 2: fp16 activations (up to 16 rows in one pass); 4: fp32 (up to 4 rows, with optional in_scales [K]).
+ * for bit.  a_elemsize 2: fp16 activations (up to 16 rows in one pass); 4: fp32 (up to 16 rows, with optional in_scales [K]).
  * All matrices share K, bits and block; N, the packed weights and descales, C (c_dev or its entries may be null), its broadcast
  * type, alpha, beta (null: 1) and the outputs are per matrix, count <= 8.  A decode-sized launch is paced by its ramp and tail,
  * not by bandwidth: one launch over 2 x 45.8 MB reaches what two launches of 45.8 MB cannot.  Shapes the one-pass kernel does

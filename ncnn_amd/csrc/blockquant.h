@@ -200,6 +200,11 @@ static inline bool halves_layout(int bits, int block)
 // weights): every matrix of mm on the same rows, one launch.
 int launch_blockquant_rows_f16(const uint16_t* a, size_t a_stride, int M, int K, int bits, int block, const BqMulti& mm, hipStream_t stream);
 
+// The same with fp32 rows (16-byte aligned) and optional input scales; and about how long that takes (tiles: of 16 weight rows, of all
+// matrices), with the shape it will take.
+double blockquant_rows_f32_us(int M, int K, long long tiles, int* mg, int* rt);
+int launch_blockquant_rows_f32(const float* a, size_t a_stride, int M, int K, int bits, int block, const float* in_scales, const BqMulti& mm, hipStream_t stream);
+
 } // namespace ncnnhip
 
 #endif // NCNNHIP_BLOCKQUANT_H

@@ -2310,6 +2310,25 @@ static bool many_rows_f16(int M, long long N, int K, int bits, int block)
     return weights * M > 750000000 || (K > 8192 && weights > 64000000);
 }
 
+// fp32 rows, without a workspace: the one-pass kernel holds three planes of at most 4 rows in LDS, 4 up to K = 4096, 2 up to 8192, else
+// one; the many-row kernel splits the activations as it multiplies.  us one-pass / many-row, 8 bits in blocks of 64: 4096 x 4096 4 rows
+// 7.4 / 10.9, 11008 x 4096 2 rows 12.2 / 15.8, 4 rows 18.1 / 15.8, 4096 x 11008 2 rows 23.7 / 22.4; 4 bits: 1249 x 6848 4 rows 16.6 / 13.0,
+// 5575 x 5760 2 rows 13.1 / 15.7.  (N is left out of the rule: several matrices in one call take the kernel that each would take alone.)
+static bool many_rows_f32(int M, int K)
+{
+    return M > 4 || (M > 2 && K > 4096) || (M == 2 && K > 8192);
+}
+
+static BqMulti one_matrix(int N, const uint8_t* w, const float4* d, const float* c, int bt, float alpha, float beta, float* out, size_t out_stride)
+{
+    BqMulti one;
+    memset(&one, 0, sizeof(one));
+    one.count = 1;
+    one.N[0] = N, one.bt[0] = bt, one.alpha[0] = alpha, one.beta[0] = beta;
+    one.wpk[0] = w, one.dpk[0] = d, one.c[0] = c, one.out[0] = out, one.out_stride[0] = out_stride;
+    return one;
+}
+
 // shared body of the two packed entry points; ain = 2 (fp16 activations) or 4 (fp32)
 static int gemm_blockquant_packed(const char* who, const void* a_dev, int ain, size_t a_stride, int M, int N, int K, const uint8_t* packed_w_dev,
                                   const float* packed_descale_dev, int bits, int block, const float* in_scales_dev, const float* c_dev, int broadcast_type_c,
@@ -2332,14 +2351,11 @@ static int gemm_blockquant_packed(const char* who, const void* a_dev, int ain, s
     const int split = block == 32 ? 1 : 0;
     hipStream_t st = as_stream(stream);
     if (ain == 2 && many_rows_f16(M, N, K, bits, block))
-    {
-        BqMulti one;
-        memset(&one, 0, sizeof(one));
-        one.count = 1;
-        one.N[0] = N, one.bt[0] = bt, one.alpha[0] = alpha, one.beta[0] = beta;
-        one.wpk[0] = packed_w_dev, one.dpk[0] = dpk, one.c[0] = c_dev, one.out[0] = out_dev, one.out_stride[0] = out_stride;
-        return launch_blockquant_rows_f16(static_cast<const uint16_t*>(a_dev), a_stride, M, K, bits, block, one, st);
-    }
+        return launch_blockquant_rows_f16(static_cast<const uint16_t*>(a_dev), a_stride, M, K, bits, block,
+                                          one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride), st);
+    if (ain == 4 && many_rows_f32(M, K))
+        return launch_blockquant_rows_f32(static_cast<const float*>(a_dev), a_stride, M, K, bits, block, in_scales_dev,
+                                          one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride), st);
     // one pass over the weights for rows m0 .. m0 + mc - 1
     auto upfront = [&](int m0, int mc, bool* handled) -> int {
         const float* cc = c_dev;
@@ -2441,6 +2457,18 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
     hipStream_t st = as_stream(stream);
     const float4* dpk = reinterpret_cast<const float4*>(packed_descale_dev);
     const int split = block == 32 ? 1 : 0;
+    // One launch without the split pass, where that is quicker than the tiled kernel after it, which takes about 9.5 us + K / 1024 x 8.25
+    // us in one round of 64 x 64 tiles on 256 units, 15 in one of 512, then 18 per 512 tiles (18 shapes, 97 to 482 rows; 5 % less here, so
+    // that it stays where the two are close).  us before (the
+    // better of the two below) / here: 8 bits, 4096 x 4096 16 rows 12.4 / 10.7, 32 20.1 / 12.9, 64 34 / 17.5, 128 41 / 30; 11008 x 4096 16
+    // rows 26.5 / 16.6, 32 46 / 26.5; 4096 x 11008 64 rows 84 / 40, 128 93 / 66; 4 bits, 1730 x 1472 186 rows 21.4 / 12.0, 734 x 6016 477
+    // rows 61 / 30.  Its 16-byte loads need aligned rows.
+    const bool aligned = al16(a_dev) && a_stride % 4 == 0 && (!in_scales_dev || al16(in_scales_dev));
+    const long long tiles64 = (long long)((ntiles + 3) / 4) * (Mp / 64);
+    int mg, rt;
+    if (aligned && blockquant_rows_f32_us(M, K, ntiles, &mg, &rt) < 9.0 + K / 1024.0 * (tiles64 <= 256 ? 7.8 : tiles64 <= 512 ? 14.2 : 17.0 * tiles64 / 512.0))
+        return launch_blockquant_rows_f32(a_dev, a_stride, M, K, bits, block, in_scales_dev, one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride),
+                                          st);
     // Which form: the 16-row passes (all in one launch, spread over the chip; every pass streams the weights again, from L2
     // after the first) cost about 5 us + passes x weight bytes at 2 TB/s; the tiled kernel's 64-row tiles about 6 us + K / 85
     // whatever the row count up to 64 (18-20 us at K = 1024, 54-58 at K = 4096).  Measured on 16..96 rows: 3072 x 1024
@@ -2588,7 +2616,7 @@ int ncnnhip_gemm_blockquant_packed(const float* a_dev, size_t a_stride, int M, i
                                   c_dev, broadcast_type_c, alpha, beta, out_dev, out_stride, stream);
 }
 
-// Several matrices on the same activation rows in one launch (see BqMulti).  Shapes without a kernel for that (more than 4 rows
+// Several matrices on the same activation rows in one launch (see BqMulti).  Shapes without a kernel for that (more than 16 rows
 // of fp32 activations, long K) run matrix by matrix through the single-matrix entries.
 int ncnnhip_gemm_blockquant_packed_multi(const void* a_dev, int a_elemsize, size_t a_stride, int M, int K, int count, const int* N,
                                          const uint8_t* const* packed_w_dev, const float* const* packed_descale_dev, int bits, int block,
@@ -2606,7 +2634,7 @@ int ncnnhip_gemm_blockquant_packed_multi(const void* a_dev, int a_elemsize, size
                                       broadcast_type_c ? broadcast_type_c[i] : -1, alpha ? alpha[i] : 1.f, beta ? beta[i] : 1.f, out_dev[i], out_stride[i], stream);
     };
     const bool halves = halves_layout(bits, block);
-    bool one_pass = count > 1 && M >= 1 && K >= 1 && K % 16 == 0 && K <= 16384 && (a_elemsize == 2 || M <= 4) && (bits == 4 || bits == 6 || bits == 8) &&
+    bool one_pass = count > 1 && M >= 1 && K >= 1 && K % 16 == 0 && K <= 16384 && (a_elemsize == 2 || M <= 16) && (bits == 4 || bits == 6 || bits == 8) &&
                     (block == 32 || block == 64 || block == 128) && a_stride >= (size_t)K && a_stride % (16 / a_elemsize) == 0 && al16(a_dev) &&
                     (!in_scales_dev || al16(in_scales_dev));
     BqMulti mm;
@@ -2635,6 +2663,8 @@ int ncnnhip_gemm_blockquant_packed_multi(const void* a_dev, int a_elemsize, size
         mm.wpk[i] = 0, mm.dpk[i] = 0, mm.c[i] = 0, mm.out[i] = 0, mm.out_stride[i] = 0;
     }
     if (one_pass && a_elemsize == 2 && many_rows_f16(M, tiles * 16, K, bits, block)) return launch_blockquant_rows_f16(static_cast<const uint16_t*>(a_dev), a_stride, M, K, bits, block, mm, as_stream(stream));
+    if (one_pass && a_elemsize == 4 && many_rows_f32(M, K))
+        return launch_blockquant_rows_f32(static_cast<const float*>(a_dev), a_stride, M, K, bits, block, in_scales_dev, mm, as_stream(stream));
     if (one_pass)
     {
         const int split = block == 32 ? 1 : 0;

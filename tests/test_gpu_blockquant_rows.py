@@ -1,9 +1,12 @@
 """Block-quantised Gemm on many activation rows: groups of 16 rows, tiles of 16 weight rows and the K steps of 64 at
 their edges, every packed layout, alone and with several matrices in one call: against the oracle and a float64 value."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from ncnn_amd import synth
+from ncnn_amd.hip import DeviceBuffer, check, lib
 from oracle import oracle
 from tests import npref
 
@@ -101,3 +104,75 @@ def test_an_infinity_stays_an_infinity_fp32(rt, m, n, k, rows, bits, block):
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isinf(want).any()
     inf = np.isinf(want)
     assert np.array_equal(got[inf], want[inf])
+
+
+# (m, n): every pair of 1 or 2 groups of rows and 1 to 4 tiles a workgroup, with rows and weight rows that fill neither
+@pytest.mark.parametrize("m,n,k", [(5, 33, 80), (16, 16, 64), (5, 4100, 80), (9, 8200, 144), (5, 13000, 80), (17, 8200, 80), (20, 12410, 64), (130, 50, 1040), (547, 137, 64), (40, 300, 592)])
+@pytest.mark.parametrize("bits,block", [(8, 64), (8, 32), (6, 128), (6, 32), (4, 64), (4, 32)])
+@pytest.mark.parametrize("rows", [False, True])
+def test_fp32_rows_split_as_they_are_multiplied(rt, m, n, k, bits, block, rows):
+    print("[case]", m, n, k, bits, block, rows, flush=True)
+    a, packed, scales = synth.blockquant_operands(m + n + k, m, n, k, bits, block, half_exact=False)
+    rng = np.random.default_rng(n)
+    c, ins = rng.normal(size=(m, n)).astype(F), rng.uniform(0.5, 1.5, k).astype(F)
+    pw, pd = rt.blockquant_pack(packed, scales, block, bits=bits, k=k)
+    got = rt.gemm_blockquant_packed(a, pw, pd, n, c, 3, 0.75, 1.5, bits=bits, block=block, in_scales=ins, rows_kernel=rows)
+    val, floor = npref.blockquant_gemm_f64(a, packed, scales, bits, block, ins, c, 3, 0.75, 1.5)
+    assert np.all(np.abs(got - val) <= 1e-5 * floor + 1e-30)
+    got = rt.gemm_blockquant_packed(a, pw, pd, n, bits=bits, block=block, rows_kernel=rows)
+    val, floor = npref.blockquant_gemm_f64(a, packed, scales, bits, block)
+    assert np.all(np.abs(got - val) <= 1e-5 * floor + 1e-30)
+
+
+@pytest.mark.parametrize("m,n,k", [(7, 40, 144), (17, 8200, 80)])
+def test_special_values_in_fp32_rows(rt, m, n, k):
+    """The sums are made without a look at the values and repeated with one where they turn out not to be numbers: infinities, the largest
+    finite value and a NaN must give what the careful split gives, also beside an input scale, also in the padding of a ragged K."""
+    a, packed, scales = synth.blockquant_operands(m + n, m, n, k, 8, 64, half_exact=False)
+    a[0, 0], a[2, k - 1], a[3, 1], a[4, 2] = np.inf, -np.inf, np.finfo(F).max * F(1e-3), np.nan
+    ins = np.ones(k, F)
+    ins[0] = 2.0
+    pw, pd = rt.blockquant_pack(packed, scales, 64, k=k)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = oracle.gemm_blockquant(a, packed, scales, 8, 64, ins)
+    got = rt.gemm_blockquant_packed(a, pw, pd, n, in_scales=ins)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isinf(want[0]).any() and np.isnan(want[4]).all()
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf])
+    fine = np.isfinite(want)
+    val, floor = npref.blockquant_gemm_f64(np.where(np.isfinite(a), a, 0), packed, scales, 8, 64, ins)
+    rows = [i for i in range(m) if i not in (0, 2, 4)]
+    assert np.all(np.abs(got[rows] - val[rows])[fine[rows]] <= 1e-5 * floor[rows][fine[rows]])
+
+
+def test_fp32_rows_off_16_bytes_take_the_general_forms(rt):
+    """packed_rows takes activations and outputs of any 4-byte alignment: what the aligned call gives, to the order of the sums."""
+    m, n, k = 24, 100, 208
+    a, packed, scales = synth.blockquant_operands(5, m, n, k, 4, 64, half_exact=False)
+    pw, pd = rt.blockquant_pack(packed, scales, 64, bits=4, k=k)
+    w, d = rt.up(pw), rt.up(pd)
+    size = C.c_size_t()
+    check(lib().ncnnhip_gemm_blockquant_packed_rows_workspace_bytes(m, k, C.byref(size)))
+    ws = DeviceBuffer.empty((size.value,), np.uint8)
+    val, floor = npref.blockquant_gemm_f64(a, packed, scales, 4, 64)
+    for a_stride, a_off, o_stride, o_off in ((k, 0, n, 0), (k + 1, 0, n + 1, 0), (k + 4, 1, n + 4, 1), (k + 4, 0, n + 4, 2), (k + 3, 3, n + 3, 3)):
+        buf = np.full(m * a_stride + 8, np.nan, F)
+        buf[a_off:a_off + m * a_stride].reshape(m, a_stride)[:, :k] = a
+        src, dst = rt.up(buf), rt.up(np.full(m * o_stride + 8, 7.0, F))
+        at = lambda t, off: C.c_void_p(t.ptr.value + 4 * off)
+        check(lib().ncnnhip_gemm_blockquant_packed_rows(at(src, a_off), a_stride, m, n, k, w.ptr, d.ptr, 4, 64, None, None, -1, 1.0, 1.0, at(dst, o_off), o_stride, ws.ptr,
+                                                        size.value, rt.stream))
+        out = dst.to_numpy(rt.stream)
+        got = out[o_off:o_off + m * o_stride].reshape(m, o_stride)
+        assert np.all(np.abs(got[:, :n] - val) <= 1e-5 * floor), (a_stride, a_off)
+        assert np.all(got[:, n:] == 7.0) and np.all(out[:o_off] == 7.0), (o_stride, o_off)
+
+
+@pytest.mark.parametrize("m,k", [(3, 144), (4, 4112), (9, 208), (16, 1040), (17, 208)])
+def test_several_matrices_of_fp32_rows_get_the_bits_of_single_calls(rt, m, k):
+    ns = (50, 16, 4200)
+    ops = [synth.blockquant_operands(10 + i, m, n, k, 8, 64, half_exact=False) for i, n in enumerate(ns)]
+    a = ops[0][0]
+    mats = [rt.blockquant_pack(p, s, 64, k=k) + (n, None, -1, 1.0, 1.0) for (_, p, s), n in zip(ops, ns)]
+    for got, (pw, pd, n, *_) in zip(rt.gemm_blockquant_packed_multi(a, mats), mats):
+        assert np.array_equal(got, rt.gemm_blockquant_packed(a, pw, pd, n))
