@@ -60,22 +60,18 @@ __global__ __launch_bounds__(256) void fc_gemv_kernel(const int8_t* __restrict__
     }
 }
 
-// Up to 16 rows of A on the matrix cores: a workgroup owns 16 rows of B, its four wavefronts every fourth 64-wide K step each
-// (v_mfma_i32_16x16x64_i8: the rows of B as one operand, the rows of A as the other, so a lane ends up with four consecutive
-// columns of one output row); eight steps of B and A are requested before the first product; the four partial tiles are
-// added through LDS.  B is read once; A (at most 16 x K bytes) comes from the cache.
-// ANY: rows that begin at any byte and K that is no multiple of 64: 16-byte loads at any address, and the wavefront whose turn
-// it would be multiplies what is left of K (K >= 16).
-// ROW_FIRST: the epilogue takes (activation row, output column, acc), as Gemm's does; else (output channel, row, acc)
+// Up to 16 input rows on the matrix cores: a workgroup owns 16 output channels, its four wavefronts every fourth 64-wide K step each
+// (v_mfma_i32_16x16x64_i8: the weights as one operand, the input rows as the other); eight steps of both are requested before the
+// first product; the four partial tiles are added through LDS.  The weights are read once; the input (at most 16 x K bytes) comes
+// from the cache.  K % 64 == 0, operands aligned.
 typedef int v4i_sk __attribute__((ext_vector_type(4)));
-template<typename Epilogue, bool ROW_FIRST, bool ANY>
-__global__ __launch_bounds__(256) void gemm_skinny_int8_kernel(const int8_t* __restrict__ a, size_t as, int M_total, const int8_t* __restrict__ b, size_t bs, int N, int K,
-                                                                Epilogue epi)
+__global__ __launch_bounds__(256) void fc_skinny_int8_kernel(const int8_t* __restrict__ a, size_t as, int M_total, const int8_t* __restrict__ b, size_t bs, int N, int K,
+                                                             FcEpilogue epi)
 {
     __shared__ int red[4][64][4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, q = lane >> 4;
     const int tile = blockIdx.x;
-    const int row0 = blockIdx.y * 16; // blockIdx.y: which 16 rows of A (every group of 16 reads B again, from the cache after the first)
+    const int row0 = blockIdx.y * 16; // blockIdx.y: which 16 rows (every group of 16 reads the weights again, from the cache after the first)
     const int M = M_total - row0 < 16 ? M_total - row0 : 16;
     a += (size_t)row0 * as;
     const int brow = tile * 16 + c16 < N ? tile * 16 + c16 : N - 1; // rows past the end repeat the last one; nothing of theirs is stored
@@ -84,16 +80,6 @@ __global__ __launch_bounds__(256) void gemm_skinny_int8_kernel(const int8_t* __r
     const int8_t* ap = a + (size_t)arow * as + q * 16;
     const int ksteps = K >> 6;
     v4i_sk acc = {0, 0, 0, 0};
-    // what is left of K: a chunk that K ends in is cut out of the row's last 16 bytes
-    const bool tail = ANY && (K & 63) != 0 && (ksteps & 3) == wave;
-    const int tail_drop = ksteps * 64 + q * 16 + 16 - K;
-    v4i_sk tw = {0, 0, 0, 0}, tx = {0, 0, 0, 0};
-    if (tail)
-    {
-        const int k = tail_drop > 0 ? K - 16 - q * 16 : ksteps * 64;
-        tw = load16(bp + k);
-        tx = load16(ap + k);
-    }
     for (int k0 = wave; k0 < ksteps; k0 += 32) // this wavefront's steps k0, k0 + 4, ..., eight at a time
     {
         v4i_sk wv[8], xv[8];
@@ -102,17 +88,12 @@ __global__ __launch_bounds__(256) void gemm_skinny_int8_kernel(const int8_t* __r
         {
             const int ks = k0 + 4 * u;
             const int kk = ks < ksteps ? ks : k0; // past the end: a step that is there, its product dropped below
-            wv[u] = ANY ? load16(bp + (size_t)kk * 64) : *reinterpret_cast<const v4i_sk*>(bp + (size_t)kk * 64);
-            xv[u] = ANY ? load16(ap + (size_t)kk * 64) : *reinterpret_cast<const v4i_sk*>(ap + (size_t)kk * 64);
+            wv[u] = *reinterpret_cast<const v4i_sk*>(bp + (size_t)kk * 64);
+            xv[u] = *reinterpret_cast<const v4i_sk*>(ap + (size_t)kk * 64);
         }
 #pragma unroll
         for (int u = 0; u < 8; u++)
             if (k0 + 4 * u < ksteps) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wv[u], xv[u], acc, 0, 0, 0);
-    }
-    if (tail)
-    {
-        const int drop = tail_drop < 0 ? 0 : tail_drop > 16 ? 16 : tail_drop;
-        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(drop_bytes(tw, drop), drop_bytes(tx, drop), acc, 0, 0, 0);
     }
 #pragma unroll
     for (int r = 0; r < 4; r++) red[wave][lane][r] = acc[r];
@@ -123,23 +104,17 @@ __global__ __launch_bounds__(256) void gemm_skinny_int8_kernel(const int8_t* __r
     {
         const int v = (red[0][lane][r] + red[1][lane][r]) + (red[2][lane][r] + red[3][lane][r]);
         const int j = tile * 16 + 4 * q + r;
-        if (c16 < M && j < N)
-        {
-            if (ROW_FIRST)
-                epi(row0 + c16, j, v); // Gemm's epilogue: (row of A, column)
-            else
-                epi(j, row0 + c16, v); // InnerProduct's: (output channel, row)
-        }
+        if (c16 < M && j < N) epi(j, row0 + c16, v);
     }
 }
 
-// InnerProduct on 2 to 48 rows (a batch through the classifier of a net): the same kernel with InnerProduct's epilogue, above 16 rows
-// under an estimate like Gemm's, against about 4 us + K / 300 for the convolution's kernel (ncnnhip_innerproduct_int8_ws).  false: the
-// shape is not one it takes.
+// InnerProduct on 2 to 48 rows (a batch through the classifier of a net), above 16 rows while reading the weights once per 16 rows (about
+// 3 us + groups x bytes at 4 TB/s) stays below about 4 us + K / 300 for the convolution's kernel (ncnnhip_innerproduct_int8_ws).
+// false: the shape is not one it takes.
 static bool launch_fc_skinny(const int8_t* x_dev, size_t x_stride, int rows, int num_input, int num_output, const int8_t* weight_dev, const FcEpilogue& epi,
                              hipStream_t stream);
 
-constexpr int GEMM_SKINNY_MAX_ROWS = 48;
+constexpr int FC_SKINNY_MAX_ROWS = 48;
 static inline bool aligned16(const void* p)
 {
     return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
@@ -156,7 +131,7 @@ int launch_gemm_tile_operand(const int8_t* src, size_t stride, int rows, int K, 
 // the shapes the few-row kernel takes for InnerProduct (operands aligned): no workspace, no hand-off between workgroups
 bool fc_skinny_takes(int rows, int num_input, int num_output)
 {
-    if (rows < 2 || rows > GEMM_SKINNY_MAX_ROWS || num_output < 64 || num_input % 64 != 0) return false;
+    if (rows < 2 || rows > FC_SKINNY_MAX_ROWS || num_output < 64 || num_input % 64 != 0) return false;
     const int groups16 = (rows + 15) / 16;
     return !(rows > 16 && 3.0 + groups16 * ((double)num_output * (double)num_input / 4.0e6) > 4.0 + num_input / 300.0);
 }
@@ -167,7 +142,7 @@ static bool launch_fc_skinny(const int8_t* x_dev, size_t x_stride, int rows, int
     if (!fc_skinny_takes(rows, num_input, num_output)) return false;
     if (!aligned16(x_dev) || !aligned16(weight_dev) || x_stride % 16 != 0) return false;
     const int groups16 = (rows + 15) / 16;
-    hipLaunchKernelGGL((gemm_skinny_int8_kernel<FcEpilogue, false, false>), dim3(ceil_div(num_output, 16), groups16), dim3(256), 0, stream, x_dev, x_stride, rows, weight_dev,
+    hipLaunchKernelGGL(fc_skinny_int8_kernel, dim3(ceil_div(num_output, 16), groups16), dim3(256), 0, stream, x_dev, x_stride, rows, weight_dev,
                        (size_t)num_input, num_output, num_input, epi);
     return true;
 }
@@ -205,34 +180,24 @@ int ncnnhip_gemm_int8(const int8_t* aq_dev, size_t aq_stride, const int8_t* bq_d
     epi.N = N;
     epi.acc_out = acc_out_dev;
 
-    // up to 16 rows of A, or up to 48 while reading B once per 16 rows (about 3 us + groups x bytes of B at 4 TB/s, from the cache
-    // after the first) stays below what the general kernel takes for so few rows (about 4 us + K / 450): quantise + Gemm for
-    // 16 / 32 rows 4096 x 4096 10.1 / 13.6 us, 1024 x 1024 7.2 / 7.5; one row 8.7 / 7.5
-    const int groups16 = (M + 15) / 16;
-    const bool skinny_pays = M <= 16 || 3.0 + groups16 * ((double)N * (double)K / 4.0e6) <= 4.0 + K / 450.0;
-    if (skinny_pays && M <= GEMM_SKINNY_MAX_ROWS && N >= 64 && K >= 16)
+    const bool aligned = K % 16 == 0 && aligned16(aq_dev) && aligned16(bq_dev) && aq_stride % 16 == 0 && bq_stride % 16 == 0;
+    if (!gemm_int8_streams(M, N, K, aligned))
     {
-        const dim3 grid(ceil_div(N, 16), ceil_div(M, 16));
-        if (K % 64 == 0 && aligned16(aq_dev) && aligned16(bq_dev) && aq_stride % 16 == 0 && bq_stride % 16 == 0)
-            hipLaunchKernelGGL((gemm_skinny_int8_kernel<GemmEpilogue, true, false>), grid, dim3(256), 0, as_stream(stream), aq_dev, aq_stride, M, bq_dev, bq_stride, N, K, epi);
-        else
-            hipLaunchKernelGGL((gemm_skinny_int8_kernel<GemmEpilogue, true, true>), grid, dim3(256), 0, as_stream(stream), aq_dev, aq_stride, M, bq_dev, bq_stride, N, K, epi);
-        return launch_status("gemm_skinny_int8_kernel");
-    }
-    // big aligned problems: the 256x256 kernel (it needs a few hundred tiles to fill the chip)
-    bool handled = false;
-    int ret = NCNNHIP_OK;
-    if ((long long)M * N >= 256ll * 256 * 128)
-    {
-        ret = launch_gemm_int8_pipelined(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, epi, as_stream(stream), &handled);
-        if (handled) return ret;
-    }
-    // too few 256x256 tiles for that: the same ring on 128x128 tiles, from 48 of them up (below, the general kernel's 64-row tiles
-    // spread the work over more CUs)
-    if ((long long)(M / 128) * (N / 128) >= 48)
-    {
-        ret = launch_gemm_int8_ring128(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, epi, as_stream(stream), &handled);
-        if (handled) return ret;
+        // big aligned problems: the 256x256 kernel (it needs a few hundred tiles to fill the chip)
+        bool handled = false;
+        int ret = NCNNHIP_OK;
+        if ((long long)M * N >= 256ll * 256 * 128)
+        {
+            ret = launch_gemm_int8_pipelined(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, epi, as_stream(stream), &handled);
+            if (handled) return ret;
+        }
+        // too few 256x256 tiles for that: the same ring on 128x128 tiles, from 48 of them up (below, the general kernel's 64-row tiles
+        // spread the work over more CUs)
+        if ((long long)(M / 128) * (N / 128) >= 48)
+        {
+            ret = launch_gemm_int8_ring128(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, epi, as_stream(stream), &handled);
+            if (handled) return ret;
+        }
     }
     return launch_gemm_int8_general(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, epi, as_stream(stream));
 }
@@ -254,7 +219,7 @@ int ncnnhip_innerproduct_int8(const int8_t* x_dev, size_t x_stride, int rows, in
     epi.num_output = num_output;
     epi.acc_out = acc_out_dev;
 
-    if (launch_fc_skinny(x_dev, x_stride, rows, num_input, num_output, weight_dev, epi, as_stream(stream))) return launch_status("gemm_skinny_int8_kernel<fc>");
+    if (launch_fc_skinny(x_dev, x_stride, rows, num_input, num_output, weight_dev, epi, as_stream(stream))) return launch_status("fc_skinny_int8_kernel");
     if (rows <= 64)
     {
         const int vec = aligned16(x_dev) && aligned16(weight_dev) && x_stride % 16 == 0 && num_input % 16 == 0;
@@ -292,7 +257,7 @@ int ncnnhip_innerproduct_int8_ws(const int8_t* x_dev, size_t x_stride, int rows,
         fe.out_stride = out_stride;
         fe.num_output = num_output;
         fe.acc_out = 0;
-        if (launch_fc_skinny(x_dev, x_stride, rows, num_input, num_output, weight_dev, fe, as_stream(stream))) return launch_status("gemm_skinny_int8_kernel<fc>");
+        if (launch_fc_skinny(x_dev, x_stride, rows, num_input, num_output, weight_dev, fe, as_stream(stream))) return launch_status("fc_skinny_int8_kernel");
     }
     if (rows >= 8)
     {

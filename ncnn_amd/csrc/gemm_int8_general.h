@@ -30,6 +30,9 @@ __device__ __forceinline__ v4i drop_bytes(v4i w, int drop)
     return v;
 }
 
+// whether the general entry points below take their streaming kernel for this shape (aligned: rows, strides and K in multiples of 16 bytes)
+bool gemm_int8_streams(int M, int N, int K, bool aligned);
+
 // any M, N, K >= 1, strides >= K, any alignment, every form of the epilogue
 int launch_gemm_int8_general(const int8_t* a, size_t lda, const int8_t* b, size_t ldb, int M, int N, int K, const GemmEpilogue& epi, hipStream_t stream);
 int launch_fc_int8_general(const int8_t* x, size_t xs, const int8_t* w, size_t ws, int rows, int num_output, int K, const FcEpilogue& epi, hipStream_t stream);

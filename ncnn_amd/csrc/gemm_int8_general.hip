@@ -9,8 +9,8 @@
 // A workgroup is four wavefronts, 2 x 2, on a BM x BN tile; a K step is 128 bytes of every row.  LDS holds two steps; row r
 // keeps its eight 16-byte chunks at positions c ^ ((r >> 1) & 7), so that any 16 consecutive rows read at one K offset meet
 // 16 different bank groups.  One barrier per step: the buffer that step t + 1 is written into was last read in step t - 1.
-// Bound by latency at the sizes it is for (a few hundred tiles of 64 x 64): 1501 x 1000 x 2008 168 us with the byte gathers
-// of the kernel before this one.
+// Bound by latency at the sizes it is for (some hundred tiles of 64 x 64): 1501 x 1000 x 2008 168 us with the byte gathers
+// of the kernel before this one.  Fewer tiles go to gemm_int8_stream_kernel below.
 #include "conv_nhwc.h"
 #include "epilogues.h"
 #include "gemm_int8_general.h"
@@ -274,6 +274,125 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
     }
 }
 
+// Few tiles (gemm_int8_streams): the W wavefronts of a workgroup each multiply the whole BM x BN tile over a run of K steps of their own.
+// A wavefront fetches 128 bytes of each of its rows into registers (coalesced, any alignment), turns them into the operand mapping through
+// a piece of LDS that belongs to it alone -- LDS serves a wavefront in order, so no barrier stands in the loop -- and requests the next
+// step before it multiplies.  The sums meet in LDS at the end.  Bound by latency: a launch, one trip to memory for every one to four
+// steps, the sums; 32 x 32 tiles put four times as many workgroups on the chip as 64 x 64.
+template<int BM, int BN, int W, typename Epilogue>
+__global__ __launch_bounds__(64 * W) void gemm_int8_stream_kernel(const int8_t* __restrict__ A, size_t lda, const int8_t* __restrict__ B, size_t ldb, int M, int N, int K,
+                                                                  Epilogue epi)
+{
+    constexpr int TM = BM / 32, TN = BN / 32; // 32 x 32 blocks
+    constexpr int LA = BM / 8, LB = BN / 8;   // loads of 8 rows x 128 bytes
+    constexpr int STEP_BYTES = (BM + BN) * KSTEP;
+    static_assert(BM * BN * 4 <= STEP_BYTES, "a wavefront's sums fit its piece of LDS");
+    __shared__ __attribute__((aligned(16))) int8_t smem_all[W * STEP_BYTES];
+    __shared__ float row_value[BM];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, lhi = lane >> 5;
+    int8_t* smem = smem_all + wave * STEP_BYTES;
+
+    const int row0 = blockIdx.y * BM, col0 = blockIdx.x * BN;
+
+    // this wavefront's K steps; the last of all may end inside: its chunks beyond K are fetched from the row's end and cut when they go to LDS
+    const int all = (K + KSTEP - 1) / KSTEP;
+    const int step0 = all * wave / W, steps = all * (wave + 1) / W - step0;
+    const int cut_step = K % KSTEP ? all - 1 - step0 : -1;
+    const int ld_row = lane >> 3, ld_chunk = lane & 7;
+    const int8_t* pa = A + (size_t)row0 * lda;
+    const int8_t* pb = B + (size_t)col0 * ldb;
+    size_t off_a[LA], off_b[LB];
+#pragma unroll
+    for (int i = 0; i < LA; i++) off_a[i] = (size_t)(row0 + i * 8 + ld_row < M ? i * 8 + ld_row : M - 1 - row0) * lda;
+#pragma unroll
+    for (int i = 0; i < LB; i++) off_b[i] = (size_t)(col0 + i * 8 + ld_row < N ? i * 8 + ld_row : N - 1 - col0) * ldb;
+    v4i ra[LA], rb[LB];
+    auto fetch = [&](int t) {
+        const int k = (step0 + (t < steps ? t : 0)) * KSTEP + ld_chunk * 16;
+        const int kk = k < K - 16 ? k : K - 16;
+#pragma unroll
+        for (int i = 0; i < LA; i++) ra[i] = load16(pa + off_a[i] + kk);
+#pragma unroll
+        for (int i = 0; i < LB; i++) rb[i] = load16(pb + off_b[i] + kk);
+    };
+    fetch(0);
+
+    // what the end needs besides the sums
+    const int in_col = threadIdx.x % BN, col = col0 + in_col;
+    if ((int)threadIdx.x < BM) row_value[threadIdx.x] = row0 + (int)threadIdx.x < M ? epi.row_value(row0 + threadIdx.x) : 0.f;
+    float scale = 0.f, add = 0.f;
+    if (col < N) epi.column(col, scale, add);
+
+    v16i acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0;
+    // row r of an operand keeps chunk c at position c ^ ((r >> 1) & 7): r = i * 8 + ld_row when written, i * 32 + l32 when read
+    const int wr0 = ld_row * KSTEP + (ld_chunk ^ (ld_row >> 1)) * 16, wr1 = ld_row * KSTEP + (ld_chunk ^ (ld_row >> 1) ^ 4) * 16;
+    int rd[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) rd[q] = l32 * KSTEP + (((2 * q + lhi) ^ (l32 >> 1)) & 7) * 16;
+
+    for (int t = 0; t < steps; t++)
+    {
+        if (t == cut_step) // uniform
+        {
+            const int over = (step0 + t) * KSTEP + ld_chunk * 16 + 16 - K, drop = over < 0 ? 0 : over > 16 ? 16 : over;
+#pragma unroll
+            for (int i = 0; i < LA; i++) ra[i] = drop_bytes(ra[i], drop);
+#pragma unroll
+            for (int i = 0; i < LB; i++) rb[i] = drop_bytes(rb[i], drop);
+        }
+#pragma unroll
+        for (int i = 0; i < LA; i++) *reinterpret_cast<v4i*>(smem + i * 1024 + (i & 1 ? wr1 : wr0)) = ra[i];
+#pragma unroll
+        for (int i = 0; i < LB; i++) *reinterpret_cast<v4i*>(smem + BM * KSTEP + i * 1024 + (i & 1 ? wr1 : wr0)) = rb[i];
+        __builtin_amdgcn_wave_barrier();
+        fetch(t + 1); // (past the last step: the first again)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+        {
+            v4i fa[TM], fb[TN];
+#pragma unroll
+            for (int i = 0; i < TM; i++) fa[i] = *reinterpret_cast<const v4i*>(smem + i * 32 * KSTEP + rd[q]);
+#pragma unroll
+            for (int j = 0; j < TN; j++) fb[j] = *reinterpret_cast<const v4i*>(smem + (BM + j * 32) * KSTEP + rd[q]);
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+
+    int* sums = reinterpret_cast<int*>(smem);
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) sums[(i * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3)) * BN + j * 32 + l32] = acc[i][j][r];
+    __syncthreads();
+    if (col >= N) return;
+    // every thread finishes one column of the tile, every (64 * W / BN)-th row
+    const int* from = reinterpret_cast<const int*>(smem_all) + in_col;
+#pragma unroll 4
+    for (int in_tile = threadIdx.x / BN; in_tile < BM; in_tile += 64 * W / BN)
+    {
+        if (row0 + in_tile >= M) break;
+        int v = 0;
+#pragma unroll
+        for (int w = 0; w < W; w++) v += from[w * (STEP_BYTES / 4) + in_tile * BN];
+        epi.store(row0 + in_tile, col, v, row_value[in_tile], scale, add);
+    }
+}
+
 // K below 16: a thread per output
 template<typename Epilogue>
 __global__ __launch_bounds__(256) void gemm_int8_short_k_kernel(const int8_t* __restrict__ A, size_t lda, const int8_t* __restrict__ B, size_t ldb, int M, int N, int K,
@@ -298,6 +417,36 @@ static int launch_tile(const int8_t* a, size_t lda, const int8_t* b, size_t ldb,
     return launch_status("gemm_int8_general_kernel");
 }
 
+template<int BM, int BN, int W, typename Epilogue>
+static int launch_stream(const int8_t* a, size_t lda, const int8_t* b, size_t ldb, int M, int N, int K, const Epilogue& epi, hipStream_t stream)
+{
+    const long long tm = ceil_div(M, BM), tn = ceil_div(N, BN);
+    hipLaunchKernelGGL((gemm_int8_stream_kernel<BM, BN, W, Epilogue>), dim3((unsigned)tn, (unsigned)tm), dim3(64 * W), 0, stream, a, lda, b, ldb, M, N, K, epi);
+    return launch_status("gemm_int8_stream_kernel");
+}
+
+static inline bool rows_aligned16(const int8_t* p, size_t stride, int K)
+{
+    return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && stride % 16 == 0 && K % 16 == 0;
+}
+
+// Where the streaming kernel is the quicker one.  Up to 16 rows always: it reads B once, at 5.5 TB/s where B is large.  Else by its tiles: it
+// reads the operands of each 32 x 32 tile, four times the bytes a product that 128 x 128 tiles read, and rows off 16 bytes cost two cache
+// lines for one.  us, Gemm alone, the quickest other kernel here -> this one: 1 x 8192 x 8192 16.5 -> 12.0, 32 x 4096 x 4096 11.0 -> 5.8, 64 x 512
+// x 512 5.2 -> 4.6, 281 x 720 x 2048 8.8 -> 4.6, 360 x 936 x 4672 13.9 -> 10.1, 551 x 1024 x 2048 9.0 -> 7.6, 1024 cubed 8.2 -> 6.8, 512 x
+// 2048 x 2048 11.1 -> 8.9; 256 x 4096 x 4096 17.3 -> 12.2 with 64 x 64 tiles and eight wavefronts; off 16 bytes 16 x 8000 x 8001 42 -> 17, 895 x
+// 456 x 473 6.5 -> 5.8; and where it is not taken: 1226 x 1344 x 2944 17.0 -> 18.0, 330 x 6616 x 896 10.2 -> 11.7, 2284 x 336 x 1216 7.4 ->
+// 7.9, off 16 bytes 148 x 3311 x 537 6.8 -> 7.8.  (From 640 to 1024 tiles it is better than the 128 x 128 tiles of whole multiples, not than
+// 64 x 64.)  Eight wavefronts a tile up to one tile a unit and from nine K steps (128 x 1024 x 4096 5.7, four 6.2), else four.
+bool gemm_int8_streams(int M, int N, int K, bool aligned)
+{
+    if (K < 16) return false;
+    if (M <= 16) return true;
+    const long long tiles32 = (long long)ceil_div(M, 32) * ceil_div(N, 32);
+    if (!aligned) return tiles32 <= 450;
+    return tiles32 <= 640 || (tiles32 <= 1024 && (K >= 3072 || (M % 128 == 0 && N % 128 == 0)));
+}
+
 template<typename Epilogue>
 static int launch_any(const int8_t* a, size_t lda, const int8_t* b, size_t ldb, int M, int N, int K, const Epilogue& epi, hipStream_t stream)
 {
@@ -308,10 +457,17 @@ static int launch_any(const int8_t* a, size_t lda, const int8_t* b, size_t ldb, 
         hipLaunchKernelGGL((gemm_int8_short_k_kernel<Epilogue>), dim3((unsigned)blocks), dim3(256), 0, stream, a, lda, b, ldb, M, N, K, epi);
         return launch_status("gemm_int8_short_k_kernel");
     }
+    if (gemm_int8_streams(M, N, K, rows_aligned16(a, lda, K) && rows_aligned16(b, ldb, K)))
+    {
+        const long long tiles32 = (long long)ceil_div(M, 32) * ceil_div(N, 32);
+        if (M > 16 && tiles32 > 512 && K >= 3072) return launch_stream<64, 64, 8>(a, lda, b, ldb, M, N, K, epi, stream);
+        if (tiles32 <= 256 && K > 1024) return launch_stream<32, 32, 8>(a, lda, b, ldb, M, N, K, epi, stream);
+        return launch_stream<32, 32, 4>(a, lda, b, ldb, M, N, K, epi, stream);
+    }
     // 64 x 64 tiles keep the most compute units busy and are the fastest up to about six of them per unit; beyond that the
     // operand bytes per product decide, half as many with 128 x 128 tiles (2000 x 4000 x 4096: 74 -> 53 us, 2500 cubed 56 ->
-    // 41, 2048 cubed the same 20).  With few tiles and a long K two groups of wavefronts halve the chain of steps (96 x 8192
-    // x 8192 26 -> 21.5, 1100 x 520 x 7000 23.4 -> 20.2; 333 x 777 x 999 7.4 -> 8.6: not below some 24 steps).
+    // 41, 2048 cubed the same 20).  With few tiles and a long K two groups of wavefronts halve the chain of steps (1100 x 520 x 7000
+    // 23.4 -> 20.2; not below some 24 steps).
     const long long tiles = (long long)ceil_div(M, 64) * ceil_div(N, 64);
     if (tiles >= 1536) return launch_tile<128, 128, 1>(a, lda, b, ldb, M, N, K, epi, stream);
     if (tiles <= 512 && K >= 3072) return launch_tile<64, 64, 2>(a, lda, b, ldb, M, N, K, epi, stream);

@@ -20,8 +20,12 @@ SHAPES = [
     (65, 63, 15), (17, 64, 16), (63, 65, 17), (64, 129, 63), (129, 64, 65), (127, 128, 127), (128, 127, 128), (66, 70, 129), (130, 66, 143), (70, 70, 271), (64, 64, 400),
     # few rows (one workgroup per 16 rows of B), with K of 0 and more whole 64-byte steps
     (1, 64, 16), (3, 65, 63), (16, 79, 65), (17, 100, 321), (2, 63, 77), (1, 130, 2047),
-    # two groups of wavefronts per tile from K = 3072, one K step more or less than the other's
+    # long K on few tiles: eight wavefronts with runs of several K steps, the last cut
     (70, 65, 3072), (130, 65, 3073), (65, 66, 3200), (64, 64, 3327),
+    # four wavefronts a tile of 32 x 32 from 257 tiles, some without a step; 64 x 64 tiles with eight from 513 tiles and K = 3072
+    (300, 900, 144), (260, 1000, 1039), (16, 9000, 48), (620, 1000, 528), (768, 1024, 80), (530, 1000, 3088),
+    # beyond the streaming kernel (450 tiles of 32 x 32, 640 or 1024 where rows are aligned): one and two groups of wavefronts per tile of 64 x 64
+    (700, 700, 65), (720, 650, 271), (1000, 700, 528), (470, 970, 3073), (465, 990, 3327),
     # 128 x 128 tiles from 1536 tiles of 64 x 64
     (2497, 2497, 33), (1, 5000, 50), (3000, 2176, 130),
 ]
