@@ -444,7 +444,7 @@ bool gemm_int8_streams(int M, int N, int K, bool aligned)
     if (M <= 16) return true;
     const long long tiles32 = (long long)ceil_div(M, 32) * ceil_div(N, 32);
     if (!aligned) return tiles32 <= 450;
-    return tiles32 <= 640 || (tiles32 <= 1024 && (K >= 3072 || (M % 128 == 0 && N % 128 == 0)));
+    return tiles32 <= 640 || (tiles32 <= 1024 && M % 128 == 0 && N % 128 == 0);
 }
 
 template<typename Epilogue>
@@ -460,7 +460,7 @@ static int launch_any(const int8_t* a, size_t lda, const int8_t* b, size_t ldb, 
     if (gemm_int8_streams(M, N, K, rows_aligned16(a, lda, K) && rows_aligned16(b, ldb, K)))
     {
         const long long tiles32 = (long long)ceil_div(M, 32) * ceil_div(N, 32);
-        if (M > 16 && tiles32 > 512 && K >= 3072) return launch_stream<64, 64, 8>(a, lda, b, ldb, M, N, K, epi, stream);
+        if (M > 16 && tiles32 > 640 && K >= 3072) return launch_stream<64, 64, 8>(a, lda, b, ldb, M, N, K, epi, stream);
         if (tiles32 <= 256 && K > 1024) return launch_stream<32, 32, 8>(a, lda, b, ldb, M, N, K, epi, stream);
         return launch_stream<32, 32, 4>(a, lda, b, ldb, M, N, K, epi, stream);
     }

@@ -292,9 +292,9 @@ constexpr int QT = 128;
 constexpr int Q_OPERAND = QT * PK;     // 8 KB
 constexpr int Q_STAGE = 2 * Q_OPERAND; // 16 KB
 
-template<bool PER_COL, int BT, int S>
+template<bool PER_COL, int BT, int S, bool RAGGED>
 __global__ __launch_bounds__(256) void gemm_int8_128x128_kernel(const int8_t* __restrict__ A, size_t lda, const int8_t* __restrict__ B, size_t ldb, int nk,
-                                                                 int tiles_m, int tiles_n, const float* __restrict__ a_scales,
+                                                                 int M, int N, int tiles_m, int tiles_n, const float* __restrict__ a_scales,
                                                                  const float* __restrict__ b_scales, const float* __restrict__ cvec, float alpha, float beta,
                                                                  float* __restrict__ out, size_t ldo)
 {
@@ -322,13 +322,16 @@ __global__ __launch_bounds__(256) void gemm_int8_128x128_kernel(const int8_t* __
     // load i (0, 1) of wave w fills LDS rows i*64 + w*16 .. +16 of an operand stage; chunks swizzled as in the 256x256 kernel
     const int ld_row = wave * 16 + (lane >> 2);
     const int ld_chunk = (lane & 3) ^ ((lane >> 4) & 3);
-    const int8_t* ga = A + ((size_t)tile_m * QT + ld_row) * lda + ld_chunk * 16;
     // LDS row wn*64 + j*32 + l holds B row wn*64 + 2*l + j: the two accumulator blocks j of a lane are two consecutive output
     // columns (8-byte stores).  LDS row of this lane in half i = i*64 + wave*16 + (lane >> 2): wn = i, j = wave >> 1,
     // l = (wave & 1)*16 + (lane >> 2).
     const int ld_row_b = 2 * ((wave & 1) * 16 + (lane >> 2)) + (wave >> 1);
-    const int8_t* gb = B + ((size_t)tile_n * QT + ld_row_b) * ldb + ld_chunk * 16;
-    const size_t a_half = 64 * lda, b_half = 64 * ldb;
+    // RAGGED: rows past the end repeat the last one and are not stored
+    const int rows_a = RAGGED ? M - tile_m * QT : QT, rows_b = RAGGED ? N - tile_n * QT : QT;
+    const int8_t* ga = A + ((size_t)tile_m * QT + (RAGGED && ld_row >= rows_a ? rows_a - 1 : ld_row)) * lda + ld_chunk * 16;
+    const int8_t* gb = B + ((size_t)tile_n * QT + (RAGGED && ld_row_b >= rows_b ? rows_b - 1 : ld_row_b)) * ldb + ld_chunk * 16;
+    const size_t a_half = RAGGED && ld_row + 64 >= rows_a ? (size_t)(rows_a - 1 > ld_row ? rows_a - 1 - ld_row : 0) * lda : 64 * lda;
+    const size_t b_half = RAGGED && ld_row_b + 64 >= rows_b ? (size_t)(rows_b - 1 > ld_row_b ? rows_b - 1 - ld_row_b : 0) * ldb : 64 * ldb;
 
     auto issue_one = [&](int t, int i, int which) {
         int8_t* sa = smem + (t & (S - 1)) * Q_STAGE + wave * 1024 + i * 4096;
@@ -358,13 +361,14 @@ __global__ __launch_bounds__(256) void gemm_int8_128x128_kernel(const int8_t* __
     // the values to a point behind the K loop, where every load of the wavefront has returned)
     float early_sa, early_sb[2] = {0.f, 0.f}, early_c[2] = {0.f, 0.f};
 #define EARLY_LOAD(dst, ptr) asm volatile("global_load_dword %0, %1, off" : "=v"(dst) : "v"(ptr) : "memory")
-    EARLY_LOAD(early_sa, a_scales + tile_m * QT + (threadIdx.x & (QT - 1)));
-    EARLY_LOAD(early_sb[0], b_scales + (PER_COL ? col_base : 0));
-    if (PER_COL) EARLY_LOAD(early_sb[1], b_scales + col_base + 1);
+    const int early_row = threadIdx.x & (QT - 1), col0 = RAGGED && col_base >= N ? N - 1 : col_base, col1 = RAGGED && col_base + 1 >= N ? N - 1 : col_base + 1;
+    EARLY_LOAD(early_sa, a_scales + tile_m * QT + (RAGGED && early_row >= rows_a ? rows_a - 1 : early_row));
+    EARLY_LOAD(early_sb[0], b_scales + (PER_COL ? col0 : 0));
+    if (PER_COL) EARLY_LOAD(early_sb[1], b_scales + col1);
     if (BT == 4)
     {
-        EARLY_LOAD(early_c[0], cvec + col_base);
-        EARLY_LOAD(early_c[1], cvec + col_base + 1);
+        EARLY_LOAD(early_c[0], cvec + col0);
+        EARLY_LOAD(early_c[1], cvec + col1);
     }
 #undef EARLY_LOAD
 #define EARLY_ARRIVED asm volatile("s_waitcnt vmcnt(0)" : "+v"(early_sa), "+v"(early_sb[0]), "+v"(early_sb[1]), "+v"(early_c[0]), "+v"(early_c[1]))
@@ -487,7 +491,10 @@ __global__ __launch_bounds__(256) void gemm_int8_128x128_kernel(const int8_t* __
                 if (BT == 4) f = add_rn(f, colc[j]);
                 f2[j] = mul_rn(f, alpha);
             }
-            *reinterpret_cast<float2*>(orow) = make_float2(f2[0], f2[1]);
+            if (!RAGGED || (row_in_tile < rows_a && col_base + 1 < N))
+                *reinterpret_cast<float2*>(orow) = make_float2(f2[0], f2[1]);
+            else if (row_in_tile < rows_a && col_base < N)
+                orow[0] = f2[0];
         }
     }
 }
@@ -549,9 +556,9 @@ constexpr int R_OPERAND = QT * RK;     // 16 KB
 constexpr int R_STAGE = 2 * R_OPERAND; // 32 KB
 constexpr int R_STAGES = 4;
 
-template<bool PER_COL, int BT>
+template<bool PER_COL, int BT, bool RAGGED>
 __global__ __launch_bounds__(256) void gemm_int8_128x128_k128_kernel(const int8_t* __restrict__ A, size_t lda, const int8_t* __restrict__ B, size_t ldb,
-                                                                      int nk, int tiles_m, int tiles_n, const float* __restrict__ a_scales,
+                                                                      int nk, int M, int N, int tiles_m, int tiles_n, const float* __restrict__ a_scales,
                                                                       const float* __restrict__ b_scales, const float* __restrict__ cvec, float alpha,
                                                                       float beta, float* __restrict__ out, size_t ldo)
 {
@@ -580,14 +587,18 @@ __global__ __launch_bounds__(256) void gemm_int8_128x128_k128_kernel(const int8_
     const int ld_chunk = (lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7);
     const int8_t* ua = A + (size_t)tile_m * QT * lda; // uniform
     const int8_t* ub = B + (size_t)tile_n * QT * ldb;
+    // RAGGED: rows past the end repeat the last one and are not stored
+    const int rows_a = RAGGED ? M - tile_m * QT : QT, rows_b = RAGGED ? N - tile_n * QT : QT;
     unsigned off_a[4], off_b[4];
 #pragma unroll
     for (int i = 0; i < 4; i++)
     {
-        const int row_a = (i * 4 + wave) * 8 + (lane >> 3);
+        int row_a = (i * 4 + wave) * 8 + (lane >> 3);
         // LDS row wn*64 + j*32 + l holds B row wn*64 + 2*l + j (two consecutive output columns per lane): here wn = i >> 1, j = i & 1,
         // l = wave*8 + (lane >> 3)
-        const int row_b = (i >> 1) * 64 + 2 * (wave * 8 + (lane >> 3)) + (i & 1);
+        int row_b = (i >> 1) * 64 + 2 * (wave * 8 + (lane >> 3)) + (i & 1);
+        if (RAGGED && row_a >= rows_a) row_a = rows_a - 1;
+        if (RAGGED && row_b >= rows_b) row_b = rows_b - 1;
         off_a[i] = (unsigned)(row_a * lda + ld_chunk * 16);
         off_b[i] = (unsigned)(row_b * ldb + ld_chunk * 16);
     }
@@ -621,13 +632,14 @@ __global__ __launch_bounds__(256) void gemm_int8_128x128_k128_kernel(const int8_
     // the values to a point behind the K loop, where every load of the wavefront has returned)
     float early_sa, early_sb[2] = {0.f, 0.f}, early_c[2] = {0.f, 0.f};
 #define EARLY_LOAD(dst, ptr) asm volatile("global_load_dword %0, %1, off" : "=v"(dst) : "v"(ptr) : "memory")
-    EARLY_LOAD(early_sa, a_scales + tile_m * QT + (threadIdx.x & (QT - 1)));
-    EARLY_LOAD(early_sb[0], b_scales + (PER_COL ? col_base : 0));
-    if (PER_COL) EARLY_LOAD(early_sb[1], b_scales + col_base + 1);
+    const int early_row = threadIdx.x & (QT - 1), col0 = RAGGED && col_base >= N ? N - 1 : col_base, col1 = RAGGED && col_base + 1 >= N ? N - 1 : col_base + 1;
+    EARLY_LOAD(early_sa, a_scales + tile_m * QT + (RAGGED && early_row >= rows_a ? rows_a - 1 : early_row));
+    EARLY_LOAD(early_sb[0], b_scales + (PER_COL ? col0 : 0));
+    if (PER_COL) EARLY_LOAD(early_sb[1], b_scales + col1);
     if (BT == 4)
     {
-        EARLY_LOAD(early_c[0], cvec + col_base);
-        EARLY_LOAD(early_c[1], cvec + col_base + 1);
+        EARLY_LOAD(early_c[0], cvec + col0);
+        EARLY_LOAD(early_c[1], cvec + col1);
     }
 #undef EARLY_LOAD
 #define EARLY_ARRIVED asm volatile("s_waitcnt vmcnt(0)" : "+v"(early_sa), "+v"(early_sb[0]), "+v"(early_sb[1]), "+v"(early_c[0]), "+v"(early_c[1]))
@@ -761,7 +773,10 @@ __global__ __launch_bounds__(256) void gemm_int8_128x128_k128_kernel(const int8_
                 if (BT == 4) f = add_rn(f, colc[j]);
                 f2[j] = mul_rn(f, alpha);
             }
-            *reinterpret_cast<float2*>(orow) = make_float2(f2[0], f2[1]);
+            if (!RAGGED || (row_in_tile < rows_a && col_base + 1 < N))
+                *reinterpret_cast<float2*>(orow) = make_float2(f2[0], f2[1]);
+            else if (row_in_tile < rows_a && col_base < N)
+                orow[0] = f2[0];
         }
     }
 }
@@ -769,17 +784,25 @@ __global__ __launch_bounds__(256) void gemm_int8_128x128_k128_kernel(const int8_
 template<int KSTEP>
 static int launch_128x128(const int8_t* aq, size_t aq_stride, const int8_t* bq, size_t bq_stride, int M, int N, int K, const GemmEpilogue& epi, hipStream_t stream)
 {
-    const int tm = M / QT, tn = N / QT, nk = K / KSTEP;
+    const int tm = (M + QT - 1) / QT, tn = (N + QT - 1) / QT, nk = K / KSTEP;
     dim3 grid(tm * tn), block(256);
-#define LAUNCH(PC, BTV)                                                                                                                              \
+#define LAUNCH_RAGGED(PC, BTV, RAGGED_)                                                                                                              \
     do                                                                                                                                               \
     {                                                                                                                                                \
         if (KSTEP == 128)                                                                                                                            \
-            hipLaunchKernelGGL((gemm_int8_128x128_k128_kernel<PC, BTV>), grid, block, 0, stream, aq, aq_stride, bq, bq_stride, nk, tm, tn,           \
-                               epi.a_scales, epi.b_scales, epi.c, epi.alpha, epi.beta, epi.out, epi.out_stride);                                     \
+            hipLaunchKernelGGL((gemm_int8_128x128_k128_kernel<PC, BTV, RAGGED_>), grid, block, 0, stream, aq, aq_stride, bq, bq_stride, nk, M, N,    \
+                               tm, tn, epi.a_scales, epi.b_scales, epi.c, epi.alpha, epi.beta, epi.out, epi.out_stride);                             \
         else                                                                                                                                         \
-            hipLaunchKernelGGL((gemm_int8_128x128_kernel<PC, BTV, 4>), grid, block, 0, stream, aq, aq_stride, bq, bq_stride, nk, tm, tn,             \
-                               epi.a_scales, epi.b_scales, epi.c, epi.alpha, epi.beta, epi.out, epi.out_stride);                                     \
+            hipLaunchKernelGGL((gemm_int8_128x128_kernel<PC, BTV, 4, RAGGED_>), grid, block, 0, stream, aq, aq_stride, bq, bq_stride, nk, M, N,      \
+                               tm, tn, epi.a_scales, epi.b_scales, epi.c, epi.alpha, epi.beta, epi.out, epi.out_stride);                             \
+    } while (0)
+#define LAUNCH(PC, BTV)                    \
+    do                                     \
+    {                                      \
+        if (M % QT || N % QT)              \
+            LAUNCH_RAGGED(PC, BTV, true);  \
+        else                               \
+            LAUNCH_RAGGED(PC, BTV, false); \
     } while (0)
     if (epi.per_col)
     {
@@ -796,25 +819,30 @@ static int launch_128x128(const int8_t* aq, size_t aq_stride, const int8_t* bq, 
             LAUNCH(false, -1);
     }
 #undef LAUNCH
+#undef LAUNCH_RAGGED
     return launch_status("gemm_int8_128x128_kernel");
 }
 
-// Problems between the few-row kernels and the 256x256 kernel: M and N multiples of 128 (the caller decides from how many tiles up).
-// K % 128 == 0 takes the form with 128-byte K steps, other K % 64 == 0 the form with 64-byte steps.
+// Problems between the few-row kernels and the 256x256 kernel, and those whose M or N is no multiple of 256 (the caller decides from how
+// many tiles up).  K % 128 == 0 takes the form with 128-byte K steps up to one tile a unit (its ring leaves room for one workgroup) and,
+// in whole tiles, for long K, other K % 64 == 0 and the rest the form with 64-byte steps, of which a unit holds two: 128- / 64-byte form, us, 2268 x 1512 x
+// 1152 12.3 / 12.4, 1417 x 2464 x 3968 21.8 / 24.2, 1045 x 5376 x 512 15.8 / 12.7, 2834 x 6048 x 1280 50.6 / 43.4, 1208 x 4472 x 8064 71.8 / 79.6.
 // NCNNHIP_GEMM_RING128 (read at every call): 0 switches both off, 64 forces the 64-byte form.
 int launch_gemm_int8_ring128(const int8_t* aq, size_t aq_stride, const int8_t* bq, size_t bq_stride, int M, int N, int K, const GemmEpilogue& epi,
                              hipStream_t stream, bool* handled)
 {
     *handled = false;
-    if (M % QT || N % QT || K % PK || aq_stride % 16 || bq_stride % 16 || !al16(aq) || !al16(bq)) return NCNNHIP_OK;
+    if (K % PK || aq_stride % 16 || bq_stride % 16 || !al16(aq) || !al16(bq)) return NCNNHIP_OK;
     if (epi.transpose || epi.acc_out || !(epi.bt == -1 || epi.bt == 4)) return NCNNHIP_OK;
     if (epi.out_stride % 2 || (reinterpret_cast<uintptr_t>(epi.out) & 7)) return NCNNHIP_OK; // the epilogue stores 8 bytes per lane
+    if ((long long)((M + QT - 1) / QT) * ((N + QT - 1) / QT) > 0x7fffffff) return NCNNHIP_OK;
     if ((unsigned long long)QT * aq_stride + 256 > 0xffffffffull || (unsigned long long)QT * bq_stride + 256 > 0xffffffffull) return NCNNHIP_OK; // 32-bit lane offsets
     const char* e = getenv("NCNNHIP_GEMM_RING128");
     const int mode = e ? atoi(e) : 128;
     if (mode == 0) return NCNNHIP_OK;
     *handled = true;
-    if (K % RK == 0 && mode != 64) return launch_128x128<128>(aq, aq_stride, bq, bq_stride, M, N, K, epi, stream);
+    const long long tiles = (long long)((M + QT - 1) / QT) * ((N + QT - 1) / QT);
+    if (K % RK == 0 && mode != 64 && (tiles <= 256 || (K > 4096 && M % QT == 0 && N % QT == 0))) return launch_128x128<128>(aq, aq_stride, bq, bq_stride, M, N, K, epi, stream);
     return launch_128x128<64>(aq, aq_stride, bq, bq_stride, M, N, K, epi, stream);
 }
 

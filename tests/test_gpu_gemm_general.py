@@ -3,8 +3,9 @@ bit (src/layer/gemm.cpp:745-966)."""
 import numpy as np
 import pytest
 
+from ncnn_amd.hip import check, lib
 from oracle import oracle
-from tests import cases
+from tests import cases, npref
 
 pytestmark = pytest.mark.gpu
 
@@ -22,8 +23,8 @@ SHAPES = [
     (1, 64, 16), (3, 65, 63), (16, 79, 65), (17, 100, 321), (2, 63, 77), (1, 130, 2047),
     # long K on few tiles: eight wavefronts with runs of several K steps, the last cut
     (70, 65, 3072), (130, 65, 3073), (65, 66, 3200), (64, 64, 3327),
-    # four wavefronts a tile of 32 x 32 from 257 tiles, some without a step; 64 x 64 tiles with eight from 513 tiles and K = 3072
-    (300, 900, 144), (260, 1000, 1039), (16, 9000, 48), (620, 1000, 528), (768, 1024, 80), (530, 1000, 3088),
+    # four wavefronts a tile of 32 x 32 from 257 tiles, some without a step; 64 x 64 tiles with eight from 641 tiles and K = 3072
+    (300, 900, 144), (260, 1000, 1039), (16, 9000, 48), (620, 1000, 528), (768, 1024, 80), (530, 1000, 3088), (896, 768, 3088),
     # beyond the streaming kernel (450 tiles of 32 x 32, 640 or 1024 where rows are aligned): one and two groups of wavefronts per tile of 64 x 64
     (700, 700, 65), (720, 650, 271), (1000, 700, 528), (470, 970, 3073), (465, 990, 3327),
     # 128 x 128 tiles from 1536 tiles of 64 x 64
@@ -43,3 +44,21 @@ def test_gemm_int8_any_shape_equals_the_oracle(rt, m, n, k):
     # the general form of the epilogue: accumulators too, the output transposed
     got, acc = rt.gemm_int8(aq, bq, sa, sb, bias, 4, 0.5, 1.5, output_transpose=True, want_acc=True)
     assert np.array_equal(acc, wacc) and np.array_equal(got.T, want)
+
+
+@pytest.mark.parametrize("m,n,k", [(1793, 1794, 512), (1920, 1802, 576), (1799, 1792, 640), (2050, 2178, 64), (2048, 2178, 192), (2050, 2176, 256)])
+@pytest.mark.parametrize("per_col", [True, False])
+def test_128x128_tiles_cut_at_the_end(rt, m, n, k, per_col):
+    """200 tiles of 128 x 128 and more with a cut last row or column of tiles, in both forms of the K step: rows past the end repeat the
+    last one, and nothing is written outside the output (an odd number of columns in rows of an even stride)."""
+    print("[case]", m, n, k, per_col, flush=True)
+    a, bq, sb, bias = cases.gemm_case(m + n + k, m, n, k, per_col=per_col)
+    aq, sa = rt.gemm_quantize_rows(a)
+    want, _ = npref.gemm_int8(aq, bq, sa, sb, bias, 4, acc=npref.gemm_acc_exact(aq, bq))
+    assert np.array_equal(rt.gemm_int8(aq, bq, sa, sb, bias, 4), want)
+    cols = n - 1
+    da, db, dsa, dsb, dc = rt.up(aq), rt.up(bq), rt.up(sa), rt.up(sb[:cols] if per_col else sb), rt.up(bias.reshape(-1)[:cols])
+    out = rt.up(np.full((m + 1, n + 2), 7.0, np.float32))
+    check(lib().ncnnhip_gemm_int8(da.ptr, k, db.ptr, k, m, cols, k, dsa.ptr, dsb.ptr, cols if per_col else 1, dc.ptr, 4, 1.0, 1.0, 0, out.ptr, n + 2, None, rt.stream))
+    got = out.to_numpy(rt.stream)
+    assert np.array_equal(got[:m, :cols], want[:, :cols]) and np.all(got[:m, cols:] == 7.0) and np.all(got[m] == 7.0)
