@@ -451,9 +451,12 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
  * per head, scores = q k^T (+ mask), softmax over the keys, times v.  q (already scaled) and out are
  * [seq][num_heads*head_dim]; kt / vt are [num_heads*head_dim][dst_seqlen] with row stride kv_stride, the layout of
  * the layer's cache blobs; mask is additive, [src][dst] (mask_heads 1) or [num_heads][src][dst], or NULL.
- * Head dimensions 32/64/96/128 run on the fp32 matrix cores with any dst_seqlen; others need head_dim + dst_seqlen <= 4096.
+ * Head dimensions 32/64/96/128 run on the matrix cores with any dst_seqlen; others need head_dim + dst_seqlen <= 4096.
+ * With the scratch ncnnhip_attention_workspace_bytes asks for (16-byte aligned) and queries enough for it, keys and values are
+ * first split into three bf16 numbers each (6 bytes for every float) for the bf16 matrix cores, six products for one; without
+ * it, or with infinities that those cannot carry, the fp32 matrix cores run.
  * With few queries and many keys (decoding against a cache) the keys are split over workgroups if the caller passes
- * the scratch ncnnhip_attention_workspace_bytes asks for (may be 0 / NULL: then one workgroup per head and 32 queries);
+ * the scratch (may be 0 / NULL: then one workgroup per head and 32 queries);
  * one to four queries on 256 to 32768 keys then run on a streaming kernel of their own (64 keys per workgroup, any
  * head_dim up to 256) followed by a merge. */
 int ncnnhip_attention_workspace_bytes(int num_heads, int head_dim, int src_seqlen, int dst_seqlen, size_t* workspace_bytes);
@@ -470,8 +473,8 @@ int ncnnhip_attention_f32_strided(const float* q_dev, size_t q_stride, float q_s
  * 2*embed_dim): the new keys and values are first written as columns past_seqlen.. of kt / vt (rows of kv_stride >=
  * past_seqlen + src_seqlen; columns 0..past_seqlen-1 hold the cache), then the attention runs over all past_seqlen +
  * src_seqlen keys - what src/layer/multiheadattention.cpp:640-746 does by writing k_affine / v_affine behind the cached
- * columns.  One to four queries on 256 keys and more write the columns inside the attention kernel (no launch of their
- * own); other shapes run ncnnhip_transpose_pair_f32 first.  Workspace as for ncnnhip_attention_f32 with dst_seqlen =
+ * columns.  One to four queries on 256 keys and more write the columns inside the attention kernel, and so does the kernel
+ * that splits keys and values (no launch of their own); other shapes run ncnnhip_transpose_pair_f32 first.  Workspace as for ncnnhip_attention_f32 with dst_seqlen =
  * past_seqlen + src_seqlen. */
 int ncnnhip_attention_f32_append(const float* qkv_dev, size_t qkv_stride, float q_scale, float* kt_dev, float* vt_dev, size_t kv_stride,
                                  int past_seqlen, const float* mask_dev, int mask_heads, int num_heads, int head_dim, int src_seqlen,

@@ -196,39 +196,27 @@ __device__ __forceinline__ float running_softmax_step(v16f_at& s, float& m, floa
     return corr;
 }
 
+// A wavefront's share of the keys [key_begin, key_end) for the 32 queries of its workgroup: maximum, sum and unnormalised output (transposed)
 template<int HD>
-__global__ __launch_bounds__(256) void attention_f32_mfma_kernel(const float* __restrict__ q, const float* __restrict__ kt, const float* __restrict__ vt,
-                                                                 const float* __restrict__ mask, int mask_heads, int embed_dim, int src, int dst,
-                                                                 size_t kv_stride, float* __restrict__ out, int v_vec_ok, int keys_per_split,
-                                                                 float* __restrict__ partial, size_t q_stride, float q_scale)
+__device__ __forceinline__ void attention_share_f32(const float* __restrict__ q, int qi, int h, const float* __restrict__ kt, const float* __restrict__ vt, const float* mrow,
+                                                    int dst, size_t kv_stride, int v_vec_ok, int key_begin, int key_end, size_t q_stride, float q_scale,
+                                                    v16f_at (&o)[HD / 32], float& m, float& l)
 {
-    // keys_per_split > 0: blockIdx.z takes keys [z*keys_per_split, ...) and leaves (m, l, unnormalised o) in `partial`
-    // for attention_merge_kernel; 0: the workgroup sees every key and writes the result
     constexpr int CB = HD / 32;
-    constexpr int LD = 33;
-    __shared__ float o_s[HD * LD];
-    __shared__ float m_s[4][32], l_s[4][32];
-    const int h = blockIdx.y, i0 = blockIdx.x * 32;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hh = lane >> 5;
-    const int qi = i0 + l32 < src ? i0 + l32 : src - 1; // lanes past the last query repeat it; nothing of theirs is stored
-
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, hh = lane >> 5;
     float qreg[HD / 2];
 #pragma unroll
     for (int kk = 0; kk < HD / 2; kk++) qreg[kk] = mul_rn(q[(size_t)qi * q_stride + h * HD + 2 * kk + hh], q_scale);
 
-    v16f_at o[CB];
 #pragma unroll
     for (int cb = 0; cb < CB; cb++)
 #pragma unroll
         for (int r = 0; r < 16; r++) o[cb][r] = 0.f;
-    float m = -FLT_MAX, l = 0.f;
+    m = -FLT_MAX;
+    l = 0.f;
 
     const float* kh = kt + (size_t)h * HD * kv_stride;
     const float* vh = vt + (size_t)h * HD * kv_stride;
-    const float* mrow = mask ? mask + ((size_t)(mask_heads > 1 ? h : 0) * src + qi) * dst : nullptr;
-
-    const int key_begin = keys_per_split > 0 ? (int)blockIdx.z * keys_per_split : 0;
-    const int key_end = keys_per_split > 0 && key_begin + keys_per_split < dst ? key_begin + keys_per_split : dst; // a multiple of 32, or dst
     // Key loads: channel pair kk starts at a wave-uniform address (scalar registers), the lane adds one 32-bit offset that
     // is the same for every kk (the host checks that kv_stride + dst fits) - 64-bit per-lane addresses for 32 rows would
     // cost 64 registers and with them the second wavefront per SIMD.
@@ -336,8 +324,18 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(const float* __
         }
         s_cur = s_next;
     }
+}
 
-    // ---- merge the four shares: common maximum, then each wavefront adds its rescaled part in turn
+// The four wavefronts' shares become the result, or the record of a key split
+template<int HD>
+__device__ __forceinline__ void attention_merge_shares(const v16f_at (&o)[HD / 32], float m, float l, int h, int i0, int src, int embed_dim, float* __restrict__ out,
+                                                       bool split, float* __restrict__ rec)
+{
+    constexpr int CB = HD / 32;
+    constexpr int LD = 33;
+    __shared__ float o_s[HD * LD];
+    __shared__ float m_s[4][32], l_s[4][32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hh = lane >> 5;
     if (hh == 0)
     {
         m_s[wave][l32] = m;
@@ -362,10 +360,9 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(const float* __
         }
         __syncthreads();
     }
-    if (keys_per_split > 0)
+    if (split)
     {
-        // [query block][head][split] records of 32 maxima, 32 sums, 32 x HD outputs (query-major; only real queries are written)
-        float* rec = partial + (((size_t)blockIdx.x * gridDim.y + h) * gridDim.z + blockIdx.z) * (size_t)(64 + HD * 32);
+        // a record: 32 maxima, 32 sums, 32 x HD outputs (query-major; only real queries are written)
         const int nq = src - i0 < 32 ? src - i0 : 32;
         if (tid < 32)
         {
@@ -392,18 +389,337 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(const float* __
     }
 }
 
-// merges the records of the key splits: one workgroup per (query block, head).  First every (split, query) pair gets its factor
+template<int HD>
+__global__ __launch_bounds__(256) void attention_f32_mfma_kernel(const float* __restrict__ q, const float* __restrict__ kt, const float* __restrict__ vt,
+                                                                 const float* __restrict__ mask, int mask_heads, int embed_dim, int src, int dst,
+                                                                 size_t kv_stride, float* __restrict__ out, int v_vec_ok, int keys_per_split,
+                                                                 float* __restrict__ partial, size_t q_stride, float q_scale)
+{
+    // keys_per_split > 0: blockIdx.z takes keys [z*keys_per_split, ...) and leaves (m, l, unnormalised o) in `partial`
+    // for attention_merge_kernel; 0: the workgroup sees every key and writes the result
+    const int h = blockIdx.y, i0 = blockIdx.x * 32, l32 = threadIdx.x & 31;
+    const int qi = i0 + l32 < src ? i0 + l32 : src - 1; // lanes past the last query repeat it; nothing of theirs is stored
+    const float* mrow = mask ? mask + ((size_t)(mask_heads > 1 ? h : 0) * src + qi) * dst : nullptr;
+    const int key_begin = keys_per_split > 0 ? (int)blockIdx.z * keys_per_split : 0;
+    const int key_end = keys_per_split > 0 && key_begin + keys_per_split < dst ? key_begin + keys_per_split : dst; // a multiple of 32, or dst
+    v16f_at o[HD / 32];
+    float m, l;
+    attention_share_f32<HD>(q, qi, h, kt, vt, mrow, dst, kv_stride, v_vec_ok, key_begin, key_end, q_stride, q_scale, o, m, l);
+    // records: [head][query block][split]
+    attention_merge_shares<HD>(o, m, l, h, i0, src, embed_dim, out, keys_per_split > 0,
+                               partial + (((size_t)h * gridDim.x + blockIdx.x) * gridDim.z + blockIdx.z) * (size_t)(64 + HD * 32));
+}
+
+// ---- the same on the bf16 matrix cores, every fp32 number as three bf16 numbers ----------------------------------------
+// x = hi + mid + lo, each the nearest bf16 of what is left: 24 bits, exact, the remainders of either sign.  A product is then the six
+// products hi hi, hi mid, mid hi, mid mid, hi lo, lo hi; what is left out, mid lo, lo mid and lo lo, is at most 2^-23 of it, of random
+// sign.  Six instructions of 32 x 32 x 16 in place of eight of 32 x 32 x 2 at a sixteenth of the rate: 1536 matrix-core cycles for 32 keys
+// and queries at head dimension 64 where the kernel above takes 4096.  The least products are added first.
+// Keys and values are split once, by attention_split_kernel, into the workspace, in operand order: per head and 32 keys the HD / 16 x 3
+// fragments of the keys and the HD / 16 x 3 of the values, 64 lanes x 16 bytes each, so that every load of the core is 1 KB of consecutive
+// memory.  The queries' fragments are made by the workgroup and stay in LDS (in registers, 96 of them at head dimension 64, short sequences
+// run 5 % longer and the longest 2 % shorter).
+// Bound by the matrix cores and the vector unit (softmax, the probabilities' split) of two wavefronts per SIMD: at head dimension 64 an
+// iteration is 1536 cycles of products and takes 4500 for two wavefronts.  16 heads of 64: 1500 queries and keys 134 us -> 82 with
+// attention_split_kernel and the merge, 700: 57 -> 34; 12 of 128, 500: 83 -> 35; 20 of 96, 300 on 600: 75 -> 34.
+// (Three wavefronts per SIMD in 168 registers, eight to a workgroup, or a start at another key for each workgroup: no faster.)
+// An infinity times a part that is zero is no number where the product of the whole was one; a wavefront that ends with one repeats its
+// share with the kernel above's arithmetic.
+typedef __bf16 v8bf_at __attribute__((ext_vector_type(8)));
+
+// two floats -> their three bf16 pairs
+__device__ __forceinline__ void split_pair(float a, float b, unsigned (&part)[3])
+{
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+    {
+        asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(part[p]) : "v"(a), "v"(b));
+        a -= __uint_as_float(part[p] << 16);
+        b -= __uint_as_float(part[p] & 0xFFFF0000u);
+    }
+}
+__device__ __forceinline__ void split_store(const float (&x)[8], uint4* to, int stride) // to, to + stride, to + 2 * stride
+{
+    unsigned f[4][3];
+#pragma unroll
+    for (int e = 0; e < 4; e++) split_pair(x[2 * e], x[2 * e + 1], f[e]);
+#pragma unroll
+    for (int p = 0; p < 3; p++) to[p * stride] = make_uint4(f[0][p], f[1][p], f[2][p], f[3][p]);
+}
+
+// One workgroup: 32 keys of one head.  new_k / new_v (or null): the keys and values of the positions from `past` on, rows of new_stride floats
+// ([position][embed]); they are copied into kt / vt on the way (appending to the cache is then no launch of its own).
+// Bound by memory, with 20 bytes moved for a float (28 for a new one), and on few keys by its latency: every load of a thread is requested
+// before the first is used, and LDS is sized by the head dimension (1500 new keys of 16 heads of 64, 43 MB: 13 us with loads as they come
+// and room for 128 channels in 32 KB).
+template<int HD>
+__global__ __launch_bounds__(256) void attention_split_kernel(float* kt, float* vt, size_t kv_stride, int dst, const float* __restrict__ new_k,
+                                                              const float* __restrict__ new_v, size_t new_stride, int past, uint4* __restrict__ frags)
+{
+    constexpr int EACH = HD / 8, STEPS = HD / 16;
+    __shared__ float tile[2][HD][33];
+    const int j0 = blockIdx.x * 32, h = blockIdx.y, tid = threadIdx.x;
+    const size_t row0 = (size_t)h * HD;
+    const int known = new_k ? past : dst; // columns of kt / vt that are there
+    float x[2][EACH];
+    // channel-major from kt / vt, thread = (key, every eighth channel); position-major from the new rows, consecutive threads = consecutive channels
+    const int key = tid & 31, c0 = tid >> 5, j = j0 + key;
+    if (j0 < known || j0 + 32 > dst) // uniform, like the next: a tile may be of both kinds
+    {
+        const size_t at = (row0 + c0) * kv_stride + j;
+        const bool there = j < known;
+#pragma unroll
+        for (int i = 0; i < EACH; i++)
+        {
+            x[0][i] = there ? kt[at + (size_t)(8 * i) * kv_stride] : 0.f;
+            x[1][i] = there ? vt[at + (size_t)(8 * i) * kv_stride] : 0.f;
+        }
+        if (there || j >= dst)
+        {
+#pragma unroll
+            for (int i = 0; i < EACH; i++)
+            {
+                tile[0][c0 + 8 * i][key] = x[0][i];
+                tile[1][c0 + 8 * i][key] = x[1][i];
+            }
+        }
+    }
+    if (j0 + 32 > known)
+    {
+#pragma unroll
+        for (int i = 0; i < EACH; i++)
+        {
+            const int e = tid + 256 * i, k = e / HD, c = e - k * HD, jn = j0 + k;
+            const bool fresh = jn >= known && jn < dst;
+            const size_t from = (size_t)(fresh ? jn - past : 0) * new_stride + row0 + c;
+            x[0][i] = new_k ? new_k[from] : 0.f;
+            x[1][i] = new_k ? new_v[from] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < EACH; i++)
+        {
+            const int e = tid + 256 * i, k = e / HD, c = e - k * HD, jn = j0 + k;
+            if (jn >= known && jn < dst)
+            {
+                tile[0][c][k] = x[0][i];
+                tile[1][c][k] = x[1][i];
+            }
+        }
+    }
+    __syncthreads();
+    if (j >= known && j < dst)
+    {
+#pragma unroll
+        for (int i = 0; i < EACH; i++)
+        {
+            kt[(row0 + c0 + 8 * i) * kv_stride + j] = tile[0][c0 + 8 * i][key];
+            vt[(row0 + c0 + 8 * i) * kv_stride + j] = tile[1][c0 + 8 * i][key];
+        }
+    }
+    uint4* to = frags + ((size_t)h * gridDim.x + blockIdx.x) * (size_t)(STEPS * 6 * 64);
+    for (int e = tid; e < STEPS * 64; e += 256)
+    {
+        const int step = e >> 6, lane = e & 63, l32 = lane & 31, hh = lane >> 5;
+        float y[8];
+        // keys: lane = key, channels step * 16 + hh * 8 ..; values: step = 32 channels and half of the keys, in the order of the accumulators
+#pragma unroll
+        for (int i = 0; i < 8; i++) y[i] = tile[0][step * 16 + hh * 8 + i][l32];
+        split_store(y, to + step * 3 * 64 + lane, 64);
+#pragma unroll
+        for (int i = 0; i < 8; i++) y[i] = tile[1][(step >> 1) * 32 + l32][(step & 1) * 16 + 8 * (i >> 2) + 4 * hh + (i & 3)];
+        split_store(y, to + (STEPS + step) * 3 * 64 + lane, 64);
+    }
+}
+
+template<int HD>
+__global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attention_bf16x3_kernel(const float* __restrict__ q, const float* __restrict__ kt, const float* __restrict__ vt,
+                                                               const uint4* __restrict__ frags, const float* __restrict__ mask, int mask_heads, int embed_dim, int src,
+                                                               int dst, size_t kv_stride, float* __restrict__ out, int v_vec_ok, int keys_per_split,
+                                                               float* __restrict__ partial, size_t q_stride, float q_scale, int query_blocks, int splits)
+{
+    constexpr int CB = HD / 32, STEPS = HD / 16;
+    __shared__ uint4 q_s[STEPS * 3 * 64];
+    // The query blocks of a head read the same fragments, 384 bytes a key and 32 channels: they follow one another on one die (workgroups are
+    // dealt to the 8 dies in turn), whose L2 then holds a few heads at a time instead of all of them (16 heads of 64, 256 queries, 2304 keys:
+    // 64 us without, 46 with).  With `splits` beyond 1 that many workgroups share a unit's keys.
+    const int T = gridDim.x, die = blockIdx.x & 7, more = T & 7, at = die * (T >> 3) + (die < more ? die : more) + (int)(blockIdx.x >> 3);
+    const int unit = at / splits, z = at - unit * splits;
+    const int h = unit / query_blocks, i0 = (unit - h * query_blocks) * 32;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
+    const int qi = i0 + l32 < src ? i0 + l32 : src - 1; // lanes past the last query repeat it; nothing of theirs is stored
+    const float* mrow = mask ? mask + ((size_t)(mask_heads > 1 ? h : 0) * src + qi) * dst : nullptr;
+    const int key_begin = z * keys_per_split;
+    const int key_end = splits > 1 && key_begin + keys_per_split < dst ? key_begin + keys_per_split : dst; // a multiple of 32, or dst
+
+    for (int step = wave; step < STEPS; step += 4)
+    {
+        const float* from = q + (size_t)qi * q_stride + h * HD + step * 16 + hh * 8;
+        float x[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[i] = mul_rn(from[i], q_scale);
+        split_store(x, q_s + step * 3 * 64 + lane, 64);
+    }
+    __syncthreads();
+
+    union Frag
+    {
+        uint4 u;
+        v8bf_at h;
+    };
+    v16f_at o[CB];
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[cb][r] = 0.f;
+    float m = -FLT_MAX, l = 0.f;
+    // pairs (of the first operand, of the second) in the order they are added
+    constexpr int PA[6] = {1, 0, 2, 0, 1, 0}, PB[6] = {1, 2, 0, 1, 0, 0};
+
+    const int t_first = key_begin / 32 + wave, t_end = (key_end + 31) / 32;
+    const uint4* base = frags + (size_t)h * ((dst + 31) / 32) * (size_t)(STEPS * 6 * 64) + lane;
+    Frag kf[STEPS * 3];
+    auto load_keys = [&](int t) {
+        const uint4* f = base + (size_t)t * (STEPS * 6 * 64);
+#pragma unroll
+        for (int i = 0; i < STEPS * 3; i++) kf[i].u = f[i * 64];
+    };
+    auto scores = [&](v16f_at& s) {
+        unsigned at = lane; // (opaque: the queries' fragments are read again for every tile, not kept in 48 registers)
+        asm volatile("" : "+v"(at));
+#pragma unroll
+        for (int pr = 0; pr < 6; pr++)
+#pragma unroll
+            for (int step = 0; step < STEPS; step++)
+            {
+                Frag qf;
+                qf.u = q_s[(step * 3 + PB[pr]) * 64 + at];
+                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[step * 3 + PA[pr]].h, qf.h, s, 0, 0, 0);
+            }
+    };
+    v16f_at s_cur;
+#pragma unroll
+    for (int r = 0; r < 16; r++) s_cur[r] = 0.f;
+    // pipelined like the kernel above: the scores of the next tile are made while the softmax of this one runs, its keys are requested an
+    // iteration ahead
+    if (t_first < t_end)
+    {
+        load_keys(t_first);
+        scores(s_cur);
+        asm volatile("" : "+v"(s_cur));
+        ATT_PHASE_BOUNDARY();
+        load_keys(t_first + 4 < t_end ? t_first + 4 : t_first);
+    }
+    for (int t = t_first; t < t_end; t += 4)
+    {
+        const int j0 = t * 32;
+        const uint4* vfrom = base + (size_t)t * (STEPS * 6 * 64) + STEPS * 3 * 64;
+        constexpr int VB = CB <= 2 ? CB : 1; // value blocks requested ahead: all of them while the registers last, else one at a time
+        Frag vf[VB * 6];
+        if constexpr (CB <= 2)
+        {
+#pragma unroll
+            for (int i = 0; i < VB * 6; i++) vf[i].u = vfrom[i * 64];
+        }
+        if (mrow)
+        {
+            float mv[16];
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+            {
+                const int key = j0 + 8 * (r >> 2) + 4 * hh + (r & 3);
+                mv[r] = mrow[key < dst ? key : dst - 1];
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) s_cur[r] = add_rn(s_cur[r], mv[r]);
+        }
+        if (j0 + 32 > dst)
+        {
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                if (j0 + 8 * (r >> 2) + 4 * hh + (r & 3) >= dst) s_cur[r] = -INFINITY;
+        }
+        ATT_PHASE_BOUNDARY();
+        v16f_at s_next;
+#pragma unroll
+        for (int r = 0; r < 16; r++) s_next[r] = 0.f;
+        float corr;
+        if (t + 4 < t_end)
+        {
+            scores(s_next);
+            corr = running_softmax_step(s_cur, m, l);
+            // issue order: one product, then five of the vector instructions, while these last
+#pragma unroll
+            for (int i = 0; i < STEPS * 6; i++)
+            {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 20 / STEPS, 0);
+            }
+        }
+        else
+            corr = running_softmax_step(s_cur, m, l);
+        asm volatile("" : "+v"(s_next), "+v"(s_cur));
+        ATT_PHASE_BOUNDARY();
+        load_keys(t + 8 < t_end ? t + 8 : t);
+        ATT_PHASE_BOUNDARY();
+        if (__any(corr != 1.f))
+        {
+#pragma unroll
+            for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) o[cb][r] *= corr;
+        }
+        // the probabilities' parts: registers 8 * s .. + 7 are the second operand of the values' step s
+        Frag pf[2][3];
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+        {
+            unsigned f[4][3];
+#pragma unroll
+            for (int e = 0; e < 4; e++) split_pair(s_cur[8 * s + 2 * e], s_cur[8 * s + 2 * e + 1], f[e]);
+#pragma unroll
+            for (int p = 0; p < 3; p++) pf[s][p].u = make_uint4(f[0][p], f[1][p], f[2][p], f[3][p]);
+        }
+#pragma unroll
+        for (int c0 = 0; c0 < CB; c0 += VB)
+        {
+            if constexpr (CB > 2)
+            {
+#pragma unroll
+                for (int i = 0; i < 6; i++) vf[i].u = vfrom[(c0 * 6 + i) * 64];
+            }
+#pragma unroll
+            for (int s = 0; s < 2; s++)
+#pragma unroll
+                for (int pr = 0; pr < 6; pr++)
+#pragma unroll
+                    for (int c = 0; c < VB; c++)
+                        o[c0 + c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[c * 6 + s * 3 + PA[pr]].h, pf[s][PB[pr]].h, o[c0 + c], 0, 0, 0);
+        }
+        s_cur = s_next;
+    }
+    float nan = l != l ? 1.f : 0.f;
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) nan = o[cb][r] != o[cb][r] ? 1.f : nan;
+    if (__any(nan != 0.f))
+        attention_share_f32<HD>(q, qi, h, kt, vt, mrow, dst, kv_stride, v_vec_ok, key_begin, key_end, q_stride, q_scale, o, m, l);
+    attention_merge_shares<HD>(o, m, l, h, i0, src, embed_dim, out, splits > 1, partial + ((size_t)unit * splits + z) * (size_t)(64 + HD * 32));
+}
+
+// merges the records of the key splits: one workgroup per (head, query block).  First every (split, query) pair gets its factor
 // exp(m_split - m) and the queries their sums, through LDS; then the outputs are added with eight independent loads in
 // flight per thread (a thread that walks the splits for each of its outputs, one dependent load after the other, took 35 us
 // for 64 queries x 16 heads x 11 splits).
-__global__ __launch_bounds__(256) void attention_merge_kernel(const float* __restrict__ partial, int splits, int head_dim, int embed_dim, int src,
-                                                              float* __restrict__ out)
+__global__ __launch_bounds__(256) void attention_merge_kernel(const float* __restrict__ partial, int query_blocks, int splits, int head_dim,
+                                                              int embed_dim, int src, float* __restrict__ out)
 {
     __shared__ float fac[64][32]; // splits <= 64 (attention_key_splits)
     __shared__ float l_all[32];
-    const int h = blockIdx.y, i0 = blockIdx.x * 32;
+    const int unit = blockIdx.x, h = unit / query_blocks, i0 = (unit - h * query_blocks) * 32;
     const size_t rec_size = (size_t)(64 + head_dim * 32);
-    const float* rec0 = partial + ((size_t)blockIdx.x * gridDim.y + h) * splits * rec_size;
+    const float* rec0 = partial + (size_t)blockIdx.x * splits * rec_size;
     const int nq = src - i0 < 32 ? src - i0 : 32;
     const int tid = threadIdx.x;
     for (int e = tid; e < splits * 32; e += 256) fac[e >> 5][e & 31] = rec0[(size_t)(e >> 5) * rec_size + (e & 31)];
@@ -422,9 +738,9 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const float* __res
         l_all[tid] = lt;
     }
     __syncthreads();
-    // the outputs of the block are shared out over gridDim.z workgroups (each makes the factors for itself: they are cheap)
-    const int total = nq * head_dim, share = (total + (int)gridDim.z - 1) / (int)gridDim.z;
-    const int begin = (int)blockIdx.z * share, end = begin + share < total ? begin + share : total;
+    // the outputs of the block are shared out over gridDim.y workgroups (each makes the factors for itself: they are cheap)
+    const int total = nq * head_dim, share = (total + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int begin = (int)blockIdx.y * share, end = begin + share < total ? begin + share : total;
     for (int idx = begin + tid; idx < end; idx += 256)
     {
         const int qq = idx / head_dim, ch = idx - qq * head_dim;
@@ -706,6 +1022,53 @@ static int attention_key_splits(int num_heads, int src, int dst)
     return want < 2 ? 1 : (int)want;
 }
 
+// Splitting the keys and values first costs a launch and 20 bytes of traffic for each of their floats, which the query blocks have to win back:
+// with Q blocks of 32 queries and head dimension D it pays (us, the fp32 kernel and this one)
+//   from D Q = 256 on up to 256 D Q keys x heads: 16 heads of 64, 128 queries: 16.1 13.1 alone, 30.9 27.3 on 1000 keys, 49.7 41.7 on 4000;
+//   16 x 128, 64 queries on 4000: 70.2 59.4; beyond, 32 x 128, 64 queries on 4000: 99 131;
+//   below that up to 64 D Q: 16 x 64, 64 queries: 13.7 12.2 alone, 21.4 18.0 on 250; beyond, on 1000: 21.6 24.8; 32 x 32, 16 queries on 250: 13.9 15.4;
+//   and with 8 blocks always: 16 x 64, 320 queries on 4000: 101 65; 32 x 32 the same: 101 72.
+// One tile of keys for one small block of queries stays where it is: 16 x 64, 5 queries: 10.5 10.9.
+static bool attention_bf16x3_applies(int num_heads, int head_dim, int src, int dst)
+{
+    if (head_dim % 32 != 0 || head_dim > 128 || src <= ATT_TQ) return false;
+    const long long blocks = (src + 31) / 32, width = head_dim * blocks, keys = (long long)num_heads * dst;
+    if (blocks * num_heads > 1 << 20) return false; // the grid is one row of workgroups
+    if (dst <= 32 && head_dim <= 64) return false;
+    return blocks >= 8 || keys <= (width >= 256 ? 256 : 64) * width;
+}
+// Its workgroups run two to a CU up to head dimension 64, else one.  Units (32 queries of a head) that would leave half of these places
+// empty share their keys out over as many workgroups as there are places, at least 128 keys each.  (Rounding up as above, or sharing out
+// the last, partly filled of several rounds: 768 units at 1500 keys 82 us without, 88 with.)
+static int attention_bf16x3_splits(int num_heads, int head_dim, int src, int dst, int& keys_per_split)
+{
+    const long long units = (long long)((src + 31) / 32) * num_heads;
+    long long want = (head_dim <= 64 ? 512 : 256) / units;
+    if (want > dst / 128) want = dst / 128;
+    if (want > 64) want = 64;
+    keys_per_split = 0;
+    if (want < 2) return 1;
+    keys_per_split = (int)((dst + want - 1) / want + 31) / 32 * 32;
+    return (dst + keys_per_split - 1) / keys_per_split;
+}
+static size_t attention_record_bytes(int head_dim) { return (size_t)(64 + head_dim * 32) * sizeof(float); }
+static size_t attention_records_bytes(int num_heads, int head_dim, int src, int dst)
+{
+    const int splits = attention_key_splits(num_heads, src, dst);
+    return splits > 1 ? (size_t)((src + 31) / 32) * num_heads * splits * attention_record_bytes(head_dim) : 0;
+}
+// split keys and values, and behind them the records of the key splits
+static size_t attention_frags_bytes(int num_heads, int head_dim, int dst)
+{
+    return (size_t)num_heads * ((dst + 31) / 32) * (size_t)head_dim * 384;
+}
+static size_t attention_bf16x3_bytes(int num_heads, int head_dim, int src, int dst)
+{
+    int keys_per_split;
+    const int splits = attention_bf16x3_splits(num_heads, head_dim, src, dst, keys_per_split);
+    return attention_frags_bytes(num_heads, head_dim, dst) + (splits > 1 ? (size_t)((src + 31) / 32) * num_heads * splits * attention_record_bytes(head_dim) : 0);
+}
+
 } // namespace ncnnhip
 
 using namespace ncnnhip;
@@ -716,10 +1079,11 @@ int ncnnhip_attention_workspace_bytes(int num_heads, int head_dim, int src_seqle
 {
     NCNNHIP_REQUIRE(num_heads >= 1 && head_dim >= 1 && src_seqlen >= 1 && dst_seqlen >= 1 && workspace_bytes, "ncnnhip_attention_workspace_bytes: bad argument");
     *workspace_bytes = 0;
-    if (head_dim % 32 == 0 && head_dim <= 128)
+    if (head_dim % 32 == 0 && head_dim <= 128) *workspace_bytes = attention_records_bytes(num_heads, head_dim, src_seqlen, dst_seqlen);
+    if (attention_bf16x3_applies(num_heads, head_dim, src_seqlen, dst_seqlen))
     {
-        const int splits = attention_key_splits(num_heads, src_seqlen, dst_seqlen);
-        if (splits > 1) *workspace_bytes = (size_t)((src_seqlen + 31) / 32) * num_heads * splits * (size_t)(64 + head_dim * 32) * sizeof(float);
+        const size_t need = attention_bf16x3_bytes(num_heads, head_dim, src_seqlen, dst_seqlen);
+        if (need > *workspace_bytes) *workspace_bytes = need;
     }
     if (attention_fewq_applies(head_dim, src_seqlen, dst_seqlen))
     {
@@ -788,35 +1152,33 @@ static int attention_dispatch(const float* q_dev, size_t q_stride, float q_scale
                            num_heads * head_dim, src_seqlen, out_dev);
         return launch_status("attention_fewq_split_kernel");
     }
-    if (append_k)
+    hipStream_t st = as_stream(stream);
+    const int e = num_heads * head_dim, mh = mask_dev ? mask_heads : 0, query_blocks = (src_seqlen + 31) / 32;
+    // 16-byte loads of the values need the rows and the start aligned
+    const int v_vec_ok = (kv_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(vt_dev) & 15) == 0) ? 1 : 0;
+    const unsigned units = (unsigned)query_blocks * (unsigned)num_heads;
+    // enough workgroups for the merge: the outputs of a unit shared out over up to 8 of them
+    const auto merge = [&](const float* partial, int splits) {
+        unsigned shares = 1;
+        while (shares < 8 && units * shares < 256 && (unsigned)(32 * head_dim) / (shares * 2) >= 256) shares *= 2;
+        hipLaunchKernelGGL(attention_merge_kernel, dim3(units, shares), dim3(256), 0, st, partial, query_blocks, splits, head_dim, e, src_seqlen,
+                           out_dev);
+    };
+    if (attention_bf16x3_applies(num_heads, head_dim, src_seqlen, dst_seqlen) && workspace_dev && (reinterpret_cast<uintptr_t>(workspace_dev) & 15) == 0
+        && workspace_bytes >= attention_bf16x3_bytes(num_heads, head_dim, src_seqlen, dst_seqlen))
     {
-        // the other kernels read a finished cache: the new columns are written by a launch of their own
-        const int rc = ncnnhip_transpose_pair_f32(append_k, append_v, append_stride, dst_seqlen - past, num_heads * head_dim, kt_dev + past, vt_dev + past, kv_stride, stream);
-        if (rc != NCNNHIP_OK) return rc;
-    }
-    if (head_dim % 32 == 0 && head_dim <= 128)
-    {
-        // 16-byte loads of the values need the rows and the start aligned
-        const int v_vec_ok = (kv_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(vt_dev) & 15) == 0) ? 1 : 0;
-        // few queries (decoding): split the keys over workgroups when the caller brought the scratch for it
-        int splits = attention_key_splits(num_heads, src_seqlen, dst_seqlen);
-        size_t need = 0;
-        if (splits > 1) need = (size_t)((src_seqlen + 31) / 32) * num_heads * splits * (size_t)(64 + head_dim * 32) * sizeof(float);
-        if (splits > 1 && (!workspace_dev || workspace_bytes < need)) splits = 1;
-        int keys_per_split = 0;
-        if (splits > 1)
-        {
-            keys_per_split = ((dst_seqlen + splits - 1) / splits + 31) / 32 * 32;
-            splits = (dst_seqlen + keys_per_split - 1) / keys_per_split;
-        }
-        dim3 grid((unsigned)((src_seqlen + 31) / 32), (unsigned)num_heads, (unsigned)(splits > 1 ? splits : 1));
-        if (splits <= 1) keys_per_split = 0;
-        float* partial = (float*)workspace_dev;
-        const int e = num_heads * head_dim, mh = mask_dev ? mask_heads : 0;
-        hipStream_t st = as_stream(stream);
-#define LAUNCH_ATT(HD_) \
-    hipLaunchKernelGGL(attention_f32_mfma_kernel<HD_>, grid, dim3(256), 0, st, q_dev, kt_dev, vt_dev, mask_dev, mh, e, src_seqlen, dst_seqlen, kv_stride, out_dev, \
-                       v_vec_ok, keys_per_split, partial, q_stride, q_scale)
+        int keys_per_split;
+        const int splits = attention_bf16x3_splits(num_heads, head_dim, src_seqlen, dst_seqlen, keys_per_split);
+        uint4* frags = static_cast<uint4*>(workspace_dev);
+        float* partial = reinterpret_cast<float*>(static_cast<char*>(workspace_dev) + attention_frags_bytes(num_heads, head_dim, dst_seqlen));
+        const dim3 tiles((unsigned)((dst_seqlen + 31) / 32), (unsigned)num_heads), grid(units * (unsigned)splits);
+#define LAUNCH_ATT(HD_)                                                                                                                                            \
+    do                                                                                                                                                             \
+    {                                                                                                                                                              \
+        hipLaunchKernelGGL(attention_split_kernel<HD_>, tiles, dim3(256), 0, st, kt_dev, vt_dev, kv_stride, dst_seqlen, append_k, append_v, append_stride, past, frags); \
+        hipLaunchKernelGGL(attention_bf16x3_kernel<HD_>, grid, dim3(256), 0, st, q_dev, kt_dev, vt_dev, frags, mask_dev, mh, e, src_seqlen, dst_seqlen, kv_stride,  \
+                           out_dev, v_vec_ok, keys_per_split, partial, q_stride, q_scale, query_blocks, splits);                                 \
+    } while (0)
         if (head_dim == 32)
             LAUNCH_ATT(32);
         else if (head_dim == 64)
@@ -826,13 +1188,42 @@ static int attention_dispatch(const float* q_dev, size_t q_stride, float q_scale
         else
             LAUNCH_ATT(128);
 #undef LAUNCH_ATT
-        if (keys_per_split > 0)
+        if (splits > 1) merge(partial, splits);
+        return launch_status("attention_bf16x3_kernel");
+    }
+    if (append_k)
+    {
+        // the other kernels read a finished cache: the new columns are written by a launch of their own
+        const int rc = ncnnhip_transpose_pair_f32(append_k, append_v, append_stride, dst_seqlen - past, e, kt_dev + past, vt_dev + past, kv_stride, stream);
+        if (rc != NCNNHIP_OK) return rc;
+    }
+    if (head_dim % 32 == 0 && head_dim <= 128)
+    {
+        // few queries (decoding): split the keys over workgroups when the caller brought the scratch for it
+        int splits = attention_key_splits(num_heads, src_seqlen, dst_seqlen);
+        if (splits > 1 && (!workspace_dev || workspace_bytes < attention_records_bytes(num_heads, head_dim, src_seqlen, dst_seqlen))) splits = 1;
+        int keys_per_split = 0;
+        if (splits > 1)
         {
-            // enough workgroups for the chip: the outputs of a (query block, head) shared out over up to 8 of them
-            unsigned shares = 1;
-            while (shares < 8 && grid.x * grid.y * shares < 256 && (unsigned)(32 * head_dim) / (shares * 2) >= 256) shares *= 2;
-            hipLaunchKernelGGL(attention_merge_kernel, dim3(grid.x, grid.y, shares), dim3(256), 0, st, partial, splits, head_dim, e, src_seqlen, out_dev);
+            keys_per_split = ((dst_seqlen + splits - 1) / splits + 31) / 32 * 32;
+            splits = (dst_seqlen + keys_per_split - 1) / keys_per_split;
         }
+        dim3 grid((unsigned)query_blocks, (unsigned)num_heads, (unsigned)(splits > 1 ? splits : 1));
+        if (splits <= 1) keys_per_split = 0;
+        float* partial = (float*)workspace_dev;
+#define LAUNCH_ATT(HD_)                                                                                                                                  \
+    hipLaunchKernelGGL(attention_f32_mfma_kernel<HD_>, grid, dim3(256), 0, st, q_dev, kt_dev, vt_dev, mask_dev, mh, e, src_seqlen, dst_seqlen, kv_stride, \
+                       out_dev, v_vec_ok, keys_per_split, partial, q_stride, q_scale)
+        if (head_dim == 32)
+            LAUNCH_ATT(32);
+        else if (head_dim == 64)
+            LAUNCH_ATT(64);
+        else if (head_dim == 96)
+            LAUNCH_ATT(96);
+        else
+            LAUNCH_ATT(128);
+#undef LAUNCH_ATT
+        if (keys_per_split > 0) merge(partial, splits);
         return launch_status("attention_f32_mfma_kernel");
     }
     const size_t lds = (size_t)ATT_TQ * ((size_t)head_dim + (size_t)dst_seqlen) * sizeof(float);

@@ -350,7 +350,7 @@ int MultiHeadAttention_hip::forward(const std::vector<Mat>& bottom_blobs, std::v
     rc = ncnnhip_attention_workspace_bytes(num_heads, head_dim, src, dst, &att_ws_bytes);
     if (rc != 0) return to_ncnn_status(rc, "ncnnhip_attention_workspace_bytes");
     void* att_ws = att_ws_bytes ? leases.get(att_ws_bytes) : 0;
-    if (att_ws_bytes && !att_ws) return -100;
+    if (!att_ws) att_ws_bytes = 0; // no room: the call falls back to the kernel that needs none
     if (fused_qkv) // the new key and value columns are written behind the cache by the same call
         rc = ncnnhip_attention_f32_append(d_qa, q_stride, scale, d_kt, d_vt, (size_t)dst, past, d_mask, mask_heads, num_heads, head_dim, src, d_ctx, att_ws, att_ws_bytes, st);
     else
@@ -516,7 +516,7 @@ int MultiHeadAttention_hip::forward_hip(const std::vector<HipMat>& bottom_blobs,
     rc = ncnnhip_attention_workspace_bytes(num_heads, head_dim, src, dst, &att_ws_bytes);
     if (rc != 0) return to_ncnn_status(rc, "ncnnhip_attention_workspace_bytes");
     void* att_ws = att_ws_bytes ? scratch.get(att_ws_bytes) : 0;
-    if (att_ws_bytes && !att_ws) return -100;
+    if (!att_ws) att_ws_bytes = 0; // no room: the call falls back to the kernel that needs none
     if (fused_qkv) // the new key and value columns are written behind the cache by the same call
         rc = ncnnhip_attention_f32_append(d_qa, q_stride, scale, d_kt, d_vt, (size_t)dst, past, d_mask, mask_heads, num_heads, head_dim, src, d_ctx, att_ws, att_ws_bytes, st);
     else

@@ -797,6 +797,62 @@ def test_attention_core_matches_float64(rt, heads, hd, src, dst, mask):
     assert np.abs(plain - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
 
 
+@pytest.mark.parametrize("heads,hd,src,dst,mask", [(3, 32, 33, 33, None), (2, 96, 5, 31, "2d"), (1, 128, 32, 64, None), (5, 32, 130, 129, "3d"), (3, 64, 95, 515, "2d"),
+                                                    (20, 96, 300, 601, None), (7, 128, 257, 96, "3d"), (16, 64, 256, 2304, None), (1, 64, 6, 4096, "2d"), (9, 32, 2049, 40, None)])
+def test_attention_core_on_split_keys_and_values(rt, heads, hd, src, dst, mask):
+    """The bf16 form (three bf16 numbers for one fp32): part-filled tiles of keys and queries, one key tile and many, keys shared out
+    over workgroups or not.  x = hi + mid + lo keeps all 24 bits and what the six products leave out is 2^-23 of a product: no more
+    error against float64 than the fp32 form, which runs without the scratch, with too little of it and with an unaligned one."""
+    from ncnn_amd.hip import DeviceBuffer, check, lib
+    rng = np.random.default_rng(heads * 1000 + src)
+    e = heads * hd
+    q = (rng.normal(0, 1, (src, e)) / np.sqrt(hd)).astype(F)
+    kt, vt = (rng.normal(0, 1, (e, dst)).astype(F) for _ in range(2))
+    m = None
+    if mask:
+        m = rng.normal(0, 1, (src, dst) if mask == "2d" else (heads, src, dst)).astype(F)
+        m[..., 1:][rng.random(m[..., 1:].shape) < 0.3] = -np.finfo(F).max
+    size = C.c_size_t()
+    check(lib().ncnnhip_attention_workspace_bytes(heads, hd, src, dst, C.byref(size)))
+    assert size.value >= heads * ((dst + 31) // 32) * hd * 384
+    got = rt.attention(q, kt, vt, heads, m)
+    plain = rt.attention(q, kt, vt, heads, m, use_workspace=False)
+    want = np.empty((src, e))
+    for h in range(heads):
+        sl = slice(h * hd, (h + 1) * hd)
+        s = q[:, sl].astype(np.float64) @ kt[sl].astype(np.float64)
+        if m is not None:
+            s = s + (m if m.ndim == 2 else m[h]).astype(np.float64)
+        s = np.exp(s - s.max(axis=1, keepdims=True))
+        want[:, sl] = (s / s.sum(axis=1, keepdims=True)) @ vt[sl].astype(np.float64).T
+    assert np.sqrt(np.mean((got - want) ** 2)) <= np.sqrt(np.mean((plain - want) ** 2))
+    assert np.abs(got - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
+
+    dq, dk, dv = rt.up(q), rt.up(kt), rt.up(vt)
+    dm = None if m is None else rt.up(m)
+    ws = DeviceBuffer.empty((size.value + 16,), np.uint8)
+    for skip, short in ((4, 0), (0, 16)):  # (the key splits of the fp32 form may still be made: not bit for bit)
+        out = DeviceBuffer.empty((src, e), F)
+        check(lib().ncnnhip_attention_f32(dq.ptr, dk.ptr, dv.ptr, dst, 0 if dm is None else dm.ptr, 0 if m is None else (1 if m.ndim == 2 else heads), heads, hd, src, dst,
+                                          out.ptr, ws.ptr.value + skip, size.value - short, rt.stream))
+        assert np.abs(out.to_numpy(rt.stream) - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
+
+
+@pytest.mark.parametrize("heads,hd,src,dst", [(2, 64, 40, 100), (1, 128, 70, 300)])
+def test_attention_core_on_split_keys_and_values_with_numbers_it_cannot_carry(rt, heads, hd, src, dst):
+    rng = np.random.default_rng(src)
+    e = heads * hd
+    q = (rng.normal(0, 1, (src, e)) / np.sqrt(hd)).astype(F)
+    kt, vt = (rng.normal(0, 1, (e, dst)).astype(F) for _ in range(2))
+    vt[3, 5], vt[7, dst - 1], vt[e - 1, 2], vt[e - 2, 9] = np.inf, -np.inf, np.nan, np.finfo(F).max
+    q[1, 4] = 0
+    kt[4, 11] = np.finfo(F).max  # times zero for query 1; rounded to bf16 it is infinite
+    got, plain = rt.attention(q, kt, vt, heads), rt.attention(q, kt, vt, heads, use_workspace=False)
+    assert np.array_equal(np.isnan(got), np.isnan(plain)) and np.array_equal(np.isinf(got), np.isinf(plain))
+    ok = np.isfinite(plain)
+    assert ok.any() and not ok.all() and np.abs(got[ok] / np.maximum(np.abs(plain[ok]), 1.0) - plain[ok] / np.maximum(np.abs(plain[ok]), 1.0)).max() <= 2e-5
+
+
 @pytest.mark.parametrize("heads,hd,src,dst", [(4, 64, 37, 200), (2, 32, 1, 300), (3, 24, 5, 40)])
 def test_attention_reads_strided_queries_and_scales_them_on_load(rt, heads, hd, src, dst):
     """Queries taken out of a wider row (q, k and v made by one Gemm) and multiplied by the layer's scale where they are read:
