@@ -9,7 +9,7 @@ CSRC = os.path.join(PKG, "csrc")
 LIBDIR = os.path.join(PKG, "lib")
 LIBNCNNHIP = os.path.join(LIBDIR, "libncnnhip.so")
 
-HIP_SOURCES = ["runtime.hip", "quantize.hip", "gemm_int8.hip", "gemm_int8_pipelined.hip", "gemm_int8_general.hip", "conv_int8.hip", "conv_nhwc.hip", "conv_nhwc_pipelined.hip", "conv_nhwc_pipelined_split.hip", "conv_nhwc_pipelined_staged.hip", "conv_pointwise.hip", "conv_resident.hip", "conv_patch.hip", "nhwc_ops.hip", "attention.hip", "blockquant.hip", "blockquant_rows.hip", "peaks.hip"]
+HIP_SOURCES = ["runtime.hip", "quantize.hip", "gemm_int8.hip", "gemm_int8_pipelined.hip", "gemm_int8_general.hip", "conv_int8.hip", "conv_nhwc.hip", "conv_nhwc_pipelined.hip", "conv_nhwc_pipelined_split.hip", "conv_nhwc_pipelined_staged.hip", "conv_pointwise.hip", "conv_resident.hip", "conv_patch.hip", "nhwc_ops.hip", "attention.hip", "blockquant.hip", "blockquant_rows.hip", "blockquant_tiles.hip", "peaks.hip"]
 
 # -ffp-contract=off: the reference arithmetic is separate mul and add, never FMA.
 # packed-fp32 ops are switched off for this pool's gfx950 parts.
@@ -21,7 +21,7 @@ HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-cont
 # per-file additions.  blockquant.hip: matrix-core results that go straight into vector arithmetic (the per-block descale) stay in
 # VGPRs instead of AGPRs, which saves a register read per value (tiled kernel 135 -> 125 us at 1024 x 4096 x 4096).
 # attention.hip: the same for the scores and the context on their way into the softmax arithmetic (attention core of 1500 tokens 183 -> 155 us).
-HIPCC_FILE_FLAGS = {"blockquant.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "blockquant_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+HIPCC_FILE_FLAGS = {"blockquant.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "blockquant_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "blockquant_tiles.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                     "conv_pointwise.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "conv_resident.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 

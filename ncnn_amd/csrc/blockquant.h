@@ -205,6 +205,10 @@ int launch_blockquant_rows_f16(const uint16_t* a, size_t a_stride, int M, int K,
 double blockquant_rows_f32_us(int M, int K, long long tiles, int* mg, int* rt);
 int launch_blockquant_rows_f32(const float* a, size_t a_stride, int M, int K, int bits, int block, const float* in_scales, const BqMulti& mm, hipStream_t stream);
 
+// Many rows of fp32 activations, weights in blocks of 64 or 128 (blockquant_tiles.hip); the workspace is that of ncnnhip_gemm_blockquant_packed_rows.
+int launch_blockquant_tiles(const float* a, size_t a_stride, int M, int N, int K, int bits, const unsigned char* wpk, const float4* dpk, const float* in_scales,
+                            const float* c, int bt, float alpha, float beta, float* out, size_t out_stride, void* workspace, hipStream_t stream);
+
 } // namespace ncnnhip
 
 #endif // NCNNHIP_BLOCKQUANT_H

@@ -1523,19 +1523,17 @@ __global__ __launch_bounds__(256) void blockquant_rows_bf16x3_kernel(const unsig
 // half a step apart: while one reads and converts its operands, the other, on the same SIMDs, multiplies.  A stage is refilled as
 // soon as its operands are in registers, one and a half steps before they are due.
 // Bound by the issue slots of the conversions and the clock (1.6 to 2.1 GHz under this load); us with the split pass, 8 bits,
-// kernel above -> this one: 256 x 4096 x 4096 64 -> 50, 100 x 4096 x 11008 135 -> 93, 512 x 1024 x 1024 22.7 -> 19.3 (RW = 2);
-// 512 x 4096 x 4096 90 -> 78, 512 x 4096 x 11008 209 -> 178, 300 x 5120 x 5120 100 -> 86 (RW = 4).  Without the half step's
-// distance 512 x 4096 x 4096 took 85 us.  Error against 64 bits at that size: 1.79e-7 above, 1.44e-7 here.
-template<int BITS, bool HALVES, int RW>
+// kernel above -> this one: 256 x 4096 x 4096 64 -> 50, 100 x 4096 x 11008 135 -> 93, 512 x 1024 x 1024 22.7 -> 19.3.
+template<int BITS, bool HALVES>
 __global__ __launch_bounds__(512) void blockquant_rows_ksplit_bf16x3_kernel(const unsigned short* __restrict__ planes, int Mp, int Kp, int M, int N, int kblocks,
                                                                       int ntiles, const unsigned char* __restrict__ wpk, const float4* __restrict__ dpk, int split,
                                                                       const float* __restrict__ c, int bt, float alpha, float beta, float* __restrict__ out,
                                                                       size_t out_stride)
 {
     static_assert(HALVES || BITS == 8, "4- and 6-bit fields come in the halves layout");
-    static_assert(RW == 2 || RW == 4, "a tile of 16 weight rows is fetched by one of the two wavefronts that multiply it");
     constexpr int STAGES = 2;
-    constexpr int RWL = RW / 2;        // weight tiles a wavefront fetches
+    constexpr int RW = 2;              // weight tiles a wavefront multiplies
+    constexpr int RWL = RW / 2;        // and fetches (each is multiplied by two)
     constexpr int LOADS = 6 + 2 * RWL; // per wavefront and stage
     constexpr int CW = 2;              // groups of 16 activation rows a wavefront multiplies
     constexpr int PLANE = 64 * 128;
@@ -2457,16 +2455,20 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
     hipStream_t st = as_stream(stream);
     const float4* dpk = reinterpret_cast<const float4*>(packed_descale_dev);
     const int split = block == 32 ? 1 : 0;
-    // One launch without the split pass, where that is quicker than the tiled kernel after it, which takes about 9.5 us + K / 1024 x 8.25
-    // us in one round of 64 x 64 tiles on 256 units, 15 in one of 512, then 18 per 512 tiles (18 shapes, 97 to 482 rows; 5 % less here, so
-    // that it stays where the two are close).  us before (the
+    // One launch without the split pass, where that is quicker than the tiled kernels after it, which take about 9.5 us + K / 1024 x 8.25
+    // us in one round of 64 x 64 tiles on 256 units; beyond, in blocks of 32, 15 in one of 512, then 18 per 512 tiles (18 shapes, 97 to 482
+    // rows), in larger blocks 11 us + K / 1024 x 11.5 for every round of 256 64 x 128 tiles; 5 % less here, so that it stays where the two are
+    // close.  us before (the
     // better of the two below) / here: 8 bits, 4096 x 4096 16 rows 12.4 / 10.7, 32 20.1 / 12.9, 64 34 / 17.5, 128 41 / 30; 11008 x 4096 16
     // rows 26.5 / 16.6, 32 46 / 26.5; 4096 x 11008 64 rows 84 / 40, 128 93 / 66; 4 bits, 1730 x 1472 186 rows 21.4 / 12.0, 734 x 6016 477
     // rows 61 / 30.  Its 16-byte loads need aligned rows.
     const bool aligned = al16(a_dev) && a_stride % 4 == 0 && (!in_scales_dev || al16(in_scales_dev));
     const long long tiles64 = (long long)((ntiles + 3) / 4) * (Mp / 64);
+    const double rounds = (double)(((long long)((ntiles + 7) / 8) * (Mp / 64) + 255) / 256); // of 64 x 128 tiles
     int mg, rt;
-    if (aligned && blockquant_rows_f32_us(M, K, ntiles, &mg, &rt) < 9.0 + K / 1024.0 * (tiles64 <= 256 ? 7.8 : tiles64 <= 512 ? 14.2 : 17.0 * tiles64 / 512.0))
+    if (aligned
+        && blockquant_rows_f32_us(M, K, ntiles, &mg, &rt)
+               < 9.0 + K / 1024.0 * (tiles64 <= 256 ? 7.8 : block != 32 ? 11.0 * rounds : tiles64 <= 512 ? 14.2 : 17.0 * tiles64 / 512.0))
         return launch_blockquant_rows_f32(a_dev, a_stride, M, K, bits, block, in_scales_dev, one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride),
                                           st);
     // Which form: the 16-row passes (all in one launch, spread over the chip; every pass streams the weights again, from L2
@@ -2502,17 +2504,26 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
 #undef ROWS16
         return launch_status("blockquant_rows16_bf16x3_kernel");
     }
+    // More than one 64 x 64 tile per compute unit: the kernel with 64 x 128 tiles (one scale a step: not blocks of 32).  It is quicker there
+    // at every K and N measured (1.02 to 1.44 times, 120 shapes of 65 to 1500 rows, K 512 to 11008), with one exception: 8-bit fields in just
+    // over two rounds of it where the kernel below has one round of 64 x 192 tiles, two to a unit (K = 4096, 544 tiles of 64 x 128: 132.6
+    // us below, 140.1 there; 672: 146 148; 704: 150.5 150.1; at 512 115 105 and at 768 182 155).  With fewer tiles the kernel below that
+    // splits K over two groups puts more units to work (128 tiles of 64 x 128, 256 x 4096 x 4096: 45.7 us against 47.7).
+    const long long tiles128 = (long long)((ntiles + 7) / 8) * (Mp / 64), tiles192 = (long long)((ntiles + 11) / 12) * (Mp / 64);
+    const bool one_round = !halves && tiles128 > 512 && tiles192 <= 448;
+    if (block != 32 && tiles64 > 256 && !one_round)
+        return launch_blockquant_tiles(a_dev, a_stride, M, N, K, bits, packed_w_dev, dpk, in_scales_dev, c_dev, bt, alpha, beta, out_dev, out_stride, workspace_dev, st);
     unsigned short* planes = static_cast<unsigned short*>(workspace_dev);
     const size_t vectors = (size_t)Mp * (Kp / 8);
     hipLaunchKernelGGL(blockquant_split_activations_kernel, dim3((unsigned)((vectors + 256 * SPLIT_VECS - 1) / (256 * SPLIT_VECS))), dim3(256), 0, st, a_dev, a_stride, M, K, in_scales_dev, planes, Mp,
                        Kp);
     // Two tiles per wavefront and two stages: 66 KB of LDS, so two workgroups share a compute unit and one's loads, waits and
     // vector work overlap the other's matrix-core instructions.  Measured at 1024 x 4096 x 4096 / 2048 x 11008 x 4096: 135 / 616 us
-    // (138 / 568 -> 128 to 133 / 553 to 574 since the converted pairs are packed by one byte permute; the figures below are from before);
+    // (138 / 568 -> 128 to 133 / 553 to 574 since the converted pairs are packed by one byte permute; the figures below are from before, and
+    // all from 8-bit fields in blocks of 64, of which most go to the kernel with 64 x 128 tiles now);
     // four tiles per wavefront with three stages (one workgroup per unit, half the LDS reads per instruction) 145 / 714 us; two
     // tiles with four stages (one workgroup per unit) 172 / 795 us.  While that leaves fewer workgroups than the chip has compute
-    // units, one tile per wavefront (64 weight rows per workgroup) doubles them: 128 x 4096 x 4096 77 -> 58 us, 256 rows 82 -> 63,
-    // 512 x 1024 x 1024 28.6 -> 22.3.
+    // units, one tile per wavefront (64 weight rows per workgroup) doubles them.
     // One, two or three tiles per wavefront (64, 128 or 192 weight rows per workgroup).  The chip holds 512 workgroups at once:
     // where some choice fits in one round, the one with the most workgroups; else the fewest rounds weighted by a
     // workgroup's cost (0.68 : 1 : 1.4, measured).  1500 x 3072 x 1024 is 576 workgroups with two tiles - a second round
@@ -2542,19 +2553,10 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
             }
         }
     }
-    // Up to one 64 x 64 tile per compute unit, the kernel that splits K inside the workgroup, one tile each; between that and one
-    // 64 x 128 tile per unit, the same with the larger tile, for 8-bit weights in the plain layout and K from 1536: 700 x 1536 x
-    // 1536 37.2 -> 35.3 us, 1000 x 2048 x 2048 52 -> 48, but an attention layer's 1500 x 1024 x 1024 was 1.5 us slower.  With the halves layout (two
-    // scales a step, and 4- or 6-bit fields) the larger tile measured no better than this file's other kernel: 4 bits, 512 x 4096 x
-    // 4096 83.0 against 83.4 us, 700 x 1536 x 1536 36 against 35; the smaller tile is better there too (256 x 4096 x 4096 59 -> 53).
-    // Beyond a round of the chip the two workgroups a unit holds of the other kernel win: 1024 x 4096 x 4096 128 against 140 us.
-    int ks_tiles = 0;
-    if ((long long)((ntiles + 3) / 4) * (Mp / 64) <= 256)
-        ks_tiles = 2;
-    else if (!halves && kblocks >= 24 && (long long)((ntiles + 7) / 8) * (Mp / 64) <= 256)
-        ks_tiles = 4;
+    // Up to one 64 x 64 tile per compute unit, the kernel that splits K inside the workgroup: 4 bits, 256 x 4096 x 4096 59 -> 53 us.
+    const bool ksplit = tiles64 <= 256;
     // (a ring of four stages where a workgroup has its compute unit to itself measured the same as two: 57.6 against 57.8 us at 128 x 4096 x 4096)
-    const int wg_tiles = ks_tiles ? 2 * ks_tiles : 4 * rw_tiles;
+    const int wg_tiles = ksplit ? 4 : 4 * rw_tiles;
     const dim3 grid((ntiles + wg_tiles - 1) / wg_tiles, Mp / 64);
 #define ROWS_LAUNCH(KERNEL_, THREADS_, LDS_)                                                                                                                        \
     do                                                                                                                                                             \
@@ -2572,30 +2574,29 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
     } while (0)
 #define ROWS_RW(BITS_, HALVES_, RW_) \
     ROWS_LAUNCH((blockquant_rows_bf16x3_kernel<BITS_, HALVES_, 2, RW_>), 256, (size_t)2 * (3 * 64 * 128 + 4 * (RW_) * 1024 + 4 * (RW_) * 128))
-#define ROWS_KS(BITS_, HALVES_, RW_) \
-    ROWS_LAUNCH((blockquant_rows_ksplit_bf16x3_kernel<BITS_, HALVES_, RW_>), 512, (size_t)4 * (3 * 64 * 128 + 2 * (RW_) * 1024 + 2 * (RW_) * 128))
-#define ROWS(BITS_, HALVES_)             \
-    do                                   \
-    {                                    \
-        if (ks_tiles == 2)               \
-            ROWS_KS(BITS_, HALVES_, 2);  \
-        else if (rw_tiles == 1)          \
-            ROWS_RW(BITS_, HALVES_, 1);  \
-        else if (rw_tiles == 3)          \
-            ROWS_RW(BITS_, HALVES_, 3);  \
-        else                             \
-            ROWS_RW(BITS_, HALVES_, 2);  \
+#define ROWS_KS(BITS_, HALVES_) ROWS_LAUNCH((blockquant_rows_ksplit_bf16x3_kernel<BITS_, HALVES_>), 512, (size_t)4 * (3 * 64 * 128 + 4 * 1024 + 4 * 128))
+#define ROWS(BITS_)                  \
+    do                               \
+    {                                \
+        if (ksplit)                  \
+            ROWS_KS(BITS_, true);    \
+        else if (rw_tiles == 1)      \
+            ROWS_RW(BITS_, true, 1); \
+        else if (rw_tiles == 3)      \
+            ROWS_RW(BITS_, true, 3); \
+        else                         \
+            ROWS_RW(BITS_, true, 2); \
     } while (0)
-    if (ks_tiles == 4)
-        ROWS_KS(8, false, 4);
-    else if (!halves)
-        ROWS(8, false);
+    if (!halves && ksplit)
+        ROWS_KS(8, false);
+    else if (!halves) // (one_round: three tiles it is)
+        ROWS_RW(8, false, 3);
     else if (bits == 8)
-        ROWS(8, true);
+        ROWS(8);
     else if (bits == 6)
-        ROWS(6, true);
+        ROWS(6);
     else
-        ROWS(4, true);
+        ROWS(4);
 #undef ROWS
 #undef ROWS_KS
 #undef ROWS_RW

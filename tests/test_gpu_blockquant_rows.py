@@ -176,3 +176,38 @@ def test_several_matrices_of_fp32_rows_get_the_bits_of_single_calls(rt, m, k):
     mats = [rt.blockquant_pack(p, s, 64, k=k) + (n, None, -1, 1.0, 1.0) for (_, p, s), n in zip(ops, ns)]
     for got, (pw, pd, n, *_) in zip(rt.gemm_blockquant_packed_multi(a, mats), mats):
         assert np.array_equal(got, rt.gemm_blockquant_packed(a, pw, pd, n))
+
+
+@pytest.mark.parametrize("m,n,k", [(1030, 1000, 16), (1100, 1000, 64), (1030, 970, 80), (523, 1960, 144), (65, 8250, 208), (1025, 1010, 320), (260, 3300, 1040), (1090, 960, 1568),
+                                   (2060, 2050, 80)])
+@pytest.mark.parametrize("bits,block", [(8, 64), (8, 128), (6, 64), (4, 128)])
+def test_fp32_rows_in_64x128_tiles(rt, m, n, k, bits, block):
+    """More than 256 tiles of 64 x 64 (in the last shape the plain layout takes 64 x 192 ones): row blocks and weight tiles cut off, K groups of no, one and several steps, the last of them ragged;
+    with input scales and C, rows off 16 bytes, an infinity and a NaN (no special value beyond its own row)."""
+    print("[case]", m, n, k, bits, block, flush=True)
+    a, packed, scales = synth.blockquant_operands(m + n + k, m, n, k, bits, block, half_exact=False)
+    rng = np.random.default_rng(n)
+    c, ins = rng.normal(size=(m, n)).astype(F), rng.uniform(0.5, 2.0, k).astype(F)
+    pw, pd = rt.blockquant_pack(packed, scales, block, bits=bits, k=k)
+    got = rt.gemm_blockquant_packed(a, pw, pd, n, c, 3, 0.75, 1.5, bits=bits, block=block, in_scales=ins, rows_kernel=True)
+    val, floor = npref.blockquant_gemm_f64(a, packed, scales, bits, block, ins, c, 3, 0.75, 1.5)
+    assert np.all(np.abs(got - val) <= 1e-5 * floor + 1e-30)
+
+    w, d = rt.up(pw), rt.up(pd)
+    size = C.c_size_t()
+    check(lib().ncnnhip_gemm_blockquant_packed_rows_workspace_bytes(m, k, C.byref(size)))
+    ws = DeviceBuffer.empty((size.value,), np.uint8)
+    a[1, k - 1], a[m - 1, 0] = np.inf, np.nan
+    buf = np.full(m * (k + 3) + 8, np.nan, F)
+    buf[1:1 + m * (k + 3)].reshape(m, k + 3)[:, :k] = a
+    src, dst = rt.up(buf), rt.up(np.full(m * (n + 1) + 8, 7.0, F))
+    check(lib().ncnnhip_gemm_blockquant_packed_rows(C.c_void_p(src.ptr.value + 4), k + 3, m, n, k, w.ptr, d.ptr, bits, block, None, None, -1, 1.0, 1.0,
+                                                    C.c_void_p(dst.ptr.value + 4), n + 1, ws.ptr, size.value, rt.stream))
+    out = dst.to_numpy(rt.stream)
+    got = out[1:1 + m * (n + 1)].reshape(m, n + 1)
+    assert np.all(got[:, n] == 7.0) and out[0] == 7.0 and np.all(out[1 + m * (n + 1):] == 7.0)
+    rows = [i for i in range(m) if i not in (1, m - 1)]
+    val, floor = npref.blockquant_gemm_f64(a[rows], packed, scales, bits, block)
+    assert np.all(np.abs(got[rows, :n] - val) <= 1e-5 * floor + 1e-30)
+    q = npref.blockquant_gemm_f64(np.eye(k, dtype=F)[k - 1:], packed, scales, bits, block)[0][0]  # the weights that meet the infinity
+    assert np.array_equal(got[1, :n][q != 0], np.where(q > 0, np.inf, -np.inf)[q != 0].astype(F)) and np.all(np.isnan(got[1, :n][q == 0])) and np.all(np.isnan(got[m - 1, :n]))
