@@ -485,16 +485,18 @@ int launch_blockquant_rows_f16(const uint16_t* a, size_t a_stride, int M, int K,
     // to 4 and RT 1, 2, 3, 4, 6 at N and K 1024 to 27648, 24 to 128 rows, 4 and 8 bits, weights from HBM -- but it ranks well: what it
     // picks took 1 % more than the best pair in the median of those 120 launches, 10 % at most (24 rows of 5120 x 13824 at 4 bits 24.7
     // us with 2 x 2, 1 x 3 22.4; 100 rows of 1024 x 8192 12.1, 2 x 1 11.2).  48 rows of 11008 x 4096 get 3 x 3: 230 workgroups;
-    // 3 x 2 are 344, a second round for 88 of them.
+    // 3 x 2 are 344, a second round for 88 of them.  Several matrices are counted one by one, as no group has tiles of two: three of 4096 x
+    // 4096 are 258 groups of three tiles, not 256, and get 3 x 4 (a decoder layer's seven matrices at 4 bits, 48 rows, 76.9 -> 68.2 us;
+    // groups across matrices took 67.2 but cost every other launch up to a microsecond in looking them up).
     const int rows16 = (M + 15) / 16;
-    long long tiles = 0;
-    for (int i = 0; i < mm.count; i++) tiles += (mm.N[i] + 15) / 16;
     int mg = 4, rt = 4;
     double best = 0.0;
     for (int g = 1; g <= 4; g++)
         for (const int r : {1, 2, 3, 4, 6})
         {
-            const long long wgs = ((tiles + r - 1) / r) * ((rows16 + g - 1) / g);
+            long long wgs = 0;
+            for (int i = 0; i < mm.count; i++) wgs += ((mm.N[i] + 15) / 16 + r - 1) / r; // no group has tiles of two matrices
+            wgs *= (rows16 + g - 1) / g;
             const double cost = (double)((wgs + 255) / 256) * (1.8 * g + 1.6 * r);
             if (best == 0.0 || cost < best) best = cost, mg = g, rt = r;
         }

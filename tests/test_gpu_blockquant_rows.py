@@ -211,3 +211,13 @@ def test_fp32_rows_in_64x128_tiles(rt, m, n, k, bits, block):
     assert np.all(np.abs(got[rows, :n] - val) <= 1e-5 * floor + 1e-30)
     q = npref.blockquant_gemm_f64(np.eye(k, dtype=F)[k - 1:], packed, scales, bits, block)[0][0]  # the weights that meet the infinity
     assert np.array_equal(got[1, :n][q != 0], np.where(q > 0, np.inf, -np.inf)[q != 0].astype(F)) and np.all(np.isnan(got[1, :n][q == 0])) and np.all(np.isnan(got[m - 1, :n]))
+
+
+def test_several_matrices_whose_groups_would_fill_the_units_only_together(rt):
+    """3 x 256 tiles: in groups of three 258, in groups of four 192, which is what several matrices get; one matrix of all of them is 256 groups of three."""
+    m, k, n = 48, 64, 4096
+    ops = [synth.blockquant_operands(30 + i, m, n, k, 4, 64) for i in range(3)]
+    a = ops[0][0].astype(np.float16)
+    mats = [rt.blockquant_pack(p, s, 64, bits=4, k=k) + (n, None, -1, 1.0, 1.0) for _, p, s in ops]
+    for got, (_, packed, scales) in zip(rt.gemm_blockquant_packed_multi(a, mats, bits=4, block=64), ops):
+        _check(got, a.astype(F), packed, scales, 4, 64)
