@@ -915,7 +915,140 @@ __global__ __launch_bounds__(256) void attention_fewq_split_kernel(const float* 
     }
 }
 
-// merges the records of attention_fewq_split_kernel: one workgroup per (head, group of four queries).  The maxima and
+// The same for the head dimensions of the matrix-core kernels and TQ queries (the arithmetic of both is the same to the bit): every key and
+// value the workgroup needs, 64 x 128 of each at head dimension 128, is requested before the first wait, where the kernel above, which
+// has registers for 16 channels and 64, goes to memory four times in a row; and no more queries are multiplied than there are (all four
+// cost as long as the loads).  Keys and values past `past` are read where they come from, so that nobody waits for them to be stored.
+// Bound by the memory's latency and its rate: 32 heads of 128, one query on 1500 keys (49 MB), with the
+// merge, 19.4 -> 14.3 us (16.9 with the pieces of a head on all dies); four queries 32.2 -> 19.8; 16 of 64, one on 1001 10.1 -> 8.3.
+template<int HD, int TQ>
+__global__ __launch_bounds__(256) void attention_fewq_split_hd_kernel(const float* __restrict__ q, size_t q_stride, float q_scale, float* kt, float* vt, size_t kv_stride,
+                                                                      const float* __restrict__ mask, int mask_heads, int src, int dst, int v_vec_ok,
+                                                                      float* __restrict__ partial, const float* __restrict__ new_k, const float* __restrict__ new_v,
+                                                                      size_t new_stride, int past, int splits)
+{
+    constexpr int PER = HD / 4, NV = (HD + 63) / 64;
+    __shared__ float red[4][TQ][FEWQ_KEYS];
+    __shared__ float sc[TQ][FEWQ_KEYS];
+    // the pieces of a head follow one another on one die (workgroups are dealt to the 8 dies in turn): rows are not whole cache lines, and
+    // neighbours share the lines at their ends
+    const int T = gridDim.x, die = blockIdx.x & 7, more = T & 7, unit = die * (T >> 3) + (die < more ? die : more) + (int)(blockIdx.x >> 3);
+    const int h = unit / splits, split = unit - h * splits;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j0 = split * FEWQ_KEYS, c0 = wave * PER, kq = tid & 3;
+    const bool fresh = new_k && j0 + FEWQ_KEYS > past; // uniform: some of these keys are new
+    const int last = fresh ? past - 1 : dst - 1; // keys beyond: repeated here, replaced or dropped below
+
+    float kv[PER], vv[NV][16];
+    {
+        const float* kp = kt + ((size_t)h * HD + c0) * kv_stride + (j0 + lane < last ? j0 + lane : last);
+#pragma unroll
+        for (int i = 0; i < PER; i++) kv[i] = kp[(size_t)i * kv_stride];
+    }
+    const bool vec = v_vec_ok && j0 + FEWQ_KEYS <= last + 1;
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+    {
+        const int ch = (tid >> 2) + 64 * i < HD ? (tid >> 2) + 64 * i : HD - 1;
+        load_fewq_values(vv[i], vt + ((size_t)h * HD + ch) * kv_stride, j0 + 16 * kq, last + 1, vec);
+    }
+    if (fresh) // dst - past = src positions
+    {
+#pragma unroll
+        for (int t = 0; t < TQ; t++)
+        {
+            const size_t row = (size_t)(t < src ? t : src - 1) * new_stride + (size_t)h * HD;
+            const int at = past + (t < src ? t : src - 1) - j0; // (in this workgroup's keys, or in those of the one before)
+            float nk[PER]; // (the same for the whole wavefront)
+#pragma unroll
+            for (int i = 0; i < PER; i++) nk[i] = new_k[row + c0 + i];
+#pragma unroll
+            for (int i = 0; i < PER; i++) asm volatile("" : "+s"(nk[i])); // loaded whether the lane takes it or not
+#pragma unroll
+            for (int i = 0; i < PER; i++) kv[i] = lane == at ? nk[i] : kv[i];
+#pragma unroll
+            for (int i = 0; i < NV; i++)
+            {
+                const float v = new_v[row + ((tid >> 2) + 64 * i < HD ? (tid >> 2) + 64 * i : HD - 1)];
+#pragma unroll
+                for (int e = 0; e < 16; e++) vv[i][e] = 16 * kq + e == at ? v : vv[i][e];
+            }
+        }
+    }
+
+    // ---- scores: wavefront g takes the g-th quarter of the channels, lane = key
+    {
+        float acc[TQ];
+#pragma unroll
+        for (int t = 0; t < TQ; t++) acc[t] = 0.f;
+#pragma unroll
+        for (int t = 0; t < TQ; t++)
+        {
+            const float* qp = q + (size_t)(t < src ? t : 0) * q_stride + h * HD + c0; // (the same for the whole wavefront)
+#pragma unroll
+            for (int i = 0; i < PER; i++) acc[t] = add_rn(acc[t], mul_rn(mul_rn(qp[i], q_scale), kv[i]));
+        }
+#pragma unroll
+        for (int t = 0; t < TQ; t++) red[wave][t][lane] = acc[t];
+    }
+    __syncthreads();
+
+    // ---- softmax over this workgroup's keys: wavefront t = query t
+    float m_t = -FLT_MAX, l_t = 0.f;
+    if (wave < TQ)
+    {
+        const int t = wave;
+        float s = add_rn(add_rn(red[0][t][lane], red[1][t][lane]), add_rn(red[2][t][lane], red[3][t][lane]));
+        const bool live = j0 + lane < dst && t < src;
+        if (live && mask) s = add_rn(s, mask[((size_t)(mask_heads > 1 ? h : 0) * src + t) * dst + j0 + lane]);
+        if (!live) s = -INFINITY;
+        m_t = fmaxf(wave_max(s), -FLT_MAX); // a query that is not there (or all keys at -inf): every probability 0
+        const float pr = exp_of_nonpositive(s - m_t);
+        l_t = wave_sum(pr);
+        sc[t][lane] = pr;
+    }
+    __syncthreads();
+
+    // ---- p v: thread = (channel tid/4, keys 16*(tid%4)..+15), four lanes share a channel
+    float* rec = partial + ((size_t)h * splits + split) * (size_t)(2 * ATT_TQ + ATT_TQ * HD);
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+    {
+        const int ch = (tid >> 2) + 64 * i;
+        float acc[TQ];
+#pragma unroll
+        for (int t = 0; t < TQ; t++)
+        {
+            acc[t] = 0.f;
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[t] = add_rn(acc[t], mul_rn(sc[t][16 * kq + e], vv[i][e]));
+            acc[t] = add_rn(acc[t], __shfl_xor(acc[t], 1));
+            acc[t] = add_rn(acc[t], __shfl_xor(acc[t], 2));
+        }
+        if (kq == 0 && ch < HD)
+#pragma unroll
+            for (int t = 0; t < TQ; t++) rec[2 * ATT_TQ + t * HD + ch] = acc[t];
+    }
+    if (lane == 0)
+    {
+        rec[wave] = m_t;
+        rec[ATT_TQ + wave] = l_t;
+    }
+    if (fresh) // the new columns into the cache
+    {
+        const int kb = j0 > past ? j0 : past, ke = j0 + FEWQ_KEYS < dst ? j0 + FEWQ_KEYS : dst;
+        for (int e = tid; e < (ke - kb) * HD; e += 256)
+        {
+            const int pos = e / HD, c = e - pos * HD;
+            const size_t from = (size_t)(kb + pos - past) * new_stride + (size_t)h * HD + c;
+            const size_t to = ((size_t)h * HD + c) * kv_stride + kb + pos;
+            kt[to] = new_k[from];
+            vt[to] = new_v[from];
+        }
+    }
+}
+
+// merges the records of attention_fewq_split_kernel: one workgroup per (head, 64 outputs, group of four queries).  The maxima and
 // sums of all splits are fetched side by side into LDS (wavefront t = query t) and turned into one factor per split;
 // then four groups of 64 threads each add every fourth split's outputs, eight loads in flight, and the groups' parts
 // are added through LDS - a thread that walks the splits one load after the other takes 14 us for 24 of them.
@@ -932,13 +1065,14 @@ __global__ __launch_bounds__(256) void attention_fewq_merge_kernel(const float* 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const size_t rec_size = (size_t)(2 * ATT_TQ + ATT_TQ * head_dim);
     const float* rec0 = partial + ((size_t)blockIdx.y * gridDim.x + h) * splits * rec_size;
-    // Everything the first 64 outputs need is requested before the first wait (one trip to memory instead of three): this
-    // lane's maxima and sums of chunks lane, lane + 64, ... and, for output `lane`, the parts of this group's first 8 chunks.
+    // Everything up to 32 chunks need is requested before the first wait (one trip to memory instead of three): this lane's
+    // maxima and sums of chunks lane, lane + 64, ... and, for its output, the parts of this group's first 8 chunks.
+    const int idx = blockIdx.z * 64 + lane;
+    const float* op = rec0 + 2 * ATT_TQ + idx;
     float ofirst[8], mz[8], lz[8];
     {
-        const float* op = rec0 + 2 * ATT_TQ + lane;
 #pragma unroll
-        for (int k = 0; k < 8; k++) ofirst[k] = lane < rows * head_dim && wave + 4 * k < splits ? op[(size_t)(wave + 4 * k) * rec_size] : 0.f;
+        for (int k = 0; k < 8; k++) ofirst[k] = idx < rows * head_dim && wave + 4 * k < splits ? op[(size_t)(wave + 4 * k) * rec_size] : 0.f;
 #pragma unroll
         for (int k = 0; k < 8; k++)
         {
@@ -966,34 +1100,23 @@ __global__ __launch_bounds__(256) void attention_fewq_merge_kernel(const float* 
         if (lane == 0) l_all[t] = lt;
     }
     __syncthreads();
-    for (int base = 0; base < rows * head_dim; base += 64)
+    float ot = 0.f;
+    if (idx < rows * head_dim)
     {
-        const int idx = base + lane;
-        float ot = 0.f;
-        if (idx < rows * head_dim)
-        {
-            const int t = idx / head_dim;
-            const float* op = rec0 + 2 * ATT_TQ + idx;
-            int z = wave;
-            if (base == 0)
-            {
+        const int t = idx / head_dim;
 #pragma unroll
-                for (int k = 0; k < 8; k++)
-                    if (wave + 4 * k < splits) ot += ofirst[k] * fac[t][wave + 4 * k];
-                z = wave + 32;
-            }
+        for (int k = 0; k < 8; k++)
+            if (wave + 4 * k < splits) ot += ofirst[k] * fac[t][wave + 4 * k];
 #pragma unroll 8
-            for (; z < splits; z += 4) ot += op[z * rec_size] * fac[t][z];
-        }
-        part[wave][lane] = ot;
-        __syncthreads();
-        if (wave == 0 && idx < rows * head_dim)
-        {
-            const int t = idx / head_dim;
-            const float sum = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
-            out[(size_t)(i0 + t) * embed_dim + h * head_dim + (idx - t * head_dim)] = div_rn(sum, l_all[t]);
-        }
-        __syncthreads();
+        for (int z = wave + 32; z < splits; z += 4) ot += op[z * rec_size] * fac[t][z];
+    }
+    part[wave][lane] = ot;
+    __syncthreads();
+    if (wave == 0 && idx < rows * head_dim)
+    {
+        const int t = idx / head_dim;
+        const float sum = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+        out[(size_t)(i0 + t) * embed_dim + h * head_dim + (idx - t * head_dim)] = div_rn(sum, l_all[t]);
     }
 }
 
@@ -1143,13 +1266,39 @@ static int attention_dispatch(const float* q_dev, size_t q_stride, float q_scale
         && workspace_bytes >= attention_fewq_workspace_bytes(num_heads, head_dim, src_seqlen, dst_seqlen))
     {
         const int v_vec_ok = (kv_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(vt_dev) & 15) == 0) ? 1 : 0;
-        const int splits = (dst_seqlen + FEWQ_KEYS - 1) / FEWQ_KEYS, qgroups = (src_seqlen + ATT_TQ - 1) / ATT_TQ;
+        const int splits = (dst_seqlen + FEWQ_KEYS - 1) / FEWQ_KEYS; // (src_seqlen <= ATT_TQ: one group of queries)
         hipStream_t st = as_stream(stream);
-        hipLaunchKernelGGL(attention_fewq_split_kernel, dim3((unsigned)splits, (unsigned)num_heads, (unsigned)qgroups), dim3(256), 0, st, q_dev, q_stride, q_scale, kt_dev,
-                           vt_dev, kv_stride, mask_dev, mask_dev ? mask_heads : 0, head_dim, src_seqlen, dst_seqlen, v_vec_ok, (float*)workspace_dev, append_k, append_v,
-                           append_stride, past);
-        hipLaunchKernelGGL(attention_fewq_merge_kernel, dim3((unsigned)num_heads, (unsigned)qgroups), dim3(256), 0, st, (const float*)workspace_dev, splits, head_dim,
-                           num_heads * head_dim, src_seqlen, out_dev);
+        const dim3 grid((unsigned)splits, (unsigned)num_heads);
+        const int mh = mask_dev ? mask_heads : 0;
+#define LAUNCH_FEWQ(HD_, TQ_)                                                                                                                                      \
+    hipLaunchKernelGGL((attention_fewq_split_hd_kernel<HD_, TQ_>), dim3(grid.x * grid.y), dim3(256), 0, st, q_dev, q_stride, q_scale, kt_dev, vt_dev, kv_stride, mask_dev, mh, src_seqlen, \
+                       dst_seqlen, v_vec_ok, (float*)workspace_dev, append_k, append_v, append_stride, past, splits)
+#define LAUNCH_FEWQ_HD(HD_)         \
+    do                              \
+    {                               \
+        if (src_seqlen == 1)        \
+            LAUNCH_FEWQ(HD_, 1);    \
+        else if (src_seqlen == 2)   \
+            LAUNCH_FEWQ(HD_, 2);    \
+        else                        \
+            LAUNCH_FEWQ(HD_, 4);    \
+    } while (0)
+        const bool one_row = (long long)splits * num_heads <= 1 << 23; // of workgroups
+        if (head_dim == 32 && one_row)
+            LAUNCH_FEWQ_HD(32);
+        else if (head_dim == 64 && one_row)
+            LAUNCH_FEWQ_HD(64);
+        else if (head_dim == 96 && one_row)
+            LAUNCH_FEWQ_HD(96);
+        else if (head_dim == 128 && one_row)
+            LAUNCH_FEWQ_HD(128);
+        else
+            hipLaunchKernelGGL(attention_fewq_split_kernel, grid, dim3(256), 0, st, q_dev, q_stride, q_scale, kt_dev, vt_dev, kv_stride, mask_dev, mh, head_dim, src_seqlen,
+                               dst_seqlen, v_vec_ok, (float*)workspace_dev, append_k, append_v, append_stride, past);
+#undef LAUNCH_FEWQ_HD
+#undef LAUNCH_FEWQ
+        hipLaunchKernelGGL(attention_fewq_merge_kernel, dim3((unsigned)num_heads, 1, (unsigned)((src_seqlen * head_dim + 63) / 64)), dim3(256), 0, st,
+                           (const float*)workspace_dev, splits, head_dim, num_heads * head_dim, src_seqlen, out_dev);
         return launch_status("attention_fewq_split_kernel");
     }
     hipStream_t st = as_stream(stream);

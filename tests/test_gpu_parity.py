@@ -901,3 +901,12 @@ def test_attention_appends_the_new_keys_and_values_itself(rt, heads, hd, src, pa
     got, got_kt, got_vt = rt.attention_append(qkv, kt, vt, heads, past, scale, m)
     assert np.array_equal(got_kt, want_kt) and np.array_equal(got_vt, want_vt)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("heads,hd,src,past,mask", [(3, 32, 1, 256, None), (2, 64, 2, 318, "2d"), (3, 96, 3, 317, "3d"), (2, 128, 4, 318, None), (5, 128, 1, 319, "2d"),
+                                                    (1, 96, 4, 252, None), (9, 128, 2, 1022, None), (1, 64, 4, 1148, "3d"), (7, 128, 1, 767, None)])
+def test_attention_of_few_queries_reads_new_columns_where_they_come_from(rt, heads, hd, src, past, mask):
+    """The head dimensions with a kernel of their own: new positions in the last 64 keys, across two such pieces and alone in one; rows
+    that are and are not 16-byte aligned.  Against float64 too: fp32 sums over head_dim and dst terms of O(1) values."""
+    test_attention_appends_the_new_keys_and_values_itself(rt, heads, hd, src, past, mask)
+    test_attention_core_matches_float64(rt, heads, hd, src, past + src, mask)
