@@ -9,8 +9,9 @@
 // A workgroup is four wavefronts, 2 x 2, on a BM x BN tile; a K step is 128 bytes of every row.  LDS holds two steps; row r
 // keeps its eight 16-byte chunks at positions c ^ ((r >> 1) & 7), so that any 16 consecutive rows read at one K offset meet
 // 16 different bank groups.  One barrier per step: the buffer that step t + 1 is written into was last read in step t - 1.
-// Bound by latency at the sizes it is for (some hundred tiles of 64 x 64): 1501 x 1000 x 2008 168 us with the byte gathers
-// of the kernel before this one.  Fewer tiles go to gemm_int8_stream_kernel below.
+// Bound by latency and by the first-level cache at the sizes it is for (some hundred tiles of 64 x 64; two workgroups on one unit bring it
+// 720 cycles of lines a step, and a step takes 960): 1501 x 1000 x 2008 168 us with the byte gathers of the kernel before this one, 13.1
+// -> 12.5 since two products' operands are read at once and the rows' values in one go.  Fewer tiles go to gemm_int8_stream_kernel below.
 #include "conv_nhwc.h"
 #include "epilogues.h"
 #include "gemm_int8_general.h"
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
     constexpr int STEP_BYTES = (BM + BN) * KSTEP;
     static_assert(KG == 1 || BM * BN * 4 <= 2 * STEP_BYTES, "the sums of a group fit its buffers");
     __shared__ __attribute__((aligned(16))) int8_t smem_all[KG * 2 * STEP_BYTES];
-    __shared__ float row_value[BM];
+    __shared__ __attribute__((aligned(16))) float row_value[BM];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
@@ -176,18 +177,29 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
     auto multiply = [&](int t) {
         const int8_t* sa = smem + (t & 1) * STEP_BYTES + wm * (BM / 2) * KSTEP;
         const int8_t* sb = smem + (t & 1) * STEP_BYTES + (BM + wn * (BN / 2)) * KSTEP;
+        // Q quarters of the step are read before they are multiplied: left to itself the compiler reads two operands, waits, multiplies and
+        // reads the next two into the same registers.  As many as leave the workgroups a unit holds their registers.
+        constexpr int Q = TM * TN == 1 && KG == 1 ? 2 : 1;
 #pragma unroll
-        for (int q = 0; q < 4; q++)
+        for (int q0 = 0; q0 < 4; q0 += Q)
         {
-            v4i fa[TM], fb[TN];
+            v4i fa[Q][TM], fb[Q][TN];
 #pragma unroll
-            for (int i = 0; i < TM; i++) fa[i] = *reinterpret_cast<const v4i*>(sa + i * 32 * KSTEP + rd[q]);
+            for (int q = 0; q < Q; q++)
+            {
 #pragma unroll
-            for (int j = 0; j < TN; j++) fb[j] = *reinterpret_cast<const v4i*>(sb + j * 32 * KSTEP + rd[q]);
+                for (int i = 0; i < TM; i++) fa[q][i] = *reinterpret_cast<const v4i*>(sa + i * 32 * KSTEP + rd[q0 + q]);
 #pragma unroll
-            for (int i = 0; i < TM; i++)
+                for (int j = 0; j < TN; j++) fb[q][j] = *reinterpret_cast<const v4i*>(sb + j * 32 * KSTEP + rd[q0 + q]);
+            }
+            if (Q > 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int j = 0; j < TN; j++) accs[q % SETS][i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], accs[q % SETS][i][j], 0, 0, 0);
+            for (int q = 0; q < Q; q++)
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+                        accs[(q0 + q) % SETS][i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[q][i], fb[q][j], accs[(q0 + q) % SETS][i][j], 0, 0, 0);
         }
     };
 
@@ -257,19 +269,27 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
         return;
     }
 
+    // the rows' values in one go, four consecutive ones at a time
+    typedef float v4f_rows __attribute__((ext_vector_type(4)));
+    v4f_rows rows[TM][4];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) rows[i][e] = *reinterpret_cast<const v4f_rows*>(row_value + wm * (BM / 2) + i * 32 + 8 * e + 4 * lhi);
 #pragma unroll
     for (int j = 0; j < TN; j++)
     {
         const int col = col0 + wn * (BN / 2) + j * 32 + l32;
-        float scale = 0.f, add = 0.f;
-        if (col < N) epi.column(col, scale, add);
+        if (col >= N) continue;
+        float scale, add;
+        epi.column(col, scale, add);
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int r = 0; r < 16; r++)
             {
                 const int in_tile = wm * (BM / 2) + i * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
-                if (row0 + in_tile < M && col < N) epi.store(row0 + in_tile, col, acc[i][j][r], row_value[in_tile], scale, add);
+                if (row0 + in_tile < M) epi.store(row0 + in_tile, col, acc[i][j][r], rows[i][r >> 2][r & 3], scale, add);
             }
     }
 }
@@ -355,19 +375,22 @@ __global__ __launch_bounds__(64 * W) void gemm_int8_stream_kernel(const int8_t* 
         for (int i = 0; i < LB; i++) *reinterpret_cast<v4i*>(smem + BM * KSTEP + i * 1024 + (i & 1 ? wr1 : wr0)) = rb[i];
         __builtin_amdgcn_wave_barrier();
         fetch(t + 1); // (past the last step: the first again)
+        v4i fa[4][TM], fb[4][TN]; // every read before the first product, as above
 #pragma unroll
         for (int q = 0; q < 4; q++)
         {
-            v4i fa[TM], fb[TN];
 #pragma unroll
-            for (int i = 0; i < TM; i++) fa[i] = *reinterpret_cast<const v4i*>(smem + i * 32 * KSTEP + rd[q]);
+            for (int i = 0; i < TM; i++) fa[q][i] = *reinterpret_cast<const v4i*>(smem + i * 32 * KSTEP + rd[q]);
 #pragma unroll
-            for (int j = 0; j < TN; j++) fb[j] = *reinterpret_cast<const v4i*>(smem + (BM + j * 32) * KSTEP + rd[q]);
+            for (int j = 0; j < TN; j++) fb[q][j] = *reinterpret_cast<const v4i*>(smem + (BM + j * 32) * KSTEP + rd[q]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
+                for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[q][i], fb[q][j], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_wave_barrier();
     }
 
@@ -457,7 +480,8 @@ static int launch_any(const int8_t* a, size_t lda, const int8_t* b, size_t ldb, 
         hipLaunchKernelGGL((gemm_int8_short_k_kernel<Epilogue>), dim3((unsigned)blocks), dim3(256), 0, stream, a, lda, b, ldb, M, N, K, epi);
         return launch_status("gemm_int8_short_k_kernel");
     }
-    if (gemm_int8_streams(M, N, K, rows_aligned16(a, lda, K) && rows_aligned16(b, ldb, K)))
+    const bool aligned = rows_aligned16(a, lda, K) && rows_aligned16(b, ldb, K);
+    if (gemm_int8_streams(M, N, K, aligned))
     {
         const long long tiles32 = (long long)ceil_div(M, 32) * ceil_div(N, 32);
         if (M > 16 && tiles32 > 640 && K >= 3072) return launch_stream<64, 64, 8>(a, lda, b, ldb, M, N, K, epi, stream);
@@ -468,7 +492,13 @@ static int launch_any(const int8_t* a, size_t lda, const int8_t* b, size_t ldb, 
     // operand bytes per product decide, half as many with 128 x 128 tiles (2000 x 4000 x 4096: 74 -> 53 us, 2500 cubed 56 ->
     // 41, 2048 cubed the same 20).  With few tiles and a long K two groups of wavefronts halve the chain of steps (1100 x 520 x 7000
     // 23.4 -> 20.2; not below some 24 steps).
-    const long long tiles = (long long)ceil_div(M, 64) * ceil_div(N, 64);
+    // Rows off 16 bytes cost up to 2 times the cache lines, rows off 4 bytes 2.4 times the cycles of aligned ones (834 against 346 for 16 KB), and
+    // the bytes decide earlier: while one round of 128 x 128 tiles does it, from 800 tiles (2048 x 2048 x 2004 23.9 -> 20.1, 1792 x 2048 x 1004
+    // 14.3 -> 13.6; 768 tiles 19.2 18.4, 640 x 1004 11.9 12.8), off 4 bytes from 600 (1280 x 2048 x 2003 25.1 -> 22.5, 2048 x 2048 x 3001 42.6 ->
+    // 32.1), with more rounds from 1300 (2816 x 2048 x 2004 32.0 -> 28.2; 1152 tiles the same), and not on a short K (2048 x 2048 x 508 10.7 11.8).
+    const long long tiles = (long long)ceil_div(M, 64) * ceil_div(N, 64), tiles128 = (long long)ceil_div(M, 128) * ceil_div(N, 128);
+    const bool words = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | lda | ldb) & 3) == 0;
+    if (!aligned && K >= 1000 && tiles >= (tiles128 > 256 ? 1300 : words ? 800 : 600)) return launch_tile<128, 128, 1>(a, lda, b, ldb, M, N, K, epi, stream);
     if (tiles >= 1536) return launch_tile<128, 128, 1>(a, lda, b, ldb, M, N, K, epi, stream);
     if (tiles <= 512 && K >= 3072) return launch_tile<64, 64, 2>(a, lda, b, ldb, M, N, K, epi, stream);
     return launch_tile<64, 64, 1>(a, lda, b, ldb, M, N, K, epi, stream);

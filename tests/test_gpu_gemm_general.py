@@ -62,3 +62,19 @@ def test_128x128_tiles_cut_at_the_end(rt, m, n, k, per_col):
     check(lib().ncnnhip_gemm_int8(da.ptr, k, db.ptr, k, m, cols, k, dsa.ptr, dsb.ptr, cols if per_col else 1, dc.ptr, 4, 1.0, 1.0, 0, out.ptr, n + 2, None, rt.stream))
     got = out.to_numpy(rt.stream)
     assert np.array_equal(got[:m, :cols], want[:, :cols]) and np.all(got[:m, cols:] == 7.0) and np.all(got[m] == 7.0)
+
+
+@pytest.mark.parametrize("m,n,k,pad", [(1601, 1537, 1003, 0), (1850, 1800, 1004, 0), (1793, 1805, 1024, 1), (2305, 2241, 1002, 2)])
+def test_128x128_tiles_of_rows_off_16_bytes(rt, m, n, k, pad):
+    """Rows that begin at any byte, or at any fourth, in the sizes that take 128 x 128 tiles for it: cut tiles, K that ends inside a step."""
+    print("[case]", m, n, k, pad, flush=True)
+    a, bq, sb, bias = cases.gemm_case(m + n + k, m, n, k, per_col=True)
+    aq, sa = rt.gemm_quantize_rows(a)
+    want, _ = npref.gemm_int8(aq, bq, sa, sb, bias, 4, acc=npref.gemm_acc_exact(aq, bq))
+    wide = np.full((m, k + pad), 99, np.int8)
+    wide[:, :k] = aq
+    da, db, dsa, dsb, dc = rt.up(wide), rt.up(bq), rt.up(sa), rt.up(sb), rt.up(bias.reshape(-1))
+    out = rt.up(np.full((m + 1, n + 1), 7.0, np.float32))
+    check(lib().ncnnhip_gemm_int8(da.ptr, k + pad, db.ptr, k, m, n, k, dsa.ptr, dsb.ptr, n, dc.ptr, 4, 1.0, 1.0, 0, out.ptr, n + 1, None, rt.stream))
+    got = out.to_numpy(rt.stream)
+    assert np.array_equal(got[:m, :n], want) and np.all(got[:m, n] == 7.0) and np.all(got[m] == 7.0)
