@@ -121,17 +121,6 @@ __device__ __forceinline__ void split8_bf16x3(const float* x, v8bf (&out)[3])
     for (int pn = 0; pn < 3; pn++) out[pn] = p[pn].h;
 }
 
-template<int AIN>
-struct RowsOperand // a lane's 16 activations of a step as the matrix cores take them, 8 and 8
-{
-    typedef v8h T;
-};
-template<>
-struct RowsOperand<4>
-{
-    typedef v8bf T;
-};
-
 template<int BITS, bool HALVES, int SPLIT, int MG, int RT, int AIN>
 __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blockquant_rows_kernel(const void* __restrict__ a_, size_t a_stride, int M_total, int K, int kblocks,
                                                                               int groups, int passes, const float* __restrict__ in_scales, BqMulti mm)
@@ -234,6 +223,12 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
     }
     const unsigned rd_w = base + W_OFF + lane * (BITS == 8 ? 16 : 8), rd_w3 = base + W_OFF + 512 + lane * 4;
     const unsigned rd_d = base + D_OFF + kg * 16;
+    // two descales a tile, four groups and six tiles: the descales of a tile are read while the one before is multiplied, or registers spill
+    constexpr bool LATE = !F32 && SPLIT && MG == 4 && RT == 6;
+    auto read_descales = [&](int rt, unsigned at, v4i_bq (&dq0)[RT], v4i_bq (&dq1)[RT]) {
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dq0[rt]) : "v"(rd_d + at), "n"(rt * DPER * 16));
+        if (SPLIT) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dq1[rt]) : "v"(rd_d + at), "n"(rt * DPER * 16 + 64));
+    };
 
     for (bool careful = false;; careful = true)
     {
@@ -271,8 +266,7 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
                 else
                     asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(wlo[rt]) : "v"(rd_w + at), "n"(rt * STEP_BYTES));
                 if (BITS == 6) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(whi[rt]) : "v"(rd_w3 + at), "n"(rt * STEP_BYTES));
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dq0[rt]) : "v"(rd_d + at), "n"(rt * DPER * 16));
-                if (SPLIT) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dq1[rt]) : "v"(rd_d + at), "n"(rt * DPER * 16 + 64));
+                if (!LATE || rt == 0) read_descales(rt, at, dq0, dq1);
             }
             union Act
             {
@@ -308,25 +302,50 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
                 else
                     asm volatile("" : "+v"(wlo[rt]));
                 if (BITS == 6) asm volatile("" : "+v"(whi[rt]));
+                if (LATE && rt > 0) continue;
                 asm volatile("" : "+v"(dq0[rt]));
                 if (SPLIT) asm volatile("" : "+v"(dq1[rt]));
             }
-            typename RowsOperand<AIN>::T wa[RT], wb[RT];
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++)
-            {
-                if constexpr (F32)
-                    fields_to_bf16<BITS>(wq[rt], wlo[rt], whi[rt], wa[rt], wb[rt]);
-                else
-                    fields_to_halves<BITS>(wq[rt], wlo[rt], whi[rt], wa[rt], wb[rt]);
-            }
             const v4f zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int g = 0; g < MG; g++)
+            if constexpr (!F32)
             {
-                v4f t0[RT], t1[RT];
-                if constexpr (F32)
+                // tile by tile: with the tiles' operands and products side by side, as below, four groups and six tiles are 23 registers too
+                // many, and a spilled one waits for every load in flight (twice the time)
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++)
                 {
+                    v8h wa, wb;
+                    if (LATE && rt + 1 < RT) read_descales(rt + 1, at, dq0, dq1);
+                    fields_to_halves<BITS>(wq[rt], wlo[rt], whi[rt], wa, wb);
+#pragma unroll
+                    for (int g = 0; g < MG; g++)
+                    {
+                        v4f t0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa, x[g][0].h, zero, 0, 0, 0);
+                        const v4f t1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(wb, x[g][1].h, SPLIT ? zero : t0, 0, 0, 0);
+                        if (!SPLIT) t0 = t1;
+#pragma unroll
+                        for (int r = 0; r < 4; r++)
+                        {
+                            acc[rt][g][r] = fmaf(t0[r], __int_as_float(dq0[rt][r]), acc[rt][g][r]);
+                            if (SPLIT) acc[rt][g][r] = fmaf(t1[r], __int_as_float(dq1[rt][r]), acc[rt][g][r]);
+                        }
+                    }
+                    if (LATE && rt + 1 < RT)
+                    {
+                        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(dq0[rt + 1]), "+v"(dq1[rt + 1]));
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+            else
+            {
+                v8bf wa[RT], wb[RT];
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++) fields_to_bf16<BITS>(wq[rt], wlo[rt], whi[rt], wa[rt], wb[rt]);
+#pragma unroll
+                for (int g = 0; g < MG; g++)
+                {
+                    v4f t0[RT], t1[RT];
                     float v[16];
 #pragma unroll
                     for (int p = 0; p < PARTS; p++)
@@ -368,25 +387,15 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
                                 t0[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[rt], yb[pn], t0[rt], 0, 0, 0);
                         }
                     }
-                }
-                else
-                {
 #pragma unroll
                     for (int rt = 0; rt < RT; rt++)
-                    {
-                        t0[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa[rt], x[g][0].h, zero, 0, 0, 0);
-                        t1[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wb[rt], x[g][1].h, SPLIT ? zero : t0[rt], 0, 0, 0);
-                        if (!SPLIT) t0[rt] = t1[rt];
-                    }
+#pragma unroll
+                        for (int r = 0; r < 4; r++)
+                        {
+                            acc[rt][g][r] = fmaf(t0[rt][r], __int_as_float(dq0[rt][r]), acc[rt][g][r]);
+                            if (SPLIT) acc[rt][g][r] = fmaf(t1[rt][r], __int_as_float(dq1[rt][r]), acc[rt][g][r]);
+                        }
                 }
-#pragma unroll
-                for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                    {
-                        acc[rt][g][r] = fmaf(t0[rt][r], __int_as_float(dq0[rt][r]), acc[rt][g][r]);
-                        if (SPLIT) acc[rt][g][r] = fmaf(t1[rt][r], __int_as_float(dq1[rt][r]), acc[rt][g][r]);
-                    }
             }
         }
         WAIT_VMCNT(0); // the surplus loads of the last step must not land on the sums below, nor on the first step again

@@ -39,6 +39,13 @@ def test_many_fp16_rows(rt, m, n, k, bits, block):
     _check(got, a, packed, scales, bits, block, c, 4, 0.75, 1.5)
 
 
+@pytest.mark.parametrize("m,n,k", [(64, 9040, 144), (50, 8970, 528)])
+@pytest.mark.parametrize("bits,block", [(8, 64), (8, 32), (6, 128), (6, 32), (4, 64), (4, 32)])
+def test_four_groups_of_rows_and_six_tiles(rt, m, n, k, bits, block):
+    """The largest form, which has the fewest registers to spare: blocks of 32 read a tile's descales while the one before is multiplied."""
+    test_many_fp16_rows(rt, m, n, k, bits, block)
+
+
 @pytest.mark.parametrize("m,n,k,bits,block", [(5, 40, 8208, 4, 64), (13, 33, 9216, 6, 32), (16, 20, 8704, 8, 32), (5, 19600, 1024, 4, 128), (7, 7000, 9200, 8, 64)])
 def test_few_fp16_rows_of_large_weights(rt, m, n, k, bits, block):
     test_many_fp16_rows(rt, m, n, k, bits, block)
