@@ -39,7 +39,7 @@ def test_many_fp16_rows(rt, m, n, k, bits, block):
     _check(got, a, packed, scales, bits, block, c, 4, 0.75, 1.5)
 
 
-@pytest.mark.parametrize("m,n,k", [(64, 9040, 144), (50, 8970, 528)])
+@pytest.mark.parametrize("m,n,k", [(64, 17610, 144), (50, 16800, 336)])
 @pytest.mark.parametrize("bits,block", [(8, 64), (8, 32), (6, 128), (6, 32), (4, 64), (4, 32)])
 def test_four_groups_of_rows_and_six_tiles(rt, m, n, k, bits, block):
     """The largest form, which has the fewest registers to spare: blocks of 32 read a tile's descales while the one before is multiplied."""
