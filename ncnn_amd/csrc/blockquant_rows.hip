@@ -224,7 +224,8 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
     const unsigned rd_w = base + W_OFF + lane * (BITS == 8 ? 16 : 8), rd_w3 = base + W_OFF + 512 + lane * 4;
     const unsigned rd_d = base + D_OFF + kg * 16;
     // two descales a tile, four groups and six tiles: the descales of a tile are read while the one before is multiplied, or registers spill
-    constexpr bool LATE = !F32 && SPLIT && MG == 4 && RT == 6;
+    constexpr bool TILEWISE = F32 && MG == 2 && (RT == 4 || (RT == 3 && SPLIT)); // (fp32 rows: both groups split, then tile by tile; three tiles with one descale fit)
+    constexpr bool LATE = SPLIT && ((!F32 && MG == 4 && RT == 6) || TILEWISE);
     auto read_descales = [&](int rt, unsigned at, v4i_bq (&dq0)[RT], v4i_bq (&dq1)[RT]) {
         asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dq0[rt]) : "v"(rd_d + at), "n"(rt * DPER * 16));
         if (SPLIT) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dq1[rt]) : "v"(rd_d + at), "n"(rt * DPER * 16 + 64));
@@ -339,13 +340,7 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
             }
             else
             {
-                v8bf wa[RT], wb[RT];
-#pragma unroll
-                for (int rt = 0; rt < RT; rt++) fields_to_bf16<BITS>(wq[rt], wlo[rt], whi[rt], wa[rt], wb[rt]);
-#pragma unroll
-                for (int g = 0; g < MG; g++)
-                {
-                    v4f t0[RT], t1[RT];
+                auto split_group = [&](int g, v8bf (&ya)[3], v8bf (&yb)[3]) {
                     float v[16];
 #pragma unroll
                     for (int p = 0; p < PARTS; p++)
@@ -358,7 +353,6 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
 #pragma unroll
                             for (int e = 0; e < 4; e++) v[p * 4 + e] = mul_rn(v[p * 4 + e], sc[p].f[e]);
                     }
-                    v8bf ya[3], yb[3];
                     if (careful)
                     {
                         split8_bf16x3<false>(v, ya);
@@ -369,32 +363,69 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
                         split8_bf16x3<true>(v, ya);
                         split8_bf16x3<true>(v + 8, yb);
                     }
-                    // One chain for the whole step: the least parts first, so that only two of its six roundings are at the sum's own size
-                    // (relative error of 4096 x 4096 against 64 bits 9.2e-8 -> 7.1e-8); a chain of three is better begun with the
-                    // greatest (blocks of 32, 4 bits: 8.7e-8 against 9.1e-8).
+                };
+                // One chain for the whole step: the least parts first, so that only two of its six roundings are at the sum's own size
+                // (relative error of 4096 x 4096 against 64 bits 9.2e-8 -> 7.1e-8); a chain of three is better begun with the
+                // greatest (blocks of 32, 4 bits: 8.7e-8 against 9.1e-8).
+                auto product = [&](v4f& t0, v4f& t1, const v8bf& wa, const v8bf& wb, const v8bf (&ya)[3], const v8bf (&yb)[3], int i) {
+                    const int pn = SPLIT ? i : 2 - i;
+                    t0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, ya[pn], i ? t0 : zero, 0, 0, 0);
+                    if (SPLIT)
+                        t1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, yb[pn], i ? t1 : zero, 0, 0, 0);
+                    else
+                        t0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, yb[pn], t0, 0, 0, 0);
+                };
+                auto add = [&](int rt, int g, const v4f& t0, const v4f& t1) {
 #pragma unroll
-                    for (int i = 0; i < 3; i++)
+                    for (int r = 0; r < 4; r++)
                     {
-                        const int pn = SPLIT ? i : 2 - i;
-#pragma unroll
-                        for (int rt = 0; rt < RT; rt++) t0[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[rt], ya[pn], i ? t0[rt] : zero, 0, 0, 0);
-#pragma unroll
-                        for (int rt = 0; rt < RT; rt++)
-                        {
-                            if (SPLIT)
-                                t1[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[rt], yb[pn], i ? t1[rt] : zero, 0, 0, 0);
-                            else
-                                t0[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[rt], yb[pn], t0[rt], 0, 0, 0);
-                        }
+                        acc[rt][g][r] = fmaf(t0[r], __int_as_float(dq0[rt][r]), acc[rt][g][r]);
+                        if (SPLIT) acc[rt][g][r] = fmaf(t1[r], __int_as_float(dq1[rt][r]), acc[rt][g][r]);
                     }
+                };
+                if constexpr (TILEWISE)
+                {
+                    v8bf ya[MG][3], yb[MG][3];
+#pragma unroll
+                    for (int g = 0; g < MG; g++) split_group(g, ya[g], yb[g]);
 #pragma unroll
                     for (int rt = 0; rt < RT; rt++)
+                    {
+                        v8bf wa, wb;
+                        v4f t0[MG], t1[MG];
+                        if (LATE && rt + 1 < RT) read_descales(rt + 1, at, dq0, dq1);
+                        fields_to_bf16<BITS>(wq[rt], wlo[rt], whi[rt], wa, wb);
 #pragma unroll
-                        for (int r = 0; r < 4; r++)
+                        for (int i = 0; i < 3; i++)
+#pragma unroll
+                            for (int g = 0; g < MG; g++) product(t0[g], t1[g], wa, wb, ya[g], yb[g], i);
+#pragma unroll
+                        for (int g = 0; g < MG; g++) add(rt, g, t0[g], t1[g]);
+                        if (LATE && rt + 1 < RT)
                         {
-                            acc[rt][g][r] = fmaf(t0[rt][r], __int_as_float(dq0[rt][r]), acc[rt][g][r]);
-                            if (SPLIT) acc[rt][g][r] = fmaf(t1[rt][r], __int_as_float(dq1[rt][r]), acc[rt][g][r]);
+                            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(dq0[rt + 1]), "+v"(dq1[rt + 1]));
+                            __builtin_amdgcn_sched_barrier(0);
                         }
+                    }
+                }
+                else
+                {
+                    v8bf wa[RT], wb[RT];
+#pragma unroll
+                    for (int rt = 0; rt < RT; rt++) fields_to_bf16<BITS>(wq[rt], wlo[rt], whi[rt], wa[rt], wb[rt]);
+#pragma unroll
+                    for (int g = 0; g < MG; g++)
+                    {
+                        v8bf ya[3], yb[3];
+                        v4f t0[RT], t1[RT];
+                        split_group(g, ya, yb);
+#pragma unroll
+                        for (int i = 0; i < 3; i++)
+#pragma unroll
+                            for (int rt = 0; rt < RT; rt++) product(t0[rt], t1[rt], wa[rt], wb[rt], ya, yb, i);
+#pragma unroll
+                        for (int rt = 0; rt < RT; rt++) add(rt, g, t0[rt], t1[rt]);
+                    }
                 }
             }
         }

@@ -131,6 +131,13 @@ def test_fp32_rows_split_as_they_are_multiplied(rt, m, n, k, bits, block, rows):
     assert np.all(np.abs(got - val) <= 1e-5 * floor + 1e-30)
 
 
+@pytest.mark.parametrize("m,n,k", [(32, 14330, 144), (25, 11000, 208), (32, 16100, 592)])
+@pytest.mark.parametrize("bits,block", [(8, 64), (8, 32), (6, 128), (6, 32), (4, 64), (4, 32)])
+def test_two_groups_of_fp32_rows_and_three_or_four_tiles(rt, m, n, k, bits, block):
+    """The largest forms for fp32 rows, which go tile by tile; blocks of 32 read a tile's descales while the one before is multiplied."""
+    test_fp32_rows_split_as_they_are_multiplied(rt, m, n, k, bits, block, True)
+
+
 @pytest.mark.parametrize("m,n,k", [(7, 40, 144), (17, 8200, 80)])
 def test_special_values_in_fp32_rows(rt, m, n, k):
     """The sums are made without a look at the values and repeated with one where they turn out not to be numbers: infinities, the largest
