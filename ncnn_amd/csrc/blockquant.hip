@@ -2471,14 +2471,14 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
                < 9.0 + K / 1024.0 * (tiles64 <= 256 ? 7.8 : block != 32 ? 11.0 * rounds : tiles64 <= 512 ? 14.2 : 17.0 * tiles64 / 512.0))
         return launch_blockquant_rows_f32(a_dev, a_stride, M, K, bits, block, in_scales_dev, one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride),
                                           st);
-    // Which form: the 16-row passes (all in one launch, spread over the chip; every pass streams the weights again, from L2
-    // after the first) cost about 5 us + passes x weight bytes at 2 TB/s; the tiled kernel's 64-row tiles about 6 us + K / 85
-    // whatever the row count up to 64 (18-20 us at K = 1024, 54-58 at K = 4096).  Measured on 16..96 rows: 3072 x 1024
-    // 6.9..12.5 us against 18..20 tiled, 4096 x 4096 11.7..52.7 against 55..58, 11008 x 4096 26.8 / 49 / 72 / 90 at
-    // 16 / 32 / 48 / 64 rows against 57..59.
-    const double weight_mb = (double)N * (double)K * bits / 8.0 / 1.0e6;
+    // Which form (rows off 16 bytes, mostly): the 16-row passes, all in one launch, take about 5 us and a pass's weights at 2.35 million a us, 3.2 up
+    // to K = 2048 and less where the last of its rounds of 64 K steps is partly empty, whatever their bits, which the conversions decide; a round of the
+    // tiled kernel 7 us + K / 1024 x 7.8 whatever the row count.  us, passes / tiled at 8 bits: 4096 x 1024 97 rows 15.3 17.0; 8192 x 2048 48
+    // rows 19.7 24.2, 97 rows 42.5 26.2; 4096 x 4096 64 rows 33.8 39.9, 97 rows 56 41; 4992 x 4992 20 rows 36.8 45.4, 48 rows 49 46; 11008 x
+    // 4096 12 rows 25 38, 20 rows 44 39; 4096 x 11008 64 rows 84 89.  (By bytes, as before, 97 rows of 4992 x 4992 at 4 bits took 112 us for 51.)
     const int passes16 = (M + 15) / 16;
-    if (M <= 128 && 5.0 + passes16 * weight_mb / 2.0 <= 6.0 + K / 85.0)
+    const double weights = (double)N * (double)K / 1.0e6 * (kblocks <= 64 ? 1.0 : (kblocks + 63) / 64 * 64.0 / kblocks);
+    if (M <= 128 && 5.0 + passes16 * weights / (K <= 2048 ? 3.2 : 2.35) <= 7.0 + K / 1024.0 * 7.8)
     {
         // fewer rows than the tiled kernel can spread over the chip: 16 rows per pass in the weight-streaming shape
         // (the fragments of a pass take kblocks * 6 KB of the workspace: all passes together no more than the planes it was sized for)
