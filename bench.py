@@ -329,7 +329,7 @@ def bench_blockquant(args, n, k, m, bits=8, block=64):
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": measured_traffic("blockquant:%dx%dx%d%s%s" % (n, k, m, "" if (bits, block) == (8, 64) else ":%d:%d" % (bits, block),
                                                                               "" if half else ":" + args.act)) if packed_form else None,
-                     "kernel": ("blockquant_rows16_bf16x3_kernel" if (m <= 128 and 5.0 + ((m + 15) // 16) * (n * k * bits / 8.0 / 1.0e6) / 2.0 <= 6.0 + k / 85.0) else "blockquant_rows_bf16x3_kernel") if rows_entry else "blockquant8_upfront_kernel" if packed_form else ("blockquant8_f32_mfma_kernel" if m >= 32 else "blockquant8_stream_kernel"),
+                     "kernel": "ncnnhip_gemm_blockquant_packed_rows (blockquant_rows_kernel for few rows, blockquant_tiles_kernel for many)" if rows_entry else "blockquant8_upfront_kernel" if packed_form else ("blockquant8_f32_mfma_kernel" if m >= 32 else "blockquant8_stream_kernel"),
                      "bytes_per_launch": algo,
                      "measured_peak": floor["gbs"], "frac_of_measured": achieved / floor["gbs"],
                      "measured_peak_how": "read-only kernel over the same number of bytes, back-to-back launches over rotating copies: %.2f us per launch"
@@ -576,8 +576,8 @@ def bench_mha(args, embed, heads, src, past):
     check(lib.ncnnhip_attention_workspace_bytes(heads, embed // heads, src, dst, C.byref(wsb)))
     d_ws = ncnn_amd.DeviceBuffer.empty((max(wsb.value, 4),), np.uint8)
 
-    # the projections as the layer dispatches them (blockquant_gemm_device): fewer than 32 rows on the packed tiles four rows per pass,
-    # 32 and more through the tiled bf16 kernel with its workspace; `--act fp32-bin` keeps the kernels of the .bin layout
+    # the projections as the layer dispatches them (blockquant_gemm_device): fewer than 32 rows on the packed tiles,
+    # 32 and more through the many-row entry point with its workspace; `--act fp32-bin` keeps the kernels of the .bin layout
     packed_ok = args.act != "fp32-bin" and lib.ncnnhip_gemm_blockquant_packed_supported(embed)
     rows_ws = None
     if packed_ok and src >= 32:
@@ -623,7 +623,7 @@ def bench_mha(args, embed, heads, src, past):
         "metric": "HBM GB/s", "value": algo / (ms_per_step * 1e-3) / 1e9, "unit": "GB/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": ms_per_step, "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": "self-attention layer, embed %d, %d heads, %d new tokens on a cache of %d, 8-bit block-quantised weights (blocks of 64)"
-                               % (embed, heads, src, past), "launches_per_step": (6 if rows_ws is not None else 3) + (1 if wsb.value else 0), "projections": "tiled bf16x3 kernel" if rows_ws is not None else ("packed tiles" if packed_ok else ".bin layout"), "device_ms_per_step": k_ms, "gflop": ops / 1e9},
+                               % (embed, heads, src, past), "projections": "packed tiles, many rows" if rows_ws is not None else ("packed tiles" if packed_ok else ".bin layout"), "device_ms_per_step": k_ms, "gflop": ops / 1e9},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": None,
                      "kernel": "whole layer (q/k/v projection, cache append, attention core, output projection)", "bytes_per_launch": algo},
     }
