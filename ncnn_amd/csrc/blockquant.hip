@@ -2349,8 +2349,11 @@ static int gemm_blockquant_packed(const char* who, const void* a_dev, int ain, s
     const int split = block == 32 ? 1 : 0;
     hipStream_t st = as_stream(stream);
     if (ain == 2 && many_rows_f16(M, N, K, bits, block))
+    {
+        bool handled; // (always)
         return launch_blockquant_rows_f16(static_cast<const uint16_t*>(a_dev), a_stride, M, K, bits, block,
-                                          one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride), st);
+                                          one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride), &handled, st);
+    }
     if (ain == 4 && many_rows_f32(M, K))
         return launch_blockquant_rows_f32(static_cast<const float*>(a_dev), a_stride, M, K, bits, block, in_scales_dev,
                                           one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride), st);
@@ -2663,7 +2666,13 @@ int ncnnhip_gemm_blockquant_packed_multi(const void* a_dev, int a_elemsize, size
         mm.tile_end[i] = (int)tiles, mm.N[i] = 0, mm.bt[i] = -1, mm.alpha[i] = mm.beta[i] = 1.f;
         mm.wpk[i] = 0, mm.dpk[i] = 0, mm.c[i] = 0, mm.out[i] = 0, mm.out_stride[i] = 0;
     }
-    if (one_pass && a_elemsize == 2 && many_rows_f16(M, tiles * 16, K, bits, block)) return launch_blockquant_rows_f16(static_cast<const uint16_t*>(a_dev), a_stride, M, K, bits, block, mm, as_stream(stream));
+    if (one_pass && a_elemsize == 2 && many_rows_f16(M, tiles * 16, K, bits, block))
+    {
+        bool handled = false;
+        const int ret = launch_blockquant_rows_f16(static_cast<const uint16_t*>(a_dev), a_stride, M, K, bits, block, mm, &handled, as_stream(stream));
+        if (ret != NCNNHIP_OK || handled) return ret;
+        one_pass = false;
+    }
     if (one_pass && a_elemsize == 4 && many_rows_f32(M, K))
         return launch_blockquant_rows_f32(static_cast<const float*>(a_dev), a_stride, M, K, bits, block, in_scales_dev, mm, as_stream(stream));
     if (one_pass)

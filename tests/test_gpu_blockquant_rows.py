@@ -235,3 +235,21 @@ def test_several_matrices_whose_groups_would_fill_the_units_only_together(rt):
     mats = [rt.blockquant_pack(p, s, 64, bits=4, k=k) + (n, None, -1, 1.0, 1.0) for _, p, s in ops]
     for got, (_, packed, scales) in zip(rt.gemm_blockquant_packed_multi(a, mats, bits=4, block=64), ops):
         _check(got, a.astype(F), packed, scales, 4, 64)
+
+
+@pytest.mark.parametrize("m,k,ns,bits,block", [
+    # the cheapest shape for all matrices has fewer wavefronts than the one each matrix gets alone: 8 bits 8 and 7, 4 bits 8 and 7, 8 and 6
+    (48, 528, (4096,) * 3, 8, 64), (64, 512, (4096,) * 3, 4, 64), (64, 592, (11008,) * 2, 4, 32), (48, 512, (11008,) * 2, 8, 64),
+    # matrices that alone get different numbers of wavefronts
+    (64, 512, (4096, 11008), 8, 64), (57, 512, (16, 4096, 17600), 4, 64)])
+def test_several_matrices_of_fp16_rows_get_the_bits_of_single_calls(rt, m, k, ns, bits, block):
+    """Where the number of wavefronts that share K, and with it the order of the sums, follows from the shape of the launch."""
+    print("[case]", m, k, ns, bits, block, flush=True)
+    rng = np.random.default_rng(m + k)
+    a = rng.normal(0, 1, (m, k)).astype(np.float16)
+    mats = []
+    for n in ns:
+        fields = rng.integers(0, 256, (n, k * bits // 8), dtype=np.uint8)
+        mats.append(rt.blockquant_pack(fields, rng.uniform(50, 100, (n, -(-k // block))).astype(F), block, bits=bits, k=k) + (n, None, -1, 1.0, 1.0))
+    for got, (pw, pd, n, *_) in zip(rt.gemm_blockquant_packed_multi(a, mats, bits=bits, block=block), mats):
+        assert np.array_equal(got, rt.gemm_blockquant_packed(a, pw, pd, n, bits=bits, block=block)), n
