@@ -241,9 +241,12 @@ def test_several_matrices_whose_groups_would_fill_the_units_only_together(rt):
     # the cheapest shape for all matrices has fewer wavefronts than the one each matrix gets alone: 8 bits 8 and 7, 4 bits 8 and 7, 8 and 6
     (48, 528, (4096,) * 3, 8, 64), (64, 512, (4096,) * 3, 4, 64), (64, 592, (11008,) * 2, 4, 32), (48, 512, (11008,) * 2, 8, 64),
     # matrices that alone get different numbers of wavefronts
-    (64, 512, (4096, 11008), 8, 64), (57, 512, (16, 4096, 17600), 4, 64)])
+    (64, 512, (4096, 11008), 8, 64), (57, 512, (16, 4096, 17600), 4, 64),
+    # 5 to 16 rows: small weights go to another kernel than large ones, alone or not
+    (16, 4096, (4096,) * 2, 4, 64), (7, 4096, (4096,) * 2, 6, 32), (5, 4096, (4096, 8192), 4, 64), (16, 8208, (2000, 6000), 8, 64), (16, 4096, (4096, 7200), 8, 32), (9, 1040, (16400, 64), 8, 64)])
 def test_several_matrices_of_fp16_rows_get_the_bits_of_single_calls(rt, m, k, ns, bits, block):
-    """Where the number of wavefronts that share K, and with it the order of the sums, follows from the shape of the launch."""
+    """Where the number of wavefronts that share K, and with it the order of the sums, follows from the shape of the launch, and where
+    the kernel follows from the size of the weights."""
     print("[case]", m, k, ns, bits, block, flush=True)
     rng = np.random.default_rng(m + k)
     a = rng.normal(0, 1, (m, k)).astype(np.float16)
