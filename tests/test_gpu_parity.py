@@ -853,6 +853,33 @@ def test_attention_core_on_split_keys_and_values_with_numbers_it_cannot_carry(rt
     assert ok.any() and not ok.all() and np.abs(got[ok] / np.maximum(np.abs(plain[ok]), 1.0) - plain[ok] / np.maximum(np.abs(plain[ok]), 1.0)).max() <= 2e-5
 
 
+@pytest.mark.parametrize("heads,hd,src,dst", [(2, 64, 40, 100), (1, 128, 70, 300), (3, 32, 33, 33), (1, 96, 300, 65)])
+@pytest.mark.parametrize("exponent", [100, 111, 114, 118, 122, 124])
+def test_attention_core_on_split_keys_and_values_with_numbers_too_small_to_split(rt, heads, hd, src, dst, exponent):
+    """Below 2^-110 the least of three bf16 numbers would lie below the smallest bf16 (2^-133): values, keys and queries of that size keep
+    the error against float64 of the fp32 form, all of them being small (keys against large queries and the other way round) or one."""
+    rng = np.random.default_rng(src + exponent)
+    e, tiny, huge = heads * hd, F(2.0 ** -exponent), F(2.0 ** exponent)
+    q = (rng.normal(0, 1, (src, e)) / np.sqrt(hd)).astype(F)
+    kt, vt = (rng.normal(0, 1, (e, dst)).astype(F) for _ in range(2))
+    one = vt.copy()
+    one[hd - 3, dst - 2] = F(1.2345678) * tiny
+    one[hd - 3, : dst - 2], one[hd - 3, dst - 1] = 0, 0  # alone in its channel: its relative error is the result's
+    for a, b, c in ((q, kt, vt * tiny), (q * huge, kt * tiny, vt), (q * tiny, kt * huge, vt), (q, kt, one)):
+        got, plain = rt.attention(a, b, c, heads), rt.attention(a, b, c, heads, use_workspace=False)
+        want = np.empty((src, e))
+        for h in range(heads):
+            sl = slice(h * hd, (h + 1) * hd)
+            s = a[:, sl].astype(np.float64) @ b[sl].astype(np.float64)
+            s = np.exp(s - s.max(axis=1, keepdims=True))
+            want[:, sl] = (s / s.sum(axis=1, keepdims=True)) @ c[sl].astype(np.float64).T
+        for cols in (slice(None), slice(hd - 3, hd - 2)):  # relative to the norm of the whole, and of the channel that one small value makes alone
+            norm = np.sqrt(np.mean(want[:, cols] ** 2))
+            error, fp32 = (np.sqrt(np.mean((x[:, cols] - want[:, cols]) ** 2)) / norm for x in (got, plain))
+            # no worse than the fp32 form but for the spread between two orders of a sum (of a few terms in the least case: 2 * 2^-24)
+            assert error <= 1.25 * fp32 + 2.0 ** -23, (exponent, error, fp32)
+
+
 @pytest.mark.parametrize("heads,hd,src,dst", [(4, 64, 37, 200), (2, 32, 1, 300), (3, 24, 5, 40)])
 def test_attention_reads_strided_queries_and_scales_them_on_load(rt, heads, hd, src, dst):
     """Queries taken out of a wider row (q, k and v made by one Gemm) and multiplied by the layer's scale where they are read:
