@@ -294,6 +294,14 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
     }
 }
 
+// Between a wavefront's writes to its own piece of LDS and its reads of what other lanes wrote there: LDS serves a wavefront in order, so no
+// instruction comes of it, but the compiler may not move memory accesses across it either.
+__device__ __forceinline__ void exchange_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Few tiles (gemm_int8_streams): the W wavefronts of a workgroup each multiply the whole BM x BN tile over a run of K steps of their own.
 // A wavefront fetches 128 bytes of each of its rows into registers (coalesced, any alignment), turns them into the operand mapping through
 // a piece of LDS that belongs to it alone -- LDS serves a wavefront in order, so no barrier stands in the loop -- and requests the next
@@ -373,7 +381,7 @@ __global__ __launch_bounds__(64 * W) void gemm_int8_stream_kernel(const int8_t* 
         for (int i = 0; i < LA; i++) *reinterpret_cast<v4i*>(smem + i * 1024 + (i & 1 ? wr1 : wr0)) = ra[i];
 #pragma unroll
         for (int i = 0; i < LB; i++) *reinterpret_cast<v4i*>(smem + BM * KSTEP + i * 1024 + (i & 1 ? wr1 : wr0)) = rb[i];
-        __builtin_amdgcn_wave_barrier();
+        exchange_fence();
         fetch(t + 1); // (past the last step: the first again)
         v4i fa[4][TM], fb[4][TN]; // every read before the first product, as above
 #pragma unroll
@@ -391,7 +399,7 @@ __global__ __launch_bounds__(64 * W) void gemm_int8_stream_kernel(const int8_t* 
             for (int i = 0; i < TM; i++)
 #pragma unroll
                 for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[q][i], fb[q][j], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_wave_barrier();
+        exchange_fence();
     }
 
     int* sums = reinterpret_cast<int*>(smem);
