@@ -350,12 +350,13 @@ int MultiHeadAttention_hip::forward(const std::vector<Mat>& bottom_blobs, std::v
     rc = ncnnhip_attention_workspace_bytes(num_heads, head_dim, src, dst, &att_ws_bytes);
     if (rc != 0) return to_ncnn_status(rc, "ncnnhip_attention_workspace_bytes");
     void* att_ws = att_ws_bytes ? leases.get(att_ws_bytes) : 0;
-    if (!att_ws) att_ws_bytes = 0; // no room: the call falls back to the kernel that needs none
+    const bool no_room = att_ws_bytes && !att_ws; // the call falls back to the kernels that need none, where one takes the shape
+    if (no_room) att_ws_bytes = 0;
     if (fused_qkv) // the new key and value columns are written behind the cache by the same call
         rc = ncnnhip_attention_f32_append(d_qa, q_stride, scale, d_kt, d_vt, (size_t)dst, past, d_mask, mask_heads, num_heads, head_dim, src, d_ctx, att_ws, att_ws_bytes, st);
     else
         rc = ncnnhip_attention_f32(d_qa, d_kt, d_vt, (size_t)dst, d_mask, mask_heads, num_heads, head_dim, src, dst, d_ctx, att_ws, att_ws_bytes, st);
-    if (rc != 0) return to_ncnn_status(rc, "ncnnhip_attention_f32");
+    if (rc != 0) return no_room ? -100 : to_ncnn_status(rc, "ncnnhip_attention_f32");
     rc = blockquant_gemm_with_scratch(leases, d_ctx, E, src, qdim, embed_dim, dev[3][0], bits, block, dev[3][1], dev[3][2], dev[3][4], dev[3][5],
                                     (const float*)dev[3][3], 4, 1.f, 1.f, d_out, (size_t)qdim, st);
     if (rc != 0) return to_ncnn_status(rc, "out projection");
@@ -516,12 +517,13 @@ int MultiHeadAttention_hip::forward_hip(const std::vector<HipMat>& bottom_blobs,
     rc = ncnnhip_attention_workspace_bytes(num_heads, head_dim, src, dst, &att_ws_bytes);
     if (rc != 0) return to_ncnn_status(rc, "ncnnhip_attention_workspace_bytes");
     void* att_ws = att_ws_bytes ? scratch.get(att_ws_bytes) : 0;
-    if (!att_ws) att_ws_bytes = 0; // no room: the call falls back to the kernel that needs none
+    const bool no_room = att_ws_bytes && !att_ws; // the call falls back to the kernels that need none, where one takes the shape
+    if (no_room) att_ws_bytes = 0;
     if (fused_qkv) // the new key and value columns are written behind the cache by the same call
         rc = ncnnhip_attention_f32_append(d_qa, q_stride, scale, d_kt, d_vt, (size_t)dst, past, d_mask, mask_heads, num_heads, head_dim, src, d_ctx, att_ws, att_ws_bytes, st);
     else
         rc = ncnnhip_attention_f32(d_qa, d_kt, d_vt, (size_t)dst, d_mask, mask_heads, num_heads, head_dim, src, dst, d_ctx, att_ws, att_ws_bytes, st);
-    if (rc != 0) return to_ncnn_status(rc, "ncnnhip_attention_f32");
+    if (rc != 0) return no_room ? -100 : to_ncnn_status(rc, "ncnnhip_attention_f32");
     rc = blockquant_gemm_with_scratch(scratch, d_ctx, E, src, qdim, embed_dim, dev[3][0], bits, block, dev[3][1], dev[3][2], dev[3][4], dev[3][5],
                                     (const float*)dev[3][3], 4, 1.f, 1.f, (float*)top.data, (size_t)qdim, st);
     if (rc != 0) return to_ncnn_status(rc, "out projection");

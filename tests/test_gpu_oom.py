@@ -8,8 +8,10 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import cases
 import refnet
-from ncnn_amd import hip, host, zoo
+from ncnn_amd import hip, host, modelwriter as mw, zoo
+from oracle import oracle
 
 pytestmark = pytest.mark.gpu
 F = np.float32
@@ -144,3 +146,53 @@ def test_device_allocation_failing_gives_minus_100(resident):
         restore()
     ret, got = one_pass()
     assert ret == 0 and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("resident", [False, True], ids=["host-blobs", "device-resident"])
+@pytest.mark.parametrize("embed,heads,src,past,expected", [
+    # with the scratch refused: the fp32 matrix cores, and the general kernel where the keys fit its LDS
+    (128, 2, 300, 0, 0), (128, 2, 1, 4000, 0), (80, 2, 3, 3900, 0),
+    # head dimension 40 on 4201 keys runs on the streaming kernel only, which needs its scratch
+    (80, 2, 1, 4200, -100)])
+def test_attention_scratch_refused(embed, heads, src, past, expected, resident):
+    """The scratch of the attention core is not worth failing for where a kernel does without; where none does, the pass is out of memory."""
+    K = hip.lib()
+    case = cases.mha_case(31, embed, heads, embed, embed, embed, src, src, 8, 64, False, past, True, None)
+    bottoms, tops, lines = ["q"], ["out"], ["Input in_q 0 1 q 0=%d 1=%d" % (embed, src)]
+    if past:
+        lines += ["Input in_ck 0 1 ck", "Input in_cv 0 1 cv"]
+        bottoms, tops = ["q", "ck", "cv"], ["out", "ko", "vo"]
+    lines.append(mw.mha_param("mha", bottoms, tops, embed, heads, embed, embed, embed, attn_mask=0, kv_cache=int(bool(past)), quantize_term=801))
+    net = host.Net()
+    assert net.register_attention_layer() == 0
+    net.set_use_hip_compute(resident)
+    assert net.load_param_mem(mw.assemble_param(lines)) == 0 and net.load_model_mem(mw.mha_blockquant_weights(case["weights"])) == 0
+    size = C.c_size_t()
+    hip.check(K.ncnnhip_attention_workspace_bytes(heads, embed // heads, src, past + src, C.byref(size)))
+    refused = [0]
+
+    @MALLOC_FN
+    def refusing_malloc(dev, nbytes, user):
+        if size.value <= nbytes < size.value + 65536:  # (a pool asks for whole 64 KB)
+            refused[0] += 1
+            return -100
+        return K.ncnnhip_default_device_malloc(dev, nbytes)
+
+    @FREE_FN
+    def plain_free(dev, user):
+        return K.ncnnhip_default_device_free(dev)
+
+    ex = net.create_extractor(own_stream=not resident)
+    ex.input("q", case["q"])
+    if past:
+        ex.input("ck", case["cached_k"])
+        ex.input("cv", case["cached_v"])
+    try:
+        hip.check(K.ncnnhip_set_device_allocator(C.cast(refusing_malloc, C.c_void_p), C.cast(plain_free, C.c_void_p), None))
+        ret, got = _extract_code(ex, "out")
+    finally:
+        hip.check(K.ncnnhip_set_device_allocator(None, None, None))
+    assert refused[0] >= 1 and ret == expected
+    if ret == 0:
+        want = oracle.mha_blockquant(**dict(case, self_attention=True))[0]
+        assert np.abs(got - want).max() <= 2e-5 * max(1.0, np.abs(want).max())
