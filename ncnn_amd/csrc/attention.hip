@@ -789,6 +789,12 @@ __device__ __forceinline__ void load_fewq_values(float (&vv)[16], const float* _
         for (int e = 0; e < 16; e++) vv[e] = vr[j + e < dst ? j + e : dst - 1];
     }
 }
+// The slots behind the last key of all hold some key's value a second time: zeros instead, as their probability, zero, times an infinity is no number
+__device__ __forceinline__ void drop_fewq_values(float (&vv)[16], int j, int dst)
+{
+#pragma unroll
+    for (int e = 0; e < 16; e++) vv[e] = j + e < dst ? vv[e] : 0.f;
+}
 
 // new_k / new_v (or null): the keys and values of the last dst - past positions, rows of new_stride floats ([position][embed]).
 // The workgroup whose 64 keys reach past `past` first copies its share of them into kt / vt (appending to the cache is then
@@ -897,6 +903,7 @@ __global__ __launch_bounds__(256) void attention_fewq_split_kernel(const float* 
             }
             else
                 load_fewq_values(vv, vt + ((size_t)h * head_dim + ch) * kv_stride, j0 + 16 * kq, dst, vec);
+            if (j0 + FEWQ_KEYS > dst) drop_fewq_values(vv, j0 + 16 * kq, dst);
 #pragma unroll
             for (int e = 0; e < 16; e++)
 #pragma unroll
@@ -978,6 +985,11 @@ __global__ __launch_bounds__(256) void attention_fewq_split_hd_kernel(const floa
                 for (int e = 0; e < 16; e++) vv[i][e] = 16 * kq + e == at ? v : vv[i][e];
             }
         }
+    }
+    if (j0 + FEWQ_KEYS > dst) // uniform: the last workgroup of a head
+    {
+#pragma unroll
+        for (int i = 0; i < NV; i++) drop_fewq_values(vv[i], j0 + 16 * kq, dst);
     }
 
     // ---- scores: wavefront g takes the g-th quarter of the channels, lane = key

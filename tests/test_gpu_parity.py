@@ -937,3 +937,30 @@ def test_attention_of_few_queries_reads_new_columns_where_they_come_from(rt, hea
     that are and are not 16-byte aligned.  Against float64 too: fp32 sums over head_dim and dst terms of O(1) values."""
     test_attention_appends_the_new_keys_and_values_itself(rt, heads, hd, src, past, mask)
     test_attention_core_matches_float64(rt, heads, hd, src, past + src, mask)
+
+
+@pytest.mark.parametrize("heads,hd,src,past", [(2, 64, 1, 299), (3, 32, 3, 318), (2, 128, 2, 320), (1, 96, 4, 383), (2, 40, 1, 256), (2, 80, 2, 300)])
+def test_attention_of_few_queries_keeps_an_infinite_value_infinite(rt, heads, hd, src, past):
+    """An infinity in the last cached and in the last new value: the places of a workgroup's 64 keys behind the last key of all have no
+    part in the sums, whatever was read for them, with the new columns appended by the call and without."""
+    rng = np.random.default_rng(heads * 1000 + past)
+    e, dst = heads * hd, past + src
+    qkv = rng.normal(0, 1, (src, 3 * e)).astype(F)
+    kt, vt = (rng.normal(0, 1, (e, dst)).astype(F) for _ in range(2))
+    vt[1, past - 1], vt[e - 1, past - 1] = np.inf, -np.inf
+    qkv[src - 1, 2 * e + 4], qkv[src - 1, 3 * e - 3] = -np.inf, np.inf
+    kt[:, past:], vt[:, past:] = qkv[:, e:2 * e].T, qkv[:, 2 * e:].T
+    scale = F(1.0 / np.sqrt(hd))
+    got = rt.attention(qkv, kt, vt, heads, q_scale=scale)
+    cached = np.arange(dst) < past
+    appended = rt.attention_append(qkv, np.where(cached, kt, F(7)), np.where(cached, vt, F(7)), heads, past, scale)[0]
+    want = np.empty((src, e))
+    for h in range(heads):
+        sl = slice(h * hd, (h + 1) * hd)
+        s = (qkv[:, sl] * scale).astype(np.float64) @ kt[sl].astype(np.float64)
+        s = np.exp(s - s.max(axis=1, keepdims=True))
+        want[:, sl] = (s / s.sum(axis=1, keepdims=True)) @ vt[sl].astype(np.float64).T
+    ok = np.isfinite(want)
+    assert (~ok).sum() == 4 * src and not np.isnan(want).any()
+    for x in (got, appended):
+        assert np.array_equal(x[~ok], want[~ok]) and np.abs(x[ok] - want[ok]).max() <= 2e-5 * max(1.0, np.abs(want[ok]).max())
