@@ -216,9 +216,9 @@ static inline bool halves_layout(int bits, int block)
 // of its own (never so for one matrix).
 int launch_blockquant_rows_f16(const uint16_t* a, size_t a_stride, int M, int K, int bits, int block, const BqMulti& mm, bool* handled, hipStream_t stream);
 
-// The same with fp32 rows (16-byte aligned) and optional input scales; and about how long that takes (tiles: of 16 weight rows, of all
-// matrices), with the shape it will take.
-double blockquant_rows_f32_us(int M, int K, long long tiles, int* mg, int* rt);
+// The same with fp32 rows (16-byte aligned) and optional input scales; and about how long that takes for `count` matrices of N[i] rows, with the shape
+// it will take.
+double blockquant_rows_f32_us(int M, int K, const int* N, int count, int* mg, int* rt);
 int launch_blockquant_rows_f32(const float* a, size_t a_stride, int M, int K, int bits, int block, const float* in_scales, const BqMulti& mm, hipStream_t stream);
 
 // Many rows of fp32 activations, weights in blocks of 64 or 128 (blockquant_tiles.hip); the workspace is that of ncnnhip_gemm_blockquant_packed_rows.

@@ -2470,7 +2470,7 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
     const double rounds = (double)(((long long)((ntiles + 7) / 8) * (Mp / 64) + 255) / 256); // of 64 x 128 tiles
     int mg, rt;
     if (aligned
-        && blockquant_rows_f32_us(M, K, ntiles, &mg, &rt)
+        && blockquant_rows_f32_us(M, K, &N, 1, &mg, &rt)
                < 9.0 + K / 1024.0 * (tiles64 <= 256 ? 7.8 : block != 32 ? 11.0 * rounds : tiles64 <= 512 ? 14.2 : 17.0 * tiles64 / 512.0))
         return launch_blockquant_rows_f32(a_dev, a_stride, M, K, bits, block, in_scales_dev, one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride),
                                           st);

@@ -601,15 +601,17 @@ int launch_blockquant_rows_f16(const uint16_t* a, size_t a_stride, int M, int K,
 // fp32 rows: groups of activation rows and tiles per workgroup, the cheapest pair under rounds x (2.3 + 0.7 MG RT + K / 4096 x (4 + 2.2 MG +
 // 1.4 MG RT)) us, the form of 90 measured pairs at 8 bits (four groups leave room for 4 or 5 wavefronts and were not better anywhere).  The grid's
 // padding to 8 groups counts: 81 groups in 3 passes are 264 workgroups, a second round (37 rows of 5154 x 768 13.0 us with 1 x 4, 8.8
-// with 2 x 3).
-double blockquant_rows_f32_us(int M, int K, long long tiles, int* mg, int* rt)
+// with 2 x 3).  Several matrices are counted one by one, as for fp16 rows.
+double blockquant_rows_f32_us(int M, int K, const int* N, int count, int* mg, int* rt)
 {
     const int rows16 = (M + 15) / 16;
     double best = 0.0;
     for (int g = 1; g <= 2; g++)
         for (int r = 1; r <= 4; r++)
         {
-            const long long wgs = ((tiles + r - 1) / r + 7) / 8 * 8 * ((rows16 + g - 1) / g);
+            long long wgs = 0;
+            for (int i = 0; i < count; i++) wgs += ((N[i] + 15) / 16 + r - 1) / r;
+            wgs = (wgs + 7) / 8 * 8 * ((rows16 + g - 1) / g);
             const double us = (double)((wgs + 255) / 256) * (2.3 + 0.7 * g * r + K / 4096.0 * (4.0 + 2.2 * g + 1.4 * g * r));
             if (best == 0.0 || us < best) best = us, *mg = g, *rt = r;
         }
@@ -618,10 +620,8 @@ double blockquant_rows_f32_us(int M, int K, long long tiles, int* mg, int* rt)
 
 int launch_blockquant_rows_f32(const float* a, size_t a_stride, int M, int K, int bits, int block, const float* in_scales, const BqMulti& mm, hipStream_t stream)
 {
-    long long tiles = 0;
-    for (int i = 0; i < mm.count; i++) tiles += (mm.N[i] + 15) / 16;
     int mg = 1, rt = 1;
-    blockquant_rows_f32_us(M, K, tiles, &mg, &rt);
+    blockquant_rows_f32_us(M, K, mm.N, mm.count, &mg, &rt);
     const int passes = ((M + 15) / 16 + mg - 1) / mg;
 #define ONE(BITS_, HALVES_, SPLIT_, MG_, RT_) return launch_one<BITS_, HALVES_, SPLIT_, MG_, RT_, 4>(a, a_stride, M, K, passes, in_scales, mm, stream)
 #define ONE_RT(BITS_, HALVES_, SPLIT_, MG_)              \

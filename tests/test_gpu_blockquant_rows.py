@@ -182,9 +182,10 @@ def test_fp32_rows_off_16_bytes_take_the_general_forms(rt):
         assert np.all(got[:, n:] == 7.0) and np.all(out[:o_off] == 7.0), (o_stride, o_off)
 
 
-@pytest.mark.parametrize("m,k", [(3, 144), (4, 4112), (9, 208), (16, 1040), (17, 208)])
-def test_several_matrices_of_fp32_rows_get_the_bits_of_single_calls(rt, m, k):
-    ns = (50, 16, 4200)
+@pytest.mark.parametrize("m,k,ns", [(3, 144, (50, 16, 4200)), (4, 4112, (50, 16, 4200)), (9, 208, (50, 16, 4200)), (16, 1040, (50, 16, 4200)), (17, 208, (50, 16, 4200)),
+                                    # groups of three tiles would be 256 only if they went across matrices: groups of four, and padding to whole eights
+                                    (5, 1040, (4096,) * 3), (16, 2064, (4096, 4090, 4081)), (13, 208, (1000,) * 8)])
+def test_several_matrices_of_fp32_rows_get_the_bits_of_single_calls(rt, m, k, ns):
     ops = [synth.blockquant_operands(10 + i, m, n, k, 8, 64, half_exact=False) for i, n in enumerate(ns)]
     a = ops[0][0]
     mats = [rt.blockquant_pack(p, s, 64, k=k) + (n, None, -1, 1.0, 1.0) for (_, p, s), n in zip(ops, ns)]
