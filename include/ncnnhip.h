@@ -422,24 +422,25 @@ int ncnnhip_gemm_blockquant_packed(const float* a_dev, size_t a_stride, int M, i
 /* Several packed weight matrices on the SAME activation rows in one launch: the gate and up projections of a decoder layer, the
  * q / k / v projections of an attention layer -- in the reference one Gemm / MultiHeadAttention projection after the other
  * (src/layer/gemm.cpp:425-483 per matrix); the results are those of `count` calls of ncnnhip_gemm_blockquant_packed(_f16a), bit
- * for bit.  a_elemsize 2: fp16 activations (up to 16 rows in one pass); 4: fp32 (up to 16 rows, with optional in_scales [K]).
+ * for bit.  a_elemsize 2: fp16 activations; 4: fp32, with optional in_scales [K].
  * All matrices share K, bits and block; N, the packed weights and descales, C (c_dev or its entries may be null), its broadcast
  * type, alpha, beta (null: 1) and the outputs are per matrix, count <= 8.  A decode-sized launch is paced by its ramp and tail,
- * not by bandwidth: one launch over 2 x 45.8 MB reaches what two launches of 45.8 MB cannot.  Shapes the one-pass kernel does
- * not take run matrix by matrix. */
+ * not by bandwidth: one launch over 2 x 45.8 MB reaches what two launches of 45.8 MB cannot.  Matrix by matrix run: more than 16
+ * fp32 rows; fp16 rows where the matrices alone would take different kernels, or cut K into different numbers of pieces; and what no
+ * kernel takes whole. */
 int ncnnhip_gemm_blockquant_packed_multi(const void* a_dev, int a_elemsize, size_t a_stride, int M, int K, int count, const int* N,
                                          const uint8_t* const* packed_w_dev, const float* const* packed_descale_dev, int bits,
                                          int block, const float* in_scales_dev, const float* const* c_dev, const int* broadcast_type_c,
                                          const float* alpha, const float* beta, float* const* out_dev, const size_t* out_stride,
                                          void* stream);
 
-/* The same contract from five activation rows up, with a workspace: the three-way split is made once, by a pass of its own,
- * into the workspace (ncnnhip_gemm_blockquant_packed_rows_workspace_bytes: 6 bytes per activation, rows and K rounded up to 64).
- * Up to 128 rows, while streaming the weights once per 16 rows is cheaper than a tiled pass (small weight matrices, or few
- * rows), the weights are streamed once per 16 rows in the few-row kernel's shape, all passes in one launch, the activations
- * pre-arranged as the lanes load them; otherwise a tiled Gemm runs on the bf16 matrix cores, 128 weight rows x 64 activation
- * rows per workgroup (prefill, attention projections).  K % 16 == 0; the workspace is scratch
- * (overwritten by every call). */
+/* The same contract with a workspace (ncnnhip_gemm_blockquant_packed_rows_workspace_bytes: 6 bytes per activation, rows and K
+ * rounded up to 64), for five activation rows and more, or three and more where K is beyond 4096.  Rows (and input scales) on 16 bytes
+ * go, while that is the quicker way (some tens to some hundreds of rows), to the kernel ncnnhip_gemm_blockquant_packed has for more than
+ * four, which splits the activations as it multiplies them and leaves the workspace alone.  All others are split once, into the workspace,
+ * by a pass of its own: up to 128 rows off 16 bytes on small weights then stream the weights once per 16 rows, all passes in one launch;
+ * the rest is a tiled Gemm on the bf16 matrix cores, 64 activation rows x 64, 128 or 192 weight rows per workgroup (prefill, attention
+ * projections).  K % 16 == 0; the workspace is scratch (to be taken as overwritten by every call). */
 int ncnnhip_gemm_blockquant_packed_rows_workspace_bytes(int M, int K, size_t* bytes);
 int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int M, int N, int K, const uint8_t* packed_w_dev,
                                         const float* packed_descale_dev, int bits, int block, const float* in_scales_dev,

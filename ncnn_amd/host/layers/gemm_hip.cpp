@@ -673,8 +673,10 @@ unsigned long long Gemm_hip::hip_sibling_key() const
 }
 
 // Every member's forward_hip on the one bottom, in one launch of ncnnhip_gemm_blockquant_packed_multi: bit for bit what
-// the members give one by one (the same kernel; a workgroup only finds its matrix differently).  Up to four activation
-// rows (the one-pass form of fp32 activations) and eight members; anything else: done = false, the layers run on their own.
+// the members give one by one (the same kernel; a workgroup only finds its matrix differently).  Up to eight members and four
+// activation rows: from five on the members alone go to ncnnhip_gemm_blockquant_packed_rows, which may pick a tiled kernel with
+// another order of additions (from about 50000 weight rows at K = 1024, for one) where the shared launch has only one kernel for
+// fp32 rows.  Anything else: done = false, the layers run on their own.
 int Gemm_hip::forward_hip_siblings(const std::vector<const Layer*>& group, const HipMat& A, std::vector<HipMat>& top_blobs, HipCommand& cmd, const Option&,
                                    bool& done) const
 {

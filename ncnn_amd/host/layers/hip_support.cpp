@@ -75,10 +75,9 @@ int upload_blockquant_packed(const void* fields_host, const float* scales_host, 
 
 size_t blockquant_gemm_workspace_bytes(int M, int K, const void* d_packed)
 {
-    // 5 rows and more: the kernels that split the activations in a pass of their own (the weight-streaming one on pre-split
-    // operands, 16 rows per pass, while that is cheaper than a tiled pass; else the tiled one: the entry point picks).
-    // 3 and 4 rows of a K beyond 4096 too: the few-row kernel holds three planes per row in LDS and takes such rows one at
-    // a time, a pass over the weights each (4096 x 11008, 4 rows: 48 us against 26 us this way).
+    // 5 rows and more, and 3 and 4 of a K beyond 4096: ncnnhip_gemm_blockquant_packed_rows, which picks by its estimates between the
+    // kernel that splits the activations as it multiplies them (most calls of up to some hundred rows; the workspace stays unused)
+    // and those that split them into the workspace first.  Fewer rows, whose planes the one-pass kernel holds in LDS, need none.
     if (!d_packed || K % 16 != 0 || M < 3 || (M < 5 && K <= 4096)) return 0;
     size_t bytes = 0;
     if (ncnnhip_gemm_blockquant_packed_rows_workspace_bytes(M, K, &bytes) != 0) return 0;
@@ -89,12 +88,12 @@ int blockquant_gemm_device(const float* a_dev, size_t a_stride, int M, int N, in
                            const void* d_in_scales, const void* d_packed, const void* d_descales, const float* c_dev, int bt, float alpha, float beta,
                            float* out_dev, size_t out_stride, void* workspace, size_t workspace_bytes, void* stream)
 {
-    // five rows and more: the kernels that split the activations in a pass of their own, when the caller brought the workspace for it
+    // as above, when the caller brought the workspace for it
     const size_t need = blockquant_gemm_workspace_bytes(M, K, d_packed);
     if (need && d_descales && workspace && workspace_bytes >= need)
         return ncnnhip_gemm_blockquant_packed_rows(a_dev, a_stride, M, N, K, (const uint8_t*)d_packed, (const float*)d_descales, bits, block,
                                                    (const float*)d_in_scales, c_dev, bt, alpha, beta, out_dev, out_stride, workspace, workspace_bytes, stream);
-    // few rows: the packed tiles, one pass over the weights per four rows at most
+    // without one: the packed tiles, up to four rows in the one-pass kernel, more in the one that splits the activations itself
     if (d_packed && d_descales && M < 32 && ncnnhip_gemm_blockquant_packed_supported(K) && a_stride % 4 == 0 && ((uintptr_t)a_dev & 15) == 0
         && (!d_in_scales || ((uintptr_t)d_in_scales & 15) == 0))
         return ncnnhip_gemm_blockquant_packed(a_dev, a_stride, M, N, K, (const uint8_t*)d_packed, (const float*)d_descales, bits, block,
