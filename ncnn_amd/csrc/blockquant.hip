@@ -2507,11 +2507,16 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
 #undef ROWS16
         return launch_status("blockquant_rows16_bf16x3_kernel");
     }
-    // More than one 64 x 64 tile per compute unit: the kernel with 64 x 128 tiles (one scale a step: not blocks of 32).  It is quicker there
-    // at every K and N measured (1.02 to 1.44 times, 120 shapes of 65 to 1500 rows, K 512 to 11008), with one exception: 8-bit fields in just
-    // over two rounds of it where the kernel below has one round of 64 x 192 tiles, two to a unit (K = 4096, 544 tiles of 64 x 128: 132.6
-    // us below, 140.1 there; 672: 146 148; 704: 150.5 150.1; at 512 115 105 and at 768 182 155).  With fewer tiles the kernel below that
-    // splits K over two groups puts more units to work (128 tiles of 64 x 128, 256 x 4096 x 4096: 45.7 us against 47.7).
+    // More than one 64 x 64 tile per compute unit: the kernel with 64 x 128 tiles (one scale a step: not blocks of 32).  It is quicker there (1.02 to
+    // 1.44 times, 120 shapes of 65 to 1500 rows, K 512 to 11008; of 1600 to 24000 rows, N 192 to 4096, 191 shapes: 1.05 in the median, 14 of them below 0.98,
+    // where N is at most 1024 or K at most 512: 9000 x 192 x 512 27.2 31.7, 24000 x 256 x 512 57.4 64.6), with one exception: 8-bit fields in just over two
+    // rounds of it where the kernel below has one round of 64 x 192 tiles, two to a unit.  There the two are close, and which is the quicker depends on
+    // what runs around them: among a self-attention layer's other kernels (1500 tokens, 1024 channels: 1500 x 3072 x 1024) the layer takes 150 us with the one below
+    // and 156 with the one here.  Back to back, below / here: N 512 to 1024, K 512 to 6144 2 to 12 % less below (5504 x 768 x 4096 168 191), at K
+    // 128 and 256 within 4 % either way; N 1536 up to 5 % less below at K 768 to 2048 (3500 rows, K 1024 58.9 61.3), 2 to 10 % more at others; N
+    // 2048 to 11008, K 128 to 16384 from 2 % less below to 10 % more, 3 in the median (1500 x 3072 x 1024 54.6 51.9, 1024 x 5120 x 8192 278 262).
+    // With fewer tiles the kernel below that splits K over two groups puts more units to work (128 tiles of 64 x 128, 256 x 4096 x
+    // 4096: 45.7 us against 47.7).
     const long long tiles128 = (long long)((ntiles + 7) / 8) * (Mp / 64), tiles192 = (long long)((ntiles + 11) / 12) * (Mp / 64);
     const bool one_round = !halves && tiles128 > 512 && tiles192 <= 448;
     if (block != 32 && tiles64 > 256 && !one_round)
@@ -2559,7 +2564,7 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
     // Up to one 64 x 64 tile per compute unit, the kernel that splits K inside the workgroup: 4 bits, 256 x 4096 x 4096 59 -> 53 us.
     const bool ksplit = tiles64 <= 256;
     // (a ring of four stages where a workgroup has its compute unit to itself measured the same as two: 57.6 against 57.8 us at 128 x 4096 x 4096)
-    const int wg_tiles = ksplit ? 4 : 4 * rw_tiles;
+    const int wg_tiles = ksplit ? 4 : 4 * (one_round ? 3 : rw_tiles);
     const dim3 grid((ntiles + wg_tiles - 1) / wg_tiles, Mp / 64);
 #define ROWS_LAUNCH(KERNEL_, THREADS_, LDS_)                                                                                                                        \
     do                                                                                                                                                             \
@@ -2592,7 +2597,7 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
     } while (0)
     if (!halves && ksplit)
         ROWS_KS(8, false);
-    else if (!halves) // (one_round: three tiles it is)
+    else if (!halves) // (one_round)
         ROWS_RW(8, false, 3);
     else if (bits == 8)
         ROWS(8);

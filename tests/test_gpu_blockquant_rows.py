@@ -194,10 +194,10 @@ def test_several_matrices_of_fp32_rows_get_the_bits_of_single_calls(rt, m, k, ns
 
 
 @pytest.mark.parametrize("m,n,k", [(1030, 1000, 16), (1100, 1000, 64), (1030, 970, 80), (523, 1960, 144), (65, 8250, 208), (1025, 1010, 320), (260, 3300, 1040), (1090, 960, 1568),
-                                   (2060, 2050, 80)])
+                                   (2060, 2050, 80), (2830, 1530, 144)])
 @pytest.mark.parametrize("bits,block", [(8, 64), (8, 128), (6, 64), (4, 128)])
 def test_fp32_rows_in_64x128_tiles(rt, m, n, k, bits, block):
-    """More than 256 tiles of 64 x 64 (in the last shape the plain layout takes 64 x 192 ones): row blocks and weight tiles cut off, K groups of no, one and several steps, the last of them ragged;
+    """More than 256 tiles of 64 x 64 (in the last two shapes the plain layout takes 64 x 192 ones): row blocks and weight tiles cut off, K groups of no, one and several steps, the last of them ragged;
     with input scales and C, rows off 16 bytes, an infinity and a NaN (no special value beyond its own row)."""
     print("[case]", m, n, k, bits, block, flush=True)
     a, packed, scales = synth.blockquant_operands(m + n + k, m, n, k, bits, block, half_exact=False)
