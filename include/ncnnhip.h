@@ -421,13 +421,14 @@ int ncnnhip_gemm_blockquant_packed(const float* a_dev, size_t a_stride, int M, i
 
 /* Several packed weight matrices on the SAME activation rows in one launch: the gate and up projections of a decoder layer, the
  * q / k / v projections of an attention layer -- in the reference one Gemm / MultiHeadAttention projection after the other
- * (src/layer/gemm.cpp:425-483 per matrix); the results are those of `count` calls of ncnnhip_gemm_blockquant_packed(_f16a), bit
- * for bit.  a_elemsize 2: fp16 activations; 4: fp32, with optional in_scales [K].
+ * (src/layer/gemm.cpp:425-483 per matrix); the results are those of `count` calls of ncnnhip_gemm_blockquant_packed(_f16a): bit
+ * for bit for fp32 rows and for up to 4 fp16 rows; more fp16 rows may have their fp32 additions in another order, since the
+ * kernel and its split of K follow from the size of the whole launch (as they do from N in single calls).
+ * a_elemsize 2: fp16 activations; 4: fp32, with optional in_scales [K].
  * All matrices share K, bits and block; N, the packed weights and descales, C (c_dev or its entries may be null), its broadcast
  * type, alpha, beta (null: 1) and the outputs are per matrix, count <= 8.  A decode-sized launch is paced by its ramp and tail,
- * not by bandwidth: one launch over 2 x 45.8 MB reaches what two launches of 45.8 MB cannot.  Matrix by matrix run: more than 16
- * fp32 rows; fp16 rows where the matrices alone would take different kernels, or cut K into different numbers of pieces; and what no
- * kernel takes whole. */
+ * not by bandwidth: one launch over 2 x 45.8 MB reaches what two launches of 45.8 MB cannot.  More than 16 fp32 rows, and what no kernel
+ * takes whole, run matrix by matrix. */
 int ncnnhip_gemm_blockquant_packed_multi(const void* a_dev, int a_elemsize, size_t a_stride, int M, int K, int count, const int* N,
                                          const uint8_t* const* packed_w_dev, const float* const* packed_descale_dev, int bits,
                                          int block, const float* in_scales_dev, const float* const* c_dev, const int* broadcast_type_c,

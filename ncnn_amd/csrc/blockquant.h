@@ -212,9 +212,8 @@ static inline bool halves_layout(int bits, int block)
 }
 
 // Many rows of fp16 activations (blockquant_rows.hip; many_rows_f16 in blockquant.hip says from how many: 17 always, 5 on large
-// weights): every matrix of mm on the same rows, one launch.  handled = false: one launch would not give every matrix the bits of a call
-// of its own (never so for one matrix).
-int launch_blockquant_rows_f16(const uint16_t* a, size_t a_stride, int M, int K, int bits, int block, const BqMulti& mm, bool* handled, hipStream_t stream);
+// weights): every matrix of mm on the same rows, one launch.
+int launch_blockquant_rows_f16(const uint16_t* a, size_t a_stride, int M, int K, int bits, int block, const BqMulti& mm, hipStream_t stream);
 
 // The same with fp32 rows (16-byte aligned) and optional input scales; and about how long that takes for `count` matrices of N[i] rows, with the shape
 // it will take.

@@ -2290,7 +2290,7 @@ int ncnnhip_blockquant_pack(const uint8_t* b_host, const float* scales_host, int
     return NCNNHIP_OK;
 }
 
-// fp16 rows: which of the two forms takes M rows of N x K weights.  The one-pass kernel holds a
+// fp16 rows: which of the two forms takes M rows of N x K weights (N: of all matrices of the launch).  The one-pass kernel holds a
 // workgroup's whole share of K in registers: the shortest start, nothing shared between tiles.  The many-row kernel reads the
 // activations once for up to six tiles.  Measured over N 2048 to 27648, K 1024 to 13824, 5 to 16 rows, us one-pass / many-row:
 // unpacked fields (4 and 6 bits) cross at 20 M weights -- 4352 x 4096 8.3 / 8.7, 5120 x 5120 10.8 / 10.2, 22016 x 4096 23.6 /
@@ -2349,11 +2349,8 @@ static int gemm_blockquant_packed(const char* who, const void* a_dev, int ain, s
     const int split = block == 32 ? 1 : 0;
     hipStream_t st = as_stream(stream);
     if (ain == 2 && many_rows_f16(M, N, K, bits, block))
-    {
-        bool handled; // (always)
         return launch_blockquant_rows_f16(static_cast<const uint16_t*>(a_dev), a_stride, M, K, bits, block,
-                                          one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride), &handled, st);
-    }
+                                          one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride), st);
     if (ain == 4 && many_rows_f32(M, K))
         return launch_blockquant_rows_f32(static_cast<const float*>(a_dev), a_stride, M, K, bits, block, in_scales_dev,
                                           one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride), st);
@@ -2671,17 +2668,7 @@ int ncnnhip_gemm_blockquant_packed_multi(const void* a_dev, int a_elemsize, size
         mm.tile_end[i] = (int)tiles, mm.N[i] = 0, mm.bt[i] = -1, mm.alpha[i] = mm.beta[i] = 1.f;
         mm.wpk[i] = 0, mm.dpk[i] = 0, mm.c[i] = 0, mm.out[i] = 0, mm.out_stride[i] = 0;
     }
-    // every matrix on the kernel that it would get alone, whose order of additions is its own
-    int many = 0;
-    for (int i = 0; i < count && one_pass && a_elemsize == 2; i++) many += many_rows_f16(M, N[i], K, bits, block);
-    if (many && many < count) one_pass = false;
-    if (one_pass && many)
-    {
-        bool handled = false;
-        const int ret = launch_blockquant_rows_f16(static_cast<const uint16_t*>(a_dev), a_stride, M, K, bits, block, mm, &handled, as_stream(stream));
-        if (ret != NCNNHIP_OK || handled) return ret;
-        one_pass = false;
-    }
+    if (one_pass && a_elemsize == 2 && many_rows_f16(M, tiles * 16, K, bits, block)) return launch_blockquant_rows_f16(static_cast<const uint16_t*>(a_dev), a_stride, M, K, bits, block, mm, as_stream(stream));
     if (one_pass && a_elemsize == 4 && many_rows_f32(M, K))
         return launch_blockquant_rows_f32(static_cast<const float*>(a_dev), a_stride, M, K, bits, block, in_scales_dev, mm, as_stream(stream));
     if (one_pass)

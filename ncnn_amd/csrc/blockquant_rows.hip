@@ -518,56 +518,28 @@ static int launch_one(const void* a, size_t a_stride, int M, int K, int passes, 
     return launch_status("blockquant_rows_kernel");
 }
 
-// Groups of activation rows and tiles per workgroup: the cheapest pair under 3.7 us + rounds x K / 4096 x (1.8 MG + 1.6 RT) us (one
-// workgroup per unit, 256 units).  As a forecast that is rough -- off by 13 % in the median and up to half over every pair of MG 1
-// to 4 and RT 1, 2, 3, 4, 6 at N and K 1024 to 27648, 24 to 128 rows, 4 and 8 bits, weights from HBM -- but it ranks well: what it
-// picks took 1 % more than the best pair in the median of those 120 launches, 10 % at most (24 rows of 5120 x 13824 at 4 bits 24.7
-// us with 2 x 2, 1 x 3 22.4; 100 rows of 1024 x 8192 12.1, 2 x 1 11.2).  48 rows of 11008 x 4096 get 3 x 3: 230 workgroups;
-// 3 x 2 are 344, a second round for 88 of them.  Several matrices are counted one by one, as no group has tiles of two: three of 4096 x
-// 4096 are 258 groups of three tiles, not 256, and get 3 x 4 (a decoder layer's seven matrices at 4 bits, 48 rows, 76.9 -> 68.2 us;
-// groups across matrices took 67.2 but cost every other launch up to a microsecond in looking them up).
-struct RowsShape
+int launch_blockquant_rows_f16(const uint16_t* a, size_t a_stride, int M, int K, int bits, int block, const BqMulti& mm, hipStream_t stream)
 {
-    int mg, rt, waves;
-};
-// waves: only pairs whose workgroups have that many wavefronts (0: any); there is one if a matrix of the launch got it
-static RowsShape rows_f16_shape(int M, int K, int bits, int split, const int* N, int count, int waves)
-{
-    const int rows16 = (M + 15) / 16, kblocks = (K + 63) / 64;
-    RowsShape shape = {0, 0, 0};
+    // Groups of activation rows and tiles per workgroup: the cheapest pair under 3.7 us + rounds x K / 4096 x (1.8 MG + 1.6 RT) us (one
+    // workgroup per unit, 256 units).  As a forecast that is rough -- off by 13 % in the median and up to half over every pair of MG 1
+    // to 4 and RT 1, 2, 3, 4, 6 at N and K 1024 to 27648, 24 to 128 rows, 4 and 8 bits, weights from HBM -- but it ranks well: what it
+    // picks took 1 % more than the best pair in the median of those 120 launches, 10 % at most (24 rows of 5120 x 13824 at 4 bits 24.7
+    // us with 2 x 2, 1 x 3 22.4; 100 rows of 1024 x 8192 12.1, 2 x 1 11.2).  48 rows of 11008 x 4096 get 3 x 3: 230 workgroups;
+    // 3 x 2 are 344, a second round for 88 of them.  Several matrices are counted one by one, as no group has tiles of two: three of 4096 x
+    // 4096 are 258 groups of three tiles, not 256, and get 3 x 4 (a decoder layer's seven matrices at 4 bits, 48 rows, 76.9 -> 68.2 us;
+    // groups across matrices took 67.2 but cost every other launch up to a microsecond in looking them up).
+    const int rows16 = (M + 15) / 16;
+    int mg = 4, rt = 4;
     double best = 0.0;
     for (int g = 1; g <= 4; g++)
         for (const int r : {1, 2, 3, 4, 6})
         {
-            const int fit = rows_waves(bits, g, r, split, 2), w = kblocks < fit ? kblocks : fit;
-            if (waves && w != waves) continue;
             long long wgs = 0;
-            for (int i = 0; i < count; i++) wgs += ((N[i] + 15) / 16 + r - 1) / r;
+            for (int i = 0; i < mm.count; i++) wgs += ((mm.N[i] + 15) / 16 + r - 1) / r; // no group has tiles of two matrices
             wgs *= (rows16 + g - 1) / g;
             const double cost = (double)((wgs + 255) / 256) * (1.8 * g + 1.6 * r);
-            if (best == 0.0 || cost < best) best = cost, shape = {g, r, w};
+            if (best == 0.0 || cost < best) best = cost, mg = g, rt = r;
         }
-    return shape;
-}
-
-int launch_blockquant_rows_f16(const uint16_t* a, size_t a_stride, int M, int K, int bits, int block, const BqMulti& mm, bool* handled, hipStream_t stream)
-{
-    const bool split = block == 32;
-    // Several matrices get the bits of calls of their own: the order of a sum follows from the number of wavefronts that share K, so the pair is
-    // picked among those with the number that each would get alone.  (The cheapest of all may be a larger one with fewer wavefronts, in one round
-    // instead of two; it is left: q, k, v, gate and up of 4096 x 11008, 64 rows at 4 bits 40.9 -> 47.4 us in two launches, 48 rows the same as
-    // before; at 8 bits 45.4 -> 53.8 and 40.2 -> 45.3.)
-    int waves = 0;
-    for (int i = 0; i < mm.count && mm.count > 1; i++)
-    {
-        const int alone = rows_f16_shape(M, K, bits, split, mm.N + i, 1, 0).waves;
-        *handled = i == 0 || alone == waves;
-        if (!*handled) return NCNNHIP_OK;
-        waves = alone;
-    }
-    *handled = true;
-    const RowsShape shape = rows_f16_shape(M, K, bits, split, mm.N, mm.count, waves);
-    const int mg = shape.mg, rt = shape.rt, rows16 = (M + 15) / 16;
     const int passes = (rows16 + mg - 1) / mg;
 #define ONE(BITS_, HALVES_, SPLIT_, MG_, RT_) return launch_one<BITS_, HALVES_, SPLIT_, MG_, RT_, 2>(a, a_stride, M, K, passes, nullptr, mm, stream)
 #define ONE_RT(BITS_, HALVES_, SPLIT_, MG_)              \
@@ -587,6 +559,7 @@ int launch_blockquant_rows_f16(const uint16_t* a, size_t a_stride, int M, int K,
         if (mg == 3) ONE_RT(BITS_, HALVES_, SPLIT_, 3); \
         ONE_RT(BITS_, HALVES_, SPLIT_, 4);        \
     } while (0)
+    const bool split = block == 32;
     if (!halves_layout(bits, block)) ONE_MG(8, false, 0);
     if (bits == 8) ONE_MG(8, true, 1); // blocks of 32 only
     if (bits == 6 && split) ONE_MG(6, true, 1);

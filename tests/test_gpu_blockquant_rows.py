@@ -239,21 +239,24 @@ def test_several_matrices_whose_groups_would_fill_the_units_only_together(rt):
 
 
 @pytest.mark.parametrize("m,k,ns,bits,block", [
-    # the cheapest shape for all matrices has fewer wavefronts than the one each matrix gets alone: 8 bits 8 and 7, 4 bits 8 and 7, 8 and 6
+    # the form of all matrices shares K out over fewer wavefronts than the one each matrix gets alone: 8 bits 8 and 7, 4 bits 8 and 7, 8 and 6
     (48, 528, (4096,) * 3, 8, 64), (64, 512, (4096,) * 3, 4, 64), (64, 592, (11008,) * 2, 4, 32), (48, 512, (11008,) * 2, 8, 64),
     # matrices that alone get different numbers of wavefronts
     (64, 512, (4096, 11008), 8, 64), (57, 512, (16, 4096, 17600), 4, 64),
-    # 5 to 16 rows: small weights go to another kernel than large ones, alone or not
-    (16, 4096, (4096,) * 2, 4, 64), (7, 4096, (4096,) * 2, 6, 32), (5, 4096, (4096, 8192), 4, 64), (16, 8208, (2000, 6000), 8, 64), (16, 4096, (4096, 7200), 8, 32), (9, 1040, (16400, 64), 8, 64)])
-def test_several_matrices_of_fp16_rows_get_the_bits_of_single_calls(rt, m, k, ns, bits, block):
-    """Where the number of wavefronts that share K, and with it the order of the sums, follows from the shape of the launch, and where
-    the kernel follows from the size of the weights."""
+    # 5 to 16 rows: small weights alone go to another kernel than all of them
+    (16, 4096, (4096,) * 2, 4, 64), (7, 4096, (4096,) * 2, 6, 32), (5, 4096, (4096, 8192), 4, 64), (16, 8208, (2000, 6000), 8, 64), (16, 4096, (4096, 7200), 8, 32), (9, 1040, (16400, 64), 8, 64),
+    # up to 4 rows the same bits whatever the sizes
+    (4, 4096, (4096,) * 3, 4, 64), (3, 8208, (2000, 18000), 8, 64), (1, 1040, (16400, 64), 6, 32), (2, 4112, (40, 11008), 8, 128)])
+def test_several_matrices_of_fp16_rows_beside_single_calls(rt, m, k, ns, bits, block):
+    """Where the size of the whole launch asks for another kernel, or another split of K, than that of one matrix: the results differ by
+    the order of the additions only, and not at all up to four rows."""
     print("[case]", m, k, ns, bits, block, flush=True)
-    rng = np.random.default_rng(m + k)
-    a = rng.normal(0, 1, (m, k)).astype(np.float16)
-    mats = []
-    for n in ns:
-        fields = rng.integers(0, 256, (n, k * bits // 8), dtype=np.uint8)
-        mats.append(rt.blockquant_pack(fields, rng.uniform(50, 100, (n, -(-k // block))).astype(F), block, bits=bits, k=k) + (n, None, -1, 1.0, 1.0))
-    for got, (pw, pd, n, *_) in zip(rt.gemm_blockquant_packed_multi(a, mats, bits=bits, block=block), mats):
-        assert np.array_equal(got, rt.gemm_blockquant_packed(a, pw, pd, n, bits=bits, block=block)), n
+    ops = [synth.blockquant_operands(40 + i, m, n, k, bits, block) for i, n in enumerate(ns)]
+    a = ops[0][0].astype(np.float16)
+    mats = [rt.blockquant_pack(p, s, block, bits=bits, k=k) + (n, None, -1, 1.0, 1.0) for (_, p, s), n in zip(ops, ns)]
+    for got, (pw, pd, n, *_), (_, packed, scales) in zip(rt.gemm_blockquant_packed_multi(a, mats, bits=bits, block=block), mats, ops):
+        single = rt.gemm_blockquant_packed(a, pw, pd, n, bits=bits, block=block)
+        val, floor = npref.blockquant_gemm_f64(a.astype(F), packed, scales, bits, block)
+        tol = 1e-5 * floor + 1e-30  # as _check
+        assert np.all(np.abs(got - val) <= tol) and np.all(np.abs(single - val) <= tol), n
+        assert m > 4 or np.array_equal(got, single), n

@@ -623,7 +623,8 @@ def test_blockquant_packed_fp32_activations(rt, bits, block, m, n, k, bt, in_sc)
     ("fp16", 8, 64, 20, 1024, (64, 48), False), ("fp32", 8, 64, 4, 8192, (32, 48), False)])
 def test_blockquant_packed_multi_equals_the_single_calls_and_the_oracle(rt, act, bits, block, m, k, ns, in_sc):
     """Several weight matrices on the same activation rows in one launch: each output is bit for bit what the single-matrix entry
-    gives (same kernel, same order of additions; the workgroup only finds its matrix differently), and within the usual bound of the
+    gives (same kernel, same order of additions; the workgroup only finds its matrix differently: always so for fp32 rows and up to four fp16
+    ones, and for more fp16 rows where, as here, one matrix and all of them ask for the same form), and within the usual bound of the
     oracle's Gemm::forward_weight_block_quantize (src/layer/gemm.cpp:425-483) per matrix -- with a different C, alpha and beta each."""
     _say("blockquant multi", act, bits, block, m, k, ns, in_sc)
     from ncnn_amd import synth
