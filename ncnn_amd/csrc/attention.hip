@@ -335,7 +335,12 @@ __device__ __forceinline__ void attention_merge_shares(const v16f_at (&o)[HD / 3
     constexpr int LD = 33;
     __shared__ float o_s[HD * LD];
     __shared__ float m_s[4][32], l_s[4][32];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hh = lane >> 5;
+    unsigned thread = threadIdx.x;
+    // Head dimension 96 has no register to spare: with what is made of the thread's number kept from before the loop it took 257 and one wavefront ran
+    // on a SIMD instead of two.  (us, 257 registers and 255: fp32 core, 27 heads, 28 queries on 1504 keys 44.3 38.0; split core, 22 heads, 1710 on
+    // 1731 284 210, 15 heads, 1862 on 3740 436 287.  The others have registers enough and are 2 to 4 % slower this way on short sequences.)
+    if constexpr (HD == 96) asm volatile("" : "+v"(thread));
+    const int tid = (int)thread, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hh = lane >> 5;
     if (hh == 0)
     {
         m_s[wave][l32] = m;
@@ -1176,9 +1181,10 @@ static bool attention_bf16x3_applies(int num_heads, int head_dim, int src, int d
     if (dst <= 32 && head_dim <= 64) return false;
     return blocks >= 8 || keys <= (width >= 256 ? 256 : 64) * width;
 }
-// Its workgroups run two to a CU up to head dimension 64, else one.  Units (32 queries of a head) that would leave half of these places
-// empty share their keys out over as many workgroups as there are places, at least 128 keys each.  (Rounding up as above, or sharing out
-// the last, partly filled of several rounds: 768 units at 1500 keys 82 us without, 88 with.)
+// Its workgroups run two to a CU up to head dimension 96, else one (at 96 counted as one: with twice the splits a few hundred keys took 15 % longer,
+// some thousands up to 20 % less).  Units (32 queries of a head) that would leave half of these places empty share their keys out over as many
+// workgroups as there are places, at least 128 keys each.  (Rounding up as above, or sharing out the last, partly filled of several
+// rounds: 768 units at 1500 keys 82 us without, 88 with.)
 static int attention_bf16x3_splits(int num_heads, int head_dim, int src, int dst, int& keys_per_split)
 {
     const long long units = (long long)((src + 31) / 32) * num_heads;
