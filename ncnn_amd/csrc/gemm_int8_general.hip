@@ -467,15 +467,19 @@ static inline bool rows_aligned16(const int8_t* p, size_t stride, int K)
 // x 512 5.2 -> 4.6, 281 x 720 x 2048 8.8 -> 4.6, 360 x 936 x 4672 13.9 -> 10.1, 551 x 1024 x 2048 9.0 -> 7.6, 1024 cubed 8.2 -> 6.8, 512 x
 // 2048 x 2048 11.1 -> 8.9; 256 x 4096 x 4096 17.3 -> 12.2 with 64 x 64 tiles and eight wavefronts; off 16 bytes 16 x 8000 x 8001 42 -> 17, 895 x
 // 456 x 473 6.5 -> 5.8; and where it is not taken: 1226 x 1344 x 2944 17.0 -> 18.0, 330 x 6616 x 896 10.2 -> 11.7, 2284 x 336 x 1216 7.4 ->
-// 7.9, off 16 bytes 148 x 3311 x 537 6.8 -> 7.8.  (From 640 to 1024 tiles it is better than the 128 x 128 tiles of whole multiples, not than
-// 64 x 64.)  Eight wavefronts a tile up to one tile a unit and from nine K steps (128 x 1024 x 4096 5.7, four 6.2), else four.
+// 7.9, off 16 bytes 148 x 3311 x 537 6.8 -> 7.8.  With a long K it is left from two cut tiles a unit on (22 shapes of 515 to 638 tiles, K 2944 to 7808: 5 %
+// less here in one, 3 to 35 % more in the others: 192 x 2960 x 4480 13.0 -> 17.6, 131 x 3848 x 6464 18.4 -> 24.1, 1369 x 440 x 3392 11.3 -> 13.4; at
+// 480 to 510 tiles from 26 % less to 14 % more; of whole multiples of 128 up to 14 % less, 5 % more at worst: 256 x 2304 x 6144 16.5 ->
+// 14.5).  (From 640 to 1024 tiles it is better than the 128 x 128 tiles of whole multiples, not than 64 x 64.)  Eight wavefronts a tile
+// up to one tile a unit and from nine K steps (128 x 1024 x 4096 5.7, four 6.2), else four.
 bool gemm_int8_streams(int M, int N, int K, bool aligned)
 {
     if (K < 16) return false;
     if (M <= 16) return true;
     const long long tiles32 = (long long)ceil_div(M, 32) * ceil_div(N, 32);
     if (!aligned) return tiles32 <= 450;
-    return tiles32 <= 640 || (tiles32 <= 1024 && M % 128 == 0 && N % 128 == 0);
+    if (M % 128 == 0 && N % 128 == 0) return tiles32 <= 1024;
+    return tiles32 <= (K >= 2944 ? 512 : 640);
 }
 
 template<typename Epilogue>

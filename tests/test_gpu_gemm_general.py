@@ -27,6 +27,8 @@ SHAPES = [
     (300, 900, 144), (260, 1000, 1039), (16, 9000, 48), (620, 1000, 528), (768, 1024, 80), (530, 1000, 3088), (896, 768, 3088),
     # beyond the streaming kernel (450 tiles of 32 x 32, 640 or 1024 where rows are aligned): one and two groups of wavefronts per tile of 64 x 64
     (700, 700, 65), (720, 650, 271), (1000, 700, 528), (470, 970, 3073), (465, 990, 3327),
+    # cut tiles of aligned rows leave the streaming kernel from 513 tiles and K = 2944 on: the last it keeps on either side, and the first it does not
+    (500, 1000, 2944), (520, 1000, 2928), (513, 1000, 2944),
     # 128 x 128 tiles from 1536 tiles of 64 x 64
     (2497, 2497, 33), (1, 5000, 50), (3000, 2176, 130),
 ]
