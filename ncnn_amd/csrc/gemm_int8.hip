@@ -196,10 +196,12 @@ int ncnnhip_gemm_int8(const int8_t* aq_dev, size_t aq_stride, const int8_t* bq_d
         // unit, and beyond while K is not long.  General kernel -> ring, us: 1153 x 592 x 1600, 50 tiles, 8.4 -> 11.8; 1617 x 1104 x 1280, 117,
         // 9.7 -> 11.4; 2364 x 1528 x 256, 228, 11.7 -> 12.3; 2268 x 1512 x 1152, 216, 14.1 -> 12.3; 4036 x 792 x 2240, 224, 22.5 -> 15.7; 867 x
         // 3648 x 7744, 203, 65 -> 45; 1858 x 5336 x 320, 630, 22.8 -> 17.5; 3458 x 2704 x 1664, 616, 36.3 -> 31.6; 2161 x 6512 x 2176, 867,
-        // 59 -> 61.
-        const long long tiles128 = (long long)ceil_div(M, 128) * ceil_div(N, 128);
+        // 59 -> 61.  Beyond one a unit only where the general kernel's 64 x 64 tiles are more than four a unit, one round: 19 shapes with fewer took 5 %
+        // less to 22 % more on the ring, 15 in the median (1046 x 3682 x 256, 261 and 986 tiles, 7.8 -> 9.4; 676 x 5464 x 1216, 258 and 946, 15.5 -> 18.3),
+        // 261 with more 10 % less in the median, 5 of them 4 to 11 % more.
+        const long long tiles128 = (long long)ceil_div(M, 128) * ceil_div(N, 128), tiles64 = (long long)ceil_div(M, 64) * ceil_div(N, 64);
         const bool whole = M % 128 == 0 && N % 128 == 0;
-        if (whole ? tiles128 >= 48 : tiles128 <= 256 ? tiles128 >= 200 && K >= 512 : K <= 2048)
+        if (whole ? tiles128 >= 48 : tiles128 <= 256 ? tiles128 >= 200 && K >= 512 : K <= 2048 && tiles64 > 1024)
         {
             ret = launch_gemm_int8_ring128(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, epi, as_stream(stream), &handled);
             if (handled) return ret;
