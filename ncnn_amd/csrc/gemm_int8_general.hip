@@ -461,7 +461,9 @@ static inline bool rows_aligned16(const int8_t* p, size_t stride, int K)
     return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && stride % 16 == 0 && K % 16 == 0;
 }
 
-// Where the streaming kernel is the quicker one.  Up to 16 rows always: it reads B once, at 5.5 TB/s where B is large.  Else by its tiles: it
+// Where the streaming kernel is the quicker one.  Up to 16 rows always: it reads B once, at 5.5 TB/s where B is large (one or two rows on few
+// columns with K beyond 5000 pay for its serial steps: 1 x 1656 x 8000 7.1 us, 6.1 with 16 columns a workgroup; sixteen wavefronts a tile instead
+// of eight took 1 to 13 % longer).  Else by its tiles: it
 // reads the operands of each 32 x 32 tile, four times the bytes a product that 128 x 128 tiles read, and rows off 16 bytes cost two cache
 // lines for one.  us, Gemm alone, the quickest other kernel here -> this one: 1 x 8192 x 8192 16.5 -> 12.0, 32 x 4096 x 4096 11.0 -> 5.8, 64 x 512
 // x 512 5.2 -> 4.6, 281 x 720 x 2048 8.8 -> 4.6, 360 x 936 x 4672 13.9 -> 10.1, 551 x 1024 x 2048 9.0 -> 7.6, 1024 cubed 8.2 -> 6.8, 512 x
