@@ -69,6 +69,12 @@ bool conv_resident_fits(const NhwcGeom& g, const ConvEpilogue& epi, const ConvFu
 int launch_conv_resident(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream);
 int launch_conv_pointwise(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, int out_cp, hipStream_t stream);
 
+// The kernel for few output tiles (conv_stream.hip: K split over the wavefronts of tiles of 16 x 16 to 32 x 32, no workspace): does this
+// problem belong to it (int8 blob), and its launch.  conv_patch_pays leaves such layers to it; the pipelined launch asks after the
+// pointwise and weights-resident kernels, which want many pixels.
+bool conv_stream_fits(const NhwcGeom& g, bool fp32_out);
+int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream);
+
 // InnerProduct as a 1x1 convolution over the activation rows (rows = pixels, K = channels): same epilogue as the
 // convolution (scale_in, bias, activation), dense fp32 output with row stride out_stride.  handled = false when the
 // shape does not fit (K % 64, num_output % 4, strides, alignment, workspace) and the caller should take another kernel.

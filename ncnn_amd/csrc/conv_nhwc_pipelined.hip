@@ -90,6 +90,7 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
 {
     if (conv_pointwise_fits(g_in, epi, fusion, out_cp) || conv_pointwise_stem_fits(g_in, epi, fusion, out_cp)) return launch_conv_pointwise(g_in, wpk, x, epi, out_cp, stream);
     if (conv_resident_fits(g_in, epi, fusion, out_cp)) return launch_conv_resident(g_in, wpk, x, epi, fusion, out_cp, stream);
+    if (conv_stream_fits(g_in, !epi.scale_out)) return launch_conv_stream(g_in, wpk, x, epi, fusion, out_cp, stream);
     NhwcGeom g = g_in;
     // A 1x1, stride-1, unpadded layer reads input pixel n for output pixel n, whatever the image shape: present it as
     // one row of npix pixels, and the kernel skips the pixel -> (image, y, x) divisions.

@@ -1,0 +1,76 @@
+"""The convolution kernel for few output tiles (tiles of 16 x 16, 16 x 32 and 32 x 32 pixels x channels, K split over a workgroup's
+wavefronts) against the oracle, bit for bit, at the edges of its tiles, of its K runs and of the rule that chooses it.
+Semantics: Convolution::forward_int8 (src/layer/convolution.cpp:383-508) per sample, batch as src/net.cpp:654-700."""
+import numpy as np
+import pytest
+
+from tests import cases
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+
+@pytest.fixture(scope="module")
+def rt():
+    import ncnn_amd
+    return ncnn_amd.Runtime(0)
+
+
+NONE, SAME3 = (0, 0, 0, 0), (1, 1, 1, 1)
+SHAPES = [
+    # batch, c, h, w, outc, kernel, dilation, stride, pads.  Tiles of 16 x 16:
+    (1, 64, 1, 1, 16, (1, 1), (1, 1), (1, 1), NONE),  # one pixel, one step: three wavefronts have none
+    (1, 16, 5, 3, 17, (1, 1), (1, 1), (1, 1), NONE),  # a quarter of a step, a channel tail of one
+    (2, 144, 7, 7, 40, (1, 1), (1, 1), (1, 1), NONE),  # the third step partly beyond the pixel
+    (1, 3200, 3, 3, 40, (1, 1), (1, 1), (1, 1), NONE),  # 50 steps: two rounds of twelve, the second one step
+    (1, 256, 14, 14, 256, (3, 3), (1, 1), (1, 1), SAME3),
+    (1, 512, 7, 7, 512, (3, 3), (1, 1), (1, 1), SAME3),  # 72 steps
+    (3, 128, 9, 5, 33, (3, 3), (2, 2), (1, 1), (2, 2, 2, 2)),
+    (2, 192, 11, 9, 24, (1, 3), (1, 1), (2, 1), (0, 0, 1, 1)),  # a tap of three steps, uneven strides
+    (1, 64, 64, 64, 16, (1, 1), (1, 1), (1, 1), NONE),  # 256 tiles
+    # 16 x 32
+    (1, 64, 64, 64, 17, (1, 1), (1, 1), (1, 1), NONE),
+    (1, 128, 28, 28, 128, (3, 3), (1, 1), (1, 1), SAME3),
+    (1, 1024, 14, 14, 512, (1, 1), (1, 1), (2, 2), NONE),
+    (1, 512, 7, 7, 2000, (1, 1), (1, 1), (1, 1), NONE),
+    # 32 x 32, and what the other kernels keep: four steps and fewer to int8, more than 48 steps, 257 tiles
+    (1, 96, 63, 64, 60, (1, 1), (1, 1), (1, 1), NONE),
+    (1, 320, 63, 64, 60, (1, 1), (1, 1), (1, 1), NONE),
+    (4, 256, 14, 14, 256, (3, 3), (1, 1), (1, 1), SAME3),
+    (5, 512, 7, 8, 512, (3, 3), (1, 1), (1, 1), SAME3),
+    (1, 320, 8, 1028, 30, (1, 1), (1, 1), (1, 1), NONE),
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_few_tiles_kernel_matches_oracle(rt, shape):
+    batch, c, h, w, outc, kernel, dilation, stride, pads = shape
+    print("[case] conv few tiles", shape, flush=True)
+    for term, act, ap, bias in [(2, 1, (0.0, 0.0), True), (102, 3, (0.0, 6.0), False), (2, 2, (0.1, 0.0), False), (102, 0, (0.0, 0.0), True)]:
+        x, wq, b, ws, ins, tops = cases.conv_case(c + outc + term, c, h, w, outc, kernel, 1, term, bias, True, batch=batch)
+        d = oracle.make_desc((c, h, w), outc, kernel, dilation, stride, pads, 0.0, int(bias), 1, term, act, ap)
+        want = np.stack([oracle.convolution_int8(d, x[i], wq, b, ws, ins[0], None if tops is None else tops[0]) for i in range(batch)])
+        got = rt.conv_channels_last(x, wq, b if bias else None, ws, ins, tops, outc, kernel, dilation, stride, pads, 0.0, 1, term, act, ap)
+        assert got.dtype == want.dtype and np.array_equal(got, want), (term, act)
+
+
+@pytest.mark.parametrize("batch,c,hw,outc,kernel,pads,relu", [(1, 64, 5, 40, (1, 1), NONE, True), (1, 256, 14, 200, (3, 3), SAME3, False),
+                                                              (1, 128, 28, 140, (1, 1), NONE, True), (1, 128, 63, 60, (1, 1), NONE, False)])
+def test_few_tiles_kernel_fused_tail(rt, batch, c, hw, outc, kernel, pads, relu):
+    """Residual, ReLU layer and the quantised copy for the next convolution, on each tile; a NaN of the residual stays."""
+    print("[case] conv few tiles, fused tail", c, hw, outc, kernel, relu, flush=True)
+    x, wq, b, ws, ins, _ = cases.conv_case(c + outc, c, hw, hw, outc, kernel, 1, 2, True, True, batch=batch)
+    d = oracle.make_desc((c, hw, hw), outc, kernel, (1, 1), (1, 1), pads, 0.0, 1, 1, 2, 0, (0.0, 0.0))
+    conv = np.stack([oracle.convolution_int8(d, x[i], wq, b, ws, ins[0], None) for i in range(batch)])
+    res = np.random.default_rng(c).normal(0, 1, conv.shape).astype(F)
+    want = (conv + res).astype(F)
+    if relu:
+        want = np.maximum(want, 0)
+    scale = F(127) / np.abs(want).max()
+    res.reshape(-1)[-1] = np.nan
+    want.reshape(-1)[-1] = np.nan
+    want_q = oracle.quantize(want.reshape(batch * outc, -1), [scale]).reshape(want.shape)
+    got, got_q = rt.conv_channels_last(x, wq, b, ws, ins, None, outc, kernel, (1, 1), (1, 1), pads, 0.0, 1, 2, 0, (0.0, 0.0), residual=res, relu_after=relu,
+                                       quantise_scale=scale)
+    assert np.array_equal(got, want, equal_nan=True) and np.array_equal(got_q, want_q)
