@@ -183,6 +183,26 @@ int ncnnhip_conv_int8_nhwc_fused(const ncnnhip_conv_desc* desc, const int8_t* nh
                                  const float* scale_in_dev, const float* bias_dev, ncnnhip_activation act, float* out_dev,
                                  const ncnnhip_conv_fusion* fusion, void* workspace_dev, size_t workspace_bytes, void* stream);
 
+/* ncnnhip_conv_int8_nhwc_fused with two more choices for the end of a residual block, results unchanged:
+ *   shortcut (or NULL)  the residual is itself a 1x1 convolution of this output's shape, any stride (its own Convolution::forward_int8,
+ *                       src/layer/convolution.cpp:383-508): computed in the same launch, its fp32 blob is never written.  For
+ *                       pairs that ncnnhip_conv_shortcut_supported accepts; fusion->residual_dev must be NULL then.
+ *   out_dev NULL        only the quantised copy is written (every consumer reads that). */
+typedef struct ncnnhip_conv_shortcut
+{
+    const ncnnhip_conv_desc* desc;
+    const int8_t* nhwc_dev;
+    const int8_t* packed_weight_dev;
+    const float* scale_in_dev;
+    const float* bias_dev; /* or NULL */
+    ncnnhip_activation act;
+} ncnnhip_conv_shortcut;
+int ncnnhip_conv_shortcut_supported(const ncnnhip_conv_desc* desc, const ncnnhip_conv_desc* shortcut, int* supported);
+int ncnnhip_conv_int8_nhwc_tail(const ncnnhip_conv_desc* desc, const int8_t* nhwc_dev, const int8_t* packed_weight_dev,
+                                const float* scale_in_dev, const float* bias_dev, ncnnhip_activation act,
+                                const ncnnhip_conv_shortcut* shortcut, float* out_dev, const ncnnhip_conv_fusion* fusion,
+                                void* workspace_dev, size_t workspace_bytes, void* stream);
+
 /* The same convolution in ONE launch for an input blob that is still fp32 (elemsize 4) or fp16 (2), channels-last: the
  * layer's own Quantize pass (Quantize::forward, src/layer/quantize.cpp:48-111 as Convolution::forward_int8 calls it at
  * src/layer/convolution.cpp:392-405: q = float2int8(x * in_scale[0])) runs inside the kernel's loader, so the int8 copy of

@@ -32,6 +32,30 @@ struct ConvFusion
     float q8_scale;
 };
 
+// A second 1x1 convolution of the output's shape whose fp32 result is added (the projection shortcut of a residual block): unpadded, any
+// stride, channels in whole 64-byte steps.
+struct ConvShortcut
+{
+    const int8_t* wpk;
+    const int8_t* x;
+    int H, W, Cp; // its input; K = Cp
+    int sh, sw;
+    int outw, outh;
+    const float* scale_in;
+    const float* bias;
+    ncnnhip_activation act;
+};
+
+// the kernels' argument: nothing where there is no shortcut
+template<bool PRESENT>
+struct ConvShortcutArg
+{
+};
+template<>
+struct ConvShortcutArg<true> : ConvShortcut
+{
+};
+
 // Workspace contract of the channels-last convolutions: the first SPLIT_COUNTER_BYTES hold one arrival counter per
 // output tile of a K-split launch.  They must be zero when a call starts (the caller clears the workspace once, after
 // allocating it) and are zero again when it has finished; the rest is scratch without a contract.
@@ -74,6 +98,12 @@ int launch_conv_pointwise(const NhwcGeom& g, const int8_t* wpk, const int8_t* x,
 // pointwise and weights-resident kernels, which want many pixels.
 bool conv_stream_fits(const NhwcGeom& g, bool fp32_out);
 int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream);
+
+// The same two kernels with a projection shortcut (g: the main 1x1 convolution, stride 1, unpadded, channels in whole steps).
+int launch_conv_shortcut(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
+                         hipStream_t stream);
+int launch_conv_stream_shortcut(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion,
+                                int out_cp, hipStream_t stream);
 
 // InnerProduct as a 1x1 convolution over the activation rows (rows = pixels, K = channels): same epilogue as the
 // convolution (scale_in, bias, activation), dense fp32 output with row stride out_stride.  handled = false when the

@@ -585,7 +585,7 @@ static int conv_int8_nhwc_impl(const ncnnhip_conv_desc* desc, const void* nhwc_d
                                const float* scale_in_dev, const float* bias_dev, const float* scale_out_dev, ncnnhip_activation act, void* out_dev, int out_layout,
                                size_t out_cstep, size_t out_nstep, const ConvFusion& fusion, void* workspace_dev, size_t workspace_bytes, void* stream)
 {
-    NCNNHIP_REQUIRE(desc && nhwc_dev && packed_weight_dev && scale_in_dev && out_dev, "ncnnhip_conv_int8_nhwc: null pointer");
+    NCNNHIP_REQUIRE(desc && nhwc_dev && packed_weight_dev && scale_in_dev && (out_dev || fusion.q8_out), "ncnnhip_conv_int8_nhwc: null pointer");
     NCNNHIP_REQUIRE(desc->group == 1, "ncnnhip_conv_int8_nhwc: group must be 1");
     int outw, outh;
     int ret = ncnnhip_conv_out_shape(desc, &outw, &outh);
@@ -615,7 +615,8 @@ static int conv_int8_nhwc_impl(const ncnnhip_conv_desc* desc, const void* nhwc_d
     epi.acc_out = 0;
 
     hipStream_t st = as_stream(stream);
-    if (clast && pb == 0 && conv_patch_pays(g, d.batch, x_elemsize))
+    // (the small-tile and the weights-resident kernel always write the fp32 blob)
+    if (clast && pb == 0 && out_dev && conv_patch_pays(g, d.batch, x_elemsize))
         return launch_conv_patch(g, packed_weight_dev, nhwc_dev, x_elemsize, x_scale_dev, epi, fusion, out_cp, st);
     if (x_elemsize != 1)
     {
@@ -684,7 +685,7 @@ int ncnnhip_conv_int8_nhwc_fused(const ncnnhip_conv_desc* desc, const int8_t* nh
                                  const float* bias_dev, ncnnhip_activation act, float* out_dev, const ncnnhip_conv_fusion* fusion, void* workspace_dev,
                                  size_t workspace_bytes, void* stream)
 {
-    NCNNHIP_REQUIRE(fusion, "ncnnhip_conv_int8_nhwc_fused: null fusion");
+    NCNNHIP_REQUIRE(fusion && out_dev, "ncnnhip_conv_int8_nhwc_fused: null pointer");
     NCNNHIP_REQUIRE(ncnnhip_conv_fusion_supported(desc), "ncnnhip_conv_int8_nhwc_fused: needs group 1 and a zero border value");
     NCNNHIP_REQUIRE(!fusion->quantised_out_dev || fusion->quantise_scale != 0.f, "ncnnhip_conv_int8_nhwc_fused: quantised copy without a scale");
     ConvFusion f;
@@ -694,6 +695,75 @@ int ncnnhip_conv_int8_nhwc_fused(const ncnnhip_conv_desc* desc, const int8_t* nh
     f.q8_scale = fusion->quantise_scale;
     return conv_int8_nhwc_impl(desc, nhwc_dev, 1, 0, packed_weight_dev, scale_in_dev, bias_dev, 0, act, out_dev, NCNNHIP_CHANNELS_LAST, 0, 0, f, workspace_dev,
                                workspace_bytes, stream);
+}
+
+// 1x1, unpadded, zero border value, channels that fill whole 64-byte steps: what both convolutions of ncnnhip_conv_int8_nhwc_tail have to be
+static bool shortcut_operand(const ncnnhip_conv_desc* d, int* outw, int* outh)
+{
+    if (!ncnnhip_conv_fusion_supported(d) || d->kernel_w != 1 || d->kernel_h != 1 || padded_channels(d->c) % 64 != 0) return false;
+    if (d->pad_left > 0 || d->pad_right > 0 || d->pad_top > 0 || d->pad_bottom > 0) return false;
+    if (ncnnhip_conv_out_shape(d, outw, outh) != 0) return false;
+    const NhwcGeom g = nhwc_geometry(*d, *outw, *outh, (long long)*outw * *outh * d->batch);
+    if (g.pad_top != 0 || g.pad_left != 0 || (*outh - 1) * g.sh >= g.H || (*outw - 1) * g.sw >= g.W) return false; // (a SAME padding may add a border)
+    return (long long)*outw * *outh * d->batch < (1ll << 31) && (long long)d->h * d->w * padded_channels(d->c) < (1ll << 31);
+}
+
+static bool shortcut_supported(const ncnnhip_conv_desc& d, const ncnnhip_conv_desc& shortcut)
+{
+    int ow = 0, oh = 0, sow = 0, soh = 0;
+    return shortcut_operand(&d, &ow, &oh) && shortcut_operand(&shortcut, &sow, &soh) && d.stride_w == 1 && d.stride_h == 1 && ow == sow && oh == soh
+           && d.batch == shortcut.batch && d.num_output == shortcut.num_output;
+}
+
+int ncnnhip_conv_shortcut_supported(const ncnnhip_conv_desc* desc, const ncnnhip_conv_desc* shortcut, int* supported)
+{
+    NCNNHIP_REQUIRE(desc && shortcut && supported, "ncnnhip_conv_shortcut_supported: null pointer");
+    *supported = shortcut_supported(*desc, *shortcut) ? 1 : 0;
+    return NCNNHIP_OK;
+}
+
+int ncnnhip_conv_int8_nhwc_tail(const ncnnhip_conv_desc* desc, const int8_t* nhwc_dev, const int8_t* packed_weight_dev, const float* scale_in_dev,
+                                const float* bias_dev, ncnnhip_activation act, const ncnnhip_conv_shortcut* shortcut, float* out_dev,
+                                const ncnnhip_conv_fusion* fusion, void* workspace_dev, size_t workspace_bytes, void* stream)
+{
+    const char* who = "ncnnhip_conv_int8_nhwc_tail";
+    NCNNHIP_REQUIRE(desc && nhwc_dev && packed_weight_dev && scale_in_dev && fusion, "%s: null pointer", who);
+    NCNNHIP_REQUIRE(out_dev || fusion->quantised_out_dev, "%s: no output", who);
+    NCNNHIP_REQUIRE(!fusion->quantised_out_dev || fusion->quantise_scale != 0.f, "%s: quantised copy without a scale", who);
+    NCNNHIP_REQUIRE(ncnnhip_conv_fusion_supported(desc), "%s: needs group 1 and a zero border value", who);
+    const ConvFusion f = {fusion->residual_dev, fusion->relu_after, fusion->quantised_out_dev, fusion->quantise_scale};
+    if (!shortcut)
+        return conv_int8_nhwc_impl(desc, nhwc_dev, 1, 0, packed_weight_dev, scale_in_dev, bias_dev, 0, act, out_dev, NCNNHIP_CHANNELS_LAST, 0, 0, f, workspace_dev,
+                                   workspace_bytes, stream);
+    NCNNHIP_REQUIRE(shortcut->desc && shortcut->nhwc_dev && shortcut->packed_weight_dev && shortcut->scale_in_dev, "%s: null pointer in the shortcut", who);
+    NCNNHIP_REQUIRE(!fusion->residual_dev, "%s: a residual blob or a shortcut, not both", who);
+    NCNNHIP_REQUIRE(shortcut_supported(*desc, *shortcut->desc), "%s: the two convolutions must be 1x1, unpadded, of one output shape, the first with stride 1", who);
+    int outw = 0, outh = 0;
+    const int ret = ncnnhip_conv_out_shape(desc, &outw, &outh);
+    if (ret) return ret;
+    const NhwcGeom g = nhwc_geometry(*desc, outw, outh, (long long)outw * outh * desc->batch);
+    ConvShortcut sc;
+    sc.wpk = shortcut->packed_weight_dev;
+    sc.x = shortcut->nhwc_dev;
+    sc.H = shortcut->desc->h;
+    sc.W = shortcut->desc->w;
+    sc.Cp = padded_channels(shortcut->desc->c);
+    sc.sh = shortcut->desc->stride_h;
+    sc.sw = shortcut->desc->stride_w;
+    sc.outw = outw;
+    sc.outh = outh;
+    sc.scale_in = shortcut->scale_in_dev;
+    sc.bias = shortcut->bias_dev;
+    sc.act = shortcut->act;
+    ConvEpilogue epi = {};
+    epi.scale_in = scale_in_dev;
+    epi.bias = bias_dev;
+    epi.act = act;
+    epi.out = out_dev;
+    epi.pix_per_img = outw * outh;
+    epi.batch = desc->batch;
+    epi.num_output = desc->num_output;
+    return launch_conv_shortcut(g, packed_weight_dev, nhwc_dev, sc, epi, f, padded_channels(desc->num_output), as_stream(stream));
 }
 
 int ncnnhip_conv_from_float_supported(const ncnnhip_conv_desc* desc)
@@ -735,6 +805,7 @@ int ncnnhip_conv_int8_nhwc_from_float(const ncnnhip_conv_desc* desc, const void*
                                       ncnnhip_activation act, void* out_dev, const ncnnhip_conv_fusion* fusion, void* workspace_dev, size_t workspace_bytes,
                                       void* stream)
 {
+    NCNNHIP_REQUIRE(out_dev, "ncnnhip_conv_int8_nhwc_from_float: null pointer");
     NCNNHIP_REQUIRE(elemsize == 4 || elemsize == 2, "ncnnhip_conv_int8_nhwc_from_float: activations are fp32 (4) or fp16 (2), not %d bytes", elemsize);
     NCNNHIP_REQUIRE(ncnnhip_conv_from_float_supported(desc), "ncnnhip_conv_int8_nhwc_from_float: this layer needs its separate Quantize pass");
     NCNNHIP_REQUIRE((reinterpret_cast<uintptr_t>(nhwc_dev) & 15) == 0, "ncnnhip_conv_int8_nhwc_from_float: the blob must be 16-byte aligned");

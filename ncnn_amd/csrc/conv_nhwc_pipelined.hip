@@ -126,7 +126,7 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
     if (p.splits > 1) return launch_pipe_split(p, mode, wpk, x, g, epi, fusion, out_cp, out_cp, partial, counters, stream);
 #define LAUNCH_PIPE_MODE(BM_, BN_, MODE_, GROUPS_)                                                                                                                 \
     hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<BM_, BN_, PIPE_RING, false, MODE_, 1, GROUPS_>), grid, block, 0, stream, wpk, x, g, epi, fusion, out_cp, \
-                       out_cp, p.tiles_m, p.tiles_n, p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, (const float*)0, 0)
+                       out_cp, p.tiles_m, p.tiles_n, p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, (const float*)0, 0, ConvShortcutArg<false>())
 #define LAUNCH_PIPE(BM_, BN_)                  \
     do                                         \
     {                                          \
@@ -207,7 +207,7 @@ int launch_fc_via_conv_pipelined(const int8_t* x, size_t x_stride, int rows, int
     if (p.splits > 1) return launch_pipe_split(p, 1, weight, x, g, epi, no_fusion, (int)out_stride, num_output, partial, counters, stream);
 #define LAUNCH_FC(BN_, GROUPS_)                                                                                                                                \
     hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<64, BN_, PIPE_RING, false, 1, 1, GROUPS_>), grid, block, 0, stream, weight, x, g, epi, no_fusion, \
-                       (int)out_stride, num_output, p.tiles_m, p.tiles_n, p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, (const float*)0, 0)
+                       (int)out_stride, num_output, p.tiles_m, p.tiles_n, p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, (const float*)0, 0, ConvShortcutArg<false>())
     if (p.bn == 256)
         LAUNCH_FC(256, 1);
     else if (p.bn == 128)

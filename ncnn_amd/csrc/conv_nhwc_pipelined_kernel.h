@@ -66,6 +66,9 @@ __device__ __forceinline__ uint32_t pack4(const v4f& v)
 // A template parameter because the choice sits inside the K loop: as run-time branches there it cost the 3x3 layers
 // of ResNet-50's last stages 2-4 us each (15.4 against 11.4 us for 256 -> 256 on 14 x 14, batch 16).
 //
+// 4: dense, with a projection shortcut (ConvShortcut): the K steps of the shortcut's convolution come first, through the same ring; then its
+// accumulators are finished to fp32 and kept in registers while the main convolution's steps run, and added to its results.
+//
 // AIN: bytes per activation value.  1: the blob is int8 and goes global -> LDS directly, as described above.  4 (fp32)
 // or 2 (fp16): the layer's Quantize pass happens here (Quantize::forward, src/layer/quantize.cpp:48-111, one scale):
 // before the K loop the workgroup gathers its BM pixels x K im2col tile through registers, float2int8(value * scale)
@@ -81,12 +84,14 @@ __device__ __forceinline__ uint32_t pack4(const v4f& v)
 template<int BM, int BN, int STAGES, bool SPLITK, int MODE, int AIN = 1, int GROUPS = 1>
 __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const int8_t* __restrict__ wpk, const int8_t* __restrict__ x, NhwcGeom g, ConvEpilogue epi,
                                                                    ConvFusion fusion, int out_cp, int col_limit, int tiles_m, int tiles_n, int splits, int steps_per_split, unsigned magic_n, int32_t* __restrict__ partial, unsigned* __restrict__ counters,
-                                                                   const float* __restrict__ a_scale, int a_cache_bytes)
+                                                                   const float* __restrict__ a_scale, int a_cache_bytes, ConvShortcutArg<MODE == 4> shortcut)
 {
-    constexpr bool dense = MODE == 1;
+    constexpr bool SHORTCUT = MODE == 4;
+    constexpr bool dense = MODE == 1 || SHORTCUT;
     constexpr bool STAGED = AIN != 1;
     static_assert(GROUPS == 1 || (!STAGED && BM == 64 && BN == 64 && GROUPS == 4), "several groups of wavefronts: 64 x 64 tiles of an int8 blob");
-    static_assert(!STAGED || (MODE != 2 && MODE != 3), "the quantising loader exists for convolutions on ordinary blobs");
+    static_assert(!SHORTCUT || (GROUPS == 1 && !SPLITK), "a shortcut is finished by the wavefront that finishes the sum");
+    static_assert(!STAGED || (MODE != 2 && MODE != 3 && MODE != 4), "the quantising loader exists for convolutions on ordinary blobs");
     constexpr int TM = BM / 64, TN = BN / 64; // 32x32 blocks per wavefront along pixels / channels
     constexpr int LAR = BM / 64;              // 64-row groups of the activation tile
     constexpr int LA = STAGED ? 0 : LAR, LB = BN / 64; // direct-to-LDS loads per wavefront per stage
@@ -119,7 +124,9 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
     const int tm = rest - split * tiles_m;
     const int row0 = tm * BM, col0 = tn * BN;
 
-    const int total_steps = g.K / 64;
+    int shortcut_steps = 0;
+    if constexpr (SHORTCUT) shortcut_steps = shortcut.Cp / 64;
+    const int total_steps = g.K / 64 + shortcut_steps;
     int step_begin = SPLITK ? split * steps_per_split : 0;
     int step_end = SPLITK ? step_begin + steps_per_split : total_steps;
     if (step_end > total_steps) step_end = total_steps;
@@ -186,6 +193,25 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
         if (ch >= g.cout) ch = g.cout - 1; // a valid row; its products land in columns nobody stores
         b_ptr[i] = wpk + (size_t)ch * g.K + (size_t)step_begin * 64 + ld_chunk * 16;
     }
+    const int8_t* sa_ptr[LAR]; // the shortcut's: this lane's chunk of its pixel ...
+    const int8_t* sb_ptr[LB];  // ... and of its channel
+    if constexpr (SHORTCUT)
+    {
+#pragma unroll
+        for (int i = 0; i < LAR; i++)
+        {
+            const int n = row0 + i * 64 + ld_row, nn = n < g.npix ? n : g.npix - 1, plane = shortcut.outw * shortcut.outh;
+            const int img = g.npix < (1 << 20) ? small_div(nn, plane) : nn / plane, rem = nn - img * plane;
+            const int oy = g.npix < (1 << 20) ? small_div(rem, shortcut.outw) : rem / shortcut.outw, ox = rem - oy * shortcut.outw;
+            sa_ptr[i] = shortcut.x + (((size_t)img * shortcut.H + oy * shortcut.sh) * shortcut.W + ox * shortcut.sw) * shortcut.Cp + ld_chunk * 16;
+        }
+#pragma unroll
+        for (int i = 0; i < LB; i++)
+        {
+            const int ch = col0 + i * 64 + ld_row;
+            sb_ptr[i] = shortcut.wpk + (size_t)(ch < g.cout ? ch : g.cout - 1) * shortcut.Cp + ld_chunk * 16;
+        }
+    }
     // this lane's position in K: tap (ky,kx) and first channel q0 of its 16-byte chunk; +64 bytes per stage issued
     int q0, ky, kx, tap;
     {
@@ -241,6 +267,20 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
         // quantising loader: every step has its own place (written once); the address below is that place minus the
         // activation part a ring stage would start with
         int8_t* stage = STAGED ? a_tile + tile_steps * (BM * 64) + s * (BN * 64) - BM * 64 + wave * 1024 : smem + group * RING_BYTES + (s % STAGES) * STAGE_BYTES + wave * 1024;
+        if constexpr (SHORTCUT)
+        {
+            if (s < shortcut_steps) // (uniform)
+            {
+#pragma unroll
+                for (int i = 0; i < LA; i++)
+                    __builtin_amdgcn_global_load_lds((const AS1 void*)(sa_ptr[i] + (size_t)s * 64), (AS3 void*)(stage + i * 4096), 16, 0, 0);
+#pragma unroll
+                for (int i = 0; i < LB; i++)
+                    __builtin_amdgcn_global_load_lds((const AS1 void*)(sb_ptr[i] + (size_t)s * 64), (AS3 void*)(stage + BM * 64 + i * 4096), 16, 0, 0);
+                return;
+            }
+            s -= shortcut_steps;
+        }
         if (dense)
         {
             // one tap, no border: the row's pixel exists or it does not (a_iy0 is 0 or hugely negative)
@@ -291,7 +331,7 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
         for (int i = 0; i < LB; i++)
             __builtin_amdgcn_global_load_lds((const AS1 void*)(b_ptr[i] + (size_t)s * 64), (AS3 void*)(stage + BM * 64 + i * 4096), 16, 0, 0);
         // the lane's K position moves on by 64 bytes
-        if (MODE == 1)
+        if (dense)
         {
             q0 += 64;
             if (q0 >= g.tapK) tap = 1; // past the only tap: the rest of K is the round-up, zero-filled
@@ -354,6 +394,19 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
     // sum of its latencies).  Only the raw loads happen here, from clamped indices and always-valid pointers: a select
     // or a branch on the values would make the wavefront wait for them on the spot.
     float raw_s_in[BN / 64], raw_bias[BN / 64], raw_s_out[BN / 64];
+    float raw_sc_in[BN / 64], raw_sc_bias[BN / 64];
+    if constexpr (SHORTCUT)
+    {
+        const float* bias_src = shortcut.bias ? shortcut.bias : shortcut.scale_in;
+#pragma unroll
+        for (int c = 0; c < BN / 64; c++)
+        {
+            int ch = col0 + wn * (BN / 2) + c * 32 + l32;
+            if (ch >= g.cout) ch = g.cout - 1;
+            raw_sc_in[c] = shortcut.scale_in[ch];
+            raw_sc_bias[c] = bias_src[ch];
+        }
+    }
     {
         const float* bias_src = epi.bias ? epi.bias : epi.scale_in;
         const float* s_out_src = epi.scale_out ? epi.scale_out : epi.scale_in;
@@ -678,6 +731,7 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
         __builtin_amdgcn_s_barrier();
     }
 
+    float added[SHORTCUT ? TM : 1][SHORTCUT ? TN : 1][16]; // the shortcut's results
     for (int t = 0; t < iterations; t++)
     {
         if (GROUPS > 1 && t >= nk) // a group with fewer steps than the others: the barrier only (uniform)
@@ -734,6 +788,26 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
             for (int a = 0; a < TM; a++)
 #pragma unroll
                 for (int c = 0; c < TN; c++) acc[a][c] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[ks][a], fb[ks][c], acc[a][c], 0, 0, 0);
+        if constexpr (SHORTCUT)
+            if (t + 1 == shortcut_steps) // (uniform) the shortcut's sums are complete: its epilogue, in registers
+            {
+#pragma unroll
+                for (int c = 0; c < TN; c++)
+                {
+                    const bool exists = col0 + wn * (BN / 2) + c * 32 + l32 < g.cout;
+                    const float scale = exists ? raw_sc_in[c] : 0.f, addend = (exists && shortcut.bias) ? raw_sc_bias[c] : -0.f;
+#pragma unroll
+                    for (int a = 0; a < TM; a++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++)
+                        {
+                            float f = add_rn(mul_rn((float)acc[a][c][r], scale), addend);
+                            if (shortcut.act.type != 0) f = exists ? apply_activation(f, shortcut.act) : 0.f;
+                            added[a][c][r] = f;
+                            acc[a][c][r] = 0;
+                        }
+                }
+            }
     }
 
     // what this lane finishes: its accumulators, or with several groups of wavefronts its share of their sum
@@ -900,6 +974,7 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
                 for (int r = 0; r < NR; r++)
                 {
                     if (clear_pads && !real[c]) fr[r] = 0.f;
+                    if constexpr (SHORTCUT) fr[r] = add_rn(fr[r], added[a][c][r]);
                     tile[(8 * (r >> 2) + 4 * lhi + (r & 3)) * LD + c * 32 + l32] = fr[r];
                 }
             }
@@ -956,7 +1031,7 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
 #pragma unroll
                             for (int e = 0; e < 4; e++) v[e] = v[e] < 0.f ? 0.f : v[e]; // the ReLU LAYER's statement (src/layer/relu.cpp:36-37): a NaN stays, unlike fmaxf
                         }
-                        *reinterpret_cast<v4f*>(static_cast<float*>(epi.out) + o) = v;
+                        if (epi.out) *reinterpret_cast<v4f*>(static_cast<float*>(epi.out) + o) = v;
                         if (fusion.q8_out)
                         {
                             v4f q;

@@ -11,7 +11,7 @@ int launch_pipe_split(const PipePlan& p, int mode, const int8_t* wpk, const int8
     dim3 grid((unsigned)((long long)p.tiles_m * p.tiles_n * p.splits)), block((unsigned)(256 * p.groups));
 #define LAUNCH_SPLIT_MODE(BM_, BN_, MODE_, GROUPS_)                                                                                                              \
     hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<BM_, BN_, PIPE_RING, true, MODE_, 1, GROUPS_>), grid, block, 0, stream, wpk, x, g, epi, fusion, out_cp, \
-                       col_limit, p.tiles_m, p.tiles_n, p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, (const float*)0, 0)
+                       col_limit, p.tiles_m, p.tiles_n, p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, (const float*)0, 0, ConvShortcutArg<false>())
 #define LAUNCH_SPLIT(BM_, BN_, GROUPS_)         \
     do                                          \
     {                                           \

@@ -90,7 +90,7 @@ int launch_conv_nhwc_staged(const NhwcGeom& g_in, const int8_t* wpk, const void*
         std::call_once(once, [&]() { attr = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)STAGED_LDS_LIMIT); });  \
         NCNNHIP_CHECK(attr);                                                                                                                                 \
         hipLaunchKernelGGL(kernel, grid, block, tile_bytes + cache_bytes, stream, wpk, xb, g, epi, fusion, out_cp, out_cp, p.tiles_m, p.tiles_n, \
-                           p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, x_scale, (int)cache_bytes);                               \
+                           p.splits, p.steps_per_split, tile_magic(p.tiles_n), partial, counters, x_scale, (int)cache_bytes, ConvShortcutArg<false>());                               \
     } while (0)
 #define LAUNCH_STAGED_IN(BN_, MODE_)                 \
     do                                               \

@@ -886,6 +886,7 @@ static int resident_choose(const NhwcGeom& g, const ConvEpilogue& epi, const Con
 // the pixel threshold, NCNNHIP_RESIDENT_CFG forces one tile configuration (0..7): for measurements and tests.
 bool conv_resident_fits(const NhwcGeom& g, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp)
 {
+    if (!epi.out) return false; // it writes the fp32 blob
     if (g.ntaps < 2) return false; // first: most layers of a network are 1x1 and need not look the environment up
     if (getenv("NCNNHIP_RESIDENT_OFF")) return false;
     long long min_pixels = 40000;

@@ -1,0 +1,38 @@
+// A residual block's two 1x1 convolutions into one sum, where the block has a projection shortcut: the pipelined kernel with the shortcut's
+// K steps in front of the main convolution's (MODE 4), for layers with many tiles; conv_stream.hip has the form for few.
+//
+// The shortcut's fp32 result is neither written nor read again: for ResNet-50's second stage at 16 images 51 MB each way, half of
+// the two launches' traffic, which is what bounds them (5.5 TB/s).
+#include "conv_nhwc_pipelined_kernel.h"
+
+namespace ncnnhip {
+
+int launch_conv_shortcut(const NhwcGeom& g_in, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
+                         hipStream_t stream)
+{
+    if (conv_stream_fits(g_in, true)) return launch_conv_stream_shortcut(g_in, wpk, x, sc, epi, fusion, out_cp, stream);
+    NhwcGeom g = g_in;
+    g.H = g.outh = 1;
+    g.W = g.outw = g.npix;
+    // K stays whole: the shortcut's sums are finished where the main ones are.  64-channel tiles (six workgroups to a unit where four of 128 channels
+    // fit) until there are so many that the activations read per tile weigh more.  us, 128 channels wide / 64, fp32 and quantised output:
+    // 16 images 64 + 64 -> 256 on 56 x 56 23.5 / 22.1, 128 + 256 -> 512 on 28 x 28 20.4 / 17.2, 256 + 512 -> 1024 on 14 x 14 13.8 / 13.9, 512 + 1024 -> 2048
+    // on 7 x 7 16.3 / 14.5 (two launches: 35.7, 25.7, 16.4, 14.6); 64 images 76 / 83 (12544 tiles), 45.4 / 45.0 (6272), 36.4 / 34.8, 36.6 / 31.6
+    // (two launches: 147, 79, 44, 38).
+    const int tiles_m = ceil_div(g.npix, 64), wide = (long long)tiles_m * ceil_div(g.cout, 64) >= 8192, tiles_n = ceil_div(g.cout, wide ? 128 : 64);
+    const long long blocks = (long long)tiles_m * tiles_n;
+    NCNNHIP_REQUIRE(blocks < (1ll << 31) && blocks * tiles_n < (1ll << 32), "convolution: too many tiles");
+    ConvShortcutArg<true> arg;
+    static_cast<ConvShortcut&>(arg) = sc;
+#define LAUNCH_SHORTCUT(BN_)                                                                                                                            \
+    hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<64, BN_, PIPE_RING, false, 4>), dim3((unsigned)blocks), dim3(256), 0, stream, wpk, x, g, epi, fusion, out_cp, out_cp, \
+                       tiles_m, tiles_n, 1, g.K / 64, tile_magic(tiles_n), (int32_t*)0, (unsigned*)0, (const float*)0, 0, arg)
+    if (wide)
+        LAUNCH_SHORTCUT(128);
+    else
+        LAUNCH_SHORTCUT(64);
+#undef LAUNCH_SHORTCUT
+    return launch_status("conv_nhwc_pipelined_kernel (shortcut)");
+}
+
+} // namespace ncnnhip

@@ -22,14 +22,16 @@ constexpr int W = 4; // wavefronts a workgroup has
 
 // DENSE: 1x1, stride 1, unpadded: output pixel = input pixel.  Otherwise taps of whole 64-byte steps, so that a step lies inside one tap.
 // TP, TC: 16-pixel and 16-channel blocks of a tile.
-template<bool DENSE, int TP, int TC>
+// SHORTCUT: a projection shortcut is added (ConvShortcut), its K dealt out to the wavefronts and its sums met in the same way.
+template<bool DENSE, int TP, int TC, bool SHORTCUT = false>
 __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __restrict__ wpk, const int8_t* __restrict__ x, NhwcGeom g, ConvEpilogue epi, ConvFusion fusion,
-                                                             int out_cp, int tiles_m, unsigned magic_m, int per_wave)
+                                                             int out_cp, int tiles_m, unsigned magic_m, int per_wave, ConvShortcutArg<SHORTCUT> shortcut)
 {
     constexpr int U = 24 / (TP + TC); // K steps a wavefront has in flight, in 96 registers
     constexpr int NB = TP * TC;     // 16 x 16 blocks of the tile
     static_assert(NB <= W, "a wavefront finishes one block");
-    __shared__ v4i_cs part[W][NB][64]; // [wavefront][block][lane]
+    static_assert(!SHORTCUT || DENSE, "the sum's main convolution is 1x1");
+    __shared__ v4i_cs part[SHORTCUT ? 2 : 1][W][NB][64]; // [wavefront][block][lane]
     const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
@@ -48,6 +50,7 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
     // wavefront q < NB finishes block q: what it needs from memory, requested before the operands (clamped addresses, nothing selected)
     const int ch4 = ch0 + wave / TP * 16 + 4 * kq, pix = pix0 + wave % TP * 16 + r16;
     float s_in[4], bias[4], s_out[4];
+    float sc_in[4], sc_bias[4];
     v4f_cs res;
     const bool to_int8 = epi.scale_out != 0, with_residual = !to_int8 && fusion.residual != 0;
     if (wave < NB)
@@ -61,6 +64,17 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
             s_in[e] = epi.scale_in[ch];
             bias[e] = bias_src[ch];
             s_out[e] = s_out_src[ch];
+        }
+        if constexpr (SHORTCUT)
+        {
+            const float* sc_bias_src = shortcut.bias ? shortcut.bias : shortcut.scale_in;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+            {
+                const int ch = ch4 + e < g.cout ? ch4 + e : g.cout - 1;
+                sc_in[e] = shortcut.scale_in[ch];
+                sc_bias[e] = sc_bias_src[ch];
+            }
         }
         if (with_residual) res = *reinterpret_cast<const v4f_cs*>(fusion.residual + (size_t)(pix < g.npix ? pix : g.npix - 1) * out_cp + (ch4 < out_cp ? ch4 : out_cp - 4));
     }
@@ -97,6 +111,48 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
         q0 = begin * 64 - tap * g.tapK;
         ky = tap / g.kw;
         kx = tap - ky * g.kw;
+    }
+
+    if constexpr (SHORTCUT)
+    {
+        const int8_t* sw_row[TC];
+        const int8_t* sx_row[TP];
+#pragma unroll
+        for (int i = 0; i < TC; i++)
+        {
+            const int ch = ch0 + i * 16 + r16;
+            sw_row[i] = shortcut.wpk + (size_t)(ch < g.cout ? ch : g.cout - 1) * shortcut.Cp + kq * 16;
+        }
+#pragma unroll
+        for (int i = 0; i < TP; i++)
+        {
+            const int p = pix0 + i * 16 + r16, n = p < g.npix ? p : g.npix - 1, plane = shortcut.outw * shortcut.outh;
+            const int img = small_div(n, plane), at = n - img * plane, oy = small_div(at, shortcut.outw), ox = at - oy * shortcut.outw;
+            sx_row[i] = shortcut.x + (((size_t)img * shortcut.H + oy * shortcut.sh) * shortcut.W + ox * shortcut.sw) * shortcut.Cp + kq * 16;
+        }
+        const int steps = shortcut.Cp / 64, share = (steps + W - 1) / W;
+        const int from = wave * share, to = from + share < steps ? from + share : steps;
+        v4i_cs sum[NB];
+#pragma unroll
+        for (int q = 0; q < NB; q++) sum[q] = v4i_cs{0, 0, 0, 0};
+        for (int s0 = from; s0 < to; s0 += U)
+        {
+            v4i_cs fw[U][TC], fx[U][TP];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+            {
+#pragma unroll
+                for (int i = 0; i < TC; i++) fw[u][i] = *reinterpret_cast<const v4i_cs*>(s0 + u < to ? sw_row[i] + (size_t)(s0 + u) * 64 : zero);
+#pragma unroll
+                for (int i = 0; i < TP; i++) fx[u][i] = *reinterpret_cast<const v4i_cs*>(s0 + u < to ? sx_row[i] + (size_t)(s0 + u) * 64 : zero);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int q = 0; q < NB; q++) sum[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[u][q / TP], fx[u][q % TP], sum[q], 0, 0, 0);
+        }
+#pragma unroll
+        for (int q = 0; q < NB; q++) part[1][wave][q][lane] = sum[q];
     }
 
     v4i_cs acc[NB]; // channel block q / TP, pixel block q % TP
@@ -147,12 +203,12 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
 
     // the wavefronts' sums meet (integer addition: exact in any order)
 #pragma unroll
-    for (int q = 0; q < NB; q++) part[wave][q][lane] = acc[q];
+    for (int q = 0; q < NB; q++) part[0][wave][q][lane] = acc[q];
     __syncthreads();
     if (wave >= NB || ch4 >= out_cp || pix >= g.npix) return;
-    v4i_cs sum = part[0][wave][lane];
+    v4i_cs sum = part[0][0][wave][lane];
 #pragma unroll
-    for (int s = 1; s < W; s++) sum += part[s][wave][lane];
+    for (int s = 1; s < W; s++) sum += part[0][s][wave][lane];
 
     // the pipelined kernel's epilogue, statement by statement
     float f[4];
@@ -187,6 +243,19 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
     v4f_cs v;
 #pragma unroll
     for (int e = 0; e < 4; e++) v[e] = ch4 + e < g.cout ? f[e] : 0.f;
+    if constexpr (SHORTCUT)
+    {
+        v4i_cs other = part[1][0][wave][lane];
+#pragma unroll
+        for (int s = 1; s < W; s++) other += part[1][s][wave][lane];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+        {
+            float t = add_rn(mul_rn((float)other[e], sc_in[e]), shortcut.bias ? sc_bias[e] : -0.f);
+            if (shortcut.act.type != 0) t = apply_activation(t, shortcut.act);
+            v[e] = add_rn(v[e], ch4 + e < g.cout ? t : 0.f);
+        }
+    }
     if (with_residual)
     {
 #pragma unroll
@@ -197,7 +266,7 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] = v[e] < 0.f ? 0.f : v[e]; // the ReLU LAYER's statement (src/layer/relu.cpp:36-37): a NaN stays, unlike fmaxf
     }
-    *reinterpret_cast<v4f_cs*>(static_cast<float*>(epi.out) + o) = v;
+    if (epi.out) *reinterpret_cast<v4f_cs*>(static_cast<float*>(epi.out) + o) = v;
     if (fusion.q8_out)
     {
         float q[4];
@@ -247,7 +316,7 @@ int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, co
     const int per_wave = ceil_div(g.K / 64, W);
 #define STREAM(DENSE_, TP_, TC_)                                                                                                                            \
     hipLaunchKernelGGL((conv_stream_kernel<DENSE_, TP_, TC_>), dim3((unsigned)blocks), dim3(64 * W), 0, stream, wpk, x, g, epi, fusion, out_cp, tiles_m, magic_m, \
-                       per_wave)
+                       per_wave, ConvShortcutArg<false>())
 #define STREAM_TILE(DENSE_)       \
     do                            \
     {                             \
@@ -265,6 +334,30 @@ int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, co
 #undef STREAM_TILE
 #undef STREAM
     return launch_status("conv_stream_kernel");
+}
+
+// us, two launches / one: one image 64 + 64 -> 256 on 56 x 56 (784 tiles of 32 x 32: conv_shortcut.hip) 8.0 / 5.5, 256 + 512 -> 1024 on 14 x 14 8.4 / 6.4,
+// 512 + 1024 -> 2048 on 7 x 7 8.0 / 6.3.
+int launch_conv_stream_shortcut(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion,
+                                int out_cp, hipStream_t stream)
+{
+    const int tile = stream_tile(g, true), tp = tile / 10, tc = tile % 10;
+    NCNNHIP_REQUIRE(tile && stream_dense(g) && g.K == g.Cp && sc.Cp % 64 == 0, "convolution: this layer does not fit the kernel for few tiles");
+    const int tiles_m = ceil_div(g.npix, 16 * tp), tiles_n = ceil_div(g.cout, 16 * tc);
+    const unsigned magic_m = tiles_m > 1 ? (unsigned)((1ull << 32) / (unsigned)tiles_m + 1) : 0u;
+    ConvShortcutArg<true> arg;
+    static_cast<ConvShortcut&>(arg) = sc;
+#define STREAM(TP_, TC_)                                                                                                                                               \
+    hipLaunchKernelGGL((conv_stream_kernel<true, TP_, TC_, true>), dim3((unsigned)(tiles_m * tiles_n)), dim3(64 * W), 0, stream, wpk, x, g, epi, fusion, out_cp, tiles_m, \
+                       magic_m, ceil_div(g.K / 64, W), arg)
+    if (tile == 11)
+        STREAM(1, 1);
+    else if (tile == 12)
+        STREAM(1, 2);
+    else
+        STREAM(2, 2);
+#undef STREAM
+    return launch_status("conv_stream_kernel (shortcut)");
 }
 
 } // namespace ncnnhip

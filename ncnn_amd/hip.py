@@ -35,6 +35,11 @@ class ConvFusion(C.Structure):
     _fields_ = [("residual_dev", C.c_void_p), ("relu_after", C.c_int), ("quantised_out_dev", C.c_void_p), ("quantise_scale", C.c_float)]
 
 
+class ConvShortcut(C.Structure):
+    _fields_ = [("desc", C.POINTER(ConvDesc)), ("nhwc_dev", C.c_void_p), ("packed_weight_dev", C.c_void_p), ("scale_in_dev", C.c_void_p), ("bias_dev", C.c_void_p),
+                ("act", Activation)]
+
+
 class PoolDesc(C.Structure):
     _fields_ = [(n, C.c_int) for n in ("w", "h", "c", "batch", "pooling_type", "kernel_w", "kernel_h", "stride_w", "stride_h", "pad_top", "pad_left",
                                        "outw", "outh", "global_pooling", "avgpool_count_include_pad", "count_x0", "count_x1", "count_y0", "count_y1")]
@@ -100,6 +105,9 @@ _SIGNATURES = {
                                           C.POINTER(ConvFusion), C.c_void_p, C.c_size_t, C.c_void_p],
     "ncnnhip_conv_int8_nhwc_fused": [C.POINTER(ConvDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, Activation, C.c_void_p, C.POINTER(ConvFusion), C.c_void_p,
                                      C.c_size_t, C.c_void_p],
+    "ncnnhip_conv_shortcut_supported": [C.POINTER(ConvDesc), C.POINTER(ConvDesc), C.POINTER(C.c_int)],
+    "ncnnhip_conv_int8_nhwc_tail": [C.POINTER(ConvDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, Activation, C.POINTER(ConvShortcut), C.c_void_p,
+                                    C.POINTER(ConvFusion), C.c_void_p, C.c_size_t, C.c_void_p],
     "ncnnhip_conv_resolved_pads": [C.POINTER(ConvDesc), C.POINTER(C.c_int), C.POINTER(C.c_int)],
     "ncnnhip_padded_channels": [C.c_int],
     "ncnnhip_chw_to_nhwc": [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_size_t, C.c_size_t, C.c_void_p, C.c_void_p],

@@ -408,6 +408,105 @@ int Convolution_hip::forward_hip_fused(const HipMat& bottom, const HipMat* resid
     return forward_device(bottom, residual, relu, q8_scale, 0.f, top, cmd, opt);
 }
 
+const signed char* Convolution_hip::quantised_operand(const HipMat& bottom) const
+{
+    if (bottom.dims != 3 || bottom.narrow() || bottom_blob_int8_scales.w < 1) return 0;
+    if (bottom.elemsize == 1u) return bottom.q8_scale == 0.f || bottom.q8_scale == bottom_blob_int8_scales[0] ? (const signed char*)bottom.data : 0;
+    // (an fp32 blob may come with its producer's quantised copy)
+    return bottom.elemsize == 4u && bottom.q8 && !bottom.q8->empty() && bottom.q8_scale == bottom_blob_int8_scales[0] && bottom.q8->count() == bottom.count()
+               ? (const signed char*)bottom.q8->data
+               : 0;
+}
+
+int Convolution_hip::forward_hip_fused_quantised(const HipMat& bottom, const HipMat* residual, bool relu, float q8_scale, HipMat& top, HipCommand& cmd,
+                                                 const Option& opt) const
+{
+    bool done = false;
+    const int ret = forward_tail(bottom, residual, 0, 0, relu, q8_scale, true, top, cmd, opt, done);
+    return ret != 0 || done ? ret : forward_hip_fused(bottom, residual, relu, q8_scale, top, cmd, opt);
+}
+
+int Convolution_hip::forward_hip_shortcut(const HipMat& bottom, const Layer& shortcut, const HipMat& shortcut_bottom, bool relu, float q8_scale, bool only_quantised,
+                                          HipMat& top, HipCommand& cmd, const Option& opt, bool& folded) const
+{
+    folded = false;
+    const Convolution_hip* other = dynamic_cast<const Convolution_hip*>(&shortcut);
+    return other ? forward_tail(bottom, 0, other, &shortcut_bottom, relu, q8_scale, only_quantised, top, cmd, opt, folded) : 0;
+}
+
+// done = false: something is not as the one launch needs it; the ordinary route takes it from there, its checks and messages included.
+int Convolution_hip::forward_tail(const HipMat& bottom, const HipMat* residual, const Convolution_hip* shortcut, const HipMat* shortcut_bottom, bool relu,
+                                  float q8_scale, bool only_quantised, HipMat& top, HipCommand& cmd, const Option& opt, bool& done) const
+{
+    done = false;
+    const Convolution_hip* const convs[2] = {this, shortcut};
+    const HipMat* const blobs[2] = {&bottom, shortcut_bottom};
+    const signed char* xq[2] = {0, 0};
+    ncnnhip_conv_desc desc[2];
+    if (!opt.use_int8_inference || (only_quantised && q8_scale == 0.f)) return 0;
+    for (int i = 0; i < (shortcut ? 2 : 1); i++)
+    {
+        const Convolution_hip& c = *convs[i];
+        if (!c.hip_can_fuse_tail() || !c.d_scale_in || !c.d_weight_packed) return 0;
+        xq[i] = c.quantised_operand(*blobs[i]);
+        if (!xq[i] || c.weight_data_size != c.num_output * blobs[i]->c * c.kernel_w * c.kernel_h) return 0;
+        desc[i] = c.describe(blobs[i]->w, blobs[i]->h, blobs[i]->c, blobs[i]->n);
+    }
+    int supported = 1;
+    if (shortcut && (ncnnhip_conv_shortcut_supported(&desc[0], &desc[1], &supported) != 0 || !supported)) return 0;
+    int outw = 0, outh = 0;
+    int rc = ncnnhip_conv_out_shape(&desc[0], &outw, &outh);
+    if (rc != 0) return 0;
+    if (residual && (residual->elemsize != 4u || residual->dims != 3 || residual->narrow() || residual->w != outw || residual->h != outh || residual->c != num_output
+                     || residual->n != bottom.n))
+        return 0;
+    HipMat own;
+    own.create(outw, outh, num_output, only_quantised ? (size_t)1u : (size_t)4u, bottom.n, &cmd);
+    if (own.empty()) return -100;
+    ncnnhip_conv_fusion fu;
+    fu.residual_dev = residual ? (const float*)residual->data : 0;
+    fu.relu_after = relu ? 1 : 0;
+    fu.quantised_out_dev = only_quantised ? (int8_t*)own.data : 0;
+    fu.quantise_scale = q8_scale;
+    if (q8_scale != 0.f)
+    {
+        own.q8_scale = q8_scale;
+        if (!only_quantised)
+        {
+            own.q8.reset(new HipMat);
+            own.q8->create(outw, outh, num_output, 1u, bottom.n, &cmd);
+            if (own.q8->empty()) return -100;
+            fu.quantised_out_dev = (int8_t*)own.q8->data;
+        }
+    }
+    ncnnhip_conv_shortcut sc;
+    void* ws = 0;
+    size_t workspace_bytes = 0;
+    if (shortcut)
+    {
+        sc.desc = &desc[1];
+        sc.nhwc_dev = xq[1];
+        sc.packed_weight_dev = (const int8_t*)shortcut->d_weight_packed;
+        sc.scale_in_dev = (const float*)shortcut->d_scale_in;
+        sc.bias_dev = (const float*)shortcut->d_bias;
+        sc.act = make_activation(shortcut->activation_type, shortcut->activation_params);
+    }
+    else
+    {
+        rc = ncnnhip_conv_nhwc_sizes(&desc[0], 0, 0, &workspace_bytes);
+        if (rc != 0) return to_ncnn_status(rc, "ncnnhip_conv_nhwc_sizes");
+        ws = workspace_bytes ? cmd.zeroed_workspace(workspace_bytes) : 0;
+        if (workspace_bytes && !ws) return -100;
+    }
+    rc = ncnnhip_conv_int8_nhwc_tail(&desc[0], xq[0], (const int8_t*)d_weight_packed, (const float*)d_scale_in, (const float*)d_bias,
+                                     make_activation(activation_type, activation_params), shortcut ? &sc : 0, only_quantised ? 0 : (float*)own.data, &fu, ws,
+                                     workspace_bytes, cmd.stream);
+    if (rc != 0) return to_ncnn_status(rc, "ncnnhip_conv_int8_nhwc_tail");
+    top = own;
+    done = true;
+    return 0;
+}
+
 bool Convolution_hip::hip_accepts_narrow_input() const
 {
     return support_hip; // the narrow-input kernel quantises straight from it; any other form widens it itself

@@ -27,6 +27,10 @@ public:
     virtual bool hip_can_fuse_tail() const;
     virtual int forward_hip_fused(const ncnn::HipMat& bottom_blob, const ncnn::HipMat* residual, bool relu, float q8_scale, ncnn::HipMat& top_blob,
                                   ncnn::HipCommand& cmd, const ncnn::Option& opt) const;
+    virtual int forward_hip_fused_quantised(const ncnn::HipMat& bottom_blob, const ncnn::HipMat* residual, bool relu, float q8_scale, ncnn::HipMat& top_blob,
+                                            ncnn::HipCommand& cmd, const ncnn::Option& opt) const;
+    virtual int forward_hip_shortcut(const ncnn::HipMat& bottom_blob, const ncnn::Layer& shortcut, const ncnn::HipMat& shortcut_bottom, bool relu, float q8_scale,
+                                     bool only_quantised, ncnn::HipMat& top_blob, ncnn::HipCommand& cmd, const ncnn::Option& opt, bool& folded) const;
     virtual int hip_prepare_requantise(float scale);
     virtual bool hip_accepts_narrow_input() const;
     virtual int forward_hip_requantised(const ncnn::HipMat& bottom_blob, float scale, ncnn::HipMat& top_blob, ncnn::HipCommand& cmd,
@@ -60,6 +64,11 @@ private:
     int input_scale_count; // 1 or group
     void* d_weight_dw;     // depthwise (channels == group == num_output): [kh*kw][16*ceil(c/16)]
     bool is_depthwise() const;
+    // what both forms above share: residual or shortcut, fp32 and quantised output or the latter alone
+    int forward_tail(const ncnn::HipMat& bottom_blob, const ncnn::HipMat* residual, const Convolution_hip* shortcut, const ncnn::HipMat* shortcut_bottom, bool relu,
+                     float q8_scale, bool only_quantised, ncnn::HipMat& top_blob, ncnn::HipCommand& cmd, const ncnn::Option& opt, bool& done) const;
+    // the blob as this layer's int8 operand when it exists in that form already (0: it does not)
+    const signed char* quantised_operand(const ncnn::HipMat& bottom_blob) const;
     ncnnhip_conv_desc describe(int w, int h, int channels, int batch) const;
 };
 

@@ -117,6 +117,16 @@ int Layer::forward_hip_fused(const HipMat&, const HipMat*, bool, float, HipMat&,
 {
     return -1;
 }
+int Layer::forward_hip_fused_quantised(const HipMat& bottom_blob, const HipMat* residual, bool relu, float q8_scale, HipMat& top_blob, HipCommand& cmd,
+                                       const Option& opt) const
+{
+    return forward_hip_fused(bottom_blob, residual, relu, q8_scale, top_blob, cmd, opt);
+}
+int Layer::forward_hip_shortcut(const HipMat&, const Layer&, const HipMat&, bool, float, bool, HipMat&, HipCommand&, const Option&, bool& folded) const
+{
+    folded = false;
+    return 0;
+}
 int Layer::hip_prepare_requantise(float)
 {
     return -1;

@@ -80,6 +80,14 @@ public:
     virtual bool hip_accepts_narrow_input() const;
     // forward_hip of an int8 blob holding Quantize(x, s), s > 0, gives Quantize(forward_hip(x), s) (windowed max pooling)
     virtual bool hip_quantise_transparent() const;
+    // forward_hip_fused for a result that every consumer quantises with q8_scale: top may be that int8 blob alone (q8_scale
+    // set, as after forward_hip_requantised)
+    virtual int forward_hip_fused_quantised(const HipMat& bottom_blob, const HipMat* residual, bool relu, float q8_scale, HipMat& top_blob, HipCommand& cmd,
+                                            const Option& opt) const;
+    // ... and for a residual that is the output of another layer, read by this sum only: computed along with this layer's own.
+    // folded = false: not applicable, nothing was enqueued.  only_quantised as in forward_hip_fused_quantised.
+    virtual int forward_hip_shortcut(const HipMat& bottom_blob, const Layer& shortcut, const HipMat& shortcut_bottom, bool relu, float q8_scale, bool only_quantised,
+                                     HipMat& top_blob, HipCommand& cmd, const Option& opt, bool& folded) const;
 
     void* userdata;
     int typeindex;

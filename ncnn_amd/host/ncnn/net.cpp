@@ -253,8 +253,11 @@ public:
         int eltwise;  // the sum layer
         int residual; // blob index of the sum's other input
         bool relu;
+        int shortcut;      // the layer whose output is the residual and is read by the sum alone (a projection shortcut), -1: none
+        bool only_quantised; // every reader of L's output quantises it, with quantise_scale
     };
     std::vector<TailPlan> tail_plan;
+    std::vector<char> tail_zone; // blobs that hold quantised values when such a tail's output is emitted in that form alone
     // sibling_group[L]: the layers (L among them, in layer order) that read outputs of one Split, have equal sibling keys and
     // may therefore run as one launch; empty: none
     std::vector<std::vector<int> > sibling_group;
@@ -267,7 +270,7 @@ public:
     std::vector<char> quantised_zone;
     void build_fusion_plan();
     bool collect_quantise_scales(int blob, float& scale, bool& any) const;
-    bool all_consumers_quantise(int blob, float& scale, bool& any, std::vector<int>& zone) const;
+    bool all_consumers_quantise(int blob, float& scale, bool& any, std::vector<int>& zone, bool through_pooling = true) const;
     bool follows_requant_plan(int blob, const ExecState& st, const Option& opt) const;
     int try_fused_tail(int layer_index, ExecState& st, const Option& opt, bool& done) const;
 
@@ -322,19 +325,20 @@ bool NetPrivate::collect_quantise_scales(int blob, float& scale, bool& any) cons
 }
 
 // true when every path from the blob ends, through Split and quantise-transparent layers, in a consumer that
-// quantises with the same scale; zone collects the blobs on the way
-bool NetPrivate::all_consumers_quantise(int blob, float& scale, bool& any, std::vector<int>& zone) const
+// quantises with the same scale; zone collects the blobs on the way.  through_pooling = false: through Split layers only
+bool NetPrivate::all_consumers_quantise(int blob, float& scale, bool& any, std::vector<int>& zone, bool through_pooling) const
 {
     zone.push_back(blob);
     const int ci = blobs[(size_t)blob].consumer;
     if (ci < 0) return false; // a network output keeps the model's type
     const Layer* consumer = layers[(size_t)ci];
-    if (consumer->type == "Split" || (consumer->support_hip && consumer->one_blob_only && consumer->hip_quantise_transparent()))
+    if (consumer->type == "Split" || (through_pooling && consumer->support_hip && consumer->one_blob_only && consumer->hip_quantise_transparent()))
     {
         for (size_t i = 0; i < consumer->tops.size(); i++)
-            if (!all_consumers_quantise(consumer->tops[i], scale, any, zone)) return false;
+            if (!all_consumers_quantise(consumer->tops[i], scale, any, zone, through_pooling)) return false;
         return !consumer->tops.empty();
     }
+    if (!through_pooling && consumer->featmask) return false; // it may run on the host
     const float s = consumer->support_hip ? consumer->hip_input_quantise_scale() : 0.f;
     if (!(s > 0.f) || (any && s != scale)) return false;
     scale = s;
@@ -351,11 +355,12 @@ bool NetPrivate::follows_requant_plan(int blob, const ExecState& st, const Optio
 
 void NetPrivate::build_fusion_plan()
 {
-    const TailPlan none = {-1, -1, -1, false};
+    const TailPlan none = {-1, -1, -1, false, -1, false};
     tail_plan.assign(layers.size(), none);
     quantise_scale.assign(blobs.size(), 0.f);
     requant_scale.assign(blobs.size(), 0.f);
     quantised_zone.assign(blobs.size(), 0);
+    tail_zone.assign(blobs.size(), 0);
     for (size_t b = 0; b < blobs.size(); b++)
     {
         const int p = blobs[b].producer;
@@ -392,7 +397,11 @@ void NetPrivate::build_fusion_plan()
             }
         }
         if (best < 0) continue;
-        TailPlan tp = {best, (int)li, e->bottoms[(size_t)(1 - best_slot)], false};
+        TailPlan tp = {best, (int)li, e->bottoms[(size_t)(1 - best_slot)], false, -1, false};
+        const int rp = blobs[(size_t)tp.residual].producer;
+        if (rp >= 0 && blobs[(size_t)tp.residual].consumer == (int)li && layers[(size_t)rp]->support_hip && layers[(size_t)rp]->one_blob_only
+            && layers[(size_t)rp]->bottoms.size() == 1 && layers[(size_t)rp]->tops.size() == 1 && layers[(size_t)rp]->hip_can_fuse_tail())
+            tp.shortcut = rp;
         tail_plan[li] = tp;
         // ... followed by a plain ReLU: that layer's output comes out of the same epilogue
         const int ri = blobs[(size_t)e->tops[0]].consumer;
@@ -400,6 +409,16 @@ void NetPrivate::build_fusion_plan()
         {
             tp.relu = true;
             tail_plan[(size_t)ri] = tp;
+        }
+        // ... and alone in quantised form where nobody reads the fp32 values
+        const int last = tp.relu ? ri : (int)li;
+        float s = 0.f;
+        bool any = false;
+        std::vector<int> zone;
+        if (layers[(size_t)last]->tops.size() == 1 && all_consumers_quantise(layers[(size_t)last]->tops[0], s, any, zone, false) && any)
+        {
+            tail_plan[(size_t)last].only_quantised = true;
+            for (size_t i = 0; i < zone.size(); i++) tail_zone[(size_t)zone[i]] = 1;
         }
     }
     // layers behind one Split that can share a launch (block-quantised Gemms on the same activation rows)
@@ -515,41 +534,65 @@ int NetPrivate::try_fused_tail(int layer_index, ExecState& st, const Option& opt
     if (st.has(conv->tops[0]) || st.has(sum->tops[0])) return 0; // an intermediate exists already (fed or extracted)
     if (conv->featmask || sum->featmask || last->featmask) return 0; // a masked layer runs on its own, under its own options
 
-    const int needed[2] = {conv->bottoms[0], tp.residual};
-    for (int k = 0; k < 2; k++)
+    // the output in quantised form alone, unless this extract call asks for the blob itself
+    const bool only_quantised = tp.only_quantised && (st.wanted < 0 || !tail_zone[(size_t)st.wanted]);
+    const float q8_scale = quantise_scale[(size_t)last->tops[0]];
+    // The residual's own layer runs in the same launch when its output does not exist yet (timed runs keep one record per layer).
+    const Layer* shortcut = tp.shortcut >= 0 && !st.time_layers && !st.has(tp.residual) && !layers[(size_t)tp.shortcut]->featmask ? layers[(size_t)tp.shortcut] : 0;
+    HipMat top, ins[2];
+    for (;;)
     {
-        const int bi = needed[k];
-        if (st.has(bi)) continue;
-        const int producer = blobs[(size_t)bi].producer;
-        if (producer < 0) return 0;
-        int ret = forward_layer(producer, st, opt);
-        if (ret != 0) return ret;
-        if (!st.has(bi)) return 0;
-    }
-    if (!st.cmd) st.cmd = acquire_command();
-    HipCommand& cmd = *st.cmd;
-    int ret = cmd.ensure_ready();
-    if (ret != 0) return ret;
-    HipMat ins[2];
-    for (int k = 0; k < 2; k++)
-    {
-        const size_t bi = (size_t)needed[k];
-        if (st.dev[bi].empty())
+        const int needed[2] = {conv->bottoms[0], shortcut ? shortcut->bottoms[0] : tp.residual};
+        for (int k = 0; k < 2; k++)
         {
-            ret = cmd.upload(st.host[bi], st.dev[bi]);
+            const int bi = needed[k];
+            if (st.has(bi)) continue;
+            const int producer = blobs[(size_t)bi].producer;
+            if (producer < 0) return 0;
+            int ret = forward_layer(producer, st, opt);
+            if (ret != 0) return ret;
+            if (!st.has(bi)) return 0;
+        }
+        if (!st.cmd) st.cmd = acquire_command();
+        HipCommand& cmd = *st.cmd;
+        int ret = cmd.ensure_ready();
+        if (ret != 0) return ret;
+        for (int k = 0; k < 2; k++)
+        {
+            const size_t bi = (size_t)needed[k];
+            if (st.dev[bi].empty())
+            {
+                ret = cmd.upload(st.host[bi], st.dev[bi]);
+                if (ret != 0) return ret;
+            }
+            ins[k] = st.dev[bi];
+        }
+        bool folded = false;
+        if (shortcut)
+        {
+            ret = conv->forward_hip_shortcut(ins[0], *shortcut, ins[1], tp.relu, q8_scale, only_quantised, top, cmd, opt, folded);
+            if (ret != 0) return ret;
+            if (!folded)
+            {
+                shortcut = 0; // its layer runs on its own
+                continue;
+            }
+        }
+        else if (ins[1].elemsize != 4u || ins[1].dims != 3 || ins[1].narrow())
+            return 0; // the residual must be an ordinary fp32 blob: take the plain route
+        for (int k = 0; k < 2; k++)
+        {
+            st.dev[(size_t)needed[k]].release();
+            st.host[(size_t)needed[k]].release();
+        }
+        if (!folded)
+        {
+            ret = only_quantised ? conv->forward_hip_fused_quantised(ins[0], &ins[1], tp.relu, q8_scale, top, cmd, opt)
+                                 : conv->forward_hip_fused(ins[0], &ins[1], tp.relu, q8_scale, top, cmd, opt);
             if (ret != 0) return ret;
         }
-        ins[k] = st.dev[bi];
+        break;
     }
-    if (ins[1].elemsize != 4u || ins[1].dims != 3 || ins[1].narrow()) return 0; // the residual must be an ordinary fp32 blob: take the plain route
-    for (int k = 0; k < 2; k++)
-    {
-        st.dev[(size_t)needed[k]].release();
-        st.host[(size_t)needed[k]].release();
-    }
-    HipMat top;
-    ret = conv->forward_hip_fused(ins[0], &ins[1], tp.relu, quantise_scale[(size_t)last->tops[0]], top, cmd, opt);
-    if (ret != 0) return ret;
     st.dev[(size_t)last->tops[0]] = top;
     st.host[(size_t)last->tops[0]].release();
     done = true;
