@@ -71,6 +71,49 @@ __global__ __launch_bounds__(256) void chw_to_nhwc4_f32_kernel(const float* __re
     *reinterpret_cast<v4f*>(dst + ((size_t)img * hw + pix) * 4) = v;
 }
 
+// The same for planes that do not begin on 128-byte lines (sizes that are no multiple of 32 pixels, mostly): read over PCIe, what counts is the
+// number of requests, one a line and wavefront, and a wavefront's 256 bytes off the lines are three instead of two.  A workgroup takes 1024 pixels,
+// every load of a plane begins on a line (its edges masked), and the planes meet in LDS.  us for three images from page-locked memory, the kernel
+// above / here: 176 x 257 (planes on 64 bytes) 35.5 / 33.4, 49604 pixels (on 16) 40.1 / 37.7; with 512 pixels 34.4 and 38.9.  Planes on lines stay
+// above: 224 x 224 34.3 / 34.9.
+constexpr int LINES_PIXELS = 1024;
+__global__ __launch_bounds__(256) void chw_to_nhwc4_f32_lines_kernel(const float* __restrict__ src, size_t cstep, size_t nstep, int c, int hw, float* __restrict__ dst)
+{
+    constexpr int LOADS = LINES_PIXELS / 256 + 1;
+    __shared__ float plane[4][LINES_PIXELS];
+    const int img = blockIdx.y, p0 = blockIdx.x * LINES_PIXELS, count = hw - p0 < LINES_PIXELS ? hw - p0 : LINES_PIXELS;
+    const float* sp = src + (size_t)img * nstep + p0;
+    float x[4][LOADS]; // all requested before the first is used
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+    {
+        if (q >= c) break;
+        const float* from = sp + (size_t)q * cstep;
+        const int first = (int)threadIdx.x - (int)((reinterpret_cast<uintptr_t>(from) >> 2) & 31);
+#pragma unroll
+        for (int i = 0; i < LOADS; i++)
+            if ((unsigned)(first + i * 256) < (unsigned)count) x[q][i] = from[first + i * 256];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+    {
+        if (q >= c) break;
+        const int first = (int)threadIdx.x - (int)((reinterpret_cast<uintptr_t>(sp + (size_t)q * cstep) >> 2) & 31);
+#pragma unroll
+        for (int i = 0; i < LOADS; i++)
+            if ((unsigned)(first + i * 256) < (unsigned)count) plane[q][first + i * 256] = x[q][i];
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < count; p += 256)
+    {
+        v4f v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (q < c) v[q] = plane[q][p];
+        *reinterpret_cast<v4f*>(dst + ((size_t)img * hw + p0 + p) * 4) = v;
+    }
+}
+
 __global__ __launch_bounds__(256) void widen_nhwc4_f32_kernel(const float* __restrict__ src, float* __restrict__ dst, size_t pixels)
 {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -654,6 +697,12 @@ int ncnnhip_chw_to_nhwc(const void* src_dev, int elemsize, int c, int hw, int ba
 int ncnnhip_chw_to_nhwc4_f32(const float* src_dev, int c, int hw, int batch, size_t cstep, size_t nstep, float* dst_dev, void* stream)
 {
     NCNNHIP_REQUIRE(src_dev && dst_dev && c >= 1 && c <= 4 && hw > 0 && batch > 0 && batch <= 65535 && cstep >= (size_t)hw, "ncnnhip_chw_to_nhwc4_f32: bad argument");
+    const bool on_lines = ((reinterpret_cast<uintptr_t>(src_dev) | cstep * 4 | (batch > 1 ? nstep * 4 : 0)) & 127) == 0;
+    if (!on_lines)
+    {
+        hipLaunchKernelGGL(chw_to_nhwc4_f32_lines_kernel, dim3(ceil_div(hw, LINES_PIXELS), batch), dim3(256), 0, as_stream(stream), src_dev, cstep, nstep, c, hw, dst_dev);
+        return launch_status("chw_to_nhwc4_f32_lines_kernel");
+    }
     hipLaunchKernelGGL(chw_to_nhwc4_f32_kernel, dim3(ceil_div(hw, 256), batch), dim3(256), 0, as_stream(stream), src_dev, cstep, nstep, c, hw, dst_dev);
     return launch_status("chw_to_nhwc4_f32_kernel");
 }
