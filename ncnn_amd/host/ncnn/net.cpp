@@ -272,6 +272,7 @@ public:
     bool collect_quantise_scales(int blob, float& scale, bool& any) const;
     bool all_consumers_quantise(int blob, float& scale, bool& any, std::vector<int>& zone, bool through_pooling = true) const;
     bool follows_requant_plan(int blob, const ExecState& st, const Option& opt) const;
+    bool zone_is_consumed(int blob, const ExecState& st) const;
     int try_fused_tail(int layer_index, ExecState& st, const Option& opt, bool& done) const;
 
     int forward_layer(int layer_index, ExecState& st, const Option& opt) const;
@@ -522,6 +523,32 @@ static Option masked_option(const Option& opt, int featmask)
     return o;
 }
 
+// true when this extract call runs every layer that reads the blob (through Split layers): in light mode nothing of it is left afterwards
+bool NetPrivate::zone_is_consumed(int blob, const ExecState& st) const
+{
+    std::vector<char> runs(layers.size(), 0); // what it takes from here to the blob asked for
+    std::vector<int> todo(1, blobs[(size_t)st.wanted].producer);
+    while (!todo.empty())
+    {
+        const int l = todo.back();
+        todo.pop_back();
+        if (l < 0 || runs[(size_t)l]) continue;
+        runs[(size_t)l] = 1;
+        for (size_t i = 0; i < layers[(size_t)l]->bottoms.size(); i++)
+            if (!st.has(layers[(size_t)l]->bottoms[i])) todo.push_back(blobs[(size_t)layers[(size_t)l]->bottoms[i]].producer);
+    }
+    todo.assign(1, blob);
+    while (!todo.empty())
+    {
+        const int ci = blobs[(size_t)todo.back()].consumer;
+        todo.pop_back();
+        if (ci < 0 || !runs[(size_t)ci]) return false;
+        const Layer* consumer = layers[(size_t)ci];
+        if (consumer->type == "Split") todo.insert(todo.end(), consumer->tops.begin(), consumer->tops.end());
+    }
+    return true;
+}
+
 int NetPrivate::try_fused_tail(int layer_index, ExecState& st, const Option& opt, bool& done) const
 {
     done = false;
@@ -534,8 +561,6 @@ int NetPrivate::try_fused_tail(int layer_index, ExecState& st, const Option& opt
     if (st.has(conv->tops[0]) || st.has(sum->tops[0])) return 0; // an intermediate exists already (fed or extracted)
     if (conv->featmask || sum->featmask || last->featmask) return 0; // a masked layer runs on its own, under its own options
 
-    // the output in quantised form alone, unless this extract call asks for the blob itself
-    const bool only_quantised = tp.only_quantised && (st.wanted < 0 || !tail_zone[(size_t)st.wanted]);
     const float q8_scale = quantise_scale[(size_t)last->tops[0]];
     // The residual's own layer runs in the same launch when its output does not exist yet (timed runs keep one record per layer).
     const Layer* shortcut = tp.shortcut >= 0 && !st.time_layers && !st.has(tp.residual) && !layers[(size_t)tp.shortcut]->featmask ? layers[(size_t)tp.shortcut] : 0;
@@ -567,6 +592,10 @@ int NetPrivate::try_fused_tail(int layer_index, ExecState& st, const Option& opt
             }
             ins[k] = st.dev[bi];
         }
+        // the output in quantised form alone, unless this extract call asks for the blob itself or leaves it, or what Split makes of it, for a later
+        // one (looked up here, where the device has work already)
+        const bool only_quantised =
+            tp.only_quantised && opt.lightmode && st.wanted >= 0 && !tail_zone[(size_t)st.wanted] && zone_is_consumed(last->tops[0], st);
         bool folded = false;
         if (shortcut)
         {
