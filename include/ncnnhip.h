@@ -229,6 +229,30 @@ int ncnnhip_conv_int8_nhwc_from_float(const ncnnhip_conv_desc* desc, const void*
  * and for callers that size workspaces. */
 int ncnnhip_conv_small_tile_selected(const ncnnhip_conv_desc* desc, int elemsize);
 
+/* Which kernel, and in which form, ncnnhip_conv_int8_nhwc / _fused / _tail (without a shortcut) runs a layer on for an int8 blob, channels-last
+ * output and 16-byte aligned buffers.  fusion may be NULL; of its pointers only whether they are NULL counts.  No counterpart in the
+ * reference: a query for tests and measurements, answered by the launches' own rules. */
+enum
+{
+    NCNNHIP_CONV_GENERAL = 0,   /* any border value */
+    NCNNHIP_CONV_SMALL_TILE = 1,
+    NCNNHIP_CONV_POINTWISE = 2,
+    NCNNHIP_CONV_RESIDENT = 3,  /* weights resident in LDS */
+    NCNNHIP_CONV_FEW_TILES = 4,
+    NCNNHIP_CONV_PIPELINED = 5
+};
+typedef struct ncnnhip_conv_route
+{
+    int kernel;
+    /* the rest: few tiles (tiles only) and pipelined, else 0 */
+    int tile_pixels, tile_channels;
+    int addressing; /* 0 general, 1 dense 1x1, 2 narrow-input taps, 3 taps of whole 64-byte steps */
+    int groups;     /* of four wavefronts that share a tile's K */
+    int splits;     /* of K over workgroups */
+} ncnnhip_conv_route;
+int ncnnhip_conv_int8_nhwc_route(const ncnnhip_conv_desc* desc, ncnnhip_activation act, int int8_out, const ncnnhip_conv_fusion* fusion,
+                                 ncnnhip_conv_route* route);
+
 
 /* Convolution::forward_int8 (src/layer/convolution.cpp:383-508) for layers with at most 4 input channels (the 3-channel
  * first layer of an image net), group 1, dilation_w 1, zero border value.  The input is quantised into an image of 4 bytes

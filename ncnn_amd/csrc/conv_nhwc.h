@@ -65,7 +65,10 @@ constexpr size_t SPLIT_COUNTER_BYTES = SPLIT_MAX_TILES * sizeof(unsigned);
 // int32 words of workspace (counters included) the pipelined kernel wants for this problem (0: it does not split)
 size_t conv_nhwc_pipelined_workspace_words(int cout, long long npix, int steps);
 
-// Launches the pipelined kernel; the caller has checked: zero border byte, channels-last output.
+// The kernel launch_conv_nhwc_pipelined takes, and its form
+void conv_nhwc_pipelined_route(const NhwcGeom& g, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, ncnnhip_conv_route& route);
+
+// Launches the pipelined kernel, or the more special one that fits; the caller has checked: zero border byte, channels-last output.
 int launch_conv_nhwc_pipelined(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
                                void* workspace, size_t workspace_bytes, hipStream_t stream);
 
@@ -96,7 +99,7 @@ int launch_conv_pointwise(const NhwcGeom& g, const int8_t* wpk, const int8_t* x,
 // The kernel for few output tiles (conv_stream.hip: K split over the wavefronts of tiles of 16 x 16 to 32 x 32, no workspace): does this
 // problem belong to it (int8 blob), and its launch.  conv_patch_pays leaves such layers to it; the pipelined launch asks after the
 // pointwise and weights-resident kernels, which want many pixels.
-bool conv_stream_fits(const NhwcGeom& g, bool fp32_out);
+int conv_stream_tile(const NhwcGeom& g, bool fp32_out); // 0: it does not, else pixels / 16 * 10 + channels / 16
 int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream);
 
 // The same two kernels with a projection shortcut (g: the main 1x1 convolution, stride 1, unpadded, channels in whole steps).

@@ -787,6 +787,32 @@ int ncnnhip_conv_small_tile_selected(const ncnnhip_conv_desc* desc, int elemsize
     return conv_patch_pays(nhwc_geometry(*desc, outw, outh, npix), desc->batch, elemsize) ? 1 : 0;
 }
 
+int ncnnhip_conv_int8_nhwc_route(const ncnnhip_conv_desc* desc, ncnnhip_activation act, int int8_out, const ncnnhip_conv_fusion* fusion, ncnnhip_conv_route* route)
+{
+    NCNNHIP_REQUIRE(desc && route && desc->group == 1, "ncnnhip_conv_int8_nhwc_route: null pointer, or a grouped layer");
+    int outw = 0, outh = 0;
+    const int ret = ncnnhip_conv_out_shape(desc, &outw, &outh);
+    if (ret) return ret;
+    const long long plane = (long long)outw * outh, npix = plane * desc->batch;
+    NCNNHIP_REQUIRE(npix < (1ll << 31) && (long long)desc->h * desc->w * padded_channels(desc->c) < (1ll << 31), "ncnnhip_conv_int8_nhwc_route: layer too large");
+    const NhwcGeom g = nhwc_geometry(*desc, outw, outh, npix);
+    *route = {g.pad_word ? NCNNHIP_CONV_GENERAL : NCNNHIP_CONV_SMALL_TILE, 0, 0, 0, 0, 0};
+    if (g.pad_word || conv_patch_pays(g, desc->batch, 1)) return NCNNHIP_OK;
+    float* const some = reinterpret_cast<float*>(16); // an aligned buffer
+    ConvEpilogue epi = {};
+    epi.scale_in = some;
+    epi.scale_out = int8_out ? some : 0;
+    epi.act = act;
+    epi.out = some;
+    epi.pix_per_img = (int)plane;
+    epi.batch = desc->batch;
+    epi.num_output = desc->num_output;
+    ConvFusion f = {0, 0, 0, 0.f};
+    if (fusion) f = {fusion->residual_dev ? some : 0, fusion->relu_after, fusion->quantised_out_dev ? reinterpret_cast<int8_t*>(some) : 0, fusion->quantise_scale};
+    conv_nhwc_pipelined_route(g, epi, f, padded_channels(desc->num_output), *route);
+    return NCNNHIP_OK;
+}
+
 int ncnnhip_conv_from_float_workspace_bytes(const ncnnhip_conv_desc* desc, size_t* workspace_bytes)
 {
     NCNNHIP_REQUIRE(workspace_bytes, "ncnnhip_conv_from_float_workspace_bytes: null pointer");

@@ -85,13 +85,16 @@ size_t conv_nhwc_pipelined_workspace_words(int cout, long long npix, int steps)
     return SPLIT_COUNTER_BYTES / sizeof(int32_t) + (size_t)p.splits * p.tiles_m * p.tiles_n * p.bm * p.bn;
 }
 
-int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
-                               void* workspace, size_t workspace_bytes, hipStream_t stream)
+static int special_kernel(const NhwcGeom& g, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp)
 {
-    if (conv_pointwise_fits(g_in, epi, fusion, out_cp) || conv_pointwise_stem_fits(g_in, epi, fusion, out_cp)) return launch_conv_pointwise(g_in, wpk, x, epi, out_cp, stream);
-    if (conv_resident_fits(g_in, epi, fusion, out_cp)) return launch_conv_resident(g_in, wpk, x, epi, fusion, out_cp, stream);
-    if (conv_stream_fits(g_in, !epi.scale_out)) return launch_conv_stream(g_in, wpk, x, epi, fusion, out_cp, stream);
-    NhwcGeom g = g_in;
+    if (conv_pointwise_fits(g, epi, fusion, out_cp) || conv_pointwise_stem_fits(g, epi, fusion, out_cp)) return NCNNHIP_CONV_POINTWISE;
+    if (conv_resident_fits(g, epi, fusion, out_cp)) return NCNNHIP_CONV_RESIDENT;
+    return conv_stream_tile(g, !epi.scale_out) ? NCNNHIP_CONV_FEW_TILES : NCNNHIP_CONV_PIPELINED;
+}
+
+// the pipelined kernel's plan and addressing mode (its MODE), the layer as it sees it in g
+static int pipelined_form(NhwcGeom& g, PipePlan& p)
+{
     // A 1x1, stride-1, unpadded layer reads input pixel n for output pixel n, whatever the image shape: present it as
     // one row of npix pixels, and the kernel skips the pixel -> (image, y, x) divisions.
     const int dense = g.kw == 1 && g.kh == 1 && g.sw == 1 && g.sh == 1 && g.pad_top == 0 && g.pad_left == 0 && g.outw == g.W && g.outh == g.H && g.tapK == g.Cp;
@@ -100,7 +103,7 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
         g.H = g.outh = 1;
         g.W = g.outw = g.npix;
     }
-    PipePlan p = plan_pipelined_groups(g.cout, g.npix, g.K / 64);
+    p = plan_pipelined_groups(g.cout, g.npix, g.K / 64);
     // the narrow-input first layer has four K steps at most: from a million output pixels up, 128-pixel tiles halve the number of
     // workgroup prologues (ResNet-50's 7 x 7 first layer at batch 128: the pass 2.22 -> 2.20 ms; at batch 16, 0.2 M pixels, no gain)
     if ((g.tapK == 16 || g.tapK == 32) && p.splits == 1 && p.bm == 64 && g.npix >= (1 << 20))
@@ -108,6 +111,41 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
         p.bm = 128;
         p.tiles_m = ceil_div(g.npix, 128);
     }
+    // (the K-split kernels exist for modes 0, 1 and 3 only: a narrow-input layer has too few K steps to be split)
+    return dense ? 1 : (p.groups == 1 && (g.tapK == 16 || g.tapK == 32) && p.splits == 1) ? 2 : (g.tapK % 64 == 0 && g.tapK == g.Cp) ? 3 : 0;
+}
+
+void conv_nhwc_pipelined_route(const NhwcGeom& g_in, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, ncnnhip_conv_route& route)
+{
+    route = {special_kernel(g_in, epi, fusion, out_cp), 0, 0, 0, 0, 0};
+    if (route.kernel == NCNNHIP_CONV_FEW_TILES)
+    {
+        const int tile = conv_stream_tile(g_in, !epi.scale_out);
+        route.tile_pixels = tile / 10 * 16;
+        route.tile_channels = tile % 10 * 16;
+    }
+    if (route.kernel != NCNNHIP_CONV_PIPELINED) return;
+    NhwcGeom g = g_in;
+    PipePlan p;
+    const int mode = pipelined_form(g, p);
+    route = {NCNNHIP_CONV_PIPELINED, p.bm, p.bn, mode, p.groups, p.splits};
+}
+
+int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
+                               void* workspace, size_t workspace_bytes, hipStream_t stream)
+{
+    switch (special_kernel(g_in, epi, fusion, out_cp))
+    {
+    case NCNNHIP_CONV_POINTWISE:
+        return launch_conv_pointwise(g_in, wpk, x, epi, out_cp, stream);
+    case NCNNHIP_CONV_RESIDENT:
+        return launch_conv_resident(g_in, wpk, x, epi, fusion, out_cp, stream);
+    case NCNNHIP_CONV_FEW_TILES:
+        return launch_conv_stream(g_in, wpk, x, epi, fusion, out_cp, stream);
+    }
+    NhwcGeom g = g_in;
+    PipePlan p;
+    const int mode = pipelined_form(g, p);
     const long long blocks = (long long)p.tiles_m * p.tiles_n * p.splits;
     NCNNHIP_REQUIRE(blocks < (1ll << 31) && blocks * p.tiles_n < (1ll << 32), "convolution: too many tiles");
     int32_t* partial = 0;
@@ -120,9 +158,6 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
         partial = (int32_t*)((char*)workspace + SPLIT_COUNTER_BYTES);
     }
     dim3 grid((unsigned)blocks), block((unsigned)(256 * p.groups));
-    // addressing mode (the kernel's MODE); the K-split kernels exist for modes 0, 1 and 3 only (a narrow-input layer has
-    // too few K steps to be split)
-    const int mode = dense ? 1 : (p.groups == 1 && (g.tapK == 16 || g.tapK == 32) && p.splits == 1) ? 2 : (g.tapK % 64 == 0 && g.tapK == g.Cp) ? 3 : 0;
     if (p.splits > 1) return launch_pipe_split(p, mode, wpk, x, g, epi, fusion, out_cp, out_cp, partial, counters, stream);
 #define LAUNCH_PIPE_MODE(BM_, BN_, MODE_, GROUPS_)                                                                                                                 \
     hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<BM_, BN_, PIPE_RING, false, MODE_, 1, GROUPS_>), grid, block, 0, stream, wpk, x, g, epi, fusion, out_cp, \

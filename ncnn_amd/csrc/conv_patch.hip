@@ -415,7 +415,7 @@ bool conv_patch_pays(const NhwcGeom& g, int batch, int x_elemsize)
     // longer K (3x3 256 -> 256 on 14 x 14 8.4 -> 11.7: 36 dependent steps per wavefront) and on int8 1x1 layers (nothing
     // to share, 4.5 -> 5.7).
     // (What the kernel for few tiles takes of the int8 layers is ahead of both: 3x3 128 -> 128 on 28 x 28 4.4, 64 -> 64 on 56 x 56 4.3 -> 4.2 in a chain.)
-    if (x_elemsize == 1 && conv_stream_fits(g, false)) return false;
+    if (x_elemsize == 1 && conv_stream_tile(g, false)) return false;
     const long long tiles64 = (long long)ceil_div(g.npix, 64) * ceil_div(g.cout, 64);
     return tiles64 < 128 && (pl.nsteps + 1) / 2 <= 18 && (x_elemsize != 1 || g.ntaps > 1);
 }

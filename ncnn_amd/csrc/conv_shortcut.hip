@@ -10,7 +10,7 @@ namespace ncnnhip {
 int launch_conv_shortcut(const NhwcGeom& g_in, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
                          hipStream_t stream)
 {
-    if (conv_stream_fits(g_in, true)) return launch_conv_stream_shortcut(g_in, wpk, x, sc, epi, fusion, out_cp, stream);
+    if (conv_stream_tile(g_in, true)) return launch_conv_stream_shortcut(g_in, wpk, x, sc, epi, fusion, out_cp, stream);
     NhwcGeom g = g_in;
     g.H = g.outh = 1;
     g.W = g.outw = g.npix;

@@ -291,9 +291,9 @@ static bool stream_dense(const NhwcGeom& g)
 //   1x1 960 -> 160 on 7 x 7, fp32 out 5.0 / 3.4 / 3.6 / 4.0, 32 images 6.0 / 6.7 / 5.1 / 4.6    1x1 64 -> 384 on 14 x 14 3.0 / 2.9 / 2.9 / 3.2
 // With 32 x 32 tiles the ring is level or ahead at both ends of K: int8 out 1x1 64 -> 64 on 56 x 56 3.0 / 3.2, 256 -> 64 3.6 / 3.9, 3x3 512 -> 512 on 7 x 7,
 // eight images 10.7 / 11.0 (four, 16 x 32 tiles: 10.2 / 9.2); fp32 out is ahead from three steps on (144 -> 32 on 28 x 28, eight images 4.2 / 3.6).
-// 0: none, else pixels / 16 * 10 + channels / 16.
-static int stream_tile(const NhwcGeom& g, bool fp32_out)
+int conv_stream_tile(const NhwcGeom& g, bool fp32_out)
 {
+    if (!stream_dense(g) && !(g.tapK % 64 == 0 && g.tapK == g.Cp)) return 0;
     const int steps = g.K / 64;
     const long long m16 = ceil_div(g.npix, 16), m32 = ceil_div(g.npix, 32), n16 = ceil_div(g.cout, 16), n32 = ceil_div(g.cout, 32);
     if (m16 * n16 <= 256) return 11;
@@ -301,15 +301,9 @@ static int stream_tile(const NhwcGeom& g, bool fp32_out)
     return m32 * n32 <= 256 && steps >= (fp32_out ? 2 : 5) && steps <= 48 ? 22 : 0;
 }
 
-bool conv_stream_fits(const NhwcGeom& g, bool fp32_out)
-{
-    if (!stream_dense(g) && !(g.tapK % 64 == 0 && g.tapK == g.Cp)) return false;
-    return stream_tile(g, fp32_out) != 0;
-}
-
 int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream)
 {
-    const int tile = stream_tile(g, !epi.scale_out), tp = tile / 10, tc = tile % 10;
+    const int tile = conv_stream_tile(g, !epi.scale_out), tp = tile / 10, tc = tile % 10;
     NCNNHIP_REQUIRE(tile && !epi.acc_out, "convolution: this layer does not fit the kernel for few tiles");
     const int tiles_m = ceil_div(g.npix, 16 * tp), tiles_n = ceil_div(g.cout, 16 * tc), blocks = tiles_m * tiles_n; // 256 at most
     const unsigned magic_m = tiles_m > 1 ? (unsigned)((1ull << 32) / (unsigned)tiles_m + 1) : 0u;
@@ -341,7 +335,7 @@ int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, co
 int launch_conv_stream_shortcut(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion,
                                 int out_cp, hipStream_t stream)
 {
-    const int tile = stream_tile(g, true), tp = tile / 10, tc = tile % 10;
+    const int tile = conv_stream_tile(g, true), tp = tile / 10, tc = tile % 10;
     NCNNHIP_REQUIRE(tile && stream_dense(g) && g.K == g.Cp && sc.Cp % 64 == 0, "convolution: this layer does not fit the kernel for few tiles");
     const int tiles_m = ceil_div(g.npix, 16 * tp), tiles_n = ceil_div(g.cout, 16 * tc);
     const unsigned magic_m = tiles_m > 1 ? (unsigned)((1ull << 32) / (unsigned)tiles_m + 1) : 0u;

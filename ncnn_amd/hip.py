@@ -40,6 +40,11 @@ class ConvShortcut(C.Structure):
                 ("act", Activation)]
 
 
+class ConvRoute(C.Structure):
+    _fields_ = [(n, C.c_int) for n in ("kernel", "tile_pixels", "tile_channels", "addressing", "groups", "splits")]
+    GENERAL, SMALL_TILE, POINTWISE, RESIDENT, FEW_TILES, PIPELINED = range(6)
+
+
 class PoolDesc(C.Structure):
     _fields_ = [(n, C.c_int) for n in ("w", "h", "c", "batch", "pooling_type", "kernel_w", "kernel_h", "stride_w", "stride_h", "pad_top", "pad_left",
                                        "outw", "outh", "global_pooling", "avgpool_count_include_pad", "count_x0", "count_x1", "count_y0", "count_y1")]
@@ -108,6 +113,7 @@ _SIGNATURES = {
     "ncnnhip_conv_shortcut_supported": [C.POINTER(ConvDesc), C.POINTER(ConvDesc), C.POINTER(C.c_int)],
     "ncnnhip_conv_int8_nhwc_tail": [C.POINTER(ConvDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, Activation, C.POINTER(ConvShortcut), C.c_void_p,
                                     C.POINTER(ConvFusion), C.c_void_p, C.c_size_t, C.c_void_p],
+    "ncnnhip_conv_int8_nhwc_route": [C.POINTER(ConvDesc), Activation, C.c_int, C.POINTER(ConvFusion), C.POINTER(ConvRoute)],
     "ncnnhip_conv_resolved_pads": [C.POINTER(ConvDesc), C.POINTER(C.c_int), C.POINTER(C.c_int)],
     "ncnnhip_padded_channels": [C.c_int],
     "ncnnhip_chw_to_nhwc": [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_size_t, C.c_size_t, C.c_void_p, C.c_void_p],

@@ -97,3 +97,14 @@ MHA_CASES = [
     (8, 64, 2, 64, 64, 64, 1, 1, 8, 64, False, 300, True, None),   # decode steps on a long cache: the few-query attention kernels
     (9, 96, 4, 96, 96, 96, 3, 3, 8, 32, False, 401, True, "2d"),
 ]
+
+
+def conv_route(batch, c, h, w, outc, kernel, dilation=(1, 1), stride=(1, 1), pads=(0, 0, 0, 0), act=0, act_params=(0.0, 0.0), int8_out=False, fused=False):
+    """The kernel and form a channels-last layer with an int8 blob is launched as (hip.ConvRoute), asked of the dispatch itself."""
+    import ctypes as C
+
+    from ncnn_amd.hip import Activation, ConvDesc, ConvFusion, ConvRoute, check, lib
+    d = ConvDesc(w, h, c, batch, outc, kernel[0], kernel[1], dilation[0], dilation[1], stride[0], stride[1], pads[0], pads[1], pads[2], pads[3], 0.0, 1)
+    fusion, route = ConvFusion(C.c_void_p(16), 1, C.c_void_p(16), 1.0), ConvRoute()
+    check(lib().ncnnhip_conv_int8_nhwc_route(C.byref(d), Activation.make(act, act_params), int(int8_out), C.byref(fusion) if fused else None, C.byref(route)))
+    return route

@@ -1,0 +1,40 @@
+"""Which kernel and form a channels-last convolution takes: the dispatch's own answer (ncnnhip_conv_int8_nhwc_route), no GPU needed."""
+import ctypes as C
+
+import pytest
+
+import cases
+
+SAME3 = dict(pads=(1, 1, 1, 1))
+
+
+@pytest.mark.parametrize("shape,options,kernel", [
+    ((1, 512, 7, 7, 512, (3, 3)), SAME3, "FEW_TILES"),
+    ((5, 512, 7, 8, 512, (3, 3)), SAME3, "PIPELINED"),
+    ((1, 288, 12, 12, 160, (3, 3)), SAME3, "PIPELINED"),
+    ((16, 64, 56, 56, 64, (3, 3)), SAME3, "RESIDENT"),
+    ((32, 16, 112, 112, 96, (1, 1)), dict(int8_out=True), "POINTWISE"),
+    ((32, 16, 112, 112, 96, (1, 1)), dict(int8_out=False), "PIPELINED"),
+    ((2, 64, 45, 46, 64, (3, 3)), SAME3, "SMALL_TILE"),
+    ((1, 256, 56, 56, 64, (1, 1)), dict(fused=True), "FEW_TILES"),
+], ids=str)
+def test_kernel_of_a_layer(shape, options, kernel):
+    r = cases.conv_route(*shape, **options)
+    assert r.kernel == getattr(r, kernel)
+
+
+def test_forms_of_the_pipelined_kernel():
+    r = cases.conv_route(5, 512, 7, 8, 512, (3, 3), **SAME3)
+    assert (r.tile_pixels, r.tile_channels, r.addressing, r.groups, r.splits) == (64, 64, 3, 4, 3)
+    r = cases.conv_route(1, 288, 12, 12, 160, (3, 3), **SAME3)  # K split over workgroups of one group
+    assert (r.addressing, r.groups, r.splits) == (0, 1, 3)
+
+
+def test_layers_that_are_refused():
+    from ncnn_amd.hip import Activation, ConvDesc, ConvRoute, lib
+    r, act = ConvRoute(), Activation.make(0, (0.0, 0.0))
+    border = ConvDesc(8, 8, 64, 1, 64, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 1.0, 1)
+    assert lib().ncnnhip_conv_int8_nhwc_route(C.byref(border), act, 0, None, C.byref(r)) == 0 and r.kernel == r.GENERAL
+    grouped = ConvDesc(8, 8, 64, 1, 64, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 0.0, 2)
+    assert lib().ncnnhip_conv_int8_nhwc_route(C.byref(grouped), act, 0, None, C.byref(r)) != 0
+    assert lib().ncnnhip_conv_int8_nhwc_route(None, act, 0, None, C.byref(r)) != 0

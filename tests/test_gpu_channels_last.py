@@ -57,7 +57,8 @@ CONV_CASES = [
     (16, 20, 20, 130, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
     (64, 14, 14, 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),
     (96, 7, 7, 200, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0)),
-    (512, 7, 7, 72, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),   # K split over workgroups
+    (512, 7, 7, 72, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),   # K split over the wavefronts of small tiles
+    (288, 12, 12, 160, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)),   # over workgroups of four wavefronts (steps that meet several taps)
     (32, 150, 150, 136, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0)),  # 128-row tiles with a ragged last tile
 ]
 

@@ -36,24 +36,25 @@ def _two_streams():
 
 
 def test_k_split_convolution_200_launches_on_two_streams(rt):
-    c, hw, outc = 512, 7, 512
-    x, wq, b, ws, ins, tops = cases.conv_case(77, c, hw, hw, outc, (3, 3), 1, 1, True, True)
-    d = oracle.make_desc((c, hw, hw), outc, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 0.0, 1, 1, 1, 1, (0.0, 0.0))
-    want = oracle.convolution_int8(d, x[0], wq, b, ws, ins[0], None)            # [outc][h][w] fp32
-    want_cl = np.ascontiguousarray(want.reshape(outc, hw * hw).T)               # channels-last, outc is a multiple of 16
+    batch, c, h, w, outc = 5, 512, 7, 8, 512  # 40 tiles of 64 x 64, three splits
+    route = cases.conv_route(batch, c, h, w, outc, (3, 3), pads=(1, 1, 1, 1), act=1)
+    assert route.kernel == route.PIPELINED and route.splits == 3
+    x, wq, b, ws, ins, tops = cases.conv_case(77, c, h, w, outc, (3, 3), 1, 1, True, True, batch=batch)
+    d = oracle.make_desc((c, h, w), outc, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 0.0, 1, 1, 1, 1, (0.0, 0.0))
+    want = np.stack([oracle.convolution_int8(d, x[i], wq, b, ws, ins[0], None) for i in range(batch)])  # [n][outc][h][w] fp32
+    want_cl = np.ascontiguousarray(want.reshape(batch, outc, h * w).transpose(0, 2, 1)).reshape(-1, outc)  # channels-last, outc is a multiple of 16
 
-    desc = ConvDesc(hw, hw, c, 1, outc, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 0.0, 1)
+    desc = ConvDesc(w, h, c, batch, outc, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 0.0, 1)
     nb, wb, sb = C.c_size_t(), C.c_size_t(), C.c_size_t()
     check(lib().ncnnhip_conv_nhwc_sizes(C.byref(desc), C.byref(nb), C.byref(wb), C.byref(sb)))
-    assert sb.value > 0, "this shape is meant to take the K-split path"
-    src = rt.to_channels_last(x[0])                                              # int8 [1][49][512]
+    src = rt.to_channels_last(x)                                                 # int8 [5][56][512]
     pk = np.empty(wb.value, np.int8)
     check(lib().ncnnhip_conv_pack_weights(C.byref(desc), np.ascontiguousarray(wq, np.int8).ctypes.data, pk.ctypes.data))
     dpk, dsi, db = rt.up(pk), rt.up(rt.fold_input_scales(ws, ins, outc)), rt.up(np.asarray(b, F))
     rt.sync()
-    out_bytes = hw * hw * outc * 4
+    out_bytes = want_cl.nbytes
     streams = _two_streams()
-    outs = [DeviceBuffer.empty((ROUNDS, hw * hw, outc), F) for _ in streams]
+    outs = [DeviceBuffer.empty((ROUNDS,) + want_cl.shape, F) for _ in streams]
     wss = [DeviceBuffer.zeros(sb.value, s) for s in streams]                    # one workspace per stream: calls that share one race
     act = Activation.make(1, (0.0, 0.0))
     try:
