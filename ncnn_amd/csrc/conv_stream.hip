@@ -290,14 +290,20 @@ static bool stream_dense(const NhwcGeom& g)
 //   3x3 512 -> 512 on 7 x 7 9.9 / 7.0 / 9.2 / 10.7    3x3 128 -> 128 on 28 x 28 6.9 / 5.4 / 4.4 / 5.2    1x1 256 -> 1024 on 14 x 14, fp32 out 5.0 / 6.0 / 4.5 / 4.1
 //   1x1 960 -> 160 on 7 x 7, fp32 out 5.0 / 3.4 / 3.6 / 4.0, 32 images 6.0 / 6.7 / 5.1 / 4.6    1x1 64 -> 384 on 14 x 14 3.0 / 2.9 / 2.9 / 3.2
 // With 32 x 32 tiles the ring is level or ahead at both ends of K: int8 out 1x1 64 -> 64 on 56 x 56 3.0 / 3.2, 256 -> 64 3.6 / 3.9, 3x3 512 -> 512 on 7 x 7,
-// eight images 10.7 / 11.0 (four, 16 x 32 tiles: 10.2 / 9.2); fp32 out is ahead from three steps on (144 -> 32 on 28 x 28, eight images 4.2 / 3.6).
+// eight images 10.7 / 11.0 (four, 16 x 32 tiles: 10.2 / 9.2); fp32 out is ahead from two steps on (128 -> 64 on 56 x 56 3.34 / 3.21, 192 -> 64 3.52 / 3.31,
+// 256 -> 64 level, 3.68 / 3.71).
+// Beyond some K the ring, which splits it over workgroups, is quicker again.  The ring / here, fp32 out (steps: 64 of K): 16 x 16 tiles 192 steps 13.2 / 13.0 with
+// 4 tiles, 18.1 / 13.4 with 208; 208 steps 13.5 / 14.4 and 18.5 / 14.8;
+// 288 steps 16.8 / 18.2 with 4, 20.8 / 19.2 with 128, 19.4 / 19.0 with 208; 400 steps 20.1 / 24.7 and 21.2 / 25.8.  16 x 32 tiles 64 steps 9.4 / 8.2 (512 channels
+// on 14 x 14), 3x3 512 -> 512 (72) 9.8 / 9.2, 3x3 576 -> 512 (81) 10.3 / 7.6, 3x3 640 -> 512 (90) 10.7 / 10.4 (160 channels on 28 x 28, 80 steps: 9.6 / 9.8);
+// 96 steps 10.4 / 11.0, 144 12.7 / 15.6, 400 18.9 / 36.6.
 int conv_stream_tile(const NhwcGeom& g, bool fp32_out)
 {
     if (!stream_dense(g) && !(g.tapK % 64 == 0 && g.tapK == g.Cp)) return 0;
     const int steps = g.K / 64;
     const long long m16 = ceil_div(g.npix, 16), m32 = ceil_div(g.npix, 32), n16 = ceil_div(g.cout, 16), n32 = ceil_div(g.cout, 32);
-    if (m16 * n16 <= 256) return 11;
-    if (m16 * n32 <= 256) return 12;
+    if (m16 * n16 <= 256) return steps <= (m16 * n16 >= 128 ? 288 : 192) ? 11 : 0;
+    if (m16 * n32 <= 256) return steps <= 90 ? 12 : 0;
     return m32 * n32 <= 256 && steps >= (fp32_out ? 2 : 5) && steps <= 48 ? 22 : 0;
 }
 

@@ -38,3 +38,13 @@ def test_layers_that_are_refused():
     grouped = ConvDesc(8, 8, 64, 1, 64, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 0.0, 2)
     assert lib().ncnnhip_conv_int8_nhwc_route(C.byref(grouped), act, 0, None, C.byref(r)) != 0
     assert lib().ncnnhip_conv_int8_nhwc_route(None, act, 0, None, C.byref(r)) != 0
+
+
+@pytest.mark.parametrize("hw,outc,tile,longest", [((4, 4), 64, (16, 16), 192), ((14, 14), 256, (16, 16), 288), ((7, 7), 496, (16, 16), 192), ((14, 14), 512, (16, 32), 90), ((28, 28), 160, (16, 32), 90),
+                                                  ((28, 28), 256, (32, 32), 48)], ids=str)
+def test_few_tiles_of_a_long_k_are_left_to_k_splits(hw, outc, tile, longest):
+    r = cases.conv_route(1, 64 * longest, *hw, outc, (1, 1))
+    assert (r.kernel, r.tile_pixels, r.tile_channels) == (r.FEW_TILES,) + tile
+    for steps in (longest + 1, 400):
+        r = cases.conv_route(1, 64 * steps, *hw, outc, (1, 1))
+        assert r.kernel == r.PIPELINED and r.splits > 1
