@@ -35,7 +35,9 @@ PipePlan plan_pipelined(int cout, long long npix, int steps)
         // tile adds them up): with 8 steps each, the 16-step 1x1 layers 1024 -> 256 of ResNet-50 ran 8.6 us in two halves
         // and 6.8 whole at batch 16, the 18-step 3x3 layers 128 -> 128 9.6 and 7.5 at batch 8; summed over a pass the
         // kernels take 350 / 355 / 362 / 385 us at batch 1 with at least 8 / 12 / 16 / 24 steps, 404 / 389 / 395 / 414
-        // at batch 4, 459 / 449 / 446 / 466 at batch 8, 568 / 555 / 556 / 565 at batch 16 (MobileNetV2: no difference)
+        // at batch 4, 459 / 449 / 446 / 466 at batch 8, 568 / 555 / 556 / 565 at batch 16 (MobileNetV2: no difference).
+        // (The int8 layers of those passes with few small tiles have gone to conv_stream_kernel since; here still come InnerProduct,
+        // the loader of fp32 and fp16 blobs, taps that are no whole steps, a K too long for that kernel, and more tiles than it takes.)
         const int want = (int)((256 + t - 1) / t);
         const int max_splits = steps / SPLIT_MIN_STEPS;
         p.splits = want < max_splits ? want : max_splits;
@@ -55,13 +57,14 @@ PipePlan plan_pipelined_groups(int cout, long long npix, int steps)
     //   1x1 1024 -> 256 on 14x14: batch 1 6.3 -> 5.6, batch 16 6.5 -> 5.9    1x1 2048 -> 512 on 7x7: 8.2 -> 7.2, batch 16 9.3 -> 7.4
     //   1x1 960 -> 160 on 7x7 6.0 -> 5.2    3x3 256 -> 256 on 14x14, batch 16 11.4 -> 8.7    3x3 512 -> 512 on 7x7, batch 16 12.7 -> 11.5
     // Eight wavefronts gain about half of that.  The lines, from 1x1 and 3x3 layers of 8 to 100 steps on 2 to 441 tiles:
+    // (of these the batch-1 layers and 960 -> 160 run on conv_stream_kernel by now.)
     //   beyond 256 tiles two of them share a unit and sixteen lose: 24 steps, 196 tiles 10.1 -> 7.2, 320 tiles 9.1 -> 12.2; 72 steps
     //   196 tiles 16.2 -> 13.5, 320 tiles 20.9 -> 24.6;
     //   with 8 and 9 steps they are up to 3 % slower alone (75 tiles 4.76 -> 4.84 and 4.94 -> 5.05), from 11 on faster (5.55 -> 5.42 at
     //   12); the nets' passes, which have those layers too, were no slower with them.
     if (p.bm != 64 || p.bn != 64 || steps < 8 || t > 256) return p;
     // A few tiles of a long K want other compute units more than wavefronts of their own.  Four wavefronts in splits / sixteen in one:
-    // 3x3 of 36 steps 16 tiles 8.2 / 8.5, 52 tiles 8.9 / 8.7; 45 steps 20 tiles 8.8 / 9.6.  (From 72 steps on three splits of sixteen
+    // (InnerProduct, steps that meet several taps, a K beyond conv_stream_kernel's) 3x3 of 36 steps 16 tiles 8.2 / 8.5, 52 tiles 8.9 / 8.7; 45 steps 20 tiles 8.8 / 9.6.  (From 72 steps on three splits of sixteen
     // would be better still: 20 tiles 10.4 -> 10.1, 1x1 of 100 steps 12.0 -> 10.4.)
     if (p.splits >= 3 && t < 24) return p;
     p.groups = 4;
