@@ -186,7 +186,8 @@ int ncnnhip_conv_int8_nhwc_fused(const ncnnhip_conv_desc* desc, const int8_t* nh
 /* ncnnhip_conv_int8_nhwc_fused with two more choices for the end of a residual block, results unchanged:
  *   shortcut (or NULL)  the residual is itself a 1x1 convolution of this output's shape, any stride (its own Convolution::forward_int8,
  *                       src/layer/convolution.cpp:383-508): computed in the same launch, its fp32 blob is never written.  For
- *                       pairs that ncnnhip_conv_shortcut_supported accepts; fusion->residual_dev must be NULL then.
+ *                       pairs that ncnnhip_conv_shortcut_supported accepts; fusion->residual_dev must be NULL then.  Whether that is quicker than the
+ *                       two convolutions one after the other is what ncnnhip_conv_shortcut_pays answers (0 for pairs not supported).
  *   out_dev NULL        only the quantised copy is written (every consumer reads that). */
 typedef struct ncnnhip_conv_shortcut
 {
@@ -198,6 +199,7 @@ typedef struct ncnnhip_conv_shortcut
     ncnnhip_activation act;
 } ncnnhip_conv_shortcut;
 int ncnnhip_conv_shortcut_supported(const ncnnhip_conv_desc* desc, const ncnnhip_conv_desc* shortcut, int* supported);
+int ncnnhip_conv_shortcut_pays(const ncnnhip_conv_desc* desc, const ncnnhip_conv_desc* shortcut, int* pays);
 int ncnnhip_conv_int8_nhwc_tail(const ncnnhip_conv_desc* desc, const int8_t* nhwc_dev, const int8_t* packed_weight_dev,
                                 const float* scale_in_dev, const float* bias_dev, ncnnhip_activation act,
                                 const ncnnhip_conv_shortcut* shortcut, float* out_dev, const ncnnhip_conv_fusion* fusion,

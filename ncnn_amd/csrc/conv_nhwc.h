@@ -103,6 +103,9 @@ int conv_stream_tile(const NhwcGeom& g, bool fp32_out); // 0: it does not, else 
 int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream);
 
 // The same two kernels with a projection shortcut (g: the main 1x1 convolution, stride 1, unpadded, channels in whole steps).
+// conv_shortcut_pays: one launch is quicker than the two convolutions one after the other.
+bool conv_shortcut_pays(const NhwcGeom& g, int shortcut_steps);
+int conv_stream_shortcut_tile(const NhwcGeom& g, int shortcut_steps);
 int launch_conv_shortcut(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
                          hipStream_t stream);
 int launch_conv_stream_shortcut(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion,

@@ -722,6 +722,18 @@ int ncnnhip_conv_shortcut_supported(const ncnnhip_conv_desc* desc, const ncnnhip
     return NCNNHIP_OK;
 }
 
+int ncnnhip_conv_shortcut_pays(const ncnnhip_conv_desc* desc, const ncnnhip_conv_desc* shortcut, int* pays)
+{
+    NCNNHIP_REQUIRE(desc && shortcut && pays, "ncnnhip_conv_shortcut_pays: null pointer");
+    *pays = 0;
+    if (!shortcut_supported(*desc, *shortcut)) return NCNNHIP_OK;
+    int outw = 0, outh = 0;
+    const int ret = ncnnhip_conv_out_shape(desc, &outw, &outh);
+    if (ret) return ret;
+    *pays = conv_shortcut_pays(nhwc_geometry(*desc, outw, outh, (long long)outw * outh * desc->batch), padded_channels(shortcut->c) / 64) ? 1 : 0;
+    return NCNNHIP_OK;
+}
+
 int ncnnhip_conv_int8_nhwc_tail(const ncnnhip_conv_desc* desc, const int8_t* nhwc_dev, const int8_t* packed_weight_dev, const float* scale_in_dev,
                                 const float* bias_dev, ncnnhip_activation act, const ncnnhip_conv_shortcut* shortcut, float* out_dev,
                                 const ncnnhip_conv_fusion* fusion, void* workspace_dev, size_t workspace_bytes, void* stream)

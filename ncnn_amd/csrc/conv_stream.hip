@@ -297,14 +297,27 @@ static bool stream_dense(const NhwcGeom& g)
 // 288 steps 16.8 / 18.2 with 4, 20.8 / 19.2 with 128, 19.4 / 19.0 with 208; 400 steps 20.1 / 24.7 and 21.2 / 25.8.  16 x 32 tiles 64 steps 9.4 / 8.2 (512 channels
 // on 14 x 14), 3x3 512 -> 512 (72) 9.8 / 9.2, 3x3 576 -> 512 (81) 10.3 / 7.6, 3x3 640 -> 512 (90) 10.7 / 10.4 (160 channels on 28 x 28, 80 steps: 9.6 / 9.8);
 // 96 steps 10.4 / 11.0, 144 12.7 / 15.6, 400 18.9 / 36.6.
+static int stream_tile(const NhwcGeom& g, int steps, bool fp32_out, int convolutions)
+{
+    const long long m16 = ceil_div(g.npix, 16), m32 = ceil_div(g.npix, 32), n16 = ceil_div(g.cout, 16), n32 = ceil_div(g.cout, 32);
+    if (m16 * n16 <= 256) return steps <= convolutions * (m16 * n16 >= 128 ? 288 : 192) ? 11 : 0;
+    if (m16 * n32 <= 256) return steps <= convolutions * 90 ? 12 : 0;
+    return m32 * n32 <= 256 && steps >= (fp32_out ? 2 : 5) && steps <= convolutions * 48 ? 22 : 0;
+}
+
 int conv_stream_tile(const NhwcGeom& g, bool fp32_out)
 {
     if (!stream_dense(g) && !(g.tapK % 64 == 0 && g.tapK == g.Cp)) return 0;
-    const int steps = g.K / 64;
-    const long long m16 = ceil_div(g.npix, 16), m32 = ceil_div(g.npix, 32), n16 = ceil_div(g.cout, 16), n32 = ceil_div(g.cout, 32);
-    if (m16 * n16 <= 256) return steps <= (m16 * n16 >= 128 ? 288 : 192) ? 11 : 0;
-    if (m16 * n32 <= 256) return steps <= 90 ? 12 : 0;
-    return m32 * n32 <= 256 && steps >= (fp32_out ? 2 : 5) && steps <= 48 ? 22 : 0;
+    return stream_tile(g, g.K / 64, fp32_out, 1);
+}
+
+// With a shortcut a workgroup walks both K, one after the other, in place of two launches that walk one each: the limits hold for the two together.
+// us, two launches / one, main + shortcut steps: 512 channels on 7 x 7 (16 x 16 tiles) 8 + 16 7.6 / 5.8, 64 + 64 13.6 / 11.7, 100 + 100 18.4 / 16.3; 2048 channels
+// there (16 x 32) 8 + 16 8.9 / 6.9, 64 + 64 18.6 / 16.6; 256 channels on 28 x 28 (32 x 32) 1 + 1 7.2 / 4.5 (the ring: 5.0), 1 + 16 9.0 / 6.2 (10.0),
+// 48 + 48 17.7 / 15.5, 64 + 32 17.3 / 16.5 (35.8); beyond its limit two launches are quicker than the ring (conv_shortcut_pays).
+int conv_stream_shortcut_tile(const NhwcGeom& g, int shortcut_steps)
+{
+    return stream_dense(g) && g.K == g.Cp ? stream_tile(g, g.K / 64 + shortcut_steps, true, 2) : 0;
 }
 
 int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream)
@@ -341,8 +354,8 @@ int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, co
 int launch_conv_stream_shortcut(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion,
                                 int out_cp, hipStream_t stream)
 {
-    const int tile = conv_stream_tile(g, true), tp = tile / 10, tc = tile % 10;
-    NCNNHIP_REQUIRE(tile && stream_dense(g) && g.K == g.Cp && sc.Cp % 64 == 0, "convolution: this layer does not fit the kernel for few tiles");
+    const int tile = conv_stream_shortcut_tile(g, sc.Cp / 64), tp = tile / 10, tc = tile % 10;
+    NCNNHIP_REQUIRE(tile && sc.Cp % 64 == 0, "convolution: this layer does not fit the kernel for few tiles");
     const int tiles_m = ceil_div(g.npix, 16 * tp), tiles_n = ceil_div(g.cout, 16 * tc);
     const unsigned magic_m = tiles_m > 1 ? (unsigned)((1ull << 32) / (unsigned)tiles_m + 1) : 0u;
     ConvShortcutArg<true> arg;

@@ -111,6 +111,7 @@ _SIGNATURES = {
     "ncnnhip_conv_int8_nhwc_fused": [C.POINTER(ConvDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, Activation, C.c_void_p, C.POINTER(ConvFusion), C.c_void_p,
                                      C.c_size_t, C.c_void_p],
     "ncnnhip_conv_shortcut_supported": [C.POINTER(ConvDesc), C.POINTER(ConvDesc), C.POINTER(C.c_int)],
+    "ncnnhip_conv_shortcut_pays": [C.POINTER(ConvDesc), C.POINTER(ConvDesc), C.POINTER(C.c_int)],
     "ncnnhip_conv_int8_nhwc_tail": [C.POINTER(ConvDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, Activation, C.POINTER(ConvShortcut), C.c_void_p,
                                     C.POINTER(ConvFusion), C.c_void_p, C.c_size_t, C.c_void_p],
     "ncnnhip_conv_int8_nhwc_route": [C.POINTER(ConvDesc), Activation, C.c_int, C.POINTER(ConvFusion), C.POINTER(ConvRoute)],

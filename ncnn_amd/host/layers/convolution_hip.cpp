@@ -452,8 +452,8 @@ int Convolution_hip::forward_tail(const HipMat& bottom, const HipMat* residual, 
         if (!xq[i] || c.weight_data_size != c.num_output * blobs[i]->c * c.kernel_w * c.kernel_h) return 0;
         desc[i] = c.describe(blobs[i]->w, blobs[i]->h, blobs[i]->c, blobs[i]->n);
     }
-    int supported = 1;
-    if (shortcut && (ncnnhip_conv_shortcut_supported(&desc[0], &desc[1], &supported) != 0 || !supported)) return 0;
+    int pays = 1;
+    if (shortcut && (ncnnhip_conv_shortcut_pays(&desc[0], &desc[1], &pays) != 0 || !pays)) return 0;
     int outw = 0, outh = 0;
     int rc = ncnnhip_conv_out_shape(&desc[0], &outw, &outh);
     if (rc != 0) return 0;

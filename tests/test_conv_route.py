@@ -48,3 +48,27 @@ def test_few_tiles_of_a_long_k_are_left_to_k_splits(hw, outc, tile, longest):
     for steps in (longest + 1, 400):
         r = cases.conv_route(1, 64 * steps, *hw, outc, (1, 1))
         assert r.kernel == r.PIPELINED and r.splits > 1
+
+
+def _pays(batch, hw, outc, c, shortcut_c, stride=2):
+    from ncnn_amd.hip import ConvDesc, check, lib
+    main = ConvDesc(hw, hw, c, batch, outc, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 0.0, 1)
+    side = ConvDesc(stride * hw, stride * hw, shortcut_c, batch, outc, 1, 1, 1, 1, stride, stride, 0, 0, 0, 0, 0.0, 1)
+    r = C.c_int(-1)
+    check(lib().ncnnhip_conv_shortcut_pays(C.byref(main), C.byref(side), C.byref(r)))
+    return r.value
+
+
+@pytest.mark.parametrize("batch,hw,outc,c,shortcut_c,pays", [
+    # few tiles: both K together up to twice what one convolution may have there
+    (1, 7, 512, 6400, 6400, 1), (1, 7, 2048, 5760, 5760, 1), (1, 7, 2048, 5760, 5824, 0), (2, 14, 512, 3072, 3072, 1), (2, 14, 512, 4096, 4096, 0),
+    (1, 28, 256, 64, 1024, 1),
+    # 104 to 256 tiles of 64 x 64
+    (1, 28, 512, 128, 256, 1), (4, 14, 1024, 256, 512, 1), (5, 14, 1024, 384, 768, 1), (1, 28, 512, 1024, 64, 0), (4, 7, 2048, 512, 1024, 0), (5, 14, 1024, 448, 768, 0),
+    # more
+    (16, 7, 2048, 512, 1024, 1), (6, 14, 1024, 640, 1280, 1), (6, 14, 1024, 640, 1344, 0), (16, 28, 512, 768, 1536, 1), (16, 28, 512, 832, 1536, 0),
+    (64, 56, 256, 64, 64, 1), (64, 14, 1024, 512, 1024, 1), (64, 14, 1024, 576, 1024, 0),
+    (1, 28, 512, 96, 256, 0),  # not a pair at all: channels that fill no whole step
+], ids=str)
+def test_shortcuts_that_pay(batch, hw, outc, c, shortcut_c, pays):
+    assert _pays(batch, hw, outc, c, shortcut_c) == pays

@@ -42,6 +42,8 @@ SHAPES = [
     (1, 64, 5, 7, 40, 128, 1),  # 16 x 16 tiles, a channel tail and padding
     (1, 512, 7, 7, 2048, 1024, 2),  # 16 x 32
     (1, 256, 14, 14, 1024, 512, 2),  # 32 x 32
+    (1, 64, 28, 28, 250, 1024, 2),  # 32 x 32, most of K in the shortcut
+    (1, 64, 56, 55, 64, 64, 1),  # 32 x 32, a step of each
     (2, 1600, 6, 5, 24, 64, 3),  # one step of shortcut, two rounds of the main convolution
     (1, 64, 56, 56, 256, 64, 1),  # the ring: 64-channel tiles
     (3, 128, 29, 27, 200, 192, 2),  # ragged pixels and channels

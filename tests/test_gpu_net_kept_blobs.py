@@ -36,3 +36,18 @@ def test_later_extracts_of_the_same_pass(net, light, first, then):
     if then:
         got, want = ex.extract(then), fresh(then)
         assert got.dtype == np.float32 and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("batch,h,w", [(1, 64, 80), (2, 224, 224), (4, 224, 224)])
+def test_light_mode_changes_no_score(net, batch, h, w):
+    """Outside light mode every layer runs on its own and every sum is fp32.  In it the sums are int8, with their shortcuts in the same launch: all of them
+    with few tiles; at four images the last stage's pair is left to two launches."""
+    x = np.random.default_rng(batch).random((batch, 3, h, w), dtype=np.float32)
+    print("[case] light mode", batch, h, w, flush=True)
+    scores = []
+    for light in (True, False):
+        ex = net.create_extractor()
+        ex.set_lightmode(light)
+        ex.input("data", x)
+        scores.append(ex.extract("fc1000"))
+    assert np.array_equal(*scores)
