@@ -282,8 +282,10 @@ int ncnnhip_chw_to_nhwc(const void* src_dev, int elemsize, int c, int hw, int ba
 int ncnnhip_nhwc_to_chw(const void* src_dev, int elemsize, int c, int hw, int batch, void* dst_dev, size_t cstep, size_t nstep, void* stream);
 /* An fp32 image of at most 4 channels may stay at 4 floats per pixel, [n][h*w][4] (a quarter of the padded blob): the
  * narrow-input convolution quantises straight from it (ncnnhip_quantize_stem with src_cp = 4); ncnnhip_widen_nhwc4_f32 turns
- * it into the ordinary [n][h*w][16] blob for anything else. */
+ * it into the ordinary [n][h*w][16] blob for anything else.  _from_host: the same for planes in page-locked host memory, read over
+ * PCIe (a launch of its own, as few requests there and many workgroups in device memory want different ones). */
 int ncnnhip_chw_to_nhwc4_f32(const float* src_dev, int c, int hw, int batch, size_t cstep, size_t nstep, float* dst_dev, void* stream);
+int ncnnhip_chw_to_nhwc4_f32_from_host(const float* src_pinned, int c, int hw, int batch, size_t cstep, size_t nstep, float* dst_dev, void* stream);
 int ncnnhip_widen_nhwc4_f32(const float* src_dev, float* dst_dev, size_t pixels, void* stream);
 /* Quantize::forward (src/layer/quantize.cpp:48-111) on a channels-last fp32 blob of npix pixels: one scale or one per channel. */
 int ncnnhip_quantize_nhwc(const float* src_dev, int8_t* dst_dev, size_t npix, int c, const float* scales_dev, int nscales, void* stream);

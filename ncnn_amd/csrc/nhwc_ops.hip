@@ -71,11 +71,12 @@ __global__ __launch_bounds__(256) void chw_to_nhwc4_f32_kernel(const float* __re
     *reinterpret_cast<v4f*>(dst + ((size_t)img * hw + pix) * 4) = v;
 }
 
-// The same for planes that do not begin on 128-byte lines (sizes that are no multiple of 32 pixels, mostly): read over PCIe, what counts is the
+// The same for planes in host memory that do not begin on 128-byte lines (sizes that are no multiple of 32 pixels, mostly): read over PCIe, what counts is the
 // number of requests, one a line and wavefront, and a wavefront's 256 bytes off the lines are three instead of two.  A workgroup takes 1024 pixels,
 // every load of a plane begins on a line (its edges masked), and the planes meet in LDS.  us for three images from page-locked memory, the kernel
 // above / here: 176 x 257 (planes on 64 bytes) 35.5 / 33.4, 49604 pixels (on 16) 40.1 / 37.7; with 512 pixels 34.4 and 38.9.  Planes on lines stay
-// above: 224 x 224 34.3 / 34.9.
+// above: 224 x 224 34.3 / 34.9.  From device memory the kernel above is the quicker, with four times the workgroups and no LDS between (49601 pixels, one
+// image 2.0 / 2.9, three 2.3 / 3.1, 16 3.9 / 4.9).
 constexpr int LINES_PIXELS = 1024;
 __global__ __launch_bounds__(256) void chw_to_nhwc4_f32_lines_kernel(const float* __restrict__ src, size_t cstep, size_t nstep, int c, int hw, float* __restrict__ dst)
 {
@@ -694,17 +695,28 @@ int ncnnhip_chw_to_nhwc(const void* src_dev, int elemsize, int c, int hw, int ba
     return launch_status("chw_to_nhwc_kernel");
 }
 
+static int check_nhwc4(const char* who, const float* src, int c, int hw, int batch, size_t cstep, const float* dst)
+{
+    NCNNHIP_REQUIRE(src && dst && c >= 1 && c <= 4 && hw > 0 && batch > 0 && batch <= 65535 && cstep >= (size_t)hw, "%s: bad argument", who);
+    return NCNNHIP_OK;
+}
+
 int ncnnhip_chw_to_nhwc4_f32(const float* src_dev, int c, int hw, int batch, size_t cstep, size_t nstep, float* dst_dev, void* stream)
 {
-    NCNNHIP_REQUIRE(src_dev && dst_dev && c >= 1 && c <= 4 && hw > 0 && batch > 0 && batch <= 65535 && cstep >= (size_t)hw, "ncnnhip_chw_to_nhwc4_f32: bad argument");
-    const bool on_lines = ((reinterpret_cast<uintptr_t>(src_dev) | cstep * 4 | (batch > 1 ? nstep * 4 : 0)) & 127) == 0;
-    if (!on_lines)
-    {
-        hipLaunchKernelGGL(chw_to_nhwc4_f32_lines_kernel, dim3(ceil_div(hw, LINES_PIXELS), batch), dim3(256), 0, as_stream(stream), src_dev, cstep, nstep, c, hw, dst_dev);
-        return launch_status("chw_to_nhwc4_f32_lines_kernel");
-    }
+    const int bad = check_nhwc4("ncnnhip_chw_to_nhwc4_f32", src_dev, c, hw, batch, cstep, dst_dev);
+    if (bad) return bad;
     hipLaunchKernelGGL(chw_to_nhwc4_f32_kernel, dim3(ceil_div(hw, 256), batch), dim3(256), 0, as_stream(stream), src_dev, cstep, nstep, c, hw, dst_dev);
     return launch_status("chw_to_nhwc4_f32_kernel");
+}
+
+int ncnnhip_chw_to_nhwc4_f32_from_host(const float* src_pinned, int c, int hw, int batch, size_t cstep, size_t nstep, float* dst_dev, void* stream)
+{
+    const int bad = check_nhwc4("ncnnhip_chw_to_nhwc4_f32_from_host", src_pinned, c, hw, batch, cstep, dst_dev);
+    if (bad) return bad;
+    const bool on_lines = ((reinterpret_cast<uintptr_t>(src_pinned) | cstep * 4 | (batch > 1 ? nstep * 4 : 0)) & 127) == 0;
+    if (on_lines) return ncnnhip_chw_to_nhwc4_f32(src_pinned, c, hw, batch, cstep, nstep, dst_dev, stream);
+    hipLaunchKernelGGL(chw_to_nhwc4_f32_lines_kernel, dim3(ceil_div(hw, LINES_PIXELS), batch), dim3(256), 0, as_stream(stream), src_pinned, cstep, nstep, c, hw, dst_dev);
+    return launch_status("chw_to_nhwc4_f32_lines_kernel");
 }
 
 int ncnnhip_widen_nhwc4_f32(const float* src_dev, float* dst_dev, size_t pixels, void* stream)

@@ -128,6 +128,7 @@ _SIGNATURES = {
     "ncnnhip_scale": [C.c_void_p, C.c_void_p, C.c_size_t, C.c_float, C.c_void_p],
     "ncnnhip_eltwise": [C.POINTER(C.c_void_p), C.c_int, C.c_int, C.POINTER(C.c_float), C.c_int, C.c_void_p, C.c_size_t, C.c_void_p],
     "ncnnhip_chw_to_nhwc4_f32": [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_size_t, C.c_size_t, C.c_void_p, C.c_void_p],
+    "ncnnhip_chw_to_nhwc4_f32_from_host": [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_size_t, C.c_size_t, C.c_void_p, C.c_void_p],
     "ncnnhip_widen_nhwc4_f32": [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p],
     "ncnnhip_conv_stem_supported": [C.POINTER(ConvDesc)],
     "ncnnhip_conv_stem_sizes": [C.POINTER(ConvDesc), C.POINTER(C.c_size_t), C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)],

@@ -465,7 +465,7 @@ int HipCommand::upload_planes(const Mat& src, HipMat& dst)
             }
             unsigned char* to = (unsigned char*)dst.data + ((size_t)b * hw + p0) * dst.cp * es;
             if (dst.narrow())
-                rc = ncnnhip_chw_to_nhwc4_f32((const float*)s->data, src.c, (int)len, samples, cstep, nstep, (float*)to, stream);
+                rc = ncnnhip_chw_to_nhwc4_f32_from_host((const float*)s->data, src.c, (int)len, samples, cstep, nstep, (float*)to, stream);
             else
                 rc = ncnnhip_chw_to_nhwc(s->data, es, src.c, (int)len, samples, cstep, nstep, to, stream);
             const int mark = mark_stage(s);

@@ -1,4 +1,5 @@
-"""Planar fp32 images of at most 4 channels to 4 floats a pixel (ncnnhip_chw_to_nhwc4_f32), bit for bit: planes on 128-byte lines and off
+"""Planar fp32 images of at most 4 channels to 4 floats a pixel (ncnnhip_chw_to_nhwc4_f32 and its form for
+page-locked memory, each from both kinds of memory), bit for bit: planes on 128-byte lines and off
 them by any number of floats, at the edges of the kernels' pixel tiles, from device and page-locked memory; nothing beyond the blob is written."""
 import ctypes as C
 
@@ -39,12 +40,15 @@ def test_planes_on_and_off_lines(rt, pinned, hw, c, batch):
         else:
             src = rt.up(host)
             base = src.ptr.value
-        got = rt.up(np.full(batch * hw * 4 + 64, -7, F))
-        check(lib().ncnnhip_chw_to_nhwc4_f32(C.c_void_p(base + offset * 4), c, hw, batch, cstep, nstep, got.ptr, rt.stream))
-        out = got.to_numpy(rt.stream)
+        outs = []
+        for entry in (lib().ncnnhip_chw_to_nhwc4_f32, lib().ncnnhip_chw_to_nhwc4_f32_from_host):
+            got = rt.up(np.full(batch * hw * 4 + 64, -7, F))
+            check(entry(C.c_void_p(base + offset * 4), c, hw, batch, cstep, nstep, got.ptr, rt.stream))
+            outs.append(got.to_numpy(rt.stream))
         want = np.zeros((batch, hw, 4), F)
         for n in range(batch):
             for q in range(c):
                 at = offset + n * nstep + q * cstep
                 want[n, :, q] = host[at:at + hw]
-        assert np.array_equal(out[:batch * hw * 4].reshape(batch, hw, 4), want) and (out[batch * hw * 4:] == -7).all()
+        for out in outs:
+            assert np.array_equal(out[:batch * hw * 4].reshape(batch, hw, 4), want) and (out[batch * hw * 4:] == -7).all()
