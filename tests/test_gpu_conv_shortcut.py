@@ -104,6 +104,39 @@ def test_quantised_output_alone(rt, batch, c, hw, outc, kernel):
     assert np.array_equal(rt.from_channels_last(q8, batch, outc, hw, hw), want_q)
 
 
+def test_projection_shortcut_of_a_million_pixels(rt):
+    """From 2^20 pixels on the ring finds the shortcut's pixel by whole divisions: images, rows and columns of a stride of 2."""
+    batch, hw, c, outc = 3, 592, 64, 16
+    print("[case] conv shortcut, a million pixels", flush=True)
+    assert batch * hw * hw >= 1 << 20
+    rng = np.random.default_rng(20)
+    x, sx = (rng.integers(-127, 128, (batch, n, n, c), dtype=np.int8) for n in (hw, 2 * hw - 1))
+    scales = rng.uniform(2000, 4000, (2, outc)).astype(F)
+    bias = rng.uniform(-1, 1, outc).astype(F)
+    sides, weights = [], []
+    for blob, ws, b in ((x, scales[0], bias), (sx[:, ::2, ::2], scales[1], np.zeros(outc, F))):
+        wq = rng.integers(-127, 128, (outc, c, 1, 1)).astype(np.int8)
+        d = oracle.make_desc((c, hw, hw), outc, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), 0.0, 1, 1, 2, 0, (0.0, 0.0))
+        sides.append(np.stack([oracle.convolution_int8(d, blob[i].transpose(2, 0, 1).astype(F), wq, b, ws, F(1), None) for i in range(batch)]))
+        weights.append(wq)
+    want = np.maximum((sides[0] + sides[1]).astype(F), 0)
+    desc, sdesc = _desc(batch, c, hw, hw, outc, 1), _desc(batch, c, 2 * hw - 1, 2 * hw - 1, outc, 2)
+    dev = [rt.up(v) for v in (x, sx)]
+    packed = []
+    for d, wq in zip((desc, sdesc), weights):
+        p = np.empty(outc * c, np.int8)
+        check(lib().ncnnhip_conv_pack_weights(C.byref(d), wq.ctypes.data, p.ctypes.data))
+        packed.append(rt.up(p))
+    folded = [rt.up(rt.fold_input_scales(ws, np.array([1], F), outc)) for ws in scales]
+    b = rt.up(bias)
+    out = DeviceBuffer.empty((batch, hw * hw, outc), F)
+    act = Activation.make(0, (0.0, 0.0))
+    short = ConvShortcut(C.pointer(sdesc), dev[1].ptr, packed[1].ptr, folded[1].ptr, None, act)
+    fu = ConvFusion(None, 1, None, 0.0)
+    check(lib().ncnnhip_conv_int8_nhwc_tail(C.byref(desc), dev[0].ptr, packed[0].ptr, folded[0].ptr, b.ptr, act, C.byref(short), out.ptr, C.byref(fu), None, 0, rt.stream))
+    assert np.array_equal(rt.from_channels_last(out, batch, outc, hw, hw), want)
+
+
 def test_pairs_that_are_refused(rt):
     supported = C.c_int(1)
     main = _desc(1, 64, 8, 8, 64, 1)
