@@ -595,7 +595,7 @@ int NetPrivate::try_fused_tail(int layer_index, ExecState& st, const Option& opt
         // the output in quantised form alone, unless this extract call asks for the blob itself or leaves it, or what Split makes of it, for a later
         // one (looked up here, where the device has work already)
         const bool only_quantised =
-            tp.only_quantised && opt.lightmode && st.wanted >= 0 && !tail_zone[(size_t)st.wanted] && zone_is_consumed(last->tops[0], st);
+            tp.only_quantised && st.wanted >= 0 && !tail_zone[(size_t)st.wanted] && zone_is_consumed(last->tops[0], st);
         bool folded = false;
         if (shortcut)
         {
