@@ -901,10 +901,13 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
         bias[c] = (real[c] && epi.bias) ? raw_bias[c] : -0.f;
         s_out[c] = (real[c] && to_int8_) ? raw_s_out[c] : 0.f;
     }
-    // the activation type is uniform: branch on it once, outside the unrolled loops
-    auto finish = [&](auto act_tag) {
+    // The activation and the output type are uniform: branch on them once, outside the unrolled loops.  With the output type as a run-time branch
+    // inside, the fp32 forms paid for the int8 ones' code and registers (68 to 71 instead of 60 with 64 x 64 tiles, 104 to 106 instead of 96 with 64 x 128,
+    // where 96 are four workgroups to a unit instead of three).  us, one layer in a chain: 128 channels, fp32 out, 96 channels in, 16 images of
+    // 56 x 56 11.1 -> 9.0 (int8 out 7.1 -> 6.2), 224 in 12.9 -> 10.9; 64 x 64 tiles 1 to 3 % off fp32 results, level to 1 % on int8 ones.
+    auto finish = [&](auto act_tag, auto int8_tag) {
         constexpr int ACT = decltype(act_tag)::value;
-        const bool to_int8 = ACT == 100 || ACT == 201 || ACT == 203 || to_int8_;
+        constexpr bool to_int8 = decltype(int8_tag)::value;
         // The clamp that also holds the activation where the tables are tame (below): 103 the clip's bounds in the output scale (fp32 results are
         // clipped as written), 100 none, 201 and 203 a ReLU's and a clip's without a negative bound, so that the rounding is one conversion
         // (pack16_nonneg).  Vector instructions per value: 8 instead of 10 without an activation, 6 instead of 11 behind a ReLU, 6 instead of 8
@@ -1060,47 +1063,63 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
             if (a + 1 < TM) __syncthreads();
         }
     };
-    // To int8 without an activation or behind a ReLU: a value below 2^31 in the output scale (|acc| <= 2^31) never takes float2int8's out-of-range
-    // answer, and x -> RN(x * s) never decreases for s >= 0, so it commutes with the ReLU's max, which then is the clamp's lower bound.
-    bool small = to_int8_ && !SHORTCUT && epi.act.type <= 1;
-#pragma unroll
-    for (int c = 0; c < TN; c++) small = small && s_out[c] >= 0.f && mul_rn(add_rn(mul_rn(2147483648.f, fabsf(s_in[c])), fabsf(bias[c])), s_out[c]) < 1073741824.f;
-    small = __all(small);
-    if (epi.act.type == 0)
-    {
-        if (small)
-            finish(std::integral_constant<int, 100>{});
-        else
-            finish(std::integral_constant<int, 0>{});
-    }
-    else if (epi.act.type == 1)
-    {
-        if (small)
-            finish(std::integral_constant<int, 201>{});
-        else
-            finish(std::integral_constant<int, 1>{});
-    }
-    else if (epi.act.type == 3)
-    {
-        // Tame tables: every accumulator comes out of scale and bias finite (|acc| <= 2^31, so 2^90 and 2^120 leave
-        // room), so the clip is max-then-min; the clipped value times the output scale stays below 2^31, so float2int8
-        // needs no out-of-range branch; and the clip folds into the requantising clamp.
+    // Tame tables: every accumulator comes out of scale and bias finite (|acc| <= 2^31, so 2^90 and 2^120 leave
+    // room), so the clip is max-then-min; the clipped value times the output scale stays below 2^31, so float2int8
+    // needs no out-of-range branch; and the clip folds into the requantising clamp.
+    auto clip_is_tame = [&]() {
         const float clip_abs = fmaxf(fabsf(epi.act.p0), fabsf(epi.act.p1));
         bool tame = fabsf(epi.act.p0) < INFINITY && fabsf(epi.act.p1) < INFINITY;
 #pragma unroll
         for (int c = 0; c < TN; c++)
             tame = tame && fabsf(s_in[c]) < 0x1p90f && fabsf(bias[c]) < 0x1p120f && mul_rn(clip_abs, fabsf(s_out[c])) < 2147483648.f
                    && clip_folds_into_requantise(epi.act.p0, epi.act.p1, s_out[c]);
-        tame = __all(tame);
-        if (tame && to_int8_ && !SHORTCUT && epi.act.p0 >= 0.f)
-            finish(std::integral_constant<int, 203>{});
-        else if (tame)
-            finish(std::integral_constant<int, 103>{});
+        return (bool)__all(tame);
+    };
+    typedef std::false_type Fp32;
+    typedef std::true_type Int8;
+    if (SHORTCUT || !to_int8_) // (first: with the int8 forms in front the fp32 ones took 0.5 % more, and those no less)
+    {
+        if (epi.act.type == 0)
+            finish(std::integral_constant<int, 0>{}, Fp32{});
+        else if (epi.act.type == 1)
+            finish(std::integral_constant<int, 1>{}, Fp32{});
+        else if (epi.act.type == 3 && clip_is_tame())
+            finish(std::integral_constant<int, 103>{}, Fp32{});
+        else if (epi.act.type == 3)
+            finish(std::integral_constant<int, 3>{}, Fp32{});
         else
-            finish(std::integral_constant<int, 3>{});
+            finish(std::integral_constant<int, -1>{}, Fp32{});
+    }
+    else if (epi.act.type == 0 || epi.act.type == 1)
+    {
+        // Without an activation or behind a ReLU: a value below 2^31 in the output scale (|acc| <= 2^31) never takes float2int8's out-of-range
+        // answer, and x -> RN(x * s) never decreases for s >= 0, so it commutes with the ReLU's max, which then is the clamp's lower bound.
+        bool small = true;
+#pragma unroll
+        for (int c = 0; c < TN; c++)
+            small = small && s_out[c] >= 0.f && mul_rn(add_rn(mul_rn(2147483648.f, fabsf(s_in[c])), fabsf(bias[c])), s_out[c]) < 1073741824.f;
+        small = __all(small);
+        if (epi.act.type == 0 && small)
+            finish(std::integral_constant<int, 100>{}, Int8{});
+        else if (epi.act.type == 0)
+            finish(std::integral_constant<int, 0>{}, Int8{});
+        else if (small)
+            finish(std::integral_constant<int, 201>{}, Int8{});
+        else
+            finish(std::integral_constant<int, 1>{}, Int8{});
+    }
+    else if (epi.act.type == 3)
+    {
+        const bool tame = clip_is_tame();
+        if (tame && epi.act.p0 >= 0.f)
+            finish(std::integral_constant<int, 203>{}, Int8{});
+        else if (tame)
+            finish(std::integral_constant<int, 103>{}, Int8{});
+        else
+            finish(std::integral_constant<int, 3>{}, Int8{});
     }
     else
-        finish(std::integral_constant<int, -1>{});
+        finish(std::integral_constant<int, -1>{}, Int8{});
 }
 
 struct PipePlan
