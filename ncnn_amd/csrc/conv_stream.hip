@@ -292,23 +292,33 @@ static bool stream_dense(const NhwcGeom& g)
 // With 32 x 32 tiles the ring is level or ahead at both ends of K: int8 out 1x1 64 -> 64 on 56 x 56 3.0 / 3.2, 256 -> 64 3.6 / 3.9, 3x3 512 -> 512 on 7 x 7,
 // eight images 10.7 / 11.0 (four, 16 x 32 tiles: 10.2 / 9.2); fp32 out is ahead from two steps on (128 -> 64 on 56 x 56 3.34 / 3.21, 192 -> 64 3.52 / 3.31,
 // 256 -> 64 level, 3.68 / 3.71).
-// Beyond some K the ring, which splits it over workgroups, is quicker again.  The ring / here, fp32 out (steps: 64 of K): 16 x 16 tiles 192 steps 13.2 / 13.0 with
-// 4 tiles, 18.1 / 13.4 with 208; 208 steps 13.5 / 14.4 and 18.5 / 14.8;
-// 288 steps 16.8 / 18.2 with 4, 20.8 / 19.2 with 128, 19.4 / 19.0 with 208; 400 steps 20.1 / 24.7 and 21.2 / 25.8.  16 x 32 tiles 64 steps 9.4 / 8.2 (512 channels
-// on 14 x 14), 3x3 512 -> 512 (72) 9.8 / 9.2, 3x3 576 -> 512 (81) 10.3 / 7.6, 3x3 640 -> 512 (90) 10.7 / 10.4 (160 channels on 28 x 28, 80 steps: 9.6 / 9.8);
-// 96 steps 10.4 / 11.0, 144 12.7 / 15.6, 400 18.9 / 36.6.
-static int stream_tile(const NhwcGeom& g, int steps, bool fp32_out, int convolutions)
+// A single tap with a stride (1x1, not dense) costs its pixels' divisions and, on the ring, no more than a dense one: the ring is ahead of the smaller tiles below
+// five steps to int8 (64 -> 256 on 28 x 28, stride 2, 3.1 / 3.8; 256 -> 256 3.6 / 3.7, 320 -> 256 3.8 / 3.6) and three to fp32 (128 3.5 / 3.6, 192 3.6 / 3.6), of
+// 32 x 32 below eight and six (four images, int8 384 4.0 / 4.1, 512 5.3 / 4.5; fp32 256 3.9 / 4.2, 384 4.2 / 4.1).
+// Beyond some K the ring, which splits it over workgroups, is quicker again.  Weight rows an odd number of steps (64 bytes of K) apart come in at 1.3 times the
+// rate of an even number, so the lines lie further out there.  Time here over the ring's, fp32 out, dense:
+//   16 x 16, below 128 tiles   even: 144 steps 0.87-0.93, 176 0.94-0.99, 194 1.00-1.06, 288 1.03-1.09    odd: 193 0.8, 401 0.86-0.91, 641 0.88-0.95
+//   16 x 16, from 128 on       even: 208 0.81-0.93, 288 0.91-0.98, 322 0.98-1.08, 402 1.02-1.23          odd: 401 0.78-0.94, 641 1.09-1.20
+//   16 x 32                    even: 64 0.87-0.91, 80 0.96-1.02, 96 1.04-1.05, 144 1.2, 402 2.0          odd: 81 0.8, 145 0.92-1.00, 193 1.00-1.17
+static int stream_tile(const NhwcGeom& g, int steps, bool odd, bool fp32_out, int convolutions)
 {
     const long long m16 = ceil_div(g.npix, 16), m32 = ceil_div(g.npix, 32), n16 = ceil_div(g.cout, 16), n32 = ceil_div(g.cout, 32);
-    if (m16 * n16 <= 256) return steps <= convolutions * (m16 * n16 >= 128 ? 288 : 192) ? 11 : 0;
-    if (m16 * n32 <= 256) return steps <= convolutions * 90 ? 12 : 0;
-    return m32 * n32 <= 256 && steps >= (fp32_out ? 2 : 5) && steps <= convolutions * 48 ? 22 : 0;
+    const bool strided = g.ntaps == 1 && !stream_dense(g);
+    if (m16 * n32 <= 256)
+    {
+        if (strided && steps < (fp32_out ? 3 : 5)) return 0;
+        const bool wide = m16 * n16 > 256;
+        const int longest = wide ? (odd ? 145 : 80) : m16 * n16 < 128 ? (odd ? 641 : 192) : (odd ? 401 : 288);
+        return steps > convolutions * longest ? 0 : wide ? 12 : 11;
+    }
+    const int shortest = strided ? (fp32_out ? 6 : 8) : fp32_out ? 2 : 5;
+    return m32 * n32 <= 256 && steps >= shortest && steps <= convolutions * 48 ? 22 : 0;
 }
 
 int conv_stream_tile(const NhwcGeom& g, bool fp32_out)
 {
     if (!stream_dense(g) && !(g.tapK % 64 == 0 && g.tapK == g.Cp)) return 0;
-    return stream_tile(g, g.K / 64, fp32_out, 1);
+    return stream_tile(g, g.K / 64, g.K / 64 % 2 == 1, fp32_out, 1);
 }
 
 // With a shortcut a workgroup walks both K, one after the other, in place of two launches that walk one each: the limits hold for the two together.
@@ -317,7 +327,7 @@ int conv_stream_tile(const NhwcGeom& g, bool fp32_out)
 // 48 + 48 17.7 / 15.5, 64 + 32 17.3 / 16.5 (35.8); beyond its limit two launches are quicker than the ring (conv_shortcut_pays).
 int conv_stream_shortcut_tile(const NhwcGeom& g, int shortcut_steps)
 {
-    return stream_dense(g) && g.K == g.Cp ? stream_tile(g, g.K / 64 + shortcut_steps, true, 2) : 0;
+    return stream_dense(g) && g.K == g.Cp ? stream_tile(g, g.K / 64 + shortcut_steps, g.K / 64 % 2 == 1 && shortcut_steps % 2 == 1, true, 2) : 0;
 }
 
 int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream)

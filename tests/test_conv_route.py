@@ -40,14 +40,24 @@ def test_layers_that_are_refused():
     assert lib().ncnnhip_conv_int8_nhwc_route(None, act, 0, None, C.byref(r)) != 0
 
 
-@pytest.mark.parametrize("hw,outc,tile,longest", [((4, 4), 64, (16, 16), 192), ((14, 14), 256, (16, 16), 288), ((7, 7), 496, (16, 16), 192), ((14, 14), 512, (16, 32), 90), ((28, 28), 160, (16, 32), 90),
-                                                  ((28, 28), 256, (32, 32), 48)], ids=str)
-def test_few_tiles_of_a_long_k_are_left_to_k_splits(hw, outc, tile, longest):
-    r = cases.conv_route(1, 64 * longest, *hw, outc, (1, 1))
-    assert (r.kernel, r.tile_pixels, r.tile_channels) == (r.FEW_TILES,) + tile
-    for steps in (longest + 1, 400):
-        r = cases.conv_route(1, 64 * steps, *hw, outc, (1, 1))
+@pytest.mark.parametrize("hw,outc,tile,even,odd", [((4, 4), 64, (16, 16), 192, 641), ((14, 14), 256, (16, 16), 288, 401), ((7, 7), 496, (16, 16), 192, 641),
+                                                   ((14, 14), 512, (16, 32), 80, 145), ((28, 28), 160, (16, 32), 80, 145), ((28, 28), 256, (32, 32), 48, 47)], ids=str)
+def test_few_tiles_of_a_long_k_are_left_to_k_splits(hw, outc, tile, even, odd):
+    for longest in (even, odd):
+        r = cases.conv_route(1, 64 * longest, *hw, outc, (1, 1))
+        assert (r.kernel, r.tile_pixels, r.tile_channels) == (r.FEW_TILES,) + tile
+        r = cases.conv_route(1, 64 * (longest + 2), *hw, outc, (1, 1))
         assert r.kernel == r.PIPELINED and r.splits > 1
+
+
+@pytest.mark.parametrize("batch,outc,int8_out,shortest", [(1, 256, True, 5), (1, 256, False, 3), (1, 512, True, 5), (1, 512, False, 3), (4, 256, True, 8), (4, 256, False, 6)])
+def test_few_steps_of_a_strided_tap_are_left_to_the_ring(batch, outc, int8_out, shortest):
+    for steps, kernel in ((shortest - 1, "PIPELINED"), (shortest, "FEW_TILES")):
+        r = cases.conv_route(batch, 64 * steps, 28, 28, outc, (1, 1), stride=(2, 2), int8_out=int8_out)
+        assert r.kernel == getattr(r, kernel)
+    for kernel in ((1, 1), (3, 3)):  # dense, and several taps
+        r = cases.conv_route(1, 64, 14, 14, outc, kernel, pads=(kernel[0] // 2,) * 4, int8_out=int8_out)
+        assert r.kernel == r.FEW_TILES
 
 
 def _pays(batch, hw, outc, c, shortcut_c, stride=2):
@@ -61,7 +71,7 @@ def _pays(batch, hw, outc, c, shortcut_c, stride=2):
 
 @pytest.mark.parametrize("batch,hw,outc,c,shortcut_c,pays", [
     # few tiles: both K together up to twice what one convolution may have there
-    (1, 7, 512, 6400, 6400, 1), (1, 7, 2048, 5760, 5760, 1), (1, 7, 2048, 5760, 5824, 0), (2, 14, 512, 3072, 3072, 1), (2, 14, 512, 4096, 4096, 0),
+    (1, 7, 512, 6400, 6400, 1), (1, 7, 2048, 5120, 5120, 1), (1, 7, 2048, 5120, 5184, 0), (1, 7, 2048, 5184, 5184, 1), (2, 14, 512, 3072, 3072, 1), (2, 14, 512, 4096, 4096, 0),
     (1, 28, 256, 64, 1024, 1),
     # 104 to 256 tiles of 64 x 64
     (1, 28, 512, 128, 256, 1), (4, 14, 1024, 256, 512, 1), (5, 14, 1024, 384, 768, 1), (1, 28, 512, 1024, 64, 0), (4, 7, 2048, 512, 1024, 0), (5, 14, 1024, 448, 768, 0),

@@ -30,14 +30,17 @@ SHAPES = [
     (2, 192, 11, 9, 24, (1, 3), (1, 1), (2, 1), (0, 0, 1, 1)),  # a tap of three steps, uneven strides
     (1, 64, 64, 64, 16, (1, 1), (1, 1), (1, 1), NONE),  # 256 tiles
     (1, 3072, 2, 5, 40, (2, 2), (1, 1), (1, 1), (0, 0, 0, 0)),  # 192 steps, the longest K
-    (1, 12352, 3, 3, 40, (1, 1), (1, 1), (1, 1), NONE),  # 193: K split over workgroups
+    (1, 12416, 3, 3, 40, (1, 1), (1, 1), (1, 1), NONE),  # 194: K split over workgroups
     # 16 x 32
     (1, 64, 64, 64, 17, (1, 1), (1, 1), (1, 1), NONE),
     (1, 128, 28, 28, 128, (3, 3), (1, 1), (1, 1), SAME3),
     (1, 1024, 14, 14, 512, (1, 1), (1, 1), (2, 2), NONE),
     (1, 512, 7, 7, 2000, (1, 1), (1, 1), (1, 1), NONE),
-    (1, 2880, 8, 32, 290, (1, 2), (1, 1), (1, 1), NONE),  # 90 steps, the longest K
-    (1, 5824, 8, 32, 258, (1, 1), (1, 1), (1, 1), NONE),  # 91: K split over workgroups
+    (1, 2560, 8, 32, 290, (1, 2), (1, 1), (1, 1), NONE),  # 80 steps, the longest even K
+    (1, 5184, 8, 32, 258, (1, 1), (1, 1), (1, 1), NONE),  # 81, odd
+    (1, 5248, 8, 32, 258, (1, 1), (1, 1), (1, 1), NONE),  # 82: K split over workgroups
+    (1, 128, 28, 28, 200, (1, 1), (1, 1), (2, 2), NONE),  # a strided tap of two steps: the pipelined kernel's
+    (1, 192, 28, 28, 200, (1, 1), (1, 1), (2, 2), NONE),  # three: here to fp32, there to int8
     # 32 x 32, and what the other kernels keep: four steps and fewer to int8, more than 48 steps, 257 tiles
     (1, 96, 63, 64, 60, (1, 1), (1, 1), (1, 1), NONE),
     (1, 320, 63, 64, 60, (1, 1), (1, 1), (1, 1), NONE),
