@@ -2,7 +2,8 @@
 // K steps in front of the main convolution's (MODE 4), for layers with many tiles; conv_stream.hip has the form for few.
 //
 // The shortcut's fp32 result is neither written nor read again: for ResNet-50's second stage at 16 images 51 MB each way, half of
-// the two launches' traffic, which is what bounds them (5.5 TB/s).
+// the traffic of the two launches, which moved it at 5.5 TB/s.  The one launch is not at that rate (128 images 3.7 TB/s there, 1.3 in the last stage):
+// one to eight K steps of each convolution, two epilogues and the stores follow one another with nothing of the next tile under way.
 #include "conv_nhwc_pipelined_kernel.h"
 
 namespace ncnnhip {
@@ -30,11 +31,10 @@ int launch_conv_shortcut(const NhwcGeom& g_in, const int8_t* wpk, const int8_t* 
     NhwcGeom g = g_in;
     g.H = g.outh = 1;
     g.W = g.outw = g.npix;
-    // K stays whole: the shortcut's sums are finished where the main ones are.  64-channel tiles (six workgroups to a unit where four of 128 channels
+    // K stays whole: the shortcut's sums are finished where the main ones are.  64-channel tiles (five workgroups to a unit where three of 128 channels
     // fit) until there are so many that the activations read per tile weigh more.  us, 128 channels wide / 64, fp32 and quantised output:
-    // 16 images 64 + 64 -> 256 on 56 x 56 23.5 / 22.1, 128 + 256 -> 512 on 28 x 28 20.4 / 17.2, 256 + 512 -> 1024 on 14 x 14 13.8 / 13.9, 512 + 1024 -> 2048
-    // on 7 x 7 16.3 / 14.5 (two launches: 35.7, 25.7, 16.4, 14.6); 64 images 76 / 83 (12544 tiles), 45.4 / 45.0 (6272), 36.4 / 34.8, 36.6 / 31.6
-    // (two launches: 147, 79, 44, 38).
+    // 16 images 64 + 64 -> 256 on 56 x 56 22.2 / 18.8, 128 + 256 -> 512 on 28 x 28 19.5 / 15.7, 256 + 512 -> 1024 on 14 x 14 14.5 / 13.4, 512 + 1024 -> 2048
+    // on 7 x 7 18.5 / 14.6 (two launches 36.5, 26.6, 17.4, 15.9); 64 images 80 / 84 (12544 tiles; int8 alone 57 / 50), 44.9 / 44.4 (6272), 37.1 / 34.4, 37.8 / 32.1.
     const int tiles_m = ceil_div(g.npix, 64), wide = (long long)tiles_m * ceil_div(g.cout, 64) >= 8192, tiles_n = ceil_div(g.cout, wide ? 128 : 64);
     const long long blocks = (long long)tiles_m * tiles_n;
     NCNNHIP_REQUIRE(blocks < (1ll << 31) && blocks * tiles_n < (1ll << 32), "convolution: too many tiles");
