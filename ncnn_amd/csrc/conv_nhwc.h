@@ -100,7 +100,8 @@ int launch_conv_pointwise(const NhwcGeom& g, const int8_t* wpk, const int8_t* x,
 // problem belong to it (int8 blob), and its launch.  conv_patch_pays leaves such layers to it; the pipelined launch asks after the
 // pointwise and weights-resident kernels, which want many pixels.
 int conv_stream_tile(const NhwcGeom& g, bool fp32_out); // 0: it does not, else pixels / 16 * 10 + channels / 16
-int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream);
+int conv_stream_tile_any_k(const NhwcGeom& g); // its smaller tiles whatever K is: for a layer whose K split has no workspace
+int launch_conv_stream(const NhwcGeom& g, int tile, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream);
 
 // The same two kernels with a projection shortcut (g: the main 1x1 convolution, stride 1, unpadded, channels in whole steps).
 // conv_shortcut_pays: one launch is quicker than the two convolutions one after the other.

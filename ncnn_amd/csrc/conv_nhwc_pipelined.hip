@@ -144,7 +144,7 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
     case NCNNHIP_CONV_RESIDENT:
         return launch_conv_resident(g_in, wpk, x, epi, fusion, out_cp, stream);
     case NCNNHIP_CONV_FEW_TILES:
-        return launch_conv_stream(g_in, wpk, x, epi, fusion, out_cp, stream);
+        return launch_conv_stream(g_in, conv_stream_tile(g_in, !epi.scale_out), wpk, x, epi, fusion, out_cp, stream);
     }
     NhwcGeom g = g_in;
     PipePlan p;
@@ -156,7 +156,10 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
     if (p.splits > 1)
     {
         const size_t need = SPLIT_COUNTER_BYTES + (size_t)p.splits * p.tiles_m * p.tiles_n * p.bm * p.bn * sizeof(int32_t);
-        NCNNHIP_REQUIRE(workspace && workspace_bytes >= need, "convolution: workspace of %zu bytes required", need);
+        const bool split = workspace && workspace_bytes >= need;
+        const int tile = split ? 0 : conv_stream_tile_any_k(g_in);
+        if (tile) return launch_conv_stream(g_in, tile, wpk, x, epi, fusion, out_cp, stream);
+        NCNNHIP_REQUIRE(split, "convolution: workspace of %zu bytes required", need);
         counters = (unsigned*)workspace; // zero on entry (the caller cleared the workspace once), zero again on exit
         partial = (int32_t*)((char*)workspace + SPLIT_COUNTER_BYTES);
     }

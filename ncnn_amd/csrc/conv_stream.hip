@@ -315,10 +315,20 @@ static int stream_tile(const NhwcGeom& g, int steps, bool odd, bool fp32_out, in
     return m32 * n32 <= 256 && steps >= shortest && steps <= convolutions * 48 ? 22 : 0;
 }
 
+static bool stream_addressing(const NhwcGeom& g)
+{
+    return stream_dense(g) || (g.tapK % 64 == 0 && g.tapK == g.Cp);
+}
+
 int conv_stream_tile(const NhwcGeom& g, bool fp32_out)
 {
-    if (!stream_dense(g) && !(g.tapK % 64 == 0 && g.tapK == g.Cp)) return 0;
-    return stream_tile(g, g.K / 64, g.K / 64 % 2 == 1, fp32_out, 1);
+    return stream_addressing(g) ? stream_tile(g, g.K / 64, g.K / 64 % 2 == 1, fp32_out, 1) : 0;
+}
+
+int conv_stream_tile_any_k(const NhwcGeom& g)
+{
+    const long long m16 = ceil_div(g.npix, 16);
+    return !stream_addressing(g) ? 0 : m16 * ceil_div(g.cout, 16) <= 256 ? 11 : m16 * ceil_div(g.cout, 32) <= 256 ? 12 : 0;
 }
 
 // With a shortcut a workgroup walks both K, one after the other, in place of two launches that walk one each: the limits hold for the two together.
@@ -330,9 +340,9 @@ int conv_stream_shortcut_tile(const NhwcGeom& g, int shortcut_steps)
     return stream_dense(g) && g.K == g.Cp ? stream_tile(g, g.K / 64 + shortcut_steps, g.K / 64 % 2 == 1 && shortcut_steps % 2 == 1, true, 2) : 0;
 }
 
-int launch_conv_stream(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream)
+int launch_conv_stream(const NhwcGeom& g, int tile, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream)
 {
-    const int tile = conv_stream_tile(g, !epi.scale_out), tp = tile / 10, tc = tile % 10;
+    const int tp = tile / 10, tc = tile % 10;
     NCNNHIP_REQUIRE(tile && !epi.acc_out, "convolution: this layer does not fit the kernel for few tiles");
     const int tiles_m = ceil_div(g.npix, 16 * tp), tiles_n = ceil_div(g.cout, 16 * tc), blocks = tiles_m * tiles_n; // 256 at most
     const unsigned magic_m = tiles_m > 1 ? (unsigned)((1ull << 32) / (unsigned)tiles_m + 1) : 0u;

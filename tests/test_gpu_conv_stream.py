@@ -62,6 +62,28 @@ def test_few_tiles_kernel_matches_oracle(rt, shape):
         assert got.dtype == want.dtype and np.array_equal(got, want), (term, act)
 
 
+@pytest.mark.parametrize("c,h,w,outc", [(12416, 3, 3, 40), (5248, 8, 32, 258)])
+def test_long_k_without_a_workspace(rt, c, h, w, outc):
+    """A K that is split over workgroups given one, and taken by this kernel without."""
+    import ctypes as C
+
+    from ncnn_amd.hip import Activation, ConvDesc, DeviceBuffer, check, lib
+    print("[case] conv few tiles, no workspace", c, h, w, outc, flush=True)
+    assert cases.conv_route(1, c, h, w, outc, (1, 1)).splits > 1
+    x, wq, b, ws, ins, _ = cases.conv_case(c, c, h, w, outc, (1, 1), 1, 2, True, True)
+    d = oracle.make_desc((c, h, w), outc, (1, 1), (1, 1), (1, 1), NONE, 0.0, 1, 1, 2, 0, (0.0, 0.0))
+    want = oracle.convolution_int8(d, x[0], wq, b, ws, ins[0], None)
+    desc, size = ConvDesc(w, h, c, 1, outc, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 0.0, 1), C.c_size_t()
+    check(lib().ncnnhip_conv_nhwc_sizes(C.byref(desc), None, C.byref(size), None))
+    packed = np.empty(size.value, np.int8)
+    check(lib().ncnnhip_conv_pack_weights(C.byref(desc), np.ascontiguousarray(wq, np.int8).ctypes.data, packed.ctypes.data))
+    keep = rt.to_channels_last(x), rt.up(packed), rt.up(rt.fold_input_scales(ws, ins, outc)), rt.up(np.asarray(b, F))
+    out = DeviceBuffer.empty((1, h * w, (outc + 15) // 16 * 16), F)
+    check(lib().ncnnhip_conv_int8_nhwc(C.byref(desc), keep[0].ptr, keep[1].ptr, keep[2].ptr, keep[3].ptr, None, Activation.make(0, (0.0, 0.0)), out.ptr, 1, 0, 0, None, 0,
+                                       rt.stream))
+    assert np.array_equal(rt.from_channels_last(out, 1, outc, h, w)[0], want)
+
+
 @pytest.mark.parametrize("batch,c,hw,outc,kernel,pads,relu", [(1, 64, 5, 40, (1, 1), NONE, True), (1, 256, 14, 200, (3, 3), SAME3, False),
                                                               (1, 128, 28, 140, (1, 1), NONE, True), (1, 128, 63, 60, (1, 1), NONE, False)])
 def test_few_tiles_kernel_fused_tail(rt, batch, c, hw, outc, kernel, pads, relu):
