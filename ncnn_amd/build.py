@@ -22,7 +22,7 @@ HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-cont
 # VGPRs instead of AGPRs, which saves a register read per value (tiled kernel 135 -> 125 us at 1024 x 4096 x 4096).
 # attention.hip: the same for the scores and the context on their way into the softmax arithmetic (attention core of 1500 tokens 183 -> 155 us).
 HIPCC_FILE_FLAGS = {"blockquant.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "blockquant_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "blockquant_tiles.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-                    "conv_pointwise.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "conv_resident.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+                    "conv_pointwise.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "conv_stream.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"], "conv_resident.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _run(cmd):

@@ -101,6 +101,7 @@ int launch_conv_pointwise(const NhwcGeom& g, const int8_t* wpk, const int8_t* x,
 // pointwise and weights-resident kernels, which want many pixels.
 int conv_stream_tile(const NhwcGeom& g, bool fp32_out); // 0: it does not, else pixels / 16 * 10 + channels / 16
 int conv_stream_tile_any_k(const NhwcGeom& g); // its smaller tiles whatever K is: for a layer whose K split has no workspace
+bool conv_stream_tile_out_of_reach(const NhwcGeom& g); // ... but for its operands, 2 GiB or more
 int launch_conv_stream(const NhwcGeom& g, int tile, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream);
 
 // The same two kernels with a projection shortcut (g: the main 1x1 convolution, stride 1, unpadded, channels in whole steps).

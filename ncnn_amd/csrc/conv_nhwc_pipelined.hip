@@ -159,11 +159,16 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
         const bool split = workspace && workspace_bytes >= need;
         const int tile = split ? 0 : conv_stream_tile_any_k(g_in);
         if (tile) return launch_conv_stream(g_in, tile, wpk, x, epi, fusion, out_cp, stream);
-        NCNNHIP_REQUIRE(split, "convolution: workspace of %zu bytes required", need);
-        counters = (unsigned*)workspace; // zero on entry (the caller cleared the workspace once), zero again on exit
-        partial = (int32_t*)((char*)workspace + SPLIT_COUNTER_BYTES);
+        if (!split && conv_stream_tile_out_of_reach(g_in))
+            p.splits = 1; // (an input of 2 GiB under a few tiles: K stays whole)
+        else
+        {
+            NCNNHIP_REQUIRE(split, "convolution: workspace of %zu bytes required", need);
+            counters = (unsigned*)workspace; // zero on entry (the caller cleared the workspace once), zero again on exit
+            partial = (int32_t*)((char*)workspace + SPLIT_COUNTER_BYTES);
+        }
     }
-    dim3 grid((unsigned)blocks), block((unsigned)(256 * p.groups));
+    dim3 grid((unsigned)((long long)p.tiles_m * p.tiles_n * p.splits)), block((unsigned)(256 * p.groups));
     if (p.splits > 1) return launch_pipe_split(p, mode, wpk, x, g, epi, fusion, out_cp, out_cp, partial, counters, stream);
 #define LAUNCH_PIPE_MODE(BM_, BN_, MODE_, GROUPS_)                                                                                                                 \
     hipLaunchKernelGGL((conv_nhwc_pipelined_kernel<BM_, BN_, PIPE_RING, false, MODE_, 1, GROUPS_>), grid, block, 0, stream, wpk, x, g, epi, fusion, out_cp, \

@@ -27,7 +27,8 @@ bool conv_shortcut_pays(const NhwcGeom& g, int shortcut_steps)
 int launch_conv_shortcut(const NhwcGeom& g_in, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
                          hipStream_t stream)
 {
-    if (conv_stream_shortcut_tile(g_in, sc.Cp / 64)) return launch_conv_stream_shortcut(g_in, wpk, x, sc, epi, fusion, out_cp, stream);
+    const long long sc_bytes = (long long)(g_in.npix / (sc.outw * sc.outh)) * sc.H * sc.W * sc.Cp;
+    if (conv_stream_shortcut_tile(g_in, sc.Cp / 64) && sc_bytes < (1ll << 31)) return launch_conv_stream_shortcut(g_in, wpk, x, sc, epi, fusion, out_cp, stream);
     NhwcGeom g = g_in;
     g.H = g.outh = 1;
     g.W = g.outw = g.npix;

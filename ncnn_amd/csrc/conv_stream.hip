@@ -1,6 +1,6 @@
 // int8 Convolution (group 1, zero border) on channels-last blobs, for layers with few output tiles: a workgroup owns 16 or 32 pixels x 16
-// or 32 channels and each of its four wavefronts multiplies the whole tile over a run of K steps of its own, operands straight from
-// global memory into registers in the order the matrix cores take them, 96 registers of loads in flight at once.
+// or 32 channels and each of its wavefronts multiplies the whole tile over a run of K steps of its own, operands straight from
+// global memory into registers in the order the matrix cores take them.
 //
 // Bound by latency: with no more tiles than compute units nothing overlaps a tile but its own loads, and the pipelined kernel
 // (conv_nhwc_pipelined_kernel.h) walks K behind a barrier per 64 bytes, about 190 ns each, where here a layer is one trip to memory, a few
@@ -8,6 +8,13 @@
 //
 // v_mfma_i32_16x16x64_i8 with weights as the A operand: a lane's four results are four neighbouring channels of one pixel, so the
 // epilogue needs no transpose: four entries of each table, one 16-byte fp32 store and residual load, one 4-byte int8 store.
+//
+// One trip to memory means one: every load of the tile, the epilogue's tables among them, is issued before the first product (left alone the compiler
+// puts products between the loads and waits for each, which was a second trip).  Loads go through buffer descriptors: a step is an immediate offset, and what lies
+// outside the image, the run of steps or the tables is an offset beyond the buffer, which answers zero without a fetch.  us in a captured chain, weights from HBM,
+// before / here: 1x1 512 -> 128 on 28 x 28 3.7 / 2.9, 1024 -> 256 on 14 x 14 3.7 / 2.9, 256 -> 1024 with the fused tail 4.1 / 3.0, 3x3 256 -> 256 4.6 / 4.0,
+// 3x3 512 -> 512 on 7 x 7 7.2 / 6.4, 1x1 512 -> 2048 4.4 / 3.2, 960 -> 160 3.2 / 2.4; inside a workgroup the operands arrive 1.9 to 3.1 us after its first
+// instruction before and 1.2 to 2 here, of which 0.25 were the arguments and 1.4 the issue of loads between waits.
 #include "conv_nhwc.h"
 
 namespace ncnnhip {
@@ -15,20 +22,89 @@ namespace ncnnhip {
 typedef int v4i_cs __attribute__((ext_vector_type(4)));
 typedef float v4f_cs __attribute__((ext_vector_type(4)));
 
-// a line of zeros for operands outside the image or beyond the last K step
-static __device__ __attribute__((aligned(64))) int8_t g_stream_zero_line[64];
+constexpr unsigned BEYOND = 0x80000000u; // an offset beyond every buffer here (their sizes are below 2^31: stream_reaches)
 
-constexpr int W = 4; // wavefronts a workgroup has
+static __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, unsigned bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+static __device__ __forceinline__ v4i_cs load16(__amdgpu_buffer_rsrc_t buffer, unsigned offset)
+{
+    return __builtin_bit_cast(v4i_cs, __builtin_amdgcn_raw_buffer_load_b128(buffer, (int)offset, 0, 0));
+}
+static __device__ __forceinline__ float load_float(__amdgpu_buffer_rsrc_t buffer, unsigned offset)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer, (int)offset, 0, 0));
+}
+
+// How a step of 64 bytes of K finds its pixels where the layer is not dense.
+struct StreamTaps
+{
+    int H, W, kw, dh, dw, sh, sw, pad_top, pad_left, outw, plane; // plane: output pixels of an image
+    int steps; // of one tap
+    unsigned magic_plane, magic_outw, magic_steps, magic_kw;
+};
+
+// n / d for n below 2^16 or so, d == 1 ? n : n * (2^32 / d + 1) >> 32, exact while n * d < 2^32
+static __device__ __forceinline__ int magic_div(int n, int d, unsigned magic)
+{
+    return d == 1 ? n : (int)__umulhi((unsigned)n, magic);
+}
+static unsigned magic_of(int d)
+{
+    return d > 1 ? (unsigned)((1ull << 32) / (unsigned)d + 1) : 0u;
+}
+
+// A shortcut as the kernel walks it.
+struct StreamShortcut : ConvShortcut
+{
+    unsigned x_bytes;
+    int per_wave; // steps
+    int plane;
+    unsigned magic_plane, magic_outw;
+};
+template<bool PRESENT>
+struct StreamShortcutArg
+{
+};
+template<>
+struct StreamShortcutArg<true> : StreamShortcut
+{
+};
+
+// What a workgroup needs once its operands are on their way, and how it finds them where that is not simple.
+struct StreamEpilogue
+{
+    const float* scale_in;
+    const float* bias;
+    const float* scale_out;
+    const float* residual;
+    void* out;
+    int8_t* q8_out;
+    float q8_scale;
+    int relu_after;
+    ncnnhip_activation act;
+};
+template<bool SHORTCUT>
+struct StreamRest
+{
+    StreamEpilogue epi;
+    StreamShortcutArg<SHORTCUT> shortcut;
+    StreamTaps taps;
+};
 
 // DENSE: 1x1, stride 1, unpadded: output pixel = input pixel.  Otherwise taps of whole 64-byte steps, so that a step lies inside one tap.
-// TP, TC: 16-pixel and 16-channel blocks of a tile.
-// SHORTCUT: a projection shortcut is added (ConvShortcut), its K dealt out to the wavefronts and its sums met in the same way.
-template<bool DENSE, int TP, int TC, bool SHORTCUT = false>
-__global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __restrict__ wpk, const int8_t* __restrict__ x, NhwcGeom g, ConvEpilogue epi, ConvFusion fusion,
-                                                             int out_cp, int tiles_m, unsigned magic_m, int per_wave, ConvShortcutArg<SHORTCUT> shortcut)
+// TP, TC: 16-pixel and 16-channel blocks of a tile.  U: K steps a wavefront has in flight, at 4 (TP + TC) registers each; W: wavefronts.
+// SHORTCUT: a projection shortcut is added (ConvShortcut), its K dealt out to the wavefronts and its sums met in the same way; both convolutions'
+// loads are in flight together.
+// The arguments before `rest` are 56 bytes and arrive in registers (amdgpu-kernarg-preload-count), so that the first loads wait for no other; of
+// `rest` the epilogue's part is read behind them, through a pointer that the compiler cannot move the reads across.
+template<bool DENSE, int TP, int TC, int U, int W, bool SHORTCUT = false>
+__global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __restrict__ wpk, const int8_t* __restrict__ x, unsigned x_bytes, int K, int Cp, int npix, int cout,
+                                                             int out_cp, int tiles, int tiles_m, unsigned magic_m, int per_wave,
+                                                             StreamRest<SHORTCUT> rest)
 {
-    constexpr int U = 24 / (TP + TC); // K steps a wavefront has in flight, in 96 registers
-    constexpr int NB = TP * TC;     // 16 x 16 blocks of the tile
+    constexpr int NB = TP * TC; // 16 x 16 blocks of the tile
     static_assert(NB <= W, "a wavefront finishes one block");
     static_assert(!SHORTCUT || DENSE, "the sum's main convolution is 1x1");
     __shared__ v4i_cs part[SHORTCUT ? 2 : 1][W][NB][64]; // [wavefront][block][lane]
@@ -38,155 +114,77 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
     // XCD x gets the x-th contiguous share of the tiles, the pixel tiles of one channel tile side by side: its weights cross to one XCD
     int b = blockIdx.x;
     {
-        const int T = gridDim.x, xcd = b & 7, idx = b >> 3, rem = T & 7;
-        b = xcd * (T >> 3) + (xcd < rem ? xcd : rem) + idx;
+        const int xcd = b & 7, idx = b >> 3, rem = tiles & 7;
+        b = xcd * (tiles >> 3) + (xcd < rem ? xcd : rem) + idx;
     }
-    const int tn = tiles_m == 1 ? b : (int)__umulhi((unsigned)b, magic_m);
+    const int tn = magic_div(b, tiles_m, magic_m);
     const int pix0 = (b - tn * tiles_m) * (16 * TP), ch0 = tn * (16 * TC);
 
-    const int total = g.K / 64;
-    const int begin = wave * per_wave, end = begin + per_wave < total ? begin + per_wave : total;
+    const int total = K / 64;
+    int s0 = wave * per_wave;
+    const int end = s0 + per_wave < total ? s0 + per_wave : total;
 
-    // wavefront q < NB finishes block q: what it needs from memory, requested before the operands (clamped addresses, nothing selected)
-    const int ch4 = ch0 + wave / TP * 16 + 4 * kq, pix = pix0 + wave % TP * 16 + r16;
-    float s_in[4], bias[4], s_out[4];
-    float sc_in[4], sc_bias[4];
-    v4f_cs res;
-    const bool to_int8 = epi.scale_out != 0, with_residual = !to_int8 && fusion.residual != 0;
-    if (wave < NB)
-    {
-        const float* bias_src = epi.bias ? epi.bias : epi.scale_in;
-        const float* s_out_src = epi.scale_out ? epi.scale_out : epi.scale_in;
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-        {
-            const int ch = ch4 + e < g.cout ? ch4 + e : g.cout - 1;
-            s_in[e] = epi.scale_in[ch];
-            bias[e] = bias_src[ch];
-            s_out[e] = s_out_src[ch];
-        }
-        if constexpr (SHORTCUT)
-        {
-            const float* sc_bias_src = shortcut.bias ? shortcut.bias : shortcut.scale_in;
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-            {
-                const int ch = ch4 + e < g.cout ? ch4 + e : g.cout - 1;
-                sc_in[e] = shortcut.scale_in[ch];
-                sc_bias[e] = sc_bias_src[ch];
-            }
-        }
-        if (with_residual) res = *reinterpret_cast<const v4f_cs*>(fusion.residual + (size_t)(pix < g.npix ? pix : g.npix - 1) * out_cp + (ch4 < out_cp ? ch4 : out_cp - 4));
-    }
-
-    const int8_t* zero = g_stream_zero_line + kq * 16;
-    const int8_t* w_row[TC];
-    const int8_t* x_row[TP]; // dense: the pixel's chunk; else the pixel's image
+    const __amdgpu_buffer_rsrc_t w_buf = buffer_of(wpk, (unsigned)(cout * K)), x_buf = buffer_of(x, x_bytes);
+    const StreamTaps& g = rest.taps;
+    unsigned beyond = BEYOND;
+    asm volatile("" : "+v"(beyond)); // (in a register: steps stay immediate offsets)
+    unsigned w_off[TC], x_off[TP]; // dense: the pixel's bytes of step s0; else those of its first tap's channels
     int iy0[TP], ix0[TP];
 #pragma unroll
     for (int i = 0; i < TC; i++)
     {
         const int ch = ch0 + i * 16 + r16;
-        w_row[i] = wpk + (size_t)(ch < g.cout ? ch : g.cout - 1) * g.K + kq * 16; // (a channel beyond the last: its products are not used)
+        w_off[i] = ch < cout ? (unsigned)(ch * K + s0 * 64 + kq * 16) : beyond;
     }
 #pragma unroll
     for (int i = 0; i < TP; i++)
     {
-        const int p = pix0 + i * 16 + r16, n = p < g.npix ? p : g.npix - 1;       // (nor are a pixel's)
-        iy0[i] = ix0[i] = 0;
+        const int p = pix0 + i * 16 + r16;
         if (DENSE)
-            x_row[i] = x + (size_t)n * g.Cp + kq * 16;
+            x_off[i] = p < npix ? (unsigned)(p * Cp + s0 * 64 + kq * 16) : beyond; // (the last step may reach into the next pixel, whose bytes meet zero weights)
         else
         {
-            const int img = small_div(n, g.outw * g.outh), at = n - img * (g.outw * g.outh), oy = small_div(at, g.outw);
-            iy0[i] = oy * g.sh - g.pad_top;
+            const int img = magic_div(p, g.plane, g.magic_plane), at = p - img * g.plane, oy = magic_div(at, g.outw, g.magic_outw);
+            iy0[i] = p < npix ? oy * g.sh - g.pad_top : -0x40000000; // a pixel beyond the last fails every bounds test
             ix0[i] = (at - oy * g.outw) * g.sw - g.pad_left;
-            x_row[i] = x + (size_t)img * g.H * g.W * g.Cp + kq * 16;
+            x_off[i] = (unsigned)(((img * g.H + iy0[i]) * g.W + ix0[i]) * Cp + kq * 16);
         }
     }
-    int tap = 0, q0 = 0, ky = 0, kx = 0; // the same in every lane
+    int q = 0, ky = 0, kx = 0; // step inside the tap, and the tap: the same in every lane
     if (!DENSE)
     {
-        tap = begin * 64 / g.tapK;
-        q0 = begin * 64 - tap * g.tapK;
-        ky = tap / g.kw;
+        const int tap = magic_div(s0, g.steps, g.magic_steps);
+        q = s0 - tap * g.steps;
+        ky = magic_div(tap, g.kw, g.magic_kw);
         kx = tap - ky * g.kw;
     }
 
-    if constexpr (SHORTCUT)
-    {
-        const int8_t* sw_row[TC];
-        const int8_t* sx_row[TP];
-#pragma unroll
-        for (int i = 0; i < TC; i++)
-        {
-            const int ch = ch0 + i * 16 + r16;
-            sw_row[i] = shortcut.wpk + (size_t)(ch < g.cout ? ch : g.cout - 1) * shortcut.Cp + kq * 16;
-        }
-#pragma unroll
-        for (int i = 0; i < TP; i++)
-        {
-            const int p = pix0 + i * 16 + r16, n = p < g.npix ? p : g.npix - 1, plane = shortcut.outw * shortcut.outh;
-            const int img = small_div(n, plane), at = n - img * plane, oy = small_div(at, shortcut.outw), ox = at - oy * shortcut.outw;
-            sx_row[i] = shortcut.x + (((size_t)img * shortcut.H + oy * shortcut.sh) * shortcut.W + ox * shortcut.sw) * shortcut.Cp + kq * 16;
-        }
-        const int steps = shortcut.Cp / 64, share = (steps + W - 1) / W;
-        const int from = wave * share, to = from + share < steps ? from + share : steps;
-        v4i_cs sum[NB];
-#pragma unroll
-        for (int q = 0; q < NB; q++) sum[q] = v4i_cs{0, 0, 0, 0};
-        for (int s0 = from; s0 < to; s0 += U)
-        {
-            v4i_cs fw[U][TC], fx[U][TP];
-#pragma unroll
-            for (int u = 0; u < U; u++)
-            {
-#pragma unroll
-                for (int i = 0; i < TC; i++) fw[u][i] = *reinterpret_cast<const v4i_cs*>(s0 + u < to ? sw_row[i] + (size_t)(s0 + u) * 64 : zero);
-#pragma unroll
-                for (int i = 0; i < TP; i++) fx[u][i] = *reinterpret_cast<const v4i_cs*>(s0 + u < to ? sx_row[i] + (size_t)(s0 + u) * 64 : zero);
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++)
-#pragma unroll
-                for (int q = 0; q < NB; q++) sum[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[u][q / TP], fx[u][q % TP], sum[q], 0, 0, 0);
-        }
-#pragma unroll
-        for (int q = 0; q < NB; q++) part[1][wave][q][lane] = sum[q];
-    }
-
-    v4i_cs acc[NB]; // channel block q / TP, pixel block q % TP
-#pragma unroll
-    for (int q = 0; q < NB; q++) acc[q] = v4i_cs{0, 0, 0, 0};
-    for (int s0 = begin; s0 < end; s0 += U)
-    {
-        v4i_cs fw[U][TC], fx[U][TP];
+    v4i_cs fw[U][TC], fx[U][TP];
+    auto issue = [&] {
 #pragma unroll
         for (int u = 0; u < U; u++)
         {
-            const int s = s0 + u;
-            const bool live = s < end; // a step beyond the run multiplies zeros
+            const bool live = s0 + u < end; // a step beyond the run is nothing but zeros
 #pragma unroll
-            for (int i = 0; i < TC; i++) fw[u][i] = *reinterpret_cast<const v4i_cs*>(live ? w_row[i] + (size_t)s * 64 : zero);
-#pragma unroll
-            for (int i = 0; i < TP; i++)
+            for (int i = 0; i < TC; i++) fw[u][i] = load16(w_buf, (live ? w_off[i] : beyond) + u * 64);
+            if (DENSE)
             {
-                if (DENSE)
-                    fx[u][i] = *reinterpret_cast<const v4i_cs*>(live && s * 64 + kq * 16 < g.tapK ? x_row[i] + (size_t)s * 64 : zero);
-                else
-                {
-                    const int iy = iy0[i] + ky * g.dh, ix = ix0[i] + kx * g.dw;
-                    const bool in = live && tap < g.ntaps && (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W;
-                    fx[u][i] = *reinterpret_cast<const v4i_cs*>(in ? x_row[i] + ((size_t)iy * g.W + ix) * g.Cp + q0 : zero);
-                }
+#pragma unroll
+                for (int i = 0; i < TP; i++) fx[u][i] = load16(x_buf, (live ? x_off[i] : beyond) + u * 64);
             }
-            if (!DENSE)
+            else
             {
-                q0 += 64;
-                if (q0 >= g.tapK)
+                const int dy = ky * g.dh, dx = kx * g.dw;
+                const unsigned at = (unsigned)((dy * g.W + dx) * Cp + q * 64);
+#pragma unroll
+                for (int i = 0; i < TP; i++)
                 {
-                    q0 = 0;
-                    tap++;
+                    const bool in = live && (unsigned)(iy0[i] + dy) < (unsigned)g.H && (unsigned)(ix0[i] + dx) < (unsigned)g.W;
+                    fx[u][i] = load16(x_buf, in ? x_off[i] + at : beyond);
+                }
+                if (++q == g.steps)
+                {
+                    q = 0;
                     if (++kx == g.kw)
                     {
                         kx = 0;
@@ -195,17 +193,138 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
                 }
             }
         }
+        s0 += U;
+#pragma unroll
+        for (int i = 0; i < TC; i++) w_off[i] += U * 64;
+        if (DENSE)
+        {
+#pragma unroll
+            for (int i = 0; i < TP; i++) x_off[i] += U * 64;
+        }
+    };
+    issue();
+
+    __builtin_amdgcn_sched_barrier(0);
+    const __attribute__((address_space(4))) char* rest_at = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() + 56;
+    asm volatile("" : "+s"(rest_at));
+    const StreamRest<SHORTCUT>& late = *(const StreamRest<SHORTCUT>*)rest_at;
+    const StreamShortcutArg<SHORTCUT>& shortcut = late.shortcut;
+    const float* const scale_in = late.epi.scale_in;
+    const float* const bias_at = late.epi.bias;
+    const float* const scale_out = late.epi.scale_out;
+    const float* const residual = late.epi.residual;
+    void* const out = late.epi.out;
+    int8_t* const q8_out = late.epi.q8_out;
+    const float q8_scale = late.epi.q8_scale;
+    const int relu_after = late.epi.relu_after, act_type = late.epi.act.type;
+    asm volatile("" ::"s"(scale_in), "s"(bias_at), "s"(scale_out), "s"(residual), "s"(out), "s"(q8_out), "s"(q8_scale), "s"(relu_after), "s"(act_type)); // one read of them all
+
+    v4i_cs sw[SHORTCUT ? U : 1][TC], sx[SHORTCUT ? U : 1][TP];
+    unsigned sw_off[TC], sx_off[TP];
+    int t0 = 0, t_end = 0;
+    auto issue_shortcut = [&] {
+        if constexpr (SHORTCUT)
+        {
+            const __amdgpu_buffer_rsrc_t sw_buf = buffer_of(shortcut.wpk, (unsigned)(cout * shortcut.Cp)), sx_buf = buffer_of(shortcut.x, shortcut.x_bytes);
+#pragma unroll
+            for (int u = 0; u < U; u++)
+            {
+                const bool live = t0 + u < t_end;
+#pragma unroll
+                for (int i = 0; i < TC; i++) sw[u][i] = load16(sw_buf, (live ? sw_off[i] : beyond) + u * 64);
+#pragma unroll
+                for (int i = 0; i < TP; i++) sx[u][i] = load16(sx_buf, (live ? sx_off[i] : beyond) + u * 64);
+            }
+            t0 += U;
+#pragma unroll
+            for (int i = 0; i < TC; i++) sw_off[i] += U * 64;
+#pragma unroll
+            for (int i = 0; i < TP; i++) sx_off[i] += U * 64;
+        }
+    };
+    if constexpr (SHORTCUT)
+    {
+        const int steps = shortcut.Cp / 64;
+        t0 = wave * shortcut.per_wave;
+        t_end = t0 + shortcut.per_wave < steps ? t0 + shortcut.per_wave : steps;
+#pragma unroll
+        for (int i = 0; i < TC; i++)
+        {
+            const int ch = ch0 + i * 16 + r16;
+            sw_off[i] = ch < cout ? (unsigned)(ch * shortcut.Cp + t0 * 64 + kq * 16) : beyond;
+        }
+#pragma unroll
+        for (int i = 0; i < TP; i++)
+        {
+            const int p = pix0 + i * 16 + r16, img = magic_div(p, shortcut.plane, shortcut.magic_plane), at = p - img * shortcut.plane, oy = magic_div(at, shortcut.outw, shortcut.magic_outw), ox = at - oy * shortcut.outw;
+            sx_off[i] = p < npix ? (unsigned)(((img * shortcut.H + oy * shortcut.sh) * shortcut.W + ox * shortcut.sw) * shortcut.Cp + t0 * 64 + kq * 16) : beyond;
+        }
+        issue_shortcut();
+    }
+
+    // wavefront n < NB finishes block n: what it needs from memory, behind the operands (the others ask for nothing, without a branch: one would make every
+    // wavefront's first product wait for its last load)
+    const bool finishes = NB == W || wave < NB;
+    const int ch4 = ch0 + wave / TP * 16 + 4 * kq, pix = pix0 + wave % TP * 16 + r16;
+    float s_in[4], bias[4], s_out[4];
+    float sc_in[4], sc_bias[4];
+    const bool to_int8 = scale_out != 0, with_residual = !to_int8 && residual != 0;
+    const unsigned table = (unsigned)(cout * 4), table_at = finishes ? (unsigned)ch4 * 4 : beyond;
+    const __amdgpu_buffer_rsrc_t in_buf = buffer_of(scale_in, table), bias_buf = buffer_of(bias_at, bias_at ? table : 0), out_buf = buffer_of(scale_out, to_int8 ? table : 0);
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+    {
+        s_in[e] = load_float(in_buf, table_at + e * 4);
+        bias[e] = load_float(bias_buf, table_at + e * 4);
+        s_out[e] = load_float(out_buf, table_at + e * 4);
+    }
+    if constexpr (SHORTCUT)
+    {
+        const __amdgpu_buffer_rsrc_t sc_buf = buffer_of(shortcut.scale_in, table), sc_bias_buf = buffer_of(shortcut.bias, shortcut.bias ? table : 0);
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+        {
+            sc_in[e] = load_float(sc_buf, table_at + e * 4);
+            sc_bias[e] = load_float(sc_bias_buf, table_at + e * 4);
+        }
+    }
+    const __amdgpu_buffer_rsrc_t res_buf = buffer_of(residual, with_residual ? (unsigned)(npix * out_cp) * 4 : 0);
+    const v4f_cs res = __builtin_bit_cast(v4f_cs, load16(res_buf, finishes && pix < npix && ch4 < out_cp ? (unsigned)(pix * out_cp + ch4) * 4 : beyond));
+
+    v4i_cs acc[NB], other[NB]; // channel block n / TP, pixel block n % TP
+#pragma unroll
+    for (int n = 0; n < NB; n++) acc[n] = other[n] = v4i_cs{0, 0, 0, 0};
+    auto multiply = [&] {
+        __builtin_amdgcn_sched_barrier(0); // every load above before the first product
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int q = 0; q < NB; q++) acc[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[u][q / TP], fx[u][q % TP], acc[q], 0, 0, 0);
+            for (int n = 0; n < NB; n++) acc[n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[u][n / TP], fx[u][n % TP], acc[n], 0, 0, 0);
+        if constexpr (SHORTCUT)
+        {
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int n = 0; n < NB; n++) other[n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(sw[u][n / TP], sx[u][n % TP], other[n], 0, 0, 0);
+        }
+    };
+    multiply(); // (outside the loop, where its waits count the first round's loads alone)
+    while (s0 < end || t0 < t_end)
+    {
+        issue();
+        issue_shortcut();
+        multiply();
     }
 
     // the wavefronts' sums meet (integer addition: exact in any order)
 #pragma unroll
-    for (int q = 0; q < NB; q++) part[0][wave][q][lane] = acc[q];
+    for (int n = 0; n < NB; n++)
+    {
+        part[0][wave][n][lane] = acc[n];
+        if constexpr (SHORTCUT) part[1][wave][n][lane] = other[n];
+    }
     __syncthreads();
-    if (wave >= NB || ch4 >= out_cp || pix >= g.npix) return;
+    if (!finishes || ch4 >= out_cp || pix >= npix) return;
     v4i_cs sum = part[0][0][wave][lane];
 #pragma unroll
     for (int s = 1; s < W; s++) sum += part[0][s][wave][lane];
@@ -216,17 +335,17 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
     for (int e = 0; e < 4; e++)
     {
         f[e] = mul_rn((float)sum[e], s_in[e]);
-        f[e] = add_rn(f[e], epi.bias ? bias[e] : -0.f); // no bias: -0, the one value whose addition changes nothing
+        f[e] = add_rn(f[e], bias_at ? bias[e] : -0.f); // no bias: -0, the one value whose addition changes nothing
     }
-    if (epi.act.type == 1)
+    if (act_type == 1)
     {
 #pragma unroll
         for (int e = 0; e < 4; e++) f[e] = fmaxf(f[e], 0.f);
     }
-    else if (epi.act.type != 0)
+    else if (act_type != 0)
     {
 #pragma unroll
-        for (int e = 0; e < 4; e++) f[e] = apply_activation(f[e], epi.act);
+        for (int e = 0; e < 4; e++) f[e] = apply_activation(f[e], late.epi.act);
     }
     const size_t o = (size_t)pix * out_cp + ch4;
     if (to_int8)
@@ -236,24 +355,24 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
         float2int8_as_float_x4(f[0], f[1], f[2], f[3]);
 #pragma unroll
         for (int e = 0; e < 4; e++)
-            if (ch4 + e >= g.cout) f[e] = 0.f; // channels from cout up to out_cp are the blob's zero padding
-        *reinterpret_cast<uint32_t*>(static_cast<int8_t*>(epi.out) + o) = pack4_quantised(f[0], f[1], f[2], f[3]);
+            if (ch4 + e >= cout) f[e] = 0.f; // channels from cout up to out_cp are the blob's zero padding
+        *reinterpret_cast<uint32_t*>(static_cast<int8_t*>(out) + o) = pack4_quantised(f[0], f[1], f[2], f[3]);
         return;
     }
     v4f_cs v;
 #pragma unroll
-    for (int e = 0; e < 4; e++) v[e] = ch4 + e < g.cout ? f[e] : 0.f;
+    for (int e = 0; e < 4; e++) v[e] = ch4 + e < cout ? f[e] : 0.f;
     if constexpr (SHORTCUT)
     {
-        v4i_cs other = part[1][0][wave][lane];
+        v4i_cs sc = part[1][0][wave][lane];
 #pragma unroll
-        for (int s = 1; s < W; s++) other += part[1][s][wave][lane];
+        for (int s = 1; s < W; s++) sc += part[1][s][wave][lane];
 #pragma unroll
         for (int e = 0; e < 4; e++)
         {
-            float t = add_rn(mul_rn((float)other[e], sc_in[e]), shortcut.bias ? sc_bias[e] : -0.f);
+            float t = add_rn(mul_rn((float)sc[e], sc_in[e]), shortcut.bias ? sc_bias[e] : -0.f);
             if (shortcut.act.type != 0) t = apply_activation(t, shortcut.act);
-            v[e] = add_rn(v[e], ch4 + e < g.cout ? t : 0.f);
+            v[e] = add_rn(v[e], ch4 + e < cout ? t : 0.f);
         }
     }
     if (with_residual)
@@ -261,19 +380,19 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] = add_rn(v[e], res[e]);
     }
-    if (fusion.relu_after)
+    if (relu_after)
     {
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] = v[e] < 0.f ? 0.f : v[e]; // the ReLU LAYER's statement (src/layer/relu.cpp:36-37): a NaN stays, unlike fmaxf
     }
-    if (epi.out) *reinterpret_cast<v4f_cs*>(static_cast<float*>(epi.out) + o) = v;
-    if (fusion.q8_out)
+    if (out) *reinterpret_cast<v4f_cs*>(static_cast<float*>(out) + o) = v;
+    if (q8_out)
     {
         float q[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) q[e] = mul_rn(v[e], fusion.q8_scale);
+        for (int e = 0; e < 4; e++) q[e] = mul_rn(v[e], q8_scale);
         float2int8_as_float_x4(q[0], q[1], q[2], q[3]);
-        *reinterpret_cast<uint32_t*>(fusion.q8_out + o) = pack4_quantised(q[0], q[1], q[2], q[3]);
+        *reinterpret_cast<uint32_t*>(q8_out + o) = pack4_quantised(q[0], q[1], q[2], q[3]);
     }
 }
 
@@ -295,6 +414,7 @@ static bool stream_dense(const NhwcGeom& g)
 // A single tap with a stride (1x1, not dense) costs its pixels' divisions and, on the ring, no more than a dense one: the ring is ahead of the smaller tiles below
 // five steps to int8 (64 -> 256 on 28 x 28, stride 2, 3.1 / 3.8; 256 -> 256 3.6 / 3.7, 320 -> 256 3.8 / 3.6) and three to fp32 (128 3.5 / 3.6, 192 3.6 / 3.6), of
 // 32 x 32 below eight and six (four images, int8 384 4.0 / 4.1, 512 5.3 / 4.5; fp32 256 3.9 / 4.2, 384 4.2 / 4.1).
+// (The figures of this rule are of the loads' former issue, where a tile cost 0.5 to 1 us more: the lines below are on the safe side.)
 // Beyond some K the ring, which splits it over workgroups, is quicker again.  Weight rows an odd number of steps (64 bytes of K) apart come in at 1.3 times the
 // rate of an even number, so the lines lie further out there.  Time here over the ring's, fp32 out, dense:
 //   16 x 16, below 128 tiles   even: 144 steps 0.87-0.93, 176 0.94-0.99, 194 1.00-1.06, 288 1.03-1.09    odd: 193 0.8, 401 0.86-0.91, 641 0.88-0.95
@@ -315,20 +435,37 @@ static int stream_tile(const NhwcGeom& g, int steps, bool odd, bool fp32_out, in
     return m32 * n32 <= 256 && steps >= shortest && steps <= convolutions * 48 ? 22 : 0;
 }
 
-static bool stream_addressing(const NhwcGeom& g)
+// offsets are 32 bits wide and BEYOND lies beyond every buffer
+static bool stream_reaches(const NhwcGeom& g)
+{
+    const long long limit = 1ll << 31;
+    return (long long)(g.npix / (g.outw * g.outh)) * g.H * g.W * g.Cp < limit && (long long)g.cout * g.K < limit;
+}
+
+static bool stream_geometry(const NhwcGeom& g)
 {
     return stream_dense(g) || (g.tapK % 64 == 0 && g.tapK == g.Cp);
 }
 
 int conv_stream_tile(const NhwcGeom& g, bool fp32_out)
 {
-    return stream_addressing(g) ? stream_tile(g, g.K / 64, g.K / 64 % 2 == 1, fp32_out, 1) : 0;
+    return stream_geometry(g) && stream_reaches(g) ? stream_tile(g, g.K / 64, g.K / 64 % 2 == 1, fp32_out, 1) : 0;
+}
+
+static int stream_tile_any_k(const NhwcGeom& g)
+{
+    const long long m16 = ceil_div(g.npix, 16);
+    return !stream_geometry(g) ? 0 : m16 * ceil_div(g.cout, 16) <= 256 ? 11 : m16 * ceil_div(g.cout, 32) <= 256 ? 12 : 0;
 }
 
 int conv_stream_tile_any_k(const NhwcGeom& g)
 {
-    const long long m16 = ceil_div(g.npix, 16);
-    return !stream_addressing(g) ? 0 : m16 * ceil_div(g.cout, 16) <= 256 ? 11 : m16 * ceil_div(g.cout, 32) <= 256 ? 12 : 0;
+    return stream_reaches(g) ? stream_tile_any_k(g) : 0;
+}
+
+bool conv_stream_tile_out_of_reach(const NhwcGeom& g)
+{
+    return stream_tile_any_k(g) != 0 && !stream_reaches(g);
 }
 
 // With a shortcut a workgroup walks both K, one after the other, in place of two launches that walk one each: the limits hold for the two together.
@@ -337,35 +474,84 @@ int conv_stream_tile_any_k(const NhwcGeom& g)
 // 48 + 48 17.7 / 15.5, 64 + 32 17.3 / 16.5 (35.8); beyond its limit two launches are quicker than the ring (conv_shortcut_pays).
 int conv_stream_shortcut_tile(const NhwcGeom& g, int shortcut_steps)
 {
-    return stream_dense(g) && g.K == g.Cp ? stream_tile(g, g.K / 64 + shortcut_steps, g.K / 64 % 2 == 1 && shortcut_steps % 2 == 1, true, 2) : 0;
+    return stream_dense(g) && g.K == g.Cp && stream_reaches(g) ? stream_tile(g, g.K / 64 + shortcut_steps, g.K / 64 % 2 == 1 && shortcut_steps % 2 == 1, true, 2) : 0;
+}
+
+// Steps in flight (U) and wavefronts (W) for this many steps of K: a round costs a trip to memory, and a step that only fills up a round its loads' issue.
+// blocks: 16-byte operands a lane holds per step; 36 of them, 144 registers, are in flight at most.  Eight wavefronts from 49 steps on, where four would walk
+// two rounds: 3x3 512 -> 512 on 7 x 7 (72 steps) 7.2 -> 6.4 us, 1x1 4096 -> 512 6.9 -> 6.0.
+struct StreamForm
+{
+    int u, w;
+};
+constexpr bool stream_form_built(int u, int blocks)
+{
+    return u * blocks <= 36;
+}
+static StreamForm stream_form(int steps, int blocks)
+{
+    const int w = ceil_div(steps, 4) > 12 ? 8 : 4, per_wave = ceil_div(steps, w);
+    StreamForm best = {1, w};
+    for (int u : {2, 4, 6, 9, 12})
+        if (stream_form_built(u, blocks) && ceil_div(per_wave, u) < ceil_div(per_wave, best.u)) best.u = u;
+    return best;
+}
+
+template<bool DENSE, int TP, int TC, int W, bool SHORTCUT>
+static void launch_stream_form(int u, const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
+                               const StreamShortcutArg<SHORTCUT>& shortcut, hipStream_t stream)
+{
+    const int tiles_m = ceil_div(g.npix, 16 * TP), tiles = tiles_m * ceil_div(g.cout, 16 * TC); // 256 at most
+    const int plane = g.outw * g.outh, steps = g.tapK / 64;
+    const unsigned x_bytes = (unsigned)(g.npix / plane) * g.H * g.W * g.Cp;
+    StreamRest<SHORTCUT> rest = {{epi.scale_in, epi.bias, epi.scale_out, fusion.residual, epi.out, fusion.q8_out, fusion.q8_scale, fusion.relu_after, epi.act}, shortcut, {}};
+    if (!DENSE)
+        rest.taps = {g.H, g.W, g.kw, g.dh, g.dw, g.sh, g.sw, g.pad_top, g.pad_left, g.outw, plane, steps, magic_of(plane), magic_of(g.outw), magic_of(steps), magic_of(g.kw)};
+    constexpr int blocks = (TP + TC) * (SHORTCUT ? 2 : 1);
+#define STREAM(U_)                                                                                                                                              \
+    if constexpr (stream_form_built(U_, blocks))                                                                                                                \
+        if (u == U_)                                                                                                                                            \
+    hipLaunchKernelGGL((conv_stream_kernel<DENSE, TP, TC, U_, W, SHORTCUT>), dim3((unsigned)tiles), dim3(64 * W), 0, stream, wpk, x, x_bytes, g.K, g.Cp, g.npix, \
+                       g.cout, out_cp, tiles, tiles_m, magic_of(tiles_m), ceil_div(g.K / 64, W), rest)
+    STREAM(1);
+    STREAM(2);
+    STREAM(4);
+    STREAM(6);
+    STREAM(9);
+    STREAM(12);
+#undef STREAM
+}
+
+template<bool DENSE, bool SHORTCUT>
+static void launch_stream_tile(int tile, int steps, const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
+                               StreamShortcutArg<SHORTCUT> shortcut, hipStream_t stream)
+{
+    const StreamForm form = stream_form(steps, (tile / 10 + tile % 10) * (SHORTCUT ? 2 : 1));
+    if constexpr (SHORTCUT) shortcut.per_wave = ceil_div(shortcut.Cp / 64, form.w);
+#define STREAM_TILE(TP_, TC_)                                                                                                      \
+    do                                                                                                                             \
+    {                                                                                                                              \
+        if (form.w == 8)                                                                                                           \
+            launch_stream_form<DENSE, TP_, TC_, 8, SHORTCUT>(form.u, g, wpk, x, epi, fusion, out_cp, shortcut, stream);            \
+        else                                                                                                                       \
+            launch_stream_form<DENSE, TP_, TC_, 4, SHORTCUT>(form.u, g, wpk, x, epi, fusion, out_cp, shortcut, stream);            \
+    } while (0)
+    if (tile == 11)
+        STREAM_TILE(1, 1);
+    else if (tile == 12)
+        STREAM_TILE(1, 2);
+    else
+        STREAM_TILE(2, 2);
+#undef STREAM_TILE
 }
 
 int launch_conv_stream(const NhwcGeom& g, int tile, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream)
 {
-    const int tp = tile / 10, tc = tile % 10;
     NCNNHIP_REQUIRE(tile && !epi.acc_out, "convolution: this layer does not fit the kernel for few tiles");
-    const int tiles_m = ceil_div(g.npix, 16 * tp), tiles_n = ceil_div(g.cout, 16 * tc), blocks = tiles_m * tiles_n; // 256 at most
-    const unsigned magic_m = tiles_m > 1 ? (unsigned)((1ull << 32) / (unsigned)tiles_m + 1) : 0u;
-    const int per_wave = ceil_div(g.K / 64, W);
-#define STREAM(DENSE_, TP_, TC_)                                                                                                                            \
-    hipLaunchKernelGGL((conv_stream_kernel<DENSE_, TP_, TC_>), dim3((unsigned)blocks), dim3(64 * W), 0, stream, wpk, x, g, epi, fusion, out_cp, tiles_m, magic_m, \
-                       per_wave, ConvShortcutArg<false>())
-#define STREAM_TILE(DENSE_)       \
-    do                            \
-    {                             \
-        if (tile == 11)           \
-            STREAM(DENSE_, 1, 1); \
-        else if (tile == 12)      \
-            STREAM(DENSE_, 1, 2); \
-        else                      \
-            STREAM(DENSE_, 2, 2); \
-    } while (0)
     if (stream_dense(g))
-        STREAM_TILE(true);
+        launch_stream_tile<true, false>(tile, g.K / 64, g, wpk, x, epi, fusion, out_cp, StreamShortcutArg<false>(), stream);
     else
-        STREAM_TILE(false);
-#undef STREAM_TILE
-#undef STREAM
+        launch_stream_tile<false, false>(tile, g.K / 64, g, wpk, x, epi, fusion, out_cp, StreamShortcutArg<false>(), stream);
     return launch_status("conv_stream_kernel");
 }
 
@@ -374,22 +560,16 @@ int launch_conv_stream(const NhwcGeom& g, int tile, const int8_t* wpk, const int
 int launch_conv_stream_shortcut(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion,
                                 int out_cp, hipStream_t stream)
 {
-    const int tile = conv_stream_shortcut_tile(g, sc.Cp / 64), tp = tile / 10, tc = tile % 10;
+    const int tile = conv_stream_shortcut_tile(g, sc.Cp / 64);
     NCNNHIP_REQUIRE(tile && sc.Cp % 64 == 0, "convolution: this layer does not fit the kernel for few tiles");
-    const int tiles_m = ceil_div(g.npix, 16 * tp), tiles_n = ceil_div(g.cout, 16 * tc);
-    const unsigned magic_m = tiles_m > 1 ? (unsigned)((1ull << 32) / (unsigned)tiles_m + 1) : 0u;
-    ConvShortcutArg<true> arg;
+    const int plane = sc.outw * sc.outh;
+    StreamShortcutArg<true> arg;
     static_cast<ConvShortcut&>(arg) = sc;
-#define STREAM(TP_, TC_)                                                                                                                                               \
-    hipLaunchKernelGGL((conv_stream_kernel<true, TP_, TC_, true>), dim3((unsigned)(tiles_m * tiles_n)), dim3(64 * W), 0, stream, wpk, x, g, epi, fusion, out_cp, tiles_m, \
-                       magic_m, ceil_div(g.K / 64, W), arg)
-    if (tile == 11)
-        STREAM(1, 1);
-    else if (tile == 12)
-        STREAM(1, 2);
-    else
-        STREAM(2, 2);
-#undef STREAM
+    arg.x_bytes = (unsigned)(g.npix / plane) * sc.H * sc.W * sc.Cp;
+    arg.plane = plane;
+    arg.magic_plane = magic_of(plane);
+    arg.magic_outw = magic_of(sc.outw);
+    launch_stream_tile<true, true>(tile, sc.Cp > g.K ? sc.Cp / 64 : g.K / 64, g, wpk, x, epi, fusion, out_cp, arg, stream);
     return launch_status("conv_stream_kernel (shortcut)");
 }
 

@@ -82,3 +82,9 @@ def _pays(batch, hw, outc, c, shortcut_c, stride=2):
 ], ids=str)
 def test_shortcuts_that_pay(batch, hw, outc, c, shortcut_c, pays):
     assert _pays(batch, hw, outc, c, shortcut_c) == pays
+
+
+def test_few_tiles_of_a_large_input():
+    """Offsets of the kernel for few tiles are 32 bits wide: an input of 2 GiB goes to the ring, one of just below does not."""
+    for batch, kernel in ((1, "FEW_TILES"), (2, "PIPELINED")):
+        assert getattr((r := cases.conv_route(batch, 320, 1900, 1900, 64, (1, 1), stride=(190, 190))), kernel) == r.kernel

@@ -103,3 +103,19 @@ def test_few_tiles_kernel_fused_tail(rt, batch, c, hw, outc, kernel, pads, relu)
     got, got_q = rt.conv_channels_last(x, wq, b, ws, ins, None, outc, kernel, (1, 1), (1, 1), pads, 0.0, 1, 2, 0, (0.0, 0.0), residual=res, relu_after=relu,
                                        quantise_scale=scale)
     assert np.array_equal(got, want, equal_nan=True) and np.array_equal(got_q, want_q)
+
+
+# Steps of K a wavefront has in flight at once (1, 2, 4, 6, 9, 12), rounds of them and eight wavefronts for more than 48 steps: each
+# side of every change, dense and with taps, on 16 x 16, 16 x 32 and 32 x 32 tiles; whole runs of steps left to no wavefront.
+@pytest.mark.parametrize("steps", [1, 4, 5, 8, 9, 13, 16, 17, 24, 25, 36, 37, 48, 49, 72, 73, 96, 97, 192])
+def test_few_tiles_kernel_runs_of_steps(rt, steps):
+    print("[case] conv few tiles, steps", steps, flush=True)
+    for c, hw, outc, kernel, pads in ((64 * steps, (3, 5), 33, (1, 1), NONE), (64 * steps, (16, 16), 290, (1, 1), NONE), (64 * steps, (31, 32), 96, (1, 1), NONE),
+                                      (64 * max(1, steps // 9), (5, 4), 20, (3, 3), SAME3), (64 * max(1, steps // 9), (15, 16), 300, (3, 3), SAME3)):
+        if c * outc * hw[0] * hw[1] * kernel[0] * kernel[1] > 1 << 30:
+            continue
+        x, wq, b, ws, ins, tops = cases.conv_case(steps + outc, c, hw[0], hw[1], outc, kernel, 1, 102, True, True)
+        d = oracle.make_desc((c, hw[0], hw[1]), outc, kernel, (1, 1), (1, 1), pads, 0.0, 1, 1, 102, 1, (0.0, 0.0))
+        want = oracle.convolution_int8(d, x[0], wq, b, ws, ins[0], tops[0])
+        got = rt.conv_channels_last(x, wq, b, ws, ins, tops, outc, kernel, (1, 1), (1, 1), pads, 0.0, 1, 102, 1, (0.0, 0.0))
+        assert np.array_equal(got[0], want), (c, hw, outc, kernel)
