@@ -228,6 +228,34 @@ def test_fp32_rows_in_64x128_tiles(rt, m, n, k, bits, block):
     assert np.array_equal(got[1, :n][q != 0], np.where(q > 0, np.inf, -np.inf)[q != 0].astype(F)) and np.all(np.isnan(got[1, :n][q == 0])) and np.all(np.isnan(got[m - 1, :n]))
 
 
+@pytest.mark.parametrize("m,n,k,bits", [(130, 40, 4112, 8), (133, 130, 12304, 4), (129, 16, 12816, 8), (140, 24, 144, 6)])
+def test_fp32_rows_of_any_magnitude_in_64x128_tiles(rt, m, n, k, bits):
+    """Rows are scaled by a power of two before they are split: rows of zeros, of subnormals, next to the largest float, with few values of
+    any weight, over spans that fit the split pass's registers and beyond them.  An activation keeps 23 bits, which stay below 1e-6 of the floor with the sums' roundings, and
+    what lies above 2^-40 of its row's largest."""
+    a, packed, scales = synth.blockquant_operands(m + n, m, n, k, bits, 64, half_exact=False)
+    rng = np.random.default_rng(k)
+    scales *= 64  # outputs of the largest row stay finite
+    a[0] = 0
+    a[1], a[2], a[3] = a[1] * F(2.0 ** -130), a[2] * F(2.0 ** -112), a[3] * F(2.0 ** 120) / max(1, np.abs(a[3]).max())
+    a[4] *= np.exp2(rng.integers(-60, 60, k)).astype(F)
+    a[5, 1:] *= F(2.0 ** -35)
+    a[m - 1, : k - 1] = 0
+    pw, pd = rt.blockquant_pack(packed, scales, 64, bits=bits, k=k)
+    w, d = rt.up(pw), rt.up(pd)
+    size = C.c_size_t()
+    check(lib().ncnnhip_gemm_blockquant_packed_rows_workspace_bytes(m, k, C.byref(size)))
+    ws = DeviceBuffer.empty((size.value,), np.uint8)
+    src, dst = rt.up(np.concatenate([[F(0)], a.ravel()]).astype(F)), rt.up(np.full((m, n), 7.0, F))
+    check(lib().ncnnhip_gemm_blockquant_packed_rows(C.c_void_p(src.ptr.value + 4), k, m, n, k, w.ptr, d.ptr, bits, 64, None, None, -1, 1.0, 1.0, dst.ptr, n,
+                                                    ws.ptr, size.value, rt.stream))  # (off 16 bytes: not the one-launch form)
+    got = dst.to_numpy(rt.stream)
+    val, floor = npref.blockquant_gemm_f64(a, packed, scales, bits, 64)
+    assert np.all(np.isfinite(got)) and np.all(got[0] == 0)
+    ones = npref.blockquant_gemm_f64(np.ones((1, k), F), packed, scales, bits, 64)[1]
+    assert np.all(np.abs(got - val) <= 1e-6 * floor + 2.0 ** -40 * np.abs(a).max(axis=1, keepdims=True).astype(np.float64) * ones + 2.0 ** -148)
+
+
 def test_several_matrices_whose_groups_would_fill_the_units_only_together(rt):
     """3 x 256 tiles: in groups of three 258, in groups of four 192, which is what several matrices get; one matrix of all of them is 256 groups of three."""
     m, k, n = 48, 64, 4096
