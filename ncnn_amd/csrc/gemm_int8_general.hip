@@ -84,7 +84,11 @@ template<int BM, int BN, int KG, typename Epilogue>
 __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_t* __restrict__ A, size_t lda, const int8_t* __restrict__ B, size_t ldb, int M, int N, int K,
                                                                 int tiles_m, int tiles_n, Epilogue epi)
 {
-    constexpr int TM = BM / 64, TN = BN / 64;     // 32 x 32 blocks per wavefront
+    // a wavefront's share is BM / 2 x BN / 2, in blocks of 32 x 32 or, where that does not divide it, 16 x 16 (as many cycles and operand bytes a product)
+    constexpr int BLK = BM % 64 == 0 && BN % 64 == 0 ? 32 : 16;
+    constexpr int TM = BM / 2 / BLK, TN = BN / 2 / BLK;
+    constexpr int REGS = BLK * BLK / 64;
+    typedef int block_sums __attribute__((ext_vector_type(REGS)));
     constexpr int LA = BM / 32, LB = BN / 32;     // 16-byte loads per thread and operand: 32 rows of 8 chunks at a time
     constexpr int STEP_BYTES = (BM + BN) * KSTEP;
     static_assert(KG == 1 || BM * BN * 4 <= 2 * STEP_BYTES, "the sums of a group fit its buffers");
@@ -95,7 +99,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
     const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
     const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     int8_t* smem = smem_all + kg * 2 * STEP_BYTES;
-    const int wm = wave >> 1, wn = wave & 1, l32 = lane & 31, lhi = lane >> 5;
+    const int wm = wave >> 1, wn = wave & 1, lrow = lane & (BLK - 1), lhi = lane / BLK; // lhi: K chunk of the lane, and its rows of the sums
 
     // workgroups are dealt to the 8 dies in turn: each die takes a run of tiles that share rows of A and B in its own L2
     const int T = tiles_m * tiles_n;
@@ -161,8 +165,8 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
 
     // a wavefront with a single block keeps two sums of it: a product need not wait for the one before
     constexpr int SETS = TM * TN == 1 ? 2 : 1;
-    v16i accs[SETS][TM][TN];
-    v16i(&acc)[TM][TN] = accs[0];
+    block_sums accs[SETS][TM][TN];
+    block_sums(&acc)[TM][TN] = accs[0];
 #pragma unroll
     for (int s = 0; s < SETS; s++)
 #pragma unroll
@@ -170,27 +174,28 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
 #pragma unroll
             for (int j = 0; j < TN; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) accs[s][i][j][r] = 0;
-    int rd[4];
+                for (int r = 0; r < REGS; r++) accs[s][i][j][r] = 0;
+    constexpr int PARTS = BLK == 32 ? 4 : 2, CHUNKS = 8 / PARTS; // parts of a K step that one product takes, and their chunks
+    int rd[PARTS];
 #pragma unroll
-    for (int q = 0; q < 4; q++) rd[q] = l32 * KSTEP + (((2 * q + lhi) ^ (l32 >> 1)) & 7) * 16;
+    for (int q = 0; q < PARTS; q++) rd[q] = lrow * KSTEP + (((CHUNKS * q + lhi) ^ (lrow >> 1)) & 7) * 16;
     auto multiply = [&](int t) {
         const int8_t* sa = smem + (t & 1) * STEP_BYTES + wm * (BM / 2) * KSTEP;
         const int8_t* sb = smem + (t & 1) * STEP_BYTES + (BM + wn * (BN / 2)) * KSTEP;
-        // Q quarters of the step are read before they are multiplied: left to itself the compiler reads two operands, waits, multiplies and
+        // Q parts of the step are read before they are multiplied: left to itself the compiler reads two operands, waits, multiplies and
         // reads the next two into the same registers.  As many as leave the workgroups a unit holds their registers.
-        constexpr int Q = TM * TN == 1 && KG == 1 ? 2 : 1;
+        constexpr int Q = (TM * TN == 1 && KG == 1) || BLK == 16 ? 2 : 1;
 #pragma unroll
-        for (int q0 = 0; q0 < 4; q0 += Q)
+        for (int q0 = 0; q0 < PARTS; q0 += Q)
         {
             v4i fa[Q][TM], fb[Q][TN];
 #pragma unroll
             for (int q = 0; q < Q; q++)
             {
 #pragma unroll
-                for (int i = 0; i < TM; i++) fa[q][i] = *reinterpret_cast<const v4i*>(sa + i * 32 * KSTEP + rd[q0 + q]);
+                for (int i = 0; i < TM; i++) fa[q][i] = *reinterpret_cast<const v4i*>(sa + i * BLK * KSTEP + rd[q0 + q]);
 #pragma unroll
-                for (int j = 0; j < TN; j++) fb[q][j] = *reinterpret_cast<const v4i*>(sb + j * 32 * KSTEP + rd[q0 + q]);
+                for (int j = 0; j < TN; j++) fb[q][j] = *reinterpret_cast<const v4i*>(sb + j * BLK * KSTEP + rd[q0 + q]);
             }
             if (Q > 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -199,7 +204,13 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
                 for (int i = 0; i < TM; i++)
 #pragma unroll
                     for (int j = 0; j < TN; j++)
-                        accs[(q0 + q) % SETS][i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[q][i], fb[q][j], accs[(q0 + q) % SETS][i][j], 0, 0, 0);
+                    {
+                        block_sums& sum = accs[(q0 + q) % SETS][i][j];
+                        if constexpr (BLK == 32)
+                            sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[q][i], fb[q][j], sum, 0, 0, 0);
+                        else
+                            sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[q][i], fb[q][j], sum, 0, 0, 0);
+                    }
         }
     };
 
@@ -237,7 +248,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
 
     if (SETS == 2)
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[0][0][r] += accs[SETS - 1][0][0][r];
+        for (int r = 0; r < REGS; r++) acc[0][0][r] += accs[SETS - 1][0][0][r];
 
     if (KG > 1)
     {
@@ -248,8 +259,8 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
 #pragma unroll
             for (int j = 0; j < TN; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++)
-                    sums[(wm * (BM / 2) + i * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3)) * BN + wn * (BN / 2) + j * 32 + l32] = acc[i][j][r];
+                for (int r = 0; r < REGS; r++)
+                    sums[(wm * (BM / 2) + i * BLK + 8 * (r >> 2) + 4 * lhi + (r & 3)) * BN + wn * (BN / 2) + j * BLK + lrow] = acc[i][j][r];
         __syncthreads();
         // every thread finishes one column of the tile, every (256 * KG / BN)-th row
         const int in_col = threadIdx.x % BN, col = col0 + in_col;
@@ -271,24 +282,24 @@ __global__ __launch_bounds__(256 * KG) void gemm_int8_general_kernel(const int8_
 
     // the rows' values in one go, four consecutive ones at a time
     typedef float v4f_rows __attribute__((ext_vector_type(4)));
-    v4f_rows rows[TM][4];
+    v4f_rows rows[TM][REGS / 4];
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) rows[i][e] = *reinterpret_cast<const v4f_rows*>(row_value + wm * (BM / 2) + i * 32 + 8 * e + 4 * lhi);
+        for (int e = 0; e < REGS / 4; e++) rows[i][e] = *reinterpret_cast<const v4f_rows*>(row_value + wm * (BM / 2) + i * BLK + 8 * e + 4 * lhi);
 #pragma unroll
     for (int j = 0; j < TN; j++)
     {
-        const int col = col0 + wn * (BN / 2) + j * 32 + l32;
+        const int col = col0 + wn * (BN / 2) + j * BLK + lrow;
         if (col >= N) continue;
         float scale, add;
         epi.column(col, scale, add);
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int r = 0; r < 16; r++)
+            for (int r = 0; r < REGS; r++)
             {
-                const int in_tile = wm * (BM / 2) + i * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
+                const int in_tile = wm * (BM / 2) + i * BLK + 8 * (r >> 2) + 4 * lhi + (r & 3);
                 if (row0 + in_tile < M) epi.store(row0 + in_tile, col, acc[i][j][r], rows[i][r >> 2][r & 3], scale, add);
             }
     }
@@ -512,6 +523,17 @@ static int launch_any(const int8_t* a, size_t lda, const int8_t* b, size_t ldb, 
     // 32.1), with more rounds from 1300 (2816 x 2048 x 2004 32.0 -> 28.2; 1152 tiles the same), and not on a short K (2048 x 2048 x 508 10.7 11.8).
     const long long tiles = (long long)ceil_div(M, 64) * ceil_div(N, 64), tiles128 = (long long)ceil_div(M, 128) * ceil_div(N, 128);
     const bool words = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | lda | ldb) & 3) == 0;
+    // Tiles between the two where 64 x 64 ones would be two to some units and these are one to each: with 96 x 64 a unit reads 160 rows a step for 256.  us, 64 x 64 -> 96 x 64: off
+    // 16 bytes 1501 x 1000 x 2008 12.7 -> 11.7, 299 x 3801 x 389 8.7 -> 7.8, 2362 x 540 x 271 8.2 -> 7.4; aligned, two groups of wavefronts on a long K, 855 x 1504 x 6464
+    // 28.3 -> 22.3, 811 x 1544 x 6208 27.6 -> 21.5, 1294 x 1136 x 960 8.5 -> 8.3, and not on a short K, 999 x 1312 x 512 6.3 -> 6.6.  Off 16 bytes 96 x 96 for three and
+    // more 64 x 64 to a unit: 2902 x 740 x 1254 16.2 -> 12.8, 539 x 3870 x 549 12.9 -> 10.9, 264 x 7947 x 427 11.8 -> 10.1 (aligned 795 x 2608 x 704 9.3 -> 9.9).
+    const long long tiles96 = (long long)ceil_div(M, 96) * ceil_div(N, 64);
+    if (tiles > 256 && tiles <= 512 && tiles96 <= 256 && (aligned ? K >= 900 : K > 256))
+    {
+        if (K >= 3072) return launch_tile<96, 64, 2>(a, lda, b, ldb, M, N, K, epi, stream);
+        return launch_tile<96, 64, 1>(a, lda, b, ldb, M, N, K, epi, stream);
+    }
+    if (!aligned && tiles > 512 && K >= 400 && (long long)ceil_div(M, 96) * ceil_div(N, 96) <= 256) return launch_tile<96, 96, 1>(a, lda, b, ldb, M, N, K, epi, stream);
     if (!aligned && K >= 1000 && tiles >= (tiles128 > 256 ? 1300 : words ? 800 : 600)) return launch_tile<128, 128, 1>(a, lda, b, ldb, M, N, K, epi, stream);
     if (tiles >= 1536) return launch_tile<128, 128, 1>(a, lda, b, ldb, M, N, K, epi, stream);
     if (tiles <= 512 && K >= 3072) return launch_tile<64, 64, 2>(a, lda, b, ldb, M, N, K, epi, stream);

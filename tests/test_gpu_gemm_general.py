@@ -29,6 +29,9 @@ SHAPES = [
     (700, 700, 65), (720, 650, 271), (1000, 700, 528), (470, 970, 3073), (465, 990, 3327),
     # cut tiles of aligned rows leave the streaming kernel from 513 tiles and K = 2944 on: the last it keeps on either side, and the first it does not
     (500, 1000, 2944), (520, 1000, 2928), (513, 1000, 2944),
+    # 257 to 512 tiles of 64 x 64 that are at most 256 of 96 x 64, in one and two groups of wavefronts; more of them, at most 256 of 96 x 96; and neither
+    (1057, 1025, 273), (1056, 1024, 271), (1153, 961, 2992), (1100, 1000, 912), (1100, 1000, 3073), (1057, 1025, 3200), (2881, 705, 401), (1440, 1536, 1007), (1153, 1537, 655),
+    (2305, 705, 401),
     # 128 x 128 tiles from 1536 tiles of 64 x 64
     (2497, 2497, 33), (1, 5000, 50), (3000, 2176, 130),
 ]
