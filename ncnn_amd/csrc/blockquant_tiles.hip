@@ -9,10 +9,12 @@
 // A wavefront multiplies 64 activation rows with 64 weight rows and a workgroup holds four groups of two, each with a quarter of K: a weight
 // is converted to fp16 once for 64 rows (with 32, as blockquant.hip's kernels have it, the vector unit is as busy as the matrix cores), and
 // 256 tiles of 64 x 128, a prefill of 512 rows of 4096, still put two wavefronts on every SIMD.
-// Bound by LDS and the matrix cores in turn: half a K step is 1024 cycles of products on a SIMD and 1000 of LDS fills and reads on the unit, and takes about 1550.
-// us with the split pass, 8 bits in blocks of 64, three bf16 numbers -> here: 512 x 4096 x 4096 60.7 -> 48, 512 x 4096 x 11008
-// 133 -> 102, 512 x 11008 x 4096 145 -> 119, 333 x 4096 x 4096 at 4 bits 51.6 -> 41.6, 1500 x 3072 x 1024 52.9 -> 49.4, 1024 x 4096 x 4096 at 6 bits 111 -> 86.
-// (Weights and loads all before the products, activations requested half a stage later, where the wavefront does not multiply, two groups and two workgroups to a
+// Bound by the matrix cores' issue at the 1.79 GHz they sustain on all units, and by the fills: half a K step is 571 ns of products for the two wavefronts of a SIMD and takes
+// 921; without the fills (48 KB a unit, 13 TB/s on all of them) 700, without the vector instructions 770.  Around the 30 us of steps that 64 x 128 results of K = 4096 take
+// stand 0.5 of first loads, 1.3 of the groups' exchange and 1.5 of results.  us with the split pass, 8 bits in blocks of 64, three bf16 numbers -> here: 512 x 4096 x 4096
+// 60.7 -> 46.6, 512 x 4096 x 11008 133 -> 101, 512 x 11008 x 4096 145 -> 114, 1500 x 3072 x 1024 52.9 -> 43.9, 1500 x 1024 x 1024 24.1 -> 21.8; 1024 x 4096 x 4096 at 6
+// bits 111 -> 86.  (One barrier a stage and operands read a stage ahead, between the products, instead of two wavefronts that read and multiply in turn: 49.8, as the
+// fills are what it waits for.  Weights and loads all before the products, activations requested half a stage later, two groups and two workgroups to a
 // unit: all slower with three products.)
 #include <atomic>
 
@@ -371,6 +373,13 @@ __global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4*
 #pragma unroll
             for (int e = 0; e < 4; e++) to[e * 64] = v4f_t{acc[q][4 * e], acc[q][4 * e + 1], acc[q][4 * e + 2], acc[q][4 * e + 3]};
         }
+    // what the part's results need from memory is on its way while the groups meet (read behind their sums it was 1.5 us of a workgroup's time)
+    const int j = (tile0 + 2 * (group & 1)) * 16 + l32, i0 = row0 + (group >> 1) * 32 + 4 * hh; // result r: row i0 + 8 (r / 4) + r % 4 (`back` is padded to 64 rows)
+    v4f_t factor[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) factor[e] = *reinterpret_cast<const v4f_t*>(back + i0 + 8 * e);
+    const bool of_column = bt == 0 || bt == 4;
+    const float addend = of_column && j < N ? mul_rn(load_c(c, bt, 0, j, N), beta) : 0.f;
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 4; q++)
@@ -388,16 +397,18 @@ __global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4*
                 for (int o = 0; o < 4; o++) acc[q][4 * e + o] += v[o];
             }
         }
-        const int j = (tile0 + 2 * (q & 1)) * 16 + l32;
         if (j >= N) continue;
 #pragma unroll
         for (int r = 0; r < 16; r++)
         {
-            const int i = row0 + (q >> 1) * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
+            const int i = i0 + 8 * (r >> 2) + (r & 3);
             if (i < M)
             {
-                float v = acc[q][r] * back[i];
-                if (bt >= 0) v = add_rn(mul_rn(load_c(c, bt, i, j, N), beta), v);
+                float v = acc[q][r] * factor[r >> 2][r & 3];
+                if (of_column)
+                    v = add_rn(addend, v);
+                else if (bt >= 0)
+                    v = add_rn(mul_rn(load_c(c, bt, i, j, N), beta), v);
                 out[(size_t)i * out_stride + j] = mul_rn(v, alpha);
             }
         }
