@@ -881,6 +881,61 @@ def test_attention_core_on_split_keys_and_values_with_numbers_too_small_to_split
             assert error <= 1.25 * fp32 + 2.0 ** -23, (exponent, error, fp32)
 
 
+# 500 keys a workgroup and more: one workgroup for all keys of a unit (a last tile of 12 keys, of all 32), and three for 1530 (merged from their records)
+@pytest.mark.parametrize("heads,hd,src,dst", [(16, 32, 520, 500), (16, 64, 513, 544), (16, 96, 270, 700), (8, 128, 1030, 511), (16, 32, 300, 1530)])
+@pytest.mark.parametrize("kind", ["mask", "keys", "values", "channels", "zeros", "scaled", "special"])
+def test_attention_core_in_two_fp16_numbers(rt, heads, hd, src, dst, kind):
+    """Keys, values and queries times powers of two, as two fp16 numbers each: masks of the lowest value (of a whole row, too) and of -inf, numbers whose sizes lie too
+    far apart for a common factor in a tile of keys, between tiles and between channels, tiles of zeros, sizes near both ends of fp32: no more error against float64 than
+    the fp32 form has (but for the spread between two orders of a sum), in each channel where they differ in size; infinities and NaNs where it has them."""
+    print("[case]", heads, hd, src, dst, kind, flush=True)
+    rng = np.random.default_rng(heads * 1000 + src)
+    e = heads * hd
+    q = (rng.normal(0, 1, (src, e)) / np.sqrt(hd)).astype(F)
+    kt, vt = (rng.normal(0, 1, (e, dst)).astype(F) for _ in range(2))
+    m, big = None, F(2.0 ** 40)
+    if kind == "mask":
+        m = rng.normal(0, 1, (src, dst)).astype(F)
+        m[:, 1:][rng.random((src, dst - 1)) < 0.3] = -np.finfo(F).max
+        m[2], m[3, 5:] = -np.finfo(F).max, -np.inf
+    elif kind == "keys":
+        kt[:, 7] *= big
+        kt[:, dst - 1] = 0
+        kt[:, 64:96] /= big  # a tile of its own
+    elif kind == "values":
+        vt[:, 32:96] /= big
+        vt[:, dst - 1] *= F(2.0 ** 10)
+    elif kind == "channels":
+        vt[3] /= big
+        kt[5] *= F(2.0 ** 12)
+    elif kind == "zeros":
+        vt[:, :64], kt[:, 32:64], q[1] = 0, 0, 0
+        vt[:hd] = 0
+    elif kind == "scaled":
+        q, kt, vt = q * F(2.0 ** 90), kt * F(2.0 ** -90), vt * F(2.0 ** -100)
+    else:
+        vt[3, 5], vt[7, dst - 1], vt[e - 1, 2], vt[e - 2, 9], kt[hd, 40], q[9, 2] = np.inf, -np.inf, np.nan, np.finfo(F).max, np.inf, np.inf
+    got, plain = rt.attention(q, kt, vt, heads, m), rt.attention(q, kt, vt, heads, m, use_workspace=False)
+    if kind == "special":
+        assert np.array_equal(np.isnan(got), np.isnan(plain)) and np.array_equal(np.isinf(got), np.isinf(plain))
+        ok = np.isfinite(plain)
+        assert ok.any() and not ok.all() and np.abs(got[ok] / np.maximum(np.abs(plain[ok]), 1.0) - plain[ok] / np.maximum(np.abs(plain[ok]), 1.0)).max() <= 2e-5
+        return
+    want = np.empty((src, e))
+    for h in range(heads):
+        sl = slice(h * hd, (h + 1) * hd)
+        s = q[:, sl].astype(np.float64) @ kt[sl].astype(np.float64)
+        if m is not None:
+            s = s + m.astype(np.float64)
+        s = np.exp(s - s.max(axis=1, keepdims=True))
+        want[:, sl] = (s / s.sum(axis=1, keepdims=True)) @ vt[sl].astype(np.float64).T
+    for cols in (slice(None), slice(3, 4)) if kind == "channels" else (slice(None),):
+        norm = np.sqrt(np.mean(want[:, cols] ** 2))
+        error, fp32 = (np.sqrt(np.mean((x[:, cols] - want[:, cols]) ** 2)) / norm for x in (got, plain))
+        assert error <= 1.25 * fp32 + 2.0 ** -23, (error, fp32)
+    assert kind != "zeros" or np.all(got[:, :hd] == 0)
+
+
 @pytest.mark.parametrize("heads,hd,src,dst", [(4, 64, 37, 200), (2, 32, 1, 300), (3, 24, 5, 40)])
 def test_attention_reads_strided_queries_and_scales_them_on_load(rt, heads, hd, src, dst):
     """Queries taken out of a wider row (q, k and v made by one Gemm) and multiplied by the layer's scale where they are read:
