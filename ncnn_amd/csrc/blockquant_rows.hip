@@ -20,6 +20,11 @@
 // parts it saves that launch (5 us) and a third of the bytes.  us per call before (blockquant.hip's forms) -> here, 8 bits in blocks of 64:
 // 4096 x 4096 16 rows 12.4 -> 10.7, 32 rows 20.1 -> 12.9, 64 rows 34 -> 17.5, 128 rows 41 -> 30; 11008 x 4096 16 rows 26.5 -> 16.6, 32
 // rows 46 -> 26.5; 4096 x 11008 32 rows 45 -> 27, 128 rows 93 -> 66.
+// Two wavefronts share a SIMD and the one that multiplies goes first (left to itself the SIMD serves its oldest, which ends up to 4 us before its neighbour and leaves it
+// alone with its waits); the sums of a result are requested at once and the matrices' ends too.  us, before -> here: fp32 rows, 8 bits, 64 x 4096 x 4096 17.2 -> 16.5, 42 x
+// 6880 x 5312 34.1 -> 32.5, 16 x 4096 x 4096 10.8 -> 10.4, 6 bits 100 x 1248 x 7296 25.9 -> 24.4; fp16 rows, the four launches of a decoder layer, 48 rows at 4 bits 59.4 ->
+// 57.9 in the kernel trace.  (Loads of the stage after the next as soon as a stage is in registers: 66.6 -> 68.6 for the layer.  Without any loads its four launches take 48,
+// without the products 50, with neither 29.)
 // A lane must fetch along a row (eight lanes = one 128-byte line) and read in operand order (lane = row), so the chunks of a row
 // are swizzled on the source side: chunk c of row r lands at position c ^ ((r / 2) % 8), conflict-free both ways.
 #include <atomic>
@@ -147,9 +152,15 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
     int group = round * 8 + (in_round & 7);
     const int row0 = (in_round >> 3) * MG * 16;
     if (group >= groups) return;
-    int mat = 0; // tile_end counts groups of RT tiles here
-    while (mat + 1 < mm.count && group >= mm.tile_end[mat]) mat++;
-    group -= mat ? mm.tile_end[mat - 1] : 0;
+    int mat = 0, before = 0; // tile_end counts groups of RT tiles here; all of them are read at once
+#pragma unroll
+    for (int i = 0; i < BQ_MULTI_MAX - 1; i++)
+    {
+        const bool later = i + 1 < mm.count && group >= mm.tile_end[i];
+        mat += later;
+        before = later ? mm.tile_end[i] : before;
+    }
+    group -= before;
     const int N = mm.N[mat], ntiles = (N + 15) >> 4;
     const int M = M_total - row0 < MG * 16 ? M_total - row0 : MG * 16;
 
@@ -240,6 +251,7 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
         issue(0, 0);
         for (int s = 0; s < steps; s++)
         {
+            __builtin_amdgcn_s_setprio(0); // the neighbour on the SIMD multiplies first
             const unsigned at = (unsigned)((s & 1) * STAGE);
             // the stage multiplied in the turn before has been read (its reads were waited for): the next loads go there
             issue(s + 1 < steps ? s + 1 : s, (s + 1) & 1);
@@ -307,6 +319,7 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
                 asm volatile("" : "+v"(dq0[rt]));
                 if (SPLIT) asm volatile("" : "+v"(dq1[rt]));
             }
+            __builtin_amdgcn_s_setprio(1);
             const v4f zero = {0.f, 0.f, 0.f, 0.f};
             if constexpr (!F32)
             {
@@ -440,6 +453,7 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
                 for (int r = 0; r < 4; r++) nan = acc[rt][g][r] != acc[rt][g][r] ? 1.f : nan;
         if (!__any(nan != 0.f)) break;
     }
+    __builtin_amdgcn_s_setprio(0);
     __syncthreads();
 
     // accumulator r of lane l: weight row (l / 16) * 4 + r of the tile, activation row l % 16 of the group
@@ -461,14 +475,23 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
         const int i = g * 16 + m;
         if (i >= M) continue;
         float4 f = red[p * nwaves * 64 + lane];
-        for (int w = 1; w < nwaves; w++)
-        {
-            const float4 o = red[(p * nwaves + w) * 64 + lane];
+        const auto add = [&](const float4& o) {
             f.x = add_rn(f.x, o.x);
             f.y = add_rn(f.y, o.y);
             f.z = add_rn(f.z, o.z);
             f.w = add_rn(f.w, o.w);
+        };
+        constexpr int MOST = rows_waves(BITS, MG, RT, SPLIT, AIN);
+        if (nwaves == MOST) // nearly always: all sums requested at once
+        {
+            float4 o[MOST];
+#pragma unroll
+            for (int w = 1; w < MOST; w++) o[w] = red[(p * MOST + w) * 64 + lane];
+#pragma unroll
+            for (int w = 1; w < MOST; w++) add(o[w]);
         }
+        else
+            for (int w = 1; w < nwaves; w++) add(red[(p * nwaves + w) * 64 + lane]);
         float fr[4] = {f.x, f.y, f.z, f.w};
         const int j0 = (group * RT + rt) * 16 + kg * 4;
         float* to = out + (size_t)(row0 + i) * out_stride + j0;
