@@ -11,7 +11,7 @@ PipePlan plan_pipelined(int cout, long long npix, int steps)
 {
     PipePlan p;
     p.groups = 1;
-    // channel tile: the width that pads the channel count least (padded channels cost matrix-core time and unbalance the
+    // (A layer whose K stays whole in four wavefronts takes choose_tile's instead.)  Channel tile: the width that pads the channel count least (padded channels cost matrix-core time and unbalance the
     // wavefronts' epilogues: 144 channels in one 256-wide tile ran 34 us, in three 64-wide tiles 21), the wider on a tie
     p.bn = 64;
     for (int bn = 128; bn <= 256; bn *= 2)
@@ -95,8 +95,36 @@ static int special_kernel(const NhwcGeom& g, const ConvEpilogue& epi, const Conv
     return conv_stream_tile(g, !epi.scale_out) ? NCNNHIP_CONV_FEW_TILES : NCNNHIP_CONV_PIPELINED;
 }
 
+// The tile of a layer whose K stays whole in four wavefronts.  us in passes of ResNet-50 and MobileNetV2, 8 to 128 images:
+//   a sum (residual in, fp32 and int8 out) is bound by memory, and small tiles keep more of it in flight: 64 x 64 / 64 x 128 / 64 x 256, 50176 pixels x 512 24.8 27.0 35.5, 25088 x 1024
+//   29.7 31.0 41.6, 25088 x 512 15.0 16.8 22.7, 6272 x 1024 10.8 12.3 14.0, 50176 x 256 14.3 16.1 21.8, 12544 x 1024 21.6 22.5 28.4; from about 8000 of them on 64 x 128 is as good or
+//   better: 401408 x 256 112.7 104.8 119.3 and 185 168 175, 100352 x 512 93.0 87.1 94.4, 200704 x 256 90.9 85.6 94.6, and from 3000 on with 8 steps: 6272 x 2048 31.2 30.2 33.5;
+//   a long K is bound by LDS, of which a tile twice as wide reads half as much a product, as long as there is a tile for every unit: 64 x 64 / 64 x 128 / 128 x 128, 36 steps 25088 x 256
+//   35.6 32.6 23.6, 16 steps the same 19.2 18.9 15.8; 72 steps 6272 x 512 34.0 30.8 33.5 (196 tiles), 32 steps 19.0 17.0 18.7, 36 steps 12544 x 256 19.5 17.7 19.9, 3136 x 512 27.0
+//   29.7 33.1; 18 steps 25088 x 128 11.9 11.1 12.9; 8 steps 25088 x 256 12.6 13.0 12.0, 50176 x 128 12.7 12.9 11.6, 100352 x 128 22.5 19.8 21.5, 12544 x 256 7.8 8.2 9.9;
+//   below 8 steps 64 x 64 / 64 x 128, one step 25088 x 384 7.5 8.6, 12544 x 384 5.1 6.0 (one tile for all channels is left as wide as they are), two 12544 x 576 7.6 6.9, four and five 100352 x 128 14.4 13.9, 6272 x 1280 14.2 13.0.
+// (64 x 256 is the best nowhere, 128 x 64 where 64 x 128 is nearly as good.)
+static void choose_tile(const NhwcGeom& g, bool residual, PipePlan& p)
+{
+    const int steps = g.K / 64;
+    const auto tiles = [&](int bm, int bn) { return (long long)ceil_div(g.npix, bm) * ceil_div(g.cout, bn); };
+    const bool wide = ceil_div(g.cout, 128) * 128 <= ceil_div(g.cout, 64) * 64; // without more padded channels
+    p.bm = p.bn = 64;
+    if (residual)
+    {
+        if (wide && tiles(64, 64) >= (steps >= 8 ? 3000 : 8000)) p.bn = 128;
+    }
+    else if (wide && steps >= 8 && tiles(128, 128) >= 300 && (steps >= 16 || tiles(128, 128) <= 512))
+        p.bm = p.bn = 128;
+    else if (wide && tiles(64, 128) >= (steps >= 16 ? 300 : 900) && (steps >= 2 || g.cout <= 128))
+        p.bn = 128;
+    if (wide && tiles(64, p.bn) * ceil_div(g.cout, p.bn) >= 1ll << 32) p.bm = p.bn = 128; // (the kernel's division of a tile number: an output of 70 GB and more)
+    p.tiles_m = ceil_div(g.npix, p.bm);
+    p.tiles_n = ceil_div(g.cout, p.bn);
+}
+
 // the pipelined kernel's plan and addressing mode (its MODE), the layer as it sees it in g
-static int pipelined_form(NhwcGeom& g, PipePlan& p)
+static int pipelined_form(NhwcGeom& g, bool residual, PipePlan& p)
 {
     // A 1x1, stride-1, unpadded layer reads input pixel n for output pixel n, whatever the image shape: present it as
     // one row of npix pixels, and the kernel skips the pixel -> (image, y, x) divisions.
@@ -107,6 +135,7 @@ static int pipelined_form(NhwcGeom& g, PipePlan& p)
         g.W = g.outw = g.npix;
     }
     p = plan_pipelined_groups(g.cout, g.npix, g.K / 64);
+    if (p.groups == 1 && p.splits == 1) choose_tile(g, residual, p);
     // the narrow-input first layer has four K steps at most: from a million output pixels up, 128-pixel tiles halve the number of
     // workgroup prologues (ResNet-50's 7 x 7 first layer at batch 128: the pass 2.22 -> 2.20 ms; at batch 16, 0.2 M pixels, no gain)
     if ((g.tapK == 16 || g.tapK == 32) && p.splits == 1 && p.bm == 64 && g.npix >= (1 << 20))
@@ -130,7 +159,7 @@ void conv_nhwc_pipelined_route(const NhwcGeom& g_in, const ConvEpilogue& epi, co
     if (route.kernel != NCNNHIP_CONV_PIPELINED) return;
     NhwcGeom g = g_in;
     PipePlan p;
-    const int mode = pipelined_form(g, p);
+    const int mode = pipelined_form(g, fusion.residual != 0, p);
     route = {NCNNHIP_CONV_PIPELINED, p.bm, p.bn, mode, p.groups, p.splits};
 }
 
@@ -148,7 +177,7 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
     }
     NhwcGeom g = g_in;
     PipePlan p;
-    const int mode = pipelined_form(g, p);
+    const int mode = pipelined_form(g, fusion.residual != 0, p);
     const long long blocks = (long long)p.tiles_m * p.tiles_n * p.splits;
     NCNNHIP_REQUIRE(blocks < (1ll << 31) && blocks * p.tiles_n < (1ll << 32), "convolution: too many tiles");
     int32_t* partial = 0;
@@ -191,14 +220,12 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
         LAUNCH_PIPE_MODE(64, 64, 3, 4);
     else if (p.groups == 4)
         LAUNCH_PIPE_MODE(64, 64, 0, 4);
-    else if (p.bm == 128 && p.bn == 256)
-        LAUNCH_PIPE(128, 256);
     else if (p.bm == 128 && p.bn == 128)
         LAUNCH_PIPE(128, 128);
+    else if (p.bm == 128 && mode == 1) // narrow inputs: a 1x1 kernel, and a gathered one
+        LAUNCH_PIPE_MODE(128, 64, 1, 1);
     else if (p.bm == 128)
-        LAUNCH_PIPE(128, 64);
-    else if (p.bn == 256)
-        LAUNCH_PIPE(64, 256);
+        LAUNCH_PIPE_MODE(128, 64, 2, 1);
     else if (p.bn == 128)
         LAUNCH_PIPE(64, 128);
     else

@@ -882,6 +882,9 @@ static int resident_choose(const NhwcGeom& g, const ConvEpilogue& epi, const Con
 // the next launch starts later than behind the pipelined kernel's short ones: with every 3x3 layer on this kernel a ResNet-50
 // pass is 2 % slower at batch 32 and 1 % at batch 128 (equal at batch 16); from 40000 pixels up (the 56 x 56 maps from batch
 // 16, the 28 x 28 maps from batch 64) the passes are as fast as without it and those layers are the ones that gain most alone.
+// A long K on whole tiles of 128 channels, without a sum, is the pipelined kernel's 128 x 128 tiles' (from 40000 pixels on more than one to a unit; us
+// here / there): 18 steps 50176 x 128 19.9 / 16.3, 100352 x 128 31.8 / 30.8, 200704 x 128 53.8 / 52.1, 36 steps 50176 x 256 62.4 / 47.2.  64 channels
+// stay: 9 steps 401408 x 64 29.3 / 36.6, 200704 x 64 18.0 / 21.1, 100352 x 64 11.7 / 13.1.
 // Environment, read at every launch: NCNNHIP_RESIDENT_OFF (any value) switches the kernel off, NCNNHIP_RESIDENT_MIN sets
 // the pixel threshold, NCNNHIP_RESIDENT_CFG forces one tile configuration (0..7): for measurements and tests.
 bool conv_resident_fits(const NhwcGeom& g, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp)
@@ -890,7 +893,10 @@ bool conv_resident_fits(const NhwcGeom& g, const ConvEpilogue& epi, const ConvFu
     if (g.ntaps < 2) return false; // first: most layers of a network are 1x1 and need not look the environment up
     if (getenv("NCNNHIP_RESIDENT_OFF")) return false;
     long long min_pixels = 40000;
-    if (const char* e = getenv("NCNNHIP_RESIDENT_MIN")) min_pixels = atoll(e);
+    if (const char* e = getenv("NCNNHIP_RESIDENT_MIN"))
+        min_pixels = atoll(e);
+    else if (g.K / 64 >= 16 && (g.cout + 63) / 64 % 2 == 0 && !fusion.residual)
+        return false;
     if (g.npix < min_pixels) return false;
     ResidentPlan P;
     size_t lds_bytes;

@@ -30,6 +30,19 @@ def test_forms_of_the_pipelined_kernel():
     assert (r.addressing, r.groups, r.splits) == (0, 1, 3)
 
 
+@pytest.mark.parametrize("shape,options,tile", [
+    ((128, 256, 14, 14, 256, (3, 3)), SAME3, (128, 128)), ((64, 256, 14, 14, 256, (3, 3)), SAME3, (64, 128)),
+    ((128, 128, 28, 28, 128, (3, 3)), SAME3, (128, 128)),  # a long K of 128 channels and many pixels
+    ((128, 128, 28, 28, 512, (1, 1)), dict(fused=True), (64, 128)), ((64, 128, 28, 28, 512, (1, 1)), dict(fused=True), (64, 64)),
+    ((128, 512, 7, 7, 2048, (1, 1)), dict(fused=True), (64, 128)),
+    ((32, 64, 28, 28, 384, (1, 1)), {}, (64, 64)), ((128, 320, 7, 7, 1280, (1, 1)), {}, (64, 128)),
+    ((8, 32, 368, 368, 64, (1, 1)), {}, (128, 64)),
+], ids=str)
+def test_tile_of_the_pipelined_kernel(shape, options, tile):
+    r = cases.conv_route(*shape, **options)
+    assert (r.kernel, r.tile_pixels, r.tile_channels, r.groups, r.splits) == (r.PIPELINED,) + tile + (1, 1)
+
+
 def test_layers_that_are_refused():
     from ncnn_amd.hip import Activation, ConvDesc, ConvRoute, lib
     r, act = ConvRoute(), Activation.make(0, (0.0, 0.0))
