@@ -183,10 +183,19 @@ int ncnnhip_gemm_int8(const int8_t* aq_dev, size_t aq_stride, const int8_t* bq_d
     const bool aligned = K % 16 == 0 && aligned16(aq_dev) && aligned16(bq_dev) && aq_stride % 16 == 0 && bq_stride % 16 == 0;
     if (!gemm_int8_streams(M, N, K, aligned))
     {
-        // big aligned problems: the 256x256 kernel (it needs a few hundred tiles to fill the chip)
+        // big aligned problems: the 256x256 kernel, one workgroup to a unit.  Whole tiles from 128 of them up.  Where tiles are cut, one round of them as soon as
+        // the other kernels' 128x128 tiles are more than two to a unit, and more rounds where the last is well filled: beside a cut tile the
+        // other kernels' smaller ones lose less.  Others -> this, us: 1524 x 7496 x 768, 180 tiles, 24.4 -> 20.0; 1810 x 7480 x 1280, 240, 39.9 -> 29.1; 1318 x
+        // 6960 x 4800, 168, 80 -> 57; 2302 x 4192 x 6464, 153, 103 -> 70 (136 shapes 6 to 50 % quicker, 24 in the median); 3079 x 7816 x 2112, 403, 97 -> 75;
+        // 3200 x 7552 x 3072, 390, 112 -> 91; and where it is not taken: 1115 x 3376 x 1408, 70 tiles, 14.1 -> 21.3; 2847 x 2248 x 2624, 108, 32.5 -> 33.2; 2347 x
+        // 7624 x 3840, 300, 99 -> 101; 2176 x 4736 x 512, 153 of whole 128s, 17.9 -> 18.4.
         bool handled = false;
         int ret = NCNNHIP_OK;
-        if ((long long)M * N >= 256ll * 256 * 128)
+        const long long tiles256 = (long long)ceil_div(M, 256) * ceil_div(N, 256), room = (tiles256 + 255) / 256 * 256;
+        const long long tiles128 = (long long)ceil_div(M, 128) * ceil_div(N, 128), tiles64 = (long long)ceil_div(M, 64) * ceil_div(N, 64);
+        const bool whole = M % 128 == 0 && N % 128 == 0;
+        const bool cut_pays = (tiles256 <= 256 ? tiles128 > 512 : (double)tiles256 >= room * (K >= 1024 ? 0.7 : 0.78)) && !(whole && K < 1024);
+        if (M % 256 == 0 && N % 256 == 0 ? tiles256 >= 128 : cut_pays)
         {
             ret = launch_gemm_int8_pipelined(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, epi, as_stream(stream), &handled);
             if (handled) return ret;
@@ -199,8 +208,6 @@ int ncnnhip_gemm_int8(const int8_t* aq_dev, size_t aq_stride, const int8_t* bq_d
         // 59 -> 61.  Beyond one a unit only where the general kernel's 64 x 64 tiles are more than four a unit, one round: 19 shapes with fewer took 5 %
         // less to 22 % more on the ring, 15 in the median (1046 x 3682 x 256, 261 and 986 tiles, 7.8 -> 9.4; 676 x 5464 x 1216, 258 and 946, 15.5 -> 18.3),
         // 261 with more 10 % less in the median, 5 of them 4 to 11 % more.
-        const long long tiles128 = (long long)ceil_div(M, 128) * ceil_div(N, 128), tiles64 = (long long)ceil_div(M, 64) * ceil_div(N, 64);
-        const bool whole = M % 128 == 0 && N % 128 == 0;
         if (whole ? tiles128 >= 48 : tiles128 <= 256 ? tiles128 >= 200 && K >= 512 : K <= 2048 && tiles64 > 1024)
         {
             ret = launch_gemm_int8_ring128(aq_dev, aq_stride, bq_dev, bq_stride, M, N, K, epi, as_stream(stream), &handled);

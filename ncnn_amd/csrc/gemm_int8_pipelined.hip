@@ -20,6 +20,10 @@
 // what bounds the row-major kernel (without any fills its K loop runs 25 % faster).  The B operand is tiled with its rows
 // already in the column-interleaved order described at the loads below.
 //
+// The epilogue is issue: 256 sums a lane, one wavefront to a SIMD, nothing beside it.  What it multiplies with is made before the loop and waits in
+// LDS, and the stores' addresses are one addition a row; of row-major operands, whose last tiles are cut, a buffer that ends with the output drops
+// what lies beyond (a branch around each store instead, and 64-bit addresses: 2040 x 1992 x 64 17.6 us, without 9.5; 4096 cubed row-major 71.8 -> 68.6).
+//
 // Workgroup ids are remapped so that each of the 8 XCDs (ids are dealt round-robin to XCDs)
 // works on a compact block of output tiles and re-uses its A/B panels out of its own L2.
 #include <cstdlib>
@@ -43,14 +47,16 @@ constexpr int STAGE_BYTES = 2 * OPERAND_BYTES; // 32 KB
 #define WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | ((((n) >> 4) & 3) << 14))
 
 
+// Row-major operands end at any M and any N of whole fours: rows past the end repeat the last one and are never stored.
 template<bool PER_COL, int BT, bool TILED>
 __global__ __launch_bounds__(256) void gemm_int8_256x256_kernel(const int8_t* __restrict__ A, size_t lda, const int8_t* __restrict__ B,
-                                                                 size_t ldb, int nk, int tiles_m, int tiles_n,
+                                                                 size_t ldb, int nk, int M, int N, int tiles_m, int tiles_n,
                                                                  const float* __restrict__ a_scales, const float* __restrict__ b_scales,
                                                                  const float* __restrict__ cvec, float alpha, float beta,
                                                                  float* __restrict__ out, size_t ldo)
 {
     __shared__ __attribute__((aligned(1024))) int8_t smem[STAGES * STAGE_BYTES];
+    __shared__ __attribute__((aligned(16))) float row_scale[PT], col_scale[PT], col_add[PT]; // what the epilogue multiplies with and adds
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // wave-uniform, lives in an SGPR
@@ -60,7 +66,8 @@ __global__ __launch_bounds__(256) void gemm_int8_256x256_kernel(const int8_t* __
     // ---- XCD-aware tile choice: 8 XCDs take contiguous ranges of a 4-row-grouped tile order
     int b = blockIdx.x;
     const int T = tiles_m * tiles_n;
-    if ((T & 7) == 0) b = (b & 7) * (T >> 3) + (b >> 3);
+    const int die = b & 7, more = T & 7;
+    b = die * (T >> 3) + (die < more ? die : more) + (b >> 3);
     constexpr int GM = 4;
     const int per_group = GM * tiles_n;
     const int group = b / per_group;
@@ -74,39 +81,40 @@ __global__ __launch_bounds__(256) void gemm_int8_256x256_kernel(const int8_t* __
     // load i of wave w fills LDS rows (i*4 + w)*16 .. +16 of the operand stage
     const int ld_row = wave * 16 + (lane >> 2);                 // + i*64
     const int ld_chunk = (lane & 3) ^ ((lane >> 4) & 3);        // swizzled source chunk
-    const int8_t* ga = TILED ? A + ((size_t)tile_m * nk * PT + ld_row) * PK + ld_chunk * 16 : A + ((size_t)tile_m * PT + ld_row) * lda + ld_chunk * 16;
     // B rows are permuted on their way into LDS: LDS row wn*128 + j*32 + l holds B row wn*128 + 4*l + j, so that the four
     // accumulator blocks j of a lane are four consecutive output columns and the epilogue stores 16 bytes per lane.
     // LDS row of this lane in quarter i = i*64 + wave*16 + (lane >> 2): wn = i >> 1, j = (i & 1)*2 + (wave >> 1),
     // l = (wave & 1)*16 + (lane >> 2).
     const int ld_row_b = 4 * ((wave & 1) * 16 + (lane >> 2)) + (wave >> 1); // + (i >> 1)*128 + (i & 1)*2
-    const int8_t* gb = TILED ? B + ((size_t)tile_n * nk * PT + ld_row) * PK + ld_chunk * 16 : B + ((size_t)tile_n * PT + ld_row_b) * ldb + ld_chunk * 16;
-    const size_t a_step = 64 * lda;
+    // a uniform base, advanced per step, and an offset for each load
+    const int rows_a = M - tile_m * PT, rows_b = N - tile_n * PT;
+    const int8_t* ua = A + (TILED ? (size_t)tile_m * nk * OPERAND_BYTES : (size_t)tile_m * PT * lda);
+    const int8_t* ub = B + (TILED ? (size_t)tile_n * nk * OPERAND_BYTES : (size_t)tile_n * PT * ldb);
+    unsigned off_a[4], off_b[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+    {
+        const int ra = i * 64 + ld_row, rb = (i >> 1) * 128 + (i & 1) * 2 + ld_row_b;
+        off_a[i] = TILED ? ld_row * PK + ld_chunk * 16 : (unsigned)((ra < rows_a ? ra : rows_a - 1) * lda + ld_chunk * 16);
+        off_b[i] = TILED ? off_a[i] : (unsigned)((rb < rows_b ? rb : rows_b - 1) * ldb + ld_chunk * 16);
+    }
+    constexpr int STEP = TILED ? OPERAND_BYTES : PK;
 
-    // quarter i of the loads of step t: 16 A rows and 16 B rows per wave
-    auto issue_quarter = [&](int t, int i) {
-        int8_t* sa = smem + (t & (STAGES - 1)) * STAGE_BYTES + wave * 1024 + i * 4096;
-        const int8_t* pa = TILED ? ga + (size_t)t * OPERAND_BYTES + i * 4096 : ga + (size_t)t * PK + i * a_step;
-        const int8_t* pb = TILED ? gb + (size_t)t * OPERAND_BYTES + i * 4096 : gb + (size_t)t * PK + (size_t)((i >> 1) * 128 + (i & 1) * 2) * ldb;
-        __builtin_amdgcn_global_load_lds((const AS1 void*)pa, (AS3 void*)sa, 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((const AS1 void*)pb, (AS3 void*)(sa + OPERAND_BYTES), 16, 0, 0);
-    };
+    // quarter i of the loads of step t: 16 A rows (which = 0) or 16 B rows per wave
     auto issue_one = [&](int t, int i, int which) {
         int8_t* sa = smem + (t & (STAGES - 1)) * STAGE_BYTES + wave * 1024 + i * 4096;
         if (which == 0)
-        {
-            const int8_t* pa = TILED ? ga + (size_t)t * OPERAND_BYTES + i * 4096 : ga + (size_t)t * PK + i * a_step;
-            __builtin_amdgcn_global_load_lds((const AS1 void*)pa, (AS3 void*)sa, 16, 0, 0);
-        }
+            __builtin_amdgcn_global_load_lds((const AS1 void*)(ua + (size_t)t * STEP + (TILED ? i * 4096 : 0) + off_a[i]), (AS3 void*)sa, 16, 0, 0);
         else
-        {
-            const int8_t* pb = TILED ? gb + (size_t)t * OPERAND_BYTES + i * 4096 : gb + (size_t)t * PK + (size_t)((i >> 1) * 128 + (i & 1) * 2) * ldb;
-            __builtin_amdgcn_global_load_lds((const AS1 void*)pb, (AS3 void*)(sa + OPERAND_BYTES), 16, 0, 0);
-        }
+            __builtin_amdgcn_global_load_lds((const AS1 void*)(ub + (size_t)t * STEP + (TILED ? i * 4096 : 0) + off_b[i]), (AS3 void*)(sa + OPERAND_BYTES), 16, 0, 0);
     };
     auto issue_stage = [&](int t) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) issue_quarter(t, i);
+        for (int i = 0; i < 4; i++)
+        {
+            issue_one(t, i, 0);
+            issue_one(t, i, 1);
+        }
     };
 
     v16i acc[4][4];
@@ -124,10 +132,18 @@ __global__ __launch_bounds__(256) void gemm_int8_256x256_kernel(const int8_t* __
     const int rd_b0 = OPERAND_BYTES + (wn * 128 + l32) * PK + ((0 + lhi) ^ sw) * 16;
     const int rd_b1 = OPERAND_BYTES + (wn * 128 + l32) * PK + ((2 + lhi) ^ sw) * 16;
 
-    // ---- prologue: three steps in flight
+    // ---- prologue: three steps in flight, between them the scales: their loads and divisions are over long before the loop is
+    const int in_tile = threadIdx.x; // its row and its column
+    const int scale_row = !TILED && in_tile >= rows_a ? rows_a - 1 : in_tile, scale_col = !TILED && in_tile >= rows_b ? rows_b - 1 : in_tile;
     if (0 < nk) issue_stage(0);
+    const float sa = a_scales[tile_m * PT + scale_row], sb = b_scales[PER_COL ? tile_n * PT + scale_col : 0];
+    const float addend = BT == 4 ? cvec[tile_n * PT + scale_col] : 0.f;
     if (1 < nk) issue_stage(1);
     if (2 < nk) issue_stage(2);
+    row_scale[in_tile] = PER_COL ? div_rn(1.f, sa) : div_rn(1.f, mul_rn(sa, sb));
+    if (PER_COL) col_scale[in_tile] = div_rn(1.f, sb);
+    if (BT == 4) col_add[in_tile] = mul_rn(addend, beta);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local"); // seen by all behind the barrier in front of the loop
 
     // Fragment registers are double-buffered (F0 = first 32 bytes of a K step, F1 = second).  The LDS reads and their
     // waits are written as asm so that a wait only covers the reads the next MFMAs need and leaves the others in flight.
@@ -169,6 +185,7 @@ __global__ __launch_bounds__(256) void gemm_int8_256x256_kernel(const int8_t* __
 
     wait_step(0);
     __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     if (3 < nk) issue_stage(3);
     read_frags(0, 0, fa0, fb0);
 
@@ -241,43 +258,47 @@ __global__ __launch_bounds__(256) void gemm_int8_256x256_kernel(const int8_t* __
 
     // ---- fused epilogue: dequantise, bias, scale, store fp32
     const int col_base = tile_n * PT + wn * 128 + 4 * l32; // accumulator block j of this lane is column col_base + j
-    float colscale[4], colc[4];
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    typedef unsigned v4u __attribute__((ext_vector_type(4)));
+    const v4f colscale = *reinterpret_cast<const v4f*>(col_scale + wn * 128 + 4 * l32), colc = *reinterpret_cast<const v4f*>(col_add + wn * 128 + 4 * l32);
+    v4f rowscale[4][4]; // of the lane's rows, four consecutive ones at a time
 #pragma unroll
-    for (int j = 0; j < 4; j++)
-    {
-        const int col = col_base + j;
-        colscale[j] = PER_COL ? div_rn(1.f, b_scales[col]) : 0.f;
-        colc[j] = BT == 4 ? mul_rn(cvec[col], beta) : 0.f;
-    }
-    // one descale per row of the tile, computed once by thread `row` and handed round through LDS (the stages are free
-    // once every wavefront has left the K loop)
-    float* rowscale_lds = reinterpret_cast<float*>(smem);
-    {
-        const float sa = a_scales[tile_m * PT + threadIdx.x];
-        const float rs = PER_COL ? div_rn(1.f, sa) : div_rn(1.f, mul_rn(sa, b_scales[0]));
-        __builtin_amdgcn_s_barrier();
-        rowscale_lds[threadIdx.x] = rs;
-        __syncthreads();
-    }
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) rowscale[i][e] = *reinterpret_cast<const v4f*>(row_scale + wm * 128 + i * 32 + 8 * e + 4 * lhi);
+    float* lane_out = out + (size_t)(tile_m * PT + wm * 128 + 4 * lhi) * ldo + col_base; // TILED
+    // else a buffer that ends with the last row and column of the output: stores beyond are dropped without a branch around each
+    const int in_rows = rows_a < PT ? rows_a : PT, in_cols = rows_b < PT ? rows_b : PT, lane_col = wn * 128 + 4 * l32;
+    const auto tile_out = __builtin_amdgcn_make_buffer_rsrc(out + (size_t)tile_m * PT * ldo + (size_t)tile_n * PT, 0, (int)(((in_rows - 1) * (unsigned)ldo + in_cols) * 4), 0x00020000);
+    unsigned lane_offset = lane_col < in_cols ? ((wm * 128 + 4 * lhi) * (unsigned)ldo + lane_col) * 4 : 0x80000000u;
 #pragma unroll
     for (int i = 0; i < 4; i++)
     {
 #pragma unroll
         for (int r = 0; r < 16; r++)
         {
-            const int row_in_tile = wm * 128 + 4 * lhi + i * 32 + 8 * (r >> 2) + (r & 3);
-            const float rowscale = rowscale_lds[row_in_tile];
-            float* orow = out + (size_t)(tile_m * PT + row_in_tile) * ldo + col_base;
-            float f4[4];
+            v4f f4;
 #pragma unroll
             for (int j = 0; j < 4; j++)
             {
-                float f = mul_rn((float)acc[i][j][r], rowscale);
+                float f = mul_rn((float)acc[i][j][r], rowscale[i][r >> 2][r & 3]);
                 if (PER_COL) f = mul_rn(f, colscale[j]);
                 if (BT == 4) f = add_rn(f, colc[j]);
                 f4[j] = mul_rn(f, alpha);
             }
-            *reinterpret_cast<float4*>(orow) = make_float4(f4[0], f4[1], f4[2], f4[3]); // (non-temporal stores: neutral at 4096 cubed, 3 % slower at 8192 cubed)
+            const unsigned further = (r & 3) == 3 ? 5 : 1;
+            if constexpr (TILED)
+            {
+                *reinterpret_cast<v4f*>(lane_out) = f4; // (non-temporal stores: neutral at 4096 cubed, 3 % slower at 8192 cubed)
+                lane_out += further * ldo;
+            }
+            else
+            {
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, f4), tile_out, (int)lane_offset, 0, 0);
+                lane_offset += further * 4 * (unsigned)ldo;
+            }
+            if ((r & 7) == 7) PIN; // eight rows at once: one at a time wait for each other's results (86.8 us in place of 86.2, 4096 cubed with the pass that quantises A), without a stop
+                                   // the compiler takes the sums far ahead of their use, by way of registers that are not there (87.2)
         }
     }
 }
@@ -508,10 +529,10 @@ template<bool TILED>
 static int launch_256x256(const int8_t* aq, size_t aq_stride, const int8_t* bq, size_t bq_stride, int M, int N, int K, const GemmEpilogue& epi,
                           hipStream_t stream)
 {
-    const int tm = M / PT, tn = N / PT, nk = K / PK;
+    const int tm = ceil_div(M, PT), tn = ceil_div(N, PT), nk = K / PK;
     dim3 grid(tm * tn), block(256);
 #define LAUNCH(PC, BTV)                                                                                                                    \
-    hipLaunchKernelGGL((gemm_int8_256x256_kernel<PC, BTV, TILED>), grid, block, 0, stream, aq, aq_stride, bq, bq_stride, nk, tm, tn,        \
+    hipLaunchKernelGGL((gemm_int8_256x256_kernel<PC, BTV, TILED>), grid, block, 0, stream, aq, aq_stride, bq, bq_stride, nk, M, N, tm, tn, \
                        epi.a_scales, epi.b_scales, epi.c, epi.alpha, epi.beta, epi.out, epi.out_stride)
     if (epi.per_col)
     {
@@ -535,10 +556,12 @@ int launch_gemm_int8_pipelined(const int8_t* aq, size_t aq_stride, const int8_t*
                                const GemmEpilogue& epi, hipStream_t stream, bool* handled)
 {
     *handled = false;
-    if (M % PT || N % PT || K % PK || aq_stride % 16 || bq_stride % 16 || !al16(aq) || !al16(bq)) return NCNNHIP_OK;
+    if (K % PK || N % 4 || aq_stride % 16 || bq_stride % 16 || !al16(aq) || !al16(bq)) return NCNNHIP_OK;
     if (epi.transpose || epi.acc_out || !(epi.bt == -1 || epi.bt == 4)) return NCNNHIP_OK;
     if (epi.out_stride % 4 || !al16(epi.out)) return NCNNHIP_OK; // the epilogue stores 16 bytes per lane
-    if ((long long)(M / PT) * (N / PT) > 0x7fffffff) return NCNNHIP_OK;
+    if ((long long)ceil_div(M, PT) * ceil_div(N, PT) > 0x7fffffff) return NCNNHIP_OK;
+    if ((unsigned long long)PT * aq_stride + 256 > 0xffffffffull || (unsigned long long)PT * bq_stride + 256 > 0xffffffffull) return NCNNHIP_OK; // 32-bit lane offsets
+    if (epi.out_stride > (1u << 20)) return NCNNHIP_OK; // the same of the output: 256 rows end below 2^31 bytes
     *handled = true;
     return launch_256x256<false>(aq, aq_stride, bq, bq_stride, M, N, K, epi, stream);
 }

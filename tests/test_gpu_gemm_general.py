@@ -70,6 +70,24 @@ def test_128x128_tiles_cut_at_the_end(rt, m, n, k, per_col):
     assert np.array_equal(got[:m, :cols], want[:, :cols]) and np.all(got[:m, cols:] == 7.0) and np.all(got[m] == 7.0)
 
 
+@pytest.mark.parametrize("m,n,k", [(2945, 2900, 64), (2820, 3076, 128), (2817, 2824, 192), (3072, 2820, 256), (2821, 3072, 320), (2944, 2944, 1024), (4100, 6148, 64)])
+@pytest.mark.parametrize("per_col", [True, False])
+def test_256x256_tiles_cut_at_the_end(rt, m, n, k, per_col):
+    """More than 512 tiles of 128 x 128 in one round of 256 x 256, and a second round that is well filled, K of one step to more than the ring holds: rows past the end
+    repeat the last one, and nothing is written outside the output.  Columns that are no whole fours, and output rows off 16 bytes, take other kernels and give the same."""
+    print("[case]", m, n, k, per_col, flush=True)
+    a, bq, sb, bias = cases.gemm_case(m + n + k, m, n, k, per_col=per_col)
+    aq, sa = rt.gemm_quantize_rows(a)
+    want, _ = npref.gemm_int8(aq, bq, sa, sb, bias, 4, acc=npref.gemm_acc_exact(aq, bq))
+    assert np.array_equal(rt.gemm_int8(aq, bq, sa, sb, bias, 4), want)
+    da, db, dsa, dsb, dc = rt.up(aq), rt.up(bq), rt.up(sa), rt.up(sb), rt.up(bias.reshape(-1))
+    for cols, stride in ((n - 4, n + 4), (n - 5, n), (n, n + 2)):
+        out = rt.up(np.full((m + 1, stride), 7.0, np.float32))
+        check(lib().ncnnhip_gemm_int8(da.ptr, k, db.ptr, k, m, cols, k, dsa.ptr, dsb.ptr, cols if per_col else 1, dc.ptr, 4, 1.0, 1.0, 0, out.ptr, stride, None, rt.stream))
+        got = out.to_numpy(rt.stream)
+        assert np.array_equal(got[:m, :cols], want[:, :cols]) and np.all(got[:m, cols:] == 7.0) and np.all(got[m] == 7.0)
+
+
 @pytest.mark.parametrize("m,n,k,pad", [(1601, 1537, 1003, 0), (1850, 1800, 1004, 0), (1793, 1805, 1024, 1), (2305, 2241, 1002, 2)])
 def test_128x128_tiles_of_rows_off_16_bytes(rt, m, n, k, pad):
     """Rows that begin at any byte, or at any fourth, in the sizes that take 128 x 128 tiles for it: cut tiles, K that ends inside a step."""
