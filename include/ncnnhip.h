@@ -488,8 +488,9 @@ int ncnnhip_gemm_blockquant_packed_multi(const void* a_dev, int a_elemsize, size
  * go, while that is the quicker way (some tens to some hundreds of rows), to the kernel ncnnhip_gemm_blockquant_packed has for more than
  * four, which splits the activations as it multiplies them and leaves the workspace alone.  All others are split once, into the workspace,
  * by a pass of its own: up to 128 rows off 16 bytes on small weights then stream the weights once per 16 rows, all passes in one launch;
- * the rest is a tiled Gemm on the bf16 matrix cores, 64 activation rows x 64, 128 or 192 weight rows per workgroup (prefill, attention
- * projections).  K % 16 == 0; the workspace is scratch (to be taken as overwritten by every call). */
+ * the rest is a tiled Gemm on the matrix cores, 64 activation rows x 64, 128 or 192 weight rows per workgroup (prefill, attention
+ * projections).  For weights in blocks of 64 and 128 it scales each row by a power of two and splits it into two fp16 numbers: 23 bits of every
+ * activation, and what lies below 2^-40 of its row's largest magnitude is lost; all other forms split exactly.  K % 16 == 0; the workspace is scratch (to be taken as overwritten by every call). */
 int ncnnhip_gemm_blockquant_packed_rows_workspace_bytes(int M, int K, size_t* bytes);
 int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int M, int N, int K, const uint8_t* packed_w_dev,
                                         const float* packed_descale_dev, int bits, int block, const float* in_scales_dev,
@@ -503,8 +504,10 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
  * the layer's cache blobs; mask is additive, [src][dst] (mask_heads 1) or [num_heads][src][dst], or NULL.
  * Head dimensions 32/64/96/128 run on the matrix cores with any dst_seqlen; others need head_dim + dst_seqlen <= 4096.
  * With the scratch ncnnhip_attention_workspace_bytes asks for (16-byte aligned) and queries enough for it, keys and values are
- * first split into three bf16 numbers each (6 bytes for every float) for the bf16 matrix cores, six products for one; without
- * it, or with numbers that those cannot carry (infinities; below 2^-110 but not zero), the fp32 matrix cores run.
+ * first split into three bf16 numbers each (6 bytes for every float) for the bf16 matrix cores, six products for one, or, where a workgroup
+ * has some 500 keys and more, scaled by powers of two and split into two fp16 numbers, three products for one; without
+ * it, or with numbers that those cannot carry (infinities; bf16: below 2^-110 but not zero; fp16: magnitudes too far apart for a tile's common factor),
+ * the fp32 matrix cores run.
  * With few queries and many keys (decoding against a cache) the keys are split over workgroups if the caller passes
  * the scratch (may be 0 / NULL: then one workgroup per head and 32 queries);
  * one to four queries on 256 to 32768 keys then run on a streaming kernel of their own (64 keys per workgroup, any
