@@ -33,17 +33,21 @@ typedef float v16f_bq __attribute__((ext_vector_type(16)));
 // the row's largest what lies above 2^-40 of it.  The row's factor back goes to `back`; infinities and NaNs travel in hi alone.
 // A stage is half a K step: of the 16-byte pieces the packed weights keep for four K groups (two chunks of 8 each) those of groups 2 h and
 // 2 h + 1.  [row block of 64][K step][h] [32-row group][chunk c of the piece][part] 64 lanes x 16 bytes: lane = row l % 32, K group 2 h + l / 32.
-// Rows beyond M and K beyond the last are zeros.  One workgroup: SPLIT_ROWS whole rows, so that their factors are known and what it writes are 64-byte pieces;
-// a wavefront, of 16 or as many as there are spans of 128 columns, takes the spans in turn and keeps the first KEEP of its own in registers between the two passes.
-// us, 8 bits, before (three bf16 numbers, no factor, workgroups of 64 rows x 128 columns) / here: 512 x 4096 6.7 / 7.5, 512 x 11008 14.0 / 14.5.
-constexpr int SPLIT_ROWS = 4, SPLIT_SPAN = 512 / SPLIT_ROWS, SPLIT_WAVES = 16;
+// Rows beyond M and K beyond the last are zeros.  One workgroup: SPLIT_ROWS whole rows, so that their factors are known, and as many workgroups as that gives: 512 rows
+// are 256 of them, one to a unit (bound by memory latency: each wavefront has its loads in flight once).  What it writes are 32-byte pieces; the four workgroups of a
+// 128-byte line run on one die, so that its L2 puts the line together.
+// A wavefront, of 16 or as many as there are spans of 256 columns, takes the spans in turn and keeps the first KEEP of its own in registers between the two passes.
+// us, a decoder layer of 4096 / 11008, seven Gemms and as many of these, workgroups of four rows / here: 150 rows 367 / 354, 512 514.6 / 510.3; of 1024 / 2816, 1500 rows
+// 213.1 / 209.9; of 2048 / 5504, 700 rows 257.8 / 256.5 (258.6 with four spans kept where there are no more than two).
+constexpr int SPLIT_ROWS = 2, SPLIT_LINE = 8 / SPLIT_ROWS, SPLIT_SPAN = 512 / SPLIT_ROWS, SPLIT_WAVES = 16; // LINE: workgroups that write the same 128-byte lines
 template<bool HALVES, int KEEP>
 __global__ __launch_bounds__(64 * SPLIT_WAVES) void blockquant_split_tiles_kernel(const float* __restrict__ a, size_t a_stride, int M, int K, int kblocks,
                                                                                   const float* __restrict__ in_scales, uint4* __restrict__ frags, float* __restrict__ back)
 {
     __shared__ unsigned tops[SPLIT_WAVES][SPLIT_ROWS];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane % SPLIT_ROWS;
-    const int row = blockIdx.x * SPLIT_ROWS + r, waves = blockDim.x >> 6;
+    const int turn = (int)blockIdx.x % (8 * SPLIT_LINE), share = (int)blockIdx.x - turn + (turn & 7) * SPLIT_LINE + (turn >> 3); // (the grid is whole turns)
+    const int row = share * SPLIT_ROWS + r, waves = blockDim.x >> 6;
     const auto load = [&](int span, float (&x)[8]) {
         const int k = span * SPLIT_SPAN + lane / SPLIT_ROWS * 8;
         const bool inside = row < M && k < K; // K % 16 == 0: a chunk of 8 is all in or all out
@@ -425,17 +429,19 @@ int launch_blockquant_tiles(const float* a, size_t a_stride, int M, int N, int K
     const int spans = (kblocks * 64 + SPLIT_SPAN - 1) / SPLIT_SPAN, waves = spans < SPLIT_WAVES ? spans : SPLIT_WAVES;
 #define SPLIT(HALVES_, KEEP_) \
     hipLaunchKernelGGL((blockquant_split_tiles_kernel<HALVES_, KEEP_>), dim3((unsigned)(blocks * (64 / SPLIT_ROWS))), dim3((unsigned)(64 * waves)), 0, st, a, a_stride, M, K, kblocks, in_scales, frags, back)
-    if (spans <= 2 * SPLIT_WAVES)
-    {
-        if (bits == 8)
-            SPLIT(false, 2);
-        else
-            SPLIT(true, 2);
-    }
+    const int keep = (spans + SPLIT_WAVES - 1) / SPLIT_WAVES; // what a wavefront keeps, up to three (K = 12288)
+    if (keep == 1 && bits == 8)
+        SPLIT(false, 1);
+    else if (keep == 1)
+        SPLIT(true, 1);
+    else if (keep == 2 && bits == 8)
+        SPLIT(false, 2);
+    else if (keep == 2)
+        SPLIT(true, 2);
     else if (bits == 8)
-        SPLIT(false, 6);
+        SPLIT(false, 3);
     else
-        SPLIT(true, 6);
+        SPLIT(true, 3);
 #undef SPLIT
 #define TILES(BITS_)                                                                                                                                          \
     do                                                                                                                                                             \

@@ -256,6 +256,26 @@ def test_fp32_rows_of_any_magnitude_in_64x128_tiles(rt, m, n, k, bits):
     assert np.all(np.abs(got - val) <= 1e-6 * floor + 2.0 ** -40 * np.abs(a).max(axis=1, keepdims=True).astype(np.float64) * ones + 2.0 ** -148)
 
 
+# spans of 256 columns over 16 wavefronts: one wavefront, a part of the last span, one, two and three spans each, and what goes beyond the registers
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,k", [(129, 64), (191, 272), (131, 4096), (131, 4112), (193, 8192), (131, 8208), (131, 12288), (193, 12304)])
+def test_split_pass_of_whole_rows(rt, m, k, bits):
+    """Two rows to a workgroup, dealt out to the dies by lines: every row has its own size, so that a row, factor or span out of place shows.  The bound is that of
+    test_fp32_rows_of_any_magnitude_in_64x128_tiles: 23 bits an activation and the sums' roundings, relative to the sum of magnitudes."""
+    a, packed, scales = synth.blockquant_operands(m + k, m, 48, k, bits, 64, half_exact=False)
+    a *= np.exp2(np.arange(m) % 41 - 20).astype(F)[:, None]
+    pw, pd = rt.blockquant_pack(packed, scales, 64, bits=bits, k=k)
+    w, d = rt.up(pw), rt.up(pd)
+    size = C.c_size_t()
+    check(lib().ncnnhip_gemm_blockquant_packed_rows_workspace_bytes(m, k, C.byref(size)))
+    ws = DeviceBuffer.empty((size.value,), np.uint8)
+    src, dst = rt.up(np.concatenate([[F(0)], a.ravel()]).astype(F)), rt.up(np.full((m, 48), 7.0, F))
+    check(lib().ncnnhip_gemm_blockquant_packed_rows(C.c_void_p(src.ptr.value + 4), k, m, 48, k, w.ptr, d.ptr, bits, 64, None, None, -1, 1.0, 1.0, dst.ptr, 48,
+                                                    ws.ptr, size.value, rt.stream))  # (off 16 bytes: not the one-launch form)
+    val, floor = npref.blockquant_gemm_f64(a, packed, scales, bits, 64)
+    assert np.all(np.abs(dst.to_numpy(rt.stream) - val) <= 1e-6 * floor)
+
+
 def test_several_matrices_whose_groups_would_fill_the_units_only_together(rt):
     """3 x 256 tiles: in groups of three 258, in groups of four 192, which is what several matrices get; one matrix of all of them is 256 groups of three."""
     m, k, n = 48, 64, 4096
