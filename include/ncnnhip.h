@@ -504,10 +504,8 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
  * the layer's cache blobs; mask is additive, [src][dst] (mask_heads 1) or [num_heads][src][dst], or NULL.
  * Head dimensions 32/64/96/128 run on the matrix cores with any dst_seqlen; others need head_dim + dst_seqlen <= 4096.
  * With the scratch ncnnhip_attention_workspace_bytes asks for (16-byte aligned) and queries enough for it, keys and values are
- * first split into three bf16 numbers each (6 bytes for every float) for the bf16 matrix cores, six products for one, or, where a workgroup
- * has some 500 keys and more, scaled by powers of two and split into two fp16 numbers, three products for one; without
- * it, or with numbers that those cannot carry (infinities; bf16: below 2^-110 but not zero; fp16: magnitudes too far apart for a tile's common factor),
- * the fp32 matrix cores run.
+ * first split into three bf16 numbers each (6 bytes for every float) for the bf16 matrix cores, six products for one; without
+ * it, or with numbers that those cannot carry (infinities; below 2^-110 but not zero), the fp32 matrix cores run.
  * With few queries and many keys (decoding against a cache) the keys are split over workgroups if the caller passes
  * the scratch (may be 0 / NULL: then one workgroup per head and 32 queries);
  * one to four queries on 256 to 32768 keys then run on a streaming kernel of their own (64 keys per workgroup, any

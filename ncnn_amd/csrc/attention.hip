@@ -175,9 +175,6 @@ __device__ __forceinline__ void load_value_block(float (&vv)[16], const float* _
 // One tile's step of the running softmax of a query (lanes l and l^32 hold the two halves of its 32 scores): scores
 // become exp(score - new maximum), the running sum and maximum are brought up to date, and the factor that rescales what
 // was accumulated under the old maximum is returned.
-// LOG2: scores and m are in units of log 2, where the exponential is one instruction and has no product to round, and the sum is made in pairs (a
-// chain of sixteen rounds it more).
-template<bool LOG2>
 __device__ __forceinline__ float running_softmax_step(v16f_at& s, float& m, float& l)
 {
     float mx = -FLT_MAX;
@@ -185,28 +182,13 @@ __device__ __forceinline__ float running_softmax_step(v16f_at& s, float& m, floa
     for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[r]);
     mx = fmaxf(mx, __shfl_xor(mx, 32));
     const float m_new = fmaxf(m, mx);
-    float corr, psum = 0.f;
-    if constexpr (LOG2)
+    const float corr = exp_of_nonpositive(m - m_new);
+    float psum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; r++)
     {
-        corr = __builtin_amdgcn_exp2f(m - m_new);
-        float sums[16];
-#pragma unroll
-        for (int r = 0; r < 16; r++) sums[r] = s[r] = __builtin_amdgcn_exp2f(s[r] - m_new);
-#pragma unroll
-        for (int d = 8; d > 0; d /= 2)
-#pragma unroll
-            for (int r = 0; r < d; r++) sums[r] += sums[r + d];
-        psum = sums[0];
-    }
-    else
-    {
-        corr = exp_of_nonpositive(m - m_new);
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-        {
-            s[r] = exp_of_nonpositive(s[r] - m_new);
-            psum += s[r];
-        }
+        s[r] = exp_of_nonpositive(s[r] - m_new);
+        psum += s[r];
     }
     psum += __shfl_xor(psum, 32);
     l = l * corr + psum;
@@ -311,7 +293,7 @@ __device__ __forceinline__ void attention_share_f32(const float* __restrict__ q,
         {
 #pragma unroll
             for (int kk = 0; kk < HD / 2; kk++) s_next = __builtin_amdgcn_mfma_f32_32x32x2f32(kreg[kk], qreg[kk], s_next, 0, 0, 0);
-            corr = running_softmax_step<false>(s_cur, m, l);
+            corr = running_softmax_step(s_cur, m, l);
             // issue order within the block: one product, then three of the vector instructions, while these last
 #pragma unroll
             for (int kk = 0; kk < HD / 2; kk++)
@@ -321,7 +303,7 @@ __device__ __forceinline__ void attention_share_f32(const float* __restrict__ q,
             }
         }
         else
-            corr = running_softmax_step<false>(s_cur, m, l);
+            corr = running_softmax_step(s_cur, m, l);
         asm volatile("" : "+v"(s_next), "+v"(s_cur));
         ATT_PHASE_BOUNDARY();
         {
@@ -344,14 +326,8 @@ __device__ __forceinline__ void attention_share_f32(const float* __restrict__ q,
     }
 }
 
-template<bool LOG2>
-__device__ __forceinline__ float share_weight(float x)
-{
-    return LOG2 ? exp2f(x) : expf(x);
-}
-
-// The four wavefronts' shares become the result, or the record of a key split.  LOG2: of m
-template<int HD, bool LOG2>
+// The four wavefronts' shares become the result, or the record of a key split
+template<int HD>
 __device__ __forceinline__ void attention_merge_shares(const v16f_at (&o)[HD / 32], float m, float l, int h, int i0, int src, int embed_dim, float* __restrict__ out,
                                                        bool split, float* __restrict__ rec)
 {
@@ -372,7 +348,7 @@ __device__ __forceinline__ void attention_merge_shares(const v16f_at (&o)[HD / 3
     }
     __syncthreads();
     const float mall = fmaxf(fmaxf(m_s[0][l32], m_s[1][l32]), fmaxf(m_s[2][l32], m_s[3][l32]));
-    const float f = share_weight<LOG2>(m - mall); // a wavefront that saw no key has m = -FLT_MAX, l = 0, o = 0
+    const float f = expf(m - mall); // a wavefront that saw no key has m = -FLT_MAX, l = 0, o = 0
     for (int w = 0; w < 4; w++)
     {
         if (wave == w)
@@ -398,7 +374,7 @@ __device__ __forceinline__ void attention_merge_shares(const v16f_at (&o)[HD / 3
             const float ma = fmaxf(fmaxf(m_s[0][tid], m_s[1][tid]), fmaxf(m_s[2][tid], m_s[3][tid]));
             float lt = 0.f;
 #pragma unroll
-            for (int w = 0; w < 4; w++) lt += l_s[w][tid] * share_weight<LOG2>(m_s[w][tid] - ma);
+            for (int w = 0; w < 4; w++) lt += l_s[w][tid] * expf(m_s[w][tid] - ma);
             rec[tid] = ma;
             rec[32 + tid] = lt;
         }
@@ -412,7 +388,7 @@ __device__ __forceinline__ void attention_merge_shares(const v16f_at (&o)[HD / 3
         {
             float lt = 0.f;
 #pragma unroll
-            for (int w = 0; w < 4; w++) lt += l_s[w][qq] * share_weight<LOG2>(m_s[w][qq] - fmaxf(fmaxf(m_s[0][qq], m_s[1][qq]), fmaxf(m_s[2][qq], m_s[3][qq])));
+            for (int w = 0; w < 4; w++) lt += l_s[w][qq] * expf(m_s[w][qq] - fmaxf(fmaxf(m_s[0][qq], m_s[1][qq]), fmaxf(m_s[2][qq], m_s[3][qq])));
             out[(size_t)(i0 + qq) * embed_dim + h * HD + ch] = div_rn(o_s[ch * LD + qq], lt);
         }
     }
@@ -435,7 +411,7 @@ __global__ __launch_bounds__(256) void attention_f32_mfma_kernel(const float* __
     float m, l;
     attention_share_f32<HD>(q, qi, h, kt, vt, mrow, dst, kv_stride, v_vec_ok, key_begin, key_end, q_stride, q_scale, o, m, l);
     // records: [head][query block][split]
-    attention_merge_shares<HD, false>(o, m, l, h, i0, src, embed_dim, out, keys_per_split > 0,
+    attention_merge_shares<HD>(o, m, l, h, i0, src, embed_dim, out, keys_per_split > 0,
                                partial + (((size_t)h * gridDim.x + blockIdx.x) * gridDim.z + blockIdx.z) * (size_t)(64 + HD * 32));
 }
 
@@ -480,80 +456,18 @@ __device__ __forceinline__ void split_store(const float (&x)[8], uint4* to, int 
     for (int p = 0; p < 3; p++) to[p * stride] = make_uint4(f[0][p], f[1][p], f[2][p], f[3][p]);
 }
 
-// ---- the same with every number as two fp16 numbers, for many keys ----
-// Keys, values, queries (times log2(e)) and probabilities times a power of two, hi + lo: 23 bits, and a product is hi hi, hi lo, lo hi.  Half the
-// products of the above, and the outputs are added once a tile, from sums of the tile's own that take the least products first, where the above rounds them
-// twelve times: over the rows of 500 keys and more that it is for it is the more exact of the two (relative error against 64 bits, the above / here: 16 heads of 64, 1500 on 1500
-// 3.28e-7 / 2.1e-7, 256 on 2304 2.39 / 2.18, 12 of 128, 500 on 500 2.25 / 2.10, 32 of 32, 320 on 2320 4.02 / 2.20; 64 on 64 1.29 / 1.65, 40 on 540 in
-// four splits 1.67 / 2.03).
-// A tile of 32 keys of a head has one factor for its keys and one for its values, a query its own; the outputs keep the factor of the largest values so far and the
-// probabilities of a tile make up for its own.  Where a tile's keys, its values' channels or the tiles' values differ by more than 2^16 in their largest
-// magnitudes the smaller ones would lose bits: they are stored as no numbers, as infinities are, and the wavefront that meets one repeats its share in fp32.
-// Bound by the matrix cores and the vector unit as above: 768 cycles of products a tile at head dimension 64 for 1536, some 200 vector instructions for 220.  us, the above -> here, with
-// the split and the merge: 16 heads of 64, 1500 queries and keys 82.8 -> 61.2 (the core 72.5 -> 51.2), 256 on 2304 41.9 -> 36.1; 15 of 96, 900 on 1900 94 -> 68.5; 8 of 128, 1000 on 1500
-// 71.8 -> 59.2; 32 of 32, 320 on 2320 47.8 -> 39.4.  (Three wavefronts per SIMD in 168 registers: 69.9, the loop spills.  Scores in three bf16 numbers, outputs in two fp16: 69.)
-typedef _Float16 v8h_at __attribute__((ext_vector_type(8)));
-constexpr float LOG2_E = 1.44269504f, LOG2_E_REST = 1.92596299e-8f; // log2(e) in two numbers
-constexpr int SPLIT_SPREAD = 16;
-
-// two floats -> their two fp16 pairs; ra, rb: less than their last places, added to the lower parts
-__device__ __forceinline__ void split_pair_f16(float a, float b, unsigned (&part)[2], float ra = 0.f, float rb = 0.f)
-{
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(part[0]) : "v"(a), "v"(b));
-    asm("v_fma_mix_f32 %0, -%1, 1.0, %0 op_sel_hi:[1,0,0]" : "+v"(a) : "v"(part[0])); // exact, like the next
-    asm("v_fma_mix_f32 %0, -%1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(b) : "v"(part[0]));
-    if (ra != 0.f) a += ra;
-    if (rb != 0.f) b += rb;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(part[1]) : "v"(a), "v"(b));
-}
-__device__ __forceinline__ void split_store_f16(const float (&x)[8], float factor, uint4* to, int stride) // to, to + stride
-{
-    unsigned f[4][2];
-#pragma unroll
-    for (int e = 0; e < 4; e++) split_pair_f16(x[2 * e] * factor, x[2 * e + 1] * factor, f[e]);
-#pragma unroll
-    for (int p = 0; p < 2; p++) to[p * stride] = make_uint4(f[0][p], f[1][p], f[2][p], f[3][p]);
-}
-// the larger of `top` and x's magnitude as bits, infinities and NaNs left out
-__device__ __forceinline__ unsigned top_magnitude(unsigned top, float x)
-{
-    const unsigned b = __float_as_uint(x) & 0x7FFFFFFFu;
-    return b < 0x7F800000u && b > top ? b : top;
-}
-// the power of two that takes it into [2^14, 2^15) (1 for zero, and 2^126 at most), and the one back; both are normal numbers
-__device__ __forceinline__ float split_factor(unsigned top, float& back)
-{
-    int shift = top ? 14 + 127 - (int)(top >> 23) : 0;
-    if (shift > 126) shift = 126;
-    back = __uint_as_float((unsigned)(127 - shift) << 23);
-    return __uint_as_float((unsigned)(127 + shift) << 23);
-}
-__device__ __forceinline__ float inverse_of_power(float x) // of two, normal, up to 2^126; 2^127 for zero
-{
-    return __uint_as_float((254u << 23) - __float_as_uint(x));
-}
-// the factor of groups whose largest magnitudes lie between low and high
-__device__ __forceinline__ float factor_of_groups(unsigned high, unsigned low, float& back)
-{
-    const float f = split_factor(high, back);
-    return high && (low >> 23) + SPLIT_SPREAD < (high >> 23) ? __uint_as_float(0x7FC00000u) : f;
-}
-
 // One workgroup: 32 keys of one head.  new_k / new_v (or null): the keys and values of the positions from `past` on, rows of new_stride floats
 // ([position][embed]); they are copied into kt / vt on the way (appending to the cache is then no launch of its own).
 // Bound by memory, with 20 bytes moved for a float (28 for a new one), and on few keys by its latency: every load of a thread is requested
 // before the first is used, and LDS is sized by the head dimension (1500 new keys of 16 heads of 64, 43 MB: 13 us with loads as they come
 // and room for 128 channels in 32 KB).
-template<int HD, bool F16>
+template<int HD>
 __global__ __launch_bounds__(256) void attention_split_kernel(float* kt, float* vt, size_t kv_stride, int dst, const float* __restrict__ new_k,
-                                                              const float* __restrict__ new_v, size_t new_stride, int past, uint4* __restrict__ frags, float2* __restrict__ backs)
+                                                              const float* __restrict__ new_v, size_t new_stride, int past, uint4* __restrict__ frags)
 {
-    constexpr int EACH = HD / 8, STEPS = HD / 16, PARTS = F16 ? 2 : 3;
+    constexpr int EACH = HD / 8, STEPS = HD / 16;
     __shared__ float tile[2][HD][33];
-    __shared__ unsigned top[F16 ? 32 + HD : 1]; // largest magnitudes of the keys, of the channels of the values
-    __shared__ float factor[2];
     const int j0 = blockIdx.x * 32, h = blockIdx.y, tid = threadIdx.x;
-    if (F16 && tid < 32) top[tid] = 0;
     const size_t row0 = (size_t)h * HD;
     const int known = new_k ? past : dst; // columns of kt / vt that are there
     float x[2][EACH];
@@ -611,62 +525,7 @@ __global__ __launch_bounds__(256) void attention_split_kernel(float* kt, float* 
             vt[(row0 + c0 + 8 * i) * kv_stride + j] = tile[1][c0 + 8 * i][key];
         }
     }
-    const size_t unit = (size_t)h * gridDim.x + blockIdx.x;
-    float fk = 0.f, fv = 0.f;
-    if constexpr (F16)
-    {
-        unsigned most = 0;
-#pragma unroll
-        for (int i = 0; i < EACH; i++) most = top_magnitude(most, tile[0][c0 + 8 * i][key]);
-        atomicMax(&top[key], most);
-        for (int e = tid; e < HD * 4; e += 256) // four lanes a channel
-        {
-            most = 0;
-#pragma unroll
-            for (int i = 0; i < 8; i++) most = top_magnitude(most, tile[1][e >> 2][(e & 3) * 8 + i]);
-            unsigned other = (unsigned)__builtin_amdgcn_mov_dpp((int)most, 0xB1, 0xF, 0xF, true); // lane ^ 1
-            if (other > most) most = other;
-            other = (unsigned)__builtin_amdgcn_mov_dpp((int)most, 0x4E, 0xF, 0xF, true); // lane ^ 2
-            if (other > most) most = other;
-            if ((e & 3) == 0) top[32 + (e >> 2)] = most;
-        }
-        __syncthreads();
-        if (tid < 128) // wavefront 0: the keys' factor; 1: the values'
-        {
-            const int of = tid >> 6, count = of ? HD : 32;
-            unsigned high = 0, low = 0xFFFFFFFFu;
-            for (int i = tid & 63; i < count; i += 64)
-            {
-                const unsigned b = top[of * 32 + i];
-                if (b > high) high = b;
-                if (b && b < low) low = b;
-            }
-#pragma unroll
-            for (int d = 1; d < 64; d *= 2)
-            {
-                const unsigned a = (unsigned)__shfl_xor((int)high, d), b = (unsigned)__shfl_xor((int)low, d);
-                if (a > high) high = a;
-                if (b < low) low = b;
-            }
-            float back;
-            const float f = factor_of_groups(high, low, back);
-            if ((tid & 63) == 0)
-            {
-                factor[of] = f;
-                (of ? backs[unit].y : backs[unit].x) = of && !high ? 0.f : back; // values of zeros have no say in what the sums are scaled by
-            }
-        }
-        __syncthreads();
-        fk = factor[0];
-        fv = factor[1];
-    }
-    const auto store = [&](const float (&y)[8], float by, uint4* at) {
-        if constexpr (F16)
-            split_store_f16(y, by, at, 64);
-        else
-            split_store(y, at, 64);
-    };
-    uint4* to = frags + unit * (size_t)(STEPS * 2 * PARTS * 64);
+    uint4* to = frags + ((size_t)h * gridDim.x + blockIdx.x) * (size_t)(STEPS * 6 * 64);
     for (int e = tid; e < STEPS * 64; e += 256)
     {
         const int step = e >> 6, lane = e & 63, l32 = lane & 31, hh = lane >> 5;
@@ -674,22 +533,21 @@ __global__ __launch_bounds__(256) void attention_split_kernel(float* kt, float* 
         // keys: lane = key, channels step * 16 + hh * 8 ..; values: step = 32 channels and half of the keys, in the order of the accumulators
 #pragma unroll
         for (int i = 0; i < 8; i++) y[i] = tile[0][step * 16 + hh * 8 + i][l32];
-        store(y, fk, to + step * PARTS * 64 + lane);
+        split_store(y, to + step * 3 * 64 + lane, 64);
 #pragma unroll
         for (int i = 0; i < 8; i++) y[i] = tile[1][(step >> 1) * 32 + l32][(step & 1) * 16 + 8 * (i >> 2) + 4 * hh + (i & 3)];
-        store(y, fv, to + (STEPS + step) * PARTS * 64 + lane);
+        split_store(y, to + (STEPS + step) * 3 * 64 + lane, 64);
     }
 }
 
-template<int HD, bool F16>
-__global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attention_split_core_kernel(const float* __restrict__ q, const float* __restrict__ kt, const float* __restrict__ vt,
-                                                               const uint4* __restrict__ frags, const float2* __restrict__ backs, const float* __restrict__ mask, int mask_heads, int embed_dim, int src,
+template<int HD>
+__global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attention_bf16x3_kernel(const float* __restrict__ q, const float* __restrict__ kt, const float* __restrict__ vt,
+                                                               const uint4* __restrict__ frags, const float* __restrict__ mask, int mask_heads, int embed_dim, int src,
                                                                int dst, size_t kv_stride, float* __restrict__ out, int v_vec_ok, int keys_per_split,
                                                                float* __restrict__ partial, size_t q_stride, float q_scale, int query_blocks, int splits)
 {
-    constexpr int CB = HD / 32, STEPS = HD / 16, PARTS = F16 ? 2 : 3, PRODUCTS = F16 ? 3 : 6;
-    __shared__ uint4 q_s[STEPS * PARTS * 64];
-    __shared__ unsigned q_top[F16 ? 32 : 1];
+    constexpr int CB = HD / 32, STEPS = HD / 16;
+    __shared__ uint4 q_s[STEPS * 3 * 64];
     // The query blocks of a head read the same fragments, 384 bytes a key and 32 channels: they follow one another on one die (workgroups are
     // dealt to the 8 dies in turn), whose L2 then holds a few heads at a time instead of all of them (16 heads of 64, 256 queries, 2304 keys:
     // 64 us without, 46 with).  With `splits` beyond 1 that many workgroups share a unit's keys.
@@ -702,67 +560,20 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attention_split_core_ke
     const int key_begin = z * keys_per_split;
     const int key_end = splits > 1 && key_begin + keys_per_split < dst ? key_begin + keys_per_split : dst; // a multiple of 32, or dst
 
-    float q_back = 1.f; // of this lane's query
-    if constexpr (F16)
+    for (int step = wave; step < STEPS; step += 4)
     {
-        constexpr int QS = (STEPS + 3) / 4;
-        float x[QS][8], rest[QS][8]; // what rounding x dropped
-        unsigned most = 0;
-        if (tid < 32) q_top[tid] = 0;
-        __syncthreads();
+        const float* from = q + (size_t)qi * q_stride + h * HD + step * 16 + hh * 8;
+        float x[8];
 #pragma unroll
-        for (int u = 0; u < QS; u++)
-        {
-            const int step = wave + 4 * u < STEPS ? wave + 4 * u : STEPS - 1;
-            const float* from = q + (size_t)qi * q_stride + h * HD + step * 16 + hh * 8;
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-            {
-                const float scaled = mul_rn(from[i], q_scale);
-                x[u][i] = mul_rn(scaled, LOG2_E);
-                rest[u][i] = fmaf(scaled, LOG2_E, -x[u][i]) + scaled * LOG2_E_REST;
-                most = top_magnitude(most, x[u][i]);
-            }
-        }
-        atomicMax(&q_top[l32], most);
-        __syncthreads();
-        const float factor = split_factor(q_top[l32], q_back);
-#pragma unroll
-        for (int u = 0; u < QS; u++)
-            if (wave + 4 * u < STEPS)
-            {
-                unsigned f[4][2];
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    split_pair_f16(x[u][2 * e] * factor, x[u][2 * e + 1] * factor, f[e], rest[u][2 * e] * factor, rest[u][2 * e + 1] * factor);
-#pragma unroll
-                for (int p = 0; p < 2; p++) q_s[((wave + 4 * u) * 2 + p) * 64 + lane] = make_uint4(f[0][p], f[1][p], f[2][p], f[3][p]);
-            }
-    }
-    else
-    {
-        for (int step = wave; step < STEPS; step += 4)
-        {
-            const float* from = q + (size_t)qi * q_stride + h * HD + step * 16 + hh * 8;
-            float x[8];
-#pragma unroll
-            for (int i = 0; i < 8; i++) x[i] = mul_rn(from[i], q_scale);
-            split_store(x, q_s + step * 3 * 64 + lane, 64);
-        }
+        for (int i = 0; i < 8; i++) x[i] = mul_rn(from[i], q_scale);
+        split_store(x, q_s + step * 3 * 64 + lane, 64);
     }
     __syncthreads();
 
     union Frag
     {
         uint4 u;
-        v8bf_at b;
-        v8h_at h;
-    };
-    const auto product = [](const Frag& a, const Frag& b, v16f_at sum) {
-        if constexpr (F16)
-            return __builtin_amdgcn_mfma_f32_32x32x16_f16(a.h, b.h, sum, 0, 0, 0);
-        else
-            return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.b, b.b, sum, 0, 0, 0);
+        v8bf_at h;
     };
     v16f_at o[CB];
 #pragma unroll
@@ -771,32 +582,27 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attention_split_core_ke
         for (int r = 0; r < 16; r++) o[cb][r] = 0.f;
     float m = -FLT_MAX, l = 0.f;
     // pairs (of the first operand, of the second) in the order they are added
-    constexpr int PA[6] = {1, 0, F16 ? 0 : 2, 0, 1, 0}, PB[6] = {F16 ? 0 : 1, F16 ? 1 : 2, 0, 1, 0, 0};
+    constexpr int PA[6] = {1, 0, 2, 0, 1, 0}, PB[6] = {1, 2, 0, 1, 0, 0};
 
     const int t_first = key_begin / 32 + wave, t_end = (key_end + 31) / 32;
-    const int tiles = (dst + 31) / 32;
-    const uint4* base = frags + (size_t)h * tiles * (size_t)(STEPS * 2 * PARTS * 64) + lane;
-    const float2* back = backs + (size_t)h * tiles;
-    float2 next_back = make_float2(1.f, 0.f);
-    if (F16 && t_first < t_end) next_back = back[t_first];
-    float v_back = 0.f; // F16: times 2^-14, what takes the outputs back
-    Frag kf[STEPS * PARTS];
+    const uint4* base = frags + (size_t)h * ((dst + 31) / 32) * (size_t)(STEPS * 6 * 64) + lane;
+    Frag kf[STEPS * 3];
     auto load_keys = [&](int t) {
-        const uint4* f = base + (size_t)t * (STEPS * 2 * PARTS * 64);
+        const uint4* f = base + (size_t)t * (STEPS * 6 * 64);
 #pragma unroll
-        for (int i = 0; i < STEPS * PARTS; i++) kf[i].u = f[i * 64];
+        for (int i = 0; i < STEPS * 3; i++) kf[i].u = f[i * 64];
     };
     auto scores = [&](v16f_at& s) {
         unsigned at = lane; // (opaque: the queries' fragments are read again for every tile, not kept in 48 registers)
         asm volatile("" : "+v"(at));
 #pragma unroll
-        for (int pr = 0; pr < PRODUCTS; pr++)
+        for (int pr = 0; pr < 6; pr++)
 #pragma unroll
             for (int step = 0; step < STEPS; step++)
             {
                 Frag qf;
-                qf.u = q_s[(step * PARTS + PB[pr]) * 64 + at];
-                s = product(kf[step * PARTS + PA[pr]], qf, s);
+                qf.u = q_s[(step * 3 + PB[pr]) * 64 + at];
+                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[step * 3 + PA[pr]].h, qf.h, s, 0, 0, 0);
             }
     };
     v16f_at s_cur;
@@ -815,22 +621,13 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attention_split_core_ke
     for (int t = t_first; t < t_end; t += 4)
     {
         const int j0 = t * 32;
-        const float2 this_back = next_back;
-        if (F16) next_back = back[t + 4 < t_end ? t + 4 : t];
-        const uint4* vfrom = base + (size_t)t * (STEPS * 2 * PARTS * 64) + STEPS * PARTS * 64;
+        const uint4* vfrom = base + (size_t)t * (STEPS * 6 * 64) + STEPS * 3 * 64;
         constexpr int VB = CB <= 2 ? CB : 1; // value blocks requested ahead: all of them while the registers last, else one at a time
-        Frag vf[VB * 2 * PARTS];
+        Frag vf[VB * 6];
         if constexpr (CB <= 2)
         {
 #pragma unroll
-            for (int i = 0; i < VB * 2 * PARTS; i++) vf[i].u = vfrom[i * 64];
-        }
-        if constexpr (F16)
-        {
-            float f = this_back.x * q_back;
-            if (!(f >= FLT_MIN && f <= FLT_MAX)) f = __uint_as_float(0x7FC00000u);
-#pragma unroll
-            for (int r = 0; r < 16; r++) s_cur[r] *= f;
+            for (int i = 0; i < VB * 6; i++) vf[i].u = vfrom[i * 64];
         }
         if (mrow)
         {
@@ -842,12 +639,7 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attention_split_core_ke
                 mv[r] = mrow[key < dst ? key : dst - 1];
             }
 #pragma unroll
-            for (int r = 0; r < 16; r++)
-            {
-                float v = mv[r];
-                if (F16 && v >= -FLT_MAX) v = fmaxf(mul_rn(v, LOG2_E), -FLT_MAX); // (the type's lowest value stays that)
-                s_cur[r] = add_rn(s_cur[r], v);
-            }
+            for (int r = 0; r < 16; r++) s_cur[r] = add_rn(s_cur[r], mv[r]);
         }
         if (j0 + 32 > dst)
         {
@@ -863,32 +655,23 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attention_split_core_ke
         if (t + 4 < t_end)
         {
             scores(s_next);
-            corr = running_softmax_step<F16>(s_cur, m, l);
-            // issue order: one product, then five (of half the products eight) of the vector instructions, while these last
+            corr = running_softmax_step(s_cur, m, l);
+            // issue order: one product, then five of the vector instructions, while these last
 #pragma unroll
-            for (int i = 0; i < STEPS * PRODUCTS; i++)
+            for (int i = 0; i < STEPS * 6; i++)
             {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, (F16 ? 32 : 20) / STEPS, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 20 / STEPS, 0);
             }
         }
         else
-            corr = running_softmax_step<F16>(s_cur, m, l);
+            corr = running_softmax_step(s_cur, m, l);
         asm volatile("" : "+v"(s_next), "+v"(s_cur));
         ATT_PHASE_BOUNDARY();
         load_keys(t + 8 < t_end ? t + 8 : t);
         ATT_PHASE_BOUNDARY();
-        float p_factor = 1.f;
-        if constexpr (F16)
-        {
-            const float v_new = fmaxf(v_back, this_back.y), shrink = inverse_of_power(v_new);
-            p_factor = this_back.y * shrink * 16384.f;
-            if (this_back.y != 0.f && p_factor < 16384.f / (1 << SPLIT_SPREAD)) l = __uint_as_float(0x7FC00000u);
-            corr *= v_back * shrink;
-            v_back = v_new;
-        }
-        else if (__any(corr != 1.f))
+        if (__any(corr != 1.f))
         {
 #pragma unroll
             for (int cb = 0; cb < CB; cb++)
@@ -896,21 +679,15 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attention_split_core_ke
                 for (int r = 0; r < 16; r++) o[cb][r] *= corr;
         }
         // the probabilities' parts: registers 8 * s .. + 7 are the second operand of the values' step s
-        Frag pf[2][PARTS];
+        Frag pf[2][3];
 #pragma unroll
         for (int s = 0; s < 2; s++)
         {
-            unsigned f[4][PARTS];
+            unsigned f[4][3];
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-            {
-                if constexpr (F16)
-                    split_pair_f16(s_cur[8 * s + 2 * e] * p_factor, s_cur[8 * s + 2 * e + 1] * p_factor, f[e]);
-                else
-                    split_pair(s_cur[8 * s + 2 * e], s_cur[8 * s + 2 * e + 1], f[e]);
-            }
+            for (int e = 0; e < 4; e++) split_pair(s_cur[8 * s + 2 * e], s_cur[8 * s + 2 * e + 1], f[e]);
 #pragma unroll
-            for (int p = 0; p < PARTS; p++) pf[s][p].u = make_uint4(f[0][p], f[1][p], f[2][p], f[3][p]);
+            for (int p = 0; p < 3; p++) pf[s][p].u = make_uint4(f[0][p], f[1][p], f[2][p], f[3][p]);
         }
 #pragma unroll
         for (int c0 = 0; c0 < CB; c0 += VB)
@@ -918,44 +695,17 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attention_split_core_ke
             if constexpr (CB > 2)
             {
 #pragma unroll
-                for (int i = 0; i < 2 * PARTS; i++) vf[i].u = vfrom[(c0 * 2 * PARTS + i) * 64];
+                for (int i = 0; i < 6; i++) vf[i].u = vfrom[(c0 * 6 + i) * 64];
             }
-if constexpr (F16)
-            {
-                v16f_at sum[VB];
 #pragma unroll
-                for (int c = 0; c < VB; c++)
+            for (int s = 0; s < 2; s++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) sum[c][r] = 0.f;
+                for (int pr = 0; pr < 6; pr++)
 #pragma unroll
-                for (int pr = 0; pr < PRODUCTS; pr++)
-#pragma unroll
-                    for (int s = 0; s < 2; s++)
-#pragma unroll
-                        for (int c = 0; c < VB; c++) sum[c] = product(vf[(c * 2 + s) * PARTS + PA[pr]], pf[s][PB[pr]], sum[c]);
-#pragma unroll
-                for (int c = 0; c < VB; c++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) o[c0 + c][r] = fmaf(o[c0 + c][r], corr, sum[c][r]);
-            }
-            else
-            {
-#pragma unroll
-                for (int s = 0; s < 2; s++)
-#pragma unroll
-                    for (int pr = 0; pr < PRODUCTS; pr++)
-#pragma unroll
-                        for (int c = 0; c < VB; c++) o[c0 + c] = product(vf[(c * 2 + s) * PARTS + PA[pr]], pf[s][PB[pr]], o[c0 + c]);
-            }
+                    for (int c = 0; c < VB; c++)
+                        o[c0 + c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[c * 6 + s * 3 + PA[pr]].h, pf[s][PB[pr]].h, o[c0 + c], 0, 0, 0);
         }
         s_cur = s_next;
-    }
-    if constexpr (F16)
-    {
-#pragma unroll
-        for (int cb = 0; cb < CB; cb++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) o[cb][r] = o[cb][r] * (1.f / 16384.f) * v_back;
     }
     float nan = l != l ? 1.f : 0.f;
 #pragma unroll
@@ -963,18 +713,14 @@ if constexpr (F16)
 #pragma unroll
         for (int r = 0; r < 16; r++) nan = o[cb][r] != o[cb][r] ? 1.f : nan;
     if (__any(nan != 0.f))
-    {
         attention_share_f32<HD>(q, qi, h, kt, vt, mrow, dst, kv_stride, v_vec_ok, key_begin, key_end, q_stride, q_scale, o, m, l);
-        if (F16 && m > -FLT_MAX) m = mul_rn(m, LOG2_E);
-    }
-    attention_merge_shares<HD, F16>(o, m, l, h, i0, src, embed_dim, out, splits > 1, partial + ((size_t)unit * splits + z) * (size_t)(64 + HD * 32));
+    attention_merge_shares<HD>(o, m, l, h, i0, src, embed_dim, out, splits > 1, partial + ((size_t)unit * splits + z) * (size_t)(64 + HD * 32));
 }
 
 // merges the records of the key splits: one workgroup per (head, query block).  First every (split, query) pair gets its factor
 // exp(m_split - m) and the queries their sums, through LDS; then the outputs are added with eight independent loads in
 // flight per thread (a thread that walks the splits for each of its outputs, one dependent load after the other, took 35 us
 // for 64 queries x 16 heads x 11 splits).
-template<bool LOG2>
 __global__ __launch_bounds__(256) void attention_merge_kernel(const float* __restrict__ partial, int query_blocks, int splits, int head_dim,
                                                               int embed_dim, int src, float* __restrict__ out)
 {
@@ -994,7 +740,7 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const float* __res
         float lt = 0.f;
         for (int z = 0; z < splits; z++)
         {
-            const float f = LOG2 ? exp2f(fac[z][tid] - ma) : exp_of_nonpositive(fac[z][tid] - ma);
+            const float f = exp_of_nonpositive(fac[z][tid] - ma);
             fac[z][tid] = f;
             lt += rec0[(size_t)z * rec_size + 32 + tid] * f; // independent loads: the compiler keeps several in flight
         }
@@ -1427,7 +1173,7 @@ static int attention_key_splits(int num_heads, int src, int dst)
 //   below that up to 64 D Q: 16 x 64, 64 queries: 13.7 12.2 alone, 21.4 18.0 on 250; beyond, on 1000: 21.6 24.8; 32 x 32, 16 queries on 250: 13.9 15.4;
 //   and with 8 blocks always: 16 x 64, 320 queries on 4000: 101 65; 32 x 32 the same: 101 72.
 // One tile of keys for one small block of queries stays where it is: 16 x 64, 5 queries: 10.5 10.9.
-static bool attention_split_core_applies(int num_heads, int head_dim, int src, int dst)
+static bool attention_bf16x3_applies(int num_heads, int head_dim, int src, int dst)
 {
     if (head_dim % 32 != 0 || head_dim > 128 || src <= ATT_TQ) return false;
     const long long blocks = (src + 31) / 32, width = head_dim * blocks, keys = (long long)num_heads * dst;
@@ -1439,7 +1185,7 @@ static bool attention_split_core_applies(int num_heads, int head_dim, int src, i
 // some thousands up to 20 % less).  Units (32 queries of a head) that would leave half of these places empty share their keys out over as many
 // workgroups as there are places, at least 128 keys each.  (Rounding up as above, or sharing out the last, partly filled of several
 // rounds: 768 units at 1500 keys 82 us without, 88 with.)
-static int attention_split_core_splits(int num_heads, int head_dim, int src, int dst, int& keys_per_split)
+static int attention_bf16x3_splits(int num_heads, int head_dim, int src, int dst, int& keys_per_split)
 {
     const long long units = (long long)((src + 31) / 32) * num_heads;
     long long want = (head_dim <= 64 ? 512 : 256) / units;
@@ -1461,10 +1207,10 @@ static size_t attention_frags_bytes(int num_heads, int head_dim, int dst)
 {
     return (size_t)num_heads * ((dst + 31) / 32) * (size_t)head_dim * 384;
 }
-static size_t attention_split_core_bytes(int num_heads, int head_dim, int src, int dst)
+static size_t attention_bf16x3_bytes(int num_heads, int head_dim, int src, int dst)
 {
     int keys_per_split;
-    const int splits = attention_split_core_splits(num_heads, head_dim, src, dst, keys_per_split);
+    const int splits = attention_bf16x3_splits(num_heads, head_dim, src, dst, keys_per_split);
     return attention_frags_bytes(num_heads, head_dim, dst) + (splits > 1 ? (size_t)((src + 31) / 32) * num_heads * splits * attention_record_bytes(head_dim) : 0);
 }
 
@@ -1479,9 +1225,9 @@ int ncnnhip_attention_workspace_bytes(int num_heads, int head_dim, int src_seqle
     NCNNHIP_REQUIRE(num_heads >= 1 && head_dim >= 1 && src_seqlen >= 1 && dst_seqlen >= 1 && workspace_bytes, "ncnnhip_attention_workspace_bytes: bad argument");
     *workspace_bytes = 0;
     if (head_dim % 32 == 0 && head_dim <= 128) *workspace_bytes = attention_records_bytes(num_heads, head_dim, src_seqlen, dst_seqlen);
-    if (attention_split_core_applies(num_heads, head_dim, src_seqlen, dst_seqlen))
+    if (attention_bf16x3_applies(num_heads, head_dim, src_seqlen, dst_seqlen))
     {
-        const size_t need = attention_split_core_bytes(num_heads, head_dim, src_seqlen, dst_seqlen);
+        const size_t need = attention_bf16x3_bytes(num_heads, head_dim, src_seqlen, dst_seqlen);
         if (need > *workspace_bytes) *workspace_bytes = need;
     }
     if (attention_fewq_applies(head_dim, src_seqlen, dst_seqlen))
@@ -1583,38 +1329,26 @@ static int attention_dispatch(const float* q_dev, size_t q_stride, float q_scale
     const int v_vec_ok = (kv_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(vt_dev) & 15) == 0) ? 1 : 0;
     const unsigned units = (unsigned)query_blocks * (unsigned)num_heads;
     // enough workgroups for the merge: the outputs of a unit shared out over up to 8 of them
-    const auto merge = [&](const float* partial, int splits, bool log2) {
+    const auto merge = [&](const float* partial, int splits) {
         unsigned shares = 1;
         while (shares < 8 && units * shares < 256 && (unsigned)(32 * head_dim) / (shares * 2) >= 256) shares *= 2;
-        hipLaunchKernelGGL(log2 ? attention_merge_kernel<true> : attention_merge_kernel<false>, dim3(units, shares), dim3(256), 0, st, partial, query_blocks, splits, head_dim, e, src_seqlen,
+        hipLaunchKernelGGL(attention_merge_kernel, dim3(units, shares), dim3(256), 0, st, partial, query_blocks, splits, head_dim, e, src_seqlen,
                            out_dev);
     };
-    if (attention_split_core_applies(num_heads, head_dim, src_seqlen, dst_seqlen) && workspace_dev && (reinterpret_cast<uintptr_t>(workspace_dev) & 15) == 0
-        && workspace_bytes >= attention_split_core_bytes(num_heads, head_dim, src_seqlen, dst_seqlen))
+    if (attention_bf16x3_applies(num_heads, head_dim, src_seqlen, dst_seqlen) && workspace_dev && (reinterpret_cast<uintptr_t>(workspace_dev) & 15) == 0
+        && workspace_bytes >= attention_bf16x3_bytes(num_heads, head_dim, src_seqlen, dst_seqlen))
     {
         int keys_per_split;
-        const int splits = attention_split_core_splits(num_heads, head_dim, src_seqlen, dst_seqlen, keys_per_split);
+        const int splits = attention_bf16x3_splits(num_heads, head_dim, src_seqlen, dst_seqlen, keys_per_split);
         uint4* frags = static_cast<uint4*>(workspace_dev);
         float* partial = reinterpret_cast<float*>(static_cast<char*>(workspace_dev) + attention_frags_bytes(num_heads, head_dim, dst_seqlen));
         const dim3 tiles((unsigned)((dst_seqlen + 31) / 32), (unsigned)num_heads), grid(units * (unsigned)splits);
-        // two fp16 numbers from 500 keys a workgroup on: below, their error is the larger one and the two are as fast (16 heads of 64, 64 on 64 1.29e-7 against 1.65e-7, 12.3 us against 12.5)
-        const bool f16 = (splits > 1 ? keys_per_split : dst_seqlen) >= 500;
-        float2* backs = reinterpret_cast<float2*>(frags + (size_t)num_heads * ((dst_seqlen + 31) / 32) * (size_t)head_dim * 16); // (a tile's 16 x 16 bytes a channel are fragments)
-#define LAUNCH_ATT_AS(HD_, F16_)                                                                                                                                   \
+#define LAUNCH_ATT(HD_)                                                                                                                                            \
     do                                                                                                                                                             \
     {                                                                                                                                                              \
-        hipLaunchKernelGGL((attention_split_kernel<HD_, F16_>), tiles, dim3(256), 0, st, kt_dev, vt_dev, kv_stride, dst_seqlen, append_k, append_v, append_stride, past, \
-                           frags, backs);                                                                                                                          \
-        hipLaunchKernelGGL((attention_split_core_kernel<HD_, F16_>), grid, dim3(256), 0, st, q_dev, kt_dev, vt_dev, frags, backs, mask_dev, mh, e, src_seqlen,      \
-                           dst_seqlen, kv_stride, out_dev, v_vec_ok, keys_per_split, partial, q_stride, q_scale, query_blocks, splits);                            \
-    } while (0)
-#define LAUNCH_ATT(HD_)                \
-    do                                 \
-    {                                  \
-        if (f16)                       \
-            LAUNCH_ATT_AS(HD_, true);  \
-        else                           \
-            LAUNCH_ATT_AS(HD_, false); \
+        hipLaunchKernelGGL(attention_split_kernel<HD_>, tiles, dim3(256), 0, st, kt_dev, vt_dev, kv_stride, dst_seqlen, append_k, append_v, append_stride, past, frags); \
+        hipLaunchKernelGGL(attention_bf16x3_kernel<HD_>, grid, dim3(256), 0, st, q_dev, kt_dev, vt_dev, frags, mask_dev, mh, e, src_seqlen, dst_seqlen, kv_stride,  \
+                           out_dev, v_vec_ok, keys_per_split, partial, q_stride, q_scale, query_blocks, splits);                                 \
     } while (0)
         if (head_dim == 32)
             LAUNCH_ATT(32);
@@ -1625,9 +1359,8 @@ static int attention_dispatch(const float* q_dev, size_t q_stride, float q_scale
         else
             LAUNCH_ATT(128);
 #undef LAUNCH_ATT
-#undef LAUNCH_ATT_AS
-        if (splits > 1) merge(partial, splits, f16);
-        return launch_status("attention_split_core_kernel");
+        if (splits > 1) merge(partial, splits);
+        return launch_status("attention_bf16x3_kernel");
     }
     if (append_k)
     {
@@ -1661,7 +1394,7 @@ static int attention_dispatch(const float* q_dev, size_t q_stride, float q_scale
         else
             LAUNCH_ATT(128);
 #undef LAUNCH_ATT
-        if (keys_per_split > 0) merge(partial, splits, false);
+        if (keys_per_split > 0) merge(partial, splits);
         return launch_status("attention_f32_mfma_kernel");
     }
     const size_t lds = (size_t)ATT_TQ * ((size_t)head_dim + (size_t)dst_seqlen) * sizeof(float);

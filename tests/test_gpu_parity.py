@@ -884,9 +884,9 @@ def test_attention_core_on_split_keys_and_values_with_numbers_too_small_to_split
 # 500 keys a workgroup and more: one workgroup for all keys of a unit (a last tile of 12 keys, of all 32), and three for 1530 (merged from their records)
 @pytest.mark.parametrize("heads,hd,src,dst", [(16, 32, 520, 500), (16, 64, 513, 544), (16, 96, 270, 700), (8, 128, 1030, 511), (16, 32, 300, 1530)])
 @pytest.mark.parametrize("kind", ["mask", "keys", "values", "channels", "zeros", "scaled", "special"])
-def test_attention_core_in_two_fp16_numbers(rt, heads, hd, src, dst, kind):
-    """Keys, values and queries times powers of two, as two fp16 numbers each: masks of the lowest value (of a whole row, too) and of -inf, numbers whose sizes lie too
-    far apart for a common factor in a tile of keys, between tiles and between channels, tiles of zeros, sizes near both ends of fp32: no more error against float64 than
+def test_attention_core_on_many_keys(rt, heads, hd, src, dst, kind):
+    """The bf16 form on 500 keys a workgroup and more: masks of the lowest value (of a whole row, too) and of -inf, numbers whose sizes lie far
+    apart in a tile of keys, between tiles and between channels, tiles of zeros, sizes near both ends of fp32: no more error against float64 than
     the fp32 form has (but for the spread between two orders of a sum), in each channel where they differ in size; infinities and NaNs where it has them."""
     print("[case]", heads, hd, src, dst, kind, flush=True)
     rng = np.random.default_rng(heads * 1000 + src)
@@ -934,6 +934,59 @@ def test_attention_core_in_two_fp16_numbers(rt, heads, hd, src, dst, kind):
         error, fp32 = (np.sqrt(np.mean((x[:, cols] - want[:, cols]) ** 2)) / norm for x in (got, plain))
         assert error <= 1.25 * fp32 + 2.0 ** -23, (error, fp32)
     assert kind != "zeros" or np.all(got[:, :hd] == 0)
+
+
+@pytest.mark.parametrize("heads,hd,src,dst", [(16, 64, 513, 544), (8, 128, 1030, 511), (16, 32, 300, 1530)])
+@pytest.mark.parametrize("kind", ["last key", "a key of each tile", "faint key", "key channel", "query channel", "low masks", "lower masks", "small channel"])
+def test_attention_core_on_large_numbers_that_meet_nothing(rt, heads, hd, src, dst, kind):
+    """A key whose values are 2^30 times its neighbours' and which is masked, or attended by 2^-45 of a query; a channel that is large in the keys and zero in the queries, or
+    the other way round: what it meets is (next to) nothing, and the others keep all their bits.  Rows masked throughout by less than the lowest value, beside values so small
+    that their wavefronts go through the fp32 form: all of their keys count alike, but for those of the lowest value.  No more error against float64 than the fp32 form has but for the spread between two orders of a sum."""
+    print("[case]", heads, hd, src, dst, kind, flush=True)
+    rng = np.random.default_rng(heads * 1000 + src)
+    e = heads * hd
+    q = (rng.normal(0, 1, (src, e)) / np.sqrt(hd)).astype(F)
+    kt, vt = (rng.normal(0, 1, (e, dst)).astype(F) for _ in range(2))
+    m = None
+    if kind == "last key":
+        vt[:, dst - 1] *= F(2.0 ** 30)
+        m = np.zeros((src, dst), F)
+        m[:, dst - 1] = -np.finfo(F).max
+    elif kind == "a key of each tile":
+        vt[:, 5::32] *= F(2.0 ** 30)
+        m = np.zeros((src, dst), F)
+        m[:, 5::32] = -np.inf
+    elif kind == "faint key":
+        vt[:, dst - 1] *= F(2.0 ** 30)
+        m = np.zeros((src, dst), F)
+        m[:, dst - 1] = F(-np.log(2.0) * 45)
+    elif kind == "key channel":
+        kt[5::hd] *= F(2.0 ** 40)
+        q[:, 5::hd] = 0
+    elif kind == "query channel":
+        q[:, 5::hd] *= F(2.0 ** 40)
+        kt[5::hd] = 0
+    elif kind == "small channel":  # alone in its channel
+        vt[3::hd] *= F(2.0 ** -30)
+    else:
+        m = rng.normal(0, 1, (src, dst)).astype(F)
+        m[2:40] = F(-3e38)
+        vt[3::hd, slice(0, dst) if kind == "low masks" else slice(32, 64)] *= F(2.0 ** -115)
+        if kind == "lower masks":
+            m[2:40, dst // 2:] = -np.finfo(F).max
+    got, plain = rt.attention(q, kt, vt, heads, m), rt.attention(q, kt, vt, heads, m, use_workspace=False)
+    want = np.empty((src, e))
+    for h in range(heads):
+        sl = slice(h * hd, (h + 1) * hd)
+        s = q[:, sl].astype(np.float64) @ kt[sl].astype(np.float64)
+        if m is not None:
+            s = s + m.astype(np.float64)
+        s = np.exp(s - s.max(axis=1, keepdims=True))
+        want[:, sl] = (s / s.sum(axis=1, keepdims=True)) @ vt[sl].astype(np.float64).T
+    for cols in (slice(None),) + ((slice(3, e, hd),) if kind == "small channel" else ()):
+        norm = np.sqrt(np.mean(want[:, cols] ** 2))
+        error, fp32 = (np.sqrt(np.mean((x[:, cols] - want[:, cols]) ** 2)) / norm for x in (got, plain))
+        assert error <= 1.25 * fp32 + 2.0 ** -23, (error, fp32)
 
 
 @pytest.mark.parametrize("heads,hd,src,dst", [(4, 64, 37, 200), (2, 32, 1, 300), (3, 24, 5, 40)])
