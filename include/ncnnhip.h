@@ -488,9 +488,8 @@ int ncnnhip_gemm_blockquant_packed_multi(const void* a_dev, int a_elemsize, size
  * go, while that is the quicker way (some tens to some hundreds of rows), to the kernel ncnnhip_gemm_blockquant_packed has for more than
  * four, which splits the activations as it multiplies them and leaves the workspace alone.  All others are split once, into the workspace,
  * by a pass of its own: up to 128 rows off 16 bytes on small weights then stream the weights once per 16 rows, all passes in one launch;
- * the rest is a tiled Gemm on the matrix cores, 64 activation rows x 64, 128 or 192 weight rows per workgroup (prefill, attention
- * projections).  For weights in blocks of 64 and 128 it scales each row by a power of two and splits it into two fp16 numbers: 23 bits of every
- * activation, and what lies below 2^-40 of its row's largest magnitude is lost; all other forms split exactly.  K % 16 == 0; the workspace is scratch (to be taken as overwritten by every call). */
+ * the rest is a tiled Gemm on the bf16 matrix cores, 64 activation rows x 64, 128 or 192 weight rows per workgroup (prefill, attention
+ * projections).  All forms split exactly; products are added up 32 or 64 at a time before their scale, which holds magnitudes up to 2^114.  K % 16 == 0; the workspace is scratch (to be taken as overwritten by every call). */
 int ncnnhip_gemm_blockquant_packed_rows_workspace_bytes(int M, int K, size_t* bytes);
 int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int M, int N, int K, const uint8_t* packed_w_dev,
                                         const float* packed_descale_dev, int bits, int block, const float* in_scales_dev,

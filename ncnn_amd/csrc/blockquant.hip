@@ -1282,12 +1282,13 @@ __global__ __launch_bounds__(256) void blockquant_split_activations_kernel(const
 // A stage: 3 planes x 64 rows x 128 bytes, then the workgroup's 8 weight tiles (1 KB apiece reserved) and their descales
 // (128 bytes apiece).  Every wavefront issues exactly ten loads per stage (6 of activations, its 2 tiles, their 2 descale
 // rows; beyond the last step it loads the last step again into a stage nobody reads any more), which is what the wait counts.
-template<int BITS, int STAGES, int RW>
+template<int BITS, bool HALVES, int STAGES, int RW>
 __global__ __launch_bounds__(256) void blockquant_rows_bf16x3_kernel(const unsigned short* __restrict__ planes, int Mp, int Kp, int M, int N, int kblocks,
                                                                       int ntiles, const unsigned char* __restrict__ wpk, const float4* __restrict__ dpk, int split,
                                                                       const float* __restrict__ c, int bt, float alpha, float beta, float* __restrict__ out,
                                                                       size_t out_stride)
 {
+    static_assert(HALVES || BITS == 8, "4- and 6-bit fields come in the halves layout");
     constexpr int LOADS = 6 + 2 * RW; // per wavefront and stage
     static_assert(STAGES >= 2 && (STAGES - 2) * LOADS < 64, "the vmcnt field counts to 63");
     static_assert(RW >= 1 && RW <= 4, "one to four tiles of 16 weight rows per wavefront");
@@ -1301,7 +1302,7 @@ __global__ __launch_bounds__(256) void blockquant_rows_bf16x3_kernel(const unsig
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m = lane & 15, kg = lane >> 4;
     const int row0 = blockIdx.y * 64;
-    const int dper = 4 << split;
+    const int dper = HALVES ? 4 << split : 4;
 
     // the wavefront's RW tiles (a tile beyond the last reads the last one again and stores nothing)
     const unsigned char* wsrc[RW];
@@ -1353,8 +1354,8 @@ __global__ __launch_bounds__(256) void blockquant_rows_bf16x3_kernel(const unsig
 
     // operand reads: row cw * 16 + m, chunk positions of the lane's two K groups (the swizzle does not depend on cw)
     const int sw = (m >> 1) & 7;
-    const int rd_a = m * 128 + ((kg ^ sw) << 4);
-    const int rd_b = m * 128 + (((4 + kg) ^ sw) << 4);
+    const int rd_a = m * 128 + (((HALVES ? kg : 2 * kg) ^ sw) << 4);
+    const int rd_b = m * 128 + (((HALVES ? 4 + kg : 2 * kg + 1) ^ sw) << 4);
     const int last = kblocks - 1;
     const unsigned lds_base = (unsigned)(uintptr_t)(BQ_AS3 unsigned char*)lds_rows;
 
@@ -1467,7 +1468,10 @@ __global__ __launch_bounds__(256) void blockquant_rows_bf16x3_kernel(const unsig
 #pragma unroll
                 for (int rw = 0; rw < RW; rw++)
                 {
-                    t1[rw] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[rw], yb[set][pn].h, t1[rw], 0, 0, 0);
+                    if (HALVES)
+                        t1[rw] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[rw], yb[set][pn].h, t1[rw], 0, 0, 0);
+                    else
+                        t0[rw] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[rw], yb[set][pn].h, t0[rw], 0, 0, 0);
                 }
             }
 #pragma unroll
@@ -1478,7 +1482,10 @@ __global__ __launch_bounds__(256) void blockquant_rows_bf16x3_kernel(const unsig
 #pragma unroll
                 for (int r = 0; r < 4; r++)
                 {
-                    acc[rw][cw][r] = fmaf(t1[rw][r], db[r], fmaf(t0[rw][r], da[r], acc[rw][cw][r]));
+                    if (HALVES)
+                        acc[rw][cw][r] = fmaf(t1[rw][r], db[r], fmaf(t0[rw][r], da[r], acc[rw][cw][r]));
+                    else
+                        acc[rw][cw][r] = fmaf(t0[rw][r], da[r], acc[rw][cw][r]);
                 }
             }
         }
@@ -1517,12 +1524,13 @@ __global__ __launch_bounds__(256) void blockquant_rows_bf16x3_kernel(const unsig
 // soon as its operands are in registers, one and a half steps before they are due.
 // Bound by the issue slots of the conversions and the clock (1.6 to 2.1 GHz under this load); us with the split pass, 8 bits,
 // kernel above -> this one: 256 x 4096 x 4096 64 -> 50, 100 x 4096 x 11008 135 -> 93, 512 x 1024 x 1024 22.7 -> 19.3.
-template<int BITS>
+template<int BITS, bool HALVES>
 __global__ __launch_bounds__(512) void blockquant_rows_ksplit_bf16x3_kernel(const unsigned short* __restrict__ planes, int Mp, int Kp, int M, int N, int kblocks,
                                                                       int ntiles, const unsigned char* __restrict__ wpk, const float4* __restrict__ dpk, int split,
                                                                       const float* __restrict__ c, int bt, float alpha, float beta, float* __restrict__ out,
                                                                       size_t out_stride)
 {
+    static_assert(HALVES || BITS == 8, "4- and 6-bit fields come in the halves layout");
     constexpr int STAGES = 2;
     constexpr int RW = 2;              // weight tiles a wavefront multiplies
     constexpr int RWL = RW / 2;        // and fetches (each is multiplied by two)
@@ -1540,7 +1548,7 @@ __global__ __launch_bounds__(512) void blockquant_rows_ksplit_bf16x3_kernel(cons
     const int wa = wave & 1, ww = wave >> 1; // the wavefront's half of the activation rows and of the weight tiles
     const int m = lane & 15, kg = lane >> 4;
     const int row0 = blockIdx.y * 64;
-    const int dper = 4 << split;
+    const int dper = HALVES ? 4 << split : 4;
 
     // the RWL tiles the wavefront fetches (a tile beyond the last reads the last one again and stores nothing)
     const unsigned char* wsrc[RWL];
@@ -1592,8 +1600,8 @@ __global__ __launch_bounds__(512) void blockquant_rows_ksplit_bf16x3_kernel(cons
 
     // operand reads: row (wa * CW + cw) * 16 + m, chunk positions of the lane's two K groups (the swizzle does not depend on cw)
     const int sw = (m >> 1) & 7;
-    const int rd_a = (wa * CW * 16 + m) * 128 + ((kg ^ sw) << 4);
-    const int rd_b = (wa * CW * 16 + m) * 128 + (((4 + kg) ^ sw) << 4);
+    const int rd_a = (wa * CW * 16 + m) * 128 + (((HALVES ? kg : 2 * kg) ^ sw) << 4);
+    const int rd_b = (wa * CW * 16 + m) * 128 + (((HALVES ? 4 + kg : 2 * kg + 1) ^ sw) << 4);
     // K steps of this group of wavefronts; every wavefront of the workgroup goes through the same number of iterations
     const int iterations = (kblocks + 1) / 2;
     const int first = group * iterations;
@@ -1637,7 +1645,7 @@ __global__ __launch_bounds__(512) void blockquant_rows_ksplit_bf16x3_kernel(cons
                     asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(wlo[rw]) : "v"(wl), "n"(rw * 1024));
                 if (BITS == 6) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(whi[rw]) : "v"(wl3), "n"(rw * 1024));
                 asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dq0[rw]) : "v"(dl), "n"(rw * 128));
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dq1[rw]) : "v"(dl2), "n"(rw * 128));
+                if (HALVES) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dq1[rw]) : "v"(dl2), "n"(rw * 128));
             }
         }
         // the six operand fragments of a 16-row group (3 planes x 2 halves of the step)
@@ -1691,7 +1699,7 @@ __global__ __launch_bounds__(512) void blockquant_rows_ksplit_bf16x3_kernel(cons
         for (int rw = 0; rw < RW; rw++)
         {
             asm volatile("" : "+v"(fa[rw]), "+v"(dq0[rw])); // converted on this side of the barrier
-            asm volatile("" : "+v"(dq1[rw]));
+            if constexpr (HALVES) asm volatile("" : "+v"(dq1[rw]));
             if constexpr (BITS != 8) asm volatile("" : "+v"(fb[rw]));
         }
         __builtin_amdgcn_s_barrier(); // everybody of this group has read the stage; the other group reads and converts now
@@ -1724,7 +1732,10 @@ __global__ __launch_bounds__(512) void blockquant_rows_ksplit_bf16x3_kernel(cons
 #pragma unroll
                 for (int rw = 0; rw < RW; rw++)
                 {
-                    t1[rw] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[rw], yb[cw][pn].h, t1[rw], 0, 0, 0);
+                    if (HALVES)
+                        t1[rw] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[rw], yb[cw][pn].h, t1[rw], 0, 0, 0);
+                    else
+                        t0[rw] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[rw], yb[cw][pn].h, t0[rw], 0, 0, 0);
                 }
 #pragma unroll
             for (int rw = 0; rw < RW; rw++)
@@ -1734,7 +1745,10 @@ __global__ __launch_bounds__(512) void blockquant_rows_ksplit_bf16x3_kernel(cons
 #pragma unroll
                 for (int r = 0; r < 4; r++)
                 {
-                    acc[rw][cw][r] = fmaf(t1[rw][r], db[r], fmaf(t0[rw][r], da[r], acc[rw][cw][r]));
+                    if (HALVES)
+                        acc[rw][cw][r] = fmaf(t1[rw][r], db[r], fmaf(t0[rw][r], da[r], acc[rw][cw][r]));
+                    else
+                        acc[rw][cw][r] = fmaf(t0[rw][r], da[r], acc[rw][cw][r]);
                 }
             }
         }
@@ -2441,28 +2455,30 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
     hipStream_t st = as_stream(stream);
     const float4* dpk = reinterpret_cast<const float4*>(packed_descale_dev);
     const int split = block == 32 ? 1 : 0;
-    // One launch without the split pass, where that is quicker than the tiled kernels after it.  Those of blocks of 32 take about 9.5 us + K / 1024 x 8.25
-    // us in one round of 64 x 64 tiles on 256 units; beyond, 15 in one of 512, then 18 per 512 tiles (18 shapes, 97 to 482 rows); 5 % less here, so
-    // that it stays where the two are close.  In larger blocks the kernel with 64 x 128 tiles takes 14 us + K / 1024 x 6.4 or a little more for every round of 256: of
-    // 204 shapes (24 to 1500 rows, N and K 512 to 11008) this line picks the slower one in none by more than 4 %.  us, rows kernel / tiles of 64 x 128: 42 x 6880 x 5312
-    // 33.9 41.6, 236 x 1472 x 3840 23.5 35, 803 x 1600 x 4352 117 44, 469 x 832 x 4416 34.8 42.6, 70 x 6512 x 1728 26.0 23.1, 65 x 5904 x 1792 19.1 21.8.
-    // Its 16-byte loads need aligned rows.
+    // One launch without the split pass, where that is quicker than the tiled kernels after it, which take about 9.5 us + K / 1024 x 8.25
+    // us in one round of 64 x 64 tiles on 256 units; beyond, in blocks of 32, 15 in one of 512, then 18 per 512 tiles (18 shapes, 97 to 482
+    // rows), in larger blocks 11 us + K / 1024 x 11.5 for every round of 256 64 x 128 tiles; 5 % less here, so that it stays where the two are
+    // close.  us before (the
+    // better of the two below) / here: 8 bits, 4096 x 4096 16 rows 12.4 / 10.7, 32 20.1 / 12.9, 64 34 / 17.5, 128 41 / 30; 11008 x 4096 16
+    // rows 26.5 / 16.6, 32 46 / 26.5; 4096 x 11008 64 rows 84 / 40, 128 93 / 66; 4 bits, 1730 x 1472 186 rows 21.4 / 12.0, 734 x 6016 477
+    // rows 61 / 30.  Its 16-byte loads need aligned rows.
     const bool aligned = al16(a_dev) && a_stride % 4 == 0 && (!in_scales_dev || al16(in_scales_dev));
     const long long tiles64 = (long long)((ntiles + 3) / 4) * (Mp / 64);
     const double rounds = (double)(((long long)((ntiles + 7) / 8) * (Mp / 64) + 255) / 256); // of 64 x 128 tiles
-    const double tiled = block != 32 ? 14.0 + K / 1024.0 * 6.4 * rounds : 9.0 + K / 1024.0 * (tiles64 <= 256 ? 7.8 : tiles64 <= 512 ? 14.2 : 17.0 * tiles64 / 512.0);
     int mg, rt;
-    if (aligned && blockquant_rows_f32_us(M, K, &N, 1, &mg, &rt) < tiled)
+    if (aligned
+        && blockquant_rows_f32_us(M, K, &N, 1, &mg, &rt)
+               < 9.0 + K / 1024.0 * (tiles64 <= 256 ? 7.8 : block != 32 ? 11.0 * rounds : tiles64 <= 512 ? 14.2 : 17.0 * tiles64 / 512.0))
         return launch_blockquant_rows_f32(a_dev, a_stride, M, K, bits, block, in_scales_dev, one_matrix(N, packed_w_dev, dpk, c_dev, bt, alpha, beta, out_dev, out_stride),
                                           st);
     // Which form (rows off 16 bytes, mostly): the 16-row passes, all in one launch, take about 5 us and a pass's weights at 2.35 million a us, 3.2 up
     // to K = 2048 and less where the last of its rounds of 64 K steps is partly empty, whatever their bits, which the conversions decide; a round of the
-    // tiled kernel for blocks of 32 7 us + K / 1024 x 7.8 whatever the row count.  us, passes / that kernel at 8 bits: 4096 x 1024 97 rows 15.3 17.0; 8192 x 2048 48
+    // tiled kernel 7 us + K / 1024 x 7.8 whatever the row count.  us, passes / tiled at 8 bits: 4096 x 1024 97 rows 15.3 17.0; 8192 x 2048 48
     // rows 19.7 24.2, 97 rows 42.5 26.2; 4096 x 4096 64 rows 33.8 39.9, 97 rows 56 41; 4992 x 4992 20 rows 36.8 45.4, 48 rows 49 46; 11008 x
     // 4096 12 rows 25 38, 20 rows 44 39; 4096 x 11008 64 rows 84 89.  (By bytes, as before, 97 rows of 4992 x 4992 at 4 bits took 112 us for 51.)
     const int passes16 = (M + 15) / 16;
     const double weights = (double)N * (double)K / 1.0e6 * (kblocks <= 64 ? 1.0 : (kblocks + 63) / 64 * 64.0 / kblocks);
-    if (M <= 128 && 5.0 + passes16 * weights / (K <= 2048 ? 3.2 : 2.35) <= (block == 32 ? 7.0 + K / 1024.0 * 7.8 : 14.0 + K / 1024.0 * 6.4))
+    if (M <= 128 && 5.0 + passes16 * weights / (K <= 2048 ? 3.2 : 2.35) <= 7.0 + K / 1024.0 * 7.8)
     {
         // fewer rows than the tiled kernel can spread over the chip: 16 rows per pass in the weight-streaming shape
         // (the fragments of a pass take kblocks * 6 KB of the workspace: all passes together no more than the planes it was sized for)
@@ -2488,10 +2504,19 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
 #undef ROWS16
         return launch_status("blockquant_rows16_bf16x3_kernel");
     }
-    // Blocks of 64 and 128 (one scale a step): the kernel with 64 x 128 tiles.  Before the activations were two fp16 numbers there it was left out where there is at most one 64 x 64
-    // tile per unit, and for 8 bits at just over two rounds; us, the two kernels below / here, of 204 shapes: 236 x 1472 x 4032 43.3 38.8, 129 x 3520 x 3520 40.2
-    // 34.9, 288 x 2496 x 9024 79.1 65.4, 46 x 1888 x 9152 84.0 64.8, 1500 x 3072 x 1024 52.5 49.4; below K = 900 the other way by up to 1.5 us, where the rows kernel takes most calls.
-    if (block != 32)
+    // More than one 64 x 64 tile per compute unit: the kernel with 64 x 128 tiles (one scale a step: not blocks of 32).  It is quicker there (1.02 to
+    // 1.44 times, 120 shapes of 65 to 1500 rows, K 512 to 11008; of 1600 to 24000 rows, N 192 to 4096, 191 shapes: 1.05 in the median, 14 of them below 0.98,
+    // where N is at most 1024 or K at most 512: 9000 x 192 x 512 27.2 31.7, 24000 x 256 x 512 57.4 64.6), with one exception: 8-bit fields in just over two
+    // rounds of it where the kernel below has one round of 64 x 192 tiles, two to a unit.  There the two are close, and which is the quicker depends on
+    // what runs around them: among a self-attention layer's other kernels (1500 tokens, 1024 channels: 1500 x 3072 x 1024) the layer takes 150 us with the one below
+    // and 156 with the one here.  Back to back, below / here: N 512 to 1024, K 512 to 6144 2 to 12 % less below (5504 x 768 x 4096 168 191), at K
+    // 128 and 256 within 4 % either way; N 1536 up to 5 % less below at K 768 to 2048 (3500 rows, K 1024 58.9 61.3), 2 to 10 % more at others; N
+    // 2048 to 11008, K 128 to 16384 from 2 % less below to 10 % more, 3 in the median (1500 x 3072 x 1024 54.6 51.9, 1024 x 5120 x 8192 278 262).
+    // With fewer tiles the kernel below that splits K over two groups puts more units to work (128 tiles of 64 x 128, 256 x 4096 x
+    // 4096: 45.7 us against 47.7).
+    const long long tiles128 = (long long)((ntiles + 7) / 8) * (Mp / 64), tiles192 = (long long)((ntiles + 11) / 12) * (Mp / 64);
+    const bool one_round = !halves && tiles128 > 512 && tiles192 <= 448;
+    if (block != 32 && tiles64 > 256 && !one_round)
         return launch_blockquant_tiles(a_dev, a_stride, M, N, K, bits, packed_w_dev, dpk, in_scales_dev, c_dev, bt, alpha, beta, out_dev, out_stride, workspace_dev, st);
     unsigned short* planes = static_cast<unsigned short*>(workspace_dev);
     const size_t vectors = (size_t)Mp * (Kp / 8);
@@ -2536,7 +2561,7 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
     // Up to one 64 x 64 tile per compute unit, the kernel that splits K inside the workgroup: 4 bits, 256 x 4096 x 4096 59 -> 53 us.
     const bool ksplit = tiles64 <= 256;
     // (a ring of four stages where a workgroup has its compute unit to itself measured the same as two: 57.6 against 57.8 us at 128 x 4096 x 4096)
-    const int wg_tiles = ksplit ? 4 : 4 * rw_tiles;
+    const int wg_tiles = ksplit ? 4 : 4 * (one_round ? 3 : rw_tiles);
     const dim3 grid((ntiles + wg_tiles - 1) / wg_tiles, Mp / 64);
 #define ROWS_LAUNCH(KERNEL_, THREADS_, LDS_)                                                                                                                        \
     do                                                                                                                                                             \
@@ -2552,22 +2577,26 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
         }                                                                                                                                                          \
         hipLaunchKernelGGL(kernel, grid, dim3(THREADS_), LDS_, st, planes, Mp, Kp, M, N, kblocks, ntiles, packed_w_dev, dpk, split, c_dev, bt, alpha, beta, out_dev, out_stride); \
     } while (0)
-#define ROWS_RW(BITS_, RW_) \
-    ROWS_LAUNCH((blockquant_rows_bf16x3_kernel<BITS_, 2, RW_>), 256, (size_t)2 * (3 * 64 * 128 + 4 * (RW_) * 1024 + 4 * (RW_) * 128))
-#define ROWS_KS(BITS_) ROWS_LAUNCH((blockquant_rows_ksplit_bf16x3_kernel<BITS_>), 512, (size_t)4 * (3 * 64 * 128 + 4 * 1024 + 4 * 128))
-#define ROWS(BITS_)            \
-    do                         \
-    {                          \
-        if (ksplit)            \
-            ROWS_KS(BITS_);    \
-        else if (rw_tiles == 1) \
-            ROWS_RW(BITS_, 1); \
-        else if (rw_tiles == 3) \
-            ROWS_RW(BITS_, 3); \
-        else                   \
-            ROWS_RW(BITS_, 2); \
+#define ROWS_RW(BITS_, HALVES_, RW_) \
+    ROWS_LAUNCH((blockquant_rows_bf16x3_kernel<BITS_, HALVES_, 2, RW_>), 256, (size_t)2 * (3 * 64 * 128 + 4 * (RW_) * 1024 + 4 * (RW_) * 128))
+#define ROWS_KS(BITS_, HALVES_) ROWS_LAUNCH((blockquant_rows_ksplit_bf16x3_kernel<BITS_, HALVES_>), 512, (size_t)4 * (3 * 64 * 128 + 4 * 1024 + 4 * 128))
+#define ROWS(BITS_)                  \
+    do                               \
+    {                                \
+        if (ksplit)                  \
+            ROWS_KS(BITS_, true);    \
+        else if (rw_tiles == 1)      \
+            ROWS_RW(BITS_, true, 1); \
+        else if (rw_tiles == 3)      \
+            ROWS_RW(BITS_, true, 3); \
+        else                         \
+            ROWS_RW(BITS_, true, 2); \
     } while (0)
-    if (bits == 8)
+    if (!halves && ksplit)
+        ROWS_KS(8, false);
+    else if (!halves) // (one_round)
+        ROWS_RW(8, false, 3);
+    else if (bits == 8)
         ROWS(8);
     else if (bits == 6)
         ROWS(6);

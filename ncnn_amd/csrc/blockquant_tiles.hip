@@ -1,21 +1,16 @@
 // Block-quantised Gemm on many rows of fp32 activations (prefill, attention projections), weights in blocks of 64 or 128: the activations
-// are split into two fp16 numbers by a pass of its own, then a workgroup multiplies 64 of their rows with 128 weight rows on
-// v_mfma_f32_32x32x16_f16.
-//
-// Two fp16 numbers hold 23 bits of an activation, one less than fp32, and make two products of what were three with the exact split into bf16; with a third fewer
-// roundings in the sums the error against 64 bits is smaller than it was: N(0, 1) rows, K 1024 1.05e-7 for 1.09e-7, 4096 1.22 for 1.26, 11008 1.54 for 1.57, 12800 in
-// blocks of 128 1.61 for 1.64; one column in 97 300 times the others 1.40 for 1.39.  (The low parts of a step first: 1.20 at K = 4096, 1.59 at 11008.)
+// are split into three bf16 numbers by a pass of its own, then a workgroup multiplies 64 of their rows with 128 weight rows on
+// v_mfma_f32_32x32x16_bf16.
 //
 // A wavefront multiplies 64 activation rows with 64 weight rows and a workgroup holds four groups of two, each with a quarter of K: a weight
-// is converted to fp16 once for 64 rows (with 32, as blockquant.hip's kernels have it, the vector unit is as busy as the matrix cores), and
+// is converted to bf16 once for 64 rows (with 32, as blockquant.hip's kernels have it, the vector unit is as busy as the matrix cores), and
 // 256 tiles of 64 x 128, a prefill of 512 rows of 4096, still put two wavefronts on every SIMD.
-// Bound by the matrix cores' issue at the 1.79 GHz they sustain on all units, and by the fills: half a K step is 571 ns of products for the two wavefronts of a SIMD and takes
-// 921; without the fills (48 KB a unit, 13 TB/s on all of them) 700, without the vector instructions 770.  Around the 30 us of steps that 64 x 128 results of K = 4096 take
-// stand 0.5 of first loads, 1.3 of the groups' exchange and 1.5 of results.  us with the split pass, 8 bits in blocks of 64, three bf16 numbers -> here: 512 x 4096 x 4096
-// 60.7 -> 46.6, 512 x 4096 x 11008 133 -> 101, 512 x 11008 x 4096 145 -> 114, 1500 x 3072 x 1024 52.9 -> 43.9, 1500 x 1024 x 1024 24.1 -> 21.8; 1024 x 4096 x 4096 at 6
-// bits 111 -> 86.  (One barrier a stage and operands read a stage ahead, between the products, instead of two wavefronts that read and multiply in turn: 49.8, as the
-// fills are what it waits for.  Weights and loads all before the products, activations requested half a stage later, two groups and two workgroups to a
-// unit: all slower with three products.)
+// Bound by the matrix cores' issue and the clock, 1.8 GHz on all units: half a K step takes a wavefront about 1100 cycles of multiplying for
+// 768 of matrix-core time (the rest: nine loads, 14 of their cycles each not hidden, and the conversions), and its neighbour reads meanwhile.
+// us with the split pass (7 at 512 x 4096), 8 bits in blocks of 64, blockquant.hip's kernels -> here: 512 x 4096 x 4096 78 -> 65, 512 x 4096 x 11008
+// 178 -> 139, 512 x 11008 x 4096 162 -> 150, 333 x 4096 x 4096 66 -> 50, 1500 x 1024 x 1024 29.5 -> 24.6; 4 bits 512 x 4096 x 4096 87 -> 60.
+// Error against 64 bits 1.26e-7 for 1.44e-7.  (Weights and loads all before the products: 70; activations requested half a stage later, where the
+// wavefront does not multiply: 74; two groups and two workgroups to a unit: 68, and 4 % quicker only on many rounds.)
 #include <atomic>
 
 #include "blockquant.h"
@@ -29,129 +24,72 @@ namespace ncnnhip {
 typedef float v16f_bq __attribute__((ext_vector_type(16)));
 
 // ---- the activations in operand order ----
-// A row, times the power of two that takes its largest finite value into [2^14, 2^15), becomes hi + lo in fp16: 23 bits of a value of 24, and of values below 2^-17 of
-// the row's largest what lies above 2^-40 of it.  The row's factor back goes to `back`; infinities and NaNs travel in hi alone.
 // A stage is half a K step: of the 16-byte pieces the packed weights keep for four K groups (two chunks of 8 each) those of groups 2 h and
 // 2 h + 1.  [row block of 64][K step][h] [32-row group][chunk c of the piece][part] 64 lanes x 16 bytes: lane = row l % 32, K group 2 h + l / 32.
-// Rows beyond M and K beyond the last are zeros.  One workgroup: SPLIT_ROWS whole rows, so that their factors are known, and as many workgroups as that gives: 512 rows
-// are 256 of them, one to a unit (bound by memory latency: each wavefront has its loads in flight once).  What it writes are 32-byte pieces; the four workgroups of a
-// 128-byte line run on one die, so that its L2 puts the line together.
-// A wavefront, of 16 or as many as there are spans of 256 columns, takes the spans in turn and keeps the first KEEP of its own in registers between the two passes.
-// us, a decoder layer of 4096 / 11008, seven Gemms and as many of these, workgroups of four rows / here: 150 rows 367 / 354, 512 514.6 / 510.3; of 1024 / 2816, 1500 rows
-// 213.1 / 209.9; of 2048 / 5504, 700 rows 257.8 / 256.5 (258.6 with four spans kept where there are no more than two).
-constexpr int SPLIT_ROWS = 2, SPLIT_LINE = 8 / SPLIT_ROWS, SPLIT_SPAN = 512 / SPLIT_ROWS, SPLIT_WAVES = 16; // LINE: workgroups that write the same 128-byte lines
-template<bool HALVES, int KEEP>
-__global__ __launch_bounds__(64 * SPLIT_WAVES) void blockquant_split_tiles_kernel(const float* __restrict__ a, size_t a_stride, int M, int K, int kblocks,
-                                                                                  const float* __restrict__ in_scales, uint4* __restrict__ frags, float* __restrict__ back)
+// Rows beyond M and K beyond the last are zeros.  One workgroup: 64 rows x two K steps.
+template<bool HALVES>
+__global__ __launch_bounds__(256) void blockquant_split_tiles_kernel(const float* __restrict__ a, size_t a_stride, int M, int K, int kblocks,
+                                                                     const float* __restrict__ in_scales, uint4* __restrict__ frags)
 {
-    __shared__ unsigned tops[SPLIT_WAVES][SPLIT_ROWS];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane % SPLIT_ROWS;
-    const int turn = (int)blockIdx.x % (8 * SPLIT_LINE), share = (int)blockIdx.x - turn + (turn & 7) * SPLIT_LINE + (turn >> 3); // (the grid is whole turns)
-    const int row = share * SPLIT_ROWS + r, waves = blockDim.x >> 6;
-    const auto load = [&](int span, float (&x)[8]) {
-        const int k = span * SPLIT_SPAN + lane / SPLIT_ROWS * 8;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, hh = lane >> 5;
+    const int h = wave >> 1, c = wave & 1;
+    const int chunk = HALVES ? 2 * h + hh + 4 * c : 2 * (2 * h + hh) + c;
+    float x[4][8];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+    {
+        const int kb = blockIdx.x * 2 + (u >> 1), row = blockIdx.y * 64 + (u & 1) * 32 + l32, k = kb * 64 + chunk * 8;
         const bool inside = row < M && k < K; // K % 16 == 0: a chunk of 8 is all in or all out
         const float* p = a + (inside ? (size_t)row * a_stride + k : (size_t)0);
 #pragma unroll
-        for (int j = 0; j < 8; j++) x[j] = p[j]; // a valid address either way (K >= 16)
+        for (int j = 0; j < 8; j++) x[u][j] = p[j]; // a valid address either way (K >= 16)
         if (!inside)
         {
 #pragma unroll
-            for (int j = 0; j < 8; j++) x[j] = 0.f;
+            for (int j = 0; j < 8; j++) x[u][j] = 0.f;
         }
         else if (in_scales)
         {
 #pragma unroll
-            for (int j = 0; j < 8; j++) x[j] = mul_rn(x[j], in_scales[k + j]);
+            for (int j = 0; j < 8; j++) x[u][j] = mul_rn(x[u][j], in_scales[k + j]);
         }
-    };
-    const int spans = (kblocks * 64 + SPLIT_SPAN - 1) / SPLIT_SPAN;
-    unsigned top = 0; // the bits of the largest finite magnitude
-    const auto look = [&](const float (&x)[8]) {
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-        {
-            const unsigned b = __float_as_uint(x[j]) & 0x7FFFFFFFu;
-            if (b < 0x7F800000u && b > top) top = b;
-        }
-    };
-    float kept[KEEP][8];
-#pragma unroll
-    for (int u = 0; u < KEEP; u++) load(wave + u * waves, kept[u]);
-#pragma unroll
-    for (int u = 0; u < KEEP; u++) look(kept[u]);
-    for (int span = wave + KEEP * waves; span < spans; span += waves)
-    {
-        float x[8];
-        load(span, x);
-        look(x);
     }
 #pragma unroll
-    for (int d = SPLIT_ROWS; d < 64; d *= 2)
+    for (int u = 0; u < 4; u++)
     {
-        const unsigned o = (unsigned)__shfl_xor((int)top, d);
-        if (o > top) top = o;
-    }
-    if (lane < SPLIT_ROWS) tops[wave][lane] = top;
-    __syncthreads();
-    for (int w = 0; w < waves; w++)
-        if (tops[w][r] > top) top = tops[w][r];
-    int shift = top ? 14 + 127 - (int)(top >> 23) : 0;
-    if (shift > 126) shift = 126; // both factors are normal numbers
-    const float factor = __uint_as_float((unsigned)(127 + shift) << 23);
-    if (wave == 0 && lane < SPLIT_ROWS) back[row] = __uint_as_float((unsigned)(127 - shift) << 23);
-
-    const auto store = [&](int span, const float (&x)[8]) {
-        const int chunk_of_row = span * (SPLIT_SPAN / 8) + lane / SPLIT_ROWS, kb = chunk_of_row >> 3, chunk = chunk_of_row & 7;
-        if (kb >= kblocks) return;
-        // chunk = HALVES ? 2 h + hh + 4 c : 2 (2 h + hh) + c
-        const int c = HALVES ? chunk >> 2 : chunk & 1, hh = HALVES ? chunk & 1 : (chunk >> 1) & 1, h = HALVES ? (chunk >> 1) & 1 : chunk >> 2;
-        union
-        {
-            v8h h8;
-            uint4 u;
-        } hi, lo;
+        const int kb = blockIdx.x * 2 + (u >> 1);
+        if (kb >= kblocks) break;
+        unsigned pl[3][4];
 #pragma unroll
-        for (int j = 0; j < 8; j++)
+        for (int e = 0; e < 4; e++)
         {
-            const float v = x[j] * factor;
-            hi.h8[j] = (_Float16)v;
-            const bool finite = (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u;
-            lo.h8[j] = (_Float16)(finite ? v - (float)hi.h8[j] : 0.f);
+            unsigned part[2][3];
+#pragma unroll
+            for (int o = 0; o < 2; o++) split_bf16x3(x[u][2 * e + o], part[o][0], part[o][1], part[o][2]);
+#pragma unroll
+            for (int p = 0; p < 3; p++) pl[p][e] = (part[0][p] >> 16) | part[1][p];
         }
-        uint4* to = frags + ((((size_t)(row >> 6) * kblocks + kb) * 2 + h) * 8 + (((row >> 5) & 1) * 2 + c) * 2) * 64 + hh * 32 + (row & 31);
-        to[0] = hi.u;
-        to[64] = lo.u;
-    };
+        uint4* to = frags + ((((size_t)blockIdx.y * kblocks + kb) * 2 + h) * 12 + ((u & 1) * 2 + c) * 3) * 64 + lane;
 #pragma unroll
-    for (int u = 0; u < KEEP; u++) store(wave + u * waves, kept[u]);
-    for (int span = wave + KEEP * waves; span < spans; span += waves)
-    {
-        float x[8];
-        load(span, x);
-        store(span, x);
+        for (int p = 0; p < 3; p++) to[p * 64] = make_uint4(pl[p][0], pl[p][1], pl[p][2], pl[p][3]);
     }
 }
 
-constexpr int TILES_STAGE = 8 * 1024; // bytes of activations
+constexpr int TILES_STAGE = 12 * 1024; // bytes of activations
 constexpr int tiles_weight_bytes(int bits) { return 8 * 64 * bits + 512; }
 constexpr int KG = 4; // groups of two wavefronts
-constexpr int tiles_lds_bytes(int bits) // the rings, or later the sums
-{
-    const int rings = KG * (2 * TILES_STAGE + 3 * tiles_weight_bytes(bits)), sums = (KG - 1) * KG * 2 * 4096;
-    return rings > sums ? rings : sums;
-}
+constexpr int tiles_lds_bytes(int bits) { return KG * (2 * TILES_STAGE + 3 * tiles_weight_bytes(bits)); } // (more than the 96 KB the sums take later)
 
 // Each group has a ring of its own for two stages of activations (12 KB, read by both wavefronts) and three of weights and descales (read by
 // the wavefront that fetched them, a stage ahead, and converted while it multiplies), filled straight from global memory as soon as
 // the operands are in registers.  The last two groups run half a stage behind the first two, their neighbours on the same SIMDs: one
 // reads while the other multiplies.
 template<int BITS>
-__global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4* __restrict__ frags, const float* __restrict__ back, int M, int N, int kblocks, int ntiles,
+__global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4* __restrict__ frags, int M, int N, int kblocks, int ntiles,
                                                                    const unsigned char* __restrict__ wpk, const float4* __restrict__ dpk, const float* __restrict__ c,
                                                                    int bt, float alpha, float beta, float* __restrict__ out, size_t out_stride)
 {
-    constexpr int LOADS = 4 + (BITS == 4 ? 1 : BITS == 8 ? 2 : 3) + 1; // per wavefront and stage
+    constexpr int LOADS = 6 + (BITS == 4 ? 1 : BITS == 8 ? 2 : 3) + 1; // per wavefront and stage
     constexpr int HI_OFF = 2048, D_OFF = 8 * 64 * BITS, WSTAGE = tiles_weight_bytes(BITS), STEP_BYTES = 128 * BITS;
     constexpr int GROUP = 2 * TILES_STAGE + 3 * WSTAGE; // two slots of activations, three of weights
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds_tiles[];
@@ -164,7 +102,7 @@ __global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4*
     // last reads the last one again and stores nothing); uniform base + 32-bit offset of the lane
     const int tile0 = (int)blockIdx.x * 8 + ww * 4, tile_first = tile0 < ntiles ? tile0 : ntiles - 1;
     const auto tile_offset = [&](int t) { return (unsigned)((tile_first + t < ntiles ? tile_first + t : ntiles - 1) - tile_first) * (unsigned)kblocks; };
-    const char* const abase = reinterpret_cast<const char*>(frags + ((size_t)blockIdx.y * kblocks * 16 + ww * 4) * 64);
+    const char* const abase = reinterpret_cast<const char*>(frags + ((size_t)blockIdx.y * kblocks * 24 + ww * 6) * 64);
     const char* const wbase = reinterpret_cast<const char*>(wpk) + (size_t)tile_first * kblocks * STEP_BYTES;
     const char* const dbase = reinterpret_cast<const char*>(dpk) + (size_t)tile_first * kblocks * 64;
     unsigned woff[3];
@@ -185,16 +123,16 @@ __global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4*
     const unsigned doff = tile_offset(lane >> 4) * 64 + (lane & 15) * 4;
     const int iterations = (kblocks + KG - 1) / KG, first = group * iterations, last = kblocks - 1;
     unsigned char* const mine = lds_tiles + group * GROUP;
-    // load i of a stage: 4 of activations (of half h of K step `at`; h is also their slot), the others of weights (of a later stage)
+    // load i of a stage: 6 of activations (of half h of K step `at`; h is also their slot), the others of weights (of a later stage)
     const auto load_activations = [&](int at, int h, int i) {
         const char* from = abase + (size_t)((at < last ? at : last) * 2 + h) * TILES_STAGE;
-        __builtin_amdgcn_global_load_lds((const AS1 void*)(from + (unsigned)(lane * 16 + i * 1024)), (AS3 void*)(mine + h * TILES_STAGE + (ww * 4 + i) * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const AS1 void*)(from + (unsigned)(lane * 16 + i * 1024)), (AS3 void*)(mine + h * TILES_STAGE + (ww * 6 + i) * 1024), 16, 0, 0);
     };
     const auto load_weights = [&](int at, int h, int slot, int i) {
         const int kb = at < last ? at : last;
         unsigned char* st = mine + 2 * TILES_STAGE + slot * WSTAGE;
         const char* from = wbase + (size_t)kb * STEP_BYTES + h * (BITS == 8 ? 512 : 256);
-        if (i == LOADS - 5)
+        if (i == LOADS - 7)
             __builtin_amdgcn_global_load_lds((const AS1 void*)(dbase + (size_t)kb * 64 + doff), (AS3 void*)(st + D_OFF + ww * 256), 4, 0, 0);
         else if (BITS == 8)
             __builtin_amdgcn_global_load_lds((const AS1 void*)(from + woff[i]), (AS3 void*)(st + (ww * 2 + i) * 1024), 16, 0, 0);
@@ -205,11 +143,11 @@ __global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4*
     };
     const auto issue_activations = [&](int at, int h) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) load_activations(at, h, i);
+        for (int i = 0; i < 6; i++) load_activations(at, h, i);
     };
     const auto issue_weights = [&](int at, int h, int slot) {
 #pragma unroll
-        for (int i = 0; i < LOADS - 4; i++) load_weights(at, h, slot, i);
+        for (int i = 0; i < LOADS - 6; i++) load_weights(at, h, slot, i);
     };
 
     v16f_bq acc[4], t[4]; // 32 x 32 parts: activation rows q / 2, weight rows q % 2; lane = weight row, register r = activation row 8 (r / 4) + 4 hh + r % 4
@@ -257,17 +195,17 @@ __global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4*
             if constexpr (BITS == 6) asm volatile("" : "+v"(whi[g]));
         }
     };
-    const auto convert = [&](v8h (&w)[2][2], int part) { // [32 weight rows][chunk], in four parts
+    const auto convert = [&](v8bf (&w)[2][2], int part) { // [32 weight rows][chunk], in four parts
         const int g = part >> 1, ch = part & 1;
         if constexpr (BITS == 8)
-            w[g][ch] = bytes_to_halves(wq[g][2 * ch], wq[g][2 * ch + 1]);
+            w[g][ch] = bytes_to_bf16((unsigned)wq[g][2 * ch], (unsigned)wq[g][2 * ch + 1]);
         else if constexpr (BITS == 4)
-            w[g][ch] = nibbles_to_halves((unsigned)wlo[g][ch]);
+            w[g][ch] = nibbles_to_bf16((unsigned)wlo[g][ch]);
         else if (ch == 0)
-            sixbit_to_halves((unsigned)wlo[g][0], (unsigned)wlo[g][1], (unsigned)whi[g], w[g][0], w[g][1]);
+            sixbit_to_bf16((unsigned)wlo[g][0], (unsigned)wlo[g][1], (unsigned)whi[g], w[g][0], w[g][1]);
     };
 
-    v8h w[2][2];
+    v8bf w[2][2];
     issue_weights(first, 0, 0);
     issue_activations(first, 0);
     issue_weights(first, 1, 1);
@@ -290,11 +228,11 @@ __global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4*
         union Act
         {
             v4i_bq i4;
-            v8h b;
+            v8bf b;
         };
-        Act y[8];
+        Act y[12];
 #pragma unroll
-        for (int i = 0; i < 8; i++) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(y[i].i4) : "v"(a_at), "n"(h * TILES_STAGE + i * 1024));
+        for (int i = 0; i < 12; i++) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(y[i].i4) : "v"(a_at), "n"(h * TILES_STAGE + i * 1024));
         read_weights(next);
         if constexpr (h == 0)
         {
@@ -306,7 +244,7 @@ __global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4*
             for (int g = 0; g < 2; g++) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(d[g]) : "v"(d_at + o), "n"(g * 128));
         }
 #pragma unroll
-        for (int i = 0; i < 8; i++) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(y[i].i4));
+        for (int i = 0; i < 12; i++) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(y[i].i4));
         weights_here();
         if constexpr (h == 0) asm volatile("" : "+v"(d[0]), "+v"(d[1]));
         __builtin_amdgcn_s_barrier(); // both wavefronts of the group have read the stage
@@ -318,28 +256,28 @@ __global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4*
 #pragma unroll
                 for (int r = 0; r < 16; r++) t[q][r] = 0.f;
         }
-        v8h wn[2][2]; // the next stage's
-        // four rounds of four products; the loads and the conversions spread over them
+        v8bf wn[2][2]; // the next stage's
+        // six rounds of four products; the loads and the conversions spread over them
 #pragma unroll
-        for (int c = 0; c < 4; c++)
+        for (int c = 0; c < 6; c++)
         {
-            const int ch = c / 2, p = c % 2;
+            const int ch = c / 3, p = c % 3;
 #pragma unroll
-            for (int i = c * LOADS / 4; i < (c + 1) * LOADS / 4; i++)
+            for (int i = c * LOADS / 6; i < (c + 1) * LOADS / 6; i++)
             {
-                if (i < 4)
+                if (i < 6)
                     load_activations(kb + 1, h, i);
                 else
-                    load_weights(h == 0 ? kb + 1 : kb + 2, h ^ 1, slot, i - 4);
+                    load_weights(h == 0 ? kb + 1 : kb + 2, h ^ 1, slot, i - 6);
             }
 #pragma unroll
-            for (int q = 0; q < 4; q++) t[q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(y[((q >> 1) * 2 + ch) * 2 + p].b, w[q & 1][ch], t[q], 0, 0, 0);
-            convert(wn, c);
+            for (int q = 0; q < 4; q++) t[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(y[((q >> 1) * 2 + ch) * 3 + p].b, w[q & 1][ch], t[q], 0, 0, 0);
+            if (c < 4) convert(wn, c);
 #pragma unroll
             for (int q = 0; q < 4; q++)
             {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                if (q < (c + 1) * LOADS / 4 - c * LOADS / 4) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+                if (q < (c + 1) * LOADS / 6 - c * LOADS / 6) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -377,13 +315,6 @@ __global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4*
 #pragma unroll
             for (int e = 0; e < 4; e++) to[e * 64] = v4f_t{acc[q][4 * e], acc[q][4 * e + 1], acc[q][4 * e + 2], acc[q][4 * e + 3]};
         }
-    // what the part's results need from memory is on its way while the groups meet (read behind their sums it was 1.5 us of a workgroup's time)
-    const int j = (tile0 + 2 * (group & 1)) * 16 + l32, i0 = row0 + (group >> 1) * 32 + 4 * hh; // result r: row i0 + 8 (r / 4) + r % 4 (`back` is padded to 64 rows)
-    v4f_t factor[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) factor[e] = *reinterpret_cast<const v4f_t*>(back + i0 + 8 * e);
-    const bool of_column = bt == 0 || bt == 4;
-    const float addend = of_column && j < N ? mul_rn(load_c(c, bt, 0, j, N), beta) : 0.f;
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 4; q++)
@@ -401,18 +332,16 @@ __global__ __launch_bounds__(KG * 128) void blockquant_tiles_kernel(const uint4*
                 for (int o = 0; o < 4; o++) acc[q][4 * e + o] += v[o];
             }
         }
+        const int j = (tile0 + 2 * (q & 1)) * 16 + l32;
         if (j >= N) continue;
 #pragma unroll
         for (int r = 0; r < 16; r++)
         {
-            const int i = i0 + 8 * (r >> 2) + (r & 3);
+            const int i = row0 + (q >> 1) * 32 + 8 * (r >> 2) + 4 * hh + (r & 3);
             if (i < M)
             {
-                float v = acc[q][r] * factor[r >> 2][r & 3];
-                if (of_column)
-                    v = add_rn(addend, v);
-                else if (bt >= 0)
-                    v = add_rn(mul_rn(load_c(c, bt, i, j, N), beta), v);
+                float v = acc[q][r];
+                if (bt >= 0) v = add_rn(mul_rn(load_c(c, bt, i, j, N), beta), v);
                 out[(size_t)i * out_stride + j] = mul_rn(v, alpha);
             }
         }
@@ -424,25 +353,11 @@ int launch_blockquant_tiles(const float* a, size_t a_stride, int M, int N, int K
 {
     const int kblocks = (K + 63) / 64, ntiles = (N + 15) / 16, blocks = (M + 63) / 64;
     uint4* frags = static_cast<uint4*>(workspace);
-    float* back = reinterpret_cast<float*>(frags + (size_t)blocks * kblocks * 1024); // 4 bytes a value, and the rows' factors behind them
-    const dim3 grid((unsigned)((ntiles + 7) / 8), (unsigned)blocks);
-    const int spans = (kblocks * 64 + SPLIT_SPAN - 1) / SPLIT_SPAN, waves = spans < SPLIT_WAVES ? spans : SPLIT_WAVES;
-#define SPLIT(HALVES_, KEEP_) \
-    hipLaunchKernelGGL((blockquant_split_tiles_kernel<HALVES_, KEEP_>), dim3((unsigned)(blocks * (64 / SPLIT_ROWS))), dim3((unsigned)(64 * waves)), 0, st, a, a_stride, M, K, kblocks, in_scales, frags, back)
-    const int keep = (spans + SPLIT_WAVES - 1) / SPLIT_WAVES; // what a wavefront keeps, up to three (K = 12288)
-    if (keep == 1 && bits == 8)
-        SPLIT(false, 1);
-    else if (keep == 1)
-        SPLIT(true, 1);
-    else if (keep == 2 && bits == 8)
-        SPLIT(false, 2);
-    else if (keep == 2)
-        SPLIT(true, 2);
-    else if (bits == 8)
-        SPLIT(false, 3);
+    const dim3 sgrid((unsigned)((kblocks + 1) / 2), (unsigned)blocks), grid((unsigned)((ntiles + 7) / 8), (unsigned)blocks);
+    if (bits == 8)
+        hipLaunchKernelGGL(blockquant_split_tiles_kernel<false>, sgrid, dim3(256), 0, st, a, a_stride, M, K, kblocks, in_scales, frags);
     else
-        SPLIT(true, 3);
-#undef SPLIT
+        hipLaunchKernelGGL(blockquant_split_tiles_kernel<true>, sgrid, dim3(256), 0, st, a, a_stride, M, K, kblocks, in_scales, frags);
 #define TILES(BITS_)                                                                                                                                          \
     do                                                                                                                                                             \
     {                                                                                                                                                              \
@@ -455,7 +370,7 @@ int launch_blockquant_tiles(const float* a, size_t a_stride, int M, int N, int K
             NCNNHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));                     \
             if (device >= 0 && device < 64) raised[device].store(1, std::memory_order_release);                                                                    \
         }                                                                                                                                                          \
-        hipLaunchKernelGGL(kernel, grid, dim3(KG * 128), tiles_lds_bytes(BITS_), st, frags, back, M, N, kblocks, ntiles, wpk, dpk, c, bt, alpha, beta, out,      \
+        hipLaunchKernelGGL(kernel, grid, dim3(KG * 128), tiles_lds_bytes(BITS_), st, frags, M, N, kblocks, ntiles, wpk, dpk, c, bt, alpha, beta, out,      \
                            out_stride);                                                                                                                            \
     } while (0)
     if (bits == 8)

@@ -785,7 +785,7 @@ class Runtime:
 
     def gemm_blockquant_packed(self, a, pw, pd, n, c=None, broadcast_type_c=-1, alpha=1.0, beta=1.0, bits=8, block=64, in_scales=None, rows_kernel=False):
         """a fp16: the fp16-activation entry point; a fp32 (optionally with in_scales): the layer's contract, activations split into three bf16
-        (rows_kernel: the call for many rows, with its workspace, whose largest form splits into two fp16)."""
+        (rows_kernel: the tiled form for many rows, with its workspace)."""
         half = a.dtype == np.float16
         a = np.ascontiguousarray(a, np.float16 if half else np.float32)
         m, k = a.shape

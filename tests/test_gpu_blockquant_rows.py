@@ -228,19 +228,24 @@ def test_fp32_rows_in_64x128_tiles(rt, m, n, k, bits, block):
     assert np.array_equal(got[1, :n][q != 0], np.where(q > 0, np.inf, -np.inf)[q != 0].astype(F)) and np.all(np.isnan(got[1, :n][q == 0])) and np.all(np.isnan(got[m - 1, :n]))
 
 
-@pytest.mark.parametrize("m,n,k,bits", [(130, 40, 4112, 8), (133, 130, 12304, 4), (129, 16, 12816, 8), (140, 24, 144, 6)])
-def test_fp32_rows_of_any_magnitude_in_64x128_tiles(rt, m, n, k, bits):
-    """Rows are scaled by a power of two before they are split: rows of zeros, of subnormals, next to the largest float, with few values of
-    any weight, over spans that fit the split pass's registers and beyond them.  An activation keeps 23 bits, which stay below 1e-6 of the floor with the sums' roundings, and
-    what lies above 2^-40 of its row's largest."""
+@pytest.mark.parametrize("m,n,k,bits", [(130, 40, 4112, 8), (133, 130, 12304, 4), (129, 16, 12816, 8), (140, 24, 144, 6),  # few tiles: K over two groups of wavefronts
+                                        (1030, 1010, 400, 8), (1090, 960, 144, 4), (1030, 1000, 208, 6),                         # 64 x 128 tiles
+                                        (2060, 2050, 144, 8)])                                                                  # 64 x 192
+def test_fp32_rows_of_any_magnitude(rt, m, n, k, bits):
+    """Rows of zeros, of subnormals, as large as a K step holds, with few values of any weight, and rows whose largest values meet weights of zero: an activation keeps its 24 bits
+    whatever stands beside it (of the least of its three bf16 numbers, what lies above 2^-134), so that the sums' roundings are the only error.  A step adds up to 64 products
+    with fields of up to 127 before their scale: less than 2^13 times the largest activation, so that magnitudes up to 2^114 stay below 2^127 (every form has this limit)."""
     a, packed, scales = synth.blockquant_operands(m + n, m, n, k, bits, 64, half_exact=False)
     rng = np.random.default_rng(k)
     scales *= 64  # outputs of the largest row stay finite
     a[0] = 0
-    a[1], a[2], a[3] = a[1] * F(2.0 ** -130), a[2] * F(2.0 ** -112), a[3] * F(2.0 ** 120) / max(1, np.abs(a[3]).max())
+    a[1], a[2], a[3] = a[1] * F(2.0 ** -130), a[2] * F(2.0 ** -112), a[3] * F(2.0 ** 114) / max(1, np.abs(a[3]).max())
     a[4] *= np.exp2(rng.integers(-60, 60, k)).astype(F)
     a[5, 1:] *= F(2.0 ** -35)
     a[m - 1, : k - 1] = 0
+    a[6, 64:80] *= F(2.0 ** 50)  # a field of zero whatever its block's scale: these columns weigh nothing
+    a[7, 64:80] = F(2.0 ** 100)
+    packed[:, 64 * bits // 8:80 * bits // 8] = 0
     pw, pd = rt.blockquant_pack(packed, scales, 64, bits=bits, k=k)
     w, d = rt.up(pw), rt.up(pd)
     size = C.c_size_t()
@@ -253,15 +258,14 @@ def test_fp32_rows_of_any_magnitude_in_64x128_tiles(rt, m, n, k, bits):
     val, floor = npref.blockquant_gemm_f64(a, packed, scales, bits, 64)
     assert np.all(np.isfinite(got)) and np.all(got[0] == 0)
     ones = npref.blockquant_gemm_f64(np.ones((1, k), F), packed, scales, bits, 64)[1]
-    assert np.all(np.abs(got - val) <= 1e-6 * floor + 2.0 ** -40 * np.abs(a).max(axis=1, keepdims=True).astype(np.float64) * ones + 2.0 ** -148)
+    assert np.all(np.abs(got - val) <= 1e-6 * floor + 2.0 ** -133 * ones)
 
 
-# spans of 256 columns over 16 wavefronts: one wavefront, a part of the last span, one, two and three spans each, and what goes beyond the registers
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("m,k", [(129, 64), (191, 272), (131, 4096), (131, 4112), (193, 8192), (131, 8208), (131, 12288), (193, 12304)])
-def test_split_pass_of_whole_rows(rt, m, k, bits):
-    """Two rows to a workgroup, dealt out to the dies by lines: every row has its own size, so that a row, factor or span out of place shows.  The bound is that of
-    test_fp32_rows_of_any_magnitude_in_64x128_tiles: 23 bits an activation and the sums' roundings, relative to the sum of magnitudes."""
+def test_split_pass_of_rows_of_their_own_size(rt, m, k, bits):
+    """Every row has its own size, so that a row or a piece of one out of place shows, on K of one step to many and a part of one.  The bound is that of
+    test_fp32_rows_of_any_magnitude: the sums' roundings, relative to the sum of magnitudes."""
     a, packed, scales = synth.blockquant_operands(m + k, m, 48, k, bits, 64, half_exact=False)
     a *= np.exp2(np.arange(m) % 41 - 20).astype(F)[:, None]
     pw, pd = rt.blockquant_pack(packed, scales, 64, bits=bits, k=k)
