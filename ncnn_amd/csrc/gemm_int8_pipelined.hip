@@ -48,7 +48,8 @@ constexpr int STAGE_BYTES = 2 * OPERAND_BYTES; // 32 KB
 
 
 // Row-major operands end at any M and any N of whole fours: rows past the end repeat the last one and are never stored.
-template<bool PER_COL, int BT, bool TILED>
+// FAR: whole tiles whose rows lie too far apart for 32-bit offsets inside a tile (gemm_rows_are_far); nothing is cut then.
+template<bool PER_COL, int BT, bool TILED, bool FAR>
 __global__ __launch_bounds__(256) void gemm_int8_256x256_kernel(const int8_t* __restrict__ A, size_t lda, const int8_t* __restrict__ B,
                                                                  size_t ldb, int nk, int M, int N, int tiles_m, int tiles_n,
                                                                  const float* __restrict__ a_scales, const float* __restrict__ b_scales,
@@ -90,13 +91,14 @@ __global__ __launch_bounds__(256) void gemm_int8_256x256_kernel(const int8_t* __
     const int rows_a = M - tile_m * PT, rows_b = N - tile_n * PT;
     const int8_t* ua = A + (TILED ? (size_t)tile_m * nk * OPERAND_BYTES : (size_t)tile_m * PT * lda);
     const int8_t* ub = B + (TILED ? (size_t)tile_n * nk * OPERAND_BYTES : (size_t)tile_n * PT * ldb);
-    unsigned off_a[4], off_b[4];
+    typedef typename std::conditional<FAR, size_t, unsigned>::type offset_t;
+    offset_t off_a[4], off_b[4];
 #pragma unroll
     for (int i = 0; i < 4; i++)
     {
         const int ra = i * 64 + ld_row, rb = (i >> 1) * 128 + (i & 1) * 2 + ld_row_b;
-        off_a[i] = TILED ? ld_row * PK + ld_chunk * 16 : (unsigned)((ra < rows_a ? ra : rows_a - 1) * lda + ld_chunk * 16);
-        off_b[i] = TILED ? off_a[i] : (unsigned)((rb < rows_b ? rb : rows_b - 1) * ldb + ld_chunk * 16);
+        off_a[i] = TILED ? ld_row * PK + ld_chunk * 16 : (offset_t)((ra < rows_a ? ra : rows_a - 1) * lda + ld_chunk * 16);
+        off_b[i] = TILED ? off_a[i] : (offset_t)((rb < rows_b ? rb : rows_b - 1) * ldb + ld_chunk * 16);
     }
     constexpr int STEP = TILED ? OPERAND_BYTES : PK;
 
@@ -266,7 +268,7 @@ __global__ __launch_bounds__(256) void gemm_int8_256x256_kernel(const int8_t* __
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int e = 0; e < 4; e++) rowscale[i][e] = *reinterpret_cast<const v4f*>(row_scale + wm * 128 + i * 32 + 8 * e + 4 * lhi);
-    float* lane_out = out + (size_t)(tile_m * PT + wm * 128 + 4 * lhi) * ldo + col_base; // TILED
+    float* lane_out = out + (size_t)(tile_m * PT + wm * 128 + 4 * lhi) * ldo + col_base; // TILED, FAR
     // else a buffer that ends with the last row and column of the output: stores beyond are dropped without a branch around each
     const int in_rows = rows_a < PT ? rows_a : PT, in_cols = rows_b < PT ? rows_b : PT, lane_col = wn * 128 + 4 * l32;
     const auto tile_out = __builtin_amdgcn_make_buffer_rsrc(out + (size_t)tile_m * PT * ldo + (size_t)tile_n * PT, 0, (int)(((in_rows - 1) * (unsigned)ldo + in_cols) * 4), 0x00020000);
@@ -287,7 +289,7 @@ __global__ __launch_bounds__(256) void gemm_int8_256x256_kernel(const int8_t* __
                 f4[j] = mul_rn(f, alpha);
             }
             const unsigned further = (r & 3) == 3 ? 5 : 1;
-            if constexpr (TILED)
+            if constexpr (TILED || FAR)
             {
                 *reinterpret_cast<v4f*>(lane_out) = f4; // (non-temporal stores: neutral at 4096 cubed, 3 % slower at 8192 cubed)
                 lane_out += further * ldo;
@@ -525,14 +527,22 @@ static inline bool al16(const void* p)
     return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
 
-template<bool TILED>
+// Whether rows are too far apart for 32-bit offsets inside a 256 x 256 tile: of the operands 256 rows of 4 GiB and more, of the output of 2^30 bytes (a step past
+// the last row stays below 2^31).  us, output rows 2^20 + 4 floats apart, 128 x 128 ring / here: 512 x 32768 x 1024 41.3 / 29.0, 256 x 65536 x 512 31.3 / 23.2 (256 x 32768 x 64 9.2 / 11.0).
+static bool gemm_rows_are_far(size_t aq_stride, size_t bq_stride, size_t out_stride)
+{
+    constexpr size_t most = (0xffffffffull - 256) / PT;
+    return aq_stride > most || bq_stride > most || out_stride > (1u << 20);
+}
+
+template<bool TILED, bool FAR = false>
 static int launch_256x256(const int8_t* aq, size_t aq_stride, const int8_t* bq, size_t bq_stride, int M, int N, int K, const GemmEpilogue& epi,
                           hipStream_t stream)
 {
     const int tm = ceil_div(M, PT), tn = ceil_div(N, PT), nk = K / PK;
     dim3 grid(tm * tn), block(256);
 #define LAUNCH(PC, BTV)                                                                                                                    \
-    hipLaunchKernelGGL((gemm_int8_256x256_kernel<PC, BTV, TILED>), grid, block, 0, stream, aq, aq_stride, bq, bq_stride, nk, M, N, tm, tn, \
+    hipLaunchKernelGGL((gemm_int8_256x256_kernel<PC, BTV, TILED, FAR>), grid, block, 0, stream, aq, aq_stride, bq, bq_stride, nk, M, N, tm, tn, \
                        epi.a_scales, epi.b_scales, epi.c, epi.alpha, epi.beta, epi.out, epi.out_stride)
     if (epi.per_col)
     {
@@ -560,9 +570,10 @@ int launch_gemm_int8_pipelined(const int8_t* aq, size_t aq_stride, const int8_t*
     if (epi.transpose || epi.acc_out || !(epi.bt == -1 || epi.bt == 4)) return NCNNHIP_OK;
     if (epi.out_stride % 4 || !al16(epi.out)) return NCNNHIP_OK; // the epilogue stores 16 bytes per lane
     if ((long long)ceil_div(M, PT) * ceil_div(N, PT) > 0x7fffffff) return NCNNHIP_OK;
-    if ((unsigned long long)PT * aq_stride + 256 > 0xffffffffull || (unsigned long long)PT * bq_stride + 256 > 0xffffffffull) return NCNNHIP_OK; // 32-bit lane offsets
-    if (epi.out_stride > (1u << 20)) return NCNNHIP_OK; // the same of the output: 256 rows end below 2^31 bytes
+    const bool far = gemm_rows_are_far(aq_stride, bq_stride, epi.out_stride);
+    if (far && (M % PT || N % PT)) return NCNNHIP_OK;
     *handled = true;
+    if (far) return launch_256x256<false, true>(aq, aq_stride, bq, bq_stride, M, N, K, epi, stream);
     return launch_256x256<false>(aq, aq_stride, bq, bq_stride, M, N, K, epi, stream);
 }
 

@@ -1,9 +1,11 @@
 """The int8 Gemm on rows that begin and end at any byte, at the edges of its tiles, K steps and dispatch: against the oracle, bit for
 bit (src/layer/gemm.cpp:745-966)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from ncnn_amd.hip import check, lib
+from ncnn_amd.hip import DeviceBuffer, check, lib
 from oracle import oracle
 from tests import cases, npref
 
@@ -86,6 +88,26 @@ def test_256x256_tiles_cut_at_the_end(rt, m, n, k, per_col):
         check(lib().ncnnhip_gemm_int8(da.ptr, k, db.ptr, k, m, cols, k, dsa.ptr, dsb.ptr, cols if per_col else 1, dc.ptr, 4, 1.0, 1.0, 0, out.ptr, stride, None, rt.stream))
         got = out.to_numpy(rt.stream)
         assert np.array_equal(got[:m, :cols], want[:, :cols]) and np.all(got[:m, cols:] == 7.0) and np.all(got[m] == 7.0)
+
+
+@pytest.mark.parametrize("a_stride,o_stride", [(64, (1 << 20) + 4), ((1 << 24) + 16, 32768)])
+@pytest.mark.parametrize("per_col", [True, False])
+def test_256x256_tiles_of_rows_far_apart(rt, a_stride, o_stride, per_col):
+    """128 whole tiles of one K step whose output rows are more than 2^20 floats apart, or whose 256 rows of A take more than 4 GiB: offsets inside a tile
+    beyond 32 bits.  Nothing is written between the rows."""
+    print("[case]", a_stride, o_stride, per_col, flush=True)
+    m, n, k = 256, 32768, 64
+    a, bq, sb, bias = cases.gemm_case(a_stride % 1000, m, n, k, per_col=per_col)
+    aq, sa = rt.gemm_quantize_rows(a)
+    want, _ = npref.gemm_int8(aq, bq, sa, sb, bias, 4, acc=npref.gemm_acc_exact(aq, bq))
+    da, db, dsa, dsb, dc = DeviceBuffer((m - 1) * a_stride + k), rt.up(bq), rt.up(sa), rt.up(sb), rt.up(bias.reshape(-1))
+    for i in range(m):
+        check(lib().ncnnhip_memcpy_h2d(C.c_void_p(da.ptr.value + i * a_stride), aq[i].ctypes.data_as(C.c_void_p), k, rt.stream))
+    check(lib().ncnnhip_stream_synchronize(rt.stream))
+    out = rt.up(np.full((m, o_stride), 7.0, np.float32))
+    check(lib().ncnnhip_gemm_int8(da.ptr, a_stride, db.ptr, k, m, n, k, dsa.ptr, dsb.ptr, n if per_col else 1, dc.ptr, 4, 1.0, 1.0, 0, out.ptr, o_stride, None, rt.stream))
+    got = out.to_numpy(rt.stream)
+    assert np.array_equal(got[:, :n], want) and np.all(got[:, n:] == 7.0)
 
 
 @pytest.mark.parametrize("m,n,k,pad", [(1601, 1537, 1003, 0), (1850, 1800, 1004, 0), (1793, 1805, 1024, 1), (2305, 2241, 1002, 2)])
