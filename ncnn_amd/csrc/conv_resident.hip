@@ -886,18 +886,16 @@ static int resident_choose(const NhwcGeom& g, const ConvEpilogue& epi, const Con
 // here / there): 18 steps 50176 x 128 19.9 / 16.3, 100352 x 128 31.8 / 30.8, 200704 x 128 53.8 / 52.1, 36 steps 50176 x 256 62.4 / 47.2.  64 channels
 // stay: 9 steps 401408 x 64 29.3 / 36.6, 200704 x 64 18.0 / 21.1, 100352 x 64 11.7 / 13.1.
 // Environment, read at every launch: NCNNHIP_RESIDENT_OFF (any value) switches the kernel off, NCNNHIP_RESIDENT_MIN sets
-// the pixel threshold, NCNNHIP_RESIDENT_CFG forces one tile configuration (0..7): for measurements and tests.
+// the pixel threshold (and nothing else: what leaves for the 128 x 128 tiles does so whatever it is), NCNNHIP_RESIDENT_CFG forces one tile configuration (0..7): for measurements and tests.
 bool conv_resident_fits(const NhwcGeom& g, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp)
 {
     if (!epi.out) return false; // it writes the fp32 blob
     if (g.ntaps < 2) return false; // first: most layers of a network are 1x1 and need not look the environment up
     if (getenv("NCNNHIP_RESIDENT_OFF")) return false;
-    long long min_pixels = 40000;
-    if (const char* e = getenv("NCNNHIP_RESIDENT_MIN"))
-        min_pixels = atoll(e);
-    else if (g.K / 64 >= 16 && (g.cout + 63) / 64 % 2 == 0 && !fusion.residual)
-        return false;
-    if (g.npix < min_pixels) return false;
+    constexpr long long MANY_PIXELS = 40000;
+    if (g.npix >= MANY_PIXELS && g.K / 64 >= 16 && (g.cout + 63) / 64 % 2 == 0 && !fusion.residual) return false;
+    const char* e = getenv("NCNNHIP_RESIDENT_MIN");
+    if (g.npix < (e ? atoll(e) : MANY_PIXELS)) return false;
     ResidentPlan P;
     size_t lds_bytes;
     return resident_choose(g, epi, fusion, out_cp, P, lds_bytes) >= 0;

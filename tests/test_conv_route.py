@@ -43,6 +43,18 @@ def test_tile_of_the_pipelined_kernel(shape, options, tile):
     assert (r.kernel, r.tile_pixels, r.tile_channels, r.groups, r.splits) == (r.PIPELINED,) + tile + (1, 1)
 
 
+@pytest.mark.parametrize("threshold", [None, "40000", "1", "1000000"])
+def test_pixel_threshold_of_the_resident_kernel(monkeypatch, threshold):
+    """NCNNHIP_RESIDENT_MIN moves the threshold and nothing else: a long K on whole 128s of channels goes to the 128 x 128 tiles whether it is set or not."""
+    monkeypatch.delenv("NCNNHIP_RESIDENT_MIN", raising=False)
+    if threshold:
+        monkeypatch.setenv("NCNNHIP_RESIDENT_MIN", threshold)
+    r = cases.conv_route(64, 128, 28, 28, 128, (3, 3), **SAME3)
+    assert (r.kernel, r.tile_pixels, r.tile_channels) == (r.PIPELINED, 128, 128)
+    assert (cases.conv_route(16, 64, 56, 56, 64, (3, 3), **SAME3).kernel == r.RESIDENT) == (int(threshold or 40000) <= 16 * 56 * 56)
+    assert (cases.conv_route(32, 128, 28, 28, 128, (3, 3), **SAME3).kernel == r.RESIDENT) == (threshold == "1")
+
+
 def test_layers_that_are_refused():
     from ncnn_amd.hip import Activation, ConvDesc, ConvRoute, lib
     r, act = ConvRoute(), Activation.make(0, (0.0, 0.0))
