@@ -118,7 +118,11 @@ static void choose_tile(const NhwcGeom& g, bool residual, PipePlan& p)
         p.bm = p.bn = 128;
     else if (wide && tiles(64, 128) >= (steps >= 16 ? 300 : 900) && (steps >= 2 || g.cout <= 128))
         p.bn = 128;
-    if (wide && tiles(64, p.bn) * ceil_div(g.cout, p.bn) >= 1ll << 32) p.bm = p.bn = 128; // (the kernel's division of a tile number: an output of 70 GB and more)
+    if (tiles(64, p.bn) > MOST_BLOCKS) // (an output of 69 GB and more)
+    {
+        p.bm = 128;
+        p.bn = wide ? 128 : 64;
+    }
     p.tiles_m = ceil_div(g.npix, p.bm);
     p.tiles_n = ceil_div(g.cout, p.bn);
 }
@@ -179,7 +183,7 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
     PipePlan p;
     const int mode = pipelined_form(g, fusion.residual != 0, p);
     const long long blocks = (long long)p.tiles_m * p.tiles_n * p.splits;
-    NCNNHIP_REQUIRE(blocks < (1ll << 31) && blocks * p.tiles_n < (1ll << 32), "convolution: too many tiles");
+    NCNNHIP_REQUIRE(blocks * p.groups <= MOST_BLOCKS, "convolution: too many tiles");
     int32_t* partial = 0;
     unsigned* counters = 0;
     if (p.splits > 1)
@@ -222,10 +226,8 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
         LAUNCH_PIPE_MODE(64, 64, 0, 4);
     else if (p.bm == 128 && p.bn == 128)
         LAUNCH_PIPE(128, 128);
-    else if (p.bm == 128 && mode == 1) // narrow inputs: a 1x1 kernel, and a gathered one
-        LAUNCH_PIPE_MODE(128, 64, 1, 1);
-    else if (p.bm == 128)
-        LAUNCH_PIPE_MODE(128, 64, 2, 1);
+    else if (p.bm == 128) // narrow inputs, and more tiles than a launch holds
+        LAUNCH_PIPE(128, 64);
     else if (p.bn == 128)
         LAUNCH_PIPE(64, 128);
     else

@@ -37,9 +37,12 @@ int launch_conv_shortcut(const NhwcGeom& g_in, const int8_t* wpk, const int8_t* 
     // 16 images 64 + 64 -> 256 on 56 x 56 22.2 / 18.8, 128 + 256 -> 512 on 28 x 28 19.5 / 15.7, 256 + 512 -> 1024 on 14 x 14 14.5 / 13.4, 512 + 1024 -> 2048
     // on 7 x 7 18.5 / 14.6 (two launches 36.5, 26.6, 17.4, 15.9); 64 images 80 / 84 (12544 tiles; int8 alone 57 / 50), 44.9 / 44.4 (6272), 37.1 / 34.4, 37.8 / 32.1; 128 images 128 + 256 -> 512
     // (12544 tiles of six steps) 93.2 / 86.4.
-    const int tiles_m = ceil_div(g.npix, 64), wide = (long long)tiles_m * ceil_div(g.cout, 64) >= 8192 && g.K / 64 + sc.Cp / 64 <= 4, tiles_n = ceil_div(g.cout, wide ? 128 : 64);
+    const int tiles_m = ceil_div(g.npix, 64);
+    const long long narrow = (long long)tiles_m * ceil_div(g.cout, 64);
+    const bool wide = narrow > MOST_BLOCKS || (narrow >= 8192 && g.K / 64 + sc.Cp / 64 <= 4);
+    const int tiles_n = ceil_div(g.cout, wide ? 128 : 64);
     const long long blocks = (long long)tiles_m * tiles_n;
-    NCNNHIP_REQUIRE(blocks < (1ll << 31) && blocks * tiles_n < (1ll << 32), "convolution: too many tiles");
+    NCNNHIP_REQUIRE(blocks <= MOST_BLOCKS, "convolution: too many tiles");
     ConvShortcutArg<true> arg;
     static_cast<ConvShortcut&>(arg) = sc;
 #define LAUNCH_SHORTCUT(BN_)                                                                                                                            \
