@@ -97,8 +97,9 @@ struct StreamRest
 // TP, TC: 16-pixel and 16-channel blocks of a tile.  U: K steps a wavefront has in flight, at 4 (TP + TC) registers each; W: wavefronts.
 // SHORTCUT: a projection shortcut is added (ConvShortcut), its K dealt out to the wavefronts and its sums met in the same way; both convolutions'
 // loads are in flight together.
-// The arguments before `rest` are 56 bytes and arrive in registers (amdgpu-kernarg-preload-count), so that the first loads wait for no other; of
+// The arguments before `rest` are REST_AT bytes and arrive in registers (amdgpu-kernarg-preload-count), so that the first loads wait for no other; of
 // `rest` the epilogue's part is read behind them, through a pointer that the compiler cannot move the reads across.
+constexpr size_t REST_AT = 56;
 template<bool DENSE, int TP, int TC, int U, int W, bool SHORTCUT = false>
 __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __restrict__ wpk, const int8_t* __restrict__ x, unsigned x_bytes, int K, int Cp, int npix, int cout,
                                                              int out_cp, int tiles, int tiles_m, unsigned magic_m, int per_wave,
@@ -147,7 +148,7 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
             const int img = magic_div(p, g.plane, g.magic_plane), at = p - img * g.plane, oy = magic_div(at, g.outw, g.magic_outw);
             iy0[i] = p < npix ? oy * g.sh - g.pad_top : -0x40000000; // a pixel beyond the last fails every bounds test
             ix0[i] = (at - oy * g.outw) * g.sw - g.pad_left;
-            x_off[i] = (unsigned)(((img * g.H + iy0[i]) * g.W + ix0[i]) * Cp + kq * 16);
+            x_off[i] = ((unsigned)(img * g.H + iy0[i]) * (unsigned)g.W + (unsigned)ix0[i]) * (unsigned)Cp + kq * 16; // (modulo 2^32: a tap's offset brings it back into the image)
         }
     }
     int q = 0, ky = 0, kx = 0; // step inside the tap, and the tap: the same in every lane
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
     issue();
 
     __builtin_amdgcn_sched_barrier(0);
-    const __attribute__((address_space(4))) char* rest_at = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() + 56;
+    const __attribute__((address_space(4))) char* rest_at = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() + REST_AT;
     asm volatile("" : "+s"(rest_at));
     const StreamRest<SHORTCUT>& late = *(const StreamRest<SHORTCUT>*)rest_at;
     const StreamShortcutArg<SHORTCUT>& shortcut = late.shortcut;
@@ -477,6 +478,20 @@ int conv_stream_shortcut_tile(const NhwcGeom& g, int shortcut_steps)
     return stream_dense(g) && g.K == g.Cp && stream_reaches(g) ? stream_tile(g, g.K / 64 + shortcut_steps, g.K / 64 % 2 == 1 && shortcut_steps % 2 == 1, true, 2) : 0;
 }
 
+// where a kernel finds its last argument
+template<typename Kernel>
+struct LastArgument;
+template<typename... Arguments>
+struct LastArgument<void(Arguments...)>
+{
+    static constexpr size_t at()
+    {
+        size_t last = 0, end = 0;
+        ((last = (end + alignof(Arguments) - 1) / alignof(Arguments) * alignof(Arguments), end = last + sizeof(Arguments)), ...);
+        return last;
+    }
+};
+
 // Steps in flight (U) and wavefronts (W) for this many steps of K: a round costs a trip to memory, and a step that only fills up a round its loads' issue.
 // blocks: 16-byte operands a lane holds per step; 36 of them, 144 registers, are in flight at most.  Eight wavefronts from 49 steps on, where four would walk
 // two rounds: 3x3 512 -> 512 on 7 x 7 (72 steps) 7.2 -> 6.4 us, 1x1 4096 -> 512 6.9 -> 6.0.
@@ -508,6 +523,7 @@ static void launch_stream_form(int u, const NhwcGeom& g, const int8_t* wpk, cons
     if (!DENSE)
         rest.taps = {g.H, g.W, g.kw, g.dh, g.dw, g.sh, g.sw, g.pad_top, g.pad_left, g.outw, plane, steps, magic_of(plane), magic_of(g.outw), magic_of(steps), magic_of(g.kw)};
     constexpr int blocks = (TP + TC) * (SHORTCUT ? 2 : 1);
+    static_assert(LastArgument<decltype(conv_stream_kernel<DENSE, TP, TC, 1, W, SHORTCUT>)>::at() == REST_AT, "`rest` lies where the kernel looks for it");
 #define STREAM(U_)                                                                                                                                              \
     if constexpr (stream_form_built(U_, blocks))                                                                                                                \
         if (u == U_)                                                                                                                                            \
