@@ -324,7 +324,7 @@ __device__ __forceinline__ int small_div(int n, int d)
     return q;
 }
 
-static inline int ceil_div(long long a, long long b)
+static constexpr int ceil_div(long long a, long long b)
 {
     return (int)((a + b - 1) / b);
 }

@@ -421,6 +421,7 @@ static bool stream_dense(const NhwcGeom& g)
 //   16 x 16, below 128 tiles   even: 144 steps 0.87-0.93, 176 0.94-0.99, 194 1.00-1.06, 288 1.03-1.09    odd: 193 0.8, 401 0.86-0.91, 641 0.88-0.95
 //   16 x 16, from 128 on       even: 208 0.81-0.93, 288 0.91-0.98, 322 0.98-1.08, 402 1.02-1.23          odd: 401 0.78-0.94, 641 1.09-1.20
 //   16 x 32                    even: 64 0.87-0.91, 80 0.96-1.02, 96 1.04-1.05, 144 1.2, 402 2.0          odd: 81 0.8, 145 0.92-1.00, 193 1.00-1.17
+constexpr int LONGEST_32 = 48; // steps of a 32 x 32 tile
 static int stream_tile(const NhwcGeom& g, int steps, bool odd, bool fp32_out, int convolutions)
 {
     const long long m16 = ceil_div(g.npix, 16), m32 = ceil_div(g.npix, 32), n16 = ceil_div(g.cout, 16), n32 = ceil_div(g.cout, 32);
@@ -433,7 +434,7 @@ static int stream_tile(const NhwcGeom& g, int steps, bool odd, bool fp32_out, in
         return steps > convolutions * longest ? 0 : wide ? 12 : 11;
     }
     const int shortest = strided ? (fp32_out ? 6 : 8) : fp32_out ? 2 : 5;
-    return m32 * n32 <= 256 && steps >= shortest && steps <= convolutions * 48 ? 22 : 0;
+    return m32 * n32 <= 256 && steps >= shortest && steps <= convolutions * LONGEST_32 ? 22 : 0;
 }
 
 // offsets are 32 bits wide and BEYOND lies beyond every buffer
@@ -499,21 +500,34 @@ struct StreamForm
 {
     int u, w;
 };
-constexpr bool stream_form_built(int u, int blocks)
-{
-    return u * blocks <= 36;
-}
-static StreamForm stream_form(int steps, int blocks)
+static constexpr StreamForm stream_form(int steps, int blocks)
 {
     const int w = ceil_div(steps, 4) > 12 ? 8 : 4, per_wave = ceil_div(steps, w);
     StreamForm best = {1, w};
     for (int u : {2, 4, 6, 9, 12})
-        if (stream_form_built(u, blocks) && ceil_div(per_wave, u) < ceil_div(per_wave, best.u)) best.u = u;
+        if (u * blocks <= 36 && ceil_div(per_wave, u) < ceil_div(per_wave, best.u)) best.u = u;
     return best;
 }
 
+// Whether any number of steps up to the longest that the tile meets asks for this form: only such are built.
+constexpr bool stream_form_reached(int u, int w, int blocks, int longest)
+{
+    for (int steps = 1; steps <= longest; steps++)
+    {
+        const StreamForm f = stream_form(steps, blocks);
+        if (f.u == u && f.w == w) return true;
+    }
+    return false;
+}
+// 32 x 32 tiles end at the limits of stream_tile (of both convolutions, which have a step each at least); beyond 1281 steps, the longest pair of the smaller ones, it is always the
+// form with most in flight
+constexpr int stream_longest(int tp, bool shortcut)
+{
+    return tp == 2 ? (shortcut ? 2 * LONGEST_32 - 1 : LONGEST_32) : 1281;
+}
+
 template<bool DENSE, int TP, int TC, int W, bool SHORTCUT>
-static void launch_stream_form(int u, const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
+static bool launch_stream_form(int u, const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
                                const StreamShortcutArg<SHORTCUT>& shortcut, hipStream_t stream)
 {
     const int tiles_m = ceil_div(g.npix, 16 * TP), tiles = tiles_m * ceil_div(g.cout, 16 * TC); // 256 at most
@@ -522,13 +536,17 @@ static void launch_stream_form(int u, const NhwcGeom& g, const int8_t* wpk, cons
     StreamRest<SHORTCUT> rest = {{epi.scale_in, epi.bias, epi.scale_out, fusion.residual, epi.out, fusion.q8_out, fusion.q8_scale, fusion.relu_after, epi.act}, shortcut, {}};
     if (!DENSE)
         rest.taps = {g.H, g.W, g.kw, g.dh, g.dw, g.sh, g.sw, g.pad_top, g.pad_left, g.outw, plane, steps, magic_of(plane), magic_of(g.outw), magic_of(steps), magic_of(g.kw)};
-    constexpr int blocks = (TP + TC) * (SHORTCUT ? 2 : 1);
+    constexpr int blocks = (TP + TC) * (SHORTCUT ? 2 : 1), longest = stream_longest(TP, SHORTCUT);
     static_assert(LastArgument<decltype(conv_stream_kernel<DENSE, TP, TC, 1, W, SHORTCUT>)>::at() == REST_AT, "`rest` lies where the kernel looks for it");
 #define STREAM(U_)                                                                                                                                              \
-    if constexpr (stream_form_built(U_, blocks))                                                                                                                \
+    if constexpr (stream_form_reached(U_, W, blocks, longest))                                                                                                  \
         if (u == U_)                                                                                                                                            \
-    hipLaunchKernelGGL((conv_stream_kernel<DENSE, TP, TC, U_, W, SHORTCUT>), dim3((unsigned)tiles), dim3(64 * W), 0, stream, wpk, x, x_bytes, g.K, g.Cp, g.npix, \
-                       g.cout, out_cp, tiles, tiles_m, magic_of(tiles_m), ceil_div(g.K / 64, W), rest)
+        {                                                                                                                                                       \
+            const auto kernel = conv_stream_kernel<DENSE, TP, TC, U_, W, SHORTCUT>;                                                                             \
+            hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(64 * W), 0, stream, wpk, x, x_bytes, g.K, g.Cp, g.npix, g.cout, out_cp, tiles, tiles_m,      \
+                               magic_of(tiles_m), ceil_div(g.K / 64, W), rest);                                                                                 \
+            return true;                                                                                                                                        \
+        }
     STREAM(1);
     STREAM(2);
     STREAM(4);
@@ -536,39 +554,29 @@ static void launch_stream_form(int u, const NhwcGeom& g, const int8_t* wpk, cons
     STREAM(9);
     STREAM(12);
 #undef STREAM
+    return false;
 }
 
 template<bool DENSE, bool SHORTCUT>
-static void launch_stream_tile(int tile, int steps, const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
+static int launch_stream_tile(int tile, int steps, const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp,
                                StreamShortcutArg<SHORTCUT> shortcut, hipStream_t stream)
 {
     const StreamForm form = stream_form(steps, (tile / 10 + tile % 10) * (SHORTCUT ? 2 : 1));
     if constexpr (SHORTCUT) shortcut.per_wave = ceil_div(shortcut.Cp / 64, form.w);
 #define STREAM_TILE(TP_, TC_)                                                                                                      \
-    do                                                                                                                             \
-    {                                                                                                                              \
-        if (form.w == 8)                                                                                                           \
-            launch_stream_form<DENSE, TP_, TC_, 8, SHORTCUT>(form.u, g, wpk, x, epi, fusion, out_cp, shortcut, stream);            \
-        else                                                                                                                       \
-            launch_stream_form<DENSE, TP_, TC_, 4, SHORTCUT>(form.u, g, wpk, x, epi, fusion, out_cp, shortcut, stream);            \
-    } while (0)
-    if (tile == 11)
-        STREAM_TILE(1, 1);
-    else if (tile == 12)
-        STREAM_TILE(1, 2);
-    else
-        STREAM_TILE(2, 2);
+    (form.w == 8 ? launch_stream_form<DENSE, TP_, TC_, 8, SHORTCUT>(form.u, g, wpk, x, epi, fusion, out_cp, shortcut, stream)      \
+                 : launch_stream_form<DENSE, TP_, TC_, 4, SHORTCUT>(form.u, g, wpk, x, epi, fusion, out_cp, shortcut, stream))
+    const bool launched = tile == 11 ? STREAM_TILE(1, 1) : tile == 12 ? STREAM_TILE(1, 2) : STREAM_TILE(2, 2);
 #undef STREAM_TILE
+    NCNNHIP_REQUIRE(launched, "convolution: no form of the kernel for few tiles with %d steps in flight and %d wavefronts", form.u, form.w);
+    return launch_status(SHORTCUT ? "conv_stream_kernel (shortcut)" : "conv_stream_kernel");
 }
 
 int launch_conv_stream(const NhwcGeom& g, int tile, const int8_t* wpk, const int8_t* x, const ConvEpilogue& epi, const ConvFusion& fusion, int out_cp, hipStream_t stream)
 {
     NCNNHIP_REQUIRE(tile && !epi.acc_out, "convolution: this layer does not fit the kernel for few tiles");
-    if (stream_dense(g))
-        launch_stream_tile<true, false>(tile, g.K / 64, g, wpk, x, epi, fusion, out_cp, StreamShortcutArg<false>(), stream);
-    else
-        launch_stream_tile<false, false>(tile, g.K / 64, g, wpk, x, epi, fusion, out_cp, StreamShortcutArg<false>(), stream);
-    return launch_status("conv_stream_kernel");
+    if (stream_dense(g)) return launch_stream_tile<true, false>(tile, g.K / 64, g, wpk, x, epi, fusion, out_cp, StreamShortcutArg<false>(), stream);
+    return launch_stream_tile<false, false>(tile, g.K / 64, g, wpk, x, epi, fusion, out_cp, StreamShortcutArg<false>(), stream);
 }
 
 // us, two launches / one: one image 64 + 64 -> 256 on 56 x 56 (784 tiles of 32 x 32: conv_shortcut.hip) 8.0 / 5.5, 256 + 512 -> 1024 on 14 x 14 8.4 / 6.4,
@@ -585,8 +593,7 @@ int launch_conv_stream_shortcut(const NhwcGeom& g, const int8_t* wpk, const int8
     arg.plane = plane;
     arg.magic_plane = magic_of(plane);
     arg.magic_outw = magic_of(sc.outw);
-    launch_stream_tile<true, true>(tile, sc.Cp > g.K ? sc.Cp / 64 : g.K / 64, g, wpk, x, epi, fusion, out_cp, arg, stream);
-    return launch_status("conv_stream_kernel (shortcut)");
+    return launch_stream_tile<true, true>(tile, sc.Cp > g.K ? sc.Cp / 64 : g.K / 64, g, wpk, x, epi, fusion, out_cp, arg, stream);
 }
 
 } // namespace ncnnhip
