@@ -105,17 +105,27 @@ def test_few_tiles_kernel_fused_tail(rt, batch, c, hw, outc, kernel, pads, relu)
     assert np.array_equal(got, want, equal_nan=True) and np.array_equal(got_q, want_q)
 
 
-# Steps of K a wavefront has in flight at once (1, 2, 4, 6, 9, 12), rounds of them and eight wavefronts for more than 48 steps: each
+# Steps of K a wavefront has in flight at once (1, 2, 4, 6, 9, 12; on 32 x 32 tiles up to 9), rounds of them and eight wavefronts for more than 48 steps: each
 # side of every change, dense and with taps, on 16 x 16, 16 x 32 and 32 x 32 tiles; whole runs of steps left to no wavefront.
-@pytest.mark.parametrize("steps", [1, 4, 5, 8, 9, 13, 16, 17, 24, 25, 36, 37, 48, 49, 72, 73, 96, 97, 192])
+@pytest.mark.parametrize("steps", [1, 2, 4, 5, 8, 9, 13, 16, 17, 24, 25, 36, 37, 48, 49, 72, 73, 96, 97, 192])
 def test_few_tiles_kernel_runs_of_steps(rt, steps):
     print("[case] conv few tiles, steps", steps, flush=True)
-    for c, hw, outc, kernel, pads in ((64 * steps, (3, 5), 33, (1, 1), NONE), (64 * steps, (16, 16), 290, (1, 1), NONE), (64 * steps, (31, 32), 96, (1, 1), NONE),
-                                      (64 * max(1, steps // 9), (5, 4), 20, (3, 3), SAME3), (64 * max(1, steps // 9), (15, 16), 300, (3, 3), SAME3)):
-        if c * outc * hw[0] * hw[1] * kernel[0] * kernel[1] > 1 << 30:
+    nine = max(1, steps // 9)
+    for tile, batch, c, hw, outc, kernel, pads in ((16, 16), 1, 64 * steps, (3, 5), 33, (1, 1), NONE), ((16, 32), 1, 64 * steps, (16, 16), 290, (1, 1), NONE), \
+            ((16, 32), 1, 64 * steps, (31, 32), 96, (1, 1), NONE), ((32, 32), 1, 64 * steps, (63, 64), 60, (1, 1), NONE), ((16, 16), 1, 64 * nine, (5, 4), 20, (3, 3), SAME3), \
+            ((16, 32), 1, 64 * nine, (15, 16), 300, (3, 3), SAME3), ((32, 32), 4, 64 * nine, (13, 14), 250, (3, 3), SAME3):
+        if batch * c * outc * hw[0] * hw[1] * kernel[0] * kernel[1] > 1 << 30:
             continue
-        x, wq, b, ws, ins, tops = cases.conv_case(steps + outc, c, hw[0], hw[1], outc, kernel, 1, 102, True, True)
-        d = oracle.make_desc((c, hw[0], hw[1]), outc, kernel, (1, 1), (1, 1), pads, 0.0, 1, 1, 102, 1, (0.0, 0.0))
-        want = oracle.convolution_int8(d, x[0], wq, b, ws, ins[0], tops[0])
-        got = rt.conv_channels_last(x, wq, b, ws, ins, tops, outc, kernel, (1, 1), (1, 1), pads, 0.0, 1, 102, 1, (0.0, 0.0))
-        assert np.array_equal(got[0], want), (c, hw, outc, kernel)
+        total = c * kernel[0] * kernel[1] // 64
+        for term in (102, 2):
+            route = cases.conv_route(batch, c, *hw, outc, kernel, pads=pads, act=1, int8_out=term > 100)
+            longest = {(16, 16): (192, 641), (16, 32): (80, 145), (32, 32): (48, 48)}[tile][total % 2]
+            taken = total <= longest and (tile != (32, 32) or total >= (5 if term > 100 else 2))
+            assert (route.kernel == route.FEW_TILES) == taken and (not taken or (route.tile_pixels, route.tile_channels) == tile), (tile, total, term)
+            if tile != (32, 32) and term == 2:
+                continue
+            x, wq, b, ws, ins, tops = cases.conv_case(steps + outc, c, hw[0], hw[1], outc, kernel, 1, term, True, True, batch=batch)
+            d = oracle.make_desc((c, hw[0], hw[1]), outc, kernel, (1, 1), (1, 1), pads, 0.0, 1, 1, term, 1, (0.0, 0.0))
+            got = rt.conv_channels_last(x, wq, b, ws, ins, tops, outc, kernel, (1, 1), (1, 1), pads, 0.0, 1, term, 1, (0.0, 0.0))
+            for i in range(batch):
+                assert np.array_equal(got[i], oracle.convolution_int8(d, x[i], wq, b, ws, ins[0], None if tops is None else tops[0])), (tile, total, term, i)
