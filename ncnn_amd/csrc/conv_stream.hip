@@ -403,24 +403,24 @@ static bool stream_dense(const NhwcGeom& g)
 }
 
 // The tile: the smallest that gives no compute unit two (256 units), as what a tile costs is its operands' way to its unit, about 20 bytes a clock;
-// larger tiles (32 x 64 to 64 x 64) were quicker nowhere.  us in a captured chain, weights from HBM, the small-tile or pipelined kernel /
-// 16 x 16 / 16 pixels x 32 channels / 32 x 32 (56 x 56 to 7 x 7, one image unless said):
-//   3x3 256 -> 256 on 14 x 14 8.5 / 4.7 / 6.1 / 7.2, two images 8.6 / 6.8 / 6.1 / 7.2, four 8.6 / 10.8 / 9.6 / 7.3, eight (392 tiles of 32 x 32) 8.7 / 17 / 17 / 11.4
-//   1x1 1024 -> 256 on 14 x 14 5.8 / 3.7 / 4.1 / 4.7, eight images 6.0 / 11.6 / 9.0 / 6.7    1x1 2048 -> 512 on 7 x 7 7.4 / 4.9 / 5.6 / 7.2
-//   3x3 512 -> 512 on 7 x 7 9.9 / 7.0 / 9.2 / 10.7    3x3 128 -> 128 on 28 x 28 6.9 / 5.4 / 4.4 / 5.2    1x1 256 -> 1024 on 14 x 14, fp32 out 5.0 / 6.0 / 4.5 / 4.1
-//   1x1 960 -> 160 on 7 x 7, fp32 out 5.0 / 3.4 / 3.6 / 4.0, 32 images 6.0 / 6.7 / 5.1 / 4.6    1x1 64 -> 384 on 14 x 14 3.0 / 2.9 / 2.9 / 3.2
-// With 32 x 32 tiles the ring is level or ahead at both ends of K: int8 out 1x1 64 -> 64 on 56 x 56 3.0 / 3.2, 256 -> 64 3.6 / 3.9, 3x3 512 -> 512 on 7 x 7,
-// eight images 10.7 / 11.0 (four, 16 x 32 tiles: 10.2 / 9.2); fp32 out is ahead from two steps on (128 -> 64 on 56 x 56 3.34 / 3.21, 192 -> 64 3.52 / 3.31,
-// 256 -> 64 level, 3.68 / 3.71).
-// A single tap with a stride (1x1, not dense) costs its pixels' divisions and, on the ring, no more than a dense one: the ring is ahead of the smaller tiles below
-// five steps to int8 (64 -> 256 on 28 x 28, stride 2, 3.1 / 3.8; 256 -> 256 3.6 / 3.7, 320 -> 256 3.8 / 3.6) and three to fp32 (128 3.5 / 3.6, 192 3.6 / 3.6), of
-// 32 x 32 below eight and six (four images, int8 384 4.0 / 4.1, 512 5.3 / 4.5; fp32 256 3.9 / 4.2, 384 4.2 / 4.1).
-// (The figures of this rule are of the loads' former issue, where a tile cost 0.5 to 1 us more: the lines below are on the safe side.)
-// Beyond some K the ring, which splits it over workgroups, is quicker again.  Weight rows an odd number of steps (64 bytes of K) apart come in at 1.3 times the
+// larger tiles (32 x 64 to 64 x 64) were quicker nowhere.  us in a captured chain, each launch with weights of its own, the ring or the small-tile kernel /
+// 16 x 16 / 16 pixels x 32 channels / 32 x 32 (one image unless said):
+//   3x3 256 -> 256 on 14 x 14 7.9 / 4.1 / 5.2 / 6.4, two images 8.4 / 6.1 / 5.2 / 6.4, four 8.4 / 9.9 / 8.3 / 6.4, eight (392 tiles of 32 x 32) 8.4 / 16 / 14 / 10.4
+//   1x1 1024 -> 256 on 14 x 14 5.8 / 2.7 / 3.2 / 3.7, eight images 5.8 / 8.6 / 7.5 / 5.8    1x1 2048 -> 512 on 7 x 7 7.5 / 3.8 / 4.8 / 5.8
+//   3x3 512 -> 512 on 7 x 7 9.3 / 6.2 / 8.1 / 9.9, four images 9.8 / 10.0 / 8.2 / 10.1    3x3 128 -> 128 on 28 x 28 6.8 / 4.1 / 3.9 / 4.5
+//   1x1 256 -> 1024 on 14 x 14, fp32 out 4.2 / 3.0 / 2.7 / 2.6    1x1 960 -> 160 on 7 x 7, fp32 out 5.2 / 2.2 / 2.7 / 3.0, 32 images 5.7 / 4.2 / 3.7 / 3.4
+//   1x1 64 -> 384 on 14 x 14 2.6 / 2.1 / 2.1 / 2.3    1x1 512 -> 2048 on 7 x 7, fp32 out 4.6 / 3.0 / 2.8 / 3.2
+// The limits at the short end of K are older than the loads' present order, in which a tile costs 0.5 to 1 us less, and further in than they need be: the ring is behind there too.
+// Ring / here: dense on 32 x 32 tiles (56 x 56 and four images of 14 x 14) int8 out one step 2.7 / 2.4, two 2.9 / 2.4, four 3.2 and 3.8 / 2.5 against, from the line on,
+// five 3.4 / 2.6; fp32 out one step 3.1 / 2.3 against two 3.3 / 2.4.  A single tap with a stride on 16 x 16 tiles int8 out one step 2.7 / 2.1, four 3.3 / 2.2 against five 3.5 / 2.2;
+// fp32 out two steps 3.5 / 2.1 against three 3.6 / 2.1; on 32 x 32 int8 out seven 4.4 / 2.9 against eight 5.2 / 3.2, fp32 out five 4.5 / 2.8 against six 4.6 / 3.0.  (With two
+// tiles to a unit the two are level: 64 -> 256 on 56 x 56, 784 tiles, 2.8 / 2.8, 128 -> 128 on 40 x 56, 280 tiles, 2.9 / 2.8.)
+// Beyond some K the ring, which splits it over workgroups, is quicker.  Weight rows an odd number of steps (64 bytes of K) apart come in at 1.3 times the
 // rate of an even number, so the lines lie further out there.  Time here over the ring's, fp32 out, dense:
-//   16 x 16, below 128 tiles   even: 144 steps 0.87-0.93, 176 0.94-0.99, 194 1.00-1.06, 288 1.03-1.09    odd: 193 0.8, 401 0.86-0.91, 641 0.88-0.95
-//   16 x 16, from 128 on       even: 208 0.81-0.93, 288 0.91-0.98, 322 0.98-1.08, 402 1.02-1.23          odd: 401 0.78-0.94, 641 1.09-1.20
-//   16 x 32                    even: 64 0.87-0.91, 80 0.96-1.02, 96 1.04-1.05, 144 1.2, 402 2.0          odd: 81 0.8, 145 0.92-1.00, 193 1.00-1.17
+//   16 x 16, below 128 tiles   even: 144 steps 0.88, 176 0.95, 192 0.94, 194 0.99, 240 1.05        odd: 401 0.75, 641 1.00, 801 1.18
+//   16 x 16, from 128 on       even: 208 0.73, 240 0.86, 288 0.86-0.89, 322 0.98, 402 1.11         odd: 401 0.87, 481 0.94, 641 1.07
+//   16 x 32                    even: 64 0.82, 80 0.90-0.95, 96 0.96-0.99, 112 1.12-1.14            odd: 81 0.71-0.74, 145 0.95-1.02, 193 1.07-1.12
+//   32 x 32                    even: 40 0.74, 48 0.86, 56 0.97, 64 1.00, 72 1.05                   odd: 47 0.55, 49 0.74, 63 0.77
 constexpr int LONGEST_32 = 48; // steps of a 32 x 32 tile
 static int stream_tile(const NhwcGeom& g, int steps, bool odd, bool fp32_out, int convolutions)
 {
