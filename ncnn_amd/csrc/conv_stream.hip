@@ -296,11 +296,12 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
 #pragma unroll
     for (int n = 0; n < NB; n++) acc[n] = other[n] = v4i_cs{0, 0, 0, 0};
     auto multiply = [&] {
-        __builtin_amdgcn_sched_barrier(0); // every load above before the first product
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
             for (int n = 0; n < NB; n++) acc[n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[u][n / TP], fx[u][n % TP], acc[n], 0, 0, 0);
+    };
+    auto multiply_shortcut = [&] {
         if constexpr (SHORTCUT)
         {
 #pragma unroll
@@ -309,12 +310,32 @@ __global__ __launch_bounds__(64 * W) void conv_stream_kernel(const int8_t* __res
                 for (int n = 0; n < NB; n++) other[n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(sw[u][n / TP], sx[u][n % TP], other[n], 0, 0, 0);
         }
     };
-    multiply(); // (outside the loop, where its waits count the first round's loads alone)
-    while (s0 < end || t0 < t_end)
+    // the first round outside the loops, where its waits count its loads alone; every load above before the first product
+    __builtin_amdgcn_sched_barrier(0);
+    multiply();
+    multiply_shortcut();
+    while (SHORTCUT && s0 < end && t0 < t_end)
     {
         issue();
         issue_shortcut();
+        __builtin_amdgcn_sched_barrier(0);
         multiply();
+        multiply_shortcut();
+    }
+    // What is left of the longer K goes on alone: loads of steps that are not there cost a round as much as others.  us, with them / here: 512 channels on 7 x 7, 1 + 383 steps 25.8 /
+    // 20.7, 16 + 200 17.9 / 15.8; 2048 channels 1 + 100 15.9 / 13.9, 16 + 128 18.5 / 16.5; 256 on 28 x 28, 64 + 16 13.2 / 12.3.  (Without them in the first round, too, 1 + 383 20.2,
+    // but 8 + 16 on 2048 channels 5.0 -> 5.1: a branch there makes the first products wait for the last load.)
+    while (s0 < end)
+    {
+        issue();
+        __builtin_amdgcn_sched_barrier(0);
+        multiply();
+    }
+    while (SHORTCUT && t0 < t_end)
+    {
+        issue_shortcut();
+        __builtin_amdgcn_sched_barrier(0);
+        multiply_shortcut();
     }
 
     // the wavefronts' sums meet (integer addition: exact in any order)
@@ -470,10 +491,10 @@ bool conv_stream_tile_out_of_reach(const NhwcGeom& g)
     return stream_tile_any_k(g) != 0 && !stream_reaches(g);
 }
 
-// With a shortcut a workgroup walks both K, one after the other, in place of two launches that walk one each: the limits hold for the two together.
-// us, two launches / one, main + shortcut steps: 512 channels on 7 x 7 (16 x 16 tiles) 8 + 16 7.6 / 5.8, 64 + 64 13.6 / 11.7, 100 + 100 18.4 / 16.3; 2048 channels
-// there (16 x 32) 8 + 16 8.9 / 6.9, 64 + 64 18.6 / 16.6; 256 channels on 28 x 28 (32 x 32) 1 + 1 7.2 / 4.5 (the ring: 5.0), 1 + 16 9.0 / 6.2 (10.0),
-// 48 + 48 17.7 / 15.5, 64 + 32 17.3 / 16.5 (35.8); beyond its limit two launches are quicker than the ring (conv_shortcut_pays).
+// With a shortcut a workgroup walks both K, a round of each in flight together, in place of two launches that walk one each: the limits hold for the two together.
+// us, two launches / one, main + shortcut steps: 512 channels on 7 x 7 (16 x 16 tiles) 8 + 16 5.5 / 4.1, 64 + 64 11.7 / 9.8, 192 + 192 26.1 / 24.6, 1 + 383 20.9 / 20.7; 2048 channels
+// there (16 x 32) 8 + 16 6.7 / 5.0, 64 + 64 16.6 / 14.0, 80 + 80 20.1 / 18.0, 16 + 128 17.6 / 16.5; 256 channels on 28 x 28 (32 x 32) 1 + 1 6.7 / 3.5, 1 + 16 8.1 / 5.3,
+// 48 + 48 16.4 / 13.8, 90 + 1 14.3 / 14.7, 1 + 90 15.0 / 14.6; beyond its limit two launches are quicker than the ring (conv_shortcut_pays).
 int conv_stream_shortcut_tile(const NhwcGeom& g, int shortcut_steps)
 {
     return stream_dense(g) && g.K == g.Cp && stream_reaches(g) ? stream_tile(g, g.K / 64 + shortcut_steps, g.K / 64 % 2 == 1 && shortcut_steps % 2 == 1, true, 2) : 0;
@@ -579,8 +600,8 @@ int launch_conv_stream(const NhwcGeom& g, int tile, const int8_t* wpk, const int
     return launch_stream_tile<false, false>(tile, g.K / 64, g, wpk, x, epi, fusion, out_cp, StreamShortcutArg<false>(), stream);
 }
 
-// us, two launches / one: one image 64 + 64 -> 256 on 56 x 56 (784 tiles of 32 x 32: conv_shortcut.hip) 8.0 / 5.5, 256 + 512 -> 1024 on 14 x 14 8.4 / 6.4,
-// 512 + 1024 -> 2048 on 7 x 7 8.0 / 6.3.
+// us, two launches / one: one image 64 + 64 -> 256 on 56 x 56 (784 tiles of 32 x 32: conv_shortcut.hip) 7.3 / 5.3, 256 + 512 -> 1024 on 14 x 14 6.4 / 4.7,
+// 512 + 1024 -> 2048 on 7 x 7 6.7 / 5.0.
 int launch_conv_stream_shortcut(const NhwcGeom& g, const int8_t* wpk, const int8_t* x, const ConvShortcut& sc, const ConvEpilogue& epi, const ConvFusion& fusion,
                                 int out_cp, hipStream_t stream)
 {

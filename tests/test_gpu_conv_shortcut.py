@@ -45,6 +45,9 @@ SHAPES = [
     (1, 64, 28, 28, 250, 1024, 2),  # 32 x 32, most of K in the shortcut
     (1, 64, 56, 55, 64, 64, 1),  # 32 x 32, a step of each
     (2, 1600, 6, 5, 24, 64, 3),  # one step of shortcut, two rounds of the main convolution
+    (1, 64, 7, 7, 500, 5440, 1), (1, 5440, 7, 7, 500, 128, 2),  # 16 x 16, a K that goes on alone for rounds
+    (1, 192, 7, 7, 2000, 6400, 1), (1, 4160, 7, 7, 2048, 1088, 1),  # 16 x 32, the same
+    (1, 128, 28, 28, 256, 1600, 1), (1, 2560, 28, 28, 250, 192, 1),  # 32 x 32
     (1, 64, 56, 56, 256, 64, 1),  # the ring: 64-channel tiles
     (3, 128, 29, 27, 200, 192, 2),  # ragged pixels and channels
     (2, 64, 224, 224, 300, 64, 1),  # 128-channel tiles, the last mostly padding
