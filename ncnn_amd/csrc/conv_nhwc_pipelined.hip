@@ -118,10 +118,11 @@ static void choose_tile(const NhwcGeom& g, bool residual, PipePlan& p)
         p.bm = p.bn = 128;
     else if (wide && tiles(64, 128) >= (steps >= 16 ? 300 : 900) && (steps >= 2 || g.cout <= 128))
         p.bn = 128;
-    if (tiles(64, p.bn) > MOST_BLOCKS) // (an output of 69 GB and more)
+    if (!tiles_fit_a_launch(ceil_div(g.npix, 64), ceil_div(g.cout, p.bn))) // (an output of 69 GB and more)
     {
         p.bm = 128;
         p.bn = wide ? 128 : 64;
+        if (!tiles_fit_a_launch(ceil_div(g.npix, 128), ceil_div(g.cout, p.bn)) && ceil_div(g.cout, 256) * 256 <= ceil_div(g.cout, p.bn) * p.bn) p.bn = 256;
     }
     p.tiles_m = ceil_div(g.npix, p.bm);
     p.tiles_n = ceil_div(g.cout, p.bn);
@@ -182,8 +183,7 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
     NhwcGeom g = g_in;
     PipePlan p;
     const int mode = pipelined_form(g, fusion.residual != 0, p);
-    const long long blocks = (long long)p.tiles_m * p.tiles_n * p.splits;
-    NCNNHIP_REQUIRE(blocks * p.groups <= MOST_BLOCKS, "convolution: too many tiles");
+    NCNNHIP_REQUIRE(tiles_fit_a_launch(p.tiles_m, p.tiles_n), "convolution: too many tiles"); // (a K split is of 256 tiles at most)
     int32_t* partial = 0;
     unsigned* counters = 0;
     if (p.splits > 1)
@@ -224,6 +224,8 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
         LAUNCH_PIPE_MODE(64, 64, 3, 4);
     else if (p.groups == 4)
         LAUNCH_PIPE_MODE(64, 64, 0, 4);
+    else if (p.bm == 128 && p.bn == 256)
+        LAUNCH_PIPE(128, 256);
     else if (p.bm == 128 && p.bn == 128)
         LAUNCH_PIPE(128, 128);
     else if (p.bm == 128) // narrow inputs, and more tiles than a launch holds

@@ -116,15 +116,11 @@ __global__ __launch_bounds__(256 * GROUPS) void conv_nhwc_pipelined_kernel(const
         const int T = gridDim.x, xcd = b & 7, idx = b >> 3, rem = T & 7;
         b = xcd * (T >> 3) + (xcd < rem ? xcd : rem) + idx;
     }
-    // b / tiles_n by multiplication: with magic_n = 2^32/tiles_n + 1 it is the quotient or, of a large b * tiles_n, one more,
-    // and stays on the scalar unit, where a division would be some twenty vector instructions per wavefront
-    int rest = tiles_n == 1 ? b : (int)__umulhi((unsigned)b, magic_n);
-    int tn = b - rest * tiles_n;
-    if (tn < 0)
-    {
-        rest--;
-        tn += tiles_n;
-    }
+    // b / tiles_n by multiplication: magic_n = 2^32/tiles_n + 1 is exact while b * tiles_n < 2^32 (checked at launch),
+    // and stays on the scalar unit, where a division would be some twenty vector instructions per wavefront (a correction of the
+    // quotient, four scalar instructions in front of the first loads, costs small strided layers 1 to 4 %)
+    const int rest = tiles_n == 1 ? b : (int)__umulhi((unsigned)b, magic_n);
+    const int tn = b - rest * tiles_n;
     const int split = SPLITK ? rest / tiles_m : 0;
     const int tm = rest - split * tiles_m;
     const int row0 = tm * BM, col0 = tn * BN;
@@ -1140,14 +1136,17 @@ PipePlan plan_pipelined(int cout, long long npix, int steps);
 // takes more scratch than plan_pipelined's
 PipePlan plan_pipelined_groups(int cout, long long npix, int steps);
 
-// multiplier that turns b / tiles_n into a high multiply, which for b < 2^31 is at most one too large (tiles_n == 1 is special-cased)
+// multiplier that turns b / tiles_n into a high multiply, exact for b * tiles_n < 2^32 (tiles_n == 1 is special-cased)
 static inline unsigned tile_magic(int tiles_n)
 {
     return tiles_n > 1 ? (unsigned)((1ull << 32) / (unsigned)tiles_n + 1) : 0u;
 }
 
-// workgroups of 256 threads a launch may have: all threads are counted in 32 bits
-constexpr long long MOST_BLOCKS = (1ll << 24) - 1;
+// Whether a launch of this many tiles holds: a launch's threads, 256 to a workgroup, are counted in 32 bits, and the kernel divides a tile's number by multiplication.
+static inline bool tiles_fit_a_launch(long long tiles_m, long long tiles_n)
+{
+    return tiles_m * tiles_n < 1ll << 24 && tiles_m * tiles_n * tiles_n < 1ll << 32;
+}
 
 // The launches of conv_nhwc_pipelined_split.hip.  launch_pipe_split: the convolution kernel with K split over workgroups
 // (modes 0, 1 and 3; the grid, the partial sums and the counters come from the caller's plan).

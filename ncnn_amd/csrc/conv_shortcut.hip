@@ -39,10 +39,10 @@ int launch_conv_shortcut(const NhwcGeom& g_in, const int8_t* wpk, const int8_t* 
     // (12544 tiles of six steps) 93.2 / 86.4.
     const int tiles_m = ceil_div(g.npix, 64);
     const long long narrow = (long long)tiles_m * ceil_div(g.cout, 64);
-    const bool wide = narrow > MOST_BLOCKS || (narrow >= 8192 && g.K / 64 + sc.Cp / 64 <= 4);
+    const bool wide = !tiles_fit_a_launch(tiles_m, ceil_div(g.cout, 64)) || (narrow >= 8192 && g.K / 64 + sc.Cp / 64 <= 4);
     const int tiles_n = ceil_div(g.cout, wide ? 128 : 64);
     const long long blocks = (long long)tiles_m * tiles_n;
-    NCNNHIP_REQUIRE(blocks <= MOST_BLOCKS, "convolution: too many tiles");
+    NCNNHIP_REQUIRE(tiles_fit_a_launch(tiles_m, tiles_n), "convolution: too many tiles");
     ConvShortcutArg<true> arg;
     static_cast<ConvShortcut&>(arg) = sc;
 #define LAUNCH_SHORTCUT(BN_)                                                                                                                            \
