@@ -95,29 +95,50 @@ static int special_kernel(const NhwcGeom& g, const ConvEpilogue& epi, const Conv
     return conv_stream_tile(g, !epi.scale_out) ? NCNNHIP_CONV_FEW_TILES : NCNNHIP_CONV_PIPELINED;
 }
 
-// The tile of a layer whose K stays whole in four wavefronts.  us in passes of ResNet-50 and MobileNetV2, 8 to 128 images:
-//   a sum (residual in, fp32 and int8 out) is bound by memory, and small tiles keep more of it in flight: 64 x 64 / 64 x 128 / 64 x 256, 50176 pixels x 512 24.8 27.0 35.5, 25088 x 1024
-//   29.7 31.0 41.6, 25088 x 512 15.0 16.8 22.7, 6272 x 1024 10.8 12.3 14.0, 50176 x 256 14.3 16.1 21.8, 12544 x 1024 21.6 22.5 28.4; from about 8000 of them on 64 x 128 is as good or
-//   better: 401408 x 256 112.7 104.8 119.3 and 185 168 175, 100352 x 512 93.0 87.1 94.4, 200704 x 256 90.9 85.6 94.6, and from 3000 on with 8 steps: 6272 x 2048 31.2 30.2 33.5;
-//   a long K is bound by LDS, of which a tile twice as wide reads half as much a product, as long as there is a tile for every unit: 64 x 64 / 64 x 128 / 128 x 128, 36 steps 25088 x 256
-//   35.6 32.6 23.6, 16 steps the same 19.2 18.9 15.8; 72 steps 6272 x 512 34.0 30.8 33.5 (196 tiles), 32 steps 19.0 17.0 18.7, 36 steps 12544 x 256 19.5 17.7 19.9, 3136 x 512 27.0
-//   29.7 33.1; 18 steps 25088 x 128 11.9 11.1 12.9; 8 steps 25088 x 256 12.6 13.0 12.0, 50176 x 128 12.7 12.9 11.6, 100352 x 128 22.5 19.8 21.5, 12544 x 256 7.8 8.2 9.9;
-//   below 8 steps 64 x 64 / 64 x 128, one step 25088 x 384 7.5 8.6, 12544 x 384 5.1 6.0 (one tile for all channels is left as wide as they are), two 12544 x 576 7.6 6.9, four and five 100352 x 128 14.4 13.9, 6272 x 1280 14.2 13.0.
+// The tile of a layer whose K stays whole in four wavefronts.  A unit holds five workgroups of 64 x 64 pixels x channels, three of 64 x 128, two of 128 x 128; a wide tile reads half as much
+// from LDS for a product, and computes a pixel's address (a division, where the layer has taps or a stride) for twice the channels.  Measured in captured chains and in passes of ResNet-50 and MobileNetV2.
+//   64 x 128 over 64 x 64, by tiles of 64 x 128 (256 to 2048 channels): 384, where 64 x 64 are three to a unit, 16 and 18 steps 1.09 to 1.11, 36 1.05, 10 to 14 1.10 to 1.14, 3x3 to int8 5 1.09, 12
+//   and 14 1.01; from 400 on, where these are four: 16 and 18 steps 0.94 to 1.00, 23 and 36 0.79 to 0.91, 10 to 14 to int8 0.91 to 1.02, 3x3 to int8 5 0.93 to 1.01, 9 to 14 0.87 to 0.97, 3x3 to fp32 12 and 14
+//   0.91 to 1.02; with fewer steps, to fp32 or of a sum only beyond five to a unit (640): 10 and 14 steps to fp32 576 and 608 1.02 to 1.05, 688 0.96 to 1.01, 8 to int8 608 0.98 to 1.01, 688 0.91
+//   to 0.94, sums of 16 and 18 608 1.05, 688 0.92 to 0.94 (1040 1.06 to 1.08, 1200 0.97: between 1024 and 1160 they stay with 64 x 64), 3x3 of four to nine steps to fp32 676 0.94 to 0.96; with a short K beyond 900:
+//   one step 25088 x 384 7.5 8.6 us, 12544 x 384 5.1 6.0 (one tile for all channels is left as wide as they are), two 12544 x 576 7.6 6.9, four and five 100352 x 128 14.4 13.9, 6272 x 1280 14.2
+//   13.0; to int8 from 700 with a stride, one step 784 tiles 6.8 6.6, 1568 10.5 10.1, 1536 10.5 9.7 (500 tiles 4.7 4.8; to fp32 784 tiles 8.5 8.3, 1568 the other way by 4 to 8 %), and from 750
+//   where the one tile for all channels is partly padding, 96 channels 784 tiles 5.7 5.6, 896 6.0 5.8 (128 channels 784 tiles level).
+//   128 x 128 over 64 x 128, by tiles of 128 x 128: 384 of them 8 to 18 steps 1.00 to 1.13, 392, where 64 x 128 ones are more than three to a unit, 0.80 to 0.95 (8 steps to fp32 0.98 to 1.00, with
+//   64 x 64 the quickest); earlier from 300 with 23 steps and more, 304 0.93 to 1.04, 344 0.89 to 1.01 (a sum 1.00 to 1.04), or to int8 and more than 128 channels with 16, dense 304 0.99, 344 0.96, 3x3
+//   344 1.03, 368 1.00.  Beyond the 512 that are one round it is behind, 528 16 to 23 steps 1.08 to 1.15, 640 1.02 to 1.13, until 670, 680 0.94 to 1.07, 720 0.93 to 1.09 (to fp32 with 16
+//   and 18 until 770, 680 1.04 to 1.07, 768 1.02 and 1.04, 784 0.95 to 1.02; of a sum of 23 until 850, 640 1.17, 832 1.02, 900 0.94); with 9 to 15 steps at 784 0.95 to 1.18, and with 10 ahead again at 2256, 0.88 to
+//   1.00; a sum of 18 steps at 784 1.05.  25088 x 256, us of the three, 36 steps 35.6 32.6 23.6, 16 19.2 18.9 15.8, 8 12.6 13.0 12.0; sums 6272 x 1024, 36 steps 37.4 36.9 28.8, 12544 x 1024 69 62 56.
+//   A sum (residual in, fp32 and int8 out) of a short K is bound by memory, and small tiles keep more of it in flight: 64 x 64 / 64 x 128 50176 x 512 24.8 27.0, 25088 x 1024 29.7 31.0, 25088 x 512 15.0 16.8,
+//   6272 x 1024 10.8 12.3, 50176 x 256 14.3 16.1, 12544 x 1024 21.6 22.5; from about 7000 of them on, where its blobs no longer stay in the 256 MB in front of HBM, 64 x 128 is as good or better: 6656 tiles, 26624 x
+//   1024, two to four steps 37.5 to 40.4 / 37.4 to 41.2, 7168 47.9 46.5 to 61.1 56.5, 7680 56.9 52.6 to 69.4 60.7; 401408 x 256 112.7 104.8, 100352 x 512 93.0 87.1; with 8 steps from 3000: 6272 x 2048 31.2 30.2.
 // (64 x 256 is the best nowhere, 128 x 64 where 64 x 128 is nearly as good.)
-static void choose_tile(const NhwcGeom& g, bool residual, PipePlan& p)
+static void choose_tile(const NhwcGeom& g, bool residual, bool int8_out, bool dense, PipePlan& p)
 {
     const int steps = g.K / 64;
     const auto tiles = [&](int bm, int bn) { return (long long)ceil_div(g.npix, bm) * ceil_div(g.cout, bn); };
     const bool wide = ceil_div(g.cout, 128) * 128 <= ceil_div(g.cout, 64) * 64; // without more padded channels
+    const bool taps = g.ntaps > 1;
+    const long long t64 = tiles(64, 64), t128 = tiles(64, 128), square = tiles(128, 128);
     p.bm = p.bn = 64;
-    if (residual)
+    if (residual && steps < 14)
     {
-        if (wide && tiles(64, 64) >= (steps >= 8 ? 3000 : 8000)) p.bn = 128;
+        if (wide && t64 >= (steps >= 8 ? 3000 : 7000)) p.bn = 128;
     }
-    else if (wide && steps >= 8 && tiles(128, 128) >= 300 && (steps >= 16 || tiles(128, 128) <= 512))
-        p.bm = p.bn = 128;
-    else if (wide && tiles(64, 128) >= (steps >= 16 ? 300 : 900) && (steps >= 2 || g.cout <= 128))
-        p.bn = 128;
+    else if (wide)
+    {
+        const long long first = steps < 16 || residual ? 385 : steps >= 23 ? 300 : int8_out && g.cout > 128 ? (dense ? 300 : 360) : 385;
+        const long long again = residual ? 850 : steps < 16 ? 2000 : !int8_out && steps < 20 ? 770 : 670;
+        const bool square_pays = steps >= (int8_out ? 8 : 10) && square >= first && (square <= 512 || (square > again && steps >= (residual ? 23 : 10)));
+        const bool four_to_a_unit = residual ? steps >= 23 : steps >= 16 || (int8_out && (steps >= 10 || (taps && steps >= 5))) || (taps && steps >= 12);
+        const bool six_to_a_unit = taps || steps >= 14 || (int8_out && steps >= 8);
+        if (square_pays)
+            p.bm = p.bn = 128;
+        else if (t128 > (four_to_a_unit ? 384 : six_to_a_unit ? 640 : 899) && (steps >= 2 || g.cout <= 128))
+            p.bn = residual && steps < 23 && t128 > 1024 && t128 < 1160 ? 64 : 128;
+        else if (int8_out && ((!dense && t128 >= 700) || (g.cout < 128 && t128 >= 750)))
+            p.bn = 128;
+    }
     if (!tiles_fit_a_launch(ceil_div(g.npix, 64), ceil_div(g.cout, p.bn))) // (an output of 69 GB and more)
     {
         p.bm = 128;
@@ -129,7 +150,7 @@ static void choose_tile(const NhwcGeom& g, bool residual, PipePlan& p)
 }
 
 // the pipelined kernel's plan and addressing mode (its MODE), the layer as it sees it in g
-static int pipelined_form(NhwcGeom& g, bool residual, PipePlan& p)
+static int pipelined_form(NhwcGeom& g, const ConvEpilogue& epi, const ConvFusion& fusion, PipePlan& p)
 {
     // A 1x1, stride-1, unpadded layer reads input pixel n for output pixel n, whatever the image shape: present it as
     // one row of npix pixels, and the kernel skips the pixel -> (image, y, x) divisions.
@@ -140,7 +161,7 @@ static int pipelined_form(NhwcGeom& g, bool residual, PipePlan& p)
         g.W = g.outw = g.npix;
     }
     p = plan_pipelined_groups(g.cout, g.npix, g.K / 64);
-    if (p.groups == 1 && p.splits == 1) choose_tile(g, residual, p);
+    if (p.groups == 1 && p.splits == 1) choose_tile(g, fusion.residual != 0, epi.scale_out != 0, dense, p);
     // the narrow-input first layer has four K steps at most: from a million output pixels up, 128-pixel tiles halve the number of
     // workgroup prologues (ResNet-50's 7 x 7 first layer at batch 128: the pass 2.22 -> 2.20 ms; at batch 16, 0.2 M pixels, no gain)
     if ((g.tapK == 16 || g.tapK == 32) && p.splits == 1 && p.bm == 64 && g.npix >= (1 << 20))
@@ -164,7 +185,7 @@ void conv_nhwc_pipelined_route(const NhwcGeom& g_in, const ConvEpilogue& epi, co
     if (route.kernel != NCNNHIP_CONV_PIPELINED) return;
     NhwcGeom g = g_in;
     PipePlan p;
-    const int mode = pipelined_form(g, fusion.residual != 0, p);
+    const int mode = pipelined_form(g, epi, fusion, p);
     route = {NCNNHIP_CONV_PIPELINED, p.bm, p.bn, mode, p.groups, p.splits};
 }
 
@@ -182,7 +203,7 @@ int launch_conv_nhwc_pipelined(const NhwcGeom& g_in, const int8_t* wpk, const in
     }
     NhwcGeom g = g_in;
     PipePlan p;
-    const int mode = pipelined_form(g, fusion.residual != 0, p);
+    const int mode = pipelined_form(g, epi, fusion, p);
     NCNNHIP_REQUIRE(tiles_fit_a_launch(p.tiles_m, p.tiles_n), "convolution: too many tiles"); // (a K split is of 256 tiles at most)
     int32_t* partial = 0;
     unsigned* counters = 0;

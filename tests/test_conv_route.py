@@ -35,6 +35,16 @@ def test_forms_of_the_pipelined_kernel():
     ((128, 128, 28, 28, 128, (3, 3)), SAME3, (128, 128)),  # a long K of 128 channels and many pixels
     ((128, 128, 28, 28, 512, (1, 1)), dict(fused=True), (64, 128)), ((64, 128, 28, 28, 512, (1, 1)), dict(fused=True), (64, 64)),
     ((128, 512, 7, 7, 2048, (1, 1)), dict(fused=True), (64, 128)),
+    # sums of a long K: by LDS, as other layers of that K
+    ((64, 512, 14, 14, 512, (3, 3)), dict(fused=True, **SAME3), (128, 128)), ((80, 512, 14, 14, 1024, (3, 3)), dict(fused=True, **SAME3), (128, 128)),
+    ((8, 256, 14, 14, 2048, (3, 3)), dict(fused=True, **SAME3), (64, 128)), ((64, 128, 14, 14, 1024, (3, 3)), dict(fused=True, **SAME3), (64, 128)),
+    ((46, 512, 14, 14, 1024, (3, 3)), dict(fused=True, **SAME3), (64, 128)), ((48, 256, 14, 14, 1024, (3, 3)), SAME3, (64, 128)), ((56, 256, 14, 14, 1024, (3, 3)), SAME3, (128, 128)),
+    ((32, 256, 14, 14, 256, (3, 3)), dict(fused=True, **SAME3), (64, 64)), ((32, 96, 14, 14, 1024, (3, 3)), dict(fused=True, **SAME3), (128, 128)),
+    ((104, 128, 16, 16, 1024, (1, 1)), dict(fused=True), (64, 64)), ((112, 128, 16, 16, 1024, (1, 1)), dict(fused=True), (64, 128)),
+    # to int8: strided, and one tile that is partly padding
+    ((64, 64, 28, 28, 512, (1, 1)), dict(stride=(2, 2), int8_out=True), (64, 128)), ((64, 64, 28, 28, 512, (1, 1)), dict(stride=(2, 2)), (64, 64)),
+    ((32, 64, 28, 28, 512, (1, 1)), dict(stride=(2, 2), int8_out=True), (64, 64)),
+    ((16, 256, 56, 56, 96, (1, 1)), dict(int8_out=True), (64, 128)), ((16, 256, 56, 56, 128, (1, 1)), dict(int8_out=True), (64, 64)),
     ((32, 64, 28, 28, 384, (1, 1)), {}, (64, 64)), ((128, 320, 7, 7, 1280, (1, 1)), {}, (64, 128)),
     ((8, 32, 368, 368, 64, (1, 1)), {}, (128, 64)),
 ], ids=str)

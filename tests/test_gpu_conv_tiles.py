@@ -12,16 +12,21 @@ F = np.float32
 
 
 @pytest.mark.parametrize("batch,c,h,w,outc,kernel,term,fused,tile,addressing", [
-    (41, 1024, 21, 23, 256, (1, 1), 102, False, (128, 128), 1),
-    (41, 1024, 21, 23, 250, (1, 1), 2, False, (128, 128), 1),      # channel tail
-    (41, 128, 21, 23, 256, (3, 3), 102, False, (128, 128), 3),
-    (41, 112, 21, 23, 256, (3, 3), 2, False, (128, 128), 0),       # taps that are no whole steps
+    (52, 1024, 21, 23, 256, (1, 1), 102, False, (128, 128), 1),
+    (52, 1024, 21, 23, 250, (1, 1), 2, False, (128, 128), 1),      # channel tail
+    (52, 128, 21, 23, 256, (3, 3), 102, False, (128, 128), 3),
+    (52, 112, 21, 23, 256, (3, 3), 2, False, (128, 128), 0),       # taps that are no whole steps
     (41, 512, 21, 23, 512, (1, 1), 2, False, (64, 128), 1),        # 8 steps on more tiles of 128 x 128 than fill the chip twice
     (41, 64, 21, 23, 256, (1, 1), 102, False, (64, 64), 1),        # one step
     (41, 512, 21, 23, 192, (1, 1), 102, False, (64, 64), 1),       # channels that no 128-wide tiles cover without more padding
     (41, 512, 21, 23, 512, (1, 1), 2, True, (64, 64), 1),
     (41, 512, 21, 23, 1024, (1, 1), 2, True, (64, 128), 1),
     (41, 64, 21, 23, 1024, (3, 3), 2, True, (64, 128), 3),         # 9 steps
+    (52, 256, 21, 23, 250, (3, 3), 2, True, (128, 128), 3),        # a sum of 36 steps
+    (50, 208, 15, 17, 512, (3, 3), 2, True, (128, 128), 0),        # 30, taps that are no whole steps
+    (41, 128, 21, 23, 512, (3, 3), 2, True, (64, 128), 3),         # 18 steps on more than 512 tiles of 128 x 128
+    (41, 160, 21, 23, 256, (3, 3), 2, False, (128, 128), 0),       # 23 steps on more than 300 of them
+    (41, 128, 21, 23, 256, (3, 3), 102, False, (64, 128), 3),      # 18 on as many
 ], ids=str)
 def test_tile_of_a_layer(batch, c, h, w, outc, kernel, term, fused, tile, addressing):
     import ncnn_amd
@@ -30,7 +35,7 @@ def test_tile_of_a_layer(batch, c, h, w, outc, kernel, term, fused, tile, addres
     assert (route.kernel, route.tile_pixels, route.tile_channels, route.addressing, route.groups, route.splits) == (route.PIPELINED,) + tile + (addressing, 1, 1)
     x, wq, b, ws, ins, tops = cases.conv_case(21, c, h, w, outc, kernel, 1, term, True, True, batch=batch)
     d = oracle.make_desc((c, h, w), outc, kernel, (1, 1), (1, 1), pads, 0.0, 1, 1, term, 0 if fused else 1, (0.0, 0.0))
-    checked = (0, 1, 20, 39, 40)
+    checked = (0, 1, 20, 39, batch - 1)
     want = np.stack([oracle.convolution_int8(d, x[i], wq, b, ws, ins[0], None if tops is None else tops[0]) for i in checked])
     rt = ncnn_amd.Runtime(0)
     args = (x, wq, b, ws, ins, tops, outc, kernel, (1, 1), (1, 1), pads, 0.0, 1, term, 0 if fused else 1, (0.0, 0.0))
