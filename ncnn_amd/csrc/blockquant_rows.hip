@@ -21,9 +21,10 @@
 // 4096 x 4096 16 rows 12.4 -> 10.7, 32 rows 20.1 -> 12.9, 64 rows 34 -> 17.5, 128 rows 41 -> 30; 11008 x 4096 16 rows 26.5 -> 16.6, 32
 // rows 46 -> 26.5; 4096 x 11008 32 rows 45 -> 27, 128 rows 93 -> 66.
 // Two wavefronts share a SIMD and the one that multiplies goes first (left to itself the SIMD serves its oldest, which ends up to 4 us before its neighbour and leaves it
-// alone with its waits); the sums of a result are requested at once and the matrices' ends too.  us, before -> here: fp32 rows, 8 bits, 64 x 4096 x 4096 17.2 -> 16.5, 42 x
-// 6880 x 5312 34.1 -> 32.5, 16 x 4096 x 4096 10.8 -> 10.4, 6 bits 100 x 1248 x 7296 25.9 -> 24.4; fp16 rows, the four launches of a decoder layer, 48 rows at 4 bits 59.4 ->
-// 57.9 in the kernel trace.  (Loads of the stage after the next as soon as a stage is in registers: 66.6 -> 68.6 for the layer.  Without any loads its four launches take 48,
+// alone with its waits); the sums of a result are requested at once.  us a launch in a chain
+// of them, before -> here: fp32 rows, 8 bits, 64 x 4096 x 4096 16.4 -> 15.7, 42 x 6880 x 5312 33.6 -> 32.3, 16 x 4096 x 4096 10.5 -> 10.1, 6 bits 100 x 1248 x 7296
+// 24.6 -> 23.6; fp16 rows, the four launches of a decoder layer, 48 rows at 4 bits 54.2 -> 52.4; a K of 256 or 384 1 % slower, by the
+// branch of its sums.  (Loads of the stage after the next as soon as a stage is in registers: 66.6 -> 68.6 for the layer.  Without any loads its four launches take 48,
 // without the products 50, with neither 29.)
 // A lane must fetch along a row (eight lanes = one 128-byte line) and read in operand order (lane = row), so the chunks of a row
 // are swizzled on the source side: chunk c of row r lands at position c ^ ((r / 2) % 8), conflict-free both ways.
@@ -152,15 +153,9 @@ __global__ __launch_bounds__(rows_waves(BITS, MG, RT, SPLIT, AIN) * 64) void blo
     int group = round * 8 + (in_round & 7);
     const int row0 = (in_round >> 3) * MG * 16;
     if (group >= groups) return;
-    int mat = 0, before = 0; // tile_end counts groups of RT tiles here; all of them are read at once
-#pragma unroll
-    for (int i = 0; i < BQ_MULTI_MAX - 1; i++)
-    {
-        const bool later = i + 1 < mm.count && group >= mm.tile_end[i];
-        mat += later;
-        before = later ? mm.tile_end[i] : before;
-    }
-    group -= before;
+    int mat = 0; // tile_end counts groups of RT tiles here
+    while (mat + 1 < mm.count && group >= mm.tile_end[mat]) mat++; // (all ends read at once: 1 to 2 % slower for one matrix, 0.3 % for two to four)
+    group -= mat ? mm.tile_end[mat - 1] : 0;
     const int N = mm.N[mat], ntiles = (N + 15) >> 4;
     const int M = M_total - row0 < MG * 16 ? M_total - row0 : MG * 16;
 
