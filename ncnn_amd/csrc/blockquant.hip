@@ -2531,8 +2531,9 @@ int ncnnhip_gemm_blockquant_packed_rows(const float* a_dev, size_t a_stride, int
     // units, one tile per wavefront (64 weight rows per workgroup) doubles them.
     // One, two or three tiles per wavefront (64, 128 or 192 weight rows per workgroup).  The chip holds 512 workgroups at once:
     // where some choice fits in one round, the one with the most workgroups; else the fewest rounds weighted by a
-    // workgroup's cost (0.68 : 1 : 1.4, measured).  1500 x 3072 x 1024 is 576 workgroups with two tiles - a second round
-    // for 64 of them - and 384 with three: 63.6 -> 55.9 us; 1100 x 4096 x 4096 189 -> 173; 2048 x 11008 x 4096 672 -> 650.
+    // workgroup's cost (0.68 : 1 : 1.4, measured with blocks of 64; only blocks of 32 come here by it now).  Blocks of 32, 8 bits, us with one,
+    // two and three: 723 x 5952 x 1152 61.7, 61.5 and 53.3, the one that fits a round; 2248 x 3584 x 4608 295, 255 and 269; 682 x 12224 x 5376
+    // 367, 335 and 288.  Over 150 sizes of 200 to 3000 rows, 8 and 4 bits, the rule is 0.3 % behind the best of the three, at most 11 %.
     int rw_tiles = 2;
     {
         const long long row_tiles = Mp / 64;

@@ -20,12 +20,12 @@
 // parts it saves that launch (5 us) and a third of the bytes.  us per call before (blockquant.hip's forms) -> here, 8 bits in blocks of 64:
 // 4096 x 4096 16 rows 12.4 -> 10.7, 32 rows 20.1 -> 12.9, 64 rows 34 -> 17.5, 128 rows 41 -> 30; 11008 x 4096 16 rows 26.5 -> 16.6, 32
 // rows 46 -> 26.5; 4096 x 11008 32 rows 45 -> 27, 128 rows 93 -> 66.
-// Two wavefronts share a SIMD and the one that multiplies goes first (left to itself the SIMD serves its oldest, which ends up to 4 us before its neighbour and leaves it
-// alone with its waits); the sums of a result are requested at once.  us a launch in a chain
-// of them, before -> here: fp32 rows, 8 bits, 64 x 4096 x 4096 16.4 -> 15.7, 42 x 6880 x 5312 33.6 -> 32.3, 16 x 4096 x 4096 10.5 -> 10.1, 6 bits 100 x 1248 x 7296
-// 24.6 -> 23.6; fp16 rows, the four launches of a decoder layer, 48 rows at 4 bits 54.2 -> 52.4; a K of 256 or 384 1 % slower, by the
-// branch of its sums.  (Loads of the stage after the next as soon as a stage is in registers: 66.6 -> 68.6 for the layer.  Without any loads its four launches take 48,
-// without the products 50, with neither 29.)
+// Two wavefronts share a SIMD and the one that multiplies goes first (left to itself the SIMD serves its oldest, which ends up to 4 us
+// before its neighbour and leaves it alone with its waits); the sums of a result are requested at once.  us a launch in a chain of them,
+// before -> here: fp32 rows, 8 bits, 64 x 4096 x 4096 16.4 -> 15.7, 42 x 6880 x 5312 33.6 -> 32.3, 16 x 4096 x 4096 10.5 -> 10.1, 6 bits
+// 100 x 1248 x 7296 24.6 -> 23.6; fp16 rows, the four launches of a decoder layer, 48 rows at 4 bits 54.2 -> 52.4; a K of 256 or 384 is 1 %
+// slower, by the branch of its sums.  (Loads of the stage after the next as soon as a stage is in registers: 66.6 -> 68.6 for the layer.
+// Without any loads its four launches take 48, without the products 50, with neither 29.)
 // A lane must fetch along a row (eight lanes = one 128-byte line) and read in operand order (lane = row), so the chunks of a row
 // are swizzled on the source side: chunk c of row r lands at position c ^ ((r / 2) % 8), conflict-free both ways.
 #include <atomic>

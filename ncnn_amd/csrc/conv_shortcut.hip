@@ -11,10 +11,10 @@ namespace ncnnhip {
 // Here a workgroup walks both K whole behind one barrier a step, where each convolution alone would share its K between sixteen wavefronts or split it over
 // workgroups (up to 256 tiles) or run on wider tiles (many): what the launch saves is a launch and the fp32 blob, what it loses grows with the steps (64 of K).
 // Time of one launch over that of two, fp32 and quantised output (main + shortcut steps; tiles of 64 x 64):
-//   104 to 256 tiles   1 + 1 0.68, 4 + 8 0.82-0.86, 6 + 12 0.88-0.95, 8 + 16 1.00-1.10, 16 + 32 1.16-1.38; 1 + 16 0.91-0.95, 11 + 1 0.90-0.95, 16 + 1 1.03-1.08
-//   304 to 496         1 + 1 0.68, 8 + 16 0.91-0.94, 10 + 20 0.94-0.98, 12 + 24 0.98-1.02, 16 + 32 1.02-1.08
-//   784 and 1568       1 + 1 0.54-0.66, 8 + 16 0.82-0.87, 12 + 24 0.89-0.93, 16 + 32 0.93-0.98 (int8 alone up to 1.01)
-//   3136               1 + 1 0.58, 4 + 8 0.78, 8 + 16 0.95, 10 + 20 0.98 (int8 alone 1.03), 12 + 24 1.00 (1.08)
+//   160 tiles   1 + 1 0.70, 4 + 8 0.87, 6 + 12 0.95, 8 + 16 1.09, 16 + 32 1.37; 1 + 16 0.98, 11 + 1 0.94
+//   400         1 + 1 0.68, 8 + 16 0.95, 10 + 20 1.00, 12 + 24 1.04, 16 + 32 1.08
+//   784         1 + 1 0.66, 8 + 16 0.94, 12 + 24 1.01, 16 + 32 1.07
+//   3136        1 + 1 0.60, 4 + 8 0.81, 8 + 16 0.99, 10 + 20 1.08, 12 + 24 1.11
 bool conv_shortcut_pays(const NhwcGeom& g, int shortcut_steps)
 {
     if (conv_stream_shortcut_tile(g, shortcut_steps)) return true;
